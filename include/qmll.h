@@ -204,6 +204,29 @@ typedef struct {
  * the reference's loop starts from torch.zeros, kernel.py:134-137).  64 <= d <= 256. */
 int qmll_derivative_features_typed(const qmll_df_element* elements, int ne, double normalisation, int n, int d, int S,
                                    int T, int nmol, int overwrite, double* G, qmll_stream_t stream);
+/* The same with a row table, row_offsets i32 [nmol + 1] (device): molecule m has row_offsets[m+1] - row_offsets[m] <= 3n
+ * rows, the first so many of its Jacobian rows, which go to rows row_offsets[m].. of G f64 [row_offsets[nmol], S*d].
+ * NULL: 3n rows each. */
+int qmll_derivative_features_rows(const qmll_df_element* elements, int ne, double normalisation, const int* row_offsets, int n,
+                                  int d, int S, int T, int nmol, int overwrite, double* G, qmll_stream_t stream);
+
+/* ---- force rows of a training batch without the combinations that vanish ------------------------- */
+/* A molecule's force rows (qml_lightning/models/kernel.py:167-170) satisfy three (periodic) or up to six linear relations,
+ * its translations and rotations.  qmll_rigid_modes builds per molecule the orthogonal transformation Q whose transpose
+ * maps them onto the first modes[m] of its 3 natoms[m] rows; Z^T Z and Z^T y are the same for the rows Q^T G without
+ * those.  X f32 [B,n,3] (real atoms first), natoms / modes i32 [B] (modes: 3 translations plus the number of
+ * independent rotations to take, at most 6), row_offsets i32 [B+1] (running sum of 3 natoms - modes), work: device memory
+ * of qmll_rigid_workspace_bytes(B, n) for Q; forces f64 [B,n,3] or NULL -> targets f64 [row_offsets[B]] = the rows of
+ * Q^T y.  qmll_rigid_rows applies Q^T in place to the projected Jacobian rows grad f32 [A,3n,d] of the atoms in
+ * slots i32 [A] (molecule = slot / n); the rows that remain move to the front of each atom's block. */
+size_t qmll_rigid_workspace_bytes(int B, int n);
+int qmll_rigid_modes(const float* X, const int* natoms, const int* modes, const int* row_offsets, int B, int n, double* work,
+                     size_t work_bytes, const double* forces, double* targets, qmll_stream_t stream);
+int qmll_rigid_rows(float* grad, const int* slots, const int* natoms, const int* modes, const double* work, int A, int B, int n,
+                    int d, qmll_stream_t stream);
+/* First atom of every molecule within each element's part of the element-sorted slots (slot / n = molecule, ascending
+ * within an element): seg i32 [ne][B+1], relative to the element's first atom. */
+int qmll_typed_segments(const int* sorted_slots, const int* type_offsets, int ne, int B, int n, int* seg, qmll_stream_t stream);
 
 /* Fused predict path for one element: SORF (T = ntransforms) + cos features + energy
  * contraction + the gradient with respect to the projected representation, without ever
@@ -388,6 +411,23 @@ int qmll_rff_features(const float* x, const double* W, const double* b, const in
 int qmll_rff_derivative_features(const float* x, const float* grad, const double* W, const double* b,
                                  const int* mol_index, const int* seg_offsets, int A, int n, int d, int F,
                                  int nmol, double* G, qmll_stream_t stream);
+
+/* One element's inputs of qmll_rff_rows: projected rows f32 [A_e,d], projected Jacobian rows f32 [A_e,3n,d], W f32
+ * [d,F], b f32 [F], first atom of each molecule i32 [nmol+1] (all device pointers). */
+typedef struct {
+    const float* x;
+    const float* grad;
+    const float* W;
+    const float* b;
+    const int* seg_offsets;
+} qmll_rff_element;
+
+/* qmll_rff_features and qmll_rff_derivative_features for every element of the batch in ONE launch (the loop over
+ * elements around qml_lightning/models/random_features.py:60-67): Ze f64 [nmol,F] (NULL: not wanted) and G += the
+ * energy and force rows, or = with overwrite.  row_offsets as for qmll_derivative_features_rows; max_rows = the largest
+ * number of rows of a molecule.  d in {64,128,256}, ne <= 8. */
+int qmll_rff_rows(const qmll_rff_element* elements, int ne, const int* row_offsets, int max_rows, int n, int d, int F, int nmol,
+                  int overwrite, double* Ze, double* G, qmll_stream_t stream);
 
 /* W f32 [ne,d,F] of a RandomFourrierFeaturesModel (qml_lightning/models/random_features.py:42-55) is
  * a constant of the model: it is split ONCE into the form the fused predict kernel multiplies with

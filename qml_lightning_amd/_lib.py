@@ -28,6 +28,11 @@ class DfElement(Structure):
     _fields_ = [("cos_derivs", c_void_p), ("input_derivative", c_void_p), ("D", c_void_p), ("seg_offsets", c_void_p)]
 
 
+class RffElement(Structure):
+    """Mirror of struct qmll_rff_element (device pointers)."""
+    _fields_ = [("x", c_void_p), ("grad", c_void_p), ("W", c_void_p), ("b", c_void_p), ("seg_offsets", c_void_p)]
+
+
 P = c_void_p  # every device pointer and the stream travel as void*
 _FCHL_COMMON = [P, P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, P, P, POINTER(FchlParams)]
 
@@ -51,6 +56,11 @@ PROTOTYPES = {
     "qmll_sin_coeffs_f64": [P, P, c_int, c_int, P, P],
     "qmll_derivative_features": [P, c_double, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
     "qmll_derivative_features_typed": [POINTER(DfElement), c_int, c_double, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
+    "qmll_derivative_features_rows": [POINTER(DfElement), c_int, c_double, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
+    "qmll_rigid_workspace_bytes": [c_int, c_int],
+    "qmll_rigid_modes": [P, P, P, P, c_int, c_int, P, c_size_t, P, P, P],
+    "qmll_rigid_rows": [P, P, P, P, P, c_int, c_int, c_int, c_int, P],
+    "qmll_typed_segments": [P, P, c_int, c_int, c_int, P, P],
     "qmll_sorf_energy_fused": [P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, P, P, P],
     "qmll_sorf_energy_typed": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P, P, P],
     "qmll_sort_by_type_workspace": [c_int, c_int],
@@ -68,6 +78,7 @@ PROTOTYPES = {
     "qmll_sorf_energy_sorted": [P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, P, P, P],
     "qmll_rff_features": [P, P, P, P, c_int, c_int, c_int, c_int, P, P],
     "qmll_rff_derivative_features": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P],
+    "qmll_rff_rows": [POINTER(RffElement), c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P],
     "qmll_rff_presplit_bytes": [c_int, c_int, c_int],
     "qmll_rff_presplit": [P, c_int, c_int, c_int, P, c_size_t, P],
     "qmll_rff_energy_sorted": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, P, P, P],
@@ -87,7 +98,7 @@ PROTOTYPES = {
     "qmll_probe_rate": [c_int, c_int, c_int, P, P],
     "qmll_probe_mix": [c_int, c_int, c_int, P, P],
 }
-_RESTYPES = {"qmll_last_error": c_char_p, "qmll_rff_presplit_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
+_RESTYPES = {"qmll_last_error": c_char_p, "qmll_rigid_workspace_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
              "qmll_cholesky_workspace_bytes": c_size_t, "qmll_gram_workspace_bytes": c_size_t,
              "qmll_probe_out_bytes": c_size_t, "qmll_probe_rate": c_double,
              "qmll_probe_mix": c_double}

@@ -6,13 +6,14 @@
 //    rows (atoms, or the 3 x TJ derivative rows of one atom), whose fp32 inputs sit in LDS
 //    and are read by broadcast, so each W[k,f] load (coalesced over the workgroup) is reused
 //    for every row of the chunk.  Any atom order; molecule sums through fp64 atomics.
-//  * rff_derivative_mfma_kernel, for molecule-major atoms: a workgroup owns (molecule, 64
-//    feature columns, up to 63 derivative rows).  Each wavefront keeps its 16 columns of W as
-//    MFMA B fragments in registers for the whole molecule; per atom the 63 derivative rows
-//    plus the atom's own x row (whose product is the sine argument) form one 64 x d A tile
-//    in LDS, multiplied with v_mfma_f64_16x16x4_f64; the per-atom product is scaled by the
-//    sine column factor and summed over the molecule's atoms in registers, so G is
-//    read-modify-written once per element and no atomics are needed.
+//  * rff_rows_kernel, for molecule-major atoms: a workgroup owns (molecule, 64 feature columns,
+//    up to 63 derivative rows).  Each wavefront keeps its 16 columns of an element's W as MFMA B
+//    fragments in registers; per atom the derivative rows plus the atom's own x row (whose
+//    product is the sine argument) form one A tile of 16-row blocks in LDS, multiplied with
+//    v_mfma_f64_16x16x4_f64; the per-atom product is scaled by the sine column factor and summed
+//    over the molecule's atoms in registers, so G is written once and no atomics are needed.
+#include <type_traits>
+
 #include "qmll_common.h"
 
 namespace {
@@ -99,102 +100,173 @@ __global__ __launch_bounds__(RT) void rff_derivative_kernel(const float* __restr
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
-constexpr int MROWS = 64;   // A-tile rows: 63 derivative rows + the atom's x row
+constexpr int MROWS = 64;   // A-tile rows: up to 63 derivative rows + the atom's x row
 constexpr int MPAD = 4;     // floats of padding per LDS row: 16 rows x 4 k land in 64 distinct banks
 
-// grid (ceil(F/64), nmol, ceil(3n/63)), 256 threads.
-template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void rff_derivative_mfma_kernel(const float* __restrict__ x,
-                                                                  const float* __restrict__ grad,
-                                                                  const double* __restrict__ W,
-                                                                  const double* __restrict__ b,
-                                                                  const int* __restrict__ seg, int n, int F,
-                                                                  double* __restrict__ G) {
+// the elements of a batch (molecule-major atoms within each)
+constexpr int RFF_MAXE = 8;
+struct RffElements {
+    const float* x[RFF_MAXE];      // [A_e, d]
+    const float* grad[RFF_MAXE];   // [A_e, 3n, d]
+    const void* W[RFF_MAXE];       // [d, F]
+    const void* b[RFF_MAXE];       // [F]
+    const int* seg[RFF_MAXE];      // first atom of each molecule [nmol + 1]
+    int ne;
+};
+
+// grid (ceil(F/64), nmol, ceil(max rows / 63)), 256 threads.  All elements of the batch in one launch: G (and, when
+// asked for, the energy features, whose argument is the same product) is written once, or read and written once.
+// The tile holds as many 16-row blocks as the molecule's rows need (one matrix instruction per block and four k).
+// Bound by the fp64 matrix cores: 200 molecules of 3 to 29 atoms, 128 components, 8192 features: 7.3 ms, where a tile
+// of 64 rows for every molecule padded to 29 atoms, a launch per element and a kernel of its own for the energy
+// features took 16.3 ms (of which the rows left out by the row table are a half).  The sine and cosine cost up to a
+// sixth: every lane group of a column works them out.
+// W is fp32 in a model (converted exactly in the registers) or fp64.
+template <int D, typename TW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void rff_rows_kernel(
+    RffElements E, const int* __restrict__ row_offsets, int n, int F, int overwrite, double* __restrict__ Ze,
+    double* __restrict__ G) {
     constexpr int LD = D + MPAD;
     constexpr int KS = D / 4;                 // MFMA k-steps
-    constexpr int V4 = MROWS * D / 4 / 256;   // float4 loads per thread per tile
-    __shared__ __attribute__((aligned(16))) float tile[MROWS * LD];
+    // two tiles: the next atom's is written while this one's is read, one barrier per atom
+    __shared__ __attribute__((aligned(16))) float tiles[2][MROWS * LD];
 
     const int mol = blockIdx.y;
-    const int a_begin = seg[mol], a_end = seg[mol + 1];
-    if (a_begin >= a_end) return;
     const int rows3n = 3 * n;
+    const size_t grow0 = row_offsets ? (size_t)row_offsets[mol] : (size_t)mol * rows3n;
+    const int rows = row_offsets ? row_offsets[mol + 1] - row_offsets[mol] : rows3n;
     const int row0 = blockIdx.z * (MROWS - 1);
-    const int nrows = min(MROWS - 1, rows3n - row0);
+    const bool with_energy = Ze != nullptr && blockIdx.z == 0;
+    if (row0 >= rows && !with_energy) return;
+    const int nrows = max(0, min(MROWS - 1, rows - row0));
+    int natoms = 0;
+    for (int e = 0; e < E.ne; ++e) natoms += E.seg[e][mol + 1] - E.seg[e][mol];
+    if (natoms == 0 && !overwrite) return;
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int l16 = lane & 15, lk = lane >> 4;
     const int f = blockIdx.x * 64 + wave * 16 + l16;
     const bool fok = f < F;
-
-    // B fragments of this wavefront's 16 columns, all of K, resident for the whole molecule
-    double wreg[KS];
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk) wreg[kk] = fok ? W[(size_t)(kk * 4 + lk) * F + f] : 0.0;
-    const double bf = fok ? b[f] : 0.0;
     const double norm = sqrt(2.0 / (double)F);
+    double zacc = 0.0;
 
-    double4_t gacc[4];
+    auto body = [&](auto nbc) {
+        constexpr int NB = decltype(nbc)::value;           // 16-row blocks; the x row is the last of them
+        constexpr int V4 = (NB * 16 * D / 4 + 255) / 256;  // float4 loads per thread per tile
+        double4_t gacc[NB];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) gacc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
+        for (int p = 0; p < NB; ++p) gacc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
+        float4 stage[V4];
+        auto fetch = [&](int e, int a) {
+            const float* ge = E.grad[e] + ((size_t)a * rows3n + row0) * D;
+            const float* xe = E.x[e] + (size_t)a * D;
+#pragma unroll
+            for (int v = 0; v < V4; ++v) {
+                const int idx = v * 256 + threadIdx.x;
+                const int row = idx / (D / 4), c4 = idx % (D / 4);
+                float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (row < nrows)
+                    val = *reinterpret_cast<const float4*>(ge + (size_t)row * D + c4 * 4);
+                else if (row == NB * 16 - 1)
+                    val = *reinterpret_cast<const float4*>(xe + c4 * 4);
+                stage[v] = val;
+            }
+        };
+        // the molecule's atoms element by element; (e, a) is the atom whose rows are in flight
+        int e = 0, a = 0, aend = 0;
+        auto settle = [&]() {                               // the next element that has atoms, when this one is done
+            while (a >= aend && e < E.ne) {
+                ++e;
+                if (e < E.ne) {
+                    a = E.seg[e][mol];
+                    aend = E.seg[e][mol + 1];
+                }
+            }
+        };
+        e = -1;
+        settle();
+        if (e < E.ne) fetch(e, a);
+        int cur = -1;
+        TW wreg[KS];
+        double bf = 0.0;
+        for (int done = 0; done < natoms; ++done) {
+            const int el = e;
+            float* tile = tiles[done & 1];
+#pragma unroll
+            for (int v = 0; v < V4; ++v) {
+                const int idx = v * 256 + threadIdx.x;
+                const int row = idx / (D / 4), c4 = idx % (D / 4);
+                if (V4 * 256 == NB * 16 * D / 4 || row < NB * 16)
+                    *reinterpret_cast<float4*>(&tile[row * LD + c4 * 4]) = stage[v];
+            }
+            __syncthreads();
+            if (el != cur) {   // B fragments of this wavefront's 16 columns, all of K, resident for the element's atoms
+                const TW* We = static_cast<const TW*>(E.W[el]);
+#pragma unroll
+                for (int kk = 0; kk < KS; ++kk) wreg[kk] = fok ? We[(size_t)(kk * 4 + lk) * F + f] : (TW)0;
+                bf = fok ? (double)static_cast<const TW*>(E.b[el])[f] : 0.0;
+                cur = el;
+            }
+            ++a;
+            settle();
+            if (e < E.ne) fetch(e, a);   // in flight during the MFMAs
 
-    // tile element owned by this thread in load slot v: float4 number v*256 + tid
-    float4 stage[V4];
-    auto fetch = [&](int a) {
+            double4_t pacc[NB];
 #pragma unroll
-        for (int v = 0; v < V4; ++v) {
-            const int idx = v * 256 + threadIdx.x;
-            const int row = idx / (D / 4), c4 = idx % (D / 4);
-            float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (row < nrows)
-                val = *reinterpret_cast<const float4*>(grad + ((size_t)a * rows3n + row0 + row) * D + c4 * 4);
-            else if (row == MROWS - 1)
-                val = *reinterpret_cast<const float4*>(x + (size_t)a * D + c4 * 4);
-            stage[v] = val;
+            for (int p = 0; p < NB; ++p) pacc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int kk = 0; kk < KS; ++kk) {
+#pragma unroll
+                for (int p = 0; p < NB; ++p) {
+                    const double av = (double)tile[(p * 16 + l16) * LD + kk * 4 + lk];
+                    pacc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, (double)wreg[kk], pacc[p], 0, 0, 0);
+                }
+            }
+            // accumulator register r of a 16x16 block holds row lane/16 + 4r, column lane%16:
+            // the x row (the last of the tile) is register 3 of the last block in lanes 48..63
+            const double s0 = __shfl(pacc[NB - 1][3], 48 + l16, 64) + bf;
+            double sn, cs;
+            sincos(s0, &sn, &cs);
+            zacc += norm * cs;
+            const double fd = norm * sn;
+#pragma unroll
+            for (int p = 0; p < NB; ++p) gacc[p] += fd * pacc[p];
+        }
+        if (!fok) return;
+        if (with_energy && lk == 0) {
+            double* z = Ze + (size_t)mol * F + f;
+            *z = overwrite ? zacc : *z + zacc;
+        }
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = p * 16 + lk + 4 * r;
+                if (row < nrows) {
+                    double* dst = G + (grow0 + row0 + row) * F + f;
+                    *dst = overwrite ? gacc[p][r] : *dst + gacc[p][r];
+                }
+            }
         }
     };
-    fetch(a_begin);
-    for (int a = a_begin; a < a_end; ++a) {
-        __syncthreads();   // the previous atom's fragments have been read
-#pragma unroll
-        for (int v = 0; v < V4; ++v) {
-            const int idx = v * 256 + threadIdx.x;
-            const int row = idx / (D / 4), c4 = idx % (D / 4);
-            *reinterpret_cast<float4*>(&tile[row * LD + c4 * 4]) = stage[v];
-        }
-        __syncthreads();
-        if (a + 1 < a_end) fetch(a + 1);   // in flight during the MFMAs
+    switch ((nrows + 16) / 16) {
+        case 1: body(std::integral_constant<int, 1>{}); break;
+        case 2: body(std::integral_constant<int, 2>{}); break;
+        case 3: body(std::integral_constant<int, 3>{}); break;
+        default: body(std::integral_constant<int, 4>{}); break;
+    }
+}
 
-        double4_t pacc[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) pacc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const double av = (double)tile[(p * 16 + l16) * LD + kk * 4 + lk];
-                pacc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, wreg[kk], pacc[p], 0, 0, 0);
-            }
-        }
-        // accumulator register r of a 16x16 block holds row lane/16 + 4r, column lane%16:
-        // the x row (tile row 63) is register 3 of block 3 in lanes 48..63
-        const double s0 = __shfl(pacc[3][3], 48 + l16, 64);
-        const double fd = norm * sin(s0 + bf);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) gacc[p] += fd * pacc[p];
-    }
-    if (!fok) return;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = p * 16 + lk + 4 * r;
-            if (row < nrows) {
-                double* dst = G + ((size_t)mol * rows3n + row0 + row) * F + f;
-                *dst += gacc[p][r];
-            }
-        }
-    }
+template <typename TW>
+void launch_rff_rows(const RffElements& E, const int* row_offsets, int max_rows, int n, int d, int F, int nmol, int overwrite,
+                     double* Ze, double* G, hipStream_t stream) {
+    const dim3 grid((F + 63) / 64, nmol, max_rows > 0 ? (max_rows + MROWS - 2) / (MROWS - 1) : 1);
+    if (d == 64)
+        hipLaunchKernelGGL((rff_rows_kernel<64, TW>), grid, dim3(256), 0, stream, E, row_offsets, n, F, overwrite, Ze, G);
+    else if (d == 128)
+        hipLaunchKernelGGL((rff_rows_kernel<128, TW>), grid, dim3(256), 0, stream, E, row_offsets, n, F, overwrite, Ze, G);
+    else
+        hipLaunchKernelGGL((rff_rows_kernel<256, TW>), grid, dim3(256), 0, stream, E, row_offsets, n, F, overwrite, Ze, G);
 }
 
 
@@ -613,19 +685,16 @@ extern "C" int qmll_rff_derivative_features(const float* x, const float* grad, c
     QMLL_REQUIRE(x && grad && W && b && (mol_index || seg_offsets) && G, QMLL_ERR_INVALID,
                  "qmll_rff_derivative_features: null pointer");
     if (seg_offsets && (d == 64 || d == 128 || d == 256)) {
-        const int rg = (3 * n + MROWS - 2) / (MROWS - 1);
-        QMLL_REQUIRE(nmol <= 65535 && rg <= 65535, QMLL_ERR_INVALID,
+        QMLL_REQUIRE(nmol <= 65535 && (3 * n + MROWS - 2) / (MROWS - 1) <= 65535, QMLL_ERR_INVALID,
                      "qmll_rff_derivative_features: grid too large (nmol=%d n=%d)", nmol, n);
-        dim3 grid((F + 63) / 64, nmol, rg);
-        if (d == 64)
-            hipLaunchKernelGGL(rff_derivative_mfma_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, x, grad, W, b,
-                               seg_offsets, n, F, G);
-        else if (d == 128)
-            hipLaunchKernelGGL(rff_derivative_mfma_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, x, grad, W, b,
-                               seg_offsets, n, F, G);
-        else
-            hipLaunchKernelGGL(rff_derivative_mfma_kernel<256>, grid, dim3(256), 0, (hipStream_t)stream, x, grad, W, b,
-                               seg_offsets, n, F, G);
+        RffElements E = {};
+        E.ne = 1;
+        E.x[0] = x;
+        E.grad[0] = grad;
+        E.W[0] = W;
+        E.b[0] = b;
+        E.seg[0] = seg_offsets;
+        launch_rff_rows<double>(E, nullptr, 3 * n, n, d, F, nmol, 0, nullptr, G, (hipStream_t)stream);
         QMLL_CHECK_LAUNCH("qmll_rff_derivative_features");
         return QMLL_OK;
     }
@@ -640,6 +709,32 @@ extern "C" int qmll_rff_derivative_features(const float* x, const float* grad, c
     hipLaunchKernelGGL(rff_derivative_kernel, grid, dim3(RT), lds, (hipStream_t)stream, x, grad, W, b, mol_index, n, d, F,
                        nmol, njc, G);
     QMLL_CHECK_LAUNCH("qmll_rff_derivative_features");
+    return QMLL_OK;
+}
+
+extern "C" int qmll_rff_rows(const qmll_rff_element* elements, int ne, const int* row_offsets, int max_rows, int n, int d, int F,
+                             int nmol, int overwrite, double* Ze, double* G, qmll_stream_t stream) {
+    QMLL_REQUIRE(n >= 0 && nmol >= 0 && ne >= 0 && F > 0 && max_rows >= 0 && max_rows <= 3 * (long long)n, QMLL_ERR_INVALID,
+                 "qmll_rff_rows: bad size n=%d nmol=%d ne=%d F=%d max_rows=%d", n, nmol, ne, F, max_rows);
+    QMLL_REQUIRE(ne <= RFF_MAXE, QMLL_ERR_INVALID, "qmll_rff_rows: at most %d elements per call (got %d)", RFF_MAXE, ne);
+    QMLL_REQUIRE(d == 64 || d == 128 || d == 256, QMLL_ERR_INVALID, "qmll_rff_rows: d=%d is not 64, 128 or 256", d);
+    if (n == 0 || nmol == 0 || (ne == 0 && !overwrite)) return QMLL_OK;
+    QMLL_REQUIRE((G || max_rows == 0) && (elements || ne == 0), QMLL_ERR_INVALID, "qmll_rff_rows: null pointer");
+    QMLL_REQUIRE(nmol <= 65535 && (max_rows + MROWS - 2) / (MROWS - 1) <= 65535, QMLL_ERR_INVALID,
+                 "qmll_rff_rows: grid too large (nmol=%d n=%d)", nmol, n);
+    RffElements E = {};
+    E.ne = ne;
+    for (int e = 0; e < ne; ++e) {
+        QMLL_REQUIRE(elements[e].x && elements[e].grad && elements[e].W && elements[e].b && elements[e].seg_offsets,
+                     QMLL_ERR_INVALID, "qmll_rff_rows: null pointer in element %d", e);
+        E.x[e] = elements[e].x;
+        E.grad[e] = elements[e].grad;
+        E.W[e] = elements[e].W;
+        E.b[e] = elements[e].b;
+        E.seg[e] = elements[e].seg_offsets;
+    }
+    launch_rff_rows<float>(E, row_offsets, max_rows, n, d, F, nmol, overwrite, Ze, G, (hipStream_t)stream);
+    QMLL_CHECK_LAUNCH("qmll_rff_rows");
     return QMLL_OK;
 }
 

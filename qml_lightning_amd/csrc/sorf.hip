@@ -1209,8 +1209,8 @@ struct DfElements {
 
 template <int LOG2D>
 __global__ __launch_bounds__(DFT_THREADS) void derivative_features_typed_rows_kernel(
-    DfElements E, double normalisation, int n, int S, int T, float hscale, int nmol, int ngroups, int cap,
-    int overwrite, double* __restrict__ G) {
+    DfElements E, double normalisation, const int* __restrict__ row_offsets, int n, int S, int T, float hscale, int nmol,
+    int ngroups, int cap, int overwrite, double* __restrict__ G) {
     constexpr int d = 1 << LOG2D;
     constexpr int EPL = d / 16;
     constexpr int Q = EPL / 4;
@@ -1227,7 +1227,9 @@ __global__ __launch_bounds__(DFT_THREADS) void derivative_features_typed_rows_ke
     const int s = min(sb + L.row, S - 1);
     const size_t F = (size_t)S * d;
     const double scale = normalisation * (double)hscale;
-    const int nrows = 3 * n;
+    // rows of this molecule: all 3n, or as many as the caller's row table gives it
+    const int nrows = row_offsets ? row_offsets[mol + 1] - row_offsets[mol] : 3 * n;
+    const size_t grow0 = row_offsets ? (size_t)row_offsets[mol] : (size_t)mol * n * 3;
     const size_t rstride = (size_t)n * 3 * d;    // between the Jacobian rows of consecutive atoms
     int ntot = 0;
     for (int e = 0; e < E.ne; ++e) ntot += E.seg[e][mol + 1] - E.seg[e][mol];
@@ -1312,7 +1314,7 @@ __global__ __launch_bounds__(DFT_THREADS) void derivative_features_typed_rows_ke
             }
             const bool fresh = overwrite && c0 == 0;                       // G holds nothing yet
             if (live && (any || fresh)) {
-                double* g = G + (((size_t)mol * n) * 3 + jx) * F + (size_t)s * d + L.e0;
+                double* g = G + (grow0 + jx) * F + (size_t)s * d + L.e0;
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
                     double2* gq = reinterpret_cast<double2*>(g + q * 64);
@@ -1747,6 +1749,12 @@ extern "C" int qmll_derivative_features(const double* cos_derivs, double normali
 extern "C" int qmll_derivative_features_typed(const qmll_df_element* elements, int ne, double normalisation, int n,
                                               int d, int S, int T, int nmol, int overwrite, double* G,
                                               qmll_stream_t stream) {
+    return qmll_derivative_features_rows(elements, ne, normalisation, nullptr, n, d, S, T, nmol, overwrite, G, stream);
+}
+
+extern "C" int qmll_derivative_features_rows(const qmll_df_element* elements, int ne, double normalisation,
+                                             const int* row_offsets, int n, int d, int S, int T, int nmol, int overwrite,
+                                             double* G, qmll_stream_t stream) {
     int rc = check_sorf("qmll_derivative_features_typed", 0, d, S, T);
     if (rc) return rc;
     QMLL_REQUIRE(n >= 0 && nmol >= 0 && ne >= 0, QMLL_ERR_INVALID,
@@ -1786,7 +1794,7 @@ extern "C" int qmll_derivative_features_typed(const qmll_df_element* elements, i
     const size_t lds = (size_t)cap * per_atom;
 #define CALL(L)                                                                                                    \
     hipLaunchKernelGGL(derivative_features_typed_rows_kernel<L>, grid, dim3(DFT_THREADS), lds, (hipStream_t)stream, \
-                       E, normalisation, n, S, T, hscale, nmol, ngroups, cap, overwrite, G)
+                       E, normalisation, row_offsets, n, S, T, hscale, nmol, ngroups, cap, overwrite, G)
     switch (qmll_log2(d)) {
         case 6: CALL(6); break;
         case 7: CALL(7); break;

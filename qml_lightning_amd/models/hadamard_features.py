@@ -394,7 +394,7 @@ class HadamardFeaturesModel(BaseKernel, torch.nn.Module):
                 # all elements go through ONE launch once the batch's loop over elements is done
                 # (finish_features): every element of the force-feature block is then read and
                 # written once instead of once per element and atom chunk
-                self._pending_derivative_features.append((cos_derivs, self.Dmat[element_idx], grad, indexes))
+                self._pending_derivative_features.append((cos_derivs, self.Dmat[element_idx], grad, self._queued_segments))
                 return
             # `indexes` comes from a molecule-major gather, so the atomic-free kernel applies
             ops.derivative_features(cos_derivs, coeff_normalisation, self.Dmat[element_idx], grad, indexes,
@@ -405,12 +405,16 @@ class HadamardFeaturesModel(BaseKernel, torch.nn.Module):
         return 64 <= self.npcas <= 256 and len(self.elements) <= 8
 
     @torch.jit.unused
-    def finish_features(self, derivative_features=None, overwrite=False):
+    def finish_features(self, derivative_features=None, overwrite=False, feature_matrix=None, rows=None):
         """Force-feature rows of the elements queued by calculate_features, in one launch."""
         pending, self._pending_derivative_features = self._pending_derivative_features, []
         if derivative_features is not None and (pending or overwrite):
-            ops.derivative_features_typed(pending, float(np.sqrt(self.npcas) / self.sigma), derivative_features,
-                                          overwrite=overwrite)
+            G = derivative_features.view(-1, self.nfeatures())
+            offsets = rows['offsets']
+            if offsets is None:
+                offsets = 3 * rows['n'] * torch.arange(rows['B'] + 1, dtype=torch.int32, device=G.device)
+            ops.derivative_features_typed(pending, float(np.sqrt(self.npcas) / self.sigma), G, overwrite=overwrite,
+                                          nmol=rows['B'], n=rows['n'], row_offsets=offsets)
 
     def forward(self, X, Z, atomIDs, molIDs, atom_counts, cell: Optional[torch.Tensor] = None,
                 inv_cell: Optional[torch.Tensor] = None):

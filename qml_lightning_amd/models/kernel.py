@@ -84,11 +84,12 @@ class BaseKernel():
         self.sigma = sigma
         self.llambda = llambda
         self._queue_force_rows = False
+        self._queued_segments = None
 
     # -- to be provided by the feature model -------------------------------------------
-    def finish_features(self, derivative_matrix=None, overwrite=False):
+    def finish_features(self, derivative_matrix=None, overwrite=False, feature_matrix=None, rows=None):
         """Called once per batch after the loop over elements; models that queue work in
-        calculate_features run it here."""
+        calculate_features run it here.  rows: the batch's row table (`_drop_rigid_rows`), or None."""
         return None
 
     def writes_force_rows(self):
@@ -160,20 +161,52 @@ class BaseKernel():
                 g_all = ops.project_typed_rows(rep_derivative.view(B * n * n * 3, -1), slots, type_offsets,
                                                self.reductors, 3 * n)
             mol_of_atom = torch.div(slots, n, rounding_mode='floor')
+            segments = ops.typed_segments(slots, type_offsets, B, n) if with_forces else None
             for t in range(ne):
                 if counts[t] == 0:
                     continue
                 o0, o1 = int(offsets[t]), int(offsets[t + 1])
                 sub_grad = g_all[o0 * 3 * n:o1 * 3 * n].view(o1 - o0, n, 3, -1) if with_forces else None
-                items.append((order[t], mol_of_atom[o0:o1], x_all[o0:o1], sub_grad))
+                items.append((order[t], mol_of_atom[o0:o1], x_all[o0:o1], sub_grad,
+                              segments[t] if with_forces else None))
+            if with_forces:
+                return {'B': B, 'n': n, 'device': coordinates.device, 'items': items, 'slots': slots,
+                        'gradient_rows': g_all.view(-1, n, 3, self.reductors.shape[2])}
         return {'B': B, 'n': n, 'device': coordinates.device, 'items': items}
+
+    def _training_batch(self, data, has_E, has_F):
+        """(projected rows, targets) of a formatted training batch.  With forces, the rows of padded slots and
+        the combinations of a molecule's force rows that vanish identically (its translations, and without
+        cells its rotations) are left out of both: an orthogonal transformation of each molecule's rows
+        and targets, which leaves Z^T Z and Z^T y as they are, and up to half of the rows less."""
+        proj = self._batch_projected(data, has_F)
+        B = data['charges'].shape[0]
+        modes = data.get('rigid_modes')
+        if not has_F or modes is None or not self.writes_force_rows() or 'gradient_rows' not in proj:
+            return proj, self._targets(data, B, has_E, has_F)
+        counts, modes = modes
+        per_molecule = (3 * counts - modes).astype(np.int32)
+        table = np.concatenate((modes, [0], np.cumsum(per_molecule))).astype(np.int32)
+        dev = proj['device']
+        table = torch.from_numpy(table).to(dev)
+        nrows = int(per_molecule.sum())
+        targets = torch.empty((B + nrows, 1), dtype=torch.float64, device=dev)
+        if has_E:
+            targets[:B, 0] = data['energies']
+        else:
+            targets[:B].zero_()
+        ops.rigid_rows(proj.pop('gradient_rows'), proj.pop('slots'), data['coordinates'], data['natom_counts'], table[:B],
+                       table[B:], data['forces'].contiguous(), targets[B:])
+        proj['rows'] = {'offsets': table[B:], 'count': nrows, 'most': int(per_molecule.max()) if B else 0}
+        return proj, targets
 
     def _rows_from_projected(self, proj, with_forces, zero_energy_rows=False):
         """fp64 row matrix [B (+ B*n*3), F] from the projected rows of one batch, at the current
         sigma: B energy rows, then the B*n*3 force rows in (molecule, atom, xyz) order
         (kernel.py:134-170)."""
         B, n, F = proj['B'], proj['n'], self.nfeatures()
-        nrows = B + (B * n * 3 if with_forces else 0)
+        table = proj.get('rows') if with_forces else None      # fewer force rows than B*n*3: see _training_batch
+        nrows = B + (table['count'] if table else B * n * 3 if with_forces else 0)
         own_force_rows = with_forces and self.writes_force_rows()
         if own_force_rows:
             rows = torch.empty(nrows, F, device=proj['device'], dtype=torch.float64)
@@ -181,12 +214,18 @@ class BaseKernel():
         else:
             rows = torch.zeros(nrows, F, device=proj['device'], dtype=torch.float64)
         Zenergy = rows[:B]
-        G = rows[B:].view(B, n, 3, F) if with_forces else None
+        G = None
+        if with_forces:
+            G = rows[B:] if table else rows[B:].view(B, n, 3, F)
         self._queue_force_rows = own_force_rows     # calculate_features may queue; finish_features runs the queue
-        for e, batch_indexes, sub, sub_grad in proj['items']:
+        for e, batch_indexes, sub, sub_grad, segments in proj['items']:
+            self._queued_segments = segments
             self.calculate_features(sub, e, batch_indexes, Zenergy, sub_grad if with_forces else None, G)
         self._queue_force_rows = False
-        self.finish_features(G, overwrite=own_force_rows)
+        self._queued_segments = None
+        if with_forces:
+            rtable = {'B': B, 'n': n, 'offsets': table['offsets'] if table else None, 'most': table['most'] if table else 3 * n}
+            self.finish_features(G, overwrite=own_force_rows, feature_matrix=Zenergy, rows=rtable)
         if zero_energy_rows:
             Zenergy.fill_(0)        # energy rows stay, as zeros, so the row count is unchanged (kernel.py:164-165)
         return rows
@@ -248,9 +287,9 @@ class BaseKernel():
                                         F=F[sl] if F is not None else None,
                                         cells=cells[sl] if cells is not None else None,
                                         inv_cells=inv_cells[sl] if cells is not None else None)
-                zbatch = data['charges'].shape[0]
-                targets = self._targets(data, zbatch, E is not None, F is not None)
-                rows = self._batch_rows(data, F is not None, zero_energy_rows=E is None)
+                proj, targets = self._training_batch(data, E is not None, F is not None)
+                rows = self._rows_from_projected(proj, F is not None, zero_energy_rows=E is None)
+                del proj
                 if ntiles > 1:
                     if use_specialized_matmul:
                         matmul_and_reduce(rows[:, lo:hi].float().T.contiguous(), rows.float(), ZTZ_tile)
@@ -454,8 +493,7 @@ class BaseKernel():
                                         F=F[sl] if F is not None else None,
                                         cells=cells[sl] if cells is not None else None,
                                         inv_cells=inv_cells[sl] if cells is not None else None)
-                targets = self._targets(data, data['charges'].shape[0], E is not None, F is not None)
-                out.append((self._batch_projected(data, F is not None), targets))
+                out.append(self._training_batch(data, E is not None, F is not None))
         except torch.cuda.OutOfMemoryError:
             del out
             torch.cuda.empty_cache()
@@ -676,10 +714,33 @@ class BaseKernel():
             if self.convert_hartree2kcal():
                 forces = forces * self.hartree2kcalmol
             data['forces'] = forces * mask[:, :, None]                      # padded slots carry no target
+            data['rigid_modes'] = self._rigid_modes(np.asarray(X), hostmask.sum(axis=1), cells is not None)
         if cells is not None:
             data['cells'] = torch.from_numpy(np.asarray(cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
             data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
         return data
+
+    @staticmethod
+    def _rigid_modes(coordinates, counts, periodic):
+        """(counts, modes) int32 [B]: how many independent translations and rotations each molecule of a
+        zero-padded host batch has: 3 in a periodic cell, else 6; 5 for two atoms, 3 for one.  A molecule of
+        three or more atoms on a line (mean square distance from the line below 1e-3 of that from the centre)
+        keeps all of its rows (0): its third rotation is undefined, and the angular terms' derivatives are
+        singular there."""
+        counts = np.asarray(counts, dtype=np.int32)
+        modes = np.where(counts > 0, 3, 0).astype(np.int32)
+        if periodic or coordinates.shape[1] < 2:
+            return counts, modes
+        X = coordinates.astype(np.float32, copy=False)
+        live = (np.arange(X.shape[1]) < counts[:, None])[:, :, None]
+        d = np.where(live, X - (X * live).sum(axis=1, keepdims=True) / np.maximum(counts, 1)[:, None, None], 0.0)
+        T = np.matmul(d.transpose(0, 2, 1), d).astype(np.float64)
+        trace = T[:, 0, 0] + T[:, 1, 1] + T[:, 2, 2]
+        # sum of the principal 2 x 2 minors = l1 l2 + l1 l3 + l2 l3, about trace (l2 + l3) for a line
+        minors = 0.5 * (trace * trace - (T * T).sum(axis=(1, 2)))
+        modes[counts == 2] = 5
+        modes[counts >= 3] = np.where(minors > 1e-3 * trace * trace, 6, 0)[counts >= 3]
+        return counts, modes
 
     def _element_counts(self, flat_charges):
         """{element: number of atoms} of a batch from the host copy of its charges (one bincount)."""
@@ -769,6 +830,7 @@ class BaseKernel():
             if self.convert_hartree2kcal():
                 forces *= self.hartree2kcalmol
             data['forces'] = torch.from_numpy(forces).to(dev)
+            data['rigid_modes'] = self._rigid_modes(coords, counts, cells is not None)
         if cells is not None:
             data['cells'] = torch.from_numpy(np.asarray(cells, dtype=np.float32).reshape(zbatch, 3, 3)).to(dev)
             data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(zbatch, 3, 3)).to(dev)

@@ -36,6 +36,7 @@ class RandomFourrierFeaturesModel(BaseKernel, torch.nn.Module):
                              "operator sequence of the reference" % (npcas, nstacks * npcas))
         self.fused = has_kernel if fused is None else bool(fused)
         self.separate_ops = separate_ops   # fused route as five operators (one node each) instead of one
+        self._pending_rows = []
         self.nbatch_train = nbatch_train
         self.nbatch_test = nbatch_test
         self._nfeatures = nstacks * self.npcas
@@ -63,12 +64,28 @@ class RandomFourrierFeaturesModel(BaseKernel, torch.nn.Module):
     @torch.jit.unused
     def calculate_features(self, rep, element, indexes, feature_matrix, grad=None, derivative_matrix=None):
         """fp64 features / force features of one element (random_features.py:60-67)."""
-        idx = self.element2index[int(element)]
+        idx = int(self.element2index[int(element)])
+        if derivative_matrix is not None and grad is not None and self._queue_force_rows:
+            # energy and force rows of all elements go through ONE launch at the end of the batch (finish_features)
+            self._pending_rows.append((rep, grad, self.W[idx], self.b[idx], self._queued_segments))
+            return
         W, b = self.W[idx].double(), self.b[idx].double()
         get_rff(rep, W, b, indexes, feature_matrix)
         if derivative_matrix is not None and grad is not None:
             # the batch's atoms are molecule-major: atomic-free matrix-core kernel
             ops.rff_derivative_features(rep, grad, W, b, indexes, derivative_matrix, molecule_major=True)
+
+    @torch.jit.unused
+    def writes_force_rows(self):
+        return self.npcas in (64, 128, 256) and len(self.elements) <= 8
+
+    @torch.jit.unused
+    def finish_features(self, derivative_matrix=None, overwrite=False, feature_matrix=None, rows=None):
+        """Energy and force rows of the elements queued by calculate_features, in one launch."""
+        pending, self._pending_rows = self._pending_rows, []
+        if derivative_matrix is not None and (pending or overwrite):
+            ops.rff_rows(pending, feature_matrix, derivative_matrix.view(-1, self.nfeatures()), rows['B'], rows['n'],
+                         row_offsets=rows['offsets'], max_rows=rows['most'], overwrite=overwrite)
 
     def forward(self, X, Z, atomIDs, molIDs, atom_counts, cell: Optional[torch.Tensor] = None,
                 inv_cell: Optional[torch.Tensor] = None):

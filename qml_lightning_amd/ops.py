@@ -322,20 +322,66 @@ def derivative_features(cos_derivs, normalisation, D, input_derivatives, mol_ind
     return G
 
 
-def derivative_features_typed(items, normalisation, G, overwrite=False):
+def typed_segments(sorted_slots, type_offsets, B, n):
+    """int32 [ne, B+1]: first atom of every molecule within each element's part of the element-sorted slots,
+    relative to the element's first atom."""
+    sorted_slots, type_offsets = _i32(sorted_slots), _i32(type_offsets)
+    ne = int(type_offsets.shape[0]) - 1
+    seg = torch.empty((ne, int(B) + 1), dtype=torch.int32, device=sorted_slots.device)
+    check(_lib.lib().qmll_typed_segments(_ptr(sorted_slots), _ptr(type_offsets), ne, int(B), int(n), _ptr(seg), _stream()),
+          "qmll_typed_segments")
+    return seg
+
+
+def rigid_rows(grad, sorted_slots, X, natoms, modes, row_offsets, forces=None, targets=None):
+    """The projected Jacobian rows grad f32 [A,n,3,d] with Q^T applied in place, Q the orthogonal
+    transformation that maps modes[m] vanishing combinations (translations, rotations) of molecule m's
+    3 natoms[m] force rows onto its first rows; the rows that remain move to the front of each atom's block.
+    forces f64 [B,n,3] -> targets f64 [row_offsets[B]] = the same rows of Q^T y."""
+    A, n, _, d = grad.shape
+    B = int(natoms.shape[0])
+    if grad.dtype != torch.float32 or not grad.is_contiguous() or int(sorted_slots.shape[0]) != A:
+        raise RuntimeError("rigid_rows: grad %s for %d atoms" % (tuple(grad.shape), int(sorted_slots.shape[0])))
+    if (forces is None) != (targets is None):
+        raise RuntimeError("rigid_rows: forces and targets must both be given or both be None")
+    X, natoms, modes, row_offsets, sorted_slots = _f32(X), _i32(natoms), _i32(modes), _i32(row_offsets), _i32(sorted_slots)
+    if tuple(X.shape) != (B, n, 3) or modes.numel() != B or row_offsets.numel() != B + 1:
+        raise RuntimeError("rigid_rows: coordinates %s, %d modes, %d row offsets for %d molecules"
+                           % (tuple(X.shape), modes.numel(), row_offsets.numel(), B))
+    if forces is not None and (forces.dtype != torch.float64 or not forces.is_contiguous() or forces.numel() != B * n * 3
+                               or targets.dtype != torch.float64 or not targets.is_contiguous()):
+        raise RuntimeError("rigid_rows: forces and targets must be contiguous float64 tensors")
+    L = _lib.lib()
+    nbytes = int(L.qmll_rigid_workspace_bytes(B, n))
+    work = torch.empty(max(nbytes // 8, 1), dtype=torch.float64, device=grad.device)
+    check(L.qmll_rigid_modes(_ptr(X), _ptr(natoms), _ptr(modes), _ptr(row_offsets), B, n, _ptr(work), nbytes, _ptr(forces),
+                             _ptr(targets), _stream()), "qmll_rigid_modes")
+    check(L.qmll_rigid_rows(_ptr(grad), _ptr(sorted_slots), _ptr(natoms), _ptr(modes), _ptr(work), A, B, n, d, _stream()),
+          "qmll_rigid_rows")
+    return grad
+
+
+def derivative_features_typed(items, normalisation, G, overwrite=False, nmol=None, n=None, row_offsets=None):
     """G += force-feature rows of every element of the batch in one launch.  items: one tuple
     (cos_derivs f64 [A_e,F], D f32 [T,S,d], input_derivatives f32 [A_e,n,3,d], mol_index i32 [A_e],
     non-decreasing) per element.  Each G element is read and written once, instead of once per
     element and atom chunk as with `derivative_features`; with overwrite, G = those rows and is
-    only written (it may come from torch.empty).  64 <= d <= 256, at most 8 elements."""
-    if not items:
+    only written (it may come from torch.empty).  64 <= d <= 256, at most 8 elements.
+
+    With a row table (row_offsets i32 [nmol+1], and nmol, n) G is [row_offsets[nmol], S*d]: molecule m has the
+    first row_offsets[m+1] - row_offsets[m] of its 3n rows.  In place of mol_index an item may hold the element's
+    segment table i32 [nmol+1] (`typed_segments`)."""
+    if not items or G.numel() == 0:
         return G.zero_() if overwrite else G
     if G.dtype != torch.float64 or not G.is_contiguous():
         raise RuntimeError("derivative features need a contiguous float64 output")
-    nmol, n = int(G.shape[0]), int(G.shape[1])
+    if row_offsets is None:
+        nmol, n = int(G.shape[0]), int(G.shape[1])
+    else:
+        row_offsets = _i32(row_offsets)
     keep, structs = [], (_lib.DfElement * len(items))()
     T = S = d = None
-    bounds = torch.arange(nmol + 1, dtype=torch.int32, device=G.device)
+    bounds = None
     for k, (cos_derivs, D, u, mol_index) in enumerate(items):
         D, u, mol_index = _f32(D), _f32(u), _i32(mol_index)
         if cos_derivs.dtype != torch.float64 or not cos_derivs.is_contiguous():
@@ -344,17 +390,25 @@ def derivative_features_typed(items, normalisation, G, overwrite=False):
             T, S, d = (int(v) for v in D.shape)
         if tuple(D.shape) != (T, S, d) or tuple(u.shape[1:]) != (n, 3, d) or cos_derivs.shape != (u.shape[0], S * d):
             raise RuntimeError("derivative_features_typed: element %d does not fit [T,S,d] = %s, n = %d" % (k, (T, S, d), n))
-        seg = torch.searchsorted(mol_index, bounds).to(torch.int32)
+        if row_offsets is not None:
+            seg = mol_index
+            if seg.numel() != nmol + 1:
+                raise RuntimeError("derivative_features_typed: a segment table of %d entries for %d molecules"
+                                   % (seg.numel(), nmol))
+        else:
+            if bounds is None:
+                bounds = torch.arange(nmol + 1, dtype=torch.int32, device=G.device)
+            seg = torch.searchsorted(mol_index, bounds).to(torch.int32)
         keep.append((cos_derivs, D, u, seg))
         structs[k].cos_derivs = cos_derivs.data_ptr()
         structs[k].input_derivative = u.data_ptr()
         structs[k].D = D.data_ptr()
         structs[k].seg_offsets = seg.data_ptr()
-    if G.shape[3] != S * d:
+    if G.shape[-1] != S * d or G.dim() != (4 if row_offsets is None else 2):
         raise RuntimeError("feature_derivatives has shape %s, expected [nmol,%d,3,%d]" % (tuple(G.shape), n, S * d))
-    check(_lib.lib().qmll_derivative_features_typed(structs, len(items), float(normalisation), n, d, S, T, nmol,
-                                                    int(bool(overwrite)), _ptr(G), _stream()),
-          "qmll_derivative_features_typed")
+    check(_lib.lib().qmll_derivative_features_rows(structs, len(items), float(normalisation), _ptr(row_offsets), n, d, S, T,
+                                                   nmol, int(bool(overwrite)), _ptr(G), _stream()),
+          "qmll_derivative_features_rows")
     return G
 
 
@@ -642,6 +696,34 @@ def rff_derivative_features(x, grad, W, b, mol_index, G, molecule_major=False):
         seg = torch.searchsorted(mol_index, bounds).to(torch.int32)
     check(_lib.lib().qmll_rff_derivative_features(_ptr(x), _ptr(grad), _ptr(W), _ptr(b), _ptr(mol_index), _ptr(seg), A, n,
                                                   d, F, nmol, _ptr(G), _stream()), "qmll_rff_derivative_features")
+    return G
+
+
+def rff_rows(items, Ze, G, nmol, n, row_offsets=None, max_rows=None, overwrite=False):
+    """Energy features Ze f64 [nmol,F] (or None) and force rows G of every element of the batch in one launch, added or
+    (overwrite) written.  items: one tuple (x f32 [A_e,d], grad f32 [A_e,n,3,d], W f32 [d,F], b f32 [F], segment table
+    i32 [nmol+1]) per element, atoms molecule-major; row_offsets as for `derivative_features_typed`, max_rows the
+    largest number of rows of a molecule (3n without a table).  d in 64 / 128 / 256, at most 8 elements."""
+    F, d = int(G.shape[-1]), None
+    keep, structs = [], (_lib.RffElement * max(len(items), 1))()
+    for t in (Ze, G):
+        if t is not None and (t.dtype != torch.float64 or not t.is_contiguous() or t.shape[-1] != F):
+            raise RuntimeError("rff_rows needs contiguous float64 outputs with %d columns" % F)
+    for k, (x, grad, W, b, seg) in enumerate(items):
+        x, grad, W, b, seg = _f32(x), _f32(grad), _f32(W), _f32(b), _i32(seg)
+        d = int(W.shape[0]) if d is None else d
+        if (tuple(W.shape) != (d, F) or b.numel() != F or x.shape[1] != d or tuple(grad.shape) != (x.shape[0], n, 3, d)
+                or seg.numel() != nmol + 1):
+            raise RuntimeError("rff_rows: element %d: x %s, grad %s, W %s, b with %d entries, %d segments do not fit together"
+                               % (k, tuple(x.shape), tuple(grad.shape), tuple(W.shape), b.numel(), seg.numel()))
+        keep.append((x, grad, W, b, seg))
+        for name, t in (("x", x), ("grad", grad), ("W", W), ("b", b), ("seg_offsets", seg)):
+            setattr(structs[k], name, t.data_ptr())
+    if row_offsets is not None:
+        row_offsets = _i32(row_offsets)
+    check(_lib.lib().qmll_rff_rows(structs, len(items), _ptr(row_offsets), 3 * n if max_rows is None else int(max_rows), n,
+                                   64 if d is None else d, F, nmol, int(bool(overwrite)), _ptr(Ze), _ptr(G), _stream()),
+          "qmll_rff_rows")
     return G
 
 

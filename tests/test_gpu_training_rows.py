@@ -1,0 +1,70 @@
+"""Training rows without the combinations that vanish (translations, rotations, padded slots): Z^T Z and Z^T y equal
+those of the full rows, which other tests pin to the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from tests import helpers
+from tests.test_gpu_kernels import close, dev
+from tests.test_gpu_model import build_rff_model, build_sorf_model
+
+pytestmark = pytest.mark.gpu
+
+
+def molecules(sizes, seed):
+    """One molecule per size; a negative size -k is k atoms on a line."""
+    rng = np.random.default_rng(seed)
+    X, Q = [], []
+    for k in sizes:
+        if k < 0:
+            axis = rng.normal(size=3)
+            x = np.arange(-k)[:, None] * 1.2 * axis / np.linalg.norm(axis)
+        else:
+            x = helpers.random_geometry(rng, k, 1.7 * k ** (1 / 3) + 1.0, 0.95)
+        X.append(x.astype(np.float32))
+        Q.append(np.array(([6, 1, 8, 1, 1] * 20)[:abs(k)]))
+    return X, Q, rng
+
+
+@pytest.mark.parametrize("kind", ["sorf", "rff"])
+@pytest.mark.parametrize("npcas", [64, 128])
+@pytest.mark.parametrize("sizes,periodic", [((1, 2, -3, 3, 5), False), ((22, 23, 24, 7), False), ((29, -4, 1), False),
+                                            ((9, 9, 9), False), ((11, 1, 6), True)])
+def test_rows_left_out_change_nothing(kind, npcas, sizes, periodic):
+    species = [1, 6, 8]
+    X, Q, rng = molecules(sizes, 4)
+    m = (build_sorf_model(species, npcas, 3) if kind == "sorf" else build_rff_model(species, npcas, 1))
+    m = m[0] if isinstance(m, tuple) else m
+    E, F = rng.normal(size=len(X)), [rng.normal(size=(len(q), 3)) for q in Q]
+    kw = {}
+    if periodic:
+        cells = np.broadcast_to(np.eye(3) * 7.0, (len(X), 3, 3)).copy()
+        kw = {"cells": cells, "inv_cells": np.linalg.inv(cells)}
+    data = m.format_data(X, Q, E=E, F=F, **kw)
+    full, y = m._batch_rows(data, True), m._targets(data, len(X), True, True)
+    proj, targets = m._training_batch(data, True, True)
+    rows = m._rows_from_projected(proj, True)
+    left_out = [3 if periodic or k == 1 else 5 if k == 2 else 6 if k > 0 else 0 for k in sizes]   # a line keeps its rows
+    assert rows.shape[0] == len(X) + sum(3 * abs(k) - o for k, o in zip(sizes, left_out))
+    close(rows.T @ rows, (full.T @ full).cpu().numpy(), 1e-6, "Z^T Z")
+    close(rows.T @ targets, (full.T @ y).cpu().numpy(), 2e-6, "Z^T y")
+    # the norm of the targets is what Q leaves of them: no more than before, and the energies as they were
+    assert float(targets.norm()) <= float(y.norm()) * (1 + 1e-12)
+    assert torch.equal(targets[:len(X)], y[:len(X)])
+    # forces alone: the energy rows stay as zeros
+    m.nbatch_train = 3
+    ztz, zty = m.build_Z_components(X, Q, E=None, F=F, print_info=False, **kw)
+    G, yf = full[len(X):], y[len(X):]
+    close(ztz, (G.T @ G).cpu().numpy(), 1e-6, "G^T G")
+    close(zty, (G.T @ yf).cpu().numpy(), 2e-6, "G^T y")
+
+
+def test_rigid_rows_rejects_what_does_not_fit():
+    from qml_lightning_amd import ops
+    g = torch.zeros(2, 2, 3, 64, device=dev())
+    i = torch.zeros(2, dtype=torch.int32, device=dev())
+    with pytest.raises(RuntimeError):
+        ops.rigid_rows(g, i, torch.zeros(1, 3, 3, device=dev()), i[:1], i[:1], i)
+    with pytest.raises(RuntimeError):
+        ops.rigid_rows(g, i, torch.zeros(1, 2, 3, device=dev()), i[:1], i[:1], i,
+                       forces=torch.zeros(1, 2, 3, device=dev(), dtype=torch.float64))
