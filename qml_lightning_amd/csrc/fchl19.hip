@@ -20,6 +20,7 @@
 // da/dR_i = u_ij, da/dR_j = -u_ij, db/dR_i = u_ik, db/dR_k = -u_ik, dc/dR_j = u_jk,
 // dc/dR_k = -u_jk.  This is algebraically the reference's 40-term expansion; the
 // degenerate-angle guard sqrt(max(1e-10, a^2 b^2 - (d_ij.d_ik)^2)) is kept.
+#include <algorithm>
 #include <type_traits>
 
 #include "qmll_common.h"
@@ -59,8 +60,8 @@ struct FchlArgs {
     float gscale;  // the backward kernel returns gscale * J^T g (folded into the staged gradient row)
 };
 
-constexpr int TCH = 256;      // smallest triple table
-constexpr int TCH_MAX = 1024; // largest (16 KB): beyond, element pairs are processed in chunks
+constexpr int TCH_MAX = 1024;  // largest triple table of the one-wavefront forward kernel (16 KB)
+constexpr int TCH_WIDE = 768;  // largest of the several-wavefront one (12 KB): beyond, the triple list is taken in chunks
 constexpr float PI_F = 3.14159265358979323846f;
 // three floats read from a 16-byte-aligned LDS entry with a single 12-byte instruction (a 16-byte
 // read of the same entry occupies the LDS pipe a third longer)
@@ -244,6 +245,61 @@ __device__ __forceinline__ int visit_neighbours(const FchlArgs& a, int* goff, in
     return nn;
 }
 
+// visit_neighbours for a workgroup of NW wavefronts.  Up to 64 candidates every wavefront does the same single pass
+// (equal values go to the same LDS words).  Beyond, each wavefront takes 64 candidates of its own, all loads in
+// flight at once, and the places follow from a scan over the (type, wavefront) counts; wcount: NW * nspecies ints of LDS.
+// More than 64 NW candidates, or more than 64 / NW types: the two passes of visit_neighbours on every wavefront.
+// The caller has a barrier before it reads the list.
+template <int NW, class Emit>
+__device__ __forceinline__ int visit_neighbours_wide(const FchlArgs& a, int* goff, int* wcount, int m, int i, int tid, Emit emit) {
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ns = a.p.nspecies;
+    const bool have_list = a.nlist != nullptr;
+    int total;
+    if (have_list) total = min(a.nneigh[(size_t)m * a.n + i], a.nn_stride);
+    else total = min(a.natoms[m], a.n);
+    if (total <= QMLL_WAVE || total > QMLL_WAVE * NW || ns * NW > QMLL_WAVE) return visit_neighbours(a, goff, m, i, lane, emit);
+    const float* Xm = a.X + (size_t)m * a.n * 3;
+    const int* tm = a.types + (size_t)m * a.n;
+    int j = tid;
+    bool ok = tid < total;
+    if (have_list) j = ok ? a.nlist[((size_t)m * a.n + i) * a.nn_stride + tid] : 0;
+    ok = ok && j >= 0 && j < a.n;
+    const int jj = ok ? j : 0;
+    float dx = Xm[i * 3 + 0] - Xm[jj * 3 + 0], dy = Xm[i * 3 + 1] - Xm[jj * 3 + 1], dz = Xm[i * 3 + 2] - Xm[jj * 3 + 2];
+    const int e = tm[jj];
+    if (a.cell != nullptr) min_image(dx, dy, dz, a.cell + (size_t)m * 9, a.inv_cell + (size_t)m * 9);
+    const float r2 = dx * dx + dy * dy + dz * dz;
+    ok = ok && (have_list ? r2 > 0.0f : (r2 < a.p.rcut * a.p.rcut && r2 > 0.0f)) && e >= 0 && e < ns;
+    int before = 0;                                     // earlier lanes of this wavefront with the same type
+    for (int ep = 0; ep < ns; ++ep) {
+        const unsigned long long mask = __ballot(ok && e == ep);
+        if (e == ep) before = __popcll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0) wcount[ep * NW + wave] = __popcll(mask);
+    }
+    __syncthreads();
+    // exclusive scan over the counts, on every wavefront
+    const int c = lane < ns * NW ? wcount[lane] : 0;
+    int incl = c;
+    for (int o = 1; o < ns * NW; o <<= 1) {
+        const int up = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += up;
+    }
+    const int excl = incl - c;
+    const int nn = min(__shfl(incl, ns * NW - 1, 64), a.cap);
+    const int es = ok ? e : 0;
+    const int first = __shfl(excl, es * NW, 64);                       // of the type
+    const int last = __shfl(incl, es * NW + NW - 1, 64);
+    const int pos = __shfl(excl, es * NW + wave, 64) + before;
+    if (wave == 0) {
+        const int g = __shfl(excl, min(lane * NW, 63), 64);
+        if (lane < ns) goff[lane] = g;
+        if (lane == 0) goff[ns] = nn;
+    }
+    if (ok && pos < a.cap) emit(pos, pos - first, last - first, e, j, dx, dy, dz, r2);
+    return nn;
+}
+
 // the cosine cutoff fc = (cos(pi r / rc) + 1) / 2 and its r-derivative from one sine / cosine pair
 __device__ __forceinline__ void cutoff(float r, float inv_rc, float& fc, float& dfc) {
     float sn, cs;
@@ -338,6 +394,46 @@ __device__ __forceinline__ Triple triple_geometry(const Stage& s, int j, int k) 
     return t;
 }
 
+// what the forward kernels keep of a neighbour, written by the lane that found it: d_ij and 1 / r; sk3 r / 2, fc r^-d3,
+// element type, index within the type | neighbours of the type << 16; mu_j, log2(e) / (2 sigma_j^2),
+// r^-d2 fc / (sigma sqrt(2 pi))
+__device__ __forceinline__ void forward_records(const qmll_fchl_params& p, float sk3, float inv_rc, float* recA, float* recB,
+                                                float* s2b, int pos, int rank, int count, int e, float dx, float dy, float dz,
+                                                float r2) {
+    const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+    float fc, dfc;
+    cutoff(r, inv_rc, fc, dfc);
+    const float l2r = flog2(r);
+    const float s2 = flog(fmaf(p.eta2 * ir, ir, 1.0f));
+    reinterpret_cast<float4*>(s2b)[pos] = make_float4(
+        fmaf(l2r, 0.6931471805599453f, -0.5f * s2),   // ln(r / sqrt(1 + eta2/r^2))
+        0.5f * LOG2E * frcp(s2),
+        frsq(s2) * 0.3989422804014327f * fexp2(-p.two_body_decay * l2r) * fc, 0.0f);
+    reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, ir);
+    reinterpret_cast<float4*>(recB)[pos] = make_float4(sk3 * 0.5f * r, fc * fexp2(-p.three_body_decay * l2r),
+                                                       __int_as_float(e), __int_as_float(rank | (count << 16)));
+}
+
+// one table entry per triple: (sk3 rho, K cos, K sin, -) from the two neighbours' records.  With
+// a = d_ij, b = d_ik, c = b - a: cos_i cos_j cos_k = -(a.b)(a.c)(c.b) / (|a| |b| |c|)^2, the decay
+// (|a| |b| |c|)^-d3 is the product of the neighbours' factors and |c|^-d3 = exp2(-d3 log2(c.c) / 2);
+// sin_i = |a x b| / (|a| |b|) keeps full relative accuracy near collinear triples.
+__device__ __forceinline__ float4 table_entry(float zw3, float hd3, const float4 Aj, const float4 Bj, const float4 Ak,
+                                              const float4 Bk) {
+    const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
+    const float c2 = cx * cx + cy * cy + cz * cz;
+    const float vi = Aj.x * Ak.x + Aj.y * Ak.y + Aj.z * Ak.z;
+    const float dac = Aj.x * cx + Aj.y * cy + Aj.z * cz;
+    const float dcb = cx * Ak.x + cy * Ak.y + cz * Ak.z;
+    const float w = Aj.w * Ak.w;
+    const float W = w * frsq(c2);
+    const float px = Aj.y * Ak.z - Aj.z * Ak.y, py = Aj.z * Ak.x - Aj.x * Ak.z, pz = Aj.x * Ak.y - Aj.y * Ak.x;
+    const float f = zw3 * fmaf(-3.0f * vi * dac, dcb * W * W, 1.0f) * Bj.y * Bk.y * fexp2(hd3 * flog2(c2));
+    const float cosT = fminf(1.0f, fmaxf(-1.0f, vi * w));
+    const float sinT = fminf(1.0f, fsqrt(px * px + py * py + pz * pz) * w);
+    return make_float4(Bj.x + Bk.x, f * cosT, f * sinT, 0.0f);
+}
+
 // ---------------------------------------------------------------------------------
 // forward
 //
@@ -387,18 +483,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
     // every neighbour's factors of the two-body bins and of the triples, by the lane that found it
     const int nn = visit_neighbours(
         a, goff, m, i, lane, [&](int pos, int rank, int count, int e, int, float dx, float dy, float dz, float r2) {
-            const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
-            float fc, dfc;
-            cutoff(r, inv_rc, fc, dfc);
-            const float l2r = flog2(r);
-            const float s2 = flog(fmaf(a.p.eta2 * ir, ir, 1.0f));
-            reinterpret_cast<float4*>(s2b)[pos] = make_float4(
-                fmaf(l2r, 0.6931471805599453f, -0.5f * s2),   // ln(r / sqrt(1 + eta2/r^2))
-                0.5f * LOG2E * frcp(s2),
-                frsq(s2) * 0.3989422804014327f * fexp2(-a.p.two_body_decay * l2r) * fc, 0.0f);
-            reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, ir);
-            reinterpret_cast<float4*>(recB)[pos] = make_float4(sk3 * 0.5f * r, fc * fexp2(-a.p.three_body_decay * l2r),
-                                                               __int_as_float(e), __int_as_float(rank | (count << 16)));
+            forward_records(a.p, sk3, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
         });
     if (lane < nRs2) {
         slnRs2[lane] = flog(rs2v);
@@ -453,25 +538,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
     const int tsub = idiv_small(lane, W3), ll = lane - tsub * W3;
     constexpr int MAXLB = 4;                     // radial bins handled: up to 4 x 64
 
-    // one table entry per triple: (sk3 rho, K cos, K sin, -) from the two neighbours' records.  With
-    // a = d_ij, b = d_ik, c = b - a: cos_i cos_j cos_k = -(a.b)(a.c)(c.b) / (|a| |b| |c|)^2, the decay
-    // (|a| |b| |c|)^-d3 is the product of the neighbours' factors and |c|^-d3 = exp2(-d3 log2(c.c) / 2);
-    // sin_i = |a x b| / (|a| |b|) keeps full relative accuracy near collinear triples.
     const float zw3 = zeta2 * a.p.three_body_weight, hd3 = -0.5f * a.p.three_body_decay;
-    auto table_entry = [&](const float4 Aj, const float4 Bj, const float4 Ak, const float4 Bk) -> float4 {
-        const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
-        const float c2 = cx * cx + cy * cy + cz * cz;
-        const float vi = Aj.x * Ak.x + Aj.y * Ak.y + Aj.z * Ak.z;
-        const float dac = Aj.x * cx + Aj.y * cy + Aj.z * cz;
-        const float dcb = cx * Ak.x + cy * Ak.y + cz * Ak.z;
-        const float w = Aj.w * Ak.w;
-        const float W = w * frsq(c2);
-        const float px = Aj.y * Ak.z - Aj.z * Ak.y, py = Aj.z * Ak.x - Aj.x * Ak.z, pz = Aj.x * Ak.y - Aj.y * Ak.x;
-        const float f = zw3 * fmaf(-3.0f * vi * dac, dcb * W * W, 1.0f) * Bj.y * Bk.y * fexp2(hd3 * flog2(c2));
-        const float cosT = fminf(1.0f, fmaxf(-1.0f, vi * w));
-        const float sinT = fminf(1.0f, fsqrt(px * px + py * py + pz * pz) * w);
-        return make_float4(Bj.x + Bk.x, f * cosT, f * sinT, 0.0f);
-    };
     const float4* rA = reinterpret_cast<const float4*>(recA);
     const float4* rB = reinterpret_cast<const float4*>(recB);
     // this lane's radial grid points, pre-scaled
@@ -530,7 +597,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
                 }
             }
         };
-        if (ntrip <= a.tcap) {
+        {
             // All triples at once (three passes of 64 lanes at 20 neighbours instead of one or
             // more per element pair): the table is ordered by element pair, pbase[p*ns+q] is
             // the first entry of pair (p<=q), prounds[p*ns+q] its length in rounds, and a triple's
@@ -582,7 +649,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
                 const int jl = wj & 0xffff, kl = wk & 0xffff;
                 // any one-to-one numbering of a pair's triples does: k-major within one type, row by row else
                 const int local = (p == q ? (__mul24(kl, kl - 1) >> 1) : __mul24(kl, wj >> 16)) + jl;
-                reinterpret_cast<float4*>(trip)[pbase[__mul24(p, ns) + q] + local] = table_entry(Aj, Bj, Ak, Bk);
+                reinterpret_cast<float4*>(trip)[pbase[__mul24(p, ns) + q] + local] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
             }
             __syncthreads();
             for (int p = 0; p < ns; ++p) {
@@ -594,39 +661,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
                     store_block(pair_offset(p, q, ns, nRs2, nRs3), accc, accs);
                 }
             }
-            return;
-        }
-        // more triples than the table holds: element pair by element pair, in chunks of the table
-        for (int p = 0; p < ns; ++p) {
-            const int op = goff[p], np_ = goff[p + 1] - op;
-            for (int q = p; q < ns; ++q) {
-                const int oq = goff[q], nq = goff[q + 1] - oq;
-                const int ntr = (p == q) ? np_ * (np_ - 1) / 2 : np_ * nq;
-                float accc[MAXLB], accs[MAXLB];
-#pragma unroll
-                for (int b = 0; b < MAXLB; ++b) accc[b] = accs[b] = 0.0f;
-                for (int t0 = 0; t0 < ntr; t0 += a.tcap) {
-                    const int nchunk = min(a.tcap, ntr - t0);
-                    const int rounds = idiv_small(nchunk + TSv - 1, TSv);
-                    __syncthreads();
-                    for (int tt = lane; tt < nchunk; tt += QMLL_WAVE) {
-                        int ja, kb;
-                        if (p == q) {
-                            unrank_pair(t0 + tt, np_, ja, kb);
-                        } else {
-                            ja = (t0 + tt) / nq;
-                            kb = (t0 + tt) - ja * nq;
-                        }
-                        reinterpret_cast<float4*>(trip)[tt] =
-                            table_entry(rA[op + ja], rB[op + ja], rA[oq + kb], rB[oq + kb]);
-                    }
-                    if (lane < rounds * TSv - nchunk)
-                        *reinterpret_cast<float4*>(trip + (nchunk + lane) * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
-                    __syncthreads();
-                    accumulate(0, rounds, accc, accs);
-                }
-                store_block(pair_offset(p, q, ns, nRs2, nRs3), accc, accs);
-            }
         }
     };
     switch (TS) {
@@ -635,6 +669,225 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
         case 3: three_body(std::integral_constant<int, 3>{}); break;
         case 4: three_body(std::integral_constant<int, 4>{}); break;
         default: three_body(std::integral_constant<int, 0>{}); break;
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// forward, several wavefronts per central atom
+//
+// For neighbourhoods too large for one wavefront's table (beyond 46 atoms) and for batches of few atoms, where one
+// wavefront per atom leaves the chip idle and the launch takes as long as one atom's chain of phases.  The
+// triple list, ordered by element pair, is taken in chunks of the table (one chunk where it fits): all wavefronts fill
+// the table, each sums a run of its entries, and the NW partial blocks are added
+// in a fixed order at the end: deterministic like the kernel above.
+// ---------------------------------------------------------------------------------
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a, float* __restrict__ rep) {
+    extern __shared__ float smem[];
+    constexpr int NT = 64 * NW;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = a.molIDs[blockIdx.x];
+    const int i = a.atomIDs[blockIdx.x];
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    const int ns = a.p.nspecies, nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
+    const int np = ns * (ns + 1) / 2;
+    const int R = ns * nRs2 + 2 * np * nRs3;
+
+    const int per = 2 * nRs3;
+    float* trip = smem;                                  // [tcap + 1][4], the last entry zero
+    float* recA = trip + 4 * (a.tcap + 1);
+    float* recB = recA + 4 * a.cap;
+    float* s2b = recB + 4 * a.cap;
+    // [np][NW][2 nRs3] partial blocks; one wavefront adds into the row itself
+    float* part = NW > 1 ? s2b + 4 * a.cap : rep + ((size_t)m * a.n + i) * R + ns * nRs2;
+    int* goff = (int*)(s2b + 4 * a.cap + (NW > 1 ? (size_t)np * NW * per : 0));
+    float* slnRs2 = (float*)(goff + ns + 1);
+    float* sinvRs2 = slnRs2 + nRs2;
+    float* sRs3 = sinvRs2 + nRs2;
+    int* pbase = (int*)(sRs3 + nRs3);                    // [np + 1] first entry of each pair in the triple list
+    int* wcount = pbase + np + 1;                        // [ns * NW]
+
+    const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
+    const float sk3 = fsqrt(a.p.eta3 * LOG2E);
+    const float inv_rc = frcp(a.p.rcut);
+    const float rs2v = tid < nRs2 ? a.Rs2[tid] : 1.0f;
+    const float rs3v = tid < nRs3 ? a.Rs3[tid] : 0.0f;
+    const int nn = visit_neighbours_wide<NW>(
+        a, goff, wcount, m, i, tid, [&](int pos, int rank, int count, int e, int, float dx, float dy, float dz, float r2) {
+            forward_records(a.p, sk3, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
+        });
+    for (int t = tid; t < np * NW * per; t += NT) part[t] = 0.0f;
+    for (int t = tid; t < nRs2; t += NT) {
+        const float v = t == tid ? rs2v : a.Rs2[t];
+        slnRs2[t] = flog(v);
+        sinvRs2[t] = frcp(v);
+    }
+    for (int t = tid; t < nRs3; t += NT) sRs3[t] = t == tid ? rs3v : a.Rs3[t];
+    if (tid < 4) trip[4 * a.tcap + tid] = 0.0f;
+    __syncthreads();
+
+    float* out = rep + ((size_t)m * a.n + i) * R;
+
+    // two-body blocks: an element type per wavefront
+    {
+        const int W = nRs2 < 64 ? nRs2 : 64;
+        const int JS = idiv_small(64, W);
+        const int jsub = idiv_small(lane, W), zl = lane - jsub * W;
+        for (int e = wave; e < ns; e += NW) {
+            const int j0 = goff[e], j1 = goff[e + 1];
+            const int rounds = idiv_small(j1 - j0 + JS - 1, JS);
+            for (int zb = 0; zb < nRs2; zb += W) {
+                const int z = zb + zl;
+                const bool zok = z < nRs2 && jsub < JS;
+                const float lnRs = zok ? slnRs2[z] : 0.0f;
+                const float invRs = zok ? sinvRs2[z] : 0.0f;
+                float acc = 0.0f;
+#pragma unroll 2
+                for (int it = 0; it < rounds; ++it) {
+                    const int j = j0 + jsub + it * JS;
+                    const bool jok = zok && j < j1;
+                    const float3v f = *reinterpret_cast<const float3v*>(s2b + 4 * (jok ? j : j0));
+                    const float u = lnRs - f.x;
+                    acc = fmaf(jok ? f.z : 0.0f, fexp2(-u * u * f.y), acc);
+                }
+                acc *= invRs;
+                float tot = acc;
+                for (int k = 1; k < JS; ++k) tot += __shfl(acc, zl + W * k, 64);
+                if (zok && jsub == 0) out[e * nRs2 + z] = tot;
+            }
+        }
+    }
+    // the pairs' segments of the triple list (the same on every wavefront)
+    for (int q0 = 0, acc = 0; q0 < np; q0 += QMLL_WAVE) {
+        int size = 0;
+        if (q0 + lane < np) {
+            int p = 0, rest = q0 + lane;
+            while (rest >= ns - p) rest -= ns - p++;
+            const int q = p + rest;
+            const int np_ = goff[p + 1] - goff[p], nq = goff[q + 1] - goff[q];
+            size = p == q ? (__mul24(np_, np_ - 1) >> 1) : __mul24(np_, nq);
+        }
+        int incl = size;
+        for (int o = 1; o < QMLL_WAVE && o < np; o <<= 1) {
+            const int up = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += up;
+        }
+        if (q0 + lane < np) pbase[q0 + lane + 1] = acc + incl;
+        if (q0 == 0 && lane == 0) pbase[0] = 0;
+        acc += __shfl(incl, 63, 64);
+    }
+    __syncthreads();
+
+    const int W3 = nRs3 < 64 ? nRs3 : 64;
+    const int TS = idiv_small(64, W3);
+    const int tsub = idiv_small(lane, W3), ll = lane - tsub * W3;
+    constexpr int MAXLB = 4;                             // radial bins handled: up to 4 x 64
+    float rsl[MAXLB];
+#pragma unroll
+    for (int b = 0; b < MAXLB; ++b) {
+        const int l = b * 64 + ll;
+        rsl[b] = (b * 64 < nRs3) ? sk3 * sRs3[l < nRs3 ? l : 0] : 0.0f;
+    }
+    const float zw3 = zeta2 * a.p.three_body_weight, hd3 = -0.5f * a.p.three_body_decay;
+    const float4* rA = reinterpret_cast<const float4*>(recA);
+    const float4* rB = reinterpret_cast<const float4*>(recB);
+    const float4* tab = reinterpret_cast<const float4*>(trip);
+    const int ntrip = nn * (nn - 1) / 2;
+
+    for (int t0 = 0; t0 < ntrip; t0 += a.tcap) {
+        const int t1 = min(t0 + a.tcap, ntrip);
+        if (t0 > 0) __syncthreads();                     // the previous chunk has been read
+        for (int tt = t0 + tid; tt < t1; tt += NT) {
+            // entry tt of the list: its pair, and the triple's number within the pair
+            int p = 0, q = 0, j, k;
+            if (t0 == 0 && t1 == ntrip) {                // the whole list at once: any order of filling does
+                unrank_pair_kmajor(tt, j, k);
+            } else {
+                int pq = 0;
+                while (pq + 1 < np && tt >= pbase[pq + 1]) {
+                    ++pq;
+                    if (++q == ns) q = ++p;
+                }
+                const int local = tt - pbase[pq];
+                if (p == q) {
+                    unrank_pair_kmajor(local, j, k);
+                } else {
+                    const int nj = goff[p + 1] - goff[p];
+                    k = idiv_small(local, nj);
+                    j = local - __mul24(k, nj);
+                }
+                j += goff[p];
+                k += goff[q];
+            }
+            const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
+            int to = tt - t0;
+            if (t0 == 0 && t1 == ntrip) {
+                p = __float_as_int(Bj.z);                // p <= q: the list is sorted by type
+                q = __float_as_int(Bk.z);
+                const int wj = __float_as_int(Bj.w), wk = __float_as_int(Bk.w);
+                const int jl = wj & 0xffff, kl = wk & 0xffff;
+                to = pbase[__mul24(ns, p) - (__mul24(p, p - 1) >> 1) + q - p] +
+                     (p == q ? (__mul24(kl, kl - 1) >> 1) : __mul24(kl, wj >> 16)) + jl;
+            }
+            reinterpret_cast<float4*>(trip)[to] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
+        }
+        __syncthreads();
+        // this wavefront's share of the chunk: a run of consecutive entries, which meets few element pairs
+        const int len = t1 - t0, w0 = len * wave / NW, w1 = len * (wave + 1) / NW;
+        int pq = 0;
+        while (pq < np - 1 && pbase[pq + 1] - t0 <= w0) ++pq;
+        for (; pq < np && pbase[pq] - t0 < w1; ++pq) {
+            const int s0 = __builtin_amdgcn_readfirstlane(max(pbase[pq] - t0, w0));
+            const int count = __builtin_amdgcn_readfirstlane(min(pbase[pq + 1] - t0, w1)) - s0;
+            if (count <= 0) continue;
+            const int rounds = idiv_small(count, TS), rest = count - rounds * TS;
+            const float4* src = tab + s0 + (tsub < TS ? tsub : 0);
+            float* dst = part + ((size_t)pq * NW + wave) * per;
+#pragma unroll
+            for (int b = 0; b < MAXLB; ++b) {
+                if (b * 64 < nRs3) {
+                    float c_ = 0.0f, s_ = 0.0f;
+#pragma unroll 4
+                    for (int it = 0; it < rounds; ++it) {
+                        const float3v v = *reinterpret_cast<const float3v*>(src + it * TS);
+                        const float d = v.x - rsl[b];
+                        const float e = fexp2(-d * d);
+                        c_ = fmaf(e, v.y, c_);
+                        s_ = fmaf(e, v.z, s_);
+                    }
+                    if (rest > 0) {
+                        const float3v v = *reinterpret_cast<const float3v*>(tsub < rest ? src + rounds * TS : tab + a.tcap);
+                        const float d = v.x - rsl[b];
+                        const float e = fexp2(-d * d);
+                        c_ = fmaf(e, v.y, c_);
+                        s_ = fmaf(e, v.z, s_);
+                    }
+                    float tc = c_, tsn = s_;
+                    for (int k = 1; k < TS; ++k) {
+                        tc += __shfl(c_, ll + W3 * k, 64);
+                        tsn += __shfl(s_, ll + W3 * k, 64);
+                    }
+                    const int l = b * 64 + ll;
+                    if (tsub == 0 && l < nRs3) {          // this wavefront's words alone
+                        dst[2 * l] += tc;
+                        dst[2 * l + 1] += tsn;
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (NW == 1) return;
+    __syncthreads();
+    // the partial blocks, wavefront by wavefront; the pairs' blocks of the row follow each other in this order
+    float* out3 = out + ns * nRs2;
+    for (int t = tid; t < np * per; t += NT) {
+        const int pq = idiv_small(t, per), x = t - pq * per;
+        const float* src = part + (size_t)pq * NW * per + x;
+        float v = src[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += src[w * per];
+        out3[t] = v;
     }
 }
 
@@ -702,19 +955,30 @@ __device__ __forceinline__ TripleDeriv triple_derivatives(const Triple& t, const
     return d;
 }
 
+// copies of the neighbours' force array that one wavefront of the backward kernel needs for nn neighbours: as many
+// s = tt / nn as 64 consecutive triple numbers tt span, and at least one for the two-body part
+__host__ __device__ __forceinline__ int force_copies(int nn) {
+    if (nn < 2) return 1;
+    const int span = (62 + nn) / nn + 1, all = nn / 2;
+    return span < all ? span : all;
+}
+
 // ---------------------------------------------------------------------------------
 // VJP
 // ---------------------------------------------------------------------------------
-// TABLE: the force coefficients of a triple (j, k) go to a neighbour x neighbour matrix in LDS, entry
-// [x][y] = (ec, coefficient of d_ix) of the triple {x, y}, and every neighbour's row is summed
-// afterwards with a loop of the same length for every lane, instead of LDS atomics, which
-// serialise badly here: the 64 triples of a pass share 3-4 values of j.  a.tcap is the matrix's row
-// length (odd, so that rows start in different banks).
-template <bool TABLE>
-__global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float* __restrict__ grad_rep,
-                                                         float* __restrict__ grad_X) {
+// The forces of a triple on its two neighbours are added into LDS without atomics (ds_add_f32 costs tens of clocks
+// PER LANE here: with them 16 boxes of 96 atoms took 190 us, with their adds taken out 54): the triples are numbered so
+// that consecutive lanes have different j and different k, and a wavefront keeps as many private copies of the
+// neighbours' force array as 64 consecutive triples can meet the same neighbour (force_copies).  An instruction's lanes then
+// read, add and write different words, one 16-byte record each, and the copies are summed at the end.  NW wavefronts
+// per atom share out the triples: see wavefronts_per_atom.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const float* __restrict__ grad_rep,
+                                                              float* __restrict__ grad_X) {
     extern __shared__ float smem[];
-    const int lane = threadIdx.x;
+    constexpr int NT = 64 * NW;
+    const int tid = threadIdx.x, lane = NW == 1 ? tid : tid & 63;
+    const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = a.molIDs[blockIdx.x];
     const int i = a.atomIDs[blockIdx.x];
     if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
@@ -726,14 +990,12 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
     // (1 / r, fc, dfc / dr, element type); first in LDS, 16-byte aligned
     float* recA = smem;
     float* recB = recA + 4 * a.cap;
-    float* eo = recB + 4 * a.cap;              // TABLE: [cap][tcap][2]
-    float* gin3 = eo + (TABLE ? 2 * a.cap * a.tcap : 0);   // [NE3][2] incoming gradient of the three-body bins (cos, sin), see below; 8-byte aligned
+    float* force = recB + 4 * a.cap;           // [NW][tcap][4] forces on the neighbours: copies of nn records
+    float* gin3 = force + 4 * NW * a.tcap;   // [NE3][2] incoming gradient of the three-body bins (cos, sin), see below; 8-byte aligned
     int* sj = (int*)(gin3 + 2 * NE3);          // [cap] atom index of neighbour j
     int* goff = sj + a.cap;              // [ns+1] slices of the sorted neighbour list by type
-    float* sgx = (float*)(goff + ns + 1);   // [cap] gradient on neighbour j
-    float* sgy = sgx + a.cap;
-    float* sgz = sgy + a.cap;
-    float* slnRs2 = sgz + a.cap;     // [nRs2]
+    int* wcount = goff + ns + 1;         // [ns * NW] scratch of the staging
+    float* slnRs2 = (float*)(wcount + (NW > 1 ? ns * NW : 0));   // [nRs2]
     float* sRs3 = slnRs2 + nRs2;     // [nRs3] sk3 Rs3 (fast form: about the middle of the grid)
     float* sfac = sRs3 + nRs3;       // [nRs3] 2^(-u^2) of every bin (fast form)
     float* gin2 = sfac + nRs3;       // [R2] incoming gradient of the two-body bins, each divided by its Rs2
@@ -744,33 +1006,32 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
     // row) are issued first and consumed after the staging, so their latency overlaps the
     // staging's own loads.
     const float* gsrc = grad_rep + ((size_t)m * a.n + i) * (R2 + 2 * NE3);
-    constexpr int GREG2 = 2, GREG3 = 4;          // values / (cos, sin) pairs per lane held in registers
+    constexpr int GREG2 = NW > 2 ? 1 : 2, GREG3 = NW > 2 ? 1 : 4 / NW;   // values / (cos, sin) pairs per thread held in registers
     float gr2[GREG2], gr3c[GREG3], gr3s[GREG3];
 #pragma unroll
-    for (int k = 0; k < GREG2; ++k) gr2[k] = lane + QMLL_WAVE * k < R2 ? gsrc[lane + QMLL_WAVE * k] : 0.0f;
+    for (int k = 0; k < GREG2; ++k) gr2[k] = tid + NT * k < R2 ? gsrc[tid + NT * k] : 0.0f;
 #pragma unroll
     for (int k = 0; k < GREG3; ++k) {
-        const int e = lane + QMLL_WAVE * k;
+        const int e = tid + NT * k;
         gr3c[k] = e < NE3 ? gsrc[R2 + 2 * e] : 0.0f;
         gr3s[k] = e < NE3 ? gsrc[R2 + 2 * e + 1] : 0.0f;
     }
     const float rs2v = lane < nRs2 ? a.Rs2[lane] : 1.0f;
     const float rs3v = lane < nRs3 ? a.Rs3[lane] : 0.0f;
-    for (int t = lane; t < a.cap; t += QMLL_WAVE) {
-        sgx[t] = 0.0f;
-        sgy[t] = 0.0f;
-        sgz[t] = 0.0f;
-    }
+    float4* mine = reinterpret_cast<float4*>(force) + wave * a.tcap;   // this wavefront's copies
+    for (int t = lane; t < a.tcap; t += QMLL_WAVE) mine[t] = make_float4(0.f, 0.f, 0.f, 0.f);
     const float inv_rc = frcp(a.p.rcut);
-    const int nn = visit_neighbours(a, goff, m, i, lane,
-                                    [&](int pos, int, int, int e, int j, float dx, float dy, float dz, float r2) {
-                                        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
-                                        float fc, dfc;
-                                        cutoff(r, inv_rc, fc, dfc);
-                                        reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, r);
-                                        reinterpret_cast<float4*>(recB)[pos] = make_float4(ir, fc, dfc, __int_as_float(e));
-                                        sj[pos] = j;
-                                    });
+    auto emit = [&](int pos, int, int, int e, int j, float dx, float dy, float dz, float r2) {
+        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        float fc, dfc;
+        cutoff(r, inv_rc, fc, dfc);
+        reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, r);
+        reinterpret_cast<float4*>(recB)[pos] = make_float4(ir, fc, dfc, __int_as_float(e));
+        sj[pos] = j;
+    };
+    int nn;
+    if constexpr (NW == 1) nn = visit_neighbours(a, goff, m, i, lane, emit);
+    else nn = visit_neighbours_wide<NW>(a, goff, wcount, m, i, tid, emit);
     const float k3 = a.p.eta3 * LOG2E;
     const float sk3 = fsqrt(k3);                       // the radial grid of the triples is kept as sk3 Rs3
     const float hfac = -2.0f * a.p.eta3 * frcp(sk3);
@@ -797,14 +1058,14 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
     // the gradient of the two-body bins, each divided by its grid point (the bin's 1 / Rs2 factor)
 #pragma unroll
     for (int k = 0; k < GREG2; ++k) {
-        const int t = lane + QMLL_WAVE * k;
+        const int t = tid + NT * k;
         if (t < R2) gin2[t] = gr2[k] * (a.gscale * frcp(a.Rs2[t - nRs2 * idiv_small(t, nRs2)]));
     }
-    for (int t = lane + QMLL_WAVE * GREG2; t < R2; t += QMLL_WAVE)
+    for (int t = tid + NT * GREG2; t < R2; t += NT)
         gin2[t] = gsrc[t] * (a.gscale * frcp(a.Rs2[t - nRs2 * idiv_small(t, nRs2)]));
-    if (lane < nRs2) slnRs2[lane] = flog(rs2v);
-    for (int t = lane + QMLL_WAVE; t < nRs2; t += QMLL_WAVE) slnRs2[t] = flog(a.Rs2[t]);
-    for (int t = lane; t < nRs3; t += QMLL_WAVE) {
+    if (lane < nRs2 && wave == 0) slnRs2[lane] = flog(rs2v);
+    for (int t = tid + QMLL_WAVE; t < nRs2; t += NT) slnRs2[t] = flog(a.Rs2[t]);
+    for (int t = tid; t < nRs3; t += NT) {
         const float u = fmaf(sk3, t == lane ? rs3v : a.Rs3[t], -shift);
         sRs3[t] = u;
         sfac[t] = a.gscale * (fast ? fexp2(-u * u) : 1.0f);
@@ -819,12 +1080,8 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
     };
 #pragma unroll
     for (int k = 0; k < GREG3; ++k)
-        if (lane + QMLL_WAVE * k < NE3) stage3(lane + QMLL_WAVE * k, gr3c[k], gr3s[k]);
-    for (int e = lane + QMLL_WAVE * GREG3; e < NE3; e += QMLL_WAVE) stage3(e, gsrc[R2 + 2 * e], gsrc[R2 + 2 * e + 1]);
-    if constexpr (TABLE) {
-        // no triple writes the diagonal of the coefficient matrix
-        for (int t = lane; t < nn; t += QMLL_WAVE) reinterpret_cast<float2*>(eo)[t * a.tcap + t] = make_float2(0.0f, 0.0f);
-    }
+        if (tid + NT * k < NE3) stage3(tid + NT * k, gr3c[k], gr3s[k]);
+    for (int e = tid + NT * GREG3; e < NE3; e += NT) stage3(e, gsrc[R2 + 2 * e], gsrc[R2 + 2 * e + 1]);
     __syncthreads();
 
     float gix = 0.0f, giy = 0.0f, giz = 0.0f;
@@ -852,7 +1109,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
                 const float q1 = tb.fc * inv_s2 * tb.mup;
                 const float q2 = tb.fc * hs * inv_s2;
                 const float* gz = gin2 + __float_as_int(Bj.w) * nRs2;
-                for (int z = g; z < nRs2; z += G) {
+                for (int z = g + G * wave; z < nRs2; z += G * NW) {
                     const float u = slnRs2[z] - tb.mu;
                     const float e = fexp2(u * u * nc);
                     gr = fmaf(gz[z] * e, fmaf(fmaf(q2, u, q1), u, q0), gr);
@@ -866,9 +1123,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
                 gix += tot * ux;
                 giy += tot * uy;
                 giz += tot * uz;
-                sgx[j] -= tot * ux;   // each lane owns its own j here
-                sgy[j] -= tot * uy;
-                sgz[j] -= tot * uz;
+                mine[j] = make_float4(-tot * ux, -tot * uy, -tot * uz, 0.0f);   // each lane owns its own j here
             }
         }
     }
@@ -883,9 +1138,13 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
     const int ntrip = nn * (nn - 1) / 2;
     const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
     const float d3 = a.p.three_body_decay;
-    for (int tt = lane; tt < ntrip; tt += QMLL_WAVE) {
-        int j, k;
-        unrank_pair_kmajor(tt, j, k);                     // tt = k (k - 1) / 2 + j
+    for (int tt = tid; tt < ntrip; tt += NT) {
+        // tt = s nn + j: the pair {j, j + s + 1 mod nn} (when nn is even, the first half of the last s)
+        const int s = idiv_small(tt, nn), j = tt - __mul24(s, nn);
+        int k = j + s + 1;
+        if (k >= nn) k -= nn;
+        // the copy: 64 consecutive tt meet a neighbour once per s
+        float4* own = mine + __mul24(s - idiv_small(tt - lane, nn), nn);
         const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
         const float ia = Bj.x, ib = Bk.x;
         const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
@@ -915,8 +1174,9 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
         const float ka = fmaf(F, fmaf(3.0f, Pa3, -d3P * ia), P * dfa * fb);   // K_a / dec
         const float kb = fmaf(F, fmaf(3.0f, Pb3, -d3P * ib), P * fa * dfb);
         const float kc = F * fmaf(3.0f, Pc3, -d3P * ic);
-        // the (element pair, radial bin) entries of this triple's pair: p <= q, the list is sorted by type
-        const int tp = __float_as_int(Bj.w), tq = __float_as_int(Bk.w);
+        // the (element pair, radial bin) entries of this triple's pair
+        const int tj = __float_as_int(Bj.w), tk = __float_as_int(Bk.w);
+        const int tp = min(tj, tk), tq = max(tj, tk);
         const float2* g = reinterpret_cast<const float2*>(gin3) + __mul24(nRs3, __mul24(ns, tp) - (__mul24(tp, tp + 1) >> 1) + tq);
         // exp(-eta3 (rho - Rs)^2) = exp2(-(x - g_l)^2), x = sk3 rho, the grid stored pre-scaled;
         // d e / d rho = -2 eta3 (rho - Rs) e = hfac (x - g_l) e, the factor applied after the sums
@@ -960,18 +1220,19 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
         gix = fmaf(ea, Aj.x, fmaf(eb, Ak.x, gix));
         giy = fmaf(ea, Aj.y, fmaf(eb, Ak.y, giy));
         giz = fmaf(ea, Aj.z, fmaf(eb, Ak.z, giz));
-        if constexpr (TABLE) {
-            // force on j: ec d_ik - (ec + ea) d_ij, on k: ec d_ij - (eb + ec) d_ik
-            reinterpret_cast<float2*>(eo)[j * a.tcap + k] = make_float2(ec, ec + ea);
-            reinterpret_cast<float2*>(eo)[k * a.tcap + j] = make_float2(ec, eb + ec);
-        } else {
-            atomicAdd(&sgx[j], fmaf(ec, cx, -ea * Aj.x));
-            atomicAdd(&sgy[j], fmaf(ec, cy, -ea * Aj.y));
-            atomicAdd(&sgz[j], fmaf(ec, cz, -ea * Aj.z));
-            atomicAdd(&sgx[k], fmaf(-ec, cx, -eb * Ak.x));
-            atomicAdd(&sgy[k], fmaf(-ec, cy, -eb * Ak.y));
-            atomicAdd(&sgz[k], fmaf(-ec, cz, -eb * Ak.z));
-        }
+        // force on j: ec (d_ik - d_ij) - ea d_ij, on k: -ec (d_ik - d_ij) - eb d_ik
+        float4 f = own[j];
+        f.x += fmaf(ec, cx, -ea * Aj.x);
+        f.y += fmaf(ec, cy, -ea * Aj.y);
+        f.z += fmaf(ec, cz, -ea * Aj.z);
+        own[j] = f;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next read sees every lane's write (LDS instructions run in order)
+        f = own[k];
+        f.x += fmaf(-ec, cx, -eb * Ak.x);
+        f.y += fmaf(-ec, cy, -eb * Ak.y);
+        f.z += fmaf(-ec, cz, -eb * Ak.z);
+        own[k] = f;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     __syncthreads();
     gix = wave_sum(gix);
@@ -983,30 +1244,13 @@ __global__ __launch_bounds__(64) void fchl19_vjp_kernel(FchlArgs a, const float*
         atomicAdd(&gm[i * 3 + 1], giy);
         atomicAdd(&gm[i * 3 + 2], giz);
     }
-    if constexpr (TABLE) {
-        // lane = (neighbour x, component c): the force on x is sum_y ec(x,y) d_iy - d_ix sum_y own(x,y)
-        // over row x of the matrix, plus what the two-body part left for x
-        for (int it = lane; it < 3 * nn; it += QMLL_WAVE) {
-            const int x = idiv_small(it, 3), c = it - 3 * x;
-            float sum = c == 0 ? sgx[x] : (c == 1 ? sgy[x] : sgz[x]);
-            float own = 0.0f;
-            const float* dc = recA + c;                       // component c of d_iy at dc[4 y]
-            const float2* row = reinterpret_cast<const float2*>(eo) + x * a.tcap;
-#pragma unroll 4
-            for (int yv = 0; yv < nn; ++yv) {
-                const float2 v = row[yv];
-                sum = fmaf(v.x, dc[4 * yv], sum);
-                own += v.y;
-            }
-            atomicAdd(&gm[sj[x] * 3 + c], fmaf(-dc[4 * x], own, sum));
-        }
-    } else {
-        for (int j = lane; j < nn; j += QMLL_WAVE) {
-            const int jj = sj[j];
-            atomicAdd(&gm[jj * 3 + 0], sgx[j]);
-            atomicAdd(&gm[jj * 3 + 1], sgy[j]);
-            atomicAdd(&gm[jj * 3 + 2], sgz[j]);
-        }
+    const int ncopies = force_copies(nn);
+    for (int it = tid; it < 3 * nn; it += NT) {
+        const int x = idiv_small(it, 3), c = it - 3 * x;
+        float sum = 0.0f;
+        for (int w = 0; w < NW; ++w)
+            for (int q = 0; q < ncopies; ++q) sum += force[4 * (w * a.tcap + q * nn + x) + c];
+        atomicAdd(&gm[sj[x] * 3 + c], sum);
     }
 }
 
@@ -1324,7 +1568,7 @@ int fill_args(FchlArgs& a, const float* X, const int* types, const float* cell, 
     a.B = B;
     a.cap = nlist ? nn_stride : n;
     if (a.cap < 1) a.cap = 1;
-    a.tcap = TCH;
+    a.tcap = 0;
     a.tpad = 0;
     a.Rs2 = Rs2;
     a.Rs3 = Rs3;
@@ -1334,6 +1578,20 @@ int fill_args(FchlArgs& a, const float* X, const int* types, const float* cell, 
 }
 
 constexpr size_t LDS_LIMIT = 64 * 1024;
+
+// Wavefronts per central atom of the forward and backward kernels.  With one, a launch of A atoms is A wavefronts:
+// below about 1000 the chip (8192 slots at eight per SIMD) is idle while every atom walks through its phases alone, the
+// longer the more triples it has; beyond, the work that every wavefront of an atom repeats (staging, the scan of the
+// pairs) costs more than the idle slots.  Measured, us per launch with 1 / 4 / 8 wavefronts forward, 1 / 4 backward:
+//   21 atoms of 1 molecule 9.2 / 7.8 / 7.4, 8.7 / 7.6;    1008 atoms (21 per molecule) 10.1 / 9.0 / 13.4, 9.4 / 10.1;
+//   1200 (12 per molecule) 7.1 / 8.5 / 12.8, 7.4 / 9.6;   2016 (21) 11.7 / 16.6 / 22.5, 11.3 / 16.6;
+//   1600 (40 in a box) 22.6 / 20.0 / 28.2, 25.3 / 24.0;   1536 (96 in a box) 80 / 47 / 59, 85 / 51
+// big: the neighbourhood does not fit the one-wavefront kernel, or leaves it few wavefronts per CU.
+int wavefronts_per_atom(int A, long long triples, bool big) {
+    if (A <= 256) return 8;
+    if (triples > 100 && A <= (triples > 256 ? 2048 : 1024)) return 4;
+    return big ? 4 : 1;
+}
 
 }  // namespace
 
@@ -1350,21 +1608,41 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     QMLL_REQUIRE(prm->nRs3 <= 256, QMLL_ERR_INVALID,
                  "qmll_fchl19_forward: nRs3=%d: at most 256 three-body radial bins are supported", prm->nRs3);
     const int R = prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3;
-    // table for every triple of a full neighbourhood when that stays small: an atom has at most cap
-    // neighbours from a given list and at most max_atoms - 1 otherwise
+    // an atom has at most cap neighbours from a given list and at most max_atoms - 1 otherwise
     const long long maxnn = nlist ? a.cap : (a.cap > 1 ? a.cap - 1 : 1);
-    const long long alltrip = maxnn * (maxnn - 1) / 2;
-    a.tcap = alltrip <= TCH_MAX ? (int)(alltrip > 0 ? alltrip : 1) : TCH;
+    const long long alltrip = maxnn * (maxnn - 1) / 2 > 0 ? maxnn * (maxnn - 1) / 2 : 1;
+    const int ns = prm->nspecies, np = ns * (ns + 1) / 2;
+    hipStream_t st = (hipStream_t)stream;
+    const bool big = alltrip > TCH_MAX;
+    for (int nw = wavefronts_per_atom(A, alltrip, big); nw > 1 || big; nw /= 2) {
+        // the table holds the triple list, or 12 KB of it at a time
+        a.tcap = alltrip <= TCH_WIDE ? (int)alltrip : TCH_WIDE;
+        const size_t lds = sizeof(float) * (4 * (size_t)(a.tcap + 1) + 12 * (size_t)a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1 +
+                                            (size_t)ns * nw + (nw > 1 ? (size_t)np * nw * 2 * prm->nRs3 : 0));
+        if (lds > LDS_LIMIT) {          // many elements with fine grids: fewer wavefronts, fewer partial blocks
+            QMLL_REQUIRE(nw > 1 || !big, QMLL_ERR_INVALID,
+                         "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
+            continue;
+        }
+        if (nw == 8) hipLaunchKernelGGL(fchl19_forward_wide_kernel<8>, dim3(A), dim3(512), lds, st, a, rep);
+        else if (nw == 4) hipLaunchKernelGGL(fchl19_forward_wide_kernel<4>, dim3(A), dim3(256), lds, st, a, rep);
+        else if (nw == 2) hipLaunchKernelGGL(fchl19_forward_wide_kernel<2>, dim3(A), dim3(128), lds, st, a, rep);
+        else hipLaunchKernelGGL(fchl19_forward_wide_kernel<1>, dim3(A), dim3(64), lds, st, a, rep);
+        QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
+        return QMLL_OK;
+    }
+    // one wavefront per atom, with a table for every triple of a full neighbourhood
+    a.tcap = (int)alltrip;
     // each of the ns (ns+1)/2 segments is padded to a multiple of the triple sub-slot count
     const int tsub_slots = prm->nRs3 < 64 ? 64 / prm->nRs3 : 1;
-    a.tpad = prm->nspecies * (prm->nspecies + 1) / 2 * (tsub_slots - 1);
+    a.tpad = np * (tsub_slots - 1);
     // triple table, three per-neighbour records [cap][4], type offsets, the radial grids, the table's
     // segment starts and lengths
-    const size_t lds = sizeof(float) * ((size_t)12 * a.cap + prm->nspecies + 1 + 2 * prm->nRs2 + prm->nRs3 +
-                                        4 * (size_t)(a.tcap + a.tpad) + 2 * (size_t)prm->nspecies * prm->nspecies + 4);
+    const size_t lds = sizeof(float) * ((size_t)12 * a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 +
+                                        4 * (size_t)(a.tcap + a.tpad) + 2 * (size_t)ns * ns + 4);
     QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID,
                  "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
-    hipLaunchKernelGGL(fchl19_forward_kernel, dim3(A), dim3(64), lds, (hipStream_t)stream, a, rep);
+    hipLaunchKernelGGL(fchl19_forward_kernel, dim3(A), dim3(64), lds, st, a, rep);
     QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
     return QMLL_OK;
 }
@@ -1391,20 +1669,24 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     if (A == 0) return QMLL_OK;
     QMLL_REQUIRE(grad_rep && grad_X, QMLL_ERR_INVALID, "qmll_fchl19_vjp: null gradient pointer");
     const int R = prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3;
-    // two records [cap][4], atom indices, neighbour gradients [3][cap], type offsets, grids, the bins' constant
-    // factors, the gradient row
-    size_t lds = sizeof(float) * ((size_t)12 * a.cap + prm->nspecies + 1 + prm->nRs2 + 2 * prm->nRs3 + R);
-    QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID,
-                 "qmll_fchl19_vjp: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
-    // neighbour x neighbour coefficient matrix (two floats per entry, rows of odd length) while it stays small;
-    // LDS atomics beyond
-    a.tcap = a.cap | 1;
-    const size_t table = sizeof(float) * 2 * (size_t)a.cap * a.tcap;
-    if (table <= 24 * 1024 && lds + table <= LDS_LIMIT) {
-        lds += table;
-        hipLaunchKernelGGL(fchl19_vjp_kernel<true>, dim3(A), dim3(64), lds, (hipStream_t)stream, a, grad_rep, grad_X);
-    } else {
-        hipLaunchKernelGGL(fchl19_vjp_kernel<false>, dim3(A), dim3(64), lds, (hipStream_t)stream, a, grad_rep, grad_X);
+    // records of the force copies: the largest number any neighbour count up to cap needs
+    a.tcap = 1;
+    for (int k = 1; k <= a.cap; ++k) a.tcap = a.tcap < k * force_copies(k) ? k * force_copies(k) : a.tcap;
+    const long long maxnn = nlist ? a.cap : a.cap - 1;
+    for (int nw = std::min(4, wavefronts_per_atom(A, maxnn * (maxnn - 1) / 2, a.cap > 54));; nw /= 2) {
+        // two records [cap][4], atom indices, force copies, type offsets, grids, the bins' constant factors, the gradient row
+        const size_t lds = sizeof(float) * ((size_t)9 * a.cap + 4 * (size_t)nw * a.tcap + prm->nspecies + 1 +
+                                            (nw > 1 ? (size_t)prm->nspecies * nw : 0) + prm->nRs2 + 2 * prm->nRs3 + R);
+        if (lds > LDS_LIMIT) {
+            QMLL_REQUIRE(nw > 1, QMLL_ERR_INVALID,
+                         "qmll_fchl19_vjp: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
+            continue;
+        }
+        hipStream_t st = (hipStream_t)stream;
+        if (nw == 4) hipLaunchKernelGGL(fchl19_vjp_kernel<4>, dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);
+        else if (nw == 2) hipLaunchKernelGGL(fchl19_vjp_kernel<2>, dim3(A), dim3(128), lds, st, a, grad_rep, grad_X);
+        else hipLaunchKernelGGL(fchl19_vjp_kernel<1>, dim3(A), dim3(64), lds, st, a, grad_rep, grad_X);
+        break;
     }
     QMLL_CHECK_LAUNCH("qmll_fchl19_vjp");
     return QMLL_OK;
