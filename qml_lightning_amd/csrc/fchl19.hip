@@ -53,14 +53,14 @@ struct FchlArgs {
     int B;
     int cap;  // capacity of the LDS neighbour arrays
     int tcap; // capacity (entries) of the forward kernel's LDS triple table
-    int tpad; // extra entries for the zero padding between the table's segments
     const float* Rs2;
     const float* Rs3;
     qmll_fchl_params p;
     float gscale;  // the backward kernel returns gscale * J^T g (folded into the staged gradient row)
 };
 
-constexpr int TCH_MAX = 1024;  // largest triple table of the one-wavefront forward kernel (16 KB)
+constexpr int TCH_MAX = 1024;  // longest triple list that the one-wavefront forward kernel is given
+constexpr size_t FORWARD_LDS = 5120;   // its LDS request: 32 wavefronts share the 160 KB of a CU
 constexpr int TCH_WIDE = 768;  // largest of the several-wavefront one (12 KB): beyond, the triple list is taken in chunks
 constexpr float PI_F = 3.14159265358979323846f;
 // three floats read from a 16-byte-aligned LDS entry with a single 12-byte instruction (a 16-byte
@@ -434,16 +434,78 @@ __device__ __forceinline__ float4 table_entry(float zw3, float hd3, const float4
     return make_float4(Bj.x + Bk.x, f * cosT, f * sinT, 0.0f);
 }
 
+// The triples of an atom as one list ordered by element pair, pairs (p <= q) row by row, each pair's part padded to a multiple
+// of `unit` entries: pbase[pq] is its start (written by the wavefront that calls; np + 1 entries).  Returns its length.
+// The padding goes to trip[4 t] as zero entries, as far as the list fits tcap of them.
+__device__ __forceinline__ int pair_segments(const int* goff, int* pbase, int ns, int np, int lane, int unit, float* trip,
+                                             int tcap) {
+    int acc = 0;
+    for (int q0 = 0; q0 < np; q0 += QMLL_WAVE) {
+        int ntr = 0;
+        if (q0 + lane < np) {
+            int p = 0, rest = q0 + lane;
+            while (rest >= ns - p) rest -= ns - p++;
+            const int np_ = goff[p + 1] - goff[p], nq = goff[p + rest + 1] - goff[p + rest];
+            ntr = rest == 0 ? (__mul24(np_, np_ - 1) >> 1) : __mul24(np_, nq);
+        }
+        const int size = unit > 1 ? idiv_small(ntr + unit - 1, unit) * unit : ntr;
+        int incl = size;
+        for (int o = 1; o < QMLL_WAVE && o < np; o <<= 1) {
+            const int up = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += up;
+        }
+        if (q0 + lane < np) pbase[q0 + lane + 1] = acc + incl;
+        if (q0 == 0 && lane == 0) pbase[0] = 0;
+        if (acc + incl <= tcap)
+            for (int t = acc + incl - size + ntr; t < acc + incl; ++t)
+                reinterpret_cast<float4*>(trip)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+        acc += __shfl(incl, min(63, np - 1 - q0), 64);
+    }
+    return acc;
+}
+// where the triple of two neighbours (their second forward records, in list order) stands in the list: k-major within one
+// type, row by row else
+__device__ __forceinline__ int triple_place(const int* pbase, int ns, const float4 Bj, const float4 Bk) {
+    const int p = __float_as_int(Bj.z), q = __float_as_int(Bk.z);   // p <= q: the neighbours are sorted by type
+    const int wj = __float_as_int(Bj.w), wk = __float_as_int(Bk.w);
+    const int jl = wj & 0xffff, kl = wk & 0xffff;
+    return pbase[__mul24(ns, p) - (__mul24(p, p - 1) >> 1) + q - p] +
+           (p == q ? (__mul24(kl, kl - 1) >> 1) : __mul24(kl, wj >> 16)) + jl;
+}
+// and the neighbours of entry tt of the list; false: the entry is padding
+__device__ __forceinline__ bool unrank_triple(const int* goff, const int* pbase, int ns, int np, int tt, int& j, int& k) {
+    int p = 0, q = 0, pq = 0;
+    while (pq + 1 < np && tt >= pbase[pq + 1]) {
+        ++pq;
+        if (++q == ns) q = ++p;
+    }
+    const int local = tt - pbase[pq];
+    const int nj = goff[p + 1] - goff[p], nk = goff[q + 1] - goff[q];
+    bool ok;
+    if (p == q) {
+        unrank_pair_kmajor(local, j, k);
+        ok = k < nj;
+    } else {
+        k = idiv_small(local, nj);
+        j = local - __mul24(k, nj);
+        ok = k < nk;
+    }
+    j += goff[p];
+    k += goff[q];
+    return ok;
+}
+
 // ---------------------------------------------------------------------------------
 // forward
 //
 // Atomic-free: with the neighbours sorted by element type every output block is owned by
 // one loop nest.  Two-body block of type e: lanes = (neighbour sub-slot, radial bin z),
 // serial over the neighbours of type e, partial sums folded across sub-slots by lane
-// shuffles.  Three-body block of the type pair (p<=q): the pair's triples are evaluated
-// once (lane = triple) into an LDS table (rho, K cos, K sin), then lanes = (triple
-// sub-slot, radial bin l) run over the table with the bin sums in registers.  Rows go
-// straight from registers to global memory.
+// shuffles.  Three-body block of the type pair (p<=q): the triples are evaluated
+// once (lane = triple) into an LDS table (rho, K cos, K sin) ordered by pair, then lanes = (triple
+// sub-slot, radial bin l) run over the pair's part of it with the bin sums in registers.  Rows go
+// straight from registers to global memory.  The table holds as many triples as leave room for
+// eight wavefronts per SIMD (FORWARD_LDS); a longer list is taken piece by piece.
 // ---------------------------------------------------------------------------------
 // (96 scalar registers: the eighth wavefront per SIMD; a SIMD has 800 of them, handed out in sixteens, and left
 // alone the kernel takes 106.  The thirty-odd values that no longer fit are parked in the lanes of a vector
@@ -460,17 +522,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
 
     // LDS: the triple table, three records per neighbour (read with one instruction each), the
     // type offsets, the radial grids, the table's segments
-    float* trip = smem;                                  // [tcap + tpad][4]: sk3 rho, K cos, K sin, -
-    float* recA = trip + 4 * (a.tcap + a.tpad);          // [cap][4]: d_ij, 1 / r
+    float* trip = smem;                                  // [tcap][4]: sk3 rho, K cos, K sin, -
+    float* recA = trip + 4 * a.tcap;                     // [cap][4]: d_ij, 1 / r
     float* recB = recA + 4 * a.cap;                      // [cap][4]: sk3 r / 2, fc r^-d3, element type,
                                                          //           index within the type | neighbours of the type << 16
-    float* s2b = recB + 4 * a.cap;                       // [cap][4]: mu_j, log2(e) / (2 sigma_j^2), r^-d2 fc / (sigma sqrt(2pi)), -
-    int* goff = (int*)(s2b + 4 * a.cap);                 // [ns+1] slices of the sorted neighbour list by type
+    float* s2b = trip;                                   // [cap][4]: mu_j, log2(e) / (2 sigma_j^2), r^-d2 fc / (sigma sqrt(2pi)), -,
+                                                         //           done with before the table is filled (tcap >= cap)
+    int* goff = (int*)(recB + 4 * a.cap);                // [ns+1] slices of the sorted neighbour list by type
     float* slnRs2 = (float*)(goff + ns + 1);             // [nRs2]
     float* sinvRs2 = slnRs2 + nRs2;                      // [nRs2]
     float* sRs3 = sinvRs2 + nRs2;                        // [nRs3]
-    int* pbase = (int*)(sRs3 + nRs3);                    // [ns*ns] first table entry of each element pair
-    int* prounds = pbase + ns * ns;                      // [ns*ns] rounds of each element pair's segment
+    int* pbase = (int*)(sRs3 + nRs3);                    // [np+1] first entry of each element pair in the triple list
 
     // Global loads that do not depend on the neighbourhood are issued first and consumed after
     // the staging, so their latency overlaps the staging's own loads.
@@ -548,25 +610,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
         const int l = b * 64 + ll;
         rsl[b] = (b * 64 < nRs3) ? sk3 * sRs3[l < nRs3 ? l : 0] : 0.0f;
     }
-    // fold the triple sub-slots and store the block of pair (p,q)
-    auto store_block = [&](int sbase, const float (&accc)[MAXLB], const float (&accs)[MAXLB]) {
-#pragma unroll
-        for (int b = 0; b < MAXLB; ++b) {
-            if (b * 64 < nRs3) {
-                float tc = accc[b], tsn = accs[b];
-                for (int k = 1; k < TS; ++k) {
-                    tc += __shfl(accc[b], ll + W3 * k, 64);
-                    tsn += __shfl(accs[b], ll + W3 * k, 64);
-                }
-                const int l = b * 64 + ll;
-                if (tsub == 0 && l < nRs3) {
-                    out[sbase + 2 * l] = tc;
-                    out[sbase + 2 * l + 1] = tsn;
-                }
+    const int ntrip = nn * (nn - 1) / 2;
+    const int np = ns * (ns + 1) / 2;
+    // a pair's part of the list is padded with zero entries to whole rounds, so that every sub-slot runs the same number
+    // of rounds and the bin loop is wavefront-uniform (scalar control, unrollable)
+    const int length = __builtin_amdgcn_readfirstlane(pair_segments(goff, pbase, ns, np, lane, TS, trip, a.tcap));
+    const bool whole = length <= a.tcap;         // the list in one piece, else piece by piece
+    __syncthreads();
+    // entries t0 .. t1 of the triple list, ordered by element pair, into the table
+    auto fill = [&](int t0, int t1) {
+        if (whole) {                             // any order of filling does
+            for (int tt = lane; tt < ntrip; tt += QMLL_WAVE) {
+                int j, k;
+                unrank_pair_kmajor(tt, j, k);
+                const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
+                reinterpret_cast<float4*>(trip)[triple_place(pbase, ns, Bj, Bk)] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
             }
+            return;
+        }
+        for (int tt = t0 + lane; tt < t1; tt += QMLL_WAVE) {
+            int j, k;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (unrank_triple(goff, pbase, ns, np, tt, j, k)) v = table_entry(zw3, hd3, rA[j], rB[j], rA[k], rB[k]);
+            reinterpret_cast<float4*>(trip)[tt - t0] = v;
         }
     };
-    const int ntrip = nn * (nn - 1) / 2;
+    float* out3 = out + ns * nRs2;               // the pairs' blocks follow each other in list order
 
     // The rest of the kernel, with the sub-slot count as a compile-time constant where it is one of
     // the common ones (TSC = 0: any): the table reads of a round then sit at fixed offsets from
@@ -574,11 +643,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
     auto three_body = [&](auto tsc) {
         constexpr int TSC = decltype(tsc)::value;
         const int TSv = TSC ? TSC : TS;
-        // bin sums of `rounds` rounds of table entries starting at `first`, added to the
-        // accumulators.  A segment is padded with zero entries to whole rounds, so every sub-slot
-        // runs the same number of rounds and the loop is wavefront-uniform (scalar control, unrollable).
-        auto accumulate = [&](int first, int rounds, float (&accc)[MAXLB], float (&accs)[MAXLB]) {
-            const float4* src = reinterpret_cast<const float4*>(trip) + first + (tsub < TSv ? tsub : 0);
+        const int tsafe = tsub < TSv ? tsub : 0;
+        // bin sums of `rounds` rounds of table entries starting at `from`, added to the accumulators
+        auto accumulate = [&](int from, int rounds, float (&accc)[MAXLB], float (&accs)[MAXLB]) {
+            const float4* src = reinterpret_cast<const float4*>(trip) + from + tsafe;
 #pragma unroll
             for (int b = 0; b < MAXLB; ++b) {
                 if (b * 64 < nRs3) {
@@ -597,70 +665,50 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
                 }
             }
         };
-        {
-            // All triples at once (three passes of 64 lanes at 20 neighbours instead of one or
-            // more per element pair): the table is ordered by element pair, pbase[p*ns+q] is
-            // the first entry of pair (p<=q), prounds[p*ns+q] its length in rounds, and a triple's
-            // slot follows from its position in the sorted list.
-            if (ns * ns <= QMLL_WAVE) {
-                // lane p*ns+q takes pair (p,q); an exclusive scan over the lanes gives the starts
-                const int p = idiv_small(lane, ns), q = lane - p * ns;
-                int rounds = 0, ntr = 0;
-                if (lane < ns * ns && q >= p) {
-                    const int np_ = goff[p + 1] - goff[p], nq = goff[q + 1] - goff[q];
-                    ntr = (p == q) ? (__mul24(np_, np_ - 1) >> 1) : __mul24(np_, nq);
-                    rounds = idiv_small(ntr + TSv - 1, TSv);
-                }
-                const int size = rounds * TSv;               // segments start on a multiple of TS
-                int incl = size;
-                for (int o = 1; o < ns * ns; o <<= 1) {
-                    const int up = __shfl_up(incl, o, 64);
-                    if (lane >= o) incl += up;
-                }
-                if (lane < ns * ns) {
-                    pbase[lane] = incl - size;
-                    prounds[lane] = rounds;
-                    // the padding of the segment is zero entries: they contribute nothing
-                    for (int t = incl - size + ntr; t < incl; ++t)
-                        reinterpret_cast<float4*>(trip)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-            } else if (lane == 0) {
-                int acc = 0;
-                for (int p = 0; p < ns; ++p) {
-                    const int np_ = goff[p + 1] - goff[p];
-                    for (int q = p; q < ns; ++q) {
-                        const int ntr = (p == q) ? np_ * (np_ - 1) / 2 : np_ * (goff[q + 1] - goff[q]);
-                        const int rounds = idiv_small(ntr + TSv - 1, TSv);
-                        pbase[p * ns + q] = acc;
-                        prounds[p * ns + q] = rounds;
-                        for (int t = acc + ntr; t < acc + rounds * TSv; ++t)
-                            reinterpret_cast<float4*>(trip)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        acc += rounds * TSv;
+        // fold the triple sub-slots and store the pair's block
+        auto store_block = [&](int pq, bool any, const float (&accc)[MAXLB], const float (&accs)[MAXLB]) {
+#pragma unroll
+            for (int b = 0; b < MAXLB; ++b) {
+                if (b * 64 < nRs3) {
+                    float tc = accc[b], tsn = accs[b];
+                    if (any) {
+                        for (int k = 1; k < TSv; ++k) {
+                            tc += __shfl(accc[b], ll + W3 * k, 64);
+                            tsn += __shfl(accs[b], ll + W3 * k, 64);
+                        }
+                    }
+                    const int l = b * 64 + ll;
+                    if (tsub == 0 && l < nRs3) {
+                        const float2 v = make_float2(tc, tsn);
+                        __builtin_memcpy(out3 + 2 * (pq * nRs3 + l), &v, sizeof v);   // one 8-byte store, 4-byte aligned
                     }
                 }
             }
-            __syncthreads();
-            for (int tt = lane; tt < ntrip; tt += QMLL_WAVE) {
-                int j, k;
-                unrank_pair_kmajor(tt, j, k);
-                const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
-                const int p = __float_as_int(Bj.z), q = __float_as_int(Bk.z);   // p <= q: the list is sorted by type
-                const int wj = __float_as_int(Bj.w), wk = __float_as_int(Bk.w);
-                const int jl = wj & 0xffff, kl = wk & 0xffff;
-                // any one-to-one numbering of a pair's triples does: k-major within one type, row by row else
-                const int local = (p == q ? (__mul24(kl, kl - 1) >> 1) : __mul24(kl, wj >> 16)) + jl;
-                reinterpret_cast<float4*>(trip)[pbase[__mul24(p, ns) + q] + local] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
-            }
-            __syncthreads();
-            for (int p = 0; p < ns; ++p) {
-                for (int q = p; q < ns; ++q) {
-                    float accc[MAXLB], accs[MAXLB];
+        };
+        int first = 0, last = min(a.tcap, length);                   // what the table holds
+        fill(first, last);
+        __syncthreads();
+        int pos = 0;
+        for (int pq = 0; pq < np; ++pq) {
+            const int begin = pos, end = __builtin_amdgcn_readfirstlane(pbase[pq + 1]);
+            float accc[MAXLB], accs[MAXLB];
 #pragma unroll
-                    for (int b = 0; b < MAXLB; ++b) accc[b] = accs[b] = 0.0f;
-                    accumulate(pbase[p * ns + q], prounds[p * ns + q], accc, accs);
-                    store_block(pair_offset(p, q, ns, nRs2, nRs3), accc, accs);
-                }
+            for (int b = 0; b < MAXLB; ++b) accc[b] = accs[b] = 0.0f;
+            if (__builtin_expect(end > last, 0)) {
+                // the pair's part goes beyond the table: refill until its last piece is there
+                do {
+                    accumulate(pos - first, idiv_small(last - pos, TSv), accc, accs);
+                    pos = first = last;
+                    last = min(first + a.tcap, length);
+                    __syncthreads();
+                    fill(first, last);
+                    __syncthreads();
+                } while (end > last);
             }
+            const bool any = end > begin;        // the elements of the pair are both there
+            if (any) accumulate(pos - first, idiv_small(end - pos, TSv), accc, accs);
+            pos = end;
+            store_block(pq, any, accc, accs);
         }
     };
     switch (TS) {
@@ -758,25 +806,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
             }
         }
     }
-    // the pairs' segments of the triple list (the same on every wavefront)
-    for (int q0 = 0, acc = 0; q0 < np; q0 += QMLL_WAVE) {
-        int size = 0;
-        if (q0 + lane < np) {
-            int p = 0, rest = q0 + lane;
-            while (rest >= ns - p) rest -= ns - p++;
-            const int q = p + rest;
-            const int np_ = goff[p + 1] - goff[p], nq = goff[q + 1] - goff[q];
-            size = p == q ? (__mul24(np_, np_ - 1) >> 1) : __mul24(np_, nq);
-        }
-        int incl = size;
-        for (int o = 1; o < QMLL_WAVE && o < np; o <<= 1) {
-            const int up = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += up;
-        }
-        if (q0 + lane < np) pbase[q0 + lane + 1] = acc + incl;
-        if (q0 == 0 && lane == 0) pbase[0] = 0;
-        acc += __shfl(incl, 63, 64);
-    }
+    pair_segments(goff, pbase, ns, np, lane, 1, trip, 0);   // the same on every wavefront
     __syncthreads();
 
     const int W3 = nRs3 < 64 ? nRs3 : 64;
@@ -795,41 +825,16 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
     const float4* tab = reinterpret_cast<const float4*>(trip);
     const int ntrip = nn * (nn - 1) / 2;
 
+    const bool whole = ntrip <= a.tcap;
     for (int t0 = 0; t0 < ntrip; t0 += a.tcap) {
         const int t1 = min(t0 + a.tcap, ntrip);
         if (t0 > 0) __syncthreads();                     // the previous chunk has been read
         for (int tt = t0 + tid; tt < t1; tt += NT) {
-            // entry tt of the list: its pair, and the triple's number within the pair
-            int p = 0, q = 0, j, k;
-            if (t0 == 0 && t1 == ntrip) {                // the whole list at once: any order of filling does
-                unrank_pair_kmajor(tt, j, k);
-            } else {
-                int pq = 0;
-                while (pq + 1 < np && tt >= pbase[pq + 1]) {
-                    ++pq;
-                    if (++q == ns) q = ++p;
-                }
-                const int local = tt - pbase[pq];
-                if (p == q) {
-                    unrank_pair_kmajor(local, j, k);
-                } else {
-                    const int nj = goff[p + 1] - goff[p];
-                    k = idiv_small(local, nj);
-                    j = local - __mul24(k, nj);
-                }
-                j += goff[p];
-                k += goff[q];
-            }
+            int j, k;
+            if (whole) unrank_pair_kmajor(tt, j, k);     // any order of filling does
+            else unrank_triple(goff, pbase, ns, np, tt, j, k);
             const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
-            int to = tt - t0;
-            if (t0 == 0 && t1 == ntrip) {
-                p = __float_as_int(Bj.z);                // p <= q: the list is sorted by type
-                q = __float_as_int(Bk.z);
-                const int wj = __float_as_int(Bj.w), wk = __float_as_int(Bk.w);
-                const int jl = wj & 0xffff, kl = wk & 0xffff;
-                to = pbase[__mul24(ns, p) - (__mul24(p, p - 1) >> 1) + q - p] +
-                     (p == q ? (__mul24(kl, kl - 1) >> 1) : __mul24(kl, wj >> 16)) + jl;
-            }
+            const int to = whole ? triple_place(pbase, ns, Bj, Bk) : tt - t0;
             reinterpret_cast<float4*>(trip)[to] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
         }
         __syncthreads();
@@ -1569,7 +1574,6 @@ int fill_args(FchlArgs& a, const float* X, const int* types, const float* cell, 
     a.cap = nlist ? nn_stride : n;
     if (a.cap < 1) a.cap = 1;
     a.tcap = 0;
-    a.tpad = 0;
     a.Rs2 = Rs2;
     a.Rs3 = Rs3;
     a.p = *prm;
@@ -1631,15 +1635,15 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
         QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
         return QMLL_OK;
     }
-    // one wavefront per atom, with a table for every triple of a full neighbourhood
-    a.tcap = (int)alltrip;
-    // each of the ns (ns+1)/2 segments is padded to a multiple of the triple sub-slot count
-    const int tsub_slots = prm->nRs3 < 64 ? 64 / prm->nRs3 : 1;
-    a.tpad = np * (tsub_slots - 1);
-    // triple table, three per-neighbour records [cap][4], type offsets, the radial grids, the table's
-    // segment starts and lengths
-    const size_t lds = sizeof(float) * ((size_t)12 * a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 +
-                                        4 * (size_t)(a.tcap + a.tpad) + 2 * (size_t)ns * ns + 4);
+    // one wavefront per atom: two per-neighbour records [cap][4], type offsets, the radial grids, the pairs' segment starts,
+    // and a table of as many triples as FORWARD_LDS leaves room for
+    const size_t rest = sizeof(float) * ((size_t)8 * a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1);
+    const long long room = rest < FORWARD_LDS ? (long long)(FORWARD_LDS - rest) / 16 : 0;
+    // each pair's part of the list is padded to a multiple of the triple sub-slot count, and so is the table
+    const int unit = prm->nRs3 < 64 ? 64 / prm->nRs3 : 1;
+    a.tcap = (int)std::max<long long>(std::min(alltrip + np * (unit - 1), std::max(room - unit, 128LL)), a.cap);
+    a.tcap = (a.tcap + unit - 1) / unit * unit;
+    const size_t lds = rest + 16 * (size_t)a.tcap;
     QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID,
                  "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
     hipLaunchKernelGGL(fchl19_forward_kernel, dim3(A), dim3(64), lds, st, a, rep);
