@@ -1,0 +1,445 @@
+// Fused SORF energy and gradient on element-sorted rows (the contract of qmll_sorf_energy_sorted) with the in-row part of
+// the Walsh-Hadamard transforms on the half-precision matrix cores, for d = 64 or 128 and one or two transforms per stack.
+//
+// H_d = H_{d/16} (x) H_16.  A wavefront carries 16 atoms through a stack.  v_mfma_f32_16x16x32_f16 multiplies the
+// +-1 block H_16 (exact in fp16) with a 16 x 16 block of the vectors (index within the block x atom), each fp32 entry
+// as two fp16 parts side by side along k: 16 high parts and 16 low parts fill its k = 32, so ONE instruction is one
+// 16-point transform of 16 atoms with fp32 accumulation.  Its accumulators hold, per lane, four entries of one atom
+// (rows 4 (lane / 16) .. + 3); with d/16 of them a lane holds the remaining log2(d/16) index bits in its own registers,
+// where they are plain additions, and the accumulator layout is the operand layout of the transposed transform (a
+// lane's four entries, high and low, are its eight k values), so nothing ever crosses lanes.
+//
+// The first operand of a stack never changes but for the signs of its diagonal: x is split once per atom, and the
+// signs go into the H_16 block, which is prepared per model (qmll_sorf_signs: a block per (element, stack, transform), the
+// diagonal must hold +-1) and moved into LDS by direct loads, a round ahead.  The gradient is split per stack (a
+// conversion, a mixed-precision subtraction and a conversion per value); both parts are rounded to nearest, so a
+// value keeps 2^-24 of itself, as in fp32.  Power-of-two scales keep everything in fp16's range: x per atom
+// (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per model.
+//
+// Instruction issue bounds it, as it does the kernel without matrix instructions (sorf_energy_rows_kernel, which at
+// d = 128 spends 162 vector instructions per 4 atoms and stack, 64 of them cross-lane ones at half rate): here 16 atoms
+// and a stack take 320 plain, 64 conversion and 64 transcendental vector instructions and 16 matrix instructions, and
+// the matrix instructions take issue time of their own (giving one butterfly stage of either side to them leaves the
+// time as it was, giving them two makes it 16 % longer).  Two tiles of atoms per wavefront, one stack per barrier,
+// eight wavefronts per workgroup and four wavefronts per SIMD (with spills) were measured too: 0 to 4 % slower.
+// Measured, with the gradient / energies only, rows kernel -> this one: 86016 atoms, d = 128, 128 stacks 870 -> 694 us /
+// 478 -> 327 us; 131072 x 128 x 64: 690 -> 513 / 383 -> 239; 86016 x 64 x 128: 420 -> 325 / 255 -> 155; two
+// transforms, 32032 x 128 x 32: 168 -> 135 / 90 -> 69.  (At d = 256 the registers leave two wavefronts per SIMD and
+// it is no faster: 880 -> 890 us, so the rows kernel stays.)
+#include <type_traits>
+
+#include "qmll_common.h"
+
+namespace {
+
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef float f2_t __attribute__((ext_vector_type(2)));
+
+constexpr int SM_WAVES = 4;                  // wavefronts per workgroup
+constexpr int SM_ATOMS = 16 * SM_WAVES;
+constexpr float INV2PI = 0.15915494309189535f;
+constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are taken off the sine argument first
+
+template <int NB>
+constexpr int log2nb() { return NB == 4 ? 2 : 3; }
+
+// one 16-point block operand: half t of lane (i, q) is sign * H_16[i][4q + t % 4]
+__device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h) & 1; }
+
+// images [ne][S][T][NB][64 lanes][8 halves]; bad counts diagonal entries that are not +-1
+template <int D>
+__global__ __launch_bounds__(256) void sorf_signs_kernel(const float* __restrict__ Dmat, int T, int S, half8_t* __restrict__ images,
+                                                         int* __restrict__ bad) {
+    constexpr int NB = D / 16;
+    const int s = blockIdx.x, m = blockIdx.y, e = blockIdx.z;
+    const float* row = Dmat + (((size_t)e * T + m) * S + s) * D;
+    half8_t* dst = images + (((size_t)e * S + s) * T + m) * NB * 64;
+    for (int t = threadIdx.x; t < NB * 64; t += 256) {
+        const int b = t >> 6, lane = t & 63, i = lane & 15, q = lane >> 4;
+        half8_t v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float sd = row[16 * b + 4 * q + r];
+            const _Float16 hv = (_Float16)(h16_negative(i, 4 * q + r) ? -sd : sd);
+            v[r] = hv;
+            v[r + 4] = hv;
+            if (i == 0 && fabsf(sd) != 1.0f) atomicAdd(bad, 1);
+        }
+        dst[t] = v;
+    }
+}
+
+// alpha 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
+__global__ __launch_bounds__(1024) void sorf_alpha_kernel(const float* __restrict__ alpha, int F, int lognb, float* __restrict__ out) {
+    __shared__ float wmax[16];
+    float m = 0.0f;
+    for (int t = threadIdx.x; t < F; t += 1024) m = fmaxf(m, finite_abs(alpha[t]));
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = wmax[0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) m = fmaxf(m, wmax[w]);
+    const int k = max(scale_exponent(m) - lognb, -126);
+    const float sc = pow2i(k);
+    for (int t = threadIdx.x; t < F; t += 1024) out[t] = alpha[t] * sc;
+    if (threadIdx.x == 0) out[F] = pow2i(-k);
+}
+
+// butterflies over the block index
+template <int NB>
+__device__ __forceinline__ void block_stages(f4_t (&v)[NB]) {
+#pragma unroll
+    for (int h = 1; h < NB; h <<= 1) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if ((b & h) == 0) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float x = v[b][r], y = v[b + h][r];
+                    v[b][r] = x + y;
+                    v[b + h][r] = x - y;
+                }
+            }
+        }
+    }
+}
+
+// v minus one half of a packed pair, in one instruction (written out, the compiler converts and subtracts: two)
+__device__ __forceinline__ float minus_low(float v, half2_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    return r;
+}
+__device__ __forceinline__ float minus_high(float v, half2_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    return r;
+}
+
+// four values as the lane's eight k entries of an operand: high parts, then low parts, both rounded to nearest
+__device__ __forceinline__ half8_t split4(f4_t v) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float t = v[r];
+        asm("" : "+v"(t));        // the value as it was rounded to fp32: see split_f16
+        v[r] = t;
+    }
+    const half2_t h0 = __builtin_convertvector((f2_t){v[0], v[1]}, half2_t), h1 = __builtin_convertvector((f2_t){v[2], v[3]}, half2_t);
+    const half2_t l0 = __builtin_convertvector((f2_t){minus_low(v[0], h0), minus_high(v[1], h0)}, half2_t);
+    const half2_t l1 = __builtin_convertvector((f2_t){minus_low(v[2], h1), minus_high(v[3], h1)}, half2_t);
+    return (half8_t){h0[0], h0[1], h1[0], h1[1], l0[0], l0[1], l1[0], l1[1]};
+}
+
+template <int D, int T>
+struct StackBuffer {      // what a stack needs, in LDS
+    static constexpr int NB = D / 16;
+    half8_t signs[T * NB * 64];
+    float diag[T * D];
+    float bias[D];        // in revolutions
+    float alpha[D];       // scaled
+};
+
+// (at least two wavefronts per SIMD: with up to 256 registers the compiler lets the matrix instructions write vector
+// registers directly; asked for fewer it goes through accumulator registers, a move per value)
+template <int D, bool WITH_GRAD, int T>
+__global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void sorf_energy_matrix_kernel(
+    const float* __restrict__ x, const int* __restrict__ type_offsets, const int* __restrict__ out_index,
+    const float* __restrict__ Dmat, const half8_t* __restrict__ images, const float* __restrict__ bias_rev,
+    const float* __restrict__ alpha_scaled, const float* __restrict__ bias_absmax, int ne, int A, int S, float scale, float normf,
+    float* __restrict__ e_slots, float* __restrict__ gx) {
+    constexpr int NB = D / 16;
+    using Buffer = StackBuffer<D, T>;
+    // two buffers as two arrays: the compiler then knows that loads into one do not touch what is read from the other
+    constexpr int SPB = D * T <= 128 ? 2 : 1;            // stacks per buffer: one barrier for so many (and 3 workgroups in LDS)
+    __shared__ __attribute__((aligned(16))) Buffer buf0[SPB], buf1[SPB];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, q = lane >> 4;
+
+    int type = -1, row0 = 0, rows = 0;
+    {
+        int b = blockIdx.x;
+        for (int t = 0; t < ne; ++t) {
+            const int o0 = type_offsets[t], o1 = type_offsets[t + 1];
+            const int nt = (o1 - o0 + SM_ATOMS - 1) / SM_ATOMS;
+            if (b < nt) {
+                type = t;
+                row0 = o0 + b * SM_ATOMS;
+                rows = min(SM_ATOMS, o1 - row0);
+                break;
+            }
+            b -= nt;
+        }
+        if (type < 0) {
+            // a workgroup past the last tile: its share of the gradient rows of atoms of unknown elements, which are zero
+            if constexpr (WITH_GRAD) {
+                const int spare = b, nspare = (int)gridDim.x - ((int)blockIdx.x - b);
+                for (int r = type_offsets[ne] + spare; r < A; r += nspare)
+                    for (int c = tid; c < D; c += 64 * SM_WAVES) gx[(size_t)r * D + c] = 0.0f;
+            }
+            return;
+        }
+    }
+    const float* Dt = Dmat + (size_t)type * T * S * D;
+    const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
+    const float* bt = bias_rev + (size_t)type * S * D;
+
+    // stack s into a buffer: direct global-to-LDS loads of 16 bytes per lane, in 1 KiB blocks shared out over the wavefronts
+    auto load16 = [&](const void* src, void* dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    };
+    const unsigned lane16 = (unsigned)lane * 16u;
+    auto fetch = [&](int s, Buffer& to) {
+        const unsigned char* src = it + (size_t)s * (T * NB * 1024);
+        unsigned char* dst = reinterpret_cast<unsigned char*>(to.signs);
+#pragma unroll
+        for (int u = 0; u < T * NB; u += SM_WAVES) load16(src + (u + wave) * 1024 + lane16, dst + (u + wave) * 1024);
+        if (lane < D / 4) {      // a row of D floats
+            if (wave == 0) load16(bt + (size_t)s * D + lane * 4, to.bias);
+            if (wave == 1) load16(alpha_scaled + (size_t)s * D + lane * 4, to.alpha);
+            if constexpr (WITH_GRAD) {
+                if (wave == 2) load16(Dt + (size_t)s * D + lane * 4, to.diag);
+                if (T == 2 && wave == 3) load16(Dt + ((size_t)S + s) * D + lane * 4, to.diag + (T - 1) * D);
+            }
+        }
+    };
+    auto fetch_all = [&](int s, Buffer (&to)[SPB]) {
+#pragma unroll
+        for (int k = 0; k < SPB; ++k)
+            if (s + k < S) fetch(s + k, to[k]);
+    };
+    fetch_all(0, buf0);
+
+    const int first = 16 * wave;                         // of this wavefront's atoms
+    const bool live = first < rows;                      // of the whole wavefront
+    const bool aok = first + col < rows;
+
+    // x in revolutions, split behind the atom's power of two
+    half8_t xop[NB];
+    float inv;
+    bool track;
+    {
+        const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
+        f4_t xv[NB];
+        const float xs = scale * INV2PI;
+        float sum = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            xv[b] = *reinterpret_cast<const f4_t*>(xr + 16 * b);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                xv[b][r] = aok ? xv[b][r] * xs : 0.0f;
+                sum += fabsf(xv[b][r]);
+            }
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        // every argument is at most sum |x| (times sqrt(d) for a second transform) + |bias|: where that stays below
+        // UMAX no stack looks at its arguments
+        const float bound = fmaf(sum, T == 2 ? (float)(1 << (log2nb<NB>() / 2 + 3)) : 1.0f, *bias_absmax * INV2PI);
+        track = __any(!(bound <= UMAX));
+        const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
+        const float sx = pow2i(kx);
+        inv = pow2i(-kx);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) xv[b][r] *= sx;
+            xop[b] = split4(xv[b]);
+        }
+    }
+    // the plain H_16 block, and the one behind the second transform's adjoint, scaled back into fp16's range
+    constexpr int BACK = 4 + log2nb<NB>() - 1;
+    half8_t hop, hback;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const bool neg = h16_negative(col, 4 * q + (t & 3));
+        hop[t] = neg ? (_Float16)-1.0f : (_Float16)1.0f;
+        hback[t] = neg ? (_Float16)(-1.0f / (1 << BACK)) : (_Float16)(1.0f / (1 << BACK));
+    }
+    const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f4_t acc[NB];
+    float energy = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = zero;
+
+    auto stack = [&](const Buffer& B) {
+        const half8_t* signs = B.signs + lane;
+        f4_t v[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const half8_t a = signs[b * 64];
+            v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xop[b], zero, 0, 0, 0);
+        }
+        block_stages<NB>(v);
+        if constexpr (T == 2) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const half8_t a = signs[(NB + b) * 64];
+                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, split4(v[b]), zero, 0, 0, 0);
+            }
+            block_stages<NB>(v);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const f4_t bv = *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[b][r] = fmaf(v[b][r], inv, bv[r]);
+        }
+        if (__builtin_expect(track, 0)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (fabsf(v[b][r]) > UMAX) v[b][r] -= rintf(v[b][r]);      // exact
+        }
+        float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const f4_t av = *reinterpret_cast<const f4_t*>(B.alpha + 16 * b + 4 * q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float u = v[b][r];
+                part = fmaf(av[r], __builtin_amdgcn_cosf(u), part);
+                if constexpr (WITH_GRAD) v[b][r] = av[r] * __builtin_amdgcn_sinf(u);
+            }
+        }
+        energy += part;
+        if constexpr (WITH_GRAD) {
+            block_stages<NB>(v);
+            if constexpr (T == 2) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + D + 16 * b + 4 * q);
+                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hback, split4(v[b]), zero, 0, 0, 0) * dv;
+                }
+                block_stages<NB>(v);
+            }
+            // summed from zero and added by the vector unit: the matrix instruction aligns its products to the
+            // accumulator it is given, and against a sum over many stacks their low bits would be cut off
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hop, split4(v[b]), zero, 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + 16 * b + 4 * q);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(v[b][r], dv[r], acc[b][r]);
+            }
+        }
+    };
+    auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB]) {
+        // these stacks' data has landed (every wavefront waits for its own loads, then for the others), and the
+        // other buffer, read in the round before, is free
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        fetch_all(s + SPB, other);
+        if (!live) return;
+#pragma unroll
+        for (int k = 0; k < SPB; ++k)
+            if (s + k < S) stack(cur[k]);
+    };
+    for (int s = 0; s < S; s += 2 * SPB) {
+        round(s, buf0, buf1);
+        if (s + SPB < S) round(s + SPB, buf1, buf0);
+    }
+
+    const float inv_alpha = alpha_scaled[(size_t)S * D];
+    energy += __shfl_xor(energy, 16, 64);
+    energy += __shfl_xor(energy, 32, 64);
+    if (!aok) return;
+    const int a = row0 + first + col;
+    if (q == 0) e_slots[out_index[a]] = energy * inv_alpha * normf;
+    if constexpr (WITH_GRAD) {
+        const float gs = -scale * normf * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
+        float* gr = gx + (size_t)a * D + 4 * q;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_t*>(gr + 16 * b) = acc[b] * gs;
+    }
+}
+
+}  // namespace
+
+// One wavefront takes 16 atoms through all stacks, so the time goes in steps of 16 atoms on every SIMD (16384): 2 w x 25 us
+// per 64 stacks at d = 128 with w wavefronts per SIMD (54 w at w = 1), where the rows kernel takes 4.55 us per 1000 atoms.  A
+// step that is mostly empty is where that one is faster.  Measured lines (64 stacks, atoms from which this kernel wins):
+// with the gradient 28000 for w = 2, 39000 for w = 3, 53000 for w = 4, always for w >= 5; energies only 24000, then always;
+// the same within 2000 atoms at d = 64 and with two transforms.
+extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
+    if (qmll_sorf_signs_bytes(ne, T, S, d) == 0) return 0;
+    constexpr int STEP = 16 * 1024;
+    const int w = A / STEP + (A % STEP != 0);
+    const int empty = (A % STEP) ? STEP - A % STEP : 0;
+    return w >= 2 && (w >= 5 || empty <= (with_grad ? 4096 : 8192) * (w - 1));
+}
+
+extern "C" size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d) {
+    if (ne <= 0 || S <= 0 || (T != 1 && T != 2) || (d != 64 && d != 128)) return 0;
+    return (size_t)ne * T * S * (d / 16) * 1024 + 16;
+}
+
+extern "C" int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void* out, size_t out_bytes, qmll_stream_t stream) {
+    QMLL_REQUIRE(qmll_sorf_signs_bytes(ne, T, S, d) > 0, QMLL_ERR_INVALID, "qmll_sorf_signs: no kernel takes ne=%d T=%d S=%d d=%d",
+                 ne, T, S, d);
+    QMLL_REQUIRE(D && out && ((uintptr_t)out & 15) == 0, QMLL_ERR_INVALID, "qmll_sorf_signs: null or misaligned pointer");
+    QMLL_REQUIRE(out_bytes >= qmll_sorf_signs_bytes(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: output of %zu bytes, %zu are needed",
+                 out_bytes, qmll_sorf_signs_bytes(ne, T, S, d));
+    QMLL_REQUIRE(ne <= 65535, QMLL_ERR_INVALID, "qmll_sorf_signs: ne=%d too large", ne);
+    half8_t* images = (half8_t*)out;
+    int* bad = (int*)((char*)out + (size_t)ne * T * S * (d / 16) * 1024);
+    const dim3 grid(S, T, ne);
+    hipStream_t st = (hipStream_t)stream;
+    if (d == 64) hipLaunchKernelGGL(sorf_signs_kernel<64>, grid, dim3(256), 0, st, D, T, S, images, bad);
+    else hipLaunchKernelGGL(sorf_signs_kernel<128>, grid, dim3(256), 0, st, D, T, S, images, bad);
+    QMLL_CHECK_LAUNCH("qmll_sorf_signs");
+    return QMLL_OK;
+}
+
+extern "C" int qmll_sorf_alpha(const float* alpha, int S, int d, float* out, qmll_stream_t stream) {
+    QMLL_REQUIRE(S > 0 && (d == 64 || d == 128), QMLL_ERR_INVALID, "qmll_sorf_alpha: bad size S=%d d=%d", S, d);
+    QMLL_REQUIRE(alpha && out, QMLL_ERR_INVALID, "qmll_sorf_alpha: null pointer");
+    hipLaunchKernelGGL(sorf_alpha_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, alpha, S * d, d == 64 ? 2 : 3, out);
+    QMLL_CHECK_LAUNCH("qmll_sorf_alpha");
+    return QMLL_OK;
+}
+
+extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D,
+                                       const void* signs, const float* bias_rev, const float* alpha_scaled, const float* bias_absmax,
+                                       int A, int ne, int d, int S, int T, float normalisation, float* e_slots, float* gx,
+                                       qmll_stream_t stream) {
+    QMLL_REQUIRE(A >= 0 && qmll_sorf_signs_bytes(ne, T, S, d) > 0, QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_matrix: bad size A=%d ne=%d T=%d S=%d d=%d", A, ne, T, S, d);
+    if (A == 0) return QMLL_OK;
+    QMLL_REQUIRE(x && type_offsets && sorted_slots && D && signs && bias_rev && alpha_scaled && bias_absmax && e_slots,
+                 QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: null pointer");
+    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)D | (uintptr_t)signs | (uintptr_t)bias_rev | (uintptr_t)alpha_scaled | (uintptr_t)gx) & 15) == 0,
+                 QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: every array must be 16-byte aligned");
+    float hn = 1.0f;                                     // (1 / sqrt(d)) per transform
+    for (int m = 0; m < T; ++m) hn /= sqrtf((float)d);
+    const float scale = normalisation * hn, normf = sqrtf(2.0f / ((float)S * (float)d));
+    const dim3 grid((A + SM_ATOMS - 1) / SM_ATOMS + ne + (A >= 65536 ? 64 : (A >> 10) + 1));
+    hipStream_t st = (hipStream_t)stream;
+    auto launch = [&](auto dc, auto tc) {
+        constexpr int DD = decltype(dc)::value, TT = decltype(tc)::value;
+        if (gx)
+            hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, true, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets,
+                               sorted_slots, D, (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, scale, normf,
+                               e_slots, gx);
+        else
+            hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, false, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets,
+                               sorted_slots, D, (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, scale, normf,
+                               e_slots, gx);
+    };
+    auto by_d = [&](auto tc) {
+        if (d == 64) launch(std::integral_constant<int, 64>{}, tc);
+        else launch(std::integral_constant<int, 128>{}, tc);
+    };
+    if (T == 1) by_d(std::integral_constant<int, 1>{});
+    else by_d(std::integral_constant<int, 2>{});
+    QMLL_CHECK_LAUNCH("qmll_sorf_energy_matrix");
+    return QMLL_OK;
+}

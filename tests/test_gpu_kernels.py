@@ -641,6 +641,43 @@ def test_sorted_fused_energy_matches_per_atom_oracle(T, S, d):
     close(e2, e_ref, REL_EF, "sorted energies only")
 
 
+@pytest.mark.parametrize("A,T,S,d,scale", [(1, 1, 1, 64, 1.0), (16, 1, 2, 128, 1.0), (17, 2, 3, 128, 1.0), (64, 2, 2, 64, 1.0),
+                                           (65, 1, 5, 64, 1.0), (300, 1, 4, 128, 1.0), (300, 2, 1, 128, 1.0), (90, 1, 3, 128, 3e4),
+                                           (90, 2, 3, 64, 2e3)])
+def test_sorf_matrix_kernel_at_the_edges_of_its_tiles(monkeypatch, A, T, S, d, scale):
+    """The matrix-core kernel of large batches at sizes where a tile, a workgroup or a round of two stacks is partial; rows of
+    unknown elements; arguments large enough that whole revolutions come off first; and the rows kernel where a diagonal is
+    not +-1."""
+    from qml_lightning_amd import _lib, ops
+    monkeypatch.setattr(_lib.lib(), "qmll_sorf_matrix_pays", lambda *a: 1)
+    rng = np.random.default_rng(A + S)
+    ne, F, norm = 3, S * d, 2.0
+    types = np.sort(rng.integers(0, ne + 1, A))            # ne: unknown, the tail
+    off = np.searchsorted(types, np.arange(ne + 1)).astype(np.int32)
+    x = (rng.normal(size=(A, d)) * scale).astype(np.float32)
+    D = np.where(rng.uniform(-1, 1, (ne, T, S, d)) > 0, 1.0, -1.0).astype(np.float32)
+    b = rng.uniform(0, 2 * np.pi, (ne, F)).astype(np.float32)
+    alpha = rng.normal(size=F).astype(np.float32)
+    slots = rng.permutation(A).astype(np.int32)
+    tol = 2e-5 * max(1.0, scale)                           # an argument keeps 2^-24 of itself
+    for diagonal in (D, D * np.float32(1.5)):
+        e_ref, g_ref = np.zeros(A), np.zeros((A, d))
+        for a_ in range(int(off[ne])):
+            t_ = types[a_]
+            c = sorf.sorf_coefficients(x[a_][None, :].astype(np.float64), diagonal[t_], norm).reshape(1, F)
+            e_ref[slots[a_]] = (np.sqrt(2.0 / F) * np.cos(c + b[t_]) * alpha).sum()
+            gc = -np.sqrt(2.0 / F) * np.sin(c + b[t_]) * alpha
+            g_ref[a_] = sorf.sorf_adjoint(gc.reshape(1, S, d), diagonal[t_], norm)[0]
+        Dt, bt, at = t32(diagonal), t32(b), t32(alpha)
+        assert (ops.sorf_signs(Dt) is not None) == (diagonal is D)
+        for grad in (True, False):
+            e, gx = ops.sorf_energy_sorted(t32(x), ti32(off), ti32(slots), Dt, bt, at, norm, T, A, with_grad=grad)
+            assert np.abs(e.cpu().numpy() - e_ref).max() <= tol * max(1.0, np.abs(e_ref).max())
+            if grad:
+                assert np.abs(gx.cpu().numpy() - g_ref).max() <= tol * max(1.0, np.abs(g_ref).max())
+                assert (gx[int(off[ne]):] == 0).all()
+
+
 # ---------------------------------------------------------------------------------------
 @pytest.mark.parametrize("M,F", [(37, 24), (300, 128), (1000, 384), (513, 200), (40, 2176), (33, 3000), (20, 4224),
                                  (18, 1100), (25, 8200)])
