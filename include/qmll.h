@@ -210,20 +210,6 @@ int qmll_derivative_features_typed(const qmll_df_element* elements, int ne, doub
 int qmll_derivative_features_rows(const qmll_df_element* elements, int ne, double normalisation, const int* row_offsets, int n,
                                   int d, int S, int T, int nmol, int overwrite, double* G, qmll_stream_t stream);
 
-/* ---- force rows of a training batch without the combinations that vanish ------------------------- */
-/* A molecule's force rows (qml_lightning/models/kernel.py:167-170) satisfy three (periodic) or up to six linear relations,
- * its translations and rotations.  qmll_rigid_modes builds per molecule the orthogonal transformation Q whose transpose
- * maps them onto the first modes[m] of its 3 natoms[m] rows; Z^T Z and Z^T y are the same for the rows Q^T G without
- * those.  X f32 [B,n,3] (real atoms first), natoms / modes i32 [B] (modes: 3 translations plus the number of
- * independent rotations to take, at most 6), row_offsets i32 [B+1] (running sum of 3 natoms - modes), work: device memory
- * of qmll_rigid_workspace_bytes(B, n) for Q; forces f64 [B,n,3] or NULL -> targets f64 [row_offsets[B]] = the rows of
- * Q^T y.  qmll_rigid_rows applies Q^T in place to the projected Jacobian rows grad f32 [A,3n,d] of the atoms in
- * slots i32 [A] (molecule = slot / n); the rows that remain move to the front of each atom's block. */
-size_t qmll_rigid_workspace_bytes(int B, int n);
-int qmll_rigid_modes(const float* X, const int* natoms, const int* modes, const int* row_offsets, int B, int n, double* work,
-                     size_t work_bytes, const double* forces, double* targets, qmll_stream_t stream);
-int qmll_rigid_rows(float* grad, const int* slots, const int* natoms, const int* modes, const double* work, int A, int B, int n,
-                    int d, qmll_stream_t stream);
 /* First atom of every molecule within each element's part of the element-sorted slots (slot / n = molecule, ascending
  * within an element): seg i32 [ne][B+1], relative to the element's first atom. */
 int qmll_typed_segments(const int* sorted_slots, const int* type_offsets, int ne, int B, int n, int* seg, qmll_stream_t stream);

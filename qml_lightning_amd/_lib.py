@@ -57,9 +57,6 @@ PROTOTYPES = {
     "qmll_derivative_features": [P, c_double, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
     "qmll_derivative_features_typed": [POINTER(DfElement), c_int, c_double, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
     "qmll_derivative_features_rows": [POINTER(DfElement), c_int, c_double, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P],
-    "qmll_rigid_workspace_bytes": [c_int, c_int],
-    "qmll_rigid_modes": [P, P, P, P, c_int, c_int, P, c_size_t, P, P, P],
-    "qmll_rigid_rows": [P, P, P, P, P, c_int, c_int, c_int, c_int, P],
     "qmll_typed_segments": [P, P, c_int, c_int, c_int, P, P],
     "qmll_sorf_energy_fused": [P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, P, P, P],
     "qmll_sorf_energy_typed": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P, P, P],
@@ -103,7 +100,7 @@ PROTOTYPES = {
     "qmll_probe_rate": [c_int, c_int, c_int, P, P],
     "qmll_probe_mix": [c_int, c_int, c_int, P, P],
 }
-_RESTYPES = {"qmll_last_error": c_char_p, "qmll_rigid_workspace_bytes": c_size_t, "qmll_sorf_signs_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
+_RESTYPES = {"qmll_last_error": c_char_p, "qmll_sorf_signs_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
              "qmll_cholesky_workspace_bytes": c_size_t, "qmll_gram_workspace_bytes": c_size_t,
              "qmll_probe_out_bytes": c_size_t, "qmll_probe_rate": c_double,
              "qmll_probe_mix": c_double}

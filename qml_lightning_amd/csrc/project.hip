@@ -1179,6 +1179,22 @@ int* scratch_of_current_device() {
     }
     return scratch_ptr[dev];
 }
+// first atom of every molecule within each element's part of the sorted slots
+__global__ void typed_segments_kernel(const int* __restrict__ slots, const int* __restrict__ type_offsets, int ne, int B, int n,
+                                      int* __restrict__ seg) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ne * (B + 1)) return;
+    const int e = t / (B + 1), m = t - e * (B + 1);
+    const int o0 = type_offsets[e], o1 = type_offsets[e + 1];
+    int lo = o0, hi = o1;                    // first atom whose slot is not before molecule m
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (slots[mid] < m * n) lo = mid + 1;
+        else hi = mid;
+    }
+    seg[t] = lo - o0;
+}
+
 }  // namespace
 
 extern "C" int qmll_sort_by_type_noalloc(const int* types, const int* slots, int A, int ne, int* sorted_slots,
@@ -1408,5 +1424,15 @@ extern "C" int qmll_project_typed_backward_sums(const float* gx, const int* sort
         hipLaunchKernelGGL((typed_gemm_kernel<true, false, PN>), grid, dim3(PT), 0, (hipStream_t)stream, gx, d,
                            (const int*)nullptr, reductors, (size_t)R * d, d, g_rep, R, sorted_slots, type_offsets, ne, d, R);
     QMLL_CHECK_LAUNCH("qmll_project_typed_backward");
+    return QMLL_OK;
+}
+
+extern "C" int qmll_typed_segments(const int* sorted_slots, const int* type_offsets, int ne, int B, int n, int* seg,
+                                   qmll_stream_t stream) {
+    QMLL_REQUIRE(ne > 0 && B >= 0 && n > 0, QMLL_ERR_INVALID, "qmll_typed_segments: bad size ne=%d B=%d n=%d", ne, B, n);
+    QMLL_REQUIRE(sorted_slots && type_offsets && seg, QMLL_ERR_INVALID, "qmll_typed_segments: null pointer");
+    hipLaunchKernelGGL(typed_segments_kernel, dim3((ne * (B + 1) + 255) / 256), dim3(256), 0, (hipStream_t)stream, sorted_slots,
+                       type_offsets, ne, B, n, seg);
+    QMLL_CHECK_LAUNCH("qmll_typed_segments");
     return QMLL_OK;
 }

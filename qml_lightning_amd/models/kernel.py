@@ -89,7 +89,7 @@ class BaseKernel():
     # -- to be provided by the feature model -------------------------------------------
     def finish_features(self, derivative_matrix=None, overwrite=False, feature_matrix=None, rows=None):
         """Called once per batch after the loop over elements; models that queue work in
-        calculate_features run it here.  rows: the batch's row table (`_drop_rigid_rows`), or None."""
+        calculate_features run it here.  rows: the batch's row table, or None."""
         return None
 
     def writes_force_rows(self):
@@ -169,36 +169,27 @@ class BaseKernel():
                 sub_grad = g_all[o0 * 3 * n:o1 * 3 * n].view(o1 - o0, n, 3, -1) if with_forces else None
                 items.append((order[t], mol_of_atom[o0:o1], x_all[o0:o1], sub_grad,
                               segments[t] if with_forces else None))
-            if with_forces:
-                return {'B': B, 'n': n, 'device': coordinates.device, 'items': items, 'slots': slots,
-                        'gradient_rows': g_all.view(-1, n, 3, self.reductors.shape[2])}
         return {'B': B, 'n': n, 'device': coordinates.device, 'items': items}
 
     def _training_batch(self, data, has_E, has_F):
-        """(projected rows, targets) of a formatted training batch.  With forces, the rows of padded slots and
-        the combinations of a molecule's force rows that vanish identically (its translations, and without
-        cells its rotations) are left out of both: an orthogonal transformation of each molecule's rows
-        and targets, which leaves Z^T Z and Z^T y as they are, and up to half of the rows less."""
-        proj = self._batch_projected(data, has_F)
-        B = data['charges'].shape[0]
-        modes = data.get('rigid_modes')
-        if not has_F or modes is None or not self.writes_force_rows() or 'gradient_rows' not in proj:
-            return proj, self._targets(data, B, has_E, has_F)
-        counts, modes = modes
-        per_molecule = (3 * counts - modes).astype(np.int32)
-        table = np.concatenate((modes, [0], np.cumsum(per_molecule))).astype(np.int32)
-        dev = proj['device']
-        table = torch.from_numpy(table).to(dev)
+        """(projected rows, targets) of a formatted training batch.  The force rows of padded slots are zero, and so are
+        their targets: where a batch has some, both are left out (proj['rows']), which leaves Z^T Z and Z^T y
+        as they are."""
+        proj, targets = self._batch_projected(data, has_F), self._targets(data, data['charges'].shape[0], has_E, has_F)
+        if not has_F or not self.writes_force_rows():
+            return proj, targets
+        B, n = proj['B'], proj['n']
+        per_molecule = 3 * np.asarray(data['host_counts'], dtype=np.int64)
         nrows = int(per_molecule.sum())
-        targets = torch.empty((B + nrows, 1), dtype=torch.float64, device=dev)
-        if has_E:
-            targets[:B, 0] = data['energies']
-        else:
-            targets[:B].zero_()
-        ops.rigid_rows(proj.pop('gradient_rows'), proj.pop('slots'), data['coordinates'], data['natom_counts'], table[:B],
-                       table[B:], data['forces'].contiguous(), targets[B:])
-        proj['rows'] = {'offsets': table[B:], 'count': nrows, 'most': int(per_molecule.max()) if B else 0}
-        return proj, targets
+        if nrows == 3 * B * n or nrows == 0 or nrows >= 1 << 31:
+            return proj, targets
+        table = np.concatenate(([0], np.cumsum(per_molecule)))
+        # molecule m's rows move up by what the molecules before it have less than 3n rows each
+        first = B + 3 * n * np.arange(B) - table[:-1]
+        table, first, per_molecule = (torch.from_numpy(t).to(proj['device']) for t in (table, first, per_molecule))
+        source = torch.arange(nrows, device=proj['device']) + torch.repeat_interleave(first, per_molecule, output_size=nrows)
+        proj['rows'] = {'offsets': table.int(), 'count': nrows, 'most': 3 * int(max(data['host_counts']))}
+        return proj, torch.cat((targets[:B], targets.index_select(0, source)))
 
     def _rows_from_projected(self, proj, with_forces, zero_energy_rows=False):
         """fp64 row matrix [B (+ B*n*3), F] from the projected rows of one batch, at the current
@@ -714,33 +705,11 @@ class BaseKernel():
             if self.convert_hartree2kcal():
                 forces = forces * self.hartree2kcalmol
             data['forces'] = forces * mask[:, :, None]                      # padded slots carry no target
-            data['rigid_modes'] = self._rigid_modes(np.asarray(X), hostmask.sum(axis=1), cells is not None)
+            data['host_counts'] = hostmask.sum(axis=1)
         if cells is not None:
             data['cells'] = torch.from_numpy(np.asarray(cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
             data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
         return data
-
-    @staticmethod
-    def _rigid_modes(coordinates, counts, periodic):
-        """(counts, modes) int32 [B]: how many independent translations and rotations each molecule of a
-        zero-padded host batch has: 3 in a periodic cell, else 6; 5 for two atoms, 3 for one.  A molecule of
-        three or more atoms on a line (mean square distance from the line below 1e-3 of that from the centre)
-        keeps all of its rows (0): its third rotation is undefined, and the angular terms' derivatives are
-        singular there."""
-        counts = np.asarray(counts, dtype=np.int32)
-        modes = np.where(counts > 0, 3, 0).astype(np.int32)
-        if periodic or coordinates.shape[1] < 2:
-            return counts, modes
-        X = coordinates.astype(np.float32, copy=False)
-        live = (np.arange(X.shape[1]) < counts[:, None])[:, :, None]
-        d = np.where(live, X - (X * live).sum(axis=1, keepdims=True) / np.maximum(counts, 1)[:, None, None], 0.0)
-        T = np.matmul(d.transpose(0, 2, 1), d).astype(np.float64)
-        trace = T[:, 0, 0] + T[:, 1, 1] + T[:, 2, 2]
-        # sum of the principal 2 x 2 minors = l1 l2 + l1 l3 + l2 l3, about trace (l2 + l3) for a line
-        minors = 0.5 * (trace * trace - (T * T).sum(axis=(1, 2)))
-        modes[counts == 2] = 5
-        modes[counts >= 3] = np.where(minors > 1e-3 * trace * trace, 6, 0)[counts >= 3]
-        return counts, modes
 
     def _element_counts(self, flat_charges):
         """{element: number of atoms} of a batch from the host copy of its charges (one bincount)."""
@@ -830,7 +799,7 @@ class BaseKernel():
             if self.convert_hartree2kcal():
                 forces *= self.hartree2kcalmol
             data['forces'] = torch.from_numpy(forces).to(dev)
-            data['rigid_modes'] = self._rigid_modes(coords, counts, cells is not None)
+            data['host_counts'] = counts
         if cells is not None:
             data['cells'] = torch.from_numpy(np.asarray(cells, dtype=np.float32).reshape(zbatch, 3, 3)).to(dev)
             data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(zbatch, 3, 3)).to(dev)

@@ -333,34 +333,6 @@ def typed_segments(sorted_slots, type_offsets, B, n):
     return seg
 
 
-def rigid_rows(grad, sorted_slots, X, natoms, modes, row_offsets, forces=None, targets=None):
-    """The projected Jacobian rows grad f32 [A,n,3,d] with Q^T applied in place, Q the orthogonal
-    transformation that maps modes[m] vanishing combinations (translations, rotations) of molecule m's
-    3 natoms[m] force rows onto its first rows; the rows that remain move to the front of each atom's block.
-    forces f64 [B,n,3] -> targets f64 [row_offsets[B]] = the same rows of Q^T y."""
-    A, n, _, d = grad.shape
-    B = int(natoms.shape[0])
-    if grad.dtype != torch.float32 or not grad.is_contiguous() or int(sorted_slots.shape[0]) != A:
-        raise RuntimeError("rigid_rows: grad %s for %d atoms" % (tuple(grad.shape), int(sorted_slots.shape[0])))
-    if (forces is None) != (targets is None):
-        raise RuntimeError("rigid_rows: forces and targets must both be given or both be None")
-    X, natoms, modes, row_offsets, sorted_slots = _f32(X), _i32(natoms), _i32(modes), _i32(row_offsets), _i32(sorted_slots)
-    if tuple(X.shape) != (B, n, 3) or modes.numel() != B or row_offsets.numel() != B + 1:
-        raise RuntimeError("rigid_rows: coordinates %s, %d modes, %d row offsets for %d molecules"
-                           % (tuple(X.shape), modes.numel(), row_offsets.numel(), B))
-    if forces is not None and (forces.dtype != torch.float64 or not forces.is_contiguous() or forces.numel() != B * n * 3
-                               or targets.dtype != torch.float64 or not targets.is_contiguous()):
-        raise RuntimeError("rigid_rows: forces and targets must be contiguous float64 tensors")
-    L = _lib.lib()
-    nbytes = int(L.qmll_rigid_workspace_bytes(B, n))
-    work = torch.empty(max(nbytes // 8, 1), dtype=torch.float64, device=grad.device)
-    check(L.qmll_rigid_modes(_ptr(X), _ptr(natoms), _ptr(modes), _ptr(row_offsets), B, n, _ptr(work), nbytes, _ptr(forces),
-                             _ptr(targets), _stream()), "qmll_rigid_modes")
-    check(L.qmll_rigid_rows(_ptr(grad), _ptr(sorted_slots), _ptr(natoms), _ptr(modes), _ptr(work), A, B, n, d, _stream()),
-          "qmll_rigid_rows")
-    return grad
-
-
 def derivative_features_typed(items, normalisation, G, overwrite=False, nmol=None, n=None, row_offsets=None):
     """G += force-feature rows of every element of the batch in one launch.  items: one tuple
     (cos_derivs f64 [A_e,F], D f32 [T,S,d], input_derivatives f32 [A_e,n,3,d], mol_index i32 [A_e],
