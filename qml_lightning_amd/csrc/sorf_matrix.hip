@@ -22,10 +22,15 @@
 // the matrix instructions take issue time of their own (giving one butterfly stage of either side to them leaves the
 // time as it was, giving them two makes it 16 % longer).  Two tiles of atoms per wavefront, one stack per barrier,
 // eight wavefronts per workgroup and four wavefronts per SIMD (with spills) were measured too: 0 to 4 % slower.
-// Measured, with the gradient / energies only, rows kernel -> this one: 86016 atoms, d = 128, 128 stacks 870 -> 694 us /
-// 478 -> 327 us; 131072 x 128 x 64: 690 -> 513 / 383 -> 239; 86016 x 64 x 128: 420 -> 325 / 255 -> 155; two
-// transforms, 32032 x 128 x 32: 168 -> 135 / 90 -> 69.  (At d = 256 the registers leave two wavefronts per SIMD and
-// it is no faster: 880 -> 890 us, so the rows kernel stays.)
+//
+// A tile (64 atoms of one element) through all stacks is too coarse a unit: with the three workgroups a CU holds, the last
+// of two rounds of tiles left most of the chip idle.  A workgroup takes an equal share of all (tile, round of stacks) units
+// instead; a tile that two or more shares meet in is written in parts, which sorf_parts_kernel adds up in order.
+// Measured with the gradient / energies only, rows kernel -> whole tiles -> shares, at d = 128, 128 stacks: 86016 atoms
+// 762 -> 690 -> 643 us / 457 -> 324 -> 297; 24000 atoms 222 -> 269 -> 207 / 133 -> 137 -> 97; 131500 atoms 1166 -> 1004 -> 963 /
+// 698 -> 462 -> 449; 86016 x 64 x 128: 361 -> 317 -> 300 / 230 -> 149 -> 139; two transforms, 33000 x 128 x 32: 147 -> 164 -> 135 / 77 -> 81 -> 66.  (At d = 256 the
+// registers leave two wavefronts per SIMD and it is no faster: 880 -> 890 us, so the rows kernel stays.)
+#include <algorithm>
 #include <type_traits>
 
 #include "qmll_common.h"
@@ -39,6 +44,10 @@ constexpr int SM_WAVES = 4;                  // wavefronts per workgroup
 constexpr int SM_ATOMS = 16 * SM_WAVES;
 constexpr float INV2PI = 0.15915494309189535f;
 constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are taken off the sine argument first
+
+// stacks per buffer: one barrier for so many (and at least 3 workgroups in LDS)
+constexpr int stacks_per_round(int d, int T) { return d * T <= 128 ? 2 : 1; }
+constexpr int SM_CUS = 256;
 
 template <int NB>
 constexpr int log2nb() { return NB == 4 ? 2 : 3; }
@@ -141,240 +150,317 @@ struct StackBuffer {      // what a stack needs, in LDS
     float alpha[D];       // scaled
 };
 
+// Tiles of 64 atoms of one element; a share of the launch is a range of (tile, round of SPB stacks) units, tile after tile.
+__device__ __forceinline__ int tile_count(const int* __restrict__ type_offsets, int ne) {
+    int n = 0;
+    for (int t = 0; t < ne; ++t) n += (type_offsets[t + 1] - type_offsets[t] + SM_ATOMS - 1) / SM_ATOMS;
+    return n;
+}
+__device__ __forceinline__ void find_tile(const int* __restrict__ type_offsets, int ne, int tile, int& type, int& row0, int& rows) {
+    type = row0 = rows = 0;
+    for (int t = 0; t < ne; ++t) {
+        const int o0 = type_offsets[t], o1 = type_offsets[t + 1], nt = (o1 - o0 + SM_ATOMS - 1) / SM_ATOMS;
+        if (tile < nt) {
+            type = t;
+            row0 = o0 + tile * SM_ATOMS;
+            rows = min(SM_ATOMS, o1 - row0);
+            return;
+        }
+        tile -= nt;
+    }
+}
+// first unit of share g; with fewer units than shares the last shares are empty, else none is
+__device__ __forceinline__ int share_begin(int g, int nshares, int ntiles, int rounds) {
+    const int units = ntiles * rounds, used = min(nshares, units);
+    return g >= used ? units : (int)((long long)units * g / used);
+}
+
 // (at least two wavefronts per SIMD: with up to 256 registers the compiler lets the matrix instructions write vector
 // registers directly; asked for fewer it goes through accumulator registers, a move per value)
 template <int D, bool WITH_GRAD, int T>
 __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void sorf_energy_matrix_kernel(
     const float* __restrict__ x, const int* __restrict__ type_offsets, const int* __restrict__ out_index,
     const float* __restrict__ Dmat, const half8_t* __restrict__ images, const float* __restrict__ bias_rev,
-    const float* __restrict__ alpha_scaled, const float* __restrict__ bias_absmax, int ne, int A, int S, float scale, float normf,
-    float* __restrict__ e_slots, float* __restrict__ gx) {
+    const float* __restrict__ alpha_scaled, const float* __restrict__ bias_absmax, int ne, int A, int S, int nshares, float scale,
+    float normf, float* __restrict__ parts, float* __restrict__ e_slots, float* __restrict__ gx) {
     constexpr int NB = D / 16;
     using Buffer = StackBuffer<D, T>;
     // two buffers as two arrays: the compiler then knows that loads into one do not touch what is read from the other
-    constexpr int SPB = D * T <= 128 ? 2 : 1;            // stacks per buffer: one barrier for so many (and 3 workgroups in LDS)
+    constexpr int SPB = stacks_per_round(D, T);
     __shared__ __attribute__((aligned(16))) Buffer buf0[SPB], buf1[SPB];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4;
+    const int rounds = (S + SPB - 1) / SPB;
 
-    int type = -1, row0 = 0, rows = 0;
-    {
-        int b = blockIdx.x;
-        for (int t = 0; t < ne; ++t) {
-            const int o0 = type_offsets[t], o1 = type_offsets[t + 1];
-            const int nt = (o1 - o0 + SM_ATOMS - 1) / SM_ATOMS;
-            if (b < nt) {
-                type = t;
-                row0 = o0 + b * SM_ATOMS;
-                rows = min(SM_ATOMS, o1 - row0);
-                break;
-            }
-            b -= nt;
+    const int ntiles = tile_count(type_offsets, ne);
+    if ((int)blockIdx.x >= nshares) {
+        // a workgroup beyond the shares: its part of the gradient rows of atoms of unknown elements, which are zero
+        if constexpr (WITH_GRAD) {
+            const int spare = (int)blockIdx.x - nshares, nspare = (int)gridDim.x - nshares;
+            for (int r = type_offsets[ne] + spare; r < A; r += nspare)
+                for (int c = tid; c < D; c += 64 * SM_WAVES) gx[(size_t)r * D + c] = 0.0f;
         }
-        if (type < 0) {
-            // a workgroup past the last tile: its share of the gradient rows of atoms of unknown elements, which are zero
-            if constexpr (WITH_GRAD) {
-                const int spare = b, nspare = (int)gridDim.x - ((int)blockIdx.x - b);
-                for (int r = type_offsets[ne] + spare; r < A; r += nspare)
-                    for (int c = tid; c < D; c += 64 * SM_WAVES) gx[(size_t)r * D + c] = 0.0f;
-            }
-            return;
-        }
+        return;
     }
-    const float* Dt = Dmat + (size_t)type * T * S * D;
-    const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
-    const float* bt = bias_rev + (size_t)type * S * D;
+    const int ubeg = share_begin(blockIdx.x, nshares, ntiles, rounds), uend = share_begin(blockIdx.x + 1, nshares, ntiles, rounds);
 
-    // stack s into a buffer: direct global-to-LDS loads of 16 bytes per lane, in 1 KiB blocks shared out over the wavefronts
-    auto load16 = [&](const void* src, void* dst) {
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-    };
-    const unsigned lane16 = (unsigned)lane * 16u;
-    auto fetch = [&](int s, Buffer& to) {
-        const unsigned char* src = it + (size_t)s * (T * NB * 1024);
-        unsigned char* dst = reinterpret_cast<unsigned char*>(to.signs);
+    for (int u = ubeg; u < uend;) {
+        const int tile = u / rounds, r0 = u - tile * rounds, r1 = min(rounds, r0 + uend - u);
+        int type, row0, rows;
+        find_tile(type_offsets, ne, tile, type, row0, rows);
+        const bool whole = r1 - r0 == rounds;
+        const size_t slot = 2 * (size_t)blockIdx.x + (u != ubeg);       // of the parts, where this is one
+        if (u != ubeg) __syncthreads();                                 // the buffers of the tile before are free
+        u += r1 - r0;
+        const int s0 = r0 * SPB, s1 = min(S, r1 * SPB);
+
+        const float* Dt = Dmat + (size_t)type * T * S * D;
+        const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
+        const float* bt = bias_rev + (size_t)type * S * D;
+
+        // stack s into a buffer: direct global-to-LDS loads of 16 bytes per lane, in 1 KiB blocks shared out over the wavefronts
+        auto load16 = [&](const void* src, void* dst) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+        };
+        const unsigned lane16 = (unsigned)lane * 16u;
+        auto fetch = [&](int s, Buffer& to) {
+            const unsigned char* src = it + (size_t)s * (T * NB * 1024);
+            unsigned char* dst = reinterpret_cast<unsigned char*>(to.signs);
 #pragma unroll
-        for (int u = 0; u < T * NB; u += SM_WAVES) load16(src + (u + wave) * 1024 + lane16, dst + (u + wave) * 1024);
-        if (lane < D / 4) {      // a row of D floats
-            if (wave == 0) load16(bt + (size_t)s * D + lane * 4, to.bias);
-            if (wave == 1) load16(alpha_scaled + (size_t)s * D + lane * 4, to.alpha);
-            if constexpr (WITH_GRAD) {
-                if (wave == 2) load16(Dt + (size_t)s * D + lane * 4, to.diag);
-                if (T == 2 && wave == 3) load16(Dt + ((size_t)S + s) * D + lane * 4, to.diag + (T - 1) * D);
+            for (int u = 0; u < T * NB; u += SM_WAVES) load16(src + (u + wave) * 1024 + lane16, dst + (u + wave) * 1024);
+            if (lane < D / 4) {      // a row of D floats
+                if (wave == 0) load16(bt + (size_t)s * D + lane * 4, to.bias);
+                if (wave == 1) load16(alpha_scaled + (size_t)s * D + lane * 4, to.alpha);
+                if constexpr (WITH_GRAD) {
+                    if (wave == 2) load16(Dt + (size_t)s * D + lane * 4, to.diag);
+                    if (T == 2 && wave == 3) load16(Dt + ((size_t)S + s) * D + lane * 4, to.diag + (T - 1) * D);
+                }
             }
-        }
-    };
-    auto fetch_all = [&](int s, Buffer (&to)[SPB]) {
+        };
+        auto fetch_all = [&](int s, Buffer (&to)[SPB]) {
 #pragma unroll
-        for (int k = 0; k < SPB; ++k)
-            if (s + k < S) fetch(s + k, to[k]);
-    };
-    fetch_all(0, buf0);
+            for (int k = 0; k < SPB; ++k)
+                if (s + k < s1) fetch(s + k, to[k]);
+        };
+        fetch_all(s0, buf0);
 
-    const int first = 16 * wave;                         // of this wavefront's atoms
-    const bool live = first < rows;                      // of the whole wavefront
-    const bool aok = first + col < rows;
+        const int first = 16 * wave;                         // of this wavefront's atoms
+        const bool live = first < rows;                      // of the whole wavefront
+        const bool aok = first + col < rows;
 
-    // x in revolutions, split behind the atom's power of two
-    half8_t xop[NB];
-    float inv;
-    bool track;
-    {
-        const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
-        f4_t xv[NB];
-        const float xs = scale * INV2PI;
-        float sum = 0.0f;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            xv[b] = *reinterpret_cast<const f4_t*>(xr + 16 * b);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                xv[b][r] = aok ? xv[b][r] * xs : 0.0f;
-                sum += fabsf(xv[b][r]);
-            }
-        }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        // every argument is at most sum |x| (times sqrt(d) for a second transform) + |bias|: where that stays below
-        // UMAX no stack looks at its arguments
-        const float bound = fmaf(sum, T == 2 ? (float)(1 << (log2nb<NB>() / 2 + 3)) : 1.0f, *bias_absmax * INV2PI);
-        track = __any(!(bound <= UMAX));
-        const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
-        const float sx = pow2i(kx);
-        inv = pow2i(-kx);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) xv[b][r] *= sx;
-            xop[b] = split4(xv[b]);
-        }
-    }
-    // the plain H_16 block, and the one behind the second transform's adjoint, scaled back into fp16's range
-    constexpr int BACK = 4 + log2nb<NB>() - 1;
-    half8_t hop, hback;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const bool neg = h16_negative(col, 4 * q + (t & 3));
-        hop[t] = neg ? (_Float16)-1.0f : (_Float16)1.0f;
-        hback[t] = neg ? (_Float16)(-1.0f / (1 << BACK)) : (_Float16)(1.0f / (1 << BACK));
-    }
-    const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f4_t acc[NB];
-    float energy = 0.0f;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = zero;
-
-    auto stack = [&](const Buffer& B) {
-        const half8_t* signs = B.signs + lane;
-        f4_t v[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const half8_t a = signs[b * 64];
-            v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xop[b], zero, 0, 0, 0);
-        }
-        block_stages<NB>(v);
-        if constexpr (T == 2) {
+        // x in revolutions, split behind the atom's power of two
+        half8_t xop[NB];
+        float inv;
+        bool track;
+        {
+            const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
+            f4_t xv[NB];
+            const float xs = scale * INV2PI;
+            float sum = 0.0f;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const half8_t a = signs[(NB + b) * 64];
-                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, split4(v[b]), zero, 0, 0, 0);
+                xv[b] = *reinterpret_cast<const f4_t*>(xr + 16 * b);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    xv[b][r] = aok ? xv[b][r] * xs : 0.0f;
+                    sum += fabsf(xv[b][r]);
+                }
             }
-            block_stages<NB>(v);
-        }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            // every argument is at most sum |x| (times sqrt(d) for a second transform) + |bias|: where that stays below
+            // UMAX no stack looks at its arguments
+            const float bound = fmaf(sum, T == 2 ? (float)(1 << (log2nb<NB>() / 2 + 3)) : 1.0f, *bias_absmax * INV2PI);
+            track = __any(!(bound <= UMAX));
+            const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
+            const float sx = pow2i(kx);
+            inv = pow2i(-kx);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const f4_t bv = *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q);
+            for (int b = 0; b < NB; ++b) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[b][r] = fmaf(v[b][r], inv, bv[r]);
-        }
-        if (__builtin_expect(track, 0)) {
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (fabsf(v[b][r]) > UMAX) v[b][r] -= rintf(v[b][r]);      // exact
-        }
-        float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const f4_t av = *reinterpret_cast<const f4_t*>(B.alpha + 16 * b + 4 * q);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float u = v[b][r];
-                part = fmaf(av[r], __builtin_amdgcn_cosf(u), part);
-                if constexpr (WITH_GRAD) v[b][r] = av[r] * __builtin_amdgcn_sinf(u);
+                for (int r = 0; r < 4; ++r) xv[b][r] *= sx;
+                xop[b] = split4(xv[b]);
             }
         }
-        energy += part;
-        if constexpr (WITH_GRAD) {
+        // the plain H_16 block, and the one behind the second transform's adjoint, scaled back into fp16's range
+        constexpr int BACK = 4 + log2nb<NB>() - 1;
+        half8_t hop, hback;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const bool neg = h16_negative(col, 4 * q + (t & 3));
+            hop[t] = neg ? (_Float16)-1.0f : (_Float16)1.0f;
+            hback[t] = neg ? (_Float16)(-1.0f / (1 << BACK)) : (_Float16)(1.0f / (1 << BACK));
+        }
+        const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        f4_t acc[NB];
+        float energy = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[b] = zero;
+
+        auto stack = [&](const Buffer& B) {
+            const half8_t* signs = B.signs + lane;
+            f4_t v[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const half8_t a = signs[b * 64];
+                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xop[b], zero, 0, 0, 0);
+            }
             block_stages<NB>(v);
             if constexpr (T == 2) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + D + 16 * b + 4 * q);
-                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hback, split4(v[b]), zero, 0, 0, 0) * dv;
+                    const half8_t a = signs[(NB + b) * 64];
+                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, split4(v[b]), zero, 0, 0, 0);
                 }
                 block_stages<NB>(v);
             }
-            // summed from zero and added by the vector unit: the matrix instruction aligns its products to the
-            // accumulator it is given, and against a sum over many stacks their low bits would be cut off
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hop, split4(v[b]), zero, 0, 0, 0);
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + 16 * b + 4 * q);
+                const f4_t bv = *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(v[b][r], dv[r], acc[b][r]);
+                for (int r = 0; r < 4; ++r) v[b][r] = fmaf(v[b][r], inv, bv[r]);
             }
+            if (__builtin_expect(track, 0)) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (fabsf(v[b][r]) > UMAX) v[b][r] -= rintf(v[b][r]);      // exact
+            }
+            float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const f4_t av = *reinterpret_cast<const f4_t*>(B.alpha + 16 * b + 4 * q);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float u = v[b][r];
+                    part = fmaf(av[r], __builtin_amdgcn_cosf(u), part);
+                    if constexpr (WITH_GRAD) v[b][r] = av[r] * __builtin_amdgcn_sinf(u);
+                }
+            }
+            energy += part;
+            if constexpr (WITH_GRAD) {
+                block_stages<NB>(v);
+                if constexpr (T == 2) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + D + 16 * b + 4 * q);
+                        v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hback, split4(v[b]), zero, 0, 0, 0) * dv;
+                    }
+                    block_stages<NB>(v);
+                }
+                // summed from zero and added by the vector unit: the matrix instruction aligns its products to the
+                // accumulator it is given, and against a sum over many stacks their low bits would be cut off
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hop, split4(v[b]), zero, 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + 16 * b + 4 * q);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(v[b][r], dv[r], acc[b][r]);
+                }
+            }
+        };
+        auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB]) {
+            // these stacks' data has landed (every wavefront waits for its own loads, then for the others), and the
+            // other buffer, read in the round before, is free
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            fetch_all(s + SPB, other);
+            if (!live) return;
+#pragma unroll
+            for (int k = 0; k < SPB; ++k)
+                if (s + k < s1) stack(cur[k]);
+        };
+        for (int s = s0; s < s1; s += 2 * SPB) {
+            round(s, buf0, buf1);
+            if (s + SPB < s1) round(s + SPB, buf1, buf0);
         }
-    };
-    auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB]) {
-        // these stacks' data has landed (every wavefront waits for its own loads, then for the others), and the
-        // other buffer, read in the round before, is free
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        fetch_all(s + SPB, other);
-        if (!live) return;
-#pragma unroll
-        for (int k = 0; k < SPB; ++k)
-            if (s + k < S) stack(cur[k]);
-    };
-    for (int s = 0; s < S; s += 2 * SPB) {
-        round(s, buf0, buf1);
-        if (s + SPB < S) round(s + SPB, buf1, buf0);
-    }
 
-    const float inv_alpha = alpha_scaled[(size_t)S * D];
-    energy += __shfl_xor(energy, 16, 64);
-    energy += __shfl_xor(energy, 32, 64);
-    if (!aok) return;
-    const int a = row0 + first + col;
-    if (q == 0) e_slots[out_index[a]] = energy * inv_alpha * normf;
-    if constexpr (WITH_GRAD) {
-        const float gs = -scale * normf * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
-        float* gr = gx + (size_t)a * D + 4 * q;
+        const float inv_alpha = alpha_scaled[(size_t)S * D];
+        energy += __shfl_xor(energy, 16, 64);
+        energy += __shfl_xor(energy, 32, 64);
+        if (!aok) continue;
+        const int in_tile = first + col;
+        if (q == 0) {
+            const float e = energy * inv_alpha * normf;
+            if (whole) e_slots[out_index[row0 + in_tile]] = e;
+            else parts[slot * SM_ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
+        }
+        if constexpr (WITH_GRAD) {
+            const float gs = -scale * normf * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
+            float* to = whole ? gx + (size_t)row0 * D : parts + slot * SM_ATOMS * (D + 1) + SM_ATOMS;
+            float* gr = to + (size_t)in_tile * D + 4 * q;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_t*>(gr + 16 * b) = acc[b] * gs;
+            for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_t*>(gr + 16 * b) = acc[b] * gs;
+        }
+    }
+}
+
+// the tiles that were cut: workgroup g adds up the parts of the tile that begins in share g and ends in a later one, in order
+template <int D, bool WITH_GRAD>
+__global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__ type_offsets, const int* __restrict__ out_index, int ne,
+                                                         int rounds, const float* __restrict__ parts, float* __restrict__ e_slots,
+                                                         float* __restrict__ gx) {
+    constexpr size_t SLOT = SM_ATOMS * (WITH_GRAD ? D + 1 : 1);
+    const int g = blockIdx.x, nshares = gridDim.x, ntiles = tile_count(type_offsets, ne);
+    const int ubeg = share_begin(g, nshares, ntiles, rounds), uend = share_begin(g + 1, nshares, ntiles, rounds);
+    if (ubeg == uend) return;
+    const int tile = (uend - 1) / rounds, tbeg = tile * rounds, tend = tbeg + rounds;
+    if (tbeg < ubeg || tend <= uend) return;
+    int last = g + 1;                                    // the share in which the tile ends
+    while (share_begin(last + 1, nshares, ntiles, rounds) < tend) ++last;
+    int type, row0, rows;
+    find_tile(type_offsets, ne, tile, type, row0, rows);
+    const float* head = parts + (2 * (size_t)g + (tbeg != ubeg)) * SLOT;
+    const float* next = parts + 2 * (size_t)(g + 1) * SLOT;
+    const int nparts = last - g;
+    for (int t = threadIdx.x; t < rows; t += 256) {
+        float v = head[t];
+        for (int b = 0; b < nparts; ++b) v += next[2 * b * SLOT + t];
+        e_slots[out_index[row0 + t]] = v;
+    }
+    if constexpr (WITH_GRAD) {
+        for (int t = threadIdx.x; t < rows * (D / 4); t += 256) {
+            f4_t v = *reinterpret_cast<const f4_t*>(head + SM_ATOMS + 4 * t);
+            for (int b = 0; b < nparts; ++b) v += *reinterpret_cast<const f4_t*>(next + 2 * b * SLOT + SM_ATOMS + 4 * t);
+            *reinterpret_cast<f4_t*>(gx + (size_t)row0 * D + 4 * t) = v;
+        }
     }
 }
 
 }  // namespace
 
-// One wavefront takes 16 atoms through all stacks, so the time goes in steps of 16 atoms on every SIMD (16384): 2 w x 25 us
-// per 64 stacks at d = 128 with w wavefronts per SIMD (54 w at w = 1), where the rows kernel takes 4.55 us per 1000 atoms.  A
-// step that is mostly empty is where that one is faster.  Measured lines (64 stacks, atoms from which this kernel wins):
-// with the gradient 28000 for w = 2, 39000 for w = 3, 53000 for w = 4, always for w >= 5; energies only 24000, then always;
-// the same within 2000 atoms at d = 64 and with two transforms.
+static int matrix_rounds(int T, int S, int d) { return (S + stacks_per_round(d, T) - 1) / stacks_per_round(d, T); }
+static long long matrix_units(int A, int ne, int T, int S, int d) {
+    return ((long long)(A + SM_ATOMS - 1) / SM_ATOMS + ne) * matrix_rounds(T, S, d);
+}
+// Shares of a launch.  Three (d = 128 with the gradient) or four workgroups are resident per CU; twice as many shares level out
+// what the cut into whole shares leaves uneven, but a share of few rounds pays more for its parts than it gains.
+// Measured at d = 128, 128 stacks with the gradient, 3 / 6 shares per CU: 24000 atoms 206 / 207 us, 86016 atoms 668 / 643, and with two
+// transforms, 32 stacks, 24000 atoms 102 / 110.
+static int matrix_shares(long long units, int with_grad) {
+    const long long per_cu = units / (SM_CUS * (with_grad ? 24 : 16));
+    return (int)std::min(units, (long long)SM_CUS * std::max(3ll, std::min(6ll, per_cu)));
+}
+
+extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, int d, int with_grad) {
+    if (A <= 0 || qmll_sorf_signs_bytes(ne, T, S, d) == 0) return 0;
+    return (size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * 2 * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float);
+}
+
+// What this kernel gains per atom and stack has to carry a launch more and the parts of the cut tiles, 20 us with the gradient
+// and 10 us without.  Measured, rows kernel / this one, with the gradient: d = 128, 128 stacks, 16384 atoms 157 / 152 us (2.1e6 in
+// the units below), 24000 atoms 222 / 206; two transforms, 32 stacks, 16384 atoms 78 / 83 (1.05e6), 24000 atoms 108 / 102 (1.5e6); d = 64,
+// 128 stacks, 16384 atoms 76 / 79, 24000 atoms 105 / 102; 8 stacks, 131500 atoms 101 / 98.  Energies only: d = 128, 128 stacks, 4096
+// atoms 31 / 33 (0.52e6), 8192 atoms 51 / 48; two transforms, 32 stacks, 16384 atoms 42 / 41; 8 stacks, 86016 atoms 42 / 38.
 extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
-    if (qmll_sorf_signs_bytes(ne, T, S, d) == 0) return 0;
-    constexpr int STEP = 16 * 1024;
-    const int w = A / STEP + (A % STEP != 0);
-    const int empty = (A % STEP) ? STEP - A % STEP : 0;
-    return w >= 2 && (w >= 5 || empty <= (with_grad ? 4096 : 8192) * (w - 1));
+    if (qmll_sorf_signs_bytes(ne, T, S, d) == 0 || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
+    return (double)A * S * T * d / 128.0 >= (with_grad ? 1.6e6 : 0.8e6);
 }
 
 extern "C" size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d) {
@@ -409,34 +495,43 @@ extern "C" int qmll_sorf_alpha(const float* alpha, int S, int d, float* out, qml
 
 extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D,
                                        const void* signs, const float* bias_rev, const float* alpha_scaled, const float* bias_absmax,
-                                       int A, int ne, int d, int S, int T, float normalisation, float* e_slots, float* gx,
-                                       qmll_stream_t stream) {
+                                       int A, int ne, int d, int S, int T, float normalisation, float* work, size_t work_bytes,
+                                       float* e_slots, float* gx, qmll_stream_t stream) {
     QMLL_REQUIRE(A >= 0 && qmll_sorf_signs_bytes(ne, T, S, d) > 0, QMLL_ERR_INVALID,
                  "qmll_sorf_energy_matrix: bad size A=%d ne=%d T=%d S=%d d=%d", A, ne, T, S, d);
     if (A == 0) return QMLL_OK;
     QMLL_REQUIRE(x && type_offsets && sorted_slots && D && signs && bias_rev && alpha_scaled && bias_absmax && e_slots,
                  QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: null pointer");
-    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)D | (uintptr_t)signs | (uintptr_t)bias_rev | (uintptr_t)alpha_scaled | (uintptr_t)gx) & 15) == 0,
+    QMLL_REQUIRE(work && work_bytes >= qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr), QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_matrix: workspace of %zu bytes, %zu are needed", work ? work_bytes : (size_t)0,
+                 qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr));
+    QMLL_REQUIRE(matrix_units(A, ne, T, S, d) < (1ll << 31), QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_matrix: %d atoms times %d stacks are too many for one launch", A, S);
+    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)work | (uintptr_t)D | (uintptr_t)signs | (uintptr_t)bias_rev | (uintptr_t)alpha_scaled |
+                   (uintptr_t)gx) & 15) == 0,
                  QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: every array must be 16-byte aligned");
     float hn = 1.0f;                                     // (1 / sqrt(d)) per transform
     for (int m = 0; m < T; ++m) hn /= sqrtf((float)d);
     const float scale = normalisation * hn, normf = sqrtf(2.0f / ((float)S * (float)d));
-    const dim3 grid((A + SM_ATOMS - 1) / SM_ATOMS + ne + (A >= 65536 ? 64 : (A >> 10) + 1));
+    const int nshares = matrix_shares(matrix_units(A, ne, T, S, d), gx != nullptr);
+    const dim3 grid(nshares + (gx ? (A >= 65536 ? 64 : (A >> 10) + 1) : 0));
     hipStream_t st = (hipStream_t)stream;
-    auto launch = [&](auto dc, auto tc) {
+    auto launch = [&](auto dc, auto tc, auto gc) {
         constexpr int DD = decltype(dc)::value, TT = decltype(tc)::value;
-        if (gx)
-            hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, true, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets,
-                               sorted_slots, D, (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, scale, normf,
-                               e_slots, gx);
-        else
-            hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, false, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets,
-                               sorted_slots, D, (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, scale, normf,
-                               e_slots, gx);
+        constexpr bool GG = decltype(gc)::value;
+        hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, GG, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets, sorted_slots, D,
+                           (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, nshares, scale, normf, work, e_slots,
+                           gx);
+        hipLaunchKernelGGL((sorf_parts_kernel<DD, GG>), dim3(nshares), dim3(256), 0, st, type_offsets, sorted_slots, ne,
+                           matrix_rounds(TT, S, DD), work, e_slots, gx);
+    };
+    auto by_grad = [&](auto dc, auto tc) {
+        if (gx) launch(dc, tc, std::true_type{});
+        else launch(dc, tc, std::false_type{});
     };
     auto by_d = [&](auto tc) {
-        if (d == 64) launch(std::integral_constant<int, 64>{}, tc);
-        else launch(std::integral_constant<int, 128>{}, tc);
+        if (d == 64) by_grad(std::integral_constant<int, 64>{}, tc);
+        else by_grad(std::integral_constant<int, 128>{}, tc);
     };
     if (T == 1) by_d(std::integral_constant<int, 1>{});
     else by_d(std::integral_constant<int, 2>{});

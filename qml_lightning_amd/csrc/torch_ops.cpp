@@ -85,7 +85,8 @@ Tensor prepared_form(const Tensor& t, int kind, const std::function<Tensor(const
     return buffer;
 }
 
-// a form whose making waits for the device can only be used under graph capture when it was made before
+// under graph capture a form can only be used when it was made before: its making would wait for the device, or happen at the
+// replay while the form is taken for made
 bool form_at_hand(const Tensor& t, int kind) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing((hipStream_t)stream(), &status) == hipSuccess && status == hipStreamCaptureStatusNone) return true;
@@ -557,7 +558,8 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
                 " elements and ", S * d, " features");
     // the largest |bias|, a constant of the model: computed once per tensor version, kept on the device
     Tensor bmax = prepared_form(bb, 2, [](const Tensor& b) { return b.abs().max().reshape({1}); });
-    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr) && form_at_hand(DD, 4)) {
+    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr) && form_at_hand(DD, 4) && form_at_hand(bb, 5) &&
+        form_at_hand(al, 6 + d)) {
         // large batches: the half-precision matrix cores, with the diagonals' signs, bias in revolutions and alpha scaled
         // once per tensor version; an empty form says that the diagonals are not all +-1
         Tensor signs = prepared_form(DD, 4, [&](const Tensor& D) {
@@ -575,8 +577,10 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
                 check(qmll_sorf_alpha(fp(a), S, d, out.data_ptr<float>(), stream()), "qmll_sorf_alpha");
                 return out;
             });
+            const size_t work_bytes = qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr);
+            Tensor work = at::empty({(int64_t)(work_bytes / 4)}, DD.options().dtype(at::kFloat));
             check(qmll_sorf_energy_matrix(x, off, ss, fp(DD), signs.const_data_ptr(), fp(rev), fp(scaled), fp(bmax), A, ne, d, S, T,
-                                          scalar(cn), e, A ? gx : nullptr, stream()),
+                                          scalar(cn), work.data_ptr<float>(), work_bytes, e, A ? gx : nullptr, stream()),
                   "qmll_sorf_energy_matrix");
             return;
         }

@@ -648,17 +648,20 @@ def sorf_energy_sorted(x, type_offsets, sorted_slots, Dmat, bias, alpha, normali
     gx = torch.empty((A, d), dtype=torch.float32, device=x.device) if with_grad else None
     # the largest |bias|, a constant of the model, computed once per tensor version and left on the device
     bmax = presplit_cached(bias, "absmax", lambda t: t.abs().max().reshape(1))
-    # large batches run on the half-precision matrix cores (the form's making waits for the device: not under capture)
+    # large batches run on the half-precision matrix cores; under capture only with forms made before (the making of one waits
+    # for the device, and that of the others would happen at the replay)
     matrix = _lib.lib().qmll_sorf_matrix_pays(A, ne, T, S, d, int(with_grad))
     if matrix and torch.cuda.is_current_stream_capturing():
-        matrix = (id(Dmat), "signs") in _PRESPLIT
+        matrix = all(_presplit_hit(t, k) for t, k in ((Dmat, "signs"), (bias, "revolutions"), (alpha, "sorf %d" % d)))
     signs = presplit_cached(Dmat, "signs", sorf_signs) if matrix else None
     if signs is not None:
         rev = presplit_cached(bias, "revolutions", lambda t: t * (0.5 / math.pi))
         scaled = presplit_cached(alpha, "sorf %d" % d, lambda t: sorf_alpha(t, S, d))
+        nbytes = int(_lib.lib().qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, int(with_grad)))
+        work = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
         check(_lib.lib().qmll_sorf_energy_matrix(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(signs), _ptr(rev),
-                                                 _ptr(scaled), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(e_slots),
-                                                 _ptr(gx), _stream()), "qmll_sorf_energy_matrix")
+                                                 _ptr(scaled), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(work), nbytes,
+                                                 _ptr(e_slots), _ptr(gx), _stream()), "qmll_sorf_energy_matrix")
         return e_slots, gx
     check(_lib.lib().qmll_sorf_energy_sorted(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(bias),
                                              _ptr(alpha), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(e_slots),
@@ -741,14 +744,18 @@ def _version(t):
         return -1
 
 
+def _presplit_hit(t, kind):
+    hit = _PRESPLIT.get((id(t), kind))
+    return hit if hit is not None and hit[0]() is t and hit[1] == _version(t) and hit[2] == t.data_ptr() else None
+
+
 def presplit_cached(t, kind, make):
     """The prepared (pre-split) form of a model constant `t`, made once by `make(t)` and reused until
     the tensor object dies, is written to in place (its version counter moves) or changes its storage."""
-    key = (id(t), kind)
-    hit = _PRESPLIT.get(key)
-    if hit is not None and hit[0]() is t and hit[1] == _version(t) and hit[2] == t.data_ptr():
+    hit = _presplit_hit(t, kind)
+    if hit is not None:
         return hit[3]
-    buf = make(t)
+    key, buf = (id(t), kind), make(t)
     _PRESPLIT[key] = (weakref.ref(t, lambda _r, k=key: _PRESPLIT.pop(k, None)), _version(t), t.data_ptr(), buf)
     return buf
 
