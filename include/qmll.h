@@ -461,6 +461,13 @@ int qmll_rff_presplit(const float* W, int ne, int d, int F, void* W_split, size_
 int qmll_rff_energy_sorted(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split,
                            const float* b, const float* alpha, int A, int ne, int d, int F, float* e_slots,
                            float* gx, qmll_stream_t stream);
+/* The same with device memory for this call alone, of qmll_rff_energy_workspace_bytes: tiles of atoms that several workgroups
+ * share are then summed from it in a fixed order and e_slots need not be zero, where the call above adds into the zero-filled
+ * outputs with atomics (slower, and the last bit varies from run to run). */
+size_t qmll_rff_energy_workspace_bytes(int A, int ne, int d, int F, int with_grad);
+int qmll_rff_energy_shares(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split, const float* b,
+                           const float* alpha, int A, int ne, int d, int F, float* work, size_t work_bytes, float* e_slots,
+                           float* gx, qmll_stream_t stream);
 
 /* ---- Gram ------------------------------------------------------------------------ */
 

@@ -85,6 +85,8 @@ PROTOTYPES = {
     "qmll_rff_presplit_bytes": [c_int, c_int, c_int],
     "qmll_rff_presplit": [P, c_int, c_int, c_int, P, c_size_t, P],
     "qmll_rff_energy_sorted": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, P, P, P],
+    "qmll_rff_energy_workspace_bytes": [c_int] * 5,
+    "qmll_rff_energy_shares": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, P, c_size_t, P, P, P],
     "qmll_gram_f64": [P, P, c_int, c_int, P, P, P],
     "qmll_gram_upper_f64": [P, P, c_int, c_int, P, P, P],
     "qmll_gram_workspace_bytes": [],
@@ -101,7 +103,7 @@ PROTOTYPES = {
     "qmll_probe_rate": [c_int, c_int, c_int, P, P],
     "qmll_probe_mix": [c_int, c_int, c_int, P, P],
 }
-_RESTYPES = {"qmll_last_error": c_char_p, "qmll_sorf_signs_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_sorf_matrix_workspace_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
+_RESTYPES = {"qmll_last_error": c_char_p, "qmll_sorf_signs_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_rff_energy_workspace_bytes": c_size_t, "qmll_sorf_matrix_workspace_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
              "qmll_cholesky_workspace_bytes": c_size_t, "qmll_gram_workspace_bytes": c_size_t,
              "qmll_probe_out_bytes": c_size_t, "qmll_probe_rate": c_double,
              "qmll_probe_mix": c_double}

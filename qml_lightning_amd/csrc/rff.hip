@@ -14,6 +14,9 @@
 //    over the molecule's atoms in registers, so G is written once and no atomics are needed.
 #include <type_traits>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "qmll_common.h"
 
 namespace {
@@ -380,11 +383,31 @@ __global__ __launch_bounds__(RE_T) void rff_presplit_kernel(const float* __restr
     for (int t = tid; t < Img::BYTES / 16; t += RE_T) dst[t] = reinterpret_cast<const float4*>(img)[t];
 }
 
+// tile `tile` of RE_M atoms of one element; false past the last
+__device__ __forceinline__ bool find_tile(const int* __restrict__ type_offsets, int ne, int tile, int& type, int& row0, int& rows) {
+    for (int t = 0; t < ne; ++t) {
+        const int o0 = type_offsets[t], o1 = type_offsets[t + 1], nt = (o1 - o0 + RE_M - 1) / RE_M;
+        if (tile < nt) {
+            type = t;
+            row0 = o0 + tile * RE_M;
+            rows = min(RE_M, o1 - row0);
+            return true;
+        }
+        tile -= nt;
+    }
+    return false;
+}
+
+// a part of a tile's result: its energies, then (with the gradient) its rows
+__host__ __device__ constexpr size_t part_floats(int d, bool with_grad) { return (size_t)RE_M * (with_grad ? d + 1 : 1); }
+
 template <int D, bool WITH_GRAD>
 __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void rff_energy_sorted_f16_kernel(
     const float* __restrict__ x, const int* __restrict__ type_offsets, const int* __restrict__ sorted_slots,
     const _Float16* __restrict__ images, const int* __restrict__ exponents, const float* __restrict__ b,
-    const float* __restrict__ alpha, int ne, int F, float norm, float* __restrict__ e_slots, float* __restrict__ gx) {
+    const float* __restrict__ alpha, int ne, int F, int nwhole, int nparts, float norm, float* __restrict__ parts,
+    float* __restrict__ e_slots,
+    float* __restrict__ gx) {
     using Img = RffImage<D>;
     constexpr int LD1 = Img::LD1, LD2 = Img::LD2;
     constexpr int KS = D / 16;                // matrix instructions along k per product term
@@ -393,31 +416,21 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
     __shared__ __attribute__((aligned(16))) _Float16 simg0[Img::HALVES], simg1[Img::HALVES];
     __shared__ __attribute__((aligned(16))) float sba[2 * 2 * RE_FC];     // [2][2][RE_FC]: b / 2 pi, alpha norm 2^kp of the two chunks
 
-    int type = -1, row0 = 0, rows = 0;
-    {
-        int bidx = blockIdx.x;
-        for (int t = 0; t < ne; ++t) {
-            const int o0 = type_offsets[t], o1 = type_offsets[t + 1];
-            const int nt = (o1 - o0 + RE_M - 1) / RE_M;
-            if (bidx < nt) {
-                type = t;
-                row0 = o0 + bidx * RE_M;
-                rows = min(RE_M, o1 - row0);
-                break;
-            }
-            bidx -= nt;
-        }
-    }
-    if (type < 0) return;
-    const float* bt = b + (size_t)type * F;
-
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 31, h = lane >> 5;
+    const int nchunks = F / RE_FC;
+    // workgroups below `whole` take a tile's chunks all, the others a share of 1 / nparts of them
+    const bool whole = (int)blockIdx.x < nwhole;
+    const int piece = whole ? 0 : (int)blockIdx.x - nwhole;
+    const int c0 = whole ? 0 : (int)((long long)nchunks * (piece % nparts) / nparts);
+    const int c1 = whole ? nchunks : (int)((long long)nchunks * (piece % nparts + 1) / nparts);
+    int type, row0, rows;
+    if (!find_tile(type_offsets, ne, whole ? (int)blockIdx.x : nwhole + piece / nparts, type, row0, rows)) return;
+    float* part_out = parts ? parts + (size_t)piece * part_floats(D, WITH_GRAD) : nullptr;
+    const float* bt = b + (size_t)type * F;
     const int arow = 32 * wave + i;
     const bool aok = arow < rows;
-    const int fsplit = F / (int)gridDim.y;
-    const int fbeg = (int)blockIdx.y * fsplit, fend = fbeg + fsplit;
-    const int nchunks = F / RE_FC;
+    const int fbeg = c0 * RE_FC, fend = c1 * RE_FC;
     // a scalar base and one per-lane offset: the loads then need no per-lane 64-bit addresses
     const unsigned char* img0 = reinterpret_cast<const unsigned char*>(images) + (size_t)type * nchunks * Img::BYTES;
     const int wave_s = __builtin_amdgcn_readfirstlane(wave);
@@ -617,32 +630,60 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
     }
 
     energy = (energy + __shfl_xor(energy, 32, 64)) * inv_sp;
-    if (gridDim.y == 1) {
-        if (h == 0 && aok) e_slots[sorted_slots[row0 + arow]] = energy;
+    if (!aok) return;
+    if (whole || part_out) {
+        if (h == 0) {
+            if (whole) e_slots[sorted_slots[row0 + arow]] = energy;
+            else part_out[arow] = energy;
+        }
         if constexpr (WITH_GRAD) {
-            if (aok) {
-                float* gr = gx + (size_t)(row0 + arow) * D;
+            float* gr = (whole ? gx + (size_t)row0 * D : part_out + RE_M) + (size_t)arow * D;
 #pragma unroll
-                for (int blk = 0; blk < D / 32; ++blk)
+            for (int blk = 0; blk < D / 32; ++blk)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        *reinterpret_cast<float4*>(gr + 32 * blk + 8 * q + 4 * h) =
-                            make_float4(gacc[blk][4 * q] * inv_sp, gacc[blk][4 * q + 1] * inv_sp,
-                                        gacc[blk][4 * q + 2] * inv_sp, gacc[blk][4 * q + 3] * inv_sp);
-            }
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(gr + 32 * blk + 8 * q + 4 * h) =
+                        make_float4(gacc[blk][4 * q] * inv_sp, gacc[blk][4 * q + 1] * inv_sp,
+                                    gacc[blk][4 * q + 2] * inv_sp, gacc[blk][4 * q + 3] * inv_sp);
         }
     } else {
-        // the feature parts add into zero-filled outputs
-        if (h == 0 && aok) atomicAdd(&e_slots[sorted_slots[row0 + arow]], energy);
+        // no workspace: the parts add into zero-filled outputs
+        if (h == 0) atomicAdd(&e_slots[sorted_slots[row0 + arow]], energy);
         if constexpr (WITH_GRAD) {
-            if (aok) {
-                float* gr = gx + (size_t)(row0 + arow) * D;
+            float* gr = gx + (size_t)(row0 + arow) * D;
 #pragma unroll
-                for (int blk = 0; blk < D / 32; ++blk)
+            for (int blk = 0; blk < D / 32; ++blk)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        atomicAdd(gr + 32 * blk + 8 * (r / 4) + 4 * h + (r % 4), gacc[blk][r] * inv_sp);
+                for (int r = 0; r < 16; ++r)
+                    atomicAdd(gr + 32 * blk + 8 * (r / 4) + 4 * h + (r % 4), gacc[blk][r] * inv_sp);
+        }
+    }
+}
+
+// the parts of the tiles nwhole + blockIdx.x, added up in order; grid (tiles, column slices).  HBM bound.
+template <int D, bool WITH_GRAD>
+__global__ __launch_bounds__(256) void rff_sum_parts_kernel(const int* __restrict__ type_offsets, const int* __restrict__ sorted_slots,
+                                                            int ne, int nwhole, int nparts, const float* __restrict__ parts,
+                                                            float* __restrict__ e_slots, float* __restrict__ gx) {
+    constexpr size_t SLOT = part_floats(D, WITH_GRAD);
+    int type, row0, rows;
+    if (!find_tile(type_offsets, ne, nwhole + (int)blockIdx.x, type, row0, rows)) return;
+    const float* src = parts + (size_t)blockIdx.x * nparts * SLOT;
+    if (blockIdx.y == 0 && (int)threadIdx.x < rows) {
+        float v = 0.0f;
+#pragma unroll 8
+        for (int k = 0; k < nparts; ++k) v += src[k * SLOT + threadIdx.x];
+        e_slots[sorted_slots[row0 + threadIdx.x]] = v;
+    }
+    if constexpr (WITH_GRAD) {
+        for (int t = blockIdx.y * 256 + threadIdx.x; t < rows * (D / 4); t += gridDim.y * 256) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+            for (int k = 0; k < nparts; ++k) {
+                const float4 w = *reinterpret_cast<const float4*>(src + k * SLOT + RE_M + 4 * t);
+                v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
             }
+            *reinterpret_cast<float4*>(gx + (size_t)row0 * D + 4 * t) = v;
         }
     }
 }
@@ -769,9 +810,46 @@ extern "C" int qmll_rff_presplit(const float* W, int ne, int d, int F, void* out
     return QMLL_OK;
 }
 
-extern "C" int qmll_rff_energy_sorted(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split,
-                                      const float* b, const float* alpha, int A, int ne, int d, int F, float* e_slots,
-                                      float* gx, qmll_stream_t stream) {
+// How the tiles of a launch (128 atoms of one element each) are shared out.  Two workgroups fit a CU (two wavefronts per SIMD; four
+// at d = 64 without the gradient) and all walk the chunks of W at the same pace, which is what lets the workgroups of an
+// XCD share its L2: W's images are 116 MB at 32768 features, and shares that begin anywhere in W, though of equal size, were bound by their traffic (86016 atoms: 5.4 ms).  So
+// as many full rounds of 512 tiles as there are run whole, and each tile of the rest is cut into nparts ranges of chunks.
+// In units of one chunk (2.4 us with 512 workgroups resident): a part costs three more for its x and alpha, a launch more
+// three, and 72 parts written and read back one.
+// The parts used to be added into zero-filled outputs with atomics, 4 bytes each at a stride of a row, which took 2 to 3 ms per
+// launch whatever its work.  Measured with the gradient, atomics -> parts: d = 128, 32768 features, 86016 atoms 4.99 -> 4.53 ms, 10000
+// atoms 2.06 -> 0.58, 300 atoms 146 -> 67 us; 2048 features, 33000 atoms 3.27 ms -> 173 us; d = 64, 8192 features, 4000 atoms
+// 434 -> 55 us.  Energies only, where the atomics were few: 2048 features, 10000 atoms 87 -> 32 us, 21 atoms 8 -> 11.
+struct RffSplit { int nwhole, ntail, nparts; };
+static RffSplit rff_split(int A, int ne, int d, int F, bool with_grad) {
+    const int SLOTS = (d == 64 && !with_grad ? 4 : 2) * 256;
+    const int tiles = (A + RE_M - 1) / RE_M + ne, nchunks = F / RE_FC;      // at most: every element's last tile may be partial
+    RffSplit p = {tiles / SLOTS * SLOTS, tiles % SLOTS, 1};
+    double best = nchunks + 3.0;
+    for (int k = 2; k <= 64 && nchunks / k >= 4; ++k) {
+        const int pieces = p.ntail * k;
+        const double cost = ((pieces + SLOTS - 1) / SLOTS) * ((nchunks + k - 1) / k + 3.0) + 3.0 + pieces / 72.0;
+        if (cost < best) {
+            best = cost;
+            p.nparts = k;
+        }
+    }
+    if (p.nparts == 1) {
+        p.nwhole = tiles;
+        p.ntail = 0;
+    }
+    return p;
+}
+
+extern "C" size_t qmll_rff_energy_workspace_bytes(int A, int ne, int d, int F, int with_grad) {
+    if (A <= 0 || ne <= 0 || d <= 0 || F < RE_FC) return 0;
+    const RffSplit p = rff_split(A, ne, d, F, with_grad != 0);
+    return (size_t)p.ntail * p.nparts * part_floats(d, with_grad) * sizeof(float);
+}
+
+extern "C" int qmll_rff_energy_shares(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split,
+                                      const float* b, const float* alpha, int A, int ne, int d, int F, float* work,
+                                      size_t work_bytes, float* e_slots, float* gx, qmll_stream_t stream) {
     QMLL_REQUIRE(A >= 0 && ne > 0 && d > 0 && F > 0, QMLL_ERR_INVALID, "qmll_rff_energy_sorted: bad size A=%d ne=%d d=%d F=%d",
                  A, ne, d, F);
     QMLL_REQUIRE(d == 64 || d == 128, QMLL_ERR_INVALID, "qmll_rff_energy_sorted: d=%d is not 64 or 128", d);
@@ -779,45 +857,45 @@ extern "C" int qmll_rff_energy_sorted(const float* x, const int* type_offsets, c
     if (A == 0) return QMLL_OK;
     QMLL_REQUIRE(x && type_offsets && sorted_slots && W_split && b && alpha && e_slots, QMLL_ERR_INVALID,
                  "qmll_rff_energy_sorted: null pointer");
-    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)W_split | (uintptr_t)gx) & 15) == 0, QMLL_ERR_INVALID,
-                 "qmll_rff_energy_sorted: x, W_split and gx must be 16-byte aligned");
+    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)W_split | (uintptr_t)work | (uintptr_t)gx) & 15) == 0, QMLL_ERR_INVALID,
+                 "qmll_rff_energy_sorted: x, W_split, work and gx must be 16-byte aligned");
+    QMLL_REQUIRE(!work || work_bytes >= qmll_rff_energy_workspace_bytes(A, ne, d, F, gx != nullptr), QMLL_ERR_INVALID,
+                 "qmll_rff_energy_sorted: workspace of %zu bytes, %zu are needed", work_bytes,
+                 qmll_rff_energy_workspace_bytes(A, ne, d, F, gx != nullptr));
     const _Float16* images = (const _Float16*)W_split;
     const int* exponents = (const int*)((const char*)W_split + (size_t)ne * (F / RE_FC) * rff_image_bytes(d));
     const float norm = sqrtf(2.0f / (float)F);
     hipStream_t st = (hipStream_t)stream;
-    // Two workgroups fit a CU (two wavefronts per SIMD) and all run the same chunk loop, so the launch takes ceil(workgroups / 512) rounds of 1/fs of a tile's work
-    // when the features are split over fs workgroups per tile.  fs is the power of two up to
-    // 64 with the shortest estimate (a larger one has to win by 5 %): 672 tiles take 2 rounds
-    // with fs = 1 and 21/16 with fs = 16; one molecule takes 1/64 instead of 1.  For fs > 1
-    // the parts add their energies and gradients into zero-filled outputs with fp32 atomics
-    // (from fs = 4 on the order of the terms, hence the last bit, varies from run to run).
-    const int tiles = (A + RE_M - 1) / RE_M, slots = 2 * 256;
-    auto rounds = [&](int k) { return (double)(((long long)(tiles + ne) * k + slots - 1) / slots) / k; };
-    int fs = 1;
-    for (int k = 2; k <= 64 && F % (k * RE_FC) == 0; k *= 2)
-        if (rounds(k) < 0.95 * rounds(fs)) fs = k;
-    const dim3 grid(tiles + ne, fs);
-    if (fs > 1 && gx) {
+    const RffSplit p = rff_split(A, ne, d, F, gx != nullptr);
+    if (!work && p.ntail && gx) {
         hipLaunchKernelGGL(zero_fill_kernel, dim3(1024), dim3(256), 0, st, gx, (size_t)A * d);
         QMLL_CHECK_LAUNCH("qmll_rff_energy_sorted");
     }
-#define CALL(DD)                                                                                                     \
-    if (gx)                                                                                                          \
-        hipLaunchKernelGGL((rff_energy_sorted_f16_kernel<DD, true>), grid, dim3(RE_T), 0, st, x, type_offsets,         \
-                           sorted_slots, images, exponents, b, alpha, ne, F, norm, e_slots, gx);                      \
-    else                                                                                                             \
-        hipLaunchKernelGGL((rff_energy_sorted_f16_kernel<DD, false>), grid, dim3(RE_T), 0, st, x, type_offsets,        \
-                           sorted_slots, images, exponents, b, alpha, ne, F, norm, e_slots, gx);
-    if (d == 64) {
-        CALL(64)
-    } else {
-        CALL(128)
-    }
-#undef CALL
+    auto launch = [&](auto dc, auto gc) {
+        constexpr int DD = decltype(dc)::value;
+        constexpr bool GG = decltype(gc)::value;
+        hipLaunchKernelGGL((rff_energy_sorted_f16_kernel<DD, GG>), dim3(p.nwhole + p.ntail * p.nparts), dim3(RE_T), 0, st, x, type_offsets,
+                           sorted_slots, images, exponents, b, alpha, ne, F, p.nwhole, p.nparts, norm, work, e_slots, gx);
+        if (work && p.ntail)
+            hipLaunchKernelGGL((rff_sum_parts_kernel<DD, GG>), dim3(p.ntail, GG ? 8 : 1), dim3(256), 0, st, type_offsets, sorted_slots,
+                               ne, p.nwhole, p.nparts, work, e_slots, gx);
+    };
+    auto by_grad = [&](auto dc) {
+        if (gx) launch(dc, std::true_type{});
+        else launch(dc, std::false_type{});
+    };
+    if (d == 64) by_grad(std::integral_constant<int, 64>{});
+    else by_grad(std::integral_constant<int, 128>{});
     QMLL_CHECK_LAUNCH("qmll_rff_energy_sorted");
     if (gx) {
         hipLaunchKernelGGL(zero_tail_rows_kernel, dim3(64), dim3(256), 0, st, type_offsets, ne, A, d, gx);
         QMLL_CHECK_LAUNCH("qmll_rff_energy_sorted");
     }
     return QMLL_OK;
+}
+
+extern "C" int qmll_rff_energy_sorted(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split,
+                                      const float* b, const float* alpha, int A, int ne, int d, int F, float* e_slots,
+                                      float* gx, qmll_stream_t stream) {
+    return qmll_rff_energy_shares(x, type_offsets, sorted_slots, W_split, b, alpha, A, ne, d, F, nullptr, 0, e_slots, gx, stream);
 }

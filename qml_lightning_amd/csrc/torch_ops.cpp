@@ -659,8 +659,11 @@ void rff_energy_sorted_raw(const float* x, const int* off, const int* ss, int A,
         check(qmll_rff_presplit(fp(w), ne, d, F, out.data_ptr(), nbytes, stream()), "qmll_rff_presplit");
         return out;
     });
-    check(qmll_rff_energy_sorted(x, off, ss, Wsplit.const_data_ptr(), fp(bb), fp(al), A, ne, d, F, e, A ? gx : nullptr, stream()),
-          "qmll_rff_energy_sorted");
+    const size_t work_bytes = qmll_rff_energy_workspace_bytes(A, ne, d, F, gx != nullptr);
+    Tensor work = at::empty({(int64_t)(work_bytes / 4)}, bb.options());
+    check(qmll_rff_energy_shares(x, off, ss, Wsplit.const_data_ptr(), fp(bb), fp(al), A, ne, d, F, work.data_ptr<float>(), work_bytes, e,
+                                 A ? gx : nullptr, stream()),
+          "qmll_rff_energy_shares");
 }
 
 std::tuple<Tensor, Tensor> rff_energy_sorted_impl(const Tensor& x_, const Tensor& type_offsets, const Tensor& sorted_slots,

@@ -790,9 +790,11 @@ def rff_energy_sorted(x, type_offsets, sorted_slots, W, b, alpha, nslots, with_g
     Wsplit = presplit_cached(W, "rff", rff_presplit)
     e_slots = _zeroed_slots(e_zeroed, nslots, x.device)
     gx = torch.empty((A, d), dtype=torch.float32, device=x.device) if with_grad else None
-    check(_lib.lib().qmll_rff_energy_sorted(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Wsplit), _ptr(b),
-                                            _ptr(alpha), A, ne, d, F, _ptr(e_slots), _ptr(gx), _stream()),
-          "qmll_rff_energy_sorted")
+    nbytes = int(_lib.lib().qmll_rff_energy_workspace_bytes(A, ne, d, F, int(with_grad)))
+    work = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+    check(_lib.lib().qmll_rff_energy_shares(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Wsplit), _ptr(b),
+                                            _ptr(alpha), A, ne, d, F, _ptr(work), nbytes, _ptr(e_slots), _ptr(gx),
+                                            _stream()), "qmll_rff_energy_shares")
     return e_slots, gx
 
 

@@ -1006,6 +1006,43 @@ def test_rff_energy_sorted_kernel(d, F, ne, A):
     close(e2, e_ref, REL_EF, "fused rff energies only")
 
 
+@pytest.mark.parametrize("d,F,A,grad", [(64, 32, 1, True), (64, 256, 66000, True), (128, 256, 65600, True), (64, 256, 131100, False),
+                                        (128, 4096, 300, True), (128, 4096, 129, False), (64, 8192, 1000, True)])
+def test_rff_energy_parts_of_a_tile(d, F, A, grad):
+    """Whole tiles, tiles cut into parts, and both in one launch (more than a round of the chip's workgroups), with a workspace
+    and with the atomics of the call that has none, against fp64.  A product term keeps 2^-22 of itself, the sums are fp32 over
+    d terms and F features: 2e-5 of the largest entry as for the kernel's other tests."""
+    from qml_lightning_amd import _lib, ops
+    from qml_lightning_amd.ops import _ptr, _stream
+    g = torch.Generator(device=dev()).manual_seed(A)
+    ne = 2
+    cut = (2 * A) // 3
+    off = torch.tensor([0, cut, A - A // 50], dtype=torch.int32, device=dev())       # the last atoms are of no known element
+    x = torch.randn(A, d, device=dev(), generator=g)
+    W = torch.randn(ne, d, F, device=dev(), generator=g) * 0.1
+    b = torch.rand(ne, F, device=dev(), generator=g) * 6.28
+    alpha = torch.randn(F, device=dev(), generator=g)
+    slots = torch.randperm(A, device=dev(), generator=g).int()
+    e_ref = torch.zeros(A, dtype=torch.float64, device=dev())
+    g_ref = torch.zeros(A, d, dtype=torch.float64, device=dev())
+    for t in range(ne):
+        lo, hi = int(off[t]), int(off[t + 1])
+        arg = x[lo:hi].double() @ W[t].double() + b[t].double()
+        e_ref[slots[lo:hi].long()] = (2.0 / F) ** 0.5 * (torch.cos(arg) @ alpha.double())
+        g_ref[lo:hi] = -(2.0 / F) ** 0.5 * (torch.sin(arg) * alpha.double()) @ W[t].double().T.contiguous()
+    e, gx = ops.rff_energy_sorted(x, off, slots, W, b, alpha, A, with_grad=grad)
+    again = ops.rff_energy_sorted(x, off, slots, W, b, alpha, A, with_grad=grad)
+    assert torch.equal(e, again[0]) and (not grad or torch.equal(gx, again[1]))      # a fixed order of the parts
+    e0, g0 = torch.zeros(A, device=dev()), torch.empty(A, d, device=dev())
+    rc = _lib.lib().qmll_rff_energy_sorted(_ptr(x), _ptr(off), _ptr(slots), _ptr(ops.rff_presplit(W)), _ptr(b), _ptr(alpha), A, ne, d, F,
+                                           _ptr(e0), _ptr(g0) if grad else None, _stream())
+    assert rc == 0
+    for got in (e, e0):
+        assert float((got.double() - e_ref).abs().max()) <= 2e-5 * float(e_ref.abs().max())
+    for got in (gx, g0) if grad else ():
+        assert float((got.double() - g_ref).abs().max()) <= 2e-5 * float(g_ref.abs().max())
+
+
 @pytest.mark.parametrize("wscale,ascale,xscale", [(0.125, 1.0, 1.0), (1e-3, 1e4, 1.0), (1e-4, 1e20, 1.0), (0.125, 1e-6, 1.0),
                                                   (125.0, 1e-20, 1e-3), (2e-6, 1.0, 6e4), (0.125, 1.0, 0.0)])
 def test_rff_energy_sorted_kernel_over_operand_scales(wscale, ascale, xscale):
