@@ -586,6 +586,15 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
             }
         }
         if constexpr (WITH_GRAD) {
+            // at d = 128 the kernel takes all 256 registers: without this line the compiler keeps the arguments of the cosines
+            // across the second product and spills for it, and a reload waits for the next image too.  The
+            // second product goes ahead of the other wavefront's vector instructions: 86016 atoms, 32768 features
+            // 4.69 -> 4.42 ms together with the line below that holds the multiplications by b and alpha back; the same around
+            // the first product or around the sines gave nothing
+            if constexpr (D == 128) {
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_setprio(1);
+            }
             // second product: 2^kp GX^T[k, a] += 2^-kw sum_f 2^kw W[k, f] 2^kp P[f, a]; instruction t contracts the
             // features of registers 8 t .. 8 t + 7.  The chunk's contribution is summed from zero and
             // added to the running sums by the vector unit: the matrix instruction aligns its products
@@ -618,6 +627,9 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
                 for (int r = 0; r < 16; ++r) gacc[blk][r] = fmaf(part[r], inv_sw, gacc[blk][r]);
             }
         }
+        if constexpr (WITH_GRAD && D == 128) __builtin_amdgcn_s_setprio(0);
+        // (used here and no earlier: the compiler waits for them right after their loads otherwise)
+        asm volatile("" : "+v"(bnext), "+v"(anext)::"memory");
         if (more && tid < RE_FC) {
             float* nb = sba + (par ^ 1) * 2 * RE_FC;
             nb[tid] = bnext * 0.15915494309189535f;
