@@ -344,7 +344,7 @@ int qmll_project_typed_rows(const float* rows, const int* sorted_slots, const in
  * (g_rep f32 [N,R]).  Rows of slots that are not in the sorted list are not written, except
  * that with types != NULL (i32 [N]) the rows of slots whose type is outside [0,ne) are set
  * to zero.  reductors_split as for qmll_project_typed (NULL = fp32 kernels only); the fp16
- * matrix-core kernel (d = 64 or 128, batches beyond the small-batch kernels) scales the 32 gradient
+ * matrix-core kernel (d = 64 or 128, batches beyond the small-batch kernels; d = 256 from 8000 atoms) scales the 32 gradient
  * rows of a wavefront by one power of two (of their largest finite entry: a non-finite gradient row
  * spoils its own result only) and every row of U by its own. */
 int qmll_project_typed_backward(const float* gx, const int* sorted_slots, const int* type_offsets,

@@ -467,7 +467,7 @@ struct BwdImage {
     static constexpr int LDB = K + 8;                 // halves per row
     static constexpr int HALVES = 2 * 32 * LDB;       // hi and lo
     static constexpr int SINV = HALVES * 2;           // byte offset of the 32 inverse factors
-    static constexpr int BYTES = (SINV + 32 * 4 + 1023) / 1024 * 1024;    // 18432 (K = 128), 10240 (K = 64)
+    static constexpr int BYTES = (SINV + 32 * 4 + 1023) / 1024 * 1024;    // 34816 (K = 256), 18432 (K = 128), 10240 (K = 64)
 };
 
 // one wavefront's share of a 1 KiB-blocked image: blocks wave, wave + 4, ... (64 lanes x 16 bytes each)
@@ -732,14 +732,16 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     }
 }
 
-// Transpose product for a short contraction (K = projected dimension 64 or 128):
+// Transpose product for a short contraction (K = projected dimension 64, 128 or 256):
 //     C[c_rows[row], :] = A[row, :] . U_type^T,   A [rows, K] (the gradient rows), U_type [N, K] row-major.
 // A wavefront keeps its 32 rows of A in registers for the whole kernel (two fp16 parts behind the
 // wavefront's power of two), so every row of A is read exactly once; the workgroup walks the N columns
 // in blocks of 32, each block's image arriving in LDS while the previous block is multiplied, and every
 // 32 x 32 block of C leaves straight from the accumulators through the two inverse factors.
+// (K = 256: the parts of the rows take 128 registers, hence two wavefronts per SIMD.  Against fp64 the relative error is 1.9e-7,
+// of the fp32 matrix instructions 2.9e-7, from 4200 to 66000 atoms and three to five elements.)
 template <int K>
-__global__ __launch_bounds__(PT) void typed_gemm_bt_rows_f16_kernel(const float* __restrict__ A,
+__global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2 : K == 128 ? 3 : 4))) void typed_gemm_bt_rows_f16_kernel(const float* __restrict__ A,
                                                                      const unsigned char* __restrict__ images,
                                                                      float* __restrict__ C, int ldc,
                                                                      const int* __restrict__ c_rows,
@@ -1231,8 +1233,8 @@ static SplitLayout split_layout(int ne, int R, int d) {
         L.fwd_bytes = (size_t)ne * L.nchunks * L.ncb * FWD_IMG_BYTES;
         L.exp_bytes = ((size_t)ne * L.nchunks * L.ncb * sizeof(int) + 15) / 16 * 16;
     }
-    if (d == 64 || d == 128) {
-        L.bwd_image = d == 64 ? (size_t)BwdImage<64>::BYTES : (size_t)BwdImage<128>::BYTES;
+    if (d == 64 || d == 128 || d == 256) {
+        L.bwd_image = d == 64 ? BwdImage<64>::BYTES : d == 128 ? BwdImage<128>::BYTES : BwdImage<256>::BYTES;
         L.bwd_bytes = (size_t)ne * L.nblk * L.bwd_image;
     }
     return L;
@@ -1260,8 +1262,11 @@ extern "C" int qmll_reductor_presplit(const float* reductors, int ne, int R, int
         if (d == 64)
             hipLaunchKernelGGL(reductor_presplit_bwd_kernel<64>, dim3(L.nblk, ne), dim3(PT), 0, (hipStream_t)stream, reductors,
                                R, base + L.fwd_bytes);
-        else
+        else if (d == 128)
             hipLaunchKernelGGL(reductor_presplit_bwd_kernel<128>, dim3(L.nblk, ne), dim3(PT), 0, (hipStream_t)stream, reductors,
+                               R, base + L.fwd_bytes);
+        else
+            hipLaunchKernelGGL(reductor_presplit_bwd_kernel<256>, dim3(L.nblk, ne), dim3(PT), 0, (hipStream_t)stream, reductors,
                                R, base + L.fwd_bytes);
         QMLL_CHECK_LAUNCH("qmll_reductor_presplit");
     }
@@ -1404,8 +1409,10 @@ extern "C" int qmll_project_typed_backward_sums(const float* gx, const int* sort
     }
         if (A < 64) LAUNCH_BT_SMALL(1) else if (A < 512) LAUNCH_BT_SMALL(4) else LAUNCH_BT_SMALL(8)
 #undef LAUNCH_BT_SMALL
-    } else if (vec && (d == 64 || d == 128) && reductors_split) {
-        // short contraction: the gradient rows stay in registers, every row is read once
+    } else if (vec && (d == 64 || d == 128 || (d == 256 && A >= 8000)) && reductors_split) {
+        // short contraction: the gradient rows stay in registers, every row is read once.  At d = 256 a tile walks its columns
+        // at two wavefronts per SIMD, too slowly for a batch that has less than a tile for every fourth CU: fp32 kernel / this one at 496
+        // columns, 4200 atoms 29 / 34 us, 8000 atoms 41 / 35, 41796 atoms 146 / 62
         const SplitLayout L = split_layout(ne, R, d);
         QMLL_REQUIRE(aligned16(reductors_split), QMLL_ERR_INVALID,
                      "qmll_project_typed_backward: reductors_split must be 16-byte aligned");
@@ -1413,6 +1420,9 @@ extern "C" int qmll_project_typed_backward_sums(const float* gx, const int* sort
         const dim3 g1((A + PM - 1) / PM + ne);
         if (d == 128)
             hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<128>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,
+                               R, sorted_slots, type_offsets, ne, R);
+        else if (d == 256)
+            hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<256>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,
                                R, sorted_slots, type_offsets, ne, R);
         else
             hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<64>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,

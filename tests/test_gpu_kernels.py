@@ -1006,6 +1006,30 @@ def test_rff_energy_sorted_kernel(d, F, ne, A):
     close(e2, e_ref, REL_EF, "fused rff energies only")
 
 
+@pytest.mark.parametrize("A,ne,R", [(7999, 3, 168), (8000, 3, 168), (8191, 5, 720), (9001, 1, 64)])
+def test_transposed_projection_of_256_components(A, ne, R):
+    """Both sides of the line from which d = 256 runs on the half-precision matrix cores: partial tiles and column blocks, rows of
+    unknown elements.  Against fp64; a product term keeps 2^-22 of itself and a sum has 256 of them in fp32: 2e-5 of the
+    largest entry."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device=dev()).manual_seed(A)
+    gx = torch.randn(A, 256, device=dev(), generator=g)
+    red = torch.randn(ne, R, 256, device=dev(), generator=g)
+    cut = sorted(torch.randint(0, A, (ne - 1,), generator=torch.Generator().manual_seed(A)).tolist())
+    bounds = [0] + cut + [A - 37]
+    bounds = [min(b, A - 37) for b in bounds]
+    off = torch.tensor(bounds, dtype=torch.int32, device=dev())
+    slots = torch.randperm(A, device=dev(), generator=g).int()
+    types = torch.full((A,), ne, dtype=torch.int32, device=dev())
+    ref = torch.zeros(A, R, dtype=torch.float64, device=dev())
+    for t in range(ne):
+        lo, hi = bounds[t], bounds[t + 1]
+        types[slots[lo:hi].long()] = t
+        ref[slots[lo:hi].long()] = gx[lo:hi].double() @ red[t].double().T.contiguous()
+    out = ops.project_typed_backward(gx, slots, off, red, types, A)
+    assert float((out.double() - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("d,F,A,grad", [(64, 32, 1, True), (64, 256, 66000, True), (128, 256, 65600, True), (64, 256, 131100, False),
                                         (128, 4096, 300, True), (128, 4096, 129, False), (64, 8192, 1000, True)])
 def test_rff_energy_parts_of_a_tile(d, F, A, grad):
