@@ -304,7 +304,7 @@ int qmll_prepare_batch(const float* Z, const int* natoms, const float* species, 
                        float* zero, size_t zero_count, qmll_stream_t stream);
 
 /* The projection matrices ("reductors", f32 [ne,R,d], qml_lightning/models/kernel.py:28) are constants
- * of a model.  For large batches the two projections below multiply on the fp16 matrix cores with
+ * of a model.  Beyond the small-batch kernels the two projections below multiply on the fp16 matrix cores with
  * every fp32 operand as two fp16 parts behind power-of-two scales (fp32 accumulation): the
  * reductors are prepared for that ONCE, here, in the layouts the kernels keep in LDS (forward: per
  * element, 32-row chunk and 128-column block; transposed: per element and 32 rows of U), so that

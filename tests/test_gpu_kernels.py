@@ -1030,6 +1030,26 @@ def test_transposed_projection_of_256_components(A, ne, R):
     assert float((out.double() - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("A,ne,R,d", [(4097, 3, 168, 128), (5000, 5, 720, 256), (16385, 2, 168, 128), (9001, 1, 64, 384)])
+def test_projection_of_medium_batches(A, ne, R, d):
+    """Batches between the one-workgroup-per-atom kernels and a full chip: partial tiles, atoms of unknown elements, rows gathered
+    out of a larger array.  Against fp64; a product term keeps 2^-22 of itself and a sum has R of them in fp32: 2e-5 of the
+    largest entry."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device=dev()).manual_seed(A)
+    N = A + A // 3
+    rep = torch.rand(N, R, device=dev(), generator=g)
+    red = torch.randn(ne, R, d, device=dev(), generator=g)
+    bounds = [0] + sorted(torch.randint(0, A - 37, (ne - 1,), generator=torch.Generator().manual_seed(A)).tolist()) + [A - 37]
+    off = torch.tensor(bounds, dtype=torch.int32, device=dev())
+    slots = torch.randperm(N, device=dev(), generator=g)[:A].int()
+    x = ops.project_typed(rep, slots, off, red)
+    for t in range(ne):
+        lo, hi = bounds[t], bounds[t + 1]
+        ref = rep[slots[lo:hi].long()].double() @ red[t].double()
+        assert hi == lo or float((x[lo:hi].double() - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("d,F,A,grad", [(64, 32, 1, True), (64, 256, 66000, True), (128, 256, 65600, True), (64, 256, 131100, False),
                                         (128, 4096, 300, True), (128, 4096, 129, False), (64, 8192, 1000, True)])
 def test_rff_energy_parts_of_a_tile(d, F, A, grad):
