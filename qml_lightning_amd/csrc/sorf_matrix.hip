@@ -271,9 +271,9 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             }
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
-            // every argument is at most sum |x| (times sqrt(d) for a second transform) + |bias|: where that stays below
-            // UMAX no stack looks at its arguments
-            const float bound = fmaf(sum, T == 2 ? (float)(1 << (log2nb<NB>() / 2 + 3)) : 1.0f, *bias_absmax * INV2PI);
+            // every argument is at most sum |x| (times d for a second transform: an entry of H D H is a sum of d signs) + |bias|:
+            // where that stays below UMAX no stack looks at its arguments
+            const float bound = fmaf(sum, T == 2 ? (float)D : 1.0f, *bias_absmax * INV2PI);
             track = __any(!(bound <= UMAX));
             const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
             const float sx = pow2i(kx);
