@@ -62,6 +62,7 @@ struct FchlArgs {
 constexpr int TCH_MAX = 1024;  // longest triple list that the one-wavefront forward kernel is given
 constexpr size_t FORWARD_LDS = 5120;   // its LDS request: 32 wavefronts share the 160 KB of a CU
 constexpr int TCH_WIDE = 768;  // largest of the several-wavefront one (12 KB): beyond, the triple list is taken in chunks
+constexpr int TCH_LEAST = 192; // and its smallest, for capacities that leave no more (up to 1270 neighbours at the default grids)
 constexpr float PI_F = 3.14159265358979323846f;
 // three floats read from a 16-byte-aligned LDS entry with a single 12-byte instruction (a 16-byte
 // read of the same entry occupies the LDS pipe a third longer)
@@ -977,7 +978,10 @@ __host__ __device__ __forceinline__ int force_copies(int nn) {
 // neighbours' force array as 64 consecutive triples can meet the same neighbour (force_copies).  An instruction's lanes then
 // read, add and write different words, one 16-byte record each, and the copies are summed at the end.  NW wavefronts
 // per atom share out the triples: see wavefronts_per_atom.
-template <int NW>
+// COMPACT (one wavefront): the form for capacities at which the copies above do not fit.  [cap] records of three floats hold
+// as many copies as the atom's own neighbours leave room for, at least one; where an instruction's lanes would need more, its
+// s-rows take turns.
+template <int NW, bool COMPACT = false>
 __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const float* __restrict__ grad_rep,
                                                               float* __restrict__ grad_X) {
     extern __shared__ float smem[];
@@ -995,9 +999,13 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // (1 / r, fc, dfc / dr, element type); first in LDS, 16-byte aligned
     float* recA = smem;
     float* recB = recA + 4 * a.cap;
-    float* force = recB + 4 * a.cap;           // [NW][tcap][4] forces on the neighbours: copies of nn records
-    float* gin3 = force + 4 * NW * a.tcap;   // [NE3][2] incoming gradient of the three-body bins (cos, sin), see below; 8-byte aligned
-    int* sj = (int*)(gin3 + 2 * NE3);          // [cap] atom index of neighbour j
+    static_assert(!COMPACT || NW == 1, "the compact force records belong to one wavefront");
+    constexpr int FR = COMPACT ? 3 : 4;        // floats per force record
+    // [NW][tcap][FR] forces on the neighbours: copies of nn records (compact: behind gin3, which the 16-byte records precede)
+    float* force = recB + 4 * a.cap + (COMPACT ? 2 * NE3 : 0);
+    float* gin3 = COMPACT ? recB + 4 * a.cap : force + FR * NW * a.tcap;   // [NE3][2] incoming gradient of the three-body bins
+                                                                           // (cos, sin), see below; 8-byte aligned
+    int* sj = (int*)(COMPACT ? force + FR * a.tcap : gin3 + 2 * NE3);      // [cap] atom index of neighbour j
     int* goff = sj + a.cap;              // [ns+1] slices of the sorted neighbour list by type
     int* wcount = goff + ns + 1;         // [ns * NW] scratch of the staging
     float* slnRs2 = (float*)(wcount + (NW > 1 ? ns * NW : 0));   // [nRs2]
@@ -1023,8 +1031,22 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     }
     const float rs2v = lane < nRs2 ? a.Rs2[lane] : 1.0f;
     const float rs3v = lane < nRs3 ? a.Rs3[lane] : 0.0f;
-    float4* mine = reinterpret_cast<float4*>(force) + wave * a.tcap;   // this wavefront's copies
-    for (int t = lane; t < a.tcap; t += QMLL_WAVE) mine[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float* mine = force + FR * wave * a.tcap;   // this wavefront's copies
+    auto set_force = [&](float* p, float x, float y, float z) {
+        if constexpr (COMPACT) p[0] = x, p[1] = y, p[2] = z;
+        else *reinterpret_cast<float4*>(p) = make_float4(x, y, z, 0.0f);
+    };
+    auto add_force = [&](float* p, float x, float y, float z) {
+        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (COMPACT) f.x = p[0], f.y = p[1], f.z = p[2];
+        else f = *reinterpret_cast<float4*>(p);
+        f.x += x;
+        f.y += y;
+        f.z += z;
+        if constexpr (COMPACT) set_force(p, f.x, f.y, f.z);
+        else *reinterpret_cast<float4*>(p) = f;
+    };
+    for (int t = lane; t < a.tcap; t += QMLL_WAVE) set_force(mine + FR * t, 0.f, 0.f, 0.f);
     const float inv_rc = frcp(a.p.rcut);
     auto emit = [&](int pos, int, int, int e, int j, float dx, float dy, float dz, float r2) {
         const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
@@ -1128,7 +1150,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
                 gix += tot * ux;
                 giy += tot * uy;
                 giz += tot * uz;
-                mine[j] = make_float4(-tot * ux, -tot * uy, -tot * uz, 0.0f);   // each lane owns its own j here
+                set_force(mine + FR * j, -tot * ux, -tot * uy, -tot * uz);   // each lane owns its own j here
             }
         }
     }
@@ -1143,13 +1165,17 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     const int ntrip = nn * (nn - 1) / 2;
     const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
     const float d3 = a.p.three_body_decay;
+    // copies of the force records that this atom uses: one for every s-row of an instruction, or as many as there is room for
+    auto copies = [&] { return COMPACT ? min(force_copies(nn), idiv_small(a.tcap, max(nn, 1))) : force_copies(nn); };
     for (int tt = tid; tt < ntrip; tt += NT) {
         // tt = s nn + j: the pair {j, j + s + 1 mod nn} (when nn is even, the first half of the last s)
         const int s = idiv_small(tt, nn), j = tt - __mul24(s, nn);
         int k = j + s + 1;
         if (k >= nn) k -= nn;
         // the copy: 64 consecutive tt meet a neighbour once per s
-        float4* own = mine + __mul24(s - idiv_small(tt - lane, nn), nn);
+        const int row = s - idiv_small(tt - lane, nn);
+        const int turn = COMPACT ? idiv_small(row, copies()) : 0;
+        float* own = mine + FR * __mul24(COMPACT ? row - __mul24(turn, copies()) : row, nn);
         const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
         const float ia = Bj.x, ib = Bk.x;
         const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
@@ -1226,18 +1252,17 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
         giy = fmaf(ea, Aj.y, fmaf(eb, Ak.y, giy));
         giz = fmaf(ea, Aj.z, fmaf(eb, Ak.z, giz));
         // force on j: ec (d_ik - d_ij) - ea d_ij, on k: -ec (d_ik - d_ij) - eb d_ik
-        float4 f = own[j];
-        f.x += fmaf(ec, cx, -ea * Aj.x);
-        f.y += fmaf(ec, cy, -ea * Aj.y);
-        f.z += fmaf(ec, cz, -ea * Aj.z);
-        own[j] = f;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next read sees every lane's write (LDS instructions run in order)
-        f = own[k];
-        f.x += fmaf(-ec, cx, -eb * Ak.x);
-        f.y += fmaf(-ec, cy, -eb * Ak.y);
-        f.z += fmaf(-ec, cz, -eb * Ak.z);
-        own[k] = f;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const float jx = fmaf(ec, cx, -ea * Aj.x), jy = fmaf(ec, cy, -ea * Aj.y), jz = fmaf(ec, cz, -ea * Aj.z);
+        const float kx = fmaf(-ec, cx, -eb * Ak.x), ky = fmaf(-ec, cy, -eb * Ak.y), kz = fmaf(-ec, cz, -eb * Ak.z);
+        const int turns = COMPACT ? idiv_small(force_copies(nn) + copies() - 1, copies()) : 1;
+        for (int now = 0; now < turns; ++now) {
+            if (!COMPACT || now == turn) {
+                add_force(own + FR * j, jx, jy, jz);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next read sees every lane's write (LDS instructions run in order)
+                add_force(own + FR * k, kx, ky, kz);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
     }
     __syncthreads();
     gix = wave_sum(gix);
@@ -1249,12 +1274,12 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
         atomicAdd(&gm[i * 3 + 1], giy);
         atomicAdd(&gm[i * 3 + 2], giz);
     }
-    const int ncopies = force_copies(nn);
+    const int ncopies = copies();
     for (int it = tid; it < 3 * nn; it += NT) {
         const int x = idiv_small(it, 3), c = it - 3 * x;
         float sum = 0.0f;
         for (int w = 0; w < NW; ++w)
-            for (int q = 0; q < ncopies; ++q) sum += force[4 * (w * a.tcap + q * nn + x) + c];
+            for (int q = 0; q < ncopies; ++q) sum += force[FR * (w * a.tcap + q * nn + x) + c];
         atomicAdd(&gm[sj[x] * 3 + c], sum);
     }
 }
@@ -1621,8 +1646,13 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     for (int nw = wavefronts_per_atom(A, alltrip, big); nw > 1 || big; nw /= 2) {
         // the table holds the triple list, or 12 KB of it at a time
         a.tcap = alltrip <= TCH_WIDE ? (int)alltrip : TCH_WIDE;
-        const size_t lds = sizeof(float) * (4 * (size_t)(a.tcap + 1) + 12 * (size_t)a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1 +
-                                            (size_t)ns * nw + (nw > 1 ? (size_t)np * nw * 2 * prm->nRs3 : 0));
+        size_t lds = sizeof(float) * (4 * (size_t)(a.tcap + 1) + 12 * (size_t)a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1 +
+                                      (size_t)ns * nw + (nw > 1 ? (size_t)np * nw * 2 * prm->nRs3 : 0));
+        if (nw == 1 && lds > LDS_LIMIT) {      // room for the neighbours of a large capacity: smaller pieces of the list
+            const size_t less = std::min((lds - LDS_LIMIT + 15) / 16, (size_t)std::max(a.tcap - TCH_LEAST, 0));
+            a.tcap -= (int)less;
+            lds -= 16 * less;
+        }
         if (lds > LDS_LIMIT) {          // many elements with fine grids: fewer wavefronts, fewer partial blocks
             QMLL_REQUIRE(nw > 1 || !big, QMLL_ERR_INVALID,
                          "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
@@ -1643,6 +1673,8 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     const int unit = prm->nRs3 < 64 ? 64 / prm->nRs3 : 1;
     a.tcap = (int)std::max<long long>(std::min(alltrip + np * (unit - 1), std::max(room - unit, 128LL)), a.cap);
     a.tcap = (a.tcap + unit - 1) / unit * unit;
+    const int least = (a.cap + unit - 1) / unit * unit;          // the two-body factors of the neighbours lie there first
+    while (a.tcap > least && rest + 16 * (size_t)a.tcap > LDS_LIMIT) a.tcap -= unit;
     const size_t lds = rest + 16 * (size_t)a.tcap;
     QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID,
                  "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
@@ -1679,14 +1711,18 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     const long long maxnn = nlist ? a.cap : a.cap - 1;
     for (int nw = std::min(4, wavefronts_per_atom(A, maxnn * (maxnn - 1) / 2, a.cap > 54));; nw /= 2) {
         // two records [cap][4], atom indices, force copies, type offsets, grids, the bins' constant factors, the gradient row
-        const size_t lds = sizeof(float) * ((size_t)9 * a.cap + 4 * (size_t)nw * a.tcap + prm->nspecies + 1 +
-                                            (nw > 1 ? (size_t)prm->nspecies * nw : 0) + prm->nRs2 + 2 * prm->nRs3 + R);
-        if (lds > LDS_LIMIT) {
-            QMLL_REQUIRE(nw > 1, QMLL_ERR_INVALID,
-                         "qmll_fchl19_vjp: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
-            continue;
-        }
+        const size_t shared = (size_t)9 * a.cap + prm->nspecies + 1 + prm->nRs2 + 2 * prm->nRs3 + R;
+        const size_t lds = sizeof(float) * (shared + 4 * (size_t)nw * a.tcap + (nw > 1 ? (size_t)prm->nspecies * nw : 0));
+        if (lds > LDS_LIMIT && nw > 1) continue;
         hipStream_t st = (hipStream_t)stream;
+        if (lds > LDS_LIMIT) {        // beyond about 900 neighbours: one three-float record for each
+            a.tcap = a.cap;
+            const size_t compact = sizeof(float) * (shared + 3 * (size_t)a.cap);
+            QMLL_REQUIRE(compact <= LDS_LIMIT, QMLL_ERR_INVALID,
+                         "qmll_fchl19_vjp: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", compact, n, R, LDS_LIMIT);
+            hipLaunchKernelGGL((fchl19_vjp_kernel<1, true>), dim3(A), dim3(64), compact, st, a, grad_rep, grad_X);
+            break;
+        }
         if (nw == 4) hipLaunchKernelGGL(fchl19_vjp_kernel<4>, dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);
         else if (nw == 2) hipLaunchKernelGGL(fchl19_vjp_kernel<2>, dim3(A), dim3(128), lds, st, a, grad_rep, grad_X);
         else hipLaunchKernelGGL(fchl19_vjp_kernel<1>, dim3(A), dim3(64), lds, st, a, grad_rep, grad_X);

@@ -77,3 +77,55 @@ def test_every_neighbour_count_has_its_force_copies(natoms):
     charges = [rng.choice([1, 6], natoms)]
     for copies in (1, 2050 // natoms + 1):
         check(coords, charges, [1, 6], copies, False, nRs2=3, nRs3=3)
+
+
+@pytest.mark.parametrize("species,forward,backward", [([1, 6, 8], 1268, 1333), ([1, 6, 7, 8, 9], 1259, 1299)])
+def test_capacities_up_to_the_limit_of_the_lds(species, forward, backward):
+    """Small molecules padded to the largest capacities at the default grids: smaller tables and compact force records before
+    a refusal."""
+    from qml_lightning_amd import ops
+    rng = np.random.default_rng(8)
+    prm = oracle_prm(species)
+    coords = [helpers.random_geometry(rng, 19, 6.0, 0.9), helpers.random_geometry(rng, 2, 3.0, 0.9)]
+    X, Z, aid, mid, nat = make_batch(coords, [rng.choice(species, len(c)) for c in coords])
+    cnt, nl = fchl19.neighbours(X, nat, prm.rcut)
+    ty = fchl19.element_types(Z, nat, prm.species)
+    rep = fchl19.forward(X, ty, aid, mid, nl, cnt, prm)
+    g = np.random.default_rng(2).normal(size=rep.shape)
+    v = np.einsum("mif,mijxf->mjx", g, fchl19.jacobian(X, ty, aid, mid, nl, cnt, prm))
+    n = X.shape[1]
+
+    def call(op, capacity, *first):
+        def pad(a):
+            return np.pad(a, [(0, 0), (0, capacity - n)] + [(0, 0)] * (a.ndim - 2), constant_values=0 if a.ndim == 3 else -1)
+        return op(*[t32(pad(f)) for f in first], t32(pad(X)), ti32(pad(ty)), None, None, ti32(aid), ti32(mid), ti32(nat),
+                  t32(prm.Rs2), t32(prm.Rs3), gpu_prm(prm))[:, :n]
+    for capacity in (forward - 170, forward):
+        close(call(ops.fchl_forward, capacity), rep, REL_REP, "rep, capacity %d" % capacity)
+    for capacity in (backward - 400, backward - 380, backward):
+        close(call(ops.fchl_vjp, capacity, g), v, REL_EF, "vjp, capacity %d" % capacity)
+    for op, first in ((ops.fchl_forward, ()), (ops.fchl_vjp, (g,))):
+        with pytest.raises(RuntimeError, match="LDS"):
+            call(op, backward + 1, *first)
+
+
+def test_a_thousand_neighbours_and_few():
+    """1200 atoms, listed one in the middle (some 650 neighbours: its force records take turns) and one at a corner."""
+    from qml_lightning_amd import ops
+    rng = np.random.default_rng(9)
+    species = [1, 8]
+    prm = oracle_prm(species, nRs2=2, nRs3=2)
+    sites = np.stack(np.unravel_index(rng.permutation(1331)[:1200], (11, 11, 11)), 1) * 1.1
+    X, Z, aid, mid, nat = make_batch([sites + rng.uniform(-0.15, 0.15, sites.shape)], [rng.choice(species, 1200)])
+    r = np.linalg.norm(X[0] - X[0].mean(0), axis=1)
+    aid, mid = np.array([r.argmin(), r.argmax()]), np.array([0, 0])
+    cnt, nl = fchl19.neighbours(X, nat, prm.rcut)
+    assert cnt[0, aid[0]] > 600 and cnt[0, aid[1]] < 250
+    ty = fchl19.element_types(Z, nat, prm.species)
+    rep = fchl19.forward(X, ty, aid, mid, nl, cnt, prm)
+    g = np.random.default_rng(2).normal(size=rep.shape)
+    J = fchl19.jacobian(X, ty, aid, mid, nl, cnt, prm)
+    v = np.einsum("if,ijxf->jx", g[0, aid], J[0, aid])[None]
+    args = (t32(X), ti32(ty), None, None, ti32(aid), ti32(mid), ti32(nat), t32(prm.Rs2), t32(prm.Rs3), gpu_prm(prm))
+    close(ops.fchl_forward(*args)[0, aid], rep[0, aid], REL_REP, "rep")
+    close(ops.fchl_vjp(t32(g), *args), v, REL_EF, "vjp")
