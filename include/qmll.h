@@ -379,22 +379,21 @@ int qmll_sorf_energy_sorted(const float* x, const int* type_offsets, const int* 
                             const float* bias, const float* alpha, const float* bias_absmax, int A, int ne, int d, int S,
                             int T, float normalisation, float* e_slots, float* gx, qmll_stream_t stream);
 
-/* qmll_sorf_energy_sorted on the half-precision matrix cores (large batches; d = 64 or 128, T = 1 or 2, diagonals of
- * +-1), with constants of the model prepared ONCE: signs = the output of qmll_sorf_signs (qmll_sorf_signs_bytes
- * bytes, its last 16 zeroed by the caller; afterwards the int at their start counts diagonal entries that are not +-1, and
- * unless it is zero the form must not be used; 0 bytes: no kernel takes the shape), bias_rev f32 [ne,S*d] = bias / 2 pi,
- * alpha_scaled f32 [S*d + 1] = the output of qmll_sorf_alpha, bias_absmax as above (required here).  Arrays 16-byte
- * aligned.  work: device memory of qmll_sorf_matrix_workspace_bytes, for this call alone.  fp32 operands are split into
- * two fp16 parts (both rounded to nearest, fp32 accumulation). */
+/* qmll_sorf_energy_sorted on the half-precision matrix cores (large batches; d = 64 or 128, T = 1 or 2; diagonals of +-1:
+ * where the device finds others the call runs as qmll_sorf_energy_sorted does).  x, D, work and gx 16-byte aligned.
+ * work: device memory of qmll_sorf_matrix_workspace_bytes (0: no kernel takes the shape), for this call alone; the signs in
+ * the form that is multiplied with, bias in revolutions and alpha behind a power of two are made there by every call.  fp32
+ * operands are split into two fp16 parts (both rounded to nearest, fp32 accumulation).  Four launches, no synchronisation:
+ * it can be captured. */
 size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, int d, int with_grad);
-size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d);
 int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad);   /* 1: faster than qmll_sorf_energy_sorted */
+int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,
+                            const float* alpha, int A, int ne, int d, int S, int T, float normalisation, void* work,
+                            size_t work_bytes, float* e_slots, float* gx, qmll_stream_t stream);
+/* The first part of those forms alone, for whoever wants to look at them: the H_16 blocks behind the signs of D, then a
+ * float per (element, stack): the largest entry of H D_1 H (T = 1: 1), infinite where a diagonal is not +-1. */
+size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d);
 int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void* out, size_t out_bytes, qmll_stream_t stream);
-int qmll_sorf_alpha(const float* alpha, int S, int d, float* out, qmll_stream_t stream);
-int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const void* signs,
-                            const float* bias_rev, const float* alpha_scaled, const float* bias_absmax, int A, int ne, int d, int S,
-                            int T, float normalisation, float* work, size_t work_bytes, float* e_slots, float* gx,
-                            qmll_stream_t stream);
 
 /* ---- RFF ------------------------------------------------------------------------- */
 

@@ -76,9 +76,8 @@ PROTOTYPES = {
     "qmll_sorf_signs_bytes": [c_int, c_int, c_int, c_int],
     "qmll_sorf_matrix_pays": [c_int] * 6,
     "qmll_sorf_signs": [P, c_int, c_int, c_int, c_int, P, c_size_t, P],
-    "qmll_sorf_alpha": [P, c_int, c_int, P, P],
     "qmll_sorf_matrix_workspace_bytes": [c_int] * 6,
-    "qmll_sorf_energy_matrix": [P, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, P, c_size_t, P, P, P],
+    "qmll_sorf_energy_matrix": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, P, c_size_t, P, P, P],
     "qmll_rff_features": [P, P, P, P, c_int, c_int, c_int, c_int, P, P],
     "qmll_rff_derivative_features": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P],
     "qmll_rff_rows": [POINTER(RffElement), c_int, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P],

@@ -29,6 +29,11 @@ void qmll_set_error(const char* fmt, ...);
         }                                                                               \
     } while (0)
 
+// qmll_sorf_energy_sorted without a bound on |bias|, on the device only if *only_if is not 0 (64 or 128 components)
+int qmll_sorf_rows_if(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,
+                      const float* alpha, int A, int ne, int d, int S, int T, float normalisation, const int* only_if, float* e_slots,
+                      float* gx, hipStream_t stream);
+
 static inline bool qmll_is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 static inline int qmll_log2(int v) {
     int l = 0;

@@ -594,12 +594,12 @@ constexpr int ROWS_NA = 4;   // atoms per workgroup = rows of 16 lanes per wavef
 // as for T = 1, the later ones are fetched where they are used (forward and again in the adjoint).
 // NW: wavefronts per workgroup, which share out the stacks (16 for a few atoms: a molecule then takes
 // a quarter of the time, its stacks being the only parallelism there is).
-template <int LOG2D, bool WITH_GRAD, bool MULTI, int NW = SORF_WAVES>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >= 8 ? 4 : 1, 8))) void sorf_energy_rows_kernel(
-    const float* __restrict__ x, const float* __restrict__ D, const float* __restrict__ bias,
+template <int LOG2D, bool WITH_GRAD, bool MULTI, int NW>
+__device__ __forceinline__ void sorf_energy_rows(
+    int block, int nblocks, const float* __restrict__ x, const float* __restrict__ D, const float* __restrict__ bias,
     const float* __restrict__ alpha, const float* __restrict__ bias_absmax, const int* __restrict__ out_index,
-    const int* __restrict__ type_offsets, int ne, int A, int S, int T_, float scale, float normf,
-    float* __restrict__ e_atom, float* __restrict__ gx) {
+    const int* __restrict__ type_offsets, int ne, int A, int S, int T_, float scale, float normf, float* __restrict__ e_atom,
+    float* __restrict__ gx) {
     const int T = MULTI ? T_ : 1;
     constexpr int d = 1 << LOG2D;
     constexpr int EPL = d / 16;                 // registers per lane
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >
     // the NA consecutive atoms of this workgroup; with type_offsets they never straddle two types
     int row0, rows;
     if (type_offsets != nullptr) {
-        int b = blockIdx.x, t = 0;
+        int b = block, t = 0;
         rows = 0;
         for (; t < ne; ++t) {
             const int o0 = type_offsets[t], o1 = type_offsets[t + 1];
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >
             // a workgroup past the last tile (the launch adds at least one): its share of the gradient
             // rows past the last atom of a known element, which are zero
             if constexpr (WITH_GRAD) {
-                const int spare = b, nspare = (int)gridDim.x - ((int)blockIdx.x - b);
+                const int spare = b, nspare = nblocks - (block - b);
                 for (int r = type_offsets[ne] + spare; r < A; r += nspare)
                     for (int c = threadIdx.x; c < d; c += 64 * NW) gx[(size_t)r * d + c] = 0.0f;
             }
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >
         D += (size_t)t * T * S * d;
         bias += (size_t)t * S * d;
     } else {
-        row0 = blockIdx.x * NA;
+        row0 = block * NA;
         rows = min(NA, A - row0);
         if (rows <= 0) return;
     }
@@ -871,6 +871,30 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >
     }
 }
 
+template <int LOG2D, bool WITH_GRAD, bool MULTI, int NW = SORF_WAVES>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >= 8 ? 4 : 1, 8))) void sorf_energy_rows_kernel(
+    const float* __restrict__ x, const float* __restrict__ D, const float* __restrict__ bias,
+    const float* __restrict__ alpha, const float* __restrict__ bias_absmax, const int* __restrict__ out_index,
+    const int* __restrict__ type_offsets, int ne, int A, int S, int T, float scale, float normf, float* __restrict__ e_atom,
+    float* __restrict__ gx) {
+    sorf_energy_rows<LOG2D, WITH_GRAD, MULTI, NW>((int)blockIdx.x, (int)gridDim.x, x, D, bias, alpha, bias_absmax, out_index, type_offsets,
+                                                  ne, A, S, T, scale, normf, e_atom, gx);
+}
+
+// the same where *only_if is not 0, by a grid small enough to cost nothing where it is: the workgroups take tile after tile
+template <int LOG2D, bool WITH_GRAD, bool MULTI>
+__global__ __launch_bounds__(SORF_THREADS) void sorf_energy_rows_if_kernel(
+    const int* __restrict__ only_if, int nblocks, const float* __restrict__ x, const float* __restrict__ D,
+    const float* __restrict__ bias, const float* __restrict__ alpha, const int* __restrict__ out_index,
+    const int* __restrict__ type_offsets, int ne, int A, int S, int T, float scale, float normf, float* __restrict__ e_atom,
+    float* __restrict__ gx) {
+    if (*only_if == 0) return;
+    for (int block = (int)blockIdx.x; block < nblocks; block += (int)gridDim.x) {
+        sorf_energy_rows<LOG2D, WITH_GRAD, MULTI, SORF_WAVES>(block, nblocks, x, D, bias, alpha, nullptr, out_index, type_offsets, ne, A, S,
+                                                              T, scale, normf, e_atom, gx);
+        __syncthreads();
+    }
+}
 
 // ---- two-op contract in the 16-lane-row layout (64 <= d <= 256) ---------------------------
 // The four rows of a wavefront carry four consecutive stacks of ONE atom, so a workgroup has
@@ -1612,6 +1636,10 @@ extern "C" int qmll_sorf_adjoint(const float* g, const float* D, int A, int d, i
     return QMLL_OK;
 }
 
+// workgroups of the rows kernel with type offsets: up to ne tiles more than A / 4 (every type rounds up), and 1 to 64 that zero
+// the gradient rows past the last atom of a known element
+static int rows_tiles(int A, int ne) { return (A + ROWS_NA - 1) / ROWS_NA + ne + (A >= 65536 ? 64 : (A >> 10) + 1); }
+
 static int launch_fused(const char* who, const float* x, const float* D, const float* bias, const float* alpha,
                         const float* bias_absmax, const int* out_index, const int* types, const int* type_offsets, int ne, int A, int d, int S,
                         int T, float normalisation, float* e_atom, float* gx, hipStream_t stream) {
@@ -1620,10 +1648,7 @@ static int launch_fused(const char* who, const float* x, const float* D, const f
     if (d >= 64 && d <= 256 && types == nullptr) {
         // 4 to 16 registers per lane, atoms groupable by element: the instruction-lean kernel
         // (four atoms per workgroup)
-        // with type offsets: up to ne tiles more than A / 4 (every type rounds up), and 1 to 64 workgroups
-        // that zero the gradient rows past the last atom of a known element
-        const int zero_groups = A >= 65536 ? 64 : (A >> 10) + 1;
-        const dim3 grid((A + ROWS_NA - 1) / ROWS_NA + (type_offsets ? ne + zero_groups : 0));
+        const dim3 grid(type_offsets ? rows_tiles(A, ne) : (A + ROWS_NA - 1) / ROWS_NA);
         // up to some 1500 atoms the chip has idle SIMDs: sixteen wavefronts per workgroup share out the stacks
         // (measured at d = 128, 128 stacks: 17.4 -> 13.8 us at 1008 atoms, equal at 2016, slower from 2688 on)
         const bool few = A <= 1536 && S >= 64 && d <= 128 && T == 1;
@@ -1699,6 +1724,31 @@ extern "C" int qmll_sorf_energy_sorted(const float* x, const int* type_offsets, 
                  "qmll_sorf_energy_sorted: null pointer");
     return launch_fused("qmll_sorf_energy_sorted", x, D, bias, alpha, bias_absmax, sorted_slots, nullptr, type_offsets, ne, A, d, S, T,
                         normalisation, e_slots, gx, (hipStream_t)stream);
+}
+
+int qmll_sorf_rows_if(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,
+                      const float* alpha, int A, int ne, int d, int S, int T, float normalisation, const int* only_if, float* e_slots,
+                      float* gx, hipStream_t stream) {
+    const float scale = normalisation * hnorm(d, T), normf = sqrtf(2.0f / ((float)S * (float)d));
+    const int nblocks = rows_tiles(A, ne);
+    const dim3 grid(nblocks < 2048 ? nblocks : 2048);          // eight workgroups of four wavefronts per CU
+    auto launch = [&](auto log2d, auto grad, auto multi) {
+        hipLaunchKernelGGL((sorf_energy_rows_if_kernel<decltype(log2d)::value, decltype(grad)::value, decltype(multi)::value>), grid,
+                           dim3(SORF_THREADS), 0, stream, only_if, nblocks, x, D, bias, alpha, sorted_slots, type_offsets, ne, A, S, T,
+                           scale, normf, e_slots, gx);
+    };
+    auto by_transforms = [&](auto log2d, auto grad) {
+        if (T == 1) launch(log2d, grad, std::false_type{});
+        else launch(log2d, grad, std::true_type{});
+    };
+    auto by_grad = [&](auto log2d) {
+        if (gx) by_transforms(log2d, std::true_type{});
+        else by_transforms(log2d, std::false_type{});
+    };
+    if (d == 64) by_grad(std::integral_constant<int, 6>{});
+    else by_grad(std::integral_constant<int, 7>{});
+    QMLL_CHECK_LAUNCH("qmll_sorf_energy_matrix");
+    return QMLL_OK;
 }
 
 extern "C" int qmll_derivative_features(const double* cos_derivs, double normalisation, const int* mol_index,

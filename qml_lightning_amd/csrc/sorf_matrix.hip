@@ -10,11 +10,11 @@
 // lane's four entries, high and low, are its eight k values), so nothing ever crosses lanes.
 //
 // The first operand of a stack never changes but for the signs of its diagonal: x is split once per atom, and the
-// signs go into the H_16 block, which is prepared per model (qmll_sorf_signs: a block per (element, stack, transform), the
+// signs go into the H_16 block, which is prepared per call (sorf_prepare_kernel: a block per (element, stack, transform), the
 // diagonal must hold +-1) and moved into LDS by direct loads, a round ahead.  The gradient is split per stack (a
 // conversion, a mixed-precision subtraction and a conversion per value); both parts are rounded to nearest, so a
 // value keeps 2^-24 of itself, as in fp32.  Power-of-two scales keep everything in fp16's range: x per atom
-// (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per model.
+// (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per call.
 //
 // Instruction issue bounds it, as it does the kernel without matrix instructions (sorf_energy_rows_kernel, which at
 // d = 128 spends 162 vector instructions per 4 atoms and stack, 64 of them cross-lane ones at half rate): here 16 atoms
@@ -26,9 +26,9 @@
 // A tile (64 atoms of one element) through all stacks is too coarse a unit: with the three workgroups a CU holds, the last
 // of two rounds of tiles left most of the chip idle.  A workgroup takes an equal share of all (tile, round of stacks) units
 // instead; a tile that two or more shares meet in is written in parts, which sorf_parts_kernel adds up in order.
-// Measured with the gradient / energies only, rows kernel -> whole tiles -> shares, at d = 128, 128 stacks: 86016 atoms
-// 762 -> 690 -> 643 us / 457 -> 324 -> 297; 24000 atoms 222 -> 269 -> 207 / 133 -> 137 -> 97; 131500 atoms 1166 -> 1004 -> 963 /
-// 698 -> 462 -> 449; 86016 x 64 x 128: 361 -> 317 -> 300 / 230 -> 149 -> 139; two transforms, 33000 x 128 x 32: 147 -> 164 -> 135 / 77 -> 81 -> 66.  (At d = 256 the
+// Measured with the gradient / energies only, rows kernel -> this call, at d = 128, 128 stacks: 86016 atoms 764 -> 653 us / 456 -> 305;
+// 24000 atoms 222 -> 214 / 133 -> 108; two transforms, 32 stacks, 33000 atoms 148 -> 143 / 78 -> 75, 86016 atoms 369 -> 314 / 194 -> 148;
+// d = 64, 128 stacks, 86016 atoms 360 -> 309 / 230 -> 147.  Of that 5 us go to the forms and 3 to 4 to the launch behind.  (At d = 256 the
 // registers leave two wavefronts per SIMD and it is no faster: 880 -> 890 us, so the rows kernel stays.)
 #include <algorithm>
 #include <type_traits>
@@ -55,45 +55,94 @@ constexpr int log2nb() { return NB == 4 ? 2 : 3; }
 // one 16-point block operand: half t of lane (i, q) is sign * H_16[i][4q + t % 4]
 __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h) & 1; }
 
-// images [ne][S][T][NB][64 lanes][8 halves]; bad counts diagonal entries that are not +-1
-template <int D>
-__global__ __launch_bounds__(256) void sorf_signs_kernel(const float* __restrict__ Dmat, int T, int S, half8_t* __restrict__ images,
-                                                         int* __restrict__ bad) {
-    constexpr int NB = D / 16;
-    const int s = blockIdx.x, m = blockIdx.y, e = blockIdx.z;
-    const float* row = Dmat + (((size_t)e * T + m) * S + s) * D;
-    half8_t* dst = images + (((size_t)e * S + s) * T + m) * NB * 64;
-    for (int t = threadIdx.x; t < NB * 64; t += 256) {
-        const int b = t >> 6, lane = t & 63, i = lane & 15, q = lane >> 4;
-        half8_t v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float sd = row[16 * b + 4 * q + r];
-            const _Float16 hv = (_Float16)(h16_negative(i, 4 * q + r) ? -sd : sd);
-            v[r] = hv;
-            v[r + 4] = hv;
-            if (i == 0 && fabsf(sd) != 1.0f) atomicAdd(bad, 1);
-        }
-        dst[t] = v;
-    }
-}
+// What a launch needs of the model beside its tensors.  Made by every call (sorf_prepare_kernel, 4 us of 150 and more): nothing
+// is kept that a write to the tensors could leave behind, and no other stream or captured graph has to wait for it.
+struct Forms {
+    half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal
+    float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
+    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2
+    float* alpha;         // [S][d] 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
+    int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
+};
 
-// alpha 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
-__global__ __launch_bounds__(1024) void sorf_alpha_kernel(const float* __restrict__ alpha, int F, int lognb, float* __restrict__ out) {
-    __shared__ float wmax[16];
-    float m = 0.0f;
-    for (int t = threadIdx.x; t < F; t += 1024) m = fmaxf(m, finite_abs(alpha[t]));
+__device__ __forceinline__ float workgroup_max(float m, float* wmax) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    __syncthreads();
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
     m = wmax[0];
+    for (int w = 1; w < (int)blockDim.x >> 6; ++w) m = fmaxf(m, wmax[w]);
+    return m;
+}
+
+// workgroup 0: alpha; then one per (element, stack).  bias and alpha may be null: the images and bounds alone
+constexpr int PREP_THREADS = 512;
+template <int D, int T>
+__global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float* __restrict__ Dmat, const float* __restrict__ bias,
+                                                                    const float* __restrict__ alpha, int S, Forms f) {
+    constexpr int NB = D / 16;
+    __shared__ float wmax[PREP_THREADS / 64];
+    __shared__ float h[D];
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        if (alpha == nullptr) return;
+        float m = 0.0f;
+#pragma unroll 8
+        for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
+        m = workgroup_max(m, wmax);
+        const int k = max(scale_exponent(m) - log2nb<NB>(), -126);
+        const float sc = pow2i(k);
+#pragma unroll 8
+        for (int t = tid; t < S * D; t += PREP_THREADS) f.alpha[t] = alpha[t] * sc;
+        if (tid == 0) f.alpha[(size_t)S * D] = pow2i(-k);
+        return;
+    }
+    const int e = (blockIdx.x - 1) / S, s = blockIdx.x - 1 - e * S;
+    bool unfit = false;
 #pragma unroll
-    for (int w = 1; w < 16; ++w) m = fmaxf(m, wmax[w]);
-    const int k = max(scale_exponent(m) - lognb, -126);
-    const float sc = pow2i(k);
-    for (int t = threadIdx.x; t < F; t += 1024) out[t] = alpha[t] * sc;
-    if (threadIdx.x == 0) out[F] = pow2i(-k);
+    for (int m = 0; m < T; ++m) {
+        const float* row = Dmat + (((size_t)e * T + m) * S + s) * D;
+        half8_t* dst = f.images + (((size_t)e * S + s) * T + m) * NB * 64;
+        for (int t = tid; t < NB * 64; t += PREP_THREADS) {
+            const int b = t >> 6, lane = t & 63, i = lane & 15, q = lane >> 4;
+            half8_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float sd = row[16 * b + 4 * q + r];
+                const _Float16 hv = (_Float16)(h16_negative(i, 4 * q + r) ? -sd : sd);
+                v[r] = hv;
+                v[r + 4] = hv;
+                unfit |= !(fabsf(sd) == 1.0f);
+            }
+            dst[t] = v;
+        }
+    }
+    float largest = 1.0f;
+    if constexpr (T == 2) {
+        // entry (i, j) of H D_1 H is entry i ^ j of the transform of D_1's diagonal
+        if (tid < D) h[tid] = Dmat[(((size_t)e * T + 1) * S + s) * D + tid];
+        for (int o = 1; o < D; o <<= 1) {
+            __syncthreads();
+            if (tid < D / 2) {
+                const int a = (tid & ~(o - 1)) << 1 | (tid & (o - 1));
+                const float x = h[a], y = h[a + o];
+                h[a] = x + y;
+                h[a + o] = x - y;
+            }
+        }
+        __syncthreads();
+        largest = workgroup_max(tid < D ? fabsf(h[tid]) : 0.0f, wmax);
+    }
+    const bool any_unfit = __syncthreads_or(unfit);
+    if (bias != nullptr) {
+        const size_t at = ((size_t)e * S + s) * D;
+        for (int t = tid; t < D; t += PREP_THREADS) {
+            const float r = bias[at + t] * INV2PI;
+            f.bias[at + t] = r - rintf(r);
+        }
+    }
+    if (tid == 0) f.largest[(size_t)e * S + s] = any_unfit ? HUGE_VALF : largest;
 }
 
 // butterflies over the block index
@@ -181,7 +230,7 @@ template <int D, bool WITH_GRAD, int T>
 __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void sorf_energy_matrix_kernel(
     const float* __restrict__ x, const int* __restrict__ type_offsets, const int* __restrict__ out_index,
     const float* __restrict__ Dmat, const half8_t* __restrict__ images, const float* __restrict__ bias_rev,
-    const float* __restrict__ alpha_scaled, const float* __restrict__ bias_absmax, int ne, int A, int S, int nshares, float scale,
+    const float* __restrict__ alpha_scaled, const float* __restrict__ bounds, int ne, int A, int S, int nshares, float xs, float gscale,
     float normf, float* __restrict__ parts, float* __restrict__ e_slots, float* __restrict__ gx) {
     constexpr int NB = D / 16;
     using Buffer = StackBuffer<D, T>;
@@ -215,6 +264,11 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         if (u != ubeg) __syncthreads();                                 // the buffers of the tile before are free
         u += r1 - r0;
         const int s0 = r0 * SPB, s1 = min(S, r1 * SPB);
+        float largest = 0.0f;                                           // entry of H D_1 H of the element
+        for (int t = lane; t < S; t += 64) largest = fmaxf(largest, bounds[(size_t)type * S + t]);
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) largest = fmaxf(largest, __shfl_xor(largest, o, 64));
+        if (largest == HUGE_VALF) continue;                             // not +-1: the rows kernel behind this one writes all
 
         const float* Dt = Dmat + (size_t)type * T * S * D;
         const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
@@ -258,7 +312,6 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         {
             const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
             f4_t xv[NB];
-            const float xs = scale * INV2PI;
             float sum = 0.0f;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
@@ -271,9 +324,9 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             }
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
-            // every argument is at most sum |x| (times d for a second transform: an entry of H D H is a sum of d signs) + |bias|:
-            // where that stays below UMAX no stack looks at its arguments
-            const float bound = fmaf(sum, T == 2 ? (float)D : 1.0f, *bias_absmax * INV2PI);
+            // every argument is at most sum |x|, times the largest entry of H D_1 H for a second transform, + |bias|: where that
+            // stays below UMAX no stack looks at its arguments
+            const float bound = fmaf(sum, largest, 0.5f);
             track = __any(!(bound <= UMAX));
             const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
             const float sx = pow2i(kx);
@@ -392,7 +445,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             else parts[slot * SM_ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
         }
         if constexpr (WITH_GRAD) {
-            const float gs = -scale * normf * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
+            const float gs = gscale * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
             float* to = whole ? gx + (size_t)row0 * D : parts + slot * SM_ATOMS * (D + 1) + SM_ATOMS;
             float* gr = to + (size_t)in_tile * D + 4 * q;
 #pragma unroll
@@ -402,12 +455,21 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
 }
 
 // the tiles that were cut: workgroup g adds up the parts of the tile that begins in share g and ends in a later one, in order
+// (and the last one says whether the rows kernel has to take the call)
 template <int D, bool WITH_GRAD>
 __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__ type_offsets, const int* __restrict__ out_index, int ne,
-                                                         int rounds, const float* __restrict__ parts, float* __restrict__ e_slots,
-                                                         float* __restrict__ gx) {
+                                                         int S, int rounds, const float* __restrict__ parts, Forms f,
+                                                         float* __restrict__ e_slots, float* __restrict__ gx) {
     constexpr size_t SLOT = SM_ATOMS * (WITH_GRAD ? D + 1 : 1);
-    const int g = blockIdx.x, nshares = gridDim.x, ntiles = tile_count(type_offsets, ne);
+    const int g = blockIdx.x, nshares = (int)gridDim.x - 1;
+    if (g == nshares) {
+        bool unfit = false;
+        for (int t = threadIdx.x; t < ne * S; t += 256) unfit |= f.largest[t] == HUGE_VALF;
+        unfit = __syncthreads_or(unfit);
+        if (threadIdx.x == 0) *f.unfit = unfit;
+        return;
+    }
+    const int ntiles = tile_count(type_offsets, ne);
     const int ubeg = share_begin(g, nshares, ntiles, rounds), uend = share_begin(g + 1, nshares, ntiles, rounds);
     if (ubeg == uend) return;
     const int tile = (uend - 1) / rounds, tbeg = tile * rounds, tend = tbeg + rounds;
@@ -448,82 +510,105 @@ static int matrix_shares(long long units, int with_grad) {
     return (int)std::min(units, (long long)SM_CUS * std::max(3ll, std::min(6ll, per_cu)));
 }
 
-extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, int d, int with_grad) {
-    if (A <= 0 || qmll_sorf_signs_bytes(ne, T, S, d) == 0) return 0;
-    return (size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * 2 * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float);
+// the workspace of a call: the forms, every part of them 16-byte aligned, then the parts of the cut tiles; its size for base = null
+static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, int with_grad, Forms& f, float*& parts) {
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        char* p = (char*)((uintptr_t)base + at);
+        at += (bytes + 15) / 16 * 16;
+        return p;
+    };
+    f.images = (half8_t*)take((size_t)ne * T * S * (d / 16) * 1024);
+    f.largest = (float*)take((size_t)ne * S * sizeof(float));
+    f.unfit = (int*)take(sizeof(int));
+    f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
+    f.alpha = (float*)take(((size_t)S * d + 1) * sizeof(float));
+    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * 2 * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float));
+    return at;
 }
 
-// What this kernel gains per atom and stack has to carry a launch more and the parts of the cut tiles, 20 us with the gradient
-// and 10 us without.  Measured, rows kernel / this one, with the gradient: d = 128, 128 stacks, 16384 atoms 157 / 152 us (2.1e6 in
-// the units below), 24000 atoms 222 / 206; two transforms, 32 stacks, 16384 atoms 78 / 83 (1.05e6), 24000 atoms 108 / 102 (1.5e6); d = 64,
-// 128 stacks, 16384 atoms 76 / 79, 24000 atoms 105 / 102; 8 stacks, 131500 atoms 101 / 98.  Energies only: d = 128, 128 stacks, 4096
-// atoms 31 / 33 (0.52e6), 8192 atoms 51 / 48; two transforms, 32 stacks, 16384 atoms 42 / 41; 8 stacks, 86016 atoms 42 / 38.
+static int matrix_shape(int ne, int T, int S, int d) {
+    return ne > 0 && S > 0 && (T == 1 || T == 2) && (d == 64 || d == 128) && (long long)ne * S < (1ll << 31) - 1 &&
+           (long long)S * d < (1ll << 31);
+}
+
+extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, int d, int with_grad) {
+    Forms f;
+    float* parts;
+    return A <= 0 || !matrix_shape(ne, T, S, d) ? 0 : matrix_workspace(nullptr, A, ne, T, S, d, with_grad, f, parts);
+}
+
+// What this kernel gains per atom and stack has to carry three launches more and the parts of the cut tiles, 25 us with the
+// gradient and 15 us without.  Measured, rows kernel / this call, with the gradient: d = 128, 128 stacks, 12000 atoms 124 / 130 us (1.5e6
+// in the units below), 20000 atoms 191 / 186 (2.6e6); two transforms, 32 stacks, 24000 atoms 108 / 110 (1.5e6), 33000 atoms 148 / 143 (2.1e6);
+// d = 64, 128 stacks, 24000 atoms 107 / 112, 33000 atoms 144 / 138; 8 stacks, 86016 atoms 70 / 78 (0.7e6).  Energies only: d = 128, 128
+// stacks, 12000 atoms 69 / 70, 20000 atoms 112 / 94; two transforms, 32 stacks, 24000 atoms 58 / 60, 33000 atoms 78 / 75; d = 64, 128 stacks,
+// 12000 atoms 36 / 41 (0.8e6), 20000 atoms 57 / 52 (1.3e6).
 extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
-    if (qmll_sorf_signs_bytes(ne, T, S, d) == 0 || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
-    return (double)A * S * T * d / 128.0 >= (with_grad ? 1.6e6 : 0.8e6);
+    if (!matrix_shape(ne, T, S, d) || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
+    return (double)A * S * T * d / 128.0 >= (with_grad ? 2e6 : 1.5e6);
+}
+
+static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, const Forms& f,
+                           hipStream_t st) {
+    const dim3 grid(ne * S + 1), block(PREP_THREADS);
+    if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, f);
+    else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, f);
+    else if (T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, f);
+    else hipLaunchKernelGGL((sorf_prepare_kernel<128, 2>), grid, block, 0, st, D, bias, alpha, S, f);
 }
 
 extern "C" size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d) {
-    if (ne <= 0 || S <= 0 || (T != 1 && T != 2) || (d != 64 && d != 128)) return 0;
-    return (size_t)ne * T * S * (d / 16) * 1024 + 16;
+    return matrix_shape(ne, T, S, d) ? (size_t)ne * T * S * (d / 16) * 1024 + (size_t)ne * S * sizeof(float) : 0;
 }
 
 extern "C" int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void* out, size_t out_bytes, qmll_stream_t stream) {
-    QMLL_REQUIRE(qmll_sorf_signs_bytes(ne, T, S, d) > 0, QMLL_ERR_INVALID, "qmll_sorf_signs: no kernel takes ne=%d T=%d S=%d d=%d",
-                 ne, T, S, d);
+    QMLL_REQUIRE(matrix_shape(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: no kernel takes ne=%d T=%d S=%d d=%d", ne, T, S, d);
     QMLL_REQUIRE(D && out && ((uintptr_t)out & 15) == 0, QMLL_ERR_INVALID, "qmll_sorf_signs: null or misaligned pointer");
     QMLL_REQUIRE(out_bytes >= qmll_sorf_signs_bytes(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: output of %zu bytes, %zu are needed",
                  out_bytes, qmll_sorf_signs_bytes(ne, T, S, d));
-    QMLL_REQUIRE(ne <= 65535, QMLL_ERR_INVALID, "qmll_sorf_signs: ne=%d too large", ne);
-    half8_t* images = (half8_t*)out;
-    int* bad = (int*)((char*)out + (size_t)ne * T * S * (d / 16) * 1024);
-    const dim3 grid(S, T, ne);
-    hipStream_t st = (hipStream_t)stream;
-    if (d == 64) hipLaunchKernelGGL(sorf_signs_kernel<64>, grid, dim3(256), 0, st, D, T, S, images, bad);
-    else hipLaunchKernelGGL(sorf_signs_kernel<128>, grid, dim3(256), 0, st, D, T, S, images, bad);
+    Forms f = {};
+    f.images = (half8_t*)out;
+    f.largest = (float*)((char*)out + (size_t)ne * T * S * (d / 16) * 1024);
+    launch_prepare(D, nullptr, nullptr, ne, T, S, d, f, (hipStream_t)stream);
     QMLL_CHECK_LAUNCH("qmll_sorf_signs");
     return QMLL_OK;
 }
 
-extern "C" int qmll_sorf_alpha(const float* alpha, int S, int d, float* out, qmll_stream_t stream) {
-    QMLL_REQUIRE(S > 0 && (d == 64 || d == 128), QMLL_ERR_INVALID, "qmll_sorf_alpha: bad size S=%d d=%d", S, d);
-    QMLL_REQUIRE(alpha && out, QMLL_ERR_INVALID, "qmll_sorf_alpha: null pointer");
-    hipLaunchKernelGGL(sorf_alpha_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, alpha, S * d, d == 64 ? 2 : 3, out);
-    QMLL_CHECK_LAUNCH("qmll_sorf_alpha");
-    return QMLL_OK;
-}
-
 extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D,
-                                       const void* signs, const float* bias_rev, const float* alpha_scaled, const float* bias_absmax,
-                                       int A, int ne, int d, int S, int T, float normalisation, float* work, size_t work_bytes,
-                                       float* e_slots, float* gx, qmll_stream_t stream) {
-    QMLL_REQUIRE(A >= 0 && qmll_sorf_signs_bytes(ne, T, S, d) > 0, QMLL_ERR_INVALID,
+                                       const float* bias, const float* alpha, int A, int ne, int d, int S, int T,
+                                       float normalisation, void* work, size_t work_bytes, float* e_slots, float* gx,
+                                       qmll_stream_t stream) {
+    QMLL_REQUIRE(A >= 0 && matrix_shape(ne, T, S, d), QMLL_ERR_INVALID,
                  "qmll_sorf_energy_matrix: bad size A=%d ne=%d T=%d S=%d d=%d", A, ne, T, S, d);
     if (A == 0) return QMLL_OK;
-    QMLL_REQUIRE(x && type_offsets && sorted_slots && D && signs && bias_rev && alpha_scaled && bias_absmax && e_slots,
-                 QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: null pointer");
+    QMLL_REQUIRE(x && type_offsets && sorted_slots && D && bias && alpha && e_slots, QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_matrix: null pointer");
     QMLL_REQUIRE(work && work_bytes >= qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr), QMLL_ERR_INVALID,
                  "qmll_sorf_energy_matrix: workspace of %zu bytes, %zu are needed", work ? work_bytes : (size_t)0,
                  qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr));
     QMLL_REQUIRE(matrix_units(A, ne, T, S, d) < (1ll << 31), QMLL_ERR_INVALID,
                  "qmll_sorf_energy_matrix: %d atoms times %d stacks are too many for one launch", A, S);
-    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)work | (uintptr_t)D | (uintptr_t)signs | (uintptr_t)bias_rev | (uintptr_t)alpha_scaled |
-                   (uintptr_t)gx) & 15) == 0,
-                 QMLL_ERR_INVALID, "qmll_sorf_energy_matrix: every array must be 16-byte aligned");
+    QMLL_REQUIRE((((uintptr_t)x | (uintptr_t)work | (uintptr_t)D | (uintptr_t)gx) & 15) == 0, QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_matrix: x, D, work and gx must be 16-byte aligned");
+    Forms f;
+    float* parts;
+    matrix_workspace((char*)work, A, ne, T, S, d, gx != nullptr, f, parts);
     float hn = 1.0f;                                     // (1 / sqrt(d)) per transform
     for (int m = 0; m < T; ++m) hn /= sqrtf((float)d);
     const float scale = normalisation * hn, normf = sqrtf(2.0f / ((float)S * (float)d));
+    const float xs = scale * INV2PI, gscale = -scale * normf;
     const int nshares = matrix_shares(matrix_units(A, ne, T, S, d), gx != nullptr);
     const dim3 grid(nshares + (gx ? (A >= 65536 ? 64 : (A >> 10) + 1) : 0));
     hipStream_t st = (hipStream_t)stream;
+    launch_prepare(D, bias, alpha, ne, T, S, d, f, st);
     auto launch = [&](auto dc, auto tc, auto gc) {
         constexpr int DD = decltype(dc)::value, TT = decltype(tc)::value;
         constexpr bool GG = decltype(gc)::value;
         hipLaunchKernelGGL((sorf_energy_matrix_kernel<DD, GG, TT>), grid, dim3(64 * SM_WAVES), 0, st, x, type_offsets, sorted_slots, D,
-                           (const half8_t*)signs, bias_rev, alpha_scaled, bias_absmax, ne, A, S, nshares, scale, normf, work, e_slots,
-                           gx);
-        hipLaunchKernelGGL((sorf_parts_kernel<DD, GG>), dim3(nshares), dim3(256), 0, st, type_offsets, sorted_slots, ne,
-                           matrix_rounds(TT, S, DD), work, e_slots, gx);
+                           f.images, f.bias, f.alpha, f.largest, ne, A, S, nshares, xs, gscale, normf, parts, e_slots, gx);
+        hipLaunchKernelGGL((sorf_parts_kernel<DD, GG>), dim3(nshares + 1), dim3(256), 0, st, type_offsets, sorted_slots, ne, S,
+                           matrix_rounds(TT, S, DD), parts, f, e_slots, gx);
     };
     auto by_grad = [&](auto dc, auto tc) {
         if (gx) launch(dc, tc, std::true_type{});
@@ -536,5 +621,6 @@ extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, 
     if (T == 1) by_d(std::integral_constant<int, 1>{});
     else by_d(std::integral_constant<int, 2>{});
     QMLL_CHECK_LAUNCH("qmll_sorf_energy_matrix");
-    return QMLL_OK;
+    // diagonals that are not +-1, which only the device knows of: the rows kernel, whose workgroups else return at once
+    return qmll_sorf_rows_if(x, type_offsets, sorted_slots, D, bias, alpha, A, ne, d, S, T, normalisation, f.unfit, e_slots, gx, st);
 }

@@ -85,17 +85,6 @@ Tensor prepared_form(const Tensor& t, int kind, const std::function<Tensor(const
     return buffer;
 }
 
-// under graph capture a form can only be used when it was made before: its making would wait for the device, or happen at the
-// replay while the form is taken for made
-bool form_at_hand(const Tensor& t, int kind) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream(), &status) == hipSuccess && status == hipStreamCaptureStatusNone) return true;
-    std::lock_guard<std::mutex> lock(prepared_mutex);
-    const auto it = prepared.find(std::make_pair((const c10::TensorImpl*)t.unsafeGetTensorImpl(), kind));
-    return it != prepared.end() && !it->second.owner.expired() && it->second.version == version_of(t) &&
-           it->second.data == t.const_data_ptr();
-}
-
 // alpha as the kernels contract with it (fp32): a model stores it in fp64 (qml_lightning/models/kernel.py:226-234),
 // and the conversion, a launch per call otherwise, is kept per tensor version like the other prepared constants
 Tensor alpha32(const Tensor& alpha) {
@@ -556,35 +545,16 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
     TORCH_CHECK(bb.dim() == 2 && bb.size(0) == ne && bb.size(1) == (int64_t)S * d && al.numel() == (int64_t)S * d,
                 "sorf_energy_sorted: bias [", bb.sizes(), "] / alpha with ", al.numel(), " entries do not fit ", ne,
                 " elements and ", S * d, " features");
+    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr)) {      // large batches: the half-precision matrix cores
+        const size_t work_bytes = qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr);
+        Tensor work = at::empty({(int64_t)work_bytes}, DD.options().dtype(at::kByte));
+        check(qmll_sorf_energy_matrix(x, off, ss, fp(DD), fp(bb), fp(al), A, ne, d, S, T, scalar(cn), work.data_ptr(), work_bytes, e,
+                                      A ? gx : nullptr, stream()),
+              "qmll_sorf_energy_matrix");
+        return;
+    }
     // the largest |bias|, a constant of the model: computed once per tensor version, kept on the device
     Tensor bmax = prepared_form(bb, 2, [](const Tensor& b) { return b.abs().max().reshape({1}); });
-    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr) && form_at_hand(DD, 4) && form_at_hand(bb, 5) &&
-        form_at_hand(al, 6 + d)) {
-        // large batches: the half-precision matrix cores, with the diagonals' signs, bias in revolutions and alpha scaled
-        // once per tensor version; an empty form says that the diagonals are not all +-1
-        Tensor signs = prepared_form(DD, 4, [&](const Tensor& D) {
-            const size_t nbytes = qmll_sorf_signs_bytes(ne, T, S, d);
-            Tensor out = at::empty({(int64_t)nbytes}, D.options().dtype(at::kByte));
-            Tensor tail = out.narrow(0, (int64_t)nbytes - 16, 16);
-            tail.zero_();
-            check(qmll_sorf_signs(fp(D), ne, T, S, d, out.data_ptr(), nbytes, stream()), "qmll_sorf_signs");
-            return tail.view(at::kInt)[0].item<int>() == 0 ? out : at::empty({0}, out.options());
-        });
-        if (signs.numel() > 0) {
-            Tensor rev = prepared_form(bb, 5, [](const Tensor& b) { return b * 0.15915494309189535; });
-            Tensor scaled = prepared_form(al, 6 + d, [&](const Tensor& a) {
-                Tensor out = at::empty({(int64_t)S * d + 1}, a.options());
-                check(qmll_sorf_alpha(fp(a), S, d, out.data_ptr<float>(), stream()), "qmll_sorf_alpha");
-                return out;
-            });
-            const size_t work_bytes = qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr);
-            Tensor work = at::empty({(int64_t)(work_bytes / 4)}, DD.options().dtype(at::kFloat));
-            check(qmll_sorf_energy_matrix(x, off, ss, fp(DD), signs.const_data_ptr(), fp(rev), fp(scaled), fp(bmax), A, ne, d, S, T,
-                                          scalar(cn), work.data_ptr<float>(), work_bytes, e, A ? gx : nullptr, stream()),
-                  "qmll_sorf_energy_matrix");
-            return;
-        }
-    }
     check(qmll_sorf_energy_sorted(x, off, ss, fp(DD), fp(bb), fp(al), fp(bmax), A, ne, d, S, T, scalar(cn), e, A ? gx : nullptr,
                                   stream()),
           "qmll_sorf_energy_sorted");

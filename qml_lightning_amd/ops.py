@@ -12,7 +12,6 @@ Everything here requires the tensors to live on a HIP device ("cuda" in PyTorch-
 there is no CPU implementation.
 """
 import ctypes
-import math
 import os
 import weakref
 
@@ -609,23 +608,16 @@ def _zeroed_slots(e_zeroed, nslots, device):
 
 
 def sorf_signs(Dmat):
-    """The sign diagonals [ne,T,S,d] in the form the matrix-core kernel multiplies with (qmll_sorf_signs): an opaque
-    uint8 device buffer, or None when no kernel takes the shape or the diagonals are not all +-1."""
+    """The sign diagonals [ne,T,S,d] in the form that the matrix-core kernel multiplies with (qmll_sorf_signs): an opaque
+    uint8 device buffer, or None when no kernel takes the shape or the diagonals are not all +-1.  For inspection: a
+    prediction makes the form itself."""
     ne, T, S, d = Dmat.shape
     nbytes = int(_lib.lib().qmll_sorf_signs_bytes(ne, T, S, d))
     if nbytes == 0:
         return None
     out = torch.empty(nbytes, dtype=torch.uint8, device=Dmat.device)
-    out[-16:].zero_()
     check(_lib.lib().qmll_sorf_signs(_ptr(Dmat), ne, T, S, d, _ptr(out), nbytes, _stream()), "qmll_sorf_signs")
-    return out if int(out[-16:].view(torch.int32)[0].item()) == 0 else None
-
-
-def sorf_alpha(alpha, S, d):
-    """alpha behind the power of two the matrix-core kernel wants, and the inverse of that factor (qmll_sorf_alpha)."""
-    out = torch.empty(S * d + 1, dtype=torch.float32, device=alpha.device)
-    check(_lib.lib().qmll_sorf_alpha(_ptr(alpha), S, d, _ptr(out), _stream()), "qmll_sorf_alpha")
-    return out
+    return out if bool(out[-4 * ne * S:].view(torch.float32).isfinite().all()) else None
 
 
 def sorf_energy_sorted(x, type_offsets, sorted_slots, Dmat, bias, alpha, normalisation, ntransforms, nslots,
@@ -646,23 +638,15 @@ def sorf_energy_sorted(x, type_offsets, sorted_slots, Dmat, bias, alpha, normali
                            % (tuple(bias.shape), alpha.numel(), ne, S * d))
     e_slots = _zeroed_slots(e_zeroed, nslots, x.device)
     gx = torch.empty((A, d), dtype=torch.float32, device=x.device) if with_grad else None
-    # the largest |bias|, a constant of the model, computed once per tensor version and left on the device
-    bmax = presplit_cached(bias, "absmax", lambda t: t.abs().max().reshape(1))
-    # large batches run on the half-precision matrix cores; under capture only with forms made before (the making of one waits
-    # for the device, and that of the others would happen at the replay)
-    matrix = _lib.lib().qmll_sorf_matrix_pays(A, ne, T, S, d, int(with_grad))
-    if matrix and torch.cuda.is_current_stream_capturing():
-        matrix = all(_presplit_hit(t, k) for t, k in ((Dmat, "signs"), (bias, "revolutions"), (alpha, "sorf %d" % d)))
-    signs = presplit_cached(Dmat, "signs", sorf_signs) if matrix else None
-    if signs is not None:
-        rev = presplit_cached(bias, "revolutions", lambda t: t * (0.5 / math.pi))
-        scaled = presplit_cached(alpha, "sorf %d" % d, lambda t: sorf_alpha(t, S, d))
+    if _lib.lib().qmll_sorf_matrix_pays(A, ne, T, S, d, int(with_grad)):     # large batches: the half-precision matrix cores
         nbytes = int(_lib.lib().qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, int(with_grad)))
-        work = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-        check(_lib.lib().qmll_sorf_energy_matrix(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(signs), _ptr(rev),
-                                                 _ptr(scaled), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(work), nbytes,
+        work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        check(_lib.lib().qmll_sorf_energy_matrix(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(bias),
+                                                 _ptr(alpha), A, ne, d, S, T, float(normalisation), _ptr(work), nbytes,
                                                  _ptr(e_slots), _ptr(gx), _stream()), "qmll_sorf_energy_matrix")
         return e_slots, gx
+    # the largest |bias|, a constant of the model, computed once per tensor version and left on the device
+    bmax = presplit_cached(bias, "absmax", lambda t: t.abs().max().reshape(1))
     check(_lib.lib().qmll_sorf_energy_sorted(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(bias),
                                              _ptr(alpha), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(e_slots),
                                              _ptr(gx), _stream()), "qmll_sorf_energy_sorted")

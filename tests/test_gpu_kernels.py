@@ -1231,6 +1231,50 @@ def test_prepared_model_constants_follow_their_tensors():
         close(xs, ref.cpu().numpy(), REL_REP, "projection, reductors x %g" % scale)
 
 
+@pytest.mark.parametrize("T,with_grad", [(1, True), (2, False)])
+def test_large_batches_keep_nothing_of_the_model_tensors(T, with_grad):
+    """Signs, bias and alpha as they are at the call, however they were written (`.data` and DLPack writes move no version
+    counter), with diagonals that stop being +-1 and come back; and the first call of a model under capture."""
+    import qml_lightning_amd  # noqa: F401
+    g = torch.Generator(device=dev()).manual_seed(6)
+    A, S, d, ne = 60000, 64, 128, 2
+    x = torch.randn(A, d, device=dev(), generator=g)
+    off = ti32([0, A // 3, A])
+    slots = torch.randperm(A, device=dev(), generator=g).int()
+    cn, nt = torch.tensor(2.0), torch.tensor(T)
+
+    def draw():
+        D = torch.randint(0, 2, (ne, T, S, d), device=dev(), generator=g).float() * 2 - 1
+        return D, torch.rand(ne, S * d, device=dev(), generator=g) * 6.28, torch.randn(S * d, device=dev(), generator=g)
+
+    def run(D, b, alpha):
+        return torch.ops.qml_lightning_sorf.sorf_energy_sorted(x, off, slots, D, b, alpha, cn, nt, A, with_grad)
+    held, other = draw(), draw()
+    odd = (other[0] * torch.where(torch.rand(d, device=dev(), generator=g) < 0.1, 0.5, 1.0), other[1], other[2])
+    run(*held)
+    for now in (other, odd, other):
+        for t, v in zip(held, now):
+            t.data.copy_(v)
+        got, ref = run(*held), run(*[v.clone() for v in now])
+        assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+    rows = slice(0, 64)                                      # the last of them against fp64
+    c = sorf.sorf_coefficients(x[rows].double().cpu().numpy(), other[0][0].cpu().numpy(), 2.0).reshape(64, -1)
+    e_ref = (np.sqrt(2.0 / (S * d)) * np.cos(c + other[1][0].cpu().numpy()) * other[2].cpu().numpy()).sum(1)
+    close(got[0][slots[rows].long()], e_ref, 2e-6, "energies")
+    fresh = draw()                                           # never seen before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run(*fresh)
+    for now in (fresh, other, odd):
+        for t, v in zip(fresh, now):
+            t.copy_(v.clone())
+        graph.replay()
+        ref = run(*[v.clone() for v in now])
+        torch.cuda.synchronize()
+        assert torch.equal(captured[0], ref[0]) and torch.equal(captured[1], ref[1])
+
+
 def test_a_non_finite_row_spoils_only_itself_in_the_fp16_matrix_core_kernels():
     """The projection kernels on the fp16 matrix cores and the fused RFF kernel scale the 32 rows of a
     wavefront by one power of two taken from their largest FINITE entry: a row holding an infinity (or
