@@ -383,8 +383,8 @@ int qmll_sorf_energy_sorted(const float* x, const int* type_offsets, const int* 
  * where the device finds others the call runs as qmll_sorf_energy_sorted does).  x, D, work and gx 16-byte aligned.
  * work: device memory of qmll_sorf_matrix_workspace_bytes (0: no kernel takes the shape), for this call alone; the signs in
  * the form that is multiplied with, bias in revolutions and alpha behind a power of two are made there by every call.  fp32
- * operands are split into two fp16 parts (both rounded to nearest, fp32 accumulation).  Four launches, no synchronisation:
- * it can be captured. */
+ * operands are split into two fp16 parts (both rounded to nearest, 23 bits together, fp32 accumulation); the results are no
+ * further from fp64 than those of qmll_sorf_energy_sorted.  Four launches, no synchronisation: it can be captured. */
 size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, int d, int with_grad);
 int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad);   /* 1: faster than qmll_sorf_energy_sorted */
 int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,

@@ -12,8 +12,13 @@
 // The first operand of a stack never changes but for the signs of its diagonal: x is split once per atom, and the
 // signs go into the H_16 block, which is prepared per call (sorf_prepare_kernel: a block per (element, stack, transform), the
 // diagonal must hold +-1) and moved into LDS by direct loads, a round ahead.  The gradient is split per stack (a
-// conversion, a mixed-precision subtraction and a conversion per value); both parts are rounded to nearest, so a
-// value keeps 2^-24 of itself, as in fp32.  Power-of-two scales keep everything in fp16's range: x per atom
+// conversion, a mixed-precision subtraction and a conversion per value); both parts are rounded to nearest, 23 bits
+// together, one less than fp32: the largest error of an operand is 2^-23 of its binade, the root mean square 0.7 x 2^-24.
+// What that adds is taken off elsewhere, in the forms: bias is reduced to half a revolution in fp64 (the argument's rounding
+// is the largest error of either kernel) and the constant factors are rounded once.  Against fp64, root mean square of energies
+// / gradients, rows kernel -> this one, relative: d = 128, 128 stacks 3.7e-7 / 3.1e-7 -> 2.3e-7 / 2.2e-7, two transforms, 32 stacks
+// 3.1e-7 / 3.1e-7 -> 2.4e-7 / 2.4e-7; with arguments twice as large and falling components 4.7e-7 / 4.6e-7 -> 4.2e-7 / 4.3e-7 at most.
+// Power-of-two scales keep everything in fp16's range: x per atom
 // (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per call.
 //
 // Instruction issue bounds it, as it does the kernel without matrix instructions (sorf_energy_rows_kernel, which at
@@ -60,7 +65,7 @@ __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h
 struct Forms {
     half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal
     float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
-    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2
+    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2 (from fp64: the smaller the argument, the less its rounding)
     float* alpha;         // [S][d] 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
     int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
 };
@@ -138,8 +143,8 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     if (bias != nullptr) {
         const size_t at = ((size_t)e * S + s) * D;
         for (int t = tid; t < D; t += PREP_THREADS) {
-            const float r = bias[at + t] * INV2PI;
-            f.bias[at + t] = r - rintf(r);
+            const double r = (double)bias[at + t] * 0.15915494309189533577;
+            f.bias[at + t] = (float)(r - rint(r));
         }
     }
     if (tid == 0) f.largest[(size_t)e * S + s] = any_unfit ? HUGE_VALF : largest;
@@ -594,10 +599,9 @@ extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, 
     Forms f;
     float* parts;
     matrix_workspace((char*)work, A, ne, T, S, d, gx != nullptr, f, parts);
-    float hn = 1.0f;                                     // (1 / sqrt(d)) per transform
-    for (int m = 0; m < T; ++m) hn /= sqrtf((float)d);
-    const float scale = normalisation * hn, normf = sqrtf(2.0f / ((float)S * (float)d));
-    const float xs = scale * INV2PI, gscale = -scale * normf;
+    // x into revolutions, and the factors of the gradient and of the energy, each rounded once
+    const double scale = (double)normalisation / (T == 1 ? sqrt((double)d) : (double)d), norm = sqrt(2.0 / ((double)S * d));
+    const float xs = (float)(scale * 0.15915494309189533577), gscale = (float)(-scale * norm), normf = (float)norm;
     const int nshares = matrix_shares(matrix_units(A, ne, T, S, d), gx != nullptr);
     const dim3 grid(nshares + (gx ? (A >= 65536 ? 64 : (A >> 10) + 1) : 0));
     hipStream_t st = (hipStream_t)stream;

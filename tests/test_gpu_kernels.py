@@ -1231,6 +1231,37 @@ def test_prepared_model_constants_follow_their_tensors():
         close(xs, ref.cpu().numpy(), REL_REP, "projection, reductors x %g" % scale)
 
 
+@pytest.mark.parametrize("steep", [False, True])
+@pytest.mark.parametrize("d,T,S", [(128, 1, 128), (128, 2, 32), (64, 1, 128), (64, 2, 64)])
+def test_sorf_matrix_kernel_is_as_exact_as_the_rows_kernel(monkeypatch, d, T, S, steep):
+    """Against fp64 the kernel on split operands is no further off than the fp32 one: root mean square over 512 rows x S d
+    features of evenly spread and of steeply falling components (measured 0.75 to 0.96 of it)."""
+    from qml_lightning_amd import _lib, ops
+    g = torch.Generator(device=dev()).manual_seed(d + T)
+    n, norm, F = 512, 12.0 if steep else 1.5, S * d
+    x = torch.randn(n, d, device=dev(), generator=g)
+    if steep:
+        x = x * torch.logspace(0, -3, d, device=dev())
+    D = torch.randint(0, 2, (1, T, S, d), device=dev(), generator=g).float() * 2 - 1
+    b = torch.rand(1, F, device=dev(), generator=g) * 6.28
+    alpha = torch.randn(F, device=dev(), generator=g)
+    H = torch.tensor([[(-1.0) ** bin(i & j).count("1") for j in range(d)] for i in range(d)], dtype=torch.float64, device=dev())
+    c = x.double()[:, None, :]
+    for m in range(T):
+        c = (c * D[0, m].double()) @ H / d ** 0.5
+    arg = c * norm + b.double().view(S, d)
+    weight = alpha.double().view(S, d) * (2.0 / F) ** 0.5
+    e_ref, gr = (torch.cos(arg) * weight).sum((1, 2)), -torch.sin(arg) * weight * norm
+    for m in reversed(range(T)):
+        gr = gr @ H / d ** 0.5 * D[0, m].double()
+    errors = {}
+    for name in ("rows", "matrix"):
+        monkeypatch.setattr(_lib.lib(), "qmll_sorf_matrix_pays", lambda *a: int(name == "matrix"))
+        e, gx = ops.sorf_energy_sorted(x, ti32([0, n]), ti32(np.arange(n)), D, b, alpha, norm, T, n)
+        errors[name] = [float((v.double() - r).pow(2).mean().sqrt()) for v, r in ((e, e_ref), (gx, gr.sum(1)))]
+    assert errors["matrix"][0] <= errors["rows"][0] and errors["matrix"][1] <= errors["rows"][1], errors
+
+
 @pytest.mark.parametrize("T,with_grad", [(1, True), (2, False)])
 def test_large_batches_keep_nothing_of_the_model_tensors(T, with_grad):
     """Signs, bias and alpha as they are at the call, however they were written (`.data` and DLPack writes move no version
