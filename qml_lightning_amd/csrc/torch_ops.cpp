@@ -545,7 +545,8 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
     TORCH_CHECK(bb.dim() == 2 && bb.size(0) == ne && bb.size(1) == (int64_t)S * d && al.numel() == (int64_t)S * d,
                 "sorf_energy_sorted: bias [", bb.sizes(), "] / alpha with ", al.numel(), " entries do not fit ", ne,
                 " elements and ", S * d, " features");
-    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr)) {      // large batches: the half-precision matrix cores
+    // large batches: the half-precision matrix cores (16-byte loads: views at other offsets stay with the rows kernel)
+    if (qmll_sorf_matrix_pays(A, ne, T, S, d, gx != nullptr) && (((uintptr_t)x | (uintptr_t)fp(DD)) & 15) == 0) {
         const size_t work_bytes = qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, gx != nullptr);
         Tensor work = at::empty({(int64_t)work_bytes}, DD.options().dtype(at::kByte));
         check(qmll_sorf_energy_matrix(x, off, ss, fp(DD), fp(bb), fp(al), A, ne, d, S, T, scalar(cn), work.data_ptr(), work_bytes, e,

@@ -638,7 +638,8 @@ def sorf_energy_sorted(x, type_offsets, sorted_slots, Dmat, bias, alpha, normali
                            % (tuple(bias.shape), alpha.numel(), ne, S * d))
     e_slots = _zeroed_slots(e_zeroed, nslots, x.device)
     gx = torch.empty((A, d), dtype=torch.float32, device=x.device) if with_grad else None
-    if _lib.lib().qmll_sorf_matrix_pays(A, ne, T, S, d, int(with_grad)):     # large batches: the half-precision matrix cores
+    # large batches: the half-precision matrix cores (16-byte loads: views at other offsets stay with the rows kernel)
+    if _lib.lib().qmll_sorf_matrix_pays(A, ne, T, S, d, int(with_grad)) and (x.data_ptr() | Dmat.data_ptr()) % 16 == 0:
         nbytes = int(_lib.lib().qmll_sorf_matrix_workspace_bytes(A, ne, T, S, d, int(with_grad)))
         work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
         check(_lib.lib().qmll_sorf_energy_matrix(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(bias),

@@ -1306,6 +1306,31 @@ def test_large_batches_keep_nothing_of_the_model_tensors(T, with_grad):
         assert torch.equal(captured[0], ref[0]) and torch.equal(captured[1], ref[1])
 
 
+@pytest.mark.parametrize("offset", [1, 2, 4])
+@pytest.mark.parametrize("moved", ["x", "Dmat"])
+def test_large_batches_take_views_at_any_offset(moved, offset):
+    """Contiguous views that start `offset` floats into their storage, through the operator and the Python route."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device=dev()).manual_seed(7)
+    A, S, d, ne = 40000, 64, 128, 2
+    x = torch.randn(A, d, device=dev(), generator=g)
+    D = torch.randint(0, 2, (ne, 1, S, d), device=dev(), generator=g).float() * 2 - 1
+    b, alpha = torch.rand(ne, S * d, device=dev(), generator=g) * 6.28, torch.randn(S * d, device=dev(), generator=g)
+    off, slots = ti32([0, A // 3, A]), torch.arange(A, device=dev()).int()
+
+    def view(t):
+        buf = torch.empty(t.numel() + 8, device=dev())
+        buf[offset:offset + t.numel()] = t.reshape(-1)
+        return buf[offset:offset + t.numel()].view(t.shape)
+    args = (view(x) if moved == "x" else x, off, slots, view(D) if moved == "Dmat" else D, b, alpha)
+    assert args[0].is_contiguous() and args[3].is_contiguous()
+    ref = ops.sorf_energy_sorted(x, off, slots, D, b, alpha, 2.0, 1, A)
+    for got in (ops.sorf_energy_sorted(*args, 2.0, 1, A),
+                torch.ops.qml_lightning_sorf.sorf_energy_sorted(*args, torch.tensor(2.0), torch.tensor(1), A, True)):
+        for v, r in zip(got, ref):
+            close(v, r.double().cpu().numpy(), 5e-6, "view of %s at %d" % (moved, offset))
+
+
 def test_a_non_finite_row_spoils_only_itself_in_the_fp16_matrix_core_kernels():
     """The projection kernels on the fp16 matrix cores and the fused RFF kernel scale the 32 rows of a
     wavefront by one power of two taken from their largest FINITE entry: a row holding an infinity (or
