@@ -13,12 +13,15 @@
 // Host code only: no kernels here.  Loaded with torch.ops.load_library (Python) or as a
 // shared library by a C++ host; it pulls in libqmll.so from its own directory.
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/autograd.h>
 #include <torch/library.h>
 
+#include <climits>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -52,37 +55,73 @@ const int* ip(const Tensor& t) { return t.defined() && t.numel() ? t.data_ptr<in
 
 float scalar(const Tensor& t) { return t.item<float>(); }
 
-// Model constants that a kernel wants in a prepared form (fp32 operands split into fp16 parts): prepared
-// once per tensor and kept until the tensor dies, is written to in place or changes its storage.
+bool capturing() {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing((hipStream_t)stream(), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
+// Model constants that a kernel wants in a prepared form (fp32 operands split into fp16 parts): prepared once per tensor
+// and kept until the tensor dies, is written to in place or changes its storage.  A write that moves no version counter
+// (through `.data`, DLPack or a foreign kernel) is not seen: forget_prepared drops the tensor's forms.  Inference tensors have no
+// counter, and theirs are made by every call.
 struct Prepared {
     c10::weak_intrusive_ptr<c10::TensorImpl> owner;
     int64_t version;
     const void* data;
     Tensor buffer;
+    hipStream_t stream;                        // that made it
+    std::shared_ptr<ihipEvent_t> made;         // recorded behind the making, null once it was seen to have passed
 };
 std::mutex prepared_mutex;
-std::map<std::pair<const c10::TensorImpl*, int>, Prepared> prepared;
-
-int64_t version_of(const Tensor& t) { return t.is_inference() ? -1 : (int64_t)t._version(); }
+std::map<std::pair<const c10::TensorImpl*, int>, Prepared>& prepared =
+    *new std::map<std::pair<const c10::TensorImpl*, int>, Prepared>;       // outlives the runtime: freed by the process's end
 
 Tensor prepared_form(const Tensor& t, int kind, const std::function<Tensor(const Tensor&)>& make) {
+    if (t.is_inference()) return make(t);
     std::lock_guard<std::mutex> lock(prepared_mutex);
+    const auto here = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
     const auto key = std::make_pair((const c10::TensorImpl*)t.unsafeGetTensorImpl(), kind);
     auto it = prepared.find(key);
     if (it != prepared.end()) {
-        auto alive = it->second.owner.lock();
-        if (alive && alive.get() == t.unsafeGetTensorImpl() && it->second.version == version_of(t) &&
-            it->second.data == t.const_data_ptr())
-            return it->second.buffer;
-        prepared.erase(it);
+        Prepared& p = it->second;
+        auto alive = p.owner.lock();
+        if (alive && alive.get() == t.unsafeGetTensorImpl() && p.version == (int64_t)t._version() && p.data == t.const_data_ptr()) {
+            if (!p.made && p.stream == here.stream()) return p.buffer;
+            const bool captured = capturing();
+            if (p.made && !captured) {
+                if (hipEventQuery(p.made.get()) == hipSuccess) p.made.reset();
+                else (void)hipGetLastError();                                 // "not ready" is no error of the next launch
+            }
+            if (p.stream != here.stream()) {
+                // another stream waits for the making, and the buffer, if it is dropped, for that stream; a capture cannot wait
+                if (p.made && captured) return make(t);
+                if (p.made)
+                    TORCH_CHECK(hipStreamWaitEvent(here.stream(), p.made.get(), 0) == hipSuccess, "waiting for a prepared form failed");
+                if (!captured && p.buffer.defined()) p.buffer.record_stream(here.unwrap());
+            }
+            return p.buffer;
+        }
     }
-    if (prepared.size() >= 64) {      // forget tensors that are gone
+    if (capturing()) return make(t);           // at the replay, not now: nothing to keep
+    if (it != prepared.end()) prepared.erase(it);
+    if (prepared.size() >= 64) {               // forget tensors that are gone
         for (auto e = prepared.begin(); e != prepared.end();) e = e->second.owner.expired() ? prepared.erase(e) : std::next(e);
     }
     Tensor buffer = make(t);
-    prepared.emplace(key, Prepared{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), version_of(t),
-                                   t.const_data_ptr(), buffer});
+    hipEvent_t event = nullptr;
+    TORCH_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess, "no event for a prepared form");
+    std::shared_ptr<ihipEvent_t> made(event, [](hipEvent_t e) { (void)hipEventDestroy(e); });
+    TORCH_CHECK(hipEventRecord(event, here.stream()) == hipSuccess, "no event for a prepared form");
+    prepared.emplace(key, Prepared{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), (int64_t)t._version(),
+                                   t.const_data_ptr(), buffer, here.stream(), made});
     return buffer;
+}
+
+// the forms of a tensor that was written to behind its version counter
+void forget_prepared(const Tensor& t) {
+    std::lock_guard<std::mutex> lock(prepared_mutex);
+    const c10::TensorImpl* impl = t.unsafeGetTensorImpl();
+    for (auto it = prepared.lower_bound({impl, INT_MIN}); it != prepared.end() && it->first.first == impl;) it = prepared.erase(it);
 }
 
 // alpha as the kernels contract with it (fp32): a model stores it in fp64 (qml_lightning/models/kernel.py:226-234),
@@ -554,8 +593,9 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
               "qmll_sorf_energy_matrix");
         return;
     }
-    // the largest |bias|, a constant of the model: computed once per tensor version, kept on the device
-    Tensor bmax = prepared_form(bb, 2, [](const Tensor& b) { return b.abs().max().reshape({1}); });
+    // the largest |bias|, a constant of the model: computed once per tensor version, kept on the device (in a graph, where a
+    // reduction of the library may record a memset, the kernel does without)
+    Tensor bmax = prepared_form(bb, 2, [](const Tensor& b) { return capturing() ? Tensor() : b.abs().max().reshape({1}); });
     check(qmll_sorf_energy_sorted(x, off, ss, fp(DD), fp(bb), fp(al), fp(bmax), A, ne, d, S, T, scalar(cn), e, A ? gx : nullptr,
                                   stream()),
           "qmll_sorf_energy_sorted");
@@ -876,6 +916,7 @@ TORCH_LIBRARY(qml_lightning_sorf, m) {
     m.def("fchl_rff_energy", &fchl_rff_energy);
     m.def("fchl_sorf_forces", &fchl_sorf_forces);
     m.def("fchl_rff_forces", &fchl_rff_forces);
+    m.def("forget_prepared", &forget_prepared);
 }
 
 // names the loader can test for

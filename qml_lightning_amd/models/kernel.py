@@ -9,8 +9,6 @@ views of it, no concatenation copy), per-element atom indices built once on the 
 `format_data` (no boolean-mask device syncs), the hand-written fp64 MFMA Gram kernel, and
 no `empty_cache()` between batches.
 """
-import weakref
-
 import numpy as np
 import torch
 
@@ -22,20 +20,11 @@ def _default_device():
     return torch.device("cuda" if torch.cuda.is_available() else "cpu")
 
 
-_ALPHA32 = weakref.WeakKeyDictionary()    # model -> (alpha it was made from, its version, fp32 copy)
-
-
 def alpha_f32(model):
     """model.alpha as fp32 (what the predict routes contract with), converted once per value of
     alpha instead of once per call: one launch less per step, which counts for single molecules."""
     a = model.alpha
-    if a.dtype == torch.float32:
-        return a
-    hit = _ALPHA32.get(model)
-    if hit is None or hit[0] is not a or hit[1] != a._version:
-        hit = (a, a._version, a.float())
-        _ALPHA32[model] = hit
-    return hit[2]
+    return a if a.dtype == torch.float32 else ops.presplit_cached(a, "f32 model", lambda t: t.float())
 
 
 def rep_from_attribute_tree(tree):
@@ -85,6 +74,15 @@ class BaseKernel():
         self.llambda = llambda
         self._queue_force_rows = False
         self._queued_segments = None
+
+    @torch.jit.unused
+    def forget_prepared(self):
+        """The kernels keep some of the model's tensors in a form of their own (reductors and W split into parts, alpha in
+        fp32, the largest bias), and make it again when a tensor is replaced or written to in place.  Call this after
+        a write that torch does not see: through `tensor.data`, DLPack or a foreign kernel."""
+        for name in ("reductors", "Dmat", "bias", "W", "b", "alpha"):
+            if hasattr(self, name):
+                ops.forget_prepared(getattr(self, name))
 
     # -- to be provided by the feature model -------------------------------------------
     def finish_features(self, derivative_matrix=None, overwrite=False, feature_matrix=None, rows=None):

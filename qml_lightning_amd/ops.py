@@ -646,8 +646,9 @@ def sorf_energy_sorted(x, type_offsets, sorted_slots, Dmat, bias, alpha, normali
                                                  _ptr(alpha), A, ne, d, S, T, float(normalisation), _ptr(work), nbytes,
                                                  _ptr(e_slots), _ptr(gx), _stream()), "qmll_sorf_energy_matrix")
         return e_slots, gx
-    # the largest |bias|, a constant of the model, computed once per tensor version and left on the device
-    bmax = presplit_cached(bias, "absmax", lambda t: t.abs().max().reshape(1))
+    # the largest |bias|, a constant of the model, computed once per tensor version and left on the device (in a graph, where
+    # a reduction of the library may record a memset, the kernel does without)
+    bmax = presplit_cached(bias, "absmax", lambda t: None if torch.cuda.is_current_stream_capturing() else t.abs().max().reshape(1))
     check(_lib.lib().qmll_sorf_energy_sorted(_ptr(x), _ptr(type_offsets), _ptr(sorted_slots), _ptr(Dmat), _ptr(bias),
                                              _ptr(alpha), _ptr(bmax), A, ne, d, S, T, float(normalisation), _ptr(e_slots),
                                              _ptr(gx), _stream()), "qmll_sorf_energy_sorted")
@@ -719,30 +720,49 @@ def rff_rows(items, Ze, G, nmol, n, row_offsets=None, max_rows=None, overwrite=F
     return G
 
 
-_PRESPLIT = {}    # (id(tensor), kind) -> (weak reference, version, address, prepared buffer)
-
-
-def _version(t):
-    try:
-        return t._version
-    except RuntimeError:      # inference tensors keep no version counter
-        return -1
-
-
-def _presplit_hit(t, kind):
-    hit = _PRESPLIT.get((id(t), kind))
-    return hit if hit is not None and hit[0]() is t and hit[1] == _version(t) and hit[2] == t.data_ptr() else None
+_PRESPLIT = {}    # (id(tensor), kind) -> [weak reference, version, address, prepared buffer, stream, event or None]
 
 
 def presplit_cached(t, kind, make):
     """The prepared (pre-split) form of a model constant `t`, made once by `make(t)` and reused until
-    the tensor object dies, is written to in place (its version counter moves) or changes its storage."""
-    hit = _presplit_hit(t, kind)
-    if hit is not None:
-        return hit[3]
-    key, buf = (id(t), kind), make(t)
-    _PRESPLIT[key] = (weakref.ref(t, lambda _r, k=key: _PRESPLIT.pop(k, None)), _version(t), t.data_ptr(), buf)
+    the tensor object dies, is written to in place (its version counter moves) or changes its storage.
+    A write that moves no counter (through `.data` or DLPack) is not seen: see forget_prepared.  Inference tensors have
+    no counter, and theirs are made by every call; so are forms that are first needed under graph capture."""
+    if t.is_inference() or not t.is_cuda:
+        return make(t)
+    key, here = (id(t), kind), _stream().value
+    hit = _PRESPLIT.get(key)
+    if hit is not None and hit[0]() is t and hit[1] == t._version and hit[2] == t.data_ptr():
+        buf, made_on, made = hit[3:]
+        if made is None and made_on == here:
+            return buf
+        captured = torch.cuda.is_current_stream_capturing()
+        if made is not None and not captured and made.query():
+            made = hit[5] = None
+        if made_on != here:
+            # another stream waits for the making, and the buffer, if it is dropped, for that stream; a capture cannot wait
+            if made is not None and captured:
+                return make(t)
+            if not captured:
+                stream = torch.cuda.current_stream(t.device)
+                if made is not None:
+                    stream.wait_event(made)
+                if buf is not None:
+                    buf.record_stream(stream)
+        return buf
+    buf = make(t)
+    if not torch.cuda.is_current_stream_capturing():
+        _PRESPLIT[key] = [weakref.ref(t, lambda _r, k=key: _PRESPLIT.pop(k, None)), t._version, t.data_ptr(), buf, here,
+                          torch.cuda.current_stream(t.device).record_event()]
     return buf
+
+
+def forget_prepared(t):
+    """Drop the prepared forms of tensor `t`: after a write that its version counter does not show."""
+    for key in [k for k in list(_PRESPLIT) if k[0] == id(t)]:
+        _PRESPLIT.pop(key, None)
+    if OPS_BACKEND == "c++":
+        torch.ops.qml_lightning_sorf.forget_prepared(t)
 
 
 def rff_presplit(W):

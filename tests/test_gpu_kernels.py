@@ -1231,6 +1231,90 @@ def test_prepared_model_constants_follow_their_tensors():
         close(xs, ref.cpu().numpy(), REL_REP, "projection, reductors x %g" % scale)
 
 
+def prepared_form_calls(seed):
+    """(tensor, call, reference of the call) for both caches of prepared forms and both large-batch forms."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device=dev()).manual_seed(seed)
+    A, R, d, F, ne = 2304, 312, 128, 512, 2
+    types = torch.arange(A, device=dev(), dtype=torch.int32) % ne
+    ss, off = ops.sort_by_type(types, torch.arange(A, device=dev(), dtype=torch.int32), ne)
+    pick, order = types.long()[ss.long()], ss.long()
+    rep, x = torch.randn(A, R, device=dev(), generator=g), torch.randn(A, d, device=dev(), generator=g)
+    b, alpha = torch.rand(ne, F, device=dev(), generator=g) * 6.28, torch.randn(F, device=dev(), generator=g)
+
+    def project_ref(U):
+        return torch.stack([rep[order[a]].double() @ U[pick[a]].double() for a in range(0, A, 97)])
+
+    def rff_ref(W):
+        return torch.stack([(2.0 / F) ** 0.5 * (torch.cos(x[a].double() @ W[pick[a]].double() + b[pick[a]].double())
+                                                * alpha.double()).sum() for a in range(0, A, 97)])
+    so = torch.ops.qml_lightning_sorf
+    red, W = torch.randn(ne, R, d, device=dev(), generator=g), torch.randn(ne, d, F, device=dev(), generator=g) / 8
+    torch.cuda.synchronize()
+    return [(red, lambda U: ops.project_typed(rep, ss, off, U)[::97], project_ref),
+            (red.clone(), lambda U: so.project_typed(rep, ss, off, U, types)[::97], project_ref),
+            (W, lambda V: ops.rff_energy_sorted(x, off, ss, V, b, alpha, A)[0][order][::97], rff_ref),
+            (W.clone(), lambda V: so.rff_energy_sorted(x, off, ss, V, b, alpha, A, True)[0][order][::97], rff_ref)]
+
+
+def test_prepared_forms_are_waited_for_by_other_streams():
+    """A form whose making is still queued on one stream is used on another; and its buffer, dropped there, stays until the
+    second stream is done with it."""
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    for t, call, ref in prepared_form_calls(1):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(one):
+            torch.cuda._sleep(50_000_000)
+            first = call(t)
+        with torch.cuda.stream(two):
+            second = call(t)
+            torch.cuda._sleep(50_000_000)
+            third = call(t)
+        old = ref(t).cpu()                                 # on the default stream, which waits for neither
+        with torch.cuda.stream(one):
+            one.wait_stream(torch.cuda.default_stream())
+            two_done = torch.cuda.Event()
+            two_done.record(two)
+            one.wait_event(two_done)                       # t itself is written only behind the second stream's use
+            t.mul_(0.5)
+            fourth = call(t)
+        torch.cuda.synchronize()
+        for got in (first, second, third):
+            close(got, old.numpy(), REL_EF, "before the update")
+        close(fourth, ref(t).cpu().numpy(), REL_EF, "after the update")
+
+
+def test_prepared_forms_first_needed_under_capture_are_not_kept():
+    for t, call, ref in prepared_form_calls(2):
+        call(t.clone())                                    # the allocator and the library are warm, t is not prepared
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call(t)
+        close(call(t), ref(t).cpu().numpy(), REL_EF, "eager, before the first replay")
+        for scale in (1.0, 0.5, -0.25):
+            t.mul_(scale)
+            graph.replay()
+            eager = call(t)
+            torch.cuda.synchronize()
+            close(out, ref(t).cpu().numpy(), REL_EF, "replay x %g" % scale)
+            close(eager, ref(t).cpu().numpy(), REL_EF, "eager x %g" % scale)
+
+
+def test_prepared_forms_of_inference_tensors_and_after_unseen_writes():
+    from qml_lightning_amd import ops
+    for t, call, ref in prepared_form_calls(3):
+        close(call(t), ref(t).cpu().numpy(), REL_EF, "first use")
+        t.data.mul_(0.5)
+        ops.forget_prepared(t)
+        close(call(t), ref(t).cpu().numpy(), REL_EF, "after forget_prepared")
+        with torch.inference_mode():
+            u = t.clone()
+            close(call(u), ref(u).cpu().numpy(), REL_EF, "inference tensor")
+            u.mul_(-0.5)
+            close(call(u), ref(u).cpu().numpy(), REL_EF, "inference tensor, written to")
+
+
 @pytest.mark.parametrize("steep", [False, True])
 @pytest.mark.parametrize("d,T,S", [(128, 1, 128), (128, 2, 32), (64, 1, 128), (64, 2, 64)])
 def test_sorf_matrix_kernel_is_as_exact_as_the_rows_kernel(monkeypatch, d, T, S, steep):
