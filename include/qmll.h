@@ -461,8 +461,9 @@ int qmll_rff_energy_sorted(const float* x, const int* type_offsets, const int* s
                            const float* b, const float* alpha, int A, int ne, int d, int F, float* e_slots,
                            float* gx, qmll_stream_t stream);
 /* The same with device memory for this call alone, of qmll_rff_energy_workspace_bytes: tiles of atoms that several workgroups
- * share are then summed from it in a fixed order and e_slots need not be zero, where the call above adds into the zero-filled
- * outputs with atomics (slower, and the last bit varies from run to run). */
+ * share are then summed from it in a fixed order, where the call above adds into the zero-filled outputs with atomics (slower,
+ * and the last bit varies from run to run).  0 bytes: no tile is shared, or so few energies alone that the atomics are faster
+ * and are used; e_slots arrives zero-filled here too. */
 size_t qmll_rff_energy_workspace_bytes(int A, int ne, int d, int F, int with_grad);
 int qmll_rff_energy_shares(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split, const float* b,
                            const float* alpha, int A, int ne, int d, int F, float* work, size_t work_bytes, float* e_slots,

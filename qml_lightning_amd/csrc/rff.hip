@@ -12,8 +12,6 @@
 //    product is the sine argument) form one A tile of 16-row blocks in LDS, multiplied with
 //    v_mfma_f64_16x16x4_f64; the per-atom product is scaled by the sine column factor and summed
 //    over the molecule's atoms in registers, so G is written once and no atomics are needed.
-#include <type_traits>
-
 #include <algorithm>
 #include <type_traits>
 
@@ -831,12 +829,15 @@ extern "C" int qmll_rff_presplit(const float* W, int ne, int d, int F, void* out
 // The parts used to be added into zero-filled outputs with atomics, 4 bytes each at a stride of a row, which took 2 to 3 ms per
 // launch whatever its work.  Measured with the gradient, atomics -> parts: d = 128, 32768 features, 86016 atoms 4.99 -> 4.53 ms, 10000
 // atoms 2.06 -> 0.58, 300 atoms 146 -> 67 us; 2048 features, 33000 atoms 3.27 ms -> 173 us; d = 64, 8192 features, 4000 atoms
-// 434 -> 55 us.  Energies only, where the atomics were few: 2048 features, 10000 atoms 87 -> 32 us, 21 atoms 8 -> 11.
-struct RffSplit { int nwhole, ntail, nparts; };
+// 434 -> 55 us.  Energies only, where an atom adds one float a part, they stay up to 4096 of them (added): then the launch that
+// sums the parts costs more.  Parts / atomics: d = 128, 1024 features (8 parts), 21 atoms 10.4 / 8.2 us, 512 atoms 11.6 / 10.6; 2048 features
+// (16), 21 atoms 10.3 / 8.3, 128 atoms 10.9 / 9.9, 512 atoms 12.1 / 12.7; 8192 features (64), 21 atoms 12.1 / 10.0, 64 atoms 12.4 / 12.4, 256 atoms
+// 13.5 / 20.3; 32768 features, 21 atoms 26.4 / 23.3, 128 atoms 26.9 / 29.1; d = 64 alike.
+struct RffSplit { int nwhole, ntail, nparts; bool added; };
 static RffSplit rff_split(int A, int ne, int d, int F, bool with_grad) {
     const int SLOTS = (d == 64 && !with_grad ? 4 : 2) * 256;
     const int tiles = (A + RE_M - 1) / RE_M + ne, nchunks = F / RE_FC;      // at most: every element's last tile may be partial
-    RffSplit p = {tiles / SLOTS * SLOTS, tiles % SLOTS, 1};
+    RffSplit p = {tiles / SLOTS * SLOTS, tiles % SLOTS, 1, false};
     double best = nchunks + 3.0;
     for (int k = 2; k <= 64 && nchunks / k >= 4; ++k) {
         const int pieces = p.ntail * k;
@@ -850,13 +851,14 @@ static RffSplit rff_split(int A, int ne, int d, int F, bool with_grad) {
         p.nwhole = tiles;
         p.ntail = 0;
     }
+    p.added = !with_grad && p.ntail > 0 && (long long)A * p.nparts <= 4096;
     return p;
 }
 
 extern "C" size_t qmll_rff_energy_workspace_bytes(int A, int ne, int d, int F, int with_grad) {
     if (A <= 0 || ne <= 0 || d <= 0 || F < RE_FC) return 0;
     const RffSplit p = rff_split(A, ne, d, F, with_grad != 0);
-    return (size_t)p.ntail * p.nparts * part_floats(d, with_grad) * sizeof(float);
+    return p.added ? 0 : (size_t)p.ntail * p.nparts * part_floats(d, with_grad) * sizeof(float);
 }
 
 extern "C" int qmll_rff_energy_shares(const float* x, const int* type_offsets, const int* sorted_slots, const void* W_split,
@@ -879,6 +881,7 @@ extern "C" int qmll_rff_energy_shares(const float* x, const int* type_offsets, c
     const float norm = sqrtf(2.0f / (float)F);
     hipStream_t st = (hipStream_t)stream;
     const RffSplit p = rff_split(A, ne, d, F, gx != nullptr);
+    if (p.added) work = nullptr;
     if (!work && p.ntail && gx) {
         hipLaunchKernelGGL(zero_fill_kernel, dim3(1024), dim3(256), 0, st, gx, (size_t)A * d);
         QMLL_CHECK_LAUNCH("qmll_rff_energy_sorted");

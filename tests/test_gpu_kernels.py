@@ -1131,6 +1131,26 @@ def test_rff_energy_parts_of_a_tile(d, F, A, grad):
         assert float((got.double() - g_ref).abs().max()) <= 2e-5 * float(g_ref.abs().max())
 
 
+@pytest.mark.parametrize("d,F,A,added", [(64, 2048, 21, True), (128, 1024, 512, True), (128, 1024, 513, False), (128, 32768, 64, True),
+                                         (64, 32, 21, False)])
+def test_rff_energies_of_few_atoms(d, F, A, added):
+    """Energies alone: up to 4096 parts of atoms' energies are added with atomics, without a launch that sums them (8, 16 and 64
+    parts at 1024, 2048 and 32768 features, one at 32)."""
+    from qml_lightning_amd import _lib, ops
+    assert (_lib.lib().qmll_rff_energy_workspace_bytes(A, 2, d, F, 0) == 0) == (added or F == 32)
+    g = torch.Generator(device=dev()).manual_seed(A)
+    off = torch.tensor([0, (2 * A) // 3, A - 1], dtype=torch.int32, device=dev())
+    x, W = torch.randn(A, d, device=dev(), generator=g), torch.randn(2, d, F, device=dev(), generator=g) * 0.1
+    b, alpha = torch.rand(2, F, device=dev(), generator=g) * 6.28, torch.randn(F, device=dev(), generator=g)
+    slots = torch.randperm(A, device=dev(), generator=g).int()
+    e, gx = ops.rff_energy_sorted(x, off, slots, W, b, alpha, A, with_grad=False)
+    e_ref = torch.zeros(A, dtype=torch.float64, device=dev())
+    for t in range(2):
+        lo, hi = int(off[t]), int(off[t + 1])
+        e_ref[slots[lo:hi].long()] = (2.0 / F) ** 0.5 * (torch.cos(x[lo:hi].double() @ W[t].double() + b[t].double()) @ alpha.double())
+    assert gx is None and float((e.double() - e_ref).abs().max()) <= 2e-5 * float(e_ref.abs().max())
+
+
 @pytest.mark.parametrize("wscale,ascale,xscale", [(0.125, 1.0, 1.0), (1e-3, 1e4, 1.0), (1e-4, 1e20, 1.0), (0.125, 1e-6, 1.0),
                                                   (125.0, 1e-20, 1e-3), (2e-6, 1.0, 6e4), (0.125, 1.0, 0.0)])
 def test_rff_energy_sorted_kernel_over_operand_scales(wscale, ascale, xscale):
