@@ -977,7 +977,7 @@ __host__ __device__ __forceinline__ int force_copies(int nn) {
 // that consecutive lanes have different j and different k, and a wavefront keeps as many private copies of the
 // neighbours' force array as 64 consecutive triples can meet the same neighbour (force_copies).  An instruction's lanes then
 // read, add and write different words, one 16-byte record each, and the copies are summed at the end.  NW wavefronts
-// per atom share out the triples: see wavefronts_per_atom.
+// per atom share out the triples: see wavefronts_backward.
 // COMPACT (one wavefront): the form for capacities at which the copies above do not fit.  [cap] records of three floats hold
 // as many copies as the atom's own neighbours leave room for, at least one; where an instruction's lanes would need more, its
 // s-rows take turns.
@@ -1608,17 +1608,30 @@ int fill_args(FchlArgs& a, const float* X, const int* types, const float* cell, 
 
 constexpr size_t LDS_LIMIT = 64 * 1024;
 
-// Wavefronts per central atom of the forward and backward kernels.  With one, a launch of A atoms is A wavefronts:
-// below about 1000 the chip (8192 slots at eight per SIMD) is idle while every atom walks through its phases alone, the
-// longer the more triples it has; beyond, the work that every wavefront of an atom repeats (staging, the scan of the
-// pairs) costs more than the idle slots.  Measured, us per launch with 1 / 4 / 8 wavefronts forward, 1 / 4 backward:
-//   21 atoms of 1 molecule 9.2 / 7.8 / 7.4, 8.7 / 7.6;    1008 atoms (21 per molecule) 10.1 / 9.0 / 13.4, 9.4 / 10.1;
-//   1200 (12 per molecule) 7.1 / 8.5 / 12.8, 7.4 / 9.6;   2016 (21) 11.7 / 16.6 / 22.5, 11.3 / 16.6;
-//   1600 (40 in a box) 22.6 / 20.0 / 28.2, 25.3 / 24.0;   1536 (96 in a box) 80 / 47 / 59, 85 / 51
+// Wavefronts per central atom.  With one, a launch of A atoms is A wavefronts: below about 1000 the chip (8192 slots at eight
+// per SIMD) is idle while every atom walks through its phases alone, the longer the more triples it has; beyond, the work that
+// every wavefront of an atom repeats (staging, the scan of the pairs) costs more than the idle slots, and the backward kernel, which
+// also sums the wavefronts' forces, meets that with few triples at any A.  Measured, us per launch at three elements:
+//   atoms x molecules (triples of an atom)   forward 1 / 4 / 8      backward 1 / 2 / 4
+//   3 x 1 (1), 3 x 300                       6.1 / 5.8 / 5.9, 6.7 / 7.5 / 11.5        7.4 / 7.6 / 7.7, 8.3 / 8.5 / 9.5
+//   12 x 1 (55), 12 x 20, 12 x 40, 12 x 90   7.6 / 7.0 / 6.9, 7.7 / 7.5 / 7.4, 8.0 / 7.9 / 8.3, 8.7 / 9.7 / 14.6
+//                                                                   6.6 / 6.9 / 7.3, 6.7 / 6.9 / 7.4, 6.9 / 7.2 / 7.8, 7.4 / 8.0 / 9.9
+//   21 x 1 (190), 21 x 12, 21 x 24, 21 x 48  9.4 / 7.6 / 7.3, 9.5 / 8.1 / 7.8, 10.0 / 8.8 / 8.9, 10.4 / 10.0 / 15.2
+//                                                                   8.7 / 8.0 / 7.5, 9.0 / 8.1 / 7.8, 9.3 / 8.8 / 8.4, 9.3 / 9.0 / 10.1
+//   29 x 8 (378), 29 x 20, 29 x 40           15.0 / 8.6 / 8.3, 15.8 / 9.9 / 10.8, 17.0 / 12.1 / 16.8
+//                                                                   12.5 / 9.9 / 9.5, 13.2 / 11.1 / 10.9, 14.9 / 12.8 / 14.1
+//   40 x 40 in a box                         25.8 / 18.6 / 25.4     23.9 / 23.1 / 24.1
+//   96 x 2 in a box, 96 x 16                 78 / 29 / 23, 89 / 48 / 65               66 / 38 / 26, 86 / 65 / 54
+// and at five elements 12 x 40: forward 11.9 / 10.5 / 10.4, 21 x 48: 14.7 / 13.5 / 18.5 and 10.0 / 9.7 / 10.4.  2016 atoms of 21: 11.7 / 16.6 and
+// 11.3 / 16.6 with 1 / 4.
 // big: the neighbourhood does not fit the one-wavefront kernel, or leaves it few wavefronts per CU.
-int wavefronts_per_atom(int A, long long triples, bool big) {
+int wavefronts_forward(int A, long long triples, bool big) {
     if (A <= 256) return 8;
-    if (triples > 100 && A <= (triples > 256 ? 2048 : 1024)) return 4;
+    if (A <= (triples > 256 ? 2048 : triples > 100 ? 1024 : triples > 30 ? 512 : 256)) return 4;
+    return big ? 4 : 1;
+}
+int wavefronts_backward(int A, long long triples, bool big) {
+    if (A <= (triples > 256 ? 2048 : triples > 100 ? 768 : 0)) return 4;
     return big ? 4 : 1;
 }
 
@@ -1643,7 +1656,7 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     const int ns = prm->nspecies, np = ns * (ns + 1) / 2;
     hipStream_t st = (hipStream_t)stream;
     const bool big = alltrip > TCH_MAX;
-    for (int nw = wavefronts_per_atom(A, alltrip, big); nw > 1 || big; nw /= 2) {
+    for (int nw = wavefronts_forward(A, alltrip, big); nw > 1 || big; nw /= 2) {
         // the table holds the triple list, or 12 KB of it at a time
         a.tcap = alltrip <= TCH_WIDE ? (int)alltrip : TCH_WIDE;
         size_t lds = sizeof(float) * (4 * (size_t)(a.tcap + 1) + 12 * (size_t)a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1 +
@@ -1709,7 +1722,7 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     a.tcap = 1;
     for (int k = 1; k <= a.cap; ++k) a.tcap = a.tcap < k * force_copies(k) ? k * force_copies(k) : a.tcap;
     const long long maxnn = nlist ? a.cap : a.cap - 1;
-    for (int nw = std::min(4, wavefronts_per_atom(A, maxnn * (maxnn - 1) / 2, a.cap > 54));; nw /= 2) {
+    for (int nw = wavefronts_backward(A, maxnn * (maxnn - 1) / 2, a.cap > 54);; nw /= 2) {
         // two records [cap][4], atom indices, force copies, type offsets, grids, the bins' constant factors, the gradient row
         const size_t shared = (size_t)9 * a.cap + prm->nspecies + 1 + prm->nRs2 + 2 * prm->nRs3 + R;
         const size_t lds = sizeof(float) * (shared + 4 * (size_t)nw * a.tcap + (nw > 1 ? (size_t)prm->nspecies * nw : 0));

@@ -69,6 +69,14 @@ def test_many_elements(nspecies):
     check(coords, [rng.choice(species, 70)], species, 1, False, nRs2=4, nRs3=3)
 
 
+@pytest.mark.parametrize("case", ["aspirin_c2", "ragged_c3", "flexible_c4"])
+@pytest.mark.parametrize("copies", [1, 20])
+def test_few_atoms(case, copies):
+    """Up to 256 atoms and a few hundred: eight and four wavefronts forward, one and four backward by the number of triples."""
+    (coords, charges), species, kw = CASES[case]()
+    check(coords, charges, species, copies, copies == 1, **kw)
+
+
 @pytest.mark.parametrize("natoms", list(range(2, 18)) + [22, 32, 33, 34, 43, 54, 55, 63, 64, 65, 66])
 def test_every_neighbour_count_has_its_force_copies(natoms):
     """All atoms within the cutoff of each other: nn = natoms - 1 neighbours, one and several wavefronts per atom."""
@@ -79,34 +87,52 @@ def test_every_neighbour_count_has_its_force_copies(natoms):
         check(coords, charges, [1, 6], copies, False, nRs2=3, nRs3=3)
 
 
-@pytest.mark.parametrize("species,forward,backward", [([1, 6, 8], 1268, 1333), ([1, 6, 7, 8, 9], 1259, 1299)])
-def test_capacities_up_to_the_limit_of_the_lds(species, forward, backward):
-    """Small molecules padded to the largest capacities at the default grids: smaller tables and compact force records before
-    a refusal."""
-    from qml_lightning_amd import ops
-    rng = np.random.default_rng(8)
-    prm = oracle_prm(species)
-    coords = [helpers.random_geometry(rng, 19, 6.0, 0.9), helpers.random_geometry(rng, 2, 3.0, 0.9)]
-    X, Z, aid, mid, nat = make_batch(coords, [rng.choice(species, len(c)) for c in coords])
-    cnt, nl = fchl19.neighbours(X, nat, prm.rcut)
-    ty = fchl19.element_types(Z, nat, prm.species)
-    rep = fchl19.forward(X, ty, aid, mid, nl, cnt, prm)
-    g = np.random.default_rng(2).normal(size=rep.shape)
-    v = np.einsum("mif,mijxf->mjx", g, fchl19.jacobian(X, ty, aid, mid, nl, cnt, prm))
-    n = X.shape[1]
+class Padded:
+    """Two small molecules of the given elements at the default grids, in batches padded to any capacity."""
 
-    def call(op, capacity, *first):
+    def __init__(self, species, natoms):
+        rng = np.random.default_rng(8)
+        self.prm = oracle_prm(species)
+        coords = [helpers.random_geometry(rng, natoms, 6.0, 0.9), helpers.random_geometry(rng, 2, 3.0, 0.9)]
+        self.X, Z, self.aid, self.mid, self.nat = make_batch(coords, [rng.choice(species, len(c)) for c in coords])
+        cnt, nl = fchl19.neighbours(self.X, self.nat, self.prm.rcut)
+        self.ty = fchl19.element_types(Z, self.nat, self.prm.species)
+        args = (self.X, self.ty, self.aid, self.mid, nl, cnt, self.prm)
+        self.rep = fchl19.forward(*args)
+        self.g = np.random.default_rng(2).normal(size=self.rep.shape)
+        self.v = np.einsum("mif,mijxf->mjx", self.g, fchl19.jacobian(*args))
+
+    def __call__(self, op, capacity, *first):
+        n = self.X.shape[1]
+
         def pad(a):
             return np.pad(a, [(0, 0), (0, capacity - n)] + [(0, 0)] * (a.ndim - 2), constant_values=0 if a.ndim == 3 else -1)
-        return op(*[t32(pad(f)) for f in first], t32(pad(X)), ti32(pad(ty)), None, None, ti32(aid), ti32(mid), ti32(nat),
-                  t32(prm.Rs2), t32(prm.Rs3), gpu_prm(prm))[:, :n]
+        return op(*[t32(pad(f)) for f in first], t32(pad(self.X)), ti32(pad(self.ty)), None, None, ti32(self.aid), ti32(self.mid),
+                  ti32(self.nat), t32(self.prm.Rs2), t32(self.prm.Rs3), gpu_prm(self.prm))[:, :n]
+
+
+@pytest.mark.parametrize("species,forward,backward", [([1, 6, 8], 1268, 1333), ([1, 6, 7, 8, 9], 1259, 1299)])
+def test_capacities_up_to_the_limit_of_the_lds(species, forward, backward):
+    """The largest capacities: smaller tables and compact force records before a refusal."""
+    from qml_lightning_amd import ops
+    batch = Padded(species, 19)
     for capacity in (forward - 170, forward):
-        close(call(ops.fchl_forward, capacity), rep, REL_REP, "rep, capacity %d" % capacity)
+        close(batch(ops.fchl_forward, capacity), batch.rep, REL_REP, "rep, capacity %d" % capacity)
     for capacity in (backward - 400, backward - 380, backward):
-        close(call(ops.fchl_vjp, capacity, g), v, REL_EF, "vjp, capacity %d" % capacity)
-    for op, first in ((ops.fchl_forward, ()), (ops.fchl_vjp, (g,))):
+        close(batch(ops.fchl_vjp, capacity, batch.g), batch.v, REL_EF, "vjp, capacity %d" % capacity)
+    for op, first in ((ops.fchl_forward, ()), (ops.fchl_vjp, (batch.g,))):
         with pytest.raises(RuntimeError, match="LDS"):
-            call(op, backward + 1, *first)
+            batch(op, backward + 1, *first)
+
+
+@pytest.mark.parametrize("nspecies,capacity", [(10, 70), (12, 64), (16, 300)])
+def test_grids_too_large_for_more_wavefronts(nspecies, capacity):
+    """Many elements at the default grids: the partial blocks leave room for four, two and one wavefronts forward, the force
+    copies for four, four and two backward."""
+    from qml_lightning_amd import ops
+    batch = Padded(list(range(1, nspecies + 1)), 19)
+    close(batch(ops.fchl_forward, capacity), batch.rep, REL_REP, "rep")
+    close(batch(ops.fchl_vjp, capacity, batch.g), batch.v, REL_EF, "vjp")
 
 
 def test_a_thousand_neighbours_and_few():
