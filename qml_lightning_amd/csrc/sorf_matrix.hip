@@ -30,7 +30,8 @@
 //
 // A tile (64 atoms of one element) through all stacks is too coarse a unit: with the three workgroups a CU holds, the last
 // of two rounds of tiles left most of the chip idle.  A workgroup takes an equal share of all (tile, round of stacks) units
-// instead; a tile that two or more shares meet in is written in parts, which sorf_parts_kernel adds up in order.
+// instead; of a tile that two or more shares meet in the first writes its sums where they belong, the others theirs into a
+// part each, which sorf_parts_kernel adds in order.
 // Measured with the gradient / energies only, rows kernel -> this call, at d = 128, 128 stacks: 86016 atoms 764 -> 653 us / 456 -> 305;
 // 24000 atoms 222 -> 214 / 133 -> 108; two transforms, 32 stacks, 33000 atoms 148 -> 143 / 78 -> 75, 86016 atoms 369 -> 314 / 194 -> 148;
 // d = 64, 128 stacks, 86016 atoms 360 -> 309 / 230 -> 147.  Of that 5 us go to the forms and 3 to 4 to the launch behind.  (At d = 256 the
@@ -264,8 +265,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const int tile = u / rounds, r0 = u - tile * rounds, r1 = min(rounds, r0 + uend - u);
         int type, row0, rows;
         find_tile(type_offsets, ne, tile, type, row0, rows);
-        const bool whole = r1 - r0 == rounds;
-        const size_t slot = 2 * (size_t)blockIdx.x + (u != ubeg);       // of the parts, where this is one
+        const bool first_piece = r0 == 0;                               // else a part: only a share's first tile can be one
         if (u != ubeg) __syncthreads();                                 // the buffers of the tile before are free
         u += r1 - r0;
         const int s0 = r0 * SPB, s1 = min(S, r1 * SPB);
@@ -446,12 +446,12 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const int in_tile = first + col;
         if (q == 0) {
             const float e = energy * inv_alpha * normf;
-            if (whole) e_slots[out_index[row0 + in_tile]] = e;
-            else parts[slot * SM_ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
+            if (first_piece) e_slots[out_index[row0 + in_tile]] = e;
+            else parts[(size_t)blockIdx.x * SM_ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
         }
         if constexpr (WITH_GRAD) {
             const float gs = gscale * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
-            float* to = whole ? gx + (size_t)row0 * D : parts + slot * SM_ATOMS * (D + 1) + SM_ATOMS;
+            float* to = first_piece ? gx + (size_t)row0 * D : parts + (size_t)blockIdx.x * SM_ATOMS * (D + 1) + SM_ATOMS;
             float* gr = to + (size_t)in_tile * D + 4 * q;
 #pragma unroll
             for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_t*>(gr + 16 * b) = acc[b] * gs;
@@ -483,19 +483,20 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
     while (share_begin(last + 1, nshares, ntiles, rounds) < tend) ++last;
     int type, row0, rows;
     find_tile(type_offsets, ne, tile, type, row0, rows);
-    const float* head = parts + (2 * (size_t)g + (tbeg != ubeg)) * SLOT;
-    const float* next = parts + 2 * (size_t)(g + 1) * SLOT;
+    const float* next = parts + (size_t)(g + 1) * SLOT;
     const int nparts = last - g;
     for (int t = threadIdx.x; t < rows; t += 256) {
-        float v = head[t];
-        for (int b = 0; b < nparts; ++b) v += next[2 * b * SLOT + t];
-        e_slots[out_index[row0 + t]] = v;
+        float* to = e_slots + out_index[row0 + t];
+        float v = *to;
+        for (int b = 0; b < nparts; ++b) v += next[b * SLOT + t];
+        *to = v;
     }
     if constexpr (WITH_GRAD) {
         for (int t = threadIdx.x; t < rows * (D / 4); t += 256) {
-            f4_t v = *reinterpret_cast<const f4_t*>(head + SM_ATOMS + 4 * t);
-            for (int b = 0; b < nparts; ++b) v += *reinterpret_cast<const f4_t*>(next + 2 * b * SLOT + SM_ATOMS + 4 * t);
-            *reinterpret_cast<f4_t*>(gx + (size_t)row0 * D + 4 * t) = v;
+            f4_t* to = reinterpret_cast<f4_t*>(gx + (size_t)row0 * D) + t;
+            f4_t v = *to;
+            for (int b = 0; b < nparts; ++b) v += *reinterpret_cast<const f4_t*>(next + b * SLOT + SM_ATOMS + 4 * t);
+            *to = v;
         }
     }
 }
@@ -528,7 +529,7 @@ static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, i
     f.unfit = (int*)take(sizeof(int));
     f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
     f.alpha = (float*)take(((size_t)S * d + 1) * sizeof(float));
-    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * 2 * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float));
+    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float));
     return at;
 }
 

@@ -1366,6 +1366,36 @@ def test_sorf_matrix_kernel_is_as_exact_as_the_rows_kernel(monkeypatch, d, T, S,
     assert errors["matrix"][0] <= errors["rows"][0] and errors["matrix"][1] <= errors["rows"][1], errors
 
 
+@pytest.mark.parametrize("R,d,ne,A", [(312, 128, 3, 2304), (312, 128, 3, 16384), (720, 256, 5, 4200), (496, 256, 4, 8192),
+                                      (496, 256, 4, 30000)])
+def test_projections_on_split_operands_are_as_exact_as_in_fp32(monkeypatch, R, d, ne, A):
+    """Batches that ran on the fp32 matrix instructions before they took the prepared reductors: root mean square error against
+    fp64, rows of very different size (three decades) side by side, each measured against itself."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device=dev()).manual_seed(A)
+    size = 10.0 ** (3.0 * torch.rand(A, 1, device=dev(), generator=g) - 2.0)
+    rep = torch.rand(A, R, device=dev(), generator=g) ** 4 * size
+    gx = torch.randn(A, d, device=dev(), generator=g) * size
+    q, _ = torch.linalg.qr(torch.randn(ne, R, d, device=dev(), dtype=torch.float64, generator=g))
+    red = q.float().contiguous()
+    types = torch.randint(0, ne, (A,), device=dev(), generator=g).int()
+    ss, off = ops.sort_by_type(types, torch.arange(A, device=dev(), dtype=torch.int32), ne)
+    order, at = ss.long(), off.tolist()
+    forward, backward = torch.empty(A, d, dtype=torch.float64, device=dev()), torch.empty(A, R, dtype=torch.float64, device=dev())
+    for t in range(ne):
+        part = slice(at[t], at[t + 1])
+        forward[part] = rep[order[part]].double() @ red[t].double()
+        backward[order[part]] = gx[part].double() @ red[t].double().T.contiguous()
+
+    def errors():
+        got = (ops.project_typed(rep, ss, off, red), ops.project_typed_backward(gx, ss, off, red, types, A))
+        return [float(((v.double() - r).pow(2).sum(1) / r.pow(2).sum(1)).mean().sqrt()) for v, r in zip(got, (forward, backward))]
+    split = errors()
+    monkeypatch.setattr(ops, "_split_for", lambda reductors, A: None)
+    plain = errors()
+    assert split[0] <= plain[0] and split[1] <= plain[1], (split, plain)
+
+
 @pytest.mark.parametrize("T,with_grad", [(1, True), (2, False)])
 def test_large_batches_keep_nothing_of_the_model_tensors(T, with_grad):
     """Signs, bias and alpha as they are at the call, however they were written (`.data` and DLPack writes move no version

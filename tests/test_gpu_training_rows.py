@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def molecules(sizes, seed):
-    """One molecule per size; a negative size -k is k atoms on a line."""
+    """One molecule per size; a negative size -k is k atoms on a line, whose angles are degenerate."""
     rng = np.random.default_rng(seed)
     X, Q = [], []
     for k in sizes:
