@@ -21,7 +21,6 @@
 #include <climits>
 #include <functional>
 #include <map>
-#include <memory>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -70,7 +69,7 @@ struct Prepared {
     const void* data;
     Tensor buffer;
     hipStream_t stream;                        // that made it
-    std::shared_ptr<ihipEvent_t> made;         // recorded behind the making, null once it was seen to have passed
+    bool passed;                               // the making is known to be over
 };
 std::mutex prepared_mutex;
 std::map<std::pair<const c10::TensorImpl*, int>, Prepared>& prepared =
@@ -86,19 +85,17 @@ Tensor prepared_form(const Tensor& t, int kind, const std::function<Tensor(const
         Prepared& p = it->second;
         auto alive = p.owner.lock();
         if (alive && alive.get() == t.unsafeGetTensorImpl() && p.version == (int64_t)t._version() && p.data == t.const_data_ptr()) {
-            if (!p.made && p.stream == here.stream()) return p.buffer;
+            if (p.stream == here.stream()) return p.buffer;
+            // another stream waits, once, for whatever the device has to do (an event behind every making, for the few forms that
+            // are ever used elsewhere, made each model's first call some 40 us longer), and the buffer, if it is dropped, for that
+            // stream.  A capture, here or on another thread, cannot wait: it gets a form of its own
             const bool captured = capturing();
-            if (p.made && !captured) {
-                if (hipEventQuery(p.made.get()) == hipSuccess) p.made.reset();
-                else (void)hipGetLastError();                                 // "not ready" is no error of the next launch
+            if (!p.passed && !captured) {
+                p.passed = hipDeviceSynchronize() == hipSuccess;
+                if (!p.passed) (void)hipGetLastError();
             }
-            if (p.stream != here.stream()) {
-                // another stream waits for the making, and the buffer, if it is dropped, for that stream; a capture cannot wait
-                if (p.made && captured) return make(t);
-                if (p.made)
-                    TORCH_CHECK(hipStreamWaitEvent(here.stream(), p.made.get(), 0) == hipSuccess, "waiting for a prepared form failed");
-                if (!captured && p.buffer.defined()) p.buffer.record_stream(here.unwrap());
-            }
+            if (!p.passed) return make(t);
+            if (!captured && p.buffer.defined()) p.buffer.record_stream(here.unwrap());
             return p.buffer;
         }
     }
@@ -108,12 +105,8 @@ Tensor prepared_form(const Tensor& t, int kind, const std::function<Tensor(const
         for (auto e = prepared.begin(); e != prepared.end();) e = e->second.owner.expired() ? prepared.erase(e) : std::next(e);
     }
     Tensor buffer = make(t);
-    hipEvent_t event = nullptr;
-    TORCH_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess, "no event for a prepared form");
-    std::shared_ptr<ihipEvent_t> made(event, [](hipEvent_t e) { (void)hipEventDestroy(e); });
-    TORCH_CHECK(hipEventRecord(event, here.stream()) == hipSuccess, "no event for a prepared form");
     prepared.emplace(key, Prepared{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), (int64_t)t._version(),
-                                   t.const_data_ptr(), buffer, here.stream(), made});
+                                   t.const_data_ptr(), buffer, here.stream(), false});
     return buffer;
 }
 

@@ -720,7 +720,7 @@ def rff_rows(items, Ze, G, nmol, n, row_offsets=None, max_rows=None, overwrite=F
     return G
 
 
-_PRESPLIT = {}    # (id(tensor), kind) -> [weak reference, version, address, prepared buffer, stream, event or None]
+_PRESPLIT = {}    # (id(tensor), kind) -> [weak reference, version, address, prepared buffer, stream, making known to be over]
 
 
 def presplit_cached(t, kind, make):
@@ -733,27 +733,25 @@ def presplit_cached(t, kind, make):
     key, here = (id(t), kind), _stream().value
     hit = _PRESPLIT.get(key)
     if hit is not None and hit[0]() is t and hit[1] == t._version and hit[2] == t.data_ptr():
-        buf, made_on, made = hit[3:]
-        if made is None and made_on == here:
-            return buf
-        captured = torch.cuda.is_current_stream_capturing()
-        if made is not None and not captured and made.query():
-            made = hit[5] = None
-        if made_on != here:
-            # another stream waits for the making, and the buffer, if it is dropped, for that stream; a capture cannot wait
-            if made is not None and captured:
-                return make(t)
-            if not captured:
-                stream = torch.cuda.current_stream(t.device)
-                if made is not None:
-                    stream.wait_event(made)
-                if buf is not None:
-                    buf.record_stream(stream)
+        buf = hit[3]
+        if hit[4] != here:
+            # another stream waits, once, for whatever the device has to do, and the buffer, if it is dropped, for that
+            # stream; a capture, here or on another thread, cannot wait: it gets a form of its own
+            captured = torch.cuda.is_current_stream_capturing()
+            if not hit[5]:
+                if captured:
+                    return make(t)
+                try:
+                    torch.cuda.synchronize(t.device)
+                except RuntimeError:
+                    return make(t)
+                hit[5] = True
+            if not captured and buf is not None:
+                buf.record_stream(torch.cuda.current_stream(t.device))
         return buf
     buf = make(t)
     if not torch.cuda.is_current_stream_capturing():
-        _PRESPLIT[key] = [weakref.ref(t, lambda _r, k=key: _PRESPLIT.pop(k, None)), t._version, t.data_ptr(), buf, here,
-                          torch.cuda.current_stream(t.device).record_event()]
+        _PRESPLIT[key] = [weakref.ref(t, lambda _r, k=key: _PRESPLIT.pop(k, None)), t._version, t.data_ptr(), buf, here, False]
     return buf
 
 
