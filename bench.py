@@ -371,8 +371,7 @@ def main():
     from qml_lightning_amd.utils import peaks as peaks_mod
     peaks = peaks_mod.measure()
     peaks["nominal"] = dict(peaks_mod.NOMINAL)
-    # what a wavefront instruction of each class costs a SIMD, and the per-stack instruction mix of the
-    # fused SORF kernel next to the same mix with its in-row butterfly stages on the matrix pipe
+    # what a wavefront instruction of each class costs a SIMD, and the per-stack instruction mix of the fused SORF kernel
     mixes = peaks_mod.instruction_mixes()
     best = {k: min(v.values()) for k, v in mixes.items()}
     instruction_mixes = {
@@ -380,8 +379,8 @@ def main():
         "ns_per_instruction": {"plain_fp32": best["plain_fp32_x128"] / 128 * 1e9, "dpp_fmac": best["dpp_fmac_x128"] / 128 * 1e9,
                                "transcendental": best["transcendental_x128"] / 128 * 1e9},
         "fused_kernel_stack_ns": best["fused_kernel_stack"] * 1e9,
-        "note": "one iteration of fused_kernel_stack = 82 plain + 64 DPP + 16 transcendental wavefront instructions = one "
-                "stack of four atoms at 128 components",
+        "note": "one iteration of fused_kernel_stack = 307 plain + 32 packed conversions + 32 mixed-precision subtractions + 64 "
+                "transcendental + 16 matrix wavefront instructions = one stack of sixteen atoms at 128 components",
     }
     torch.cuda.empty_cache()
 
@@ -555,11 +554,12 @@ def main():
     # fused kernel, algorithmic flops per atom: forward+adjoint butterflies 2*F*log2(d), D multiplies 2F,
     # scale+bias FMA 2F, one sin and one cos per feature 2F, energy FMA 2F, alpha*norm*sin 2F
     fused_flops = A * F * (2 * log2d + 10)
-    # 162 vector instructions per wavefront and stack in the kernel's main loop at d = 128 (8 coefficients
-    # per lane; counted in its ISA): 82 plain fp32, 64 DPP butterflies, 8 v_sin_f32 + 8 v_cos_f32
+    # sorf_energy_matrix_kernel (with the launches around it): per wavefront (16 atoms) and stack at d = 128, 435 vector
+    # instructions in its main loop (counted in its ISA: 307 plain fp32, 32 packed conversions, 32 mixed-precision subtractions, 32
+    # v_sin_f32 + 32 v_cos_f32) and 16 v_mfma_f32_16x16x32_f16
     kernels["sorf_energy_fused"] = {"seconds": t_fused, "bound": "valu", "TFLOPs": fused_flops / t_fused / 1e12,
                                     "sincos_per_s": A * F / t_fused,
-                                    "valu_wave_instr_per_s": 162.0 / 8.0 * A * F / 64 / t_fused}
+                                    "valu_wave_instr_per_s": 435.0 / 16.0 * A * NSTACKS / t_fused}
     # the two-operator contract, kernel by kernel: `seconds` and the bytes are those of ONE launch, the
     # element with the most atoms (the launch the profiler's per-dispatch counters describe);
     # `seconds_all_elements` sums the launches of the three elements of one step
@@ -687,9 +687,9 @@ def main():
             v["frac"] = v["exp_per_s"] / exp_nominal
             v["frac_of_measured"] = v["exp_per_s"] / peaks["exp_per_s"]
     kernels["sorf_energy_fused"]["frac"] = kernels["sorf_energy_fused"]["TFLOPs"] / FP32_PEAK_TFLOPS
-    # a wavefront of the fused kernel carries four atoms through one stack per iteration: its time per
+    # a wavefront of the fused kernel carries sixteen atoms through one stack per iteration: its time per
     # wavefront-stack per SIMD against the bare instruction mix of such an iteration (probe kernel)
-    wave_stacks_per_simd = (A / 4.0) * NSTACKS / 1024.0
+    wave_stacks_per_simd = (A / 16.0) * NSTACKS / 1024.0
     kernels["sorf_energy_fused"]["ns_per_wavefront_stack_per_simd"] = t_fused / wave_stacks_per_simd * 1e9
     kernels["sorf_energy_fused"]["instruction_mix_ns"] = instruction_mixes["fused_kernel_stack_ns"]
     kernels["sorf_energy_fused"]["frac_of_instruction_mix"] = (
@@ -702,13 +702,13 @@ def main():
                     "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": kernels[dominant]["TFLOPs"] / FP32_PEAK_TFLOPS,
                     "frac_of_instruction_mix": kernels[dominant]["frac_of_instruction_mix"],
                     "traffic": kernels[dominant].get("traffic_bytes"),
-                    "note": "fused FWHT+sincos kernel: neither HBM nor MFMA bounds it (8d bytes per atom, no "
-                            "contraction); it is bound by vector instruction issue.  Algorithmic flops count one "
-                            "flop per sin and per cos and per butterfly add, while a butterfly across lanes issues "
-                            "at half rate and v_sin/v_cos at quarter rate, none of them an FMA, so the fraction of "
-                            "the fp32 FMA peak understates it: frac_of_instruction_mix is the time a probe kernel needs for the "
-                            "bare instruction mix of one wavefront-stack (82 plain + 64 DPP + 16 transcendental, independent "
-                            "registers, no memory access) over the kernel's own time per wavefront-stack, both measured in this run; "
+                    "note": "fused FWHT+sincos kernel: it is bound by vector instruction issue, not by HBM (8d bytes per atom) and not by "
+                            "the matrix pipe, which does the 16-point blocks of the transforms on operands split in two fp16 parts.  "
+                            "Algorithmic flops count one flop per sin and per cos and per butterfly add, while v_sin/v_cos issue at "
+                            "quarter rate and the splits are not counted, so the fraction of the fp32 FMA peak understates it: "
+                            "frac_of_instruction_mix is the time a probe kernel needs for the bare instruction mix of one "
+                            "wavefront-stack (307 plain + 64 split + 64 transcendental + 16 matrix, independent registers, no memory "
+                            "access) over the time of the whole call (forms, kernel, parts) per wavefront-stack, both measured in this run; "
                             "traffic = bytes per launch from profiles/pmc_traffic.json"}
     else:
         roofline = {"kernel": dominant, "bound": "valu", "achieved": kernels[dominant]["exp_per_s"] / 1e12,

@@ -559,7 +559,8 @@ double qmll_probe_rate(int which, int iters, int blocks_per_cu, void* out, qmll_
 
 /* Straight-line loops of the instruction classes the fused SORF kernel issues, on independent
  * registers: mix = 0 128 plain fp32, 1 128 DPP fmac, 2 128 v_sin_f32, 3 the per-stack mix of the
- * fused kernel at 128 components (82 plain + 64 DPP + 16 transcendental).
+ * matrix-core energy kernel with the gradient at 128 components (307 plain + 64 that split operands + 64 transcendental + 16
+ * matrix instructions).
  * Returns wavefront-iterations per SIMD (blocks_per_cu x iters), so
  * duration x clock / that = SIMD clocks per iteration; negative on error. */
 double qmll_probe_mix(int mix, int iters, int blocks_per_cu, void* out, qmll_stream_t stream);

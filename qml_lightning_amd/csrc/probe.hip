@@ -129,11 +129,11 @@ __global__ __launch_bounds__(PT) void probe_exp_kernel(int iters, float* __restr
 }
 
 // ---- instruction mixes -------------------------------------------------------------------
-// Straight-line loops of the instruction classes the fused SORF kernel issues, alone and mixed,
+// Straight-line loops of the instruction classes the fused SORF kernels issue, alone and mixed,
 // on independent registers: what a wavefront instruction of each class costs a SIMD.  One
-// iteration of MIX_FUSED stands for one stack of one wavefront of that kernel at 128 components
-// (8 registers per lane, four atoms per wavefront): 82 plain fp32 + 64 DPP fmac + 16
-// transcendental instructions, counted in its ISA.
+// iteration of MIX_FUSED stands for one stack of one wavefront of sorf_energy_matrix_kernel at 128 components with the
+// gradient (16 atoms per wavefront): 307 plain fp32, 32 packed conversions, 32 mixed-precision subtractions, 64 transcendental
+// and 16 matrix instructions (v_mfma_f32_16x16x32_f16), counted in its ISA.
 enum { MIX_PLAIN = 0, MIX_DPP = 1, MIX_TRANS = 2, MIX_FUSED = 3, MIX_COUNT = 4 };
 
 template <int N>
@@ -153,9 +153,32 @@ __device__ __forceinline__ void trans_ops(float (&v)[8]) {
     for (int k = 0; k < N; ++k) v[k & 7] = __builtin_amdgcn_sinf(v[k & 7]);
 }
 
+// a packed conversion to fp16 and what it left of a value
+template <int N>
+__device__ __forceinline__ void split_ops(float (&v)[8]) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        asm volatile("v_cvt_pk_f16_f32 v0, %0, %1\n\tv_fma_mix_f32 %0, v0, -1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]"
+                     : "+v"(v[k & 7]) : "v"(v[(k + 1) & 7]) : "v0");
+}
+template <int N>
+__device__ __forceinline__ void matrix_ops(floatx4 (&m)[8], half8_t a, half8_t b) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) m[k & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, m[k & 7], 0, 0, 0);
+}
+
 template <int MIX>
 __global__ __launch_bounds__(PT) void probe_mix_kernel(int iters, float* __restrict__ out) {
     float v[8];
+    [[maybe_unused]] floatx4 m[8];
+    [[maybe_unused]] half8_t a, b;
+    if constexpr (MIX == MIX_FUSED) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            a[k] = b[k] = (_Float16)(threadIdx.x & 1 ? 1.0f : -1.0f);
+            m[k] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = 0.001f * (float)((threadIdx.x & 31) + k);
     const float c = (threadIdx.x & 1) ? -0.5f : 0.5f;
@@ -164,20 +187,22 @@ __global__ __launch_bounds__(PT) void probe_mix_kernel(int iters, float* __restr
         if constexpr (MIX == MIX_DPP) dpp_ops<128>(v, c);
         if constexpr (MIX == MIX_TRANS) trans_ops<128>(v);
         if constexpr (MIX == MIX_FUSED) {
-            // forward: sign multiply + register stages, in-row stages, argument, sincos, products;
-            // adjoint: register stages, in-row stages, accumulate
-            plain_ops<28>(v, c);
-            dpp_ops<32>(v, c);
-            plain_ops<8>(v, c);
-            trans_ops<16>(v);
-            plain_ops<18>(v, c);
-            dpp_ops<32>(v, c);
-            plain_ops<28>(v, c);
+            // forward: blocks, register stages, argument, sincos, products; adjoint: register stages, split, blocks, accumulate
+            matrix_ops<8>(m, a, b);
+            plain_ops<128>(v, c);
+            trans_ops<64>(v);
+            plain_ops<147>(v, c);
+            split_ops<32>(v);
+            matrix_ops<8>(m, a, b);
+            plain_ops<32>(v, c);
         }
     }
     float s = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s += v[k];
+    for (int k = 0; k < 8; ++k) {
+        s += v[k];
+        if constexpr (MIX == MIX_FUSED) s += m[k][0];
+    }
     out[(size_t)blockIdx.x * PT + threadIdx.x] = s;
 }
 
