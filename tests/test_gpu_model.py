@@ -432,6 +432,24 @@ def test_kernels_follow_the_current_stream():
 
 
 @pytest.mark.parametrize("kind", ["sorf", "rff"])
+def test_forget_prepared_after_a_write_that_torch_does_not_see(kind):
+    """alpha (fp64) and the reductors through `.data`, 2400 atoms: beyond the small-batch kernels, which read the reductors."""
+    coords, charges = helpers.fixed_composition_batch(helpers.ASPIRIN, 115, 1)
+    m = build_sorf_model([1, 6, 8], 128, 8)[0] if kind == "sorf" else build_rff_model([1, 6, 8], 128, 8)
+    m = m[0] if isinstance(m, tuple) else m
+    args = inputs(*make_batch(coords, charges))
+    m.energies_and_forces(*args)
+    for t, by in ((m.alpha, 2.0), (m.reductors, 0.5)):
+        t.data.mul_(by)
+        m.forget_prepared()
+        e, f = m.energies_and_forces(*args)
+        fresh = t.clone()
+        setattr(m, "alpha" if t is m.alpha else "reductors", fresh)
+        e_ref, f_ref = m.energies_and_forces(*args)
+        assert (e - e_ref).abs().max() <= 1e-6 * e_ref.abs().max() and (f - f_ref).abs().max() <= 1e-5 * f_ref.abs().max()
+
+
+@pytest.mark.parametrize("kind", ["sorf", "rff"])
 def test_predict_step_replayed_from_a_captured_graph(kind):
     """The predict step allocates only through torch and records no memset nodes, so it can be captured
     in a HIP graph.  The graph is replayed five times with changed coordinates, with the program's own
