@@ -14,6 +14,8 @@
 // (gram_mirror_kernel), once per call or once after the caller's last batch.  Algorithmic work: M*F*(F+1) flops, 8*M*F bytes read once (re-reads of a
 // panel by the tiles of one row/column are served from L2: consecutive workgroup ids walk
 // along a tile row).
+// From 768 rows the full symmetric product comes from gram_modular.hip instead; this kernel keeps smaller batches, row
+// blocks (ntiles > 1), columns that cannot be scaled, and the updates of the Cholesky factorisation.
 #include "qmll_common.h"
 #include "gram_tiles.h"
 
@@ -43,7 +45,9 @@ template <bool SYM, bool GUARD, bool GEN>
 __global__ __launch_bounds__(GT, 2) void gram_kernel(const double* __restrict__ Z, int M, int F, int f0, int f1,
                                                       int nti, int ntj, TileMap tm, double* __restrict__ C,
                                                       long long ldz_, long long ldc_, double sign_,
-                                                      const double* __restrict__ Za_, long long lda_, int overwrite_) {
+                                                      const double* __restrict__ Za_, long long lda_, int overwrite_,
+                                                      const int* __restrict__ only_if_) {
+    if (GEN && only_if_ && *only_if_ == 0) return;
     unsigned bid = blockIdx.x;
     const bool split = GEN && tm.pieces > 1;          // one of several row ranges of a tile, to the workspace
     if (split) {
@@ -293,7 +297,7 @@ constexpr size_t GRAM_WS_BYTES = GRAM_WS_TILES * TILE * TILE * sizeof(double);
 static int gram_launch(const double* Z, const double* y, int M, int F, int f0, int f1, bool sym, bool mirror, double* C,
                        double* ZTy, hipStream_t stream, const char* who, long long ldz = 0, long long ldc = 0,
                        double sign = 1.0, const double* Za = nullptr, long long lda = 0, int overwrite = 0,
-                       double* ws = nullptr, size_t ws_bytes = 0) {
+                       double* ws = nullptr, size_t ws_bytes = 0, const int* only_if = nullptr) {
     if (ldz == 0) ldz = F;
     if (ldc == 0) ldc = F;
     if (!Za) {   // the Gram product: both operands are Z
@@ -354,10 +358,10 @@ static int gram_launch(const double* Z, const double* y, int M, int F, int f0, i
                        (lda % 2) != 0 || (reinterpret_cast<uintptr_t>(Z) % 16) != 0 ||
                        (reinterpret_cast<uintptr_t>(Za) % 16) != 0;
     const dim3 grid((unsigned)nblocks), block(GT);
-    const bool gen = Za != Z || ldz != F || ldc != F || lda != F || sign != 1.0 || overwrite != 0;
+    const bool gen = Za != Z || ldz != F || ldc != F || lda != F || sign != 1.0 || overwrite != 0 || only_if;
 #define QMLL_GRAM_LAUNCH(S, G, E)                                                                              \
     hipLaunchKernelGGL((gram_kernel<S, G, E>), grid, block, 0, stream, Z, M, F, sym ? 0 : f0, sym ? F : f1, nti, \
-                       ntj, tm, C, ldz, ldc, sign, Za, lda, overwrite)
+                       ntj, tm, C, ldz, ldc, sign, Za, lda, overwrite, only_if)
     if (gen) {
         if (sym && !guard) QMLL_GRAM_LAUNCH(true, false, true);
         else if (sym) QMLL_GRAM_LAUNCH(true, true, true);
@@ -375,10 +379,10 @@ static int gram_launch(const double* Z, const double* y, int M, int F, int f0, i
         const dim3 tgrid((unsigned)(ntail_ids * tail.pieces));
         if (guard)
             hipLaunchKernelGGL((gram_kernel<true, true, true>), tgrid, block, 0, stream, Z, M, F, 0, F, nti, ntj, tail, ws,
-                               ldz, ldc, sign, Za, lda, overwrite);
+                               ldz, ldc, sign, Za, lda, overwrite, nullptr);
         else
             hipLaunchKernelGGL((gram_kernel<true, false, true>), tgrid, block, 0, stream, Z, M, F, 0, F, nti, ntj, tail, ws,
-                               ldz, ldc, sign, Za, lda, overwrite);
+                               ldz, ldc, sign, Za, lda, overwrite, nullptr);
         QMLL_CHECK_LAUNCH(who);
         hipLaunchKernelGGL(gram_tail_reduce_kernel, dim3((unsigned)ntail_ids), dim3(256), 0, stream, ws, ntj, tail, F, C, ldc);
         QMLL_CHECK_LAUNCH(who);
@@ -439,6 +443,12 @@ extern "C" int qmll_matmul_and_reduce(const float* A, const float* B, int Ar, in
     hipLaunchKernelGGL(matmul_and_reduce_kernel, grid, dim3(MR * MR), 0, (hipStream_t)stream, A, B, Ar, K, Bc, C);
     QMLL_CHECK_LAUNCH("qmll_matmul_and_reduce");
     return QMLL_OK;
+}
+
+// used by gram_modular.hip: C += Z^T Z on the tiles on or above the diagonal, on the device only if *only_if is not 0
+int qmll_internal_gram_if(const double* Z, int M, int F, double* C, const int* only_if, hipStream_t stream) {
+    return gram_launch(Z, nullptr, M, F, 0, F, true, false, C, nullptr, stream, "qmll_gram_modular_f64", 0, 0, 1.0, nullptr, 0, 0,
+                       nullptr, 0, only_if);
 }
 
 // used by solve.hip: tiles on or above the diagonal of C[n,n] += sign * Z^T Z with strided operands

@@ -851,7 +851,9 @@ def _gram_workspace(device):
 def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True):
     """ZTZ += Z^T Z (or the row block f0:f1 of it), ZTy += Z^T y, fp64, in place.
     mirror=False (full matrix only) accumulates just the tiles on or above the diagonal: a
-    caller adding several batches finishes with one `gram_mirror(ZTZ)`."""
+    caller adding several batches finishes with one `gram_mirror(ZTZ)`.  From 768 rows the full matrix comes from
+    exact integer products on the int8 matrix cores (an entry is off by about 2^-54 of the product of its two
+    columns' norms); fewer rows, row blocks and columns with NaN or infinite entries take the fp64 matrix cores."""
     if Zrows.dtype != torch.float64 or not Zrows.is_contiguous():
         raise RuntimeError("gram needs a contiguous float64 row matrix")
     M, F = Zrows.shape
@@ -862,6 +864,18 @@ def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True):
             raise RuntimeError("targets have %d rows, features have %d" % (yv.shape[0], M))
     zty = ZTy if ZTy is not None else None
     if f0 is None:
+        nbytes = int(_lib.lib().qmll_gram_modular_workspace_bytes(M, F))
+        if nbytes:
+            try:
+                work = torch.empty(nbytes, dtype=torch.uint8, device=Zrows.device)
+            except torch.cuda.OutOfMemoryError:
+                work = None                     # the fp64 kernel needs no such workspace
+            if work is not None:
+                check(_lib.lib().qmll_gram_modular_f64(_ptr(Zrows), _ptr(yv), M, F, _ptr(ZTZ), _ptr(zty), _ptr(work), nbytes,
+                                                       _stream()), "qmll_gram_modular_f64")
+                if mirror:
+                    check(_lib.lib().qmll_gram_mirror_f64(_ptr(ZTZ), F, _stream()), "qmll_gram_mirror_f64")
+                return ZTZ, ZTy
         # with a workspace the last, sparsely filled round of tiles is split over the idle CUs
         ws = _gram_workspace(Zrows.device) if M >= 2048 else None
         check(_lib.lib().qmll_gram_upper_ws_f64(_ptr(Zrows), _ptr(yv), M, F, _ptr(ZTZ), _ptr(zty), _ptr(ws),

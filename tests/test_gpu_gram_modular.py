@@ -1,0 +1,131 @@
+"""Z^T Z from exact integer products (csrc/gram_modular.hip) against sums in extended precision and against the fp64 kernel."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev():
+    return torch.device("cuda:0")
+
+
+def modular(Z, y=None, start=0.0):
+    from qml_lightning_amd import _lib
+    from qml_lightning_amd.ops import _ptr, _stream
+    L = _lib.lib()
+    M, F = Z.shape
+    C = torch.full((F, F), start, dtype=torch.float64, device=dev())
+    zy = torch.full((F,), start, dtype=torch.float64, device=dev()) if y is not None else None
+    n = int(L.qmll_gram_modular_workspace_bytes(max(M, 768), F))     # what more rows need is enough for fewer
+    ws = torch.full((n,), 77, dtype=torch.uint8, device=dev())        # whatever the workspace holds must not matter
+    rc = L.qmll_gram_modular_f64(_ptr(Z), _ptr(y), M, F, _ptr(C), _ptr(zy), _ptr(ws), n, _stream())
+    assert rc == 0, _lib.last_error()
+    return C, zy
+
+
+def fp64_kernel(Z, start=0.0):
+    from qml_lightning_amd import _lib
+    from qml_lightning_amd.ops import _ptr, _stream
+    M, F = Z.shape
+    C = torch.full((F, F), start, dtype=torch.float64, device=dev())
+    rc = _lib.lib().qmll_gram_upper_f64(_ptr(Z), None, M, F, _ptr(C), None, _stream())
+    assert rc == 0, _lib.last_error()
+    return C
+
+
+def upper(F):
+    t = torch.arange(F) // 128
+    return (t[:, None] <= t[None, :]).numpy()
+
+
+def within_norms(C, Z, what):
+    """Every entry within what the rounding of the columns to norm 2^53 .. 2^54 gives: the sum over the rows of independent
+    errors of at most half a unit against the other column is normal with a standard deviation of 2^-53 sqrt(2/12) of the
+    product of the norms at most; eight of these, and the rounding of the reference's and the result's own 53 bits."""
+    ref = (Z.astype(np.longdouble).T @ Z.astype(np.longdouble))
+    norm = np.sqrt(np.diagonal(ref))
+    bound = 8 * 2.0 ** -53 * np.sqrt(2 / 12) * norm[:, None] * norm[None, :] + 2.0 ** -52 * np.abs(ref)
+    off = np.abs(C - ref) / np.maximum(bound, np.finfo(np.longdouble).tiny)
+    assert (off[upper(Z.shape[1])] <= 1.0).all(), (what, float(off[upper(Z.shape[1])].max()))
+
+
+# one tile and less, one column more than a tile, several tiles, row counts around the stage of 64 and the pair of 128 rows,
+# row ranges (few tiles, many rows)
+@pytest.mark.parametrize("M,F", [(1, 5), (63, 24), (64, 256), (129, 257), (768, 300), (1000, 600), (4100, 130)])
+def test_modular_gram_against_extended_precision(M, F):
+    rng = np.random.default_rng(M + F)
+    Z = rng.normal(size=(M, F)) * np.exp(2.0 * rng.normal(size=F))
+    y = rng.normal(size=M)
+    Zd, yd = torch.tensor(Z, device=dev()), torch.tensor(y, device=dev())
+    C, zy = modular(Zd, yd)
+    again, zy2 = modular(Zd, yd)
+    assert torch.equal(C, again) and torch.equal(zy, zy2)
+    assert (C.cpu().numpy()[~upper(F)] == 0).all()
+    within_norms(C.cpu().numpy(), Z, "plain")
+    ref = Z.astype(np.longdouble).T @ y
+    assert (np.abs(zy.cpu().numpy() - ref) <= M * 2.0 ** -53 * (np.abs(Z).T @ np.abs(y))).all()     # a sum of M products
+    onto, _ = modular(Zd, yd, 3.0)
+    assert (onto.cpu().numpy()[~upper(F)] == 3.0).all()
+    assert np.abs(onto.cpu().numpy() - 3.0 - C.cpu().numpy())[upper(F)].max() <= 2.0 ** -52 * (3.0 + C.abs().max().item())
+
+
+def test_modular_gram_of_uneven_columns():
+    """Columns of zeros, of one dominating entry (whose residues need their quotient corrected), of very small and very large
+    numbers, of exact integers."""
+    rng = np.random.default_rng(5)
+    M, F = 900, 140
+    Z = rng.normal(size=(M, F))
+    Z[:, 3] = 0.0
+    Z[:, 10:20] = 0.0
+    Z[7, 10:20] = rng.normal(size=10)                    # one entry only
+    Z[5, 20:40] *= 2.0 ** np.arange(20, 60, 2)           # one entry far above the others
+    Z[:, 40:50] *= 1e-95
+    Z[:, 50:60] *= 1e130
+    Z[:, 60:70] = rng.integers(-40, 40, (M, 10))
+    Z[:, 70:80] = 1.0                                    # equal entries
+    Z[:, 80] = -Z[:, 81]
+    C, _ = modular(torch.tensor(Z, device=dev()))
+    C = C.cpu().numpy()
+    within_norms(C, Z, "uneven")
+    assert (C[3] == 0).all() and (C[:, 3] == 0).all()
+    ints = np.r_[60:80]
+    assert np.array_equal(C[np.ix_(ints, ints)], Z[:, ints].T @ Z[:, ints])      # whole numbers stay whole
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf"), 1e160, 1e-170])
+def test_columns_that_cannot_be_scaled_take_the_fp64_kernel(value):
+    """NaN, infinities, squares that overflow or vanish: decided on the device, the result is the fp64 kernel's."""
+    g = torch.Generator(device="cpu").manual_seed(11)
+    Z = torch.randn(800, 384, dtype=torch.float64, generator=g).to(dev())
+    if value == 1e-170:
+        Z[:, 200] = 0.0
+    Z[123, 200] = value
+    C, _ = modular(Z, start=1.0)
+    assert torch.equal(torch.nan_to_num(C, nan=0.5), torch.nan_to_num(fp64_kernel(Z, 1.0), nan=0.5))
+    assert torch.equal(C.isnan(), fp64_kernel(Z, 1.0).isnan())
+
+
+def test_modular_gram_in_a_graph_is_the_eager_result():
+    g = torch.Generator(device="cpu").manual_seed(2)
+    Z = torch.randn(1100, 300, dtype=torch.float64, generator=g).to(dev())
+    from qml_lightning_amd import ops
+    C = torch.zeros(300, 300, dtype=torch.float64, device=dev())
+    ops.gram(Z, None, C, None)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ops.gram(Z, None, C.zero_(), None)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        C.zero_()
+        ops.gram(Z, None, C, None)
+    for seed in range(3):
+        Z.copy_(torch.randn(1100, 300, dtype=torch.float64, generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = torch.zeros_like(C)
+        ops.gram(Z, None, ref, None)
+        torch.cuda.synchronize()
+        assert torch.equal(C, ref), seed

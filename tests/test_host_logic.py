@@ -224,6 +224,21 @@ def test_gram_tile_map_meets_every_tile_once_and_balances_the_xcds(tmp_path):
     assert out.stdout.startswith("ok")
 
 
+def test_modular_gram_plan_covers_every_tile_and_row(tmp_path):
+    """tests/cpp/check_gram_modular.cpp: tile order, row passes, tile ranges and workspace of the modular Gram product."""
+    import shutil
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    exe = str(tmp_path / "check_gram_modular")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(root, "qml_lightning_amd", "csrc"),
+                    os.path.join(root, "tests", "cpp", "check_gram_modular.cpp"), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.startswith("ok")
+
+
 def test_rff_fused_true_refuses_a_width_without_a_fused_kernel():
     from qml_lightning_amd.models.random_features import RandomFourrierFeaturesModel
     from qml_lightning_amd.representations.FCHL import FCHLCuda
