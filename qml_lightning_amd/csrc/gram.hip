@@ -445,10 +445,10 @@ extern "C" int qmll_matmul_and_reduce(const float* A, const float* B, int Ar, in
     return QMLL_OK;
 }
 
-// used by gram_modular.hip: C += Z^T Z on the tiles on or above the diagonal, on the device only if *only_if is not 0
-int qmll_internal_gram_if(const double* Z, int M, int F, double* C, const int* only_if, hipStream_t stream) {
-    return gram_launch(Z, nullptr, M, F, 0, F, true, false, C, nullptr, stream, "qmll_gram_modular_f64", 0, 0, 1.0, nullptr, 0, 0,
-                       nullptr, 0, only_if);
+// used by gram_modular.hip: C += sign Z^T Z on the tiles on or above the diagonal, on the device only if *only_if is not 0
+int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, const int* only_if,
+                          const char* who, hipStream_t stream) {
+    return gram_launch(Z, nullptr, M, F, 0, F, true, false, C, nullptr, stream, who, ldz, ldc, sign, nullptr, 0, 0, nullptr, 0, only_if);
 }
 
 // used by solve.hip: tiles on or above the diagonal of C[n,n] += sign * Z^T Z with strided operands

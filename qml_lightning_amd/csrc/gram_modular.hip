@@ -78,8 +78,8 @@ constexpr double SHIFTER = 6755399441055744.0;     // 1.5 * 2^52: adding it roun
 
 // ---- norms -----------------------------------------------------------------------------------------
 // sums of squares (and of products with y) over NORM_ROWS rows per column; thread = column, eight rows in flight
-__global__ __launch_bounds__(256) void column_norms_kernel(const double* __restrict__ Z, const double* __restrict__ y,
-                                                           int M, int F, double* __restrict__ parts,
+__global__ __launch_bounds__(256) void column_norms_kernel(const double* __restrict__ Z, long long ldz,
+                                                           const double* __restrict__ y, int M, int F, double* __restrict__ parts,
                                                            double* __restrict__ yparts, int* __restrict__ flag) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *flag = 0;
     const int f = blockIdx.x * 256 + threadIdx.x;
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void column_norms_kernel(const double* __restr
     for (; m + 8 <= m1; m += 8) {
         double v[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = Z[(size_t)(m + q) * F + f];
+        for (int q = 0; q < 8; ++q) v[q] = Z[(size_t)(m + q) * ldz + f];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             s = fma(v[q], v[q], s);
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void column_norms_kernel(const double* __restr
         }
     }
     for (; m < m1; ++m) {
-        const double v = Z[(size_t)m * F + f];
+        const double v = Z[(size_t)m * ldz + f];
         s = fma(v, v, s);
         any |= v != 0.0;
         if (y) t = fma(v, y[m], t);
@@ -173,7 +173,7 @@ __device__ __forceinline__ void residue_bytes(const double (&v)[16], signed char
     }
 }
 
-__global__ __launch_bounds__(256) void residues_kernel(const double* __restrict__ Z, int M, int F, int Fp,
+__global__ __launch_bounds__(256) void residues_kernel(const double* __restrict__ Z, long long ldz, int M, int F, int Fp,
                                                        const double* __restrict__ scale, const int* __restrict__ flag,
                                                        signed char* __restrict__ planes, size_t plane) {
     if (*flag) return;
@@ -186,10 +186,10 @@ __global__ __launch_bounds__(256) void residues_kernel(const double* __restrict_
     const bool fin = f < F;
     if (fin && k0 + 16 <= M) {
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = Z[(size_t)(k0 + q) * F + f];
+        for (int q = 0; q < 16; ++q) v[q] = Z[(size_t)(k0 + q) * ldz + f];
     } else {
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = (fin && k0 + q < M) ? Z[(size_t)(k0 + q) * F + f] : 0.0;
+        for (int q = 0; q < 16; ++q) v[q] = (fin && k0 + q < M) ? Z[(size_t)(k0 + q) * ldz + f] : 0.0;
     }
     const double s = scale[f];
     double big = 0.0;
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, 1) void modular_gemm_kernel(const signed char*
 // integer below 2^53 and so exact in fp64; C += V 2^-(2 GAMMA - e_i - e_j)
 __global__ __launch_bounds__(256) void reconstruct_kernel(const signed char* __restrict__ res, int pieces, int nt, int t0, int ntile,
                                                           int F, const int* __restrict__ expo, const int* __restrict__ flag,
-                                                          double* __restrict__ C) {
+                                                          double sign, double* __restrict__ C, long long ldc) {
     if (*flag) return;
     const int tile = blockIdx.x >> 4, sub = blockIdx.x & 15;        // 16 workgroups of 4 wavefronts, a 16 x 64 block each
     int ti, tj;
@@ -412,34 +412,21 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(const signed char* __r
         a1 = fma(-c1, B, a1);
         a2 += c1;
         const double v = fma(fma(a2, B, a1), B, a0);
-        C[(size_t)i * F + j] += ldexp(v, expo[i] + expo[j] - 2 * GAMMA);
+        C[(size_t)i * ldc + j] += ldexp(sign * v, expo[i] + expo[j] - 2 * GAMMA);
     }
 }
 
 }  // namespace
 
 // gram.hip: the fp64 kernel over tiles on or above the diagonal, on the device only if *only_if is not 0
-int qmll_internal_gram_if(const double* Z, int M, int F, double* C, const int* only_if, hipStream_t stream);
+int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, const int* only_if,
+                          const char* who, hipStream_t stream);
 
-extern "C" size_t qmll_gram_modular_workspace_bytes(int M, int F) {
-    // Below MODULAR_MIN_ROWS rows the bytes out of the products and their reconstruction, 2.3 ms at 16384 features whatever
-    // the rows, outweigh the sums: 0.87 (fp64 kernel) against 2.3 ms for 128 rows, 1.60 / 2.64 for 320, 3.64 / 3.20 for
-    // 800, 8.6 / 4.7 for 2000; at 1024 features 0.042 / 0.055, 0.086 / 0.082, 0.25 / 0.10 and 0.41 / 0.12 ms.
-    if (M < MODULAR_MIN_ROWS || F <= 0) return 0;
-    return modular_plan(M, F).bytes;
-}
-
-extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
-                                     size_t workspace_bytes, qmll_stream_t stream_) {
-    const char* who = "qmll_gram_modular_f64";
-    hipStream_t stream = (hipStream_t)stream_;
-    QMLL_REQUIRE(M >= 0 && F > 0, QMLL_ERR_INVALID, "%s: bad size M=%d F=%d", who, M, F);
-    if (M == 0) return QMLL_OK;
-    QMLL_REQUIRE(Z && ZTZ && workspace, QMLL_ERR_INVALID, "%s: null pointer", who);
-    QMLL_REQUIRE((y == nullptr) == (ZTy == nullptr), QMLL_ERR_INVALID, "%s: y and ZTy must both be given or both be NULL", who);
-    const ModularPlan pl = modular_plan(M, F);      // any number of rows: the entry takes what it is given
-    QMLL_REQUIRE(workspace_bytes >= pl.bytes && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, QMLL_ERR_INVALID,
-                 "%s: needs %zu bytes of workspace, 16-byte aligned", who, pl.bytes);
+// C[F,F] (row stride ldc, tiles on or above the diagonal) += sign Z^T Z, Z = M rows of F columns with row stride ldz; ZTy += Z^T y.
+// Also used by solve.hip.
+int qmll_internal_modular_syrk(const double* Z, long long ldz, const double* y, int M, int F, double* C, long long ldc, double sign,
+                               double* ZTy, void* workspace, const char* who, hipStream_t stream) {
+    const ModularPlan pl = modular_plan(M, F);
     char* ws = (char*)workspace;
     int* flag = (int*)ws;
     int* expo = (int*)(ws + pl.expo);
@@ -453,16 +440,17 @@ extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, in
     QMLL_REQUIRE(attr == hipSuccess, QMLL_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(attr));
     for (int m0 = 0; m0 < M; m0 += pl.rows) {
         const int m = M - m0 < pl.rows ? M - m0 : pl.rows;
-        const double* z = Z + (size_t)m0 * F;
+        const double* z = Z + (size_t)m0 * ldz;
         const int nparts = (m + NORM_ROWS - 1) / NORM_ROWS, nk = (m + 127) / 128 * 2;
         const size_t plane = (size_t)nk * 64 * pl.Fp;
-        hipLaunchKernelGGL(column_norms_kernel, dim3((F + 255) / 256, nparts), dim3(256), 0, stream, z, y ? y + m0 : nullptr, m, F,
-                           parts, yparts, flag);
+        hipLaunchKernelGGL(column_norms_kernel, dim3((F + 255) / 256, nparts), dim3(256), 0, stream, z, ldz, y ? y + m0 : nullptr, m,
+                           F, parts, yparts, flag);
         QMLL_CHECK_LAUNCH(who);
         hipLaunchKernelGGL(column_scales_kernel, dim3(pl.Fp / 256), dim3(256), 0, stream, parts, yparts, nparts, F, pl.Fp, scale,
                            expo, ZTy, flag);
         QMLL_CHECK_LAUNCH(who);
-        hipLaunchKernelGGL(residues_kernel, dim3(pl.Fp / 64, nk), dim3(256), 0, stream, z, m, F, pl.Fp, scale, flag, planes, plane);
+        hipLaunchKernelGGL(residues_kernel, dim3(pl.Fp / 64, nk), dim3(256), 0, stream, z, ldz, m, F, pl.Fp, scale, flag, planes,
+                           plane);
         QMLL_CHECK_LAUNCH(who);
         for (int t0 = 0; t0 < pl.tiles; t0 += pl.range) {
             const int nr = pl.tiles - t0 < pl.range ? pl.tiles - t0 : pl.range;
@@ -471,11 +459,34 @@ extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, in
                                pl.Fp, nk, pl.pieces, pl.nt, t0, nr, flag, results);
             QMLL_CHECK_LAUNCH(who);
             hipLaunchKernelGGL(reconstruct_kernel, dim3((unsigned)nr * 16), dim3(256), 0, stream, results, pl.pieces, pl.nt, t0, nr, F,
-                               expo, flag, ZTZ);
+                               expo, flag, sign, C, ldc);
             QMLL_CHECK_LAUNCH(who);
         }
-        const int rc = qmll_internal_gram_if(z, m, F, ZTZ, flag, stream);
+        const int rc = qmll_internal_gram_if(z, ldz, m, F, C, ldc, sign, flag, who, stream);
         if (rc != QMLL_OK) return rc;
     }
     return QMLL_OK;
+}
+
+size_t qmll_internal_modular_bytes(int M, int F) { return modular_plan(M, F).bytes; }
+
+extern "C" size_t qmll_gram_modular_workspace_bytes(int M, int F) {
+    // Below MODULAR_MIN_ROWS rows the bytes out of the products and their reconstruction, 2.3 ms at 16384 features whatever
+    // the rows, outweigh the sums: 0.87 (fp64 kernel) against 2.3 ms for 128 rows, 1.60 / 2.64 for 320, 3.64 / 3.20 for
+    // 800, 8.6 / 4.7 for 2000; at 1024 features 0.042 / 0.055, 0.086 / 0.082, 0.25 / 0.10 and 0.41 / 0.12 ms.
+    if (M < MODULAR_MIN_ROWS || F <= 0) return 0;
+    return modular_plan(M, F).bytes;
+}
+
+extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
+                                     size_t workspace_bytes, qmll_stream_t stream) {
+    const char* who = "qmll_gram_modular_f64";
+    QMLL_REQUIRE(M >= 0 && F > 0, QMLL_ERR_INVALID, "%s: bad size M=%d F=%d", who, M, F);
+    if (M == 0) return QMLL_OK;
+    QMLL_REQUIRE(Z && ZTZ && workspace, QMLL_ERR_INVALID, "%s: null pointer", who);
+    QMLL_REQUIRE((y == nullptr) == (ZTy == nullptr), QMLL_ERR_INVALID, "%s: y and ZTy must both be given or both be NULL", who);
+    const size_t need = modular_plan(M, F).bytes;
+    QMLL_REQUIRE(workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, QMLL_ERR_INVALID,
+                 "%s: needs %zu bytes of workspace, 16-byte aligned", who, need);
+    return qmll_internal_modular_syrk(Z, F, y, M, F, ZTZ, F, 1.0, ZTy, workspace, who, (hipStream_t)stream);
 }

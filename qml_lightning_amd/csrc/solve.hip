@@ -15,7 +15,9 @@
 // For whole tiles (F a multiple of 128) a panel and the trailing update of the panel before it are ONE
 // launch (panel_kernel below); any other F takes a launch per step with the tile kernel of gram.hip.
 // Only elements on or above the diagonal are read; below the diagonal only the lower halves of
-// the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.
+// the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.  Large matrices take the update of what is below a slab of
+// 4096 rows in one piece from the int8 matrix cores (slab_end below).
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -26,6 +28,11 @@
 // of n columns with row stride ldz
 int qmll_internal_syrk_upper(const double* Z, int M, int n, long long ldz, double* C, long long ldc, double sign,
                              hipStream_t stream);
+// gram_modular.hip: C[F,F] (row stride ldc, tiles on or above the diagonal) += sign Z^T Z, and the workspace it takes
+int qmll_internal_modular_syrk(const double* Z, long long ldz, const double* y, int M, int F, double* C, long long ldc, double sign,
+                               double* ZTy, void* workspace, const char* who, hipStream_t stream);
+size_t qmll_internal_modular_bytes(int M, int F);
+
 // gram.hip: C[ra,n] = or += sign * Za^T Zb, Za = M x ra (row stride lda), Zb = M x n (row stride ldb)
 int qmll_internal_gemm_tn(const double* Za, long long lda, int ra, const double* Zb, long long ldb, int n, int M,
                           double* C, long long ldc, double sign, int overwrite, hipStream_t stream);
@@ -353,7 +360,7 @@ constexpr int P_UN = P_CPT / 2;         // 16-byte units per thread
 constexpr unsigned FLAG_DONE = 1u, FLAG_FAILED = 0x80000000u;   // (a counter never gets near the second)
 constexpr int PBLK = OB / NB;                        // blocks per panel
 constexpr int FLAGS_PER_PANEL = PBLK + PBLK * PBLK;  // "block l factored": [l]; "strip (l, b) done": [PBLK + l PBLK + b]
-constexpr int SPLIT_HEADS_BELOW = 48;       // trailing tiles per edge
+constexpr int SPLIT_HEADS_BELOW = 48 * 49 / 2;       // trailing tiles
 constexpr unsigned SPIN_LIMIT = 1u << 21;   // polls of about a microsecond each before a wait gives up
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
@@ -475,7 +482,7 @@ __device__ __forceinline__ unsigned await(unsigned* flag, unsigned target, unsig
 // then nown_pad ids for the column owners, then the tiles of the trailing matrix below this panel, nt per edge
 // (0: none).  flags: FLAGS_PER_PANEL words, then one counter per column (head tiles done), all zero.
 __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, int F, int R0, int P0, int nblk,
-                                                      int nhead_pad, int nown, int nown_pad, int nt, TileMap tm,
+                                                      int nhead_pad, int nown, int nown_pad, int ntr, int nt, TileMap tm,
                                                       double* invs, int* info, unsigned* flags, unsigned spin_limit) {
     // the tile product and the factorisation never run at the same time: one piece of LDS for both, which
     // is what lets two workgroups share a CU (2 x 74 KB)
@@ -510,7 +517,8 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
     bid -= nhead_pad;
     if (bid >= nown_pad) {                                   // a tile of the trailing matrix
         int ti, tj;
-        tile_of_block<true>((unsigned)(bid - nown_pad), nt, nt, tm, ti, tj);
+        if (ntr == nt) tile_of_block<true>((unsigned)(bid - nown_pad), nt, nt, tm, ti, tj);
+        else tile_of_block<false>((unsigned)(bid - nown_pad), ntr, nt, tm, ti, tj);
         if (ti < 0 || ti > tj) return;
         const int Q = P0 + nblk * NB;
         const int i0 = Q + ti * NB, c0 = Q + tj * NB;
@@ -711,11 +719,22 @@ __global__ __launch_bounds__(256) void fill_words64_kernel(unsigned long long* p
 // exchange copy of x of the backward solve (whole blocks each), and the flags of the panel launches (per panel:
 // FLAGS_PER_PANEL + one counter per block column)
 namespace {
+// Slabs of 4096 rows while at least 8192 rows are left below: the panels of a slab update the slab's own rows only, and what
+// is below the slab takes one update 4096 deep from the int8 matrix cores (gram_modular.hip), which at that depth run at
+// more than twice the fp64 rate (4.2 ms for the 12288 columns below the first slab of 16384, 9.6 ms as part of the panels'
+// launches).  The last 8192 and more rows keep their fp64 updates, which hide behind the chain of the panels.
+// 16384 features, factorisation and solves: 34.1 ms without slabs, 30.7 / 28.9 / 28.5 / 29.6 with 2048 / 3072 / 4096 / 6144 rows;
+// 12288 features: 18.3 and 17.5 / 17.0 / 16.9 / 17.2.
+constexpr int SLAB = 4096, SLAB_REST = 8192;
+// end of the slab of rows that starts at s0
+int slab_end(int s0, int F) { return F - s0 - SLAB >= SLAB_REST ? s0 + SLAB : F; }
+
 struct Workspace {
     double* invs;
     double* z;
     double* xs;
     unsigned* panel_flags;
+    void* slab;          // workspace of the slabs' updates
     size_t nblk, npanel, bytes;
 };
 Workspace workspace_layout(void* base, int F) {
@@ -728,6 +747,16 @@ Workspace workspace_layout(void* base, int F) {
     w.panel_flags = reinterpret_cast<unsigned*>(w.xs + w.nblk * NB);
     w.bytes = (w.nblk * 2 * NB * NB + 2 * w.nblk * NB) * sizeof(double) +
               w.npanel * (FLAGS_PER_PANEL + w.nblk) * sizeof(unsigned) + 256;
+    if (F % NB == 0 && slab_end(0, F) < F) {
+        w.bytes = (w.bytes + 1023) / 1024 * 1024;
+        w.slab = reinterpret_cast<char*>(base) + w.bytes;
+        size_t most = 0;
+        for (int s0 = 0, s1 = slab_end(0, F); s1 < F; s0 = s1, s1 = slab_end(s0, F))
+            most = std::max(most, qmll_internal_modular_bytes(s1 - s0, F - s1));
+        w.bytes += most;
+    } else {
+        w.slab = nullptr;
+    }
     return w;
 }
 }  // namespace
@@ -780,28 +809,39 @@ extern "C" int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace
         const int nflags = (F + OB - 1) / OB * per_panel;
         hipLaunchKernelGGL(zero_words_kernel, dim3((nflags + 255) / 256), dim3(256), 0, stream, flags, nflags);
         QMLL_CHECK_LAUNCH("qmll_cholesky_f64");
+        int S0 = 0, S1 = slab_end(0, F);                      // rows of this slab
         for (int P0 = 0; P0 < F; P0 += OB) {
             const int pend = P0 + OB < F ? P0 + OB : F;       // this panel: rows [P0, pend)
-            const int R0 = P0 >= OB ? P0 - OB : 0;            // the panel before it
+            if (P0 == S1) {                                   // the slab before is done: its update of everything below it
+                const int rc = qmll_internal_modular_syrk(A + (size_t)S0 * ld + S1, ld, nullptr, S1 - S0, F - S1,
+                                                          A + (size_t)S1 * ld + S1, ld, -1.0, nullptr, ws.slab, "qmll_cholesky_f64",
+                                                          stream);
+                if (rc != QMLL_OK) return rc;
+                S0 = S1;
+                S1 = slab_end(S0, F);
+            }
+            const int R0 = P0 > S0 ? P0 - OB : P0;            // the panel before it in the slab
             const int nblk = (pend - P0) / NB;
             const int ncol = (F - P0) / NB;                   // columns of tiles from the panel's first to the last
             const int nt = P0 > R0 ? (F - pend) / NB : 0;
+            const int ntr = P0 > R0 ? (S1 - pend) / NB : 0;   // rows of tiles below the panel that take its predecessor's update
+            const int ntrail = ntr * nt - ntr * (ntr - 1) / 2;
             const int nown = ncol;
             // The head tiles (this panel's rows of the update of the panel before) go to workgroups of their own
             // once the trailing matrix is small, where a launch lasts as long as its slowest owner: four head tiles
             // and ten strip / update products in a row, 540 us, against a chain of four factorisations of 390.
             // While the trailing tiles keep the chip busy for longer than that, the owners take their head tiles
             // themselves and no slot waits for another.
-            const bool split_heads = P0 > R0 && nt <= SPLIT_HEADS_BELOW;
+            const bool split_heads = P0 > R0 && ntrail <= SPLIT_HEADS_BELOW;
             const int nown_pad = (nown + NXCD - 1) / NXCD * NXCD;
             const int nhead = split_heads ? nblk * (nblk + 1) / 2 + (ncol - nblk) * nblk : 0;
             const int nhead_pad = (nhead + NXCD - 1) / NXCD * NXCD;
             long long per_xcd = 0;
-            TileMap tm = gram_tile_map(nt > 0 ? nt : 1, nt > 0 ? nt : 1, true, per_xcd);
-            const long long grid = (long long)nhead_pad + nown_pad + (nt > 0 ? per_xcd * NXCD : 0);
+            TileMap tm = gram_tile_map(ntr > 0 ? ntr : 1, nt > 0 ? nt : 1, ntr == nt, per_xcd);
+            const long long grid = (long long)nhead_pad + nown_pad + (ntr > 0 ? per_xcd * NXCD : 0);
             QMLL_REQUIRE(grid < 2147483647LL, QMLL_ERR_INVALID, "qmll_cholesky_f64: too many tiles");
             hipLaunchKernelGGL(panel_kernel, dim3((unsigned)grid), dim3(PT), 0, stream, A, ld, F, R0, P0, nblk, nhead_pad,
-                               nown, nown_pad, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
+                               nown, nown_pad, ntr, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
             QMLL_CHECK_LAUNCH("qmll_cholesky_f64");
         }
         return QMLL_OK;

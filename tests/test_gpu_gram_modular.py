@@ -129,3 +129,30 @@ def test_modular_gram_in_a_graph_is_the_eager_result():
         ops.gram(Z, None, ref, None)
         torch.cuda.synchronize()
         assert torch.equal(C, ref), seed
+
+
+def test_factorisation_in_slabs():
+    """12288 features is the smallest matrix whose first 4096 rows are a slab of their own: the residual of the solve within the
+    backward error of a factorisation of that size, a pivot that is not positive and a NaN below the slab reported."""
+    from qml_lightning_amd import ops
+    F = 12288
+    g = torch.Generator(device=dev()).manual_seed(9)
+    Z = torch.randn(F + 300, F, dtype=torch.float64, device=dev(), generator=g) * 0.01
+    Z *= torch.exp(torch.randn(F, dtype=torch.float64, device=dev(), generator=g))
+    A = torch.zeros(F, F, dtype=torch.float64, device=dev())
+    ops.gram(Z, None, A, None)
+    del Z
+    A.diagonal().add_(1e-3)
+    b = torch.randn(F, 1, dtype=torch.float64, device=dev(), generator=g)
+    x, info = ops.cholesky_solve_spd(A, b)
+    assert int(info.item()) == 0
+    # |A x - b| <= c n eps |A| |x| (a backward stable solve; c = 1 is far from what a random matrix shows)
+    assert float((A @ x - b).norm()) <= F * 2.0 ** -53 * float(A.norm()) * float(x.norm())
+    for row, col, value, expect in ((10000, 10000, -1.0, 10001), (6000, 10500, float("nan"), None)):
+        kept = A[row, col].item()
+        A[row, col] = value
+        A[col, row] = value
+        _, info = ops.cholesky_solve_spd(A, b)
+        assert int(info.item()) == expect if expect else int(info.item()) > 0
+        A[row, col] = kept
+        A[col, row] = kept
