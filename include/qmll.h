@@ -67,6 +67,14 @@ int qmll_num_neighbours(const float* X, const int* natoms, const float* cell, co
 int qmll_neighbour_list(const float* X, const int* natoms, const float* cell, const float* inv_cell,
                         int B, int n, int max_neighbours, float rcut, int* nlist, qmll_stream_t stream);
 
+/* The padded arrays of a batch (qml_lightning/models/kernel.py:630-695) from the atoms of its molecules one behind the other:
+ * x f32 [total,3], q f32 [total], forces f64 [total,3] or NULL, counts and starts i32 [B] (a molecule's atoms and its first one)
+ * -> coordinates f32 [B,n,3], charges f32 [B,n], padded_forces f64 [B,n,3] (with forces), atom_ids and mol_ids i32 [total]
+ * (index within the molecule, index of the molecule).  n is at least the largest count. */
+int qmll_format_batch(const float* x, const float* q, const double* forces, const int* counts, const int* starts, int B, int n,
+                      float* coordinates, float* charges, double* padded_forces, int* atom_ids, int* mol_ids,
+                      qmll_stream_t stream);
+
 /* Replaces fchl_gpu.get_element_types_gpu (qml_lightning/cuda/fchl_cuda.cpp:36-62, kernel
  * fchl_cuda_kernel.cu:1716-1742).  Z f32 [B,n] charges, species f32 [nspecies] ->
  * types i32 [B,n]: index of int(charge) in species, -1 if absent, 0 for padded slots. */

@@ -43,6 +43,7 @@ PROTOTYPES = {
     "qmll_num_neighbours": [P, P, P, P, c_int, c_int, c_float, P, P],
     "qmll_neighbour_list": [P, P, P, P, c_int, c_int, c_int, c_float, P, P],
     "qmll_element_types": [P, P, P, c_int, c_int, c_int, P, P],
+    "qmll_format_batch": [P, P, P, P, P, c_int, c_int, P, P, P, P, P, P],
     "qmll_fchl19_forward": _FCHL_COMMON + [P, P],
     "qmll_fchl19_vjp": _FCHL_COMMON + [P, P, P],
     "qmll_fchl19_vjp_scaled": _FCHL_COMMON + [P, c_float, P, P],
@@ -127,6 +128,27 @@ def lib():
             fn.restype = _RESTYPES.get(name, c_int)
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """libqmll_host.so, called with the interpreter lock held (loaded once).  RuntimeError when it has not been built."""
+    global _host
+    if _host is None:
+        path = os.path.join(HERE, "libqmll_host.so")
+        if not os.path.exists(path):
+            raise RuntimeError("qml_lightning_amd: %s not found -- build it with `python -m qml_lightning_amd.build`" % path)
+        handle = ctypes.PyDLL(path)
+        O = ctypes.py_object
+        handle.qmll_lists_init.argtypes = []
+        handle.qmll_lists_measure.argtypes = [O, O, O, c_longlong, P]
+        handle.qmll_lists_measure.restype = c_longlong
+        handle.qmll_lists_pack.argtypes = [O, O, O, c_longlong, P, c_longlong, P, P, P, P]
+        handle.qmll_lists_init()
+        _host = handle
+    return _host
 
 
 def check(rc, what=""):

@@ -1,5 +1,6 @@
-"""Build, in-tree: libqmll.so (the C-ABI HIP library, hipcc for gfx950) and
-libqmll_torch.so (the TORCH_LIBRARY operator registrations over that C ABI, host C++ only).
+"""Build, in-tree: libqmll.so (the C-ABI HIP library, hipcc for gfx950), libqmll_torch.so (the
+TORCH_LIBRARY operator registrations over that C ABI, host C++ only) and libqmll_host.so (lists of
+numpy arrays into upload buffers, host C++ only).
 
     python -m qml_lightning_amd.build        # or: from qml_lightning_amd.build import build; build()
 """
@@ -11,6 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqmll.so")
 TORCH_LIB = os.path.join(HERE, "libqmll_torch.so")
+HOST_LIB = os.path.join(HERE, "libqmll_host.so")
 SOURCES = ["qmll_core.cpp", "neighbours.hip", "fchl19.hip", "sorf.hip", "sorf_matrix.hip", "project.hip", "rff.hip", "gram.hip", "gram_modular.hip", "solve.hip", "probe.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
@@ -38,6 +40,7 @@ def build(verbose=True, jobs=8):
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     build_torch_ops(verbose)
+    build_host_lists(verbose)
     build_host_check(verbose)
     return LIB
 
@@ -58,6 +61,19 @@ def build_torch_ops(verbose=True):
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     return TORCH_LIB
+
+
+def build_host_lists(verbose=True):
+    """libqmll_host.so: the walk over Python lists of numpy arrays (CPython and numpy C interfaces, no GPU code)."""
+    import sysconfig
+
+    import numpy
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"],
+           "-I" + numpy.get_include(), os.path.join(CSRC, "host_lists.cpp"), "-o", HOST_LIB]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return HOST_LIB
 
 
 def _drain(procs):

@@ -565,8 +565,7 @@ class HadamardFeaturesModel(BaseKernel, torch.nn.Module):
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
         start.record()
-        predict_energies = torch.zeros(len(X), device=self.device, dtype=torch.float32)
-        predict_forces = torch.zeros(len(X), max_natoms, 3, device=self.device, dtype=torch.float32)
+        predict_energies = predict_forces = None
         step = self._fused_batch(max_natoms) if self.fused else self.nbatch_test
         for i in self._progress(range(0, len(X), step), print_info):
             sl = slice(i, i + step)
@@ -584,13 +583,21 @@ class HadamardFeaturesModel(BaseKernel, torch.nn.Module):
                 result = self.predict_opt(data['coordinates'], data['charges'], data['atomIDs'], data['molIDs'],
                                           data['natom_counts'], data['cells'], data['inv_cells'], forces=forces,
                                           print_info=False, profiler=False)
+            energies_of, forces_of = (result[0].detach(), result[1]) if forces else (result.detach(), None)
+            if len(X) <= step and energies_of.dtype == torch.float32 and (
+                    not forces or (forces_of.dtype == torch.float32 and forces_of.shape == (len(X), max_natoms, 3))):
+                predict_energies, predict_forces = energies_of, forces_of       # one batch: its results are the answer
+                break
+            if predict_energies is None:
+                predict_energies = torch.zeros(len(X), device=self.device, dtype=torch.float32)
+                predict_forces = torch.zeros(len(X), max_natoms, 3, device=self.device, dtype=torch.float32)
+            predict_energies[sl] = energies_of
             if forces:
-                predict_energies[sl] = result[0].detach()
-                n = result[1].shape[1]
                 # padded slots carry exactly zero force, so the padded block can be copied whole
-                predict_forces[sl, :n] = result[1]
-            else:
-                predict_energies[sl] = result.detach()
+                predict_forces[sl, :forces_of.shape[1]] = forces_of
+        if predict_energies is None:                                            # no molecules
+            predict_energies = torch.zeros(0, device=self.device, dtype=torch.float32)
+            predict_forces = torch.zeros(0, max_natoms, 3, device=self.device, dtype=torch.float32)
         end.record()
         torch.cuda.synchronize()
         if print_info:

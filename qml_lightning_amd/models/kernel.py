@@ -12,7 +12,7 @@ no `empty_cache()` between batches.
 import numpy as np
 import torch
 
-from .. import ops
+from .. import _lib, ops
 from ..cuda.utils_gpu import matmul_and_reduce
 
 
@@ -709,6 +709,58 @@ class BaseKernel():
             data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
         return data
 
+    def _format_lists_on_device(self, X, Q, E, F, cells, inv_cells):
+        """format_data for lists of plain numpy arrays: the arrays are packed one behind the other into one page-locked buffer
+        (csrc/host_lists.cpp), which is uploaded in one copy; padding and indices are made on the device.  None for lists
+        of anything else."""
+        host, B = _lib.host(), len(X)
+        counts = np.empty(B, dtype=np.int32)
+        total = host.qmll_lists_measure(X, Q, F, B, counts.ctypes.data)
+        if total <= 0:
+            return None
+        dev, n = self.device, int(counts.max())
+        parts, nbytes = {}, 0
+        for name, size in (('energies', 8 * B if E is not None else 0), ('forces', 24 * total if F is not None else 0),
+                           ('x', 12 * total), ('q', 4 * total), ('counts', 4 * B), ('starts', 4 * B)):
+            parts[name] = slice(nbytes, nbytes + size)
+            nbytes += size
+        stage = torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
+        staged = stage.numpy()
+
+        def at(name):
+            return stage.data_ptr() + parts[name].start
+
+        if host.qmll_lists_pack(X, Q, F, B, counts.ctypes.data, total, at('x'), at('q'), at('forces'), at('starts')) != 0:
+            return None
+        staged[parts['counts']].view(np.int32)[:] = counts
+        charges_of = staged[parts['q']].view(np.float32)
+        data = {}
+        if E is not None or F is not None:
+            data['element_counts'] = self._element_counts(charges_of)
+        if E is not None:
+            energies = np.array(E, dtype=np.float64).reshape(B).copy()
+            if self.convert_hartree2kcal():
+                energies *= self.hartree2kcalmol
+            if self.subtract_self_energies():
+                se = self.self_energy.numpy()
+                energies -= np.bincount(np.repeat(np.arange(B), counts), weights=se[charges_of.astype(np.int64)], minlength=B)
+            staged[parts['energies']].view(np.float64)[:] = energies
+        if F is not None:
+            if self.convert_hartree2kcal():
+                forces_of = staged[parts['forces']].view(np.float64)
+                forces_of *= self.hartree2kcalmol
+            data['host_counts'] = counts
+        there = stage.to(dev, non_blocking=True)
+        data['energies'] = there[parts['energies']].view(torch.float64) if E is not None else None
+        data.update(zip(('coordinates', 'charges', 'forces', 'atomIDs', 'molIDs', 'natom_counts'),
+                        ops.format_batch(there, parts, B, n, total, F is not None)))
+        data['cells'] = torch.empty((0, 3, 3), device=dev)
+        data['inv_cells'] = torch.empty((0, 3, 3), device=dev)
+        if cells is not None:
+            data['cells'] = torch.from_numpy(np.asarray(cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
+            data['inv_cells'] = torch.from_numpy(np.asarray(inv_cells, dtype=np.float32).reshape(B, 3, 3)).to(dev)
+        return data
+
     def _element_counts(self, flat_charges):
         """{element: number of atoms} of a batch from the host copy of its charges (one bincount)."""
         q = np.asarray(flat_charges).astype(np.int64, copy=False)
@@ -742,6 +794,10 @@ class BaseKernel():
         zbatch = len(X)
         if isinstance(X, np.ndarray) and X.ndim == 3 and isinstance(Q, np.ndarray) and Q.ndim == 2:
             return self._format_padded_arrays(X, Q, E, F, cells, inv_cells)
+        if dev.type == 'cuda':
+            data = self._format_lists_on_device(X, Q, E, F, cells, inv_cells)
+            if data is not None:
+                return data
         counts = np.fromiter(map(len, X), dtype=np.int32, count=zbatch)
         n = int(counts.max()) if zbatch else 0
         if zbatch and n > 0 and int(counts.min()) == n:

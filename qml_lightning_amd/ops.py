@@ -825,6 +825,26 @@ def cholesky_solve_spd(A, b, overwrite_a=False):
     return x, info
 
 
+def format_batch(packed, parts, B, n, total, with_forces):
+    """The padded tensors of a batch whose atoms lie one behind the other in the device buffer `packed` (uint8): `parts` says where
+    x [total,3] and q [total] (float32), forces [total,3] (float64), counts and starts [B] (int32) are.
+    -> coordinates [B,n,3], charges [B,n], forces [B,n,3] or None, atomIDs [total], molIDs [total], natom_counts [B]."""
+    dev, base = packed.device, _ptr(packed).value
+
+    def at(name):
+        return base + parts[name].start
+
+    coordinates = torch.empty((B, n, 3), dtype=torch.float32, device=dev)
+    charges = torch.empty((B, n), dtype=torch.float32, device=dev)
+    forces = torch.empty((B, n, 3), dtype=torch.float64, device=dev) if with_forces else None
+    atom_ids = torch.empty(total, dtype=torch.int32, device=dev)
+    mol_ids = torch.empty(total, dtype=torch.int32, device=dev)
+    check(_lib.lib().qmll_format_batch(at('x'), at('q'), at('forces') if with_forces else None, at('counts'), at('starts'), B, n,
+                                       _ptr(coordinates), _ptr(charges), _ptr(forces), _ptr(atom_ids), _ptr(mol_ids), _stream()),
+          "qmll_format_batch")
+    return coordinates, charges, forces, atom_ids, mol_ids, packed[parts['counts']].view(torch.int32)
+
+
 def gram_mirror(ZTZ):
     """Copy the upper triangle of ZTZ onto the lower one (after `gram(..., mirror=False)` calls)."""
     if ZTZ.dtype != torch.float64 or not ZTZ.is_contiguous() or ZTZ.shape[0] != ZTZ.shape[1]:

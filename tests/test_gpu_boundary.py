@@ -304,3 +304,33 @@ print("python-ops-ok")
     env = dict(os.environ, QML_LIGHTNING_AMD_PY_OPS="1")
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=600, env=env)
     assert res.returncode == 0 and "python-ops-ok" in res.stdout, (res.stdout[-1500:], res.stderr[-3000:])
+
+
+@pytest.mark.parametrize("form", ["plain", "tuples", "float32", "mixed floats", "large charges", "strided", "nested lists"])
+@pytest.mark.parametrize("targets", [False, True])
+def test_lists_formatted_on_the_device_equal_the_host_route(form, targets):
+    """format_data of lists of per-molecule arrays: packed and padded on the device against numpy's concatenations on the host."""
+    from qml_lightning_amd.models.hadamard_features import HadamardFeaturesModel
+    from qml_lightning_amd.representations.FCHL import FCHLCuda
+    from tests.test_host_logic import _list_forms
+    targets = targets and form != "large charges"        # (no element has such a charge)
+    elements = np.arange(1, 9)
+    m = HadamardFeaturesModel(rep=FCHLCuda(species=elements), elements=elements, npcas=64, nstacks=4)
+    X, Q, F = [(x, q, f) for name, x, q, f, _ in _list_forms() if name == form][0]
+    kw = {}
+    if targets:
+        rng = np.random.default_rng(1)
+        kw = dict(E=rng.normal(size=len(X)).tolist(), F=[rng.normal(size=(len(x), 3)) for x in X] if F is None else F)
+        m.set_convert_hartree2kcal(True)
+        m.self_energy = torch.tensor(rng.normal(size=m.element2index.shape[0]))
+        m.set_subtract_self_energies(True)
+    cells = np.broadcast_to(np.eye(3) * 20.0, (len(X), 3, 3)).copy()
+    got = m.format_data(X, Q, cells=cells, inv_cells=np.linalg.inv(cells), **kw)
+    m._format_lists_on_device = lambda *a: None
+    want = m.format_data(X, Q, cells=cells, inv_cells=np.linalg.inv(cells), **kw)
+    assert set(got) == set(want)
+    for key, w in want.items():
+        if torch.is_tensor(w):
+            assert got[key].dtype == w.dtype and got[key].device == w.device and torch.equal(got[key], w), key
+        else:
+            assert np.array_equal(got[key], w) if key == "host_counts" else got[key] == w, key

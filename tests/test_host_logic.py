@@ -224,6 +224,59 @@ def test_gram_tile_map_meets_every_tile_once_and_balances_the_xcds(tmp_path):
     assert out.stdout.startswith("ok")
 
 
+def _list_forms():
+    """(name, X, Q, F, accepted): lists of per-molecule arrays in the forms a caller may hand over."""
+    rng = np.random.default_rng(8)
+    ks = [3, 1, 7, 0, 5]
+    X = [rng.normal(size=(k, 3)) for k in ks]
+    Q = [rng.integers(1, 9, k) for k in ks]
+    F = [rng.normal(size=(k, 3)) for k in ks]
+    f32 = [x.astype(np.float32) for x in X]
+    yield "plain", X, Q, F, True
+    yield "tuples", tuple(X), tuple(Q), tuple(F), True
+    yield "float32", f32, [q.astype(np.float32) for q in Q], [f.astype(np.float32) for f in F], True
+    yield "mixed floats", [X[0], f32[1], X[2], f32[3], X[4]], [q.astype(np.int32) for q in Q], None, True
+    yield "large charges", X, [q + 2 ** 40 for q in Q], None, True
+    yield "small integers", X, [q.astype(np.uint8) for q in Q], None, True
+    yield "mixed charges", X, [Q[0].astype(np.float64)] + Q[1:], None, False
+    yield "nested lists", [x.tolist() for x in X], [q.tolist() for q in Q], None, False
+    yield "strided", [np.asfortranarray(x) for x in X], Q, None, False
+    yield "every second", [np.repeat(x, 2, 0)[::2] for x in X], Q, None, False
+    yield "flat rows", [x.reshape(-1) for x in X], Q, None, False
+    yield "byte order", [x.astype(">f8") for x in X], Q, None, False
+    yield "integers", [np.rint(x).astype(np.int64) for x in X], Q, None, False
+    yield "fewer charges", X, Q[:2] + [Q[2][:-1]] + Q[3:], None, False
+    yield "fewer forces", X, Q, F[:4] + [F[4][:-1]], False
+    yield "other lengths", X, Q[:4], None, False
+    yield "object array", np.array(X, dtype=object), Q, None, False
+
+
+@pytest.mark.parametrize("form", list(_list_forms()), ids=lambda f: f[0])
+def test_lists_are_packed_as_numpy_concatenates_them(form):
+    from qml_lightning_amd import _lib
+    _, X, Q, F, accepted = form
+    host, B = _lib.host(), len(X)
+    counts = np.empty(B, dtype=np.int32)
+    total = host.qmll_lists_measure(X, Q, F, B, counts.ctypes.data)
+    assert (total >= 0) == accepted
+    if not accepted:
+        return
+    assert total == sum(map(len, X)) and counts.tolist() == [len(x) for x in X]
+    x, q = np.empty((total, 3), np.float32), np.empty(total, np.float32)
+    f, starts = np.empty((total, 3)), np.empty(B, np.int32)
+
+    def pack(Xs, Qs):
+        return host.qmll_lists_pack(Xs, Qs, F, B, counts.ctypes.data, total, x.ctypes.data, q.ctypes.data, f.ctypes.data,
+                                    starts.ctypes.data)
+    assert pack(X, Q) == 0
+    assert np.array_equal(x, np.concatenate(X).astype(np.float32)) and np.array_equal(q, np.concatenate(Q).astype(np.float32))
+    assert F is None or np.array_equal(f, np.concatenate(F).astype(np.float64))
+    assert np.array_equal(starts, np.cumsum(counts) - counts)
+    # the lists changed after they were measured
+    longer = [np.concatenate((X[0], X[0]))] + list(X[1:])
+    assert pack(longer, [np.concatenate((Q[0], Q[0]))] + list(Q[1:])) == -1
+
+
 def test_modular_gram_plan_covers_every_tile_and_row(tmp_path):
     """tests/cpp/check_gram_modular.cpp: tile order, row passes, tile ranges and workspace of the modular Gram product."""
     import shutil
