@@ -161,6 +161,27 @@ __device__ __forceinline__ void split_f16(float v, _Float16& hi, _Float16& lo) {
     lo = (_Float16)(v - (float)hi);
 }
 
+// v minus one half of a packed pair, in one instruction (written out, the compiler converts and subtracts: two)
+__device__ __forceinline__ float minus_low(float v, half2_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    return r;
+}
+__device__ __forceinline__ float minus_high(float v, half2_t h) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    return r;
+}
+
+// two values split as split_f16 does it, in four instructions: two conversions of pairs and two subtractions
+__device__ __forceinline__ void split_pair(float v0, float v1, half2_t& hi, half2_t& lo) {
+    typedef float pair_t __attribute__((ext_vector_type(2)));
+    asm("" : "+v"(v0));        // the values as they were rounded to fp32: see split_f16
+    asm("" : "+v"(v1));
+    hi = __builtin_convertvector((pair_t){v0, v1}, half2_t);
+    lo = __builtin_convertvector((pair_t){minus_low(v0, hi), minus_high(v1, hi)}, half2_t);
+}
+
 // |v| for finite v, 0 for an infinity or a NaN: the operand scales below are taken from the largest
 // FINITE entry, so that a non-finite entry spoils its own row only (its parts become Inf / NaN) and
 // not the rows that share its scale (which an infinite maximum would scale down to nothing)

@@ -284,16 +284,22 @@ void launch_rff_rows(const RffElements& E, const int* row_offsets, int max_rows,
 // = feature, column = atom) are exactly the B operand the second one needs (contraction
 // index = feature): P never leaves the registers.  x^T (B operand of the first product)
 // stays in registers for the whole kernel, GX^T in accumulators.
-typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
 
 constexpr int RE_T = 256;        // threads: 4 wavefronts x 32 atoms
 constexpr int RE_M = 128;        // atoms per workgroup
 constexpr int RE_FC = 32;        // features per staged chunk (one block of 32 rows)
 
-// The products run on the half-precision matrix cores.  v_mfma_f32_32x32x16_f16 runs 13 times as fast per
-// flop as v_mfma_f32_32x32x2_f32 (40 against 64 clocks for eight times the flops), so each fp32 operand is split into two fp16 parts (hi = the value
+// The products run on the half-precision matrix cores, whose fp16 instructions do thirteen times the flops per clock of
+// v_mfma_f32_32x32x2_f32: each fp32 operand is split into two fp16 parts (hi = the value
 // rounded to fp16, lo = the rounded rest: 22 bits together) and a product becomes three matrix
 // instructions, hi.hi + hi.lo + lo.hi, accumulated in fp32; lo.lo is below the rounding of the sum.
+// The instruction is the 16 x 16 x 32 one: on operands with all their bits in use the card's power holds a loop of
+// nothing but the 32 x 32 x 16 form to 1.62 PFLOP/s and of this one to 1.90 (2.46 and 2.48 on zeros), and here the clock
+// rises from 1.60 to 1.74 GHz.  86016 atoms, 32768 features, 128 components with the gradient: 4.35 ms with the larger form,
+// 3.80 with this one; energies only 2.35 / 2.08; 64 components, 16384 features 1.31 / 1.10 and 0.65 / 0.60.  What is left is
+// issue as much as power: beside vector work of another wavefront a matrix instruction of either form takes about ten clocks
+// of the SIMD's issue, which makes 2000 clocks per wavefront and chunk with the 1050 of the vector instructions.
 // fp16 has five exponent bits, so every operand is scaled by a power of two first (exact): x by the
 // wavefront's 2^kx (largest |x| of its 32 atoms to [2^13, 2^14)), alpha by the workgroup's 2^kp (largest
 // |alpha| norm of its feature range), every chunk of W by its own 2^kw (largest |W| of the chunk); the
@@ -303,22 +309,24 @@ constexpr int RE_FC = 32;        // features per staged chunk (one block of 32 r
 //
 // W is a constant of the model, so it is split ONCE (rff_presplit_kernel) into the very bytes the
 // predict kernel wants in LDS: per element and 32-feature chunk an image holding the chunk twice,
-// feature-major with k contiguous (A operand of the first product, rows = features) and k-major with
-// the chunk's 32 features contiguous (A operand of the second, rows = k), the features in the order in
-// which the first product's accumulator registers hold them (register r of half h: feature
-// 8(r/4) + 4h + r%4), so the split P goes straight from registers into the B operand; hi and lo parts
-// each, row padding included.  The predict kernel then moves an image into LDS with direct
+// as A operands of the first product (rows = features, 32 k per step) and of the second (rows = k, the
+// chunk's 32 features), the features in the order in which the first product's accumulators hold them
+// (lane group g: 4 g + 0..3 of either tile of 16), so the split P goes straight from registers into the
+// B operand; hi and lo parts each, every operand 1 KB in the order of the lanes.  The predict kernel then moves an image into LDS with direct
 // global-to-LDS loads (no registers, no vector instructions), the next chunk's while this one is
 // multiplied.
 template <int D>
 struct RffImage {
-    static constexpr int LD1 = D + 8;                // halves per row of the feature-major copy
-    static constexpr int LD2 = RE_FC + 8;            // halves per row of the k-major copy
-    static constexpr int W1H = 0, W1L = RE_FC * LD1, W2H = 2 * RE_FC * LD1, W2L = W2H + D * LD2;
-    static constexpr int HALVES = W2L + D * LD2;
-    static constexpr int BYTES = HALVES * 2;         // 37888 (D = 128), 19456 (D = 64): whole KiB
-    static constexpr int BLOCKS = BYTES / 1024;      // 1 KiB = one wavefront's 64 x 16-byte load
-    static_assert(BYTES % 1024 == 0, "an image is moved in 1 KiB blocks");
+    static constexpr int OP = 512;                   // halves of one operand: 64 lanes x 8
+    static constexpr int KS = D / 32, KT = D / 16;   // contraction steps of the first product, row tiles of the second
+    // first product, operand (part, feature tile, step): lane (i, g) holds W[32 step + 8 g + 0..7][16 tile + i]; second product,
+    // operand (part, row tile): W[16 tile + i][features 4 g + 0..3 and 16 + 4 g + 0..3]
+    __host__ __device__ static constexpr int w1(int part, int tile, int step) { return ((part * 2 + tile) * KS + step) * OP; }
+    __host__ __device__ static constexpr int w2(int part, int tile) { return (4 * KS + part * KT + tile) * OP; }
+    static constexpr int HALVES = (4 * KS + 2 * KT) * OP;
+    static constexpr int BYTES = HALVES * 2;         // 32768 (D = 128), 16384 (D = 64)
+    static constexpr int BLOCKS = BYTES / 1024;      // 1 KiB = one operand = one wavefront's 64 x 16-byte load
+    static_assert(BLOCKS % 4 == 0, "the same number for each of four wavefronts");
 };
 
 // One workgroup per (chunk, element): the chunk's power of two, then the image through LDS.
@@ -335,8 +343,6 @@ __global__ __launch_bounds__(RE_T) void rff_presplit_kernel(const float* __restr
     const int f0 = chunk * RE_FC;
     // thread -> features sf .. sf+3 of the rows k0 = 2 (tid / 8) + 64 p and k0 + 1
     const int sf = (tid & 7) * 4, skp = 2 * (tid >> 3);
-    // place of features sf .. sf+3 in a row of the k-major copy: f = 16 t + 8 c + 4 h' + e -> 16 t + 8 h' + 4 c + e
-    const int pos2 = (sf & 16) | ((sf & 4) << 1) | ((sf & 8) >> 1);
     float4 stage[NP][2];
     float m = 0.0f;
 #pragma unroll
@@ -350,7 +356,6 @@ __global__ __launch_bounds__(RE_T) void rff_presplit_kernel(const float* __restr
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     if (lane == 0) swmax[wave] = m;
-    for (int t = tid; t < Img::HALVES / 2; t += RE_T) reinterpret_cast<unsigned*>(img)[t] = 0u;    // row padding
     __syncthreads();
     const int kw = scale_exponent(fmaxf(fmaxf(swmax[0], swmax[1]), fmaxf(swmax[2], swmax[3])));
     const float sw = pow2i(kw);
@@ -361,6 +366,8 @@ __global__ __launch_bounds__(RE_T) void rff_presplit_kernel(const float* __restr
         const float w0[4] = {stage[p][0].x * sw, stage[p][0].y * sw, stage[p][0].z * sw, stage[p][0].w * sw};
         const float w1[4] = {stage[p][1].x * sw, stage[p][1].y * sw, stage[p][1].z * sw, stage[p][1].w * sw};
         half4_t r0h, r0l, r1h, r1l;
+        // rows k0, k0 + 1 among the 32 of a step, features sf .. sf + 3 among the 16 of a tile and among a lane's eight
+        const int at1 = ((k0 & 31) >> 3) * 128 + (k0 & 7), at2 = ((sf & 15) >> 2) * 128 + (sf >> 4) * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             _Float16 a, c;
@@ -368,13 +375,14 @@ __global__ __launch_bounds__(RE_T) void rff_presplit_kernel(const float* __restr
             r0h[e] = a; r0l[e] = c;
             split_f16(w1[e], a, c);
             r1h[e] = a; r1l[e] = c;
-            *reinterpret_cast<half2_t*>(&img[Img::W1H + (sf + e) * Img::LD1 + k0]) = (half2_t){r0h[e], r1h[e]};
-            *reinterpret_cast<half2_t*>(&img[Img::W1L + (sf + e) * Img::LD1 + k0]) = (half2_t){r0l[e], r1l[e]};
+            const int to = at1 + ((sf + e) & 15) * 8;
+            *reinterpret_cast<half2_t*>(&img[Img::w1(0, sf >> 4, k0 >> 5) + to]) = (half2_t){r0h[e], r1h[e]};
+            *reinterpret_cast<half2_t*>(&img[Img::w1(1, sf >> 4, k0 >> 5) + to]) = (half2_t){r0l[e], r1l[e]};
         }
-        *reinterpret_cast<half4_t*>(&img[Img::W2H + k0 * Img::LD2 + pos2]) = r0h;
-        *reinterpret_cast<half4_t*>(&img[Img::W2L + k0 * Img::LD2 + pos2]) = r0l;
-        *reinterpret_cast<half4_t*>(&img[Img::W2H + (k0 + 1) * Img::LD2 + pos2]) = r1h;
-        *reinterpret_cast<half4_t*>(&img[Img::W2L + (k0 + 1) * Img::LD2 + pos2]) = r1l;
+        *reinterpret_cast<half4_t*>(&img[Img::w2(0, k0 >> 4) + at2 + (k0 & 15) * 8]) = r0h;
+        *reinterpret_cast<half4_t*>(&img[Img::w2(1, k0 >> 4) + at2 + (k0 & 15) * 8]) = r0l;
+        *reinterpret_cast<half4_t*>(&img[Img::w2(0, k0 >> 4) + at2 + (k0 & 15) * 8 + 8]) = r1h;
+        *reinterpret_cast<half4_t*>(&img[Img::w2(1, k0 >> 4) + at2 + (k0 & 15) * 8 + 8]) = r1l;
     }
     __syncthreads();
     float4* dst = reinterpret_cast<float4*>(images + (size_t)(type * nchunks + chunk) * Img::HALVES);
@@ -407,15 +415,14 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
     float* __restrict__ e_slots,
     float* __restrict__ gx) {
     using Img = RffImage<D>;
-    constexpr int LD1 = Img::LD1, LD2 = Img::LD2;
-    constexpr int KS = D / 16;                // matrix instructions along k per product term
+    constexpr int KS = Img::KS, KT = Img::KT;
     // two images, this chunk's and the next one's, as two arrays of their own: the compiler then knows
     // that the loads into one do not touch what is read from the other and does not wait for them
     __shared__ __attribute__((aligned(16))) _Float16 simg0[Img::HALVES], simg1[Img::HALVES];
     __shared__ __attribute__((aligned(16))) float sba[2 * 2 * RE_FC];     // [2][2][RE_FC]: b / 2 pi, alpha norm 2^kp of the two chunks
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int i = lane & 31, h = lane >> 5;
+    const int i = lane & 15, g = lane >> 4;
     const int nchunks = F / RE_FC;
     // workgroups below `whole` take a tile's chunks all, the others a share of 1 / nparts of them
     const bool whole = (int)blockIdx.x < nwhole;
@@ -426,8 +433,7 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
     if (!find_tile(type_offsets, ne, whole ? (int)blockIdx.x : nwhole + piece / nparts, type, row0, rows)) return;
     float* part_out = parts ? parts + (size_t)piece * part_floats(D, WITH_GRAD) : nullptr;
     const float* bt = b + (size_t)type * F;
-    const int arow = 32 * wave + i;
-    const bool aok = arow < rows;
+    const int arow = 32 * wave + i;                      // this lane's atoms: arow and arow + 16
     const int fbeg = c0 * RE_FC, fend = c1 * RE_FC;
     // a scalar base and one per-lane offset: the loads then need no per-lane 64-bit addresses
     const unsigned char* img0 = reinterpret_cast<const unsigned char*>(images) + (size_t)type * nchunks * Img::BYTES;
@@ -442,37 +448,42 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
 #pragma unroll
         for (int u0 = 0; u0 < Img::BLOCKS; u0 += RE_T / 64) {
             const int u = u0 + wave_s;
-            if (u < Img::BLOCKS)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + u * 1024 + lane16),
-                                                 (__attribute__((address_space(3))) void*)(dst + u * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + u * 1024 + lane16),
+                                             (__attribute__((address_space(3))) void*)(dst + u * 1024), 16, 0, 0);
         }
     };
     dma(fbeg / RE_FC, simg0);
 
-    // x^T as the B operand of the first product: instruction j contracts k = 16 j + 8 h + (0..7)
-    half8_t xh[KS], xl[KS];
+    // x^T as the B operand of the first product: step j contracts k = 32 j + 8 g + (0..7)
+    half8_t xh[2][KS], xl[2][KS];
     float inv_sx;
     {
-        float xv[KS][8];
-        const float* xr = x + (size_t)(row0 + (aok ? arow : 0)) * D + 8 * h;
+        float xv[2][KS][8];
         float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < KS; ++j) {
-            const float4 v0 = aok ? *reinterpret_cast<const float4*>(xr + 16 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
-            const float4 v1 = aok ? *reinterpret_cast<const float4*>(xr + 16 * j + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-            xv[j][0] = v0.x; xv[j][1] = v0.y; xv[j][2] = v0.z; xv[j][3] = v0.w;
-            xv[j][4] = v1.x; xv[j][5] = v1.y; xv[j][6] = v1.z; xv[j][7] = v1.w;
+        for (int t = 0; t < 2; ++t) {
+            const bool aok = arow + 16 * t < rows;
+            const float* xr = x + (size_t)(row0 + (aok ? arow + 16 * t : 0)) * D + 8 * g;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) m = fmaxf(m, fabsf(xv[j][q]));
+            for (int j = 0; j < KS; ++j) {
+                const float4 v0 = aok ? *reinterpret_cast<const float4*>(xr + 32 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float4 v1 = aok ? *reinterpret_cast<const float4*>(xr + 32 * j + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+                xv[t][j][0] = v0.x; xv[t][j][1] = v0.y; xv[t][j][2] = v0.z; xv[t][j][3] = v0.w;
+                xv[t][j][4] = v1.x; xv[t][j][5] = v1.y; xv[t][j][6] = v1.z; xv[t][j][7] = v1.w;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) m = fmaxf(m, fabsf(xv[t][j][q]));
+            }
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
         if (__builtin_expect(not_finite(m), 0)) {        // an infinity among the rows: the largest finite entry
             m = 0.0f;
 #pragma unroll
-            for (int j = 0; j < KS; ++j)
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int q = 0; q < 8; ++q) m = fmaxf(m, finite_abs(xv[j][q]));
+                for (int j = 0; j < KS; ++j)
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) m = fmaxf(m, finite_abs(xv[t][j][q]));
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
         }
@@ -480,14 +491,16 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
         const float sx = pow2i(kx);
         inv_sx = pow2i(-kx);
 #pragma unroll
-        for (int j = 0; j < KS; ++j)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                _Float16 a, c;
-                split_f16(xv[j][q] * sx, a, c);
-                xh[j][q] = a;
-                xl[j][q] = c;
-            }
+            for (int j = 0; j < KS; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    _Float16 a, c;
+                    split_f16(xv[t][j][q] * sx, a, c);
+                    xh[t][j][q] = a;
+                    xl[t][j][q] = c;
+                }
     }
     // the workgroup's alpha scale (every wavefront finds the same value)
     float sp, inv_sp;
@@ -505,14 +518,15 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
         sba[RE_FC + tid] = alpha[fbeg + tid] * norm * sp;
     }
 
-    float16_t gacc[D / 32];
+    const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f4_t gacc[KT][2];
     if constexpr (WITH_GRAD) {
 #pragma unroll
-        for (int blk = 0; blk < D / 32; ++blk)
+        for (int k = 0; k < KT; ++k)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) gacc[blk][r] = 0.0f;
+            for (int t = 0; t < 2; ++t) gacc[k][t] = zero;
     }
-    float energy = 0.0f;
+    float energy[2] = {0.0f, 0.0f};
 
     // one chunk: `img` holds it, the next one is loaded into `other`
     auto round = [&](int f0, int par, const _Float16* img, _Float16* other) {
@@ -529,7 +543,8 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
             anext = alpha[f0 + RE_FC + tid];
         }
         if (more) dma(f0 / RE_FC + 1, other);
-        const _Float16 *sW1h = img + Img::W1H, *sW1l = img + Img::W1L, *sW2h = img + Img::W2H, *sW2l = img + Img::W2L;
+        const _Float16* mine = img + lane * 8;
+        auto operand = [&](int at) { return *reinterpret_cast<const half8_t*>(mine + at); };
         const float* sb = sba + par * 2 * RE_FC;
         const float* sa = sb + RE_FC;
         const int kw = kws[f0 / RE_FC];
@@ -537,18 +552,23 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
 
         // first product: 2^(kx + kw) S^T (32 features x 32 atoms)
         const float inv_sxw = inv_sx * inv_sw;
-        float16_t sacc;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sacc[r] = 0.0f;
+        f4_t sacc[2][2];                                 // [feature tile][atom tile]
 #pragma unroll
         for (int j = 0; j < KS; ++j) {
-            const half8_t ah = *reinterpret_cast<const half8_t*>(&sW1h[i * LD1 + 16 * j + 8 * h]);
-            const half8_t al = *reinterpret_cast<const half8_t*>(&sW1l[i * LD1 + 16 * j + 8 * h]);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, xh[j], sacc, 0, 0, 0);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, xl[j], sacc, 0, 0, 0);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, xh[j], sacc, 0, 0, 0);
+            const half8_t ah[2] = {operand(Img::w1(0, 0, j)), operand(Img::w1(0, 1, j))};
+            const half8_t al[2] = {operand(Img::w1(1, 0, j)), operand(Img::w1(1, 1, j))};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                sacc[u >> 1][u & 1] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u >> 1], xh[u & 1][j], j == 0 ? zero : sacc[u >> 1][u & 1], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                sacc[u >> 1][u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u >> 1], xl[u & 1][j], sacc[u >> 1][u & 1], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                sacc[u >> 1][u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u >> 1], xh[u & 1][j], sacc[u >> 1][u & 1], 0, 0, 0);
         }
-        // accumulator register r: feature 8(r/4) + 4h + r%4 of the chunk, atom = lane%32.  The sine
+        // accumulator register r of tile (u, t): feature 16 u + 4 g + r of the chunk, atom 16 t + i.  The sine
         // argument is formed in REVOLUTIONS (b arrives divided by 2 pi, the product takes 1 / 2 pi with its
         // inverse scales): v_sin_f32 / v_cos_f32 reduce the range themselves up to 256 revolutions; the
         // rounding of the argument, |arg| 6e-8 radians, is that of an fp32 argument in radians.  Beyond
@@ -557,44 +577,47 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
         const float crev = inv_sxw * 0.15915494309189535f;
         float umax = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 bv = *reinterpret_cast<const float4*>(&sb[8 * q + 4 * h]);
-            const float bq[4] = {bv.x, bv.y, bv.z, bv.w};
+        for (int u = 0; u < 2; ++u) {
+            const f4_t bv = *reinterpret_cast<const f4_t*>(&sb[16 * u + 4 * g]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                sacc[4 * q + e] = fmaf(sacc[4 * q + e], crev, bq[e]);
-                umax = fmaxf(umax, fabsf(sacc[4 * q + e]));
-            }
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sacc[u][t][e] = fmaf(sacc[u][t][e], crev, bv[e]);
+                    umax = fmaxf(umax, fabsf(sacc[u][t][e]));
+                }
         }
         if (__builtin_expect(__any(umax > UMAX), 0)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                if (fabsf(sacc[r]) > UMAX) sacc[r] -= rintf(sacc[r]);
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (fabsf(sacc[u >> 1][u & 1][e]) > UMAX) sacc[u >> 1][u & 1][e] -= rintf(sacc[u >> 1][u & 1][e]);
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 av = *reinterpret_cast<const float4*>(&sa[8 * q + 4 * h]);
-            const float aq[4] = {av.x, av.y, av.z, av.w};
+        for (int u = 0; u < 2; ++u) {
+            const f4_t av = *reinterpret_cast<const f4_t*>(&sa[16 * u + 4 * g]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float u = sacc[4 * q + e];
-                const float sn = __builtin_amdgcn_sinf(u), cs = __builtin_amdgcn_cosf(u);
-                energy = fmaf(aq[e], cs, energy);
-                sacc[4 * q + e] = -aq[e] * sn;           // 2^kp P
-            }
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float arg = sacc[u][t][e];
+                    const float sn = __builtin_amdgcn_sinf(arg), cs = __builtin_amdgcn_cosf(arg);
+                    energy[t] = fmaf(av[e], cs, energy[t]);
+                    sacc[u][t][e] = -av[e] * sn;         // 2^kp P
+                }
         }
         if constexpr (WITH_GRAD) {
             // at d = 128 the kernel takes all 256 registers: without this line the compiler keeps the arguments of the cosines
             // across the second product and spills for it, and a reload waits for the next image too.  The
             // second product goes ahead of the other wavefront's vector instructions: 86016 atoms, 32768 features
-            // 4.69 -> 4.42 ms together with the line below that holds the multiplications by b and alpha back; the same around
-            // the first product or around the sines gave nothing
+            // 4.01 -> 3.82 ms; the same around the first product or around the sines gave nothing
             if constexpr (D == 128) {
                 __builtin_amdgcn_sched_barrier(0);
                 __builtin_amdgcn_s_setprio(1);
             }
-            // second product: 2^kp GX^T[k, a] += 2^-kw sum_f 2^kw W[k, f] 2^kp P[f, a]; instruction t contracts the
-            // features of registers 8 t .. 8 t + 7.  The chunk's contribution is summed from zero and
+            // second product: 2^kp GX^T[k, a] += 2^-kw sum_f 2^kw W[k, f] 2^kp P[f, a]; one step contracts the
+            // chunk's 32 features, a lane's eight in the order of its registers.  The chunk's contribution is summed from zero and
             // added to the running sums by the vector unit: the matrix instruction aligns its products
             // to the accumulator it is given, and against a sum over a thousand chunks their low bits
             // would be cut off
@@ -602,27 +625,28 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    _Float16 a, c;
-                    split_f16(sacc[8 * t + q], a, c);
-                    ph[t][q] = a;
-                    pl[t][q] = c;
+                for (int q = 0; q < 8; q += 2) {
+                    half2_t a, c;
+                    split_pair(sacc[q >> 2][t][q & 3], sacc[q >> 2][t][(q & 3) + 1], a, c);
+                    ph[t][q] = a[0];
+                    ph[t][q + 1] = a[1];
+                    pl[t][q] = c[0];
+                    pl[t][q + 1] = c[1];
                 }
 #pragma unroll
-            for (int blk = 0; blk < D / 32; ++blk) {
-                float16_t part;
+            for (int k = 0; k < KT; ++k) {
+                const half8_t ah = operand(Img::w2(0, k)), al = operand(Img::w2(1, k));
+                f4_t part[2];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) part[r] = 0.0f;
+                for (int t = 0; t < 2; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, ph[t], zero, 0, 0, 0);
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const half8_t ah = *reinterpret_cast<const half8_t*>(&sW2h[(32 * blk + i) * LD2 + 16 * t + 8 * h]);
-                    const half8_t al = *reinterpret_cast<const half8_t*>(&sW2l[(32 * blk + i) * LD2 + 16 * t + 8 * h]);
-                    part = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph[t], part, 0, 0, 0);
-                    part = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, pl[t], part, 0, 0, 0);
-                    part = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ph[t], part, 0, 0, 0);
-                }
+                for (int t = 0; t < 2; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, pl[t], part[t], 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) gacc[blk][r] = fmaf(part[r], inv_sw, gacc[blk][r]);
+                for (int t = 0; t < 2; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ph[t], part[t], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) gacc[k][t][r] = fmaf(part[t][r], inv_sw, gacc[k][t][r]);
             }
         }
         if constexpr (WITH_GRAD && D == 128) __builtin_amdgcn_s_setprio(0);
@@ -639,33 +663,34 @@ __global__ __launch_bounds__(RE_T) __attribute__((amdgpu_waves_per_eu(2))) void 
         if (f0 + RE_FC < fend) round(f0 + RE_FC, 1, simg1, simg0);
     }
 
-    energy = (energy + __shfl_xor(energy, 32, 64)) * inv_sp;
-    if (!aok) return;
-    if (whole || part_out) {
-        if (h == 0) {
-            if (whole) e_slots[sorted_slots[row0 + arow]] = energy;
-            else part_out[arow] = energy;
-        }
-        if constexpr (WITH_GRAD) {
-            float* gr = (whole ? gx + (size_t)row0 * D : part_out + RE_M) + (size_t)arow * D;
 #pragma unroll
-            for (int blk = 0; blk < D / 32; ++blk)
+    for (int t = 0; t < 2; ++t) {
+        float e = energy[t];
+        e += __shfl_xor(e, 16, 64);
+        e += __shfl_xor(e, 32, 64);
+        e *= inv_sp;
+        const int row = arow + 16 * t;
+        if (row >= rows) continue;
+        if (whole || part_out) {
+            if (g == 0) {
+                if (whole) e_slots[sorted_slots[row0 + row]] = e;
+                else part_out[row] = e;
+            }
+            if constexpr (WITH_GRAD) {
+                float* gr = (whole ? gx + (size_t)row0 * D : part_out + RE_M) + (size_t)row * D + 4 * g;
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    *reinterpret_cast<float4*>(gr + 32 * blk + 8 * q + 4 * h) =
-                        make_float4(gacc[blk][4 * q] * inv_sp, gacc[blk][4 * q + 1] * inv_sp,
-                                    gacc[blk][4 * q + 2] * inv_sp, gacc[blk][4 * q + 3] * inv_sp);
-        }
-    } else {
-        // no workspace: the parts add into zero-filled outputs
-        if (h == 0) atomicAdd(&e_slots[sorted_slots[row0 + arow]], energy);
-        if constexpr (WITH_GRAD) {
-            float* gr = gx + (size_t)(row0 + arow) * D;
+                for (int k = 0; k < KT; ++k) *reinterpret_cast<f4_t*>(gr + 16 * k) = gacc[k][t] * inv_sp;
+            }
+        } else {
+            // no workspace: the parts add into zero-filled outputs
+            if (g == 0) atomicAdd(&e_slots[sorted_slots[row0 + row]], e);
+            if constexpr (WITH_GRAD) {
+                float* gr = gx + (size_t)(row0 + row) * D + 4 * g;
 #pragma unroll
-            for (int blk = 0; blk < D / 32; ++blk)
+                for (int k = 0; k < KT; ++k)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    atomicAdd(gr + 32 * blk + 8 * (r / 4) + 4 * h + (r % 4), gacc[blk][r] * inv_sp);
+                    for (int r = 0; r < 4; ++r) atomicAdd(gr + 16 * k + r, gacc[k][t][r] * inv_sp);
+            }
         }
     }
 }

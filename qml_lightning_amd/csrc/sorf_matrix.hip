@@ -44,7 +44,6 @@
 namespace {
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
-typedef float f2_t __attribute__((ext_vector_type(2)));
 
 constexpr int SM_WAVES = 4;                  // wavefronts per workgroup
 constexpr int SM_ATOMS = 16 * SM_WAVES;
@@ -170,29 +169,11 @@ __device__ __forceinline__ void block_stages(f4_t (&v)[NB]) {
     }
 }
 
-// v minus one half of a packed pair, in one instruction (written out, the compiler converts and subtracts: two)
-__device__ __forceinline__ float minus_low(float v, half2_t h) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
-    return r;
-}
-__device__ __forceinline__ float minus_high(float v, half2_t h) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
-    return r;
-}
-
 // four values as the lane's eight k entries of an operand: high parts, then low parts, both rounded to nearest
 __device__ __forceinline__ half8_t split4(f4_t v) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float t = v[r];
-        asm("" : "+v"(t));        // the value as it was rounded to fp32: see split_f16
-        v[r] = t;
-    }
-    const half2_t h0 = __builtin_convertvector((f2_t){v[0], v[1]}, half2_t), h1 = __builtin_convertvector((f2_t){v[2], v[3]}, half2_t);
-    const half2_t l0 = __builtin_convertvector((f2_t){minus_low(v[0], h0), minus_high(v[1], h0)}, half2_t);
-    const half2_t l1 = __builtin_convertvector((f2_t){minus_low(v[2], h1), minus_high(v[3], h1)}, half2_t);
+    half2_t h0, h1, l0, l1;
+    split_pair(v[0], v[1], h0, l0);
+    split_pair(v[2], v[3], h1, l1);
     return (half8_t){h0[0], h0[1], h1[0], h1[1], l0[0], l0[1], l1[0], l1[1]};
 }
 
