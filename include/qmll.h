@@ -371,6 +371,13 @@ int qmll_project_typed_backward_sums(const float* gx, const int* sorted_slots, c
                                      int ne, int R, int d, float* g_rep, const float* e_slots, int B, int n,
                                      float* energies, qmll_stream_t stream);
 
+/* qmll_project_typed_backward_sums of a gradient and energies in nparts parts as qmll_sorf_energy_parts writes them (gx f32
+ * [nparts,A,d], e_slots f32 [nparts,B*n]): the parts are added in order.  Both arrays may be written. */
+int qmll_project_typed_backward_parts(float* gx, int nparts, const int* sorted_slots, const int* type_offsets,
+                                      const float* reductors, const void* reductors_split, const int* types, int A, int N,
+                                      int ne, int R, int d, float* g_rep, float* e_slots, int B, int n,
+                                      float* energies, qmll_stream_t stream);
+
 /* qmll_sorf_energy_typed on compact element-sorted rows: x f32 [A,d] as written by
  * qmll_project_typed, D f32 [ne,T,S,d], bias f32 [ne,S*d], alpha f32 [S*d].
  *   -> e_slots[sorted_slots[a]] = energy contribution of atom a (a < type_offsets[ne];
@@ -386,6 +393,15 @@ int qmll_project_typed_backward_sums(const float* gx, const int* sorted_slots, c
 int qmll_sorf_energy_sorted(const float* x, const int* type_offsets, const int* sorted_slots, const float* D,
                             const float* bias, const float* alpha, const float* bias_absmax, int A, int ne, int d, int S,
                             int T, float normalisation, float* e_slots, float* gx, qmll_stream_t stream);
+
+/* qmll_sorf_energy_sorted with the stacks shared out over nparts parts (few atoms: their tiles alone leave most of the chip
+ * idle), each with outputs of its own: e_parts f32 [nparts,nslots], zero-filled by the caller, and gx_parts f32 [nparts,A,d] or NULL.
+ * Their sums over the parts are what qmll_sorf_energy_sorted writes.  d = 64, 128 or 256.  qmll_sorf_energy_parts_count: the
+ * number that is fastest (1: use qmll_sorf_energy_sorted). */
+int qmll_sorf_energy_parts_count(int A, int ne, int d, int S, int T, int nslots);
+int qmll_sorf_energy_parts(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,
+                           const float* alpha, const float* bias_absmax, int A, int ne, int d, int S, int T, float normalisation,
+                           int nparts, float* e_parts, int nslots, float* gx_parts, qmll_stream_t stream);
 
 /* qmll_sorf_energy_sorted on the half-precision matrix cores (large batches; d = 64 or 128, T = 1 or 2; diagonals of +-1:
  * where the device finds others the call runs as qmll_sorf_energy_sorted does).  x, D, work and gx 16-byte aligned.

@@ -14,6 +14,8 @@
 // elements are touched: no work is spent on padding or on the other elements' reductors.
 #include <mutex>
 
+#include <algorithm>
+
 #include "qmll_common.h"
 
 namespace {
@@ -849,6 +851,30 @@ __device__ __forceinline__ void row_sums(const float* __restrict__ values, int B
     for (int i = 0; i < n; ++i) acc += values[(size_t)m * n + i];
     sums[m] = acc;
 }
+// the same over nparts arrays of B n values each: a wavefront per molecule, all of its values in flight at once
+__device__ __forceinline__ void row_sums_of_parts(const float* __restrict__ values, int nparts, int B, int n,
+                                                  float* __restrict__ sums, int chunk) {
+    const int m = chunk * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (m >= B) return;
+    float acc = 0.0f;
+    for (int t = lane; t < nparts * n; t += 64) {
+        const int k = t / n;
+        acc += values[(size_t)k * B * n + (size_t)m * n + (t - k * n)];
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) sums[m] = acc;
+}
+__host__ __device__ __forceinline__ int sum_chunks(int B, int nparts) { return nparts > 1 ? (B + 3) / 4 : (B + 255) / 256; }
+
+// values[i] += the other parts' (nparts arrays of count each, `stride` apart), in order
+__global__ __launch_bounds__(256) void add_parts_kernel(float* __restrict__ values, size_t count, int nparts, size_t stride) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) {
+        float v = values[i];
+        for (int k = 1; k < nparts; ++k) v += values[k * stride + i];
+        values[i] = v;
+    }
+}
+
 // rows of real atoms whose element the model does not know get a zero gradient
 // (lane = slot; the rare untyped slots of a wavefront are then zeroed row by row by all lanes)
 __device__ __forceinline__ void zero_untyped_rows(const int* __restrict__ types, int N, int ne, int R,
@@ -867,10 +893,12 @@ __device__ __forceinline__ void zero_untyped_rows(const int* __restrict__ types,
 
 __global__ __launch_bounds__(256) void zero_untyped_rows_kernel(const int* __restrict__ types, int N, int ne, int R,
                                                                 float* __restrict__ out, int zero_groups,
-                                                                const float* __restrict__ e_slots, int B, int n,
+                                                                const float* __restrict__ e_slots, int nparts, int B, int n,
                                                                 float* __restrict__ energies) {
     if ((int)blockIdx.x < zero_groups)
         zero_untyped_rows(types, N, ne, R, out, blockIdx.x);
+    else if (nparts > 1)
+        row_sums_of_parts(e_slots, nparts, B, n, energies, (int)blockIdx.x - zero_groups);
     else                                               // workgroups past the slots: the per-molecule energy sums
         row_sums(e_slots, B, n, energies, (int)blockIdx.x - zero_groups);
 }
@@ -886,7 +914,6 @@ __global__ __launch_bounds__(256) void zero_untyped_rows_kernel(const int* __res
 constexpr int SMALL_ATOMS = 4096;
 constexpr size_t SMALL_READS = 192u << 20;   // floats of reductor per atom times atoms
 __host__ inline bool small_batch(int A, int R, int d) { return A <= SMALL_ATOMS && (size_t)A * R * d <= SMALL_READS; }
-constexpr int SMALL_KS = 8;        // slices of the contraction in project_small_kernel
 
 __device__ __forceinline__ int type_of_position(const int* __restrict__ type_offsets, int ne, int p) {
     int e = 0;
@@ -911,9 +938,12 @@ __device__ __forceinline__ bool small_tile(const int* __restrict__ type_offsets,
     return false;                                      // a tile beyond the sorted list
 }
 
-// x[p, :] = rep[slot(p), :] . U_e: thread = (contraction slice, four columns), slices folded through LDS;
-// a workgroup takes NA atoms of one element, so a reductor read serves them all
-template <int NA>
+// x[p, :] = rep[slot(p), :] . U_e: thread = (contraction slice, four columns); a workgroup takes PS_COLS columns (gridDim.y
+// times make d) of NA atoms of one element, so a reductor read serves them all.  PS_COLS / 4 lanes read a reductor row side by
+// side, the slices of the contraction are folded through lanes and LDS.  The first loads of U go out before the
+// rows are staged.
+constexpr int PS_AHEAD = 8;
+template <int NA, int PS_COLS>
 __global__ __launch_bounds__(256) void project_small_kernel(const float* __restrict__ rep,
                                                             const int* __restrict__ sorted_slots,
                                                             const int* __restrict__ type_offsets,
@@ -922,53 +952,86 @@ __global__ __launch_bounds__(256) void project_small_kernel(const float* __restr
     extern __shared__ float sm[];
     const int R4 = (R + 3) & ~3;
     float* srow = sm;                                  // [NA][R4]
-    float* spart = sm + NA * R4;                       // [SMALL_KS][NA][d]
-    const int tid = threadIdx.x;
+    float* spart = sm + NA * R4;                       // [4][NA][PS_COLS]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int e, row0, rows;
     if (!small_tile<NA>(type_offsets, ne, blockIdx.x, e, row0, rows)) return;
-    for (int a = 0; a < NA; ++a) {
-        const float* row = rep + (size_t)sorted_slots[row0 + (a < rows ? a : 0)] * R;
-        for (int k = tid; k < R; k += 256) srow[a * R4 + k] = a < rows ? row[k] : 0.0f;
+    constexpr int CL = PS_COLS / 4, KS = 256 / CL;     // lanes along the columns, slices of the contraction
+    const int col = blockIdx.y * PS_COLS + 4 * (tid % CL), ks = tid / CL;
+    const bool inside = col < d;
+    const float* U = reductors + (size_t)e * R * d + (inside ? col : 0);
+    float4 u[PS_AHEAD];
+#pragma unroll
+    for (int j = 0; j < PS_AHEAD; ++j) u[j] = *reinterpret_cast<const float4*>(U + (size_t)min(ks + KS * j, R - 1) * d);
+    const float* row[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) row[a] = rep + (size_t)sorted_slots[row0 + (a < rows ? a : 0)] * R;
+    for (int k = tid; k < R; k += 256) {               // the loads of all rows in flight together
+        float v[NA];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) v[a] = row[a][k];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) srow[a * R4 + k] = a < rows ? v[a] : 0.0f;
     }
     __syncthreads();
-    const float* U = reductors + (size_t)e * R * d;
-    const int ks = tid >> 5, l32 = tid & 31;
-    for (int c4 = l32; c4 < d / 4; c4 += 32) {
-        float4 acc[NA];
+    float4 acc[NA];
 #pragma unroll
-        for (int a = 0; a < NA; ++a) acc[a] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 4
-        for (int k = ks; k < R; k += SMALL_KS) {
-            const float4 u = *reinterpret_cast<const float4*>(U + (size_t)k * d + 4 * c4);
+    for (int a = 0; a < NA; ++a) acc[a] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k0 = ks; k0 < R; k0 += KS * PS_AHEAD) {
+        float4 now[PS_AHEAD];
+#pragma unroll
+        for (int j = 0; j < PS_AHEAD; ++j) now[j] = u[j];
+        const int k1 = k0 + KS * PS_AHEAD;
+        if (k1 < R) {
+#pragma unroll
+            for (int j = 0; j < PS_AHEAD; ++j) u[j] = *reinterpret_cast<const float4*>(U + (size_t)min(k1 + KS * j, R - 1) * d);
+        }
+#pragma unroll
+        for (int j = 0; j < PS_AHEAD; ++j) {
+            const int k = k0 + KS * j;
+            if (k >= R) break;
 #pragma unroll
             for (int a = 0; a < NA; ++a) {
                 const float r = srow[a * R4 + k];
-                acc[a].x = fmaf(r, u.x, acc[a].x);
-                acc[a].y = fmaf(r, u.y, acc[a].y);
-                acc[a].z = fmaf(r, u.z, acc[a].z);
-                acc[a].w = fmaf(r, u.w, acc[a].w);
+                acc[a].x = fmaf(r, now[j].x, acc[a].x);
+                acc[a].y = fmaf(r, now[j].y, acc[a].y);
+                acc[a].z = fmaf(r, now[j].z, acc[a].z);
+                acc[a].w = fmaf(r, now[j].w, acc[a].w);
             }
         }
+    }
 #pragma unroll
-        for (int a = 0; a < NA; ++a) *reinterpret_cast<float4*>(spart + ((size_t)ks * NA + a) * d + 4 * c4) = acc[a];
+    for (int a = 0; a < NA; ++a) {
+        float* v = reinterpret_cast<float*>(&acc[a]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (CL <= 8) v[c] += lane_xor<8>(v[c]);
+            if constexpr (CL <= 16) v[c] += lane_xor<16>(v[c]);
+            v[c] += lane_xor<32>(v[c]);
+        }
+        if (lane < CL) *reinterpret_cast<float4*>(spart + ((size_t)wave * NA + a) * PS_COLS + 4 * lane) = acc[a];
     }
     __syncthreads();
-    for (int i = tid; i < rows * d; i += 256) {
-        const int a = i / d, c = i - a * d;
+    for (int i = tid; i < rows * PS_COLS; i += 256) {
+        const int a = i / PS_COLS, c = i - a * PS_COLS;
         float sum = 0.0f;
 #pragma unroll
-        for (int q = 0; q < SMALL_KS; ++q) sum += spart[((size_t)q * NA + a) * d + c];
-        x[(size_t)(row0 + a) * d + c] = sum;
+        for (int w = 0; w < 4; ++w) sum += spart[((size_t)w * NA + a) * PS_COLS + c];
+        if (blockIdx.y * PS_COLS + c < (unsigned)d) x[(size_t)(row0 + a) * d + blockIdx.y * PS_COLS + c] = sum;
     }
 }
 
-// g_rep[slot(p), :] = gx[p, :] . U_e^T: thread = output entry r, its reductor row is contiguous.  A
-// workgroup takes NA consecutive sorted atoms of one element (tiles never straddle two elements), so a
-// reductor row read serves NA atoms: with one atom per workgroup 1008 atoms read 160 MB of reductors from
-// L2 (20 us), with eight 20 MB.  Workgroups past the tiles zero the rows of slots whose type is outside
-// [0, ne), 256 slots each, and after those, when asked, sum the per-slot energies of 256 molecules each.
+// g_rep[slot(p), :] = gx[p, :] . U_e^T: four lanes share an output entry, whose reductor row they read 64 contiguous bytes at a
+// time; a workgroup has BT_ROWS entries (gridDim.y of them make R) for NA consecutive sorted atoms of one element (tiles never
+// straddle two elements), so a reductor row read serves NA atoms: with one atom per workgroup 1008 atoms read 160 MB of
+// reductors from L2, with eight 20 MB.  gx may come in nparts parts (A d floats each), which are added in order as they
+// are staged.  Workgroups past the tiles (of the first row of the grid) zero the rows of slots whose type is outside
+// [0, ne), 256 slots each, and after those, when asked, sum the per-slot energies of the molecules.
+// (A thread that took an entry by itself read 512 bytes apart from its neighbours': 21 atoms 7.2 us, now 2.6; 1536 atoms 12.8,
+// now 8.8; 600 atoms of 128 components 4.9.)
+constexpr int BT_ROWS = 64;
 template <int NA>
-__global__ __launch_bounds__(256) void project_bt_small_kernel(const float* __restrict__ gx,
+__global__ __launch_bounds__(256) void project_bt_small_kernel(const float* __restrict__ gx, int nparts, size_t part_stride,
                                                                const int* __restrict__ sorted_slots,
                                                                const int* __restrict__ type_offsets,
                                                                const float* __restrict__ reductors, int ne, int R, int d,
@@ -977,40 +1040,49 @@ __global__ __launch_bounds__(256) void project_bt_small_kernel(const float* __re
                                                                const float* __restrict__ e_slots, int B, int n,
                                                                float* __restrict__ energies) {
     extern __shared__ float sm[];                      // [NA][d]
-    if ((int)blockIdx.x >= tiles + zero_groups) {      // spare workgroups: the per-molecule energy sums
-        row_sums(e_slots, B, n, energies, (int)blockIdx.x - tiles - zero_groups);
-        return;
-    }
     if ((int)blockIdx.x >= tiles) {
-        zero_untyped_rows(types, N, ne, R, g_rep, (int)blockIdx.x - tiles);
+        if (blockIdx.y != 0) return;
+        const int spare = (int)blockIdx.x - tiles;
+        if (spare < zero_groups) zero_untyped_rows(types, N, ne, R, g_rep, spare);
+        else if (nparts > 1) row_sums_of_parts(e_slots, nparts, B, n, energies, spare - zero_groups);
+        else row_sums(e_slots, B, n, energies, spare - zero_groups);
         return;
     }
     const int tid = threadIdx.x;
     int e, row0, rows;
     if (!small_tile<NA>(type_offsets, ne, blockIdx.x, e, row0, rows)) return;
-    for (int i = tid; i < NA * d; i += 256) sm[i] = i < rows * d ? gx[(size_t)row0 * d + i] : 0.0f;
+    for (int i = tid; i < NA * d; i += 256) {
+        float v = 0.0f;
+        if (i < rows * d) {
+            const float* g = gx + (size_t)row0 * d + i;
+            v = g[0];
+#pragma unroll 8
+            for (int k = 1; k < nparts; ++k) v += g[k * part_stride];
+        }
+        sm[i] = v;
+    }
     __syncthreads();
-    const float* U = reductors + (size_t)e * R * d;
+    const int r = blockIdx.y * BT_ROWS + (tid >> 2), q = tid & 3;
+    const float4* u4 = reinterpret_cast<const float4*>(reductors + ((size_t)e * R + min(r, R - 1)) * d);
     const float4* g4 = reinterpret_cast<const float4*>(sm);
     const int d4 = d / 4;
-    for (int r = tid; r < R; r += 256) {
-        const float4* u4 = reinterpret_cast<const float4*>(U + (size_t)r * d);
-        float a0[NA], a1[NA];
+    float acc[NA];
 #pragma unroll
-        for (int a = 0; a < NA; ++a) a0[a] = a1[a] = 0.0f;
-#pragma unroll 4
-        for (int c4 = 0; c4 < d4; ++c4) {
-            const float4 u = u4[c4];
+    for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+#pragma unroll 8
+    for (int c = q; c < d4; c += 4) {
+        const float4 u = u4[c];
 #pragma unroll
-            for (int a = 0; a < NA; ++a) {
-                const float4 g = g4[a * d4 + c4];
-                a0[a] = fmaf(u.x, g.x, fmaf(u.y, g.y, a0[a]));
-                a1[a] = fmaf(u.z, g.z, fmaf(u.w, g.w, a1[a]));
-            }
+        for (int a = 0; a < NA; ++a) {
+            const float4 g = g4[a * d4 + c];
+            acc[a] = fmaf(u.x, g.x, fmaf(u.y, g.y, fmaf(u.z, g.z, fmaf(u.w, g.w, acc[a]))));
         }
+    }
 #pragma unroll
-        for (int a = 0; a < NA; ++a)
-            if (a < rows) g_rep[(size_t)sorted_slots[row0 + a] * R + r] = a0[a] + a1[a];
+    for (int a = 0; a < NA; ++a) {
+        acc[a] += lane_xor<1>(acc[a]);
+        acc[a] += lane_xor<2>(acc[a]);
+        if (q == (a & 3) && a < rows && r < R) g_rep[(size_t)sorted_slots[row0 + a] * R + r] = acc[a];
     }
 }
 
@@ -1283,25 +1355,32 @@ extern "C" int qmll_project_typed(const float* rep, const int* sorted_slots, con
                  "qmll_project_typed: null pointer");
     const bool vec = R % 4 == 0 && d % 4 == 0 && aligned16(rep) && aligned16(reductors);
     if (vec && small_batch(A, R, d)) {
-        // several atoms of one element per workgroup from some hundreds of atoms on, while their rows and partial
-        // sums fit in LDS
-        const size_t per_atom = sizeof(float) * (((size_t)R + 3) / 4 * 4 + (size_t)SMALL_KS * d);
-        // (measured at 312 x 128: one atom 8.4 us at 1008 atoms and 12.8 at 2016, two 8.1 / 8.7, four 10.2 / 10.7 and
-        // 11.8 at 4032, where two take 13.8; eight are never the fastest: the loads here are coalesced, the
-        // multiplications of a workgroup are what grows)
-        int na = A <= 768 ? 1 : (A <= 2304 ? 2 : 4);
+        // A workgroup of 32 columns has all its loads in flight at once, one of 128 stages a row for four times as many products;
+        // more atoms per workgroup save reductor reads once there are workgroups enough.  In units of 32 columns of an
+        // atom: one atom up to 500, two up to 1300, four up to 5000; then 128 columns of four atoms (32 of eight below 128
+        // components).  Measured in us, one workgroup for all columns / this rule: 312 x 128, 21 atoms 4.3 / 3.4, 300 5.0 / 4.7, 600 6.5 /
+        // 5.6, 1000 6.2 / 6.7, 1536 7.5 / 8.2, 2688 10.6 / 9.6; 496 x 128, 21 atoms 5.2 / 3.6, 600 8.8 / 6.3, 2016 12.1 / 11.0; 720 x 64, 21
+        // atoms 6.4 / 4.3, 1000 9.1 / 6.8, 4032 20.0 / 13.1; 496 x 256, 21 atoms 7.9 / 3.6, 600 14.6 / 8.5, 1536 17.8 / 15.2
+        const long long units = (long long)A * d / 32;
+        const int cols = units > 5000 && d >= 128 ? 128 : 32;
+        int na = units <= 500 ? 1 : units <= 1300 ? 2 : units <= 5000 || d >= 128 ? 4 : 8;
+        const size_t per_atom = sizeof(float) * (((size_t)R + 3) / 4 * 4 + 4 * (size_t)cols);
         while (na > 1 && na * per_atom > 64 * 1024) na >>= 1;
         if (per_atom <= 64 * 1024) {
-            const dim3 grid((A + na - 1) / na + (na > 1 ? ne : 0));
-            if (na == 1)
-                hipLaunchKernelGGL(project_small_kernel<1>, grid, dim3(256), per_atom, (hipStream_t)stream, rep, sorted_slots,
-                                   type_offsets, reductors, ne, R, d, x);
-            else if (na == 2)
-                hipLaunchKernelGGL(project_small_kernel<2>, grid, dim3(256), 2 * per_atom, (hipStream_t)stream, rep,
-                                   sorted_slots, type_offsets, reductors, ne, R, d, x);
-            else
-                hipLaunchKernelGGL(project_small_kernel<4>, grid, dim3(256), 4 * per_atom, (hipStream_t)stream, rep,
-                                   sorted_slots, type_offsets, reductors, ne, R, d, x);
+            const dim3 grid((A + na - 1) / na + (na > 1 ? ne : 0), (d + cols - 1) / cols);
+            auto launch = [&](auto nac, auto cc) {
+                constexpr int NA = decltype(nac)::value;
+                hipLaunchKernelGGL((project_small_kernel<NA, decltype(cc)::value>), grid, dim3(256), NA * per_atom, (hipStream_t)stream,
+                                   rep, sorted_slots, type_offsets, reductors, ne, R, d, x);
+            };
+            auto by_cols = [&](auto nac) {
+                if (cols == 32) launch(nac, std::integral_constant<int, 32>{});
+                else launch(nac, std::integral_constant<int, 128>{});
+            };
+            if (na == 1) by_cols(std::integral_constant<int, 1>{});
+            else if (na == 2) by_cols(std::integral_constant<int, 2>{});
+            else if (na == 4) by_cols(std::integral_constant<int, 4>{});
+            else by_cols(std::integral_constant<int, 8>{});
             QMLL_CHECK_LAUNCH("qmll_project_typed");
             return QMLL_OK;
         }
@@ -1376,19 +1455,35 @@ extern "C" int qmll_project_typed_backward_sums(const float* gx, const int* sort
                                                 const float* reductors, const void* reductors_split, const int* types,
                                                 int A, int N, int ne, int R, int d, float* g_rep, const float* e_slots,
                                                 int B, int n, float* energies, qmll_stream_t stream) {
+    // (one part: neither array is written)
+    return qmll_project_typed_backward_parts(const_cast<float*>(gx), 1, sorted_slots, type_offsets, reductors, reductors_split, types, A,
+                                             N, ne, R, d, g_rep, const_cast<float*>(e_slots), B, n, energies, stream);
+}
+
+extern "C" int qmll_project_typed_backward_parts(float* gx, int nparts, const int* sorted_slots, const int* type_offsets,
+                                                 const float* reductors, const void* reductors_split, const int* types,
+                                                 int A, int N, int ne, int R, int d, float* g_rep, float* e_slots,
+                                                 int B, int n, float* energies, qmll_stream_t stream) {
+    QMLL_REQUIRE(nparts > 0, QMLL_ERR_INVALID, "qmll_project_typed_backward: bad number of parts %d", nparts);
     QMLL_REQUIRE(A >= 0 && N >= 0 && ne > 0 && R > 0 && d > 0, QMLL_ERR_INVALID,
                  "qmll_project_typed_backward: bad size A=%d N=%d ne=%d R=%d d=%d", A, N, ne, R, d);
     const bool sums = energies != nullptr && B > 0;
     QMLL_REQUIRE(!sums || (e_slots && n > 0), QMLL_ERR_INVALID, "qmll_project_typed_backward_sums: energies without e_slots");
     const bool vec = R % 4 == 0 && d % 4 == 0 && aligned16(gx) && aligned16(reductors);
     const bool small = vec && A > 0 && small_batch(A, R, d) && (size_t)8 * d * sizeof(float) <= 64 * 1024 && N <= 256 * 256;
+    if (!small && nparts > 1 && A > 0 && gx) {                // only the small kernels add the parts of gx as they read them
+        const size_t count = (size_t)A * d;
+        hipLaunchKernelGGL(add_parts_kernel, dim3((unsigned)std::min<size_t>((count + 255) / 256, 4096)), dim3(256), 0,
+                           (hipStream_t)stream, gx, count, nparts, count);
+        QMLL_CHECK_LAUNCH("qmll_project_typed_backward");
+    }
     if (!small && ((types && N > 0) || sums)) {
         // the rows of unknown elements and the energy sums: one launch for the two
         const int zero_groups = (types && N > 0) ? (N + 255) / 256 : 0;
-        const int sum_groups = sums ? (B + 255) / 256 : 0;
+        const int sum_groups = sums ? sum_chunks(B, nparts) : 0;
         QMLL_REQUIRE(g_rep || zero_groups == 0, QMLL_ERR_INVALID, "qmll_project_typed_backward: null pointer");
         hipLaunchKernelGGL(zero_untyped_rows_kernel, dim3(zero_groups + sum_groups), dim3(256), 0, (hipStream_t)stream, types,
-                           N, ne, R, g_rep, zero_groups, e_slots, B, n, energies);
+                           N, ne, R, g_rep, zero_groups, e_slots, nparts, B, n, energies);
         QMLL_CHECK_LAUNCH("qmll_project_typed_backward");
     }
     if (A == 0) return QMLL_OK;
@@ -1399,15 +1494,15 @@ extern "C" int qmll_project_typed_backward_sums(const float* gx, const int* sort
         // one launch: a workgroup per atom, one per 256 slots for the rows of unknown elements, one per 256
         // molecules for the energy sums
         const int zero_groups = (types && N > 0) ? (N + 255) / 256 : 0;
-        const int sum_groups = sums ? (B + 255) / 256 : 0;
+        const int sum_groups = sums ? sum_chunks(B, nparts) : 0;
         // atoms per workgroup: one while the atoms are the only parallelism there is, more as the reductor
         // reads of all workgroups together begin to count
 #define LAUNCH_BT_SMALL(NA)                                                                                         \
     {                                                                                                               \
         const int tiles = (A + (NA) - 1) / (NA) + ((NA) > 1 ? ne : 0);                                              \
-        hipLaunchKernelGGL(project_bt_small_kernel<NA>, dim3(tiles + zero_groups + sum_groups), dim3(256),          \
-                           sizeof(float) * (NA) * d, (hipStream_t)stream, gx, sorted_slots, type_offsets, reductors, \
-                           ne, R, d, g_rep, tiles, types, N, zero_groups, e_slots, B, n, energies);                 \
+        hipLaunchKernelGGL(project_bt_small_kernel<NA>, dim3(tiles + zero_groups + sum_groups, (R + BT_ROWS - 1) / BT_ROWS), \
+                           dim3(256), sizeof(float) * (NA) * d, (hipStream_t)stream, gx, nparts, (size_t)A * d, sorted_slots, \
+                           type_offsets, reductors, ne, R, d, g_rep, tiles, types, N, zero_groups, e_slots, B, n, energies);  \
     }
         if (A < 64) LAUNCH_BT_SMALL(1) else if (A < 512) LAUNCH_BT_SMALL(4) else LAUNCH_BT_SMALL(8)
 #undef LAUNCH_BT_SMALL

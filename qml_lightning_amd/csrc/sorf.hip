@@ -16,6 +16,9 @@
 // VALU bound (one sincos per feature).
 #include <type_traits>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "qmll_common.h"
 
 namespace {
@@ -594,13 +597,15 @@ constexpr int ROWS_NA = 4;   // atoms per workgroup = rows of 16 lanes per wavef
 // as for T = 1, the later ones are fetched where they are used (forward and again in the adjoint).
 // NW: wavefronts per workgroup, which share out the stacks (16 for a few atoms: a molecule then takes
 // a quarter of the time, its stacks being the only parallelism there is).
+// PARTS: this workgroup takes part `part` of `nparts` of the stacks (e_atom and gx are the part's own).
 template <int LOG2D, bool WITH_GRAD, bool MULTI, int NW>
 __device__ __forceinline__ void sorf_energy_rows(
     int block, int nblocks, const float* __restrict__ x, const float* __restrict__ D, const float* __restrict__ bias,
     const float* __restrict__ alpha, const float* __restrict__ bias_absmax, const int* __restrict__ out_index,
     const int* __restrict__ type_offsets, int ne, int A, int S, int T_, float scale, float normf, float* __restrict__ e_atom,
-    float* __restrict__ gx) {
+    float* __restrict__ gx, int part = 0, int nparts = 1) {
     const int T = MULTI ? T_ : 1;
+    const int step = NW * nparts;               // stacks between two of a wavefront's
     constexpr int d = 1 << LOG2D;
     constexpr int EPL = d / 16;                 // registers per lane
     constexpr int NA = ROWS_NA;
@@ -751,14 +756,14 @@ __device__ __forceinline__ void sorf_energy_rows(
         // bias and alpha at the start of their own stack (needed after the transform)
         auto stacks = [&](auto tracked) {
             float d0[EPL], d1[EPL];
-            int s = wave;
+            int s = wave + NW * part;
             if (s < S) load_row<EPL>(d0, D + (size_t)s * d + e0);
             while (s < S) {
-                stack(tracked, d0, d1, D + (size_t)(s + NW < S ? s + NW : s) * d + e0, (size_t)s * d + e0);
-                s += NW;
+                stack(tracked, d0, d1, D + (size_t)(s + step < S ? s + step : s) * d + e0, (size_t)s * d + e0);
+                s += step;
                 if (s >= S) break;
-                stack(tracked, d1, d0, D + (size_t)(s + NW < S ? s + NW : s) * d + e0, (size_t)s * d + e0);
-                s += NW;
+                stack(tracked, d1, d0, D + (size_t)(s + step < S ? s + step : s) * d + e0, (size_t)s * d + e0);
+                s += step;
             }
         };
         if (track)
@@ -776,14 +781,14 @@ __device__ __forceinline__ void sorf_energy_rows(
     // per stack: the sign diagonal is fetched one stack ahead (it is the first thing a stack
     // needs), bias and alpha at the start of their own stack (needed after the transform)
     float dv[EPL], bv[EPL], av[EPL];
-    int s = wave;
+    int s = wave + NW * part;
     if (s < S) load_row<EPL>(dv, D + (size_t)s * d + e0);
-    for (; s < S; s += NW) {
+    for (; s < S; s += step) {
         const size_t off = (size_t)s * d + e0;               // the same for the four rows
         load_row<EPL>(bv, bias + off);
         load_row<EPL>(av, alpha + off);
         float dn[EPL];
-        load_row<EPL>(dn, D + (size_t)(s + NW < S ? s + NW : s) * d + e0);
+        load_row<EPL>(dn, D + (size_t)(s + step < S ? s + step : s) * d + e0);
 
         float v[EPL];
 #pragma unroll
@@ -879,6 +884,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LOG2D >
     float* __restrict__ gx) {
     sorf_energy_rows<LOG2D, WITH_GRAD, MULTI, NW>((int)blockIdx.x, (int)gridDim.x, x, D, bias, alpha, bias_absmax, out_index, type_offsets,
                                                   ne, A, S, T, scale, normf, e_atom, gx);
+}
+
+// Few atoms: the stacks are shared out over nparts = gridDim.y workgroups of four wavefronts as well, each with an output of its
+// own (e_parts + part * e_stride, gx_parts + part * A * d), which the kernel behind it adds up in order (project.hip).  A molecule of
+// 21 atoms is six tiles: sixteen wavefronts each on six CUs of 256 take 12.5 us for 128 stacks, bound by those CUs' vector
+// issue; twelve parts take 4.0.
+template <int LOG2D, bool WITH_GRAD, bool MULTI>
+__global__ __launch_bounds__(SORF_THREADS) void sorf_energy_parts_kernel(
+    const float* __restrict__ x, const float* __restrict__ D, const float* __restrict__ bias, const float* __restrict__ alpha,
+    const float* __restrict__ bias_absmax, const int* __restrict__ out_index, const int* __restrict__ type_offsets, int ne, int A,
+    int S, int T, float scale, float normf, float* __restrict__ e_parts, size_t e_stride, float* __restrict__ gx_parts) {
+    const int part = (int)blockIdx.y;
+    sorf_energy_rows<LOG2D, WITH_GRAD, MULTI, SORF_WAVES>((int)blockIdx.x, (int)gridDim.x, x, D, bias, alpha, bias_absmax, out_index,
+                                                          type_offsets, ne, A, S, T, scale, normf, e_parts + part * e_stride,
+                                                          WITH_GRAD ? gx_parts + (size_t)part * A * (1 << LOG2D) : nullptr, part,
+                                                          (int)gridDim.y);
 }
 
 // the same where *only_if is not 0, by a grid small enough to cost little where it is: the workgroups take tile after tile
@@ -1726,6 +1747,57 @@ extern "C" int qmll_sorf_energy_sorted(const float* x, const int* type_offsets, 
                  "qmll_sorf_energy_sorted: null pointer");
     return launch_fused("qmll_sorf_energy_sorted", x, D, bias, alpha, bias_absmax, sorted_slots, nullptr, type_offsets, ne, A, d, S, T,
                         normalisation, e_slots, gx, (hipStream_t)stream);
+}
+
+// Parts of the stacks of a small batch.  A part more shortens the chain of a wavefront's stacks and lengthens the reading of the
+// parts by the projection behind it.  Both kernels together, one part / the best number, us: 128 components, 128 stacks: 21 atoms
+// 15.2 / 7.5 (12 parts; 4: 9.4, 32: 8.8), 100 atoms 16.2 / 10.4 (12; 32: 14.1), 300 atoms 16.4 / 12.2 (3; 12: 13.3), 600 atoms 18.7 / 18.2 (3), 3000
+// atoms 42.8 (one); 64 stacks: 1536 atoms 24.9 / 20.4 (2); 32 stacks, two transforms: 21 atoms 12.8 / 7.9 (4), 1200 atoms 21.1 / 19.4 (2); 32 stacks: 300
+// atoms 10.2 / 8.6 (2 or 3); 8 stacks: one; 256 components, 128 stacks: 21 atoms 33.6 / 9.9 (12).
+// Not more energies (nslots of them a part) than a fill beside the sort hides.
+extern "C" int qmll_sorf_energy_parts_count(int A, int ne, int d, int S, int T, int nslots) {
+    if (A <= 0 || ne <= 0 || S <= 0 || T <= 0 || nslots <= 0 || d < 64 || d > 256 || !qmll_is_pow2(d)) return 1;
+    const long long tiles = ((long long)A + ROWS_NA - 1) / ROWS_NA + ne, load = d == 256 ? 2 * tiles : tiles;
+    long long p = load <= 40 ? 12 : load <= 200 ? 3 : load <= 600 ? 2 : 1;
+    p = std::min(p, (long long)(S / 8));
+    p = std::min(p, 16384ll / nslots);
+    return (int)std::max(1ll, p);
+}
+
+extern "C" int qmll_sorf_energy_parts(const float* x, const int* type_offsets, const int* sorted_slots, const float* D,
+                                      const float* bias, const float* alpha, const float* bias_absmax, int A, int ne, int d,
+                                      int S, int T, float normalisation, int nparts, float* e_parts, int nslots, float* gx_parts,
+                                      qmll_stream_t stream) {
+    int rc = check_sorf("qmll_sorf_energy_parts", A, d, S, T);
+    if (rc) return rc;
+    QMLL_REQUIRE(ne > 0 && nparts > 0 && nparts <= 65535 && nslots >= 0, QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_parts: bad size ne=%d nparts=%d nslots=%d", ne, nparts, nslots);
+    QMLL_REQUIRE(d >= 64 && d <= 256, QMLL_ERR_INVALID, "qmll_sorf_energy_parts: d=%d is not 64, 128 or 256", d);
+    if (A == 0) return QMLL_OK;
+    QMLL_REQUIRE(x && type_offsets && sorted_slots && D && bias && alpha && e_parts, QMLL_ERR_INVALID,
+                 "qmll_sorf_energy_parts: null pointer");
+    const float scale = normalisation * hnorm(d, T), normf = sqrtf(2.0f / ((float)S * (float)d));
+    const dim3 grid(rows_tiles(A, ne), nparts);
+    auto launch = [&](auto log2d, auto grad, auto multi) {
+        hipLaunchKernelGGL((sorf_energy_parts_kernel<decltype(log2d)::value, decltype(grad)::value, decltype(multi)::value>), grid,
+                           dim3(SORF_THREADS), 0, (hipStream_t)stream, x, D, bias, alpha, bias_absmax, sorted_slots, type_offsets, ne, A,
+                           S, T, scale, normf, e_parts, (size_t)nslots, gx_parts);
+    };
+    auto by_transforms = [&](auto log2d, auto grad) {
+        if (T == 1) launch(log2d, grad, std::false_type{});
+        else launch(log2d, grad, std::true_type{});
+    };
+    auto by_grad = [&](auto log2d) {
+        if (gx_parts) by_transforms(log2d, std::true_type{});
+        else by_transforms(log2d, std::false_type{});
+    };
+    switch (qmll_log2(d)) {
+        case 6: by_grad(std::integral_constant<int, 6>{}); break;
+        case 7: by_grad(std::integral_constant<int, 7>{}); break;
+        default: by_grad(std::integral_constant<int, 8>{}); break;
+    }
+    QMLL_CHECK_LAUNCH("qmll_sorf_energy_parts");
+    return QMLL_OK;
 }
 
 int qmll_sorf_rows_if(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,

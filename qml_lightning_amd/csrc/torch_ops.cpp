@@ -563,9 +563,10 @@ Tensor project_typed(const Tensor& rep, const Tensor& ss, const Tensor& off, con
 }
 
 // the fused SORF kernel on rows x f32 [A,d] of a model (ne elements): shape checks of the model's tensors and the launch;
-// e f32 [nslots] zero-filled, gx f32 [A,d] or nullptr
+// e f32 [nslots] zero-filled, gx f32 [A,d] or nullptr; nparts of both where the caller adds the parts (sorf_parts)
 void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A, int d_x, int ne_off, const Tensor& Dmat,
-                            const Tensor& bias, const Tensor& alpha, const Tensor& cn, const Tensor& nt, float* e, float* gx) {
+                            const Tensor& bias, const Tensor& alpha, const Tensor& cn, const Tensor& nt, float* e, float* gx,
+                            int nparts = 1, int64_t nslots = 0) {
     Tensor DD = f32(Dmat), bb = f32(bias), al = alpha32(alpha);
     need_cuda(DD, "Dmat");
     TORCH_CHECK(DD.dim() == 4, "sorf_energy_sorted: Dmat is [", DD.sizes(), "], expected [elements, transforms, stacks, d]");
@@ -589,9 +590,24 @@ void sorf_energy_sorted_raw(const float* x, const int* off, const int* ss, int A
     // the largest |bias|, a constant of the model: computed once per tensor version, kept on the device (in a graph, where a
     // reduction of the library may record a memset, the kernel does without)
     Tensor bmax = prepared_form(bb, 2, [](const Tensor& b) { return capturing() ? Tensor() : b.abs().max().reshape({1}); });
+    if (nparts > 1) {
+        check(qmll_sorf_energy_parts(x, off, ss, fp(DD), fp(bb), fp(al), fp(bmax), A, ne, d, S, T, scalar(cn), nparts, e, (int)nslots,
+                                     A ? gx : nullptr, stream()),
+              "qmll_sorf_energy_parts");
+        return;
+    }
     check(qmll_sorf_energy_sorted(x, off, ss, fp(DD), fp(bb), fp(al), fp(bmax), A, ne, d, S, T, scalar(cn), e, A ? gx : nullptr,
                                   stream()),
           "qmll_sorf_energy_sorted");
+}
+
+// the number of parts of the stacks for sorf_energy_sorted_raw (1 where the matrix cores take the call, and for shapes that
+// it will refuse)
+int sorf_parts(const Tensor& Dmat, int A, int64_t nslots, bool with_grad) {
+    if (Dmat.dim() != 4 || nslots > (1 << 30)) return 1;
+    const int ne = (int)Dmat.size(0), T = (int)Dmat.size(1), S = (int)Dmat.size(2), d = (int)Dmat.size(3);
+    if (qmll_sorf_matrix_pays(A, ne, T, S, d, with_grad)) return 1;
+    return qmll_sorf_energy_parts_count(A, ne, d, S, T, (int)nslots);
 }
 
 // e_zeroed: the caller's zero-filled f32 [nslots] for the energies (one fill then serves several outputs), or undefined
@@ -756,20 +772,22 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
     int* ss = types + types_ints;
     int* off = ss + A;
     int* sort_work = off + ne + 1;
-    const int64_t nzero = (with_grad ? 4 : 1) * nslots;
+    // the gradient first: what follows it is one energy per slot, or as many as the SORF call has parts
+    const int nparts = rff ? 1 : sorf_parts(Dmat, A, nslots, with_grad);
+    const int64_t ngrad = with_grad ? 3 * nslots : 0, nzero = ngrad + nparts * nslots;
     Tensor out = at::empty({nzero}, in.X.options());
-    float* e_slots = nzero ? out.data_ptr<float>() : nullptr;
+    float* e_slots = nzero ? out.data_ptr<float>() + ngrad : nullptr;
     check(qmll_prepare_batch(fp(Zb), ip(in.natoms), fp(sp), in.prm.nspecies, fp(msp), ne, ip(in.atomIDs), ip(in.molIDs), B, n,
-                             A, sort_work, sort_bytes, types, own_list ? sort_types : nullptr, ss, off, e_slots,
-                             (size_t)nzero, stream()),
+                             A, sort_work, sort_bytes, types, own_list ? sort_types : nullptr, ss, off,
+                             nzero ? out.data_ptr<float>() : nullptr, (size_t)nzero, stream()),
           "qmll_prepare_batch");
     auto pad = [](int64_t v) { return (v + 63) / 64 * 64; };          // every part 256-byte aligned
-    const int64_t rep_n = pad(nslots * R), x_n = pad((int64_t)A * d);
-    Tensor scratch = at::empty({rep_n + x_n + (with_grad ? x_n + rep_n : 0) + 64}, in.X.options());
+    const int64_t rep_n = pad(nslots * R), x_n = pad((int64_t)A * d), gx_n = pad((int64_t)A * d * nparts);
+    Tensor scratch = at::empty({rep_n + x_n + (with_grad ? gx_n + rep_n : 0) + 64}, in.X.options());
     float* rep = scratch.data_ptr<float>();
     float* x = rep + rep_n;
     float* gx = with_grad ? x + x_n : nullptr;
-    float* g_rep = with_grad ? gx + x_n : nullptr;
+    float* g_rep = with_grad ? gx + gx_n : nullptr;
     // the forward kernel writes every bin of a listed atom's row, and only the rows of listed
     // atoms are read below, so the padded rows need no clearing
     check(qmll_fchl19_forward(FCHL_ABI_T(in, types), rep, stream()), "qmll_fchl19_forward");
@@ -778,20 +796,20 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
     if (rff)
         rff_energy_sorted_raw(x, off, ss, A, d, ne, Dmat, bias, alpha, e_slots, gx);
     else
-        sorf_energy_sorted_raw(x, off, ss, A, d, ne, Dmat, bias, alpha, cn, nt, e_slots, gx);
+        sorf_energy_sorted_raw(x, off, ss, A, d, ne, Dmat, bias, alpha, cn, nt, e_slots, gx, nparts, nslots);
     Tensor energies = at::empty({B}, in.X.options());
     if (!with_grad) {        // the sums alone (A = 0), by the kernel that sums them beside the backward projection
-        check(qmll_project_typed_backward_sums(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, ne, R, d, nullptr,
-                                               e_slots, B, n, B ? energies.data_ptr<float>() : nullptr, stream()),
-              "qmll_project_typed_backward_sums");
+        check(qmll_project_typed_backward_parts(nullptr, nparts, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, ne, R, d, nullptr,
+                                                e_slots, B, n, B ? energies.data_ptr<float>() : nullptr, stream()),
+              "qmll_project_typed_backward_parts");
         return energies;
     }
     // rows of listed atoms whose element the model does not hold are zeroed (sort_types); the rows of
     // padded slots are never read by the kernel below
-    check(qmll_project_typed_backward_sums(gx, ss, off, fp(red), vp(split), sort_types, A, (int)nslots, ne, R, d, g_rep,
-                                           e_slots, B, n, B ? energies.data_ptr<float>() : nullptr, stream()),
-          "qmll_project_typed_backward_sums");
-    Tensor gX = out.narrow(0, nslots, 3 * nslots).view({B, n, 3});
+    check(qmll_project_typed_backward_parts(gx, nparts, ss, off, fp(red), vp(split), sort_types, A, (int)nslots, ne, R, d, g_rep,
+                                            e_slots, B, n, B ? energies.data_ptr<float>() : nullptr, stream()),
+          "qmll_project_typed_backward_parts");
+    Tensor gX = out.narrow(0, 0, 3 * nslots).view({B, n, 3});
     check(qmll_fchl19_vjp_scaled(FCHL_ABI_T(in, types), g_rep, gscale, nslots ? gX.data_ptr<float>() : nullptr, stream()),
           "qmll_fchl19_vjp");
     *gX_out = gX;

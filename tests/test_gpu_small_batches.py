@@ -1,0 +1,88 @@
+"""The kernels of small batches: SORF energies with the stacks in parts, and both small projections at the edges of their rule."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev():
+    return torch.device("cuda:0")
+
+
+def _model(A, ne, d, S, T, seed):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    types = torch.randint(0, ne + 1, (A,), generator=g).int()                 # the last of them is no element of the model
+    x = torch.randn(A, d, generator=g)
+    D = torch.sign(torch.rand(ne, T, S, d, generator=g) - 0.5)
+    bias = torch.rand(ne, S * d, generator=g) * 6.28
+    alpha = torch.randn(S * d, generator=g)
+    return [t.to(dev()) for t in (types, x, D, bias, alpha)]
+
+
+# one and several tiles, more parts than wavefront rounds of stacks (empty parts), both directions of the diagonal's fetch
+@pytest.mark.parametrize("A,ne,d,S,T,nparts", [(1, 1, 64, 8, 1, 2), (21, 3, 128, 128, 1, 12), (50, 4, 256, 20, 1, 3), (33, 2, 128, 6, 1, 5),
+                                               (21, 3, 64, 32, 2, 4), (130, 4, 256, 9, 2, 2)])
+@pytest.mark.parametrize("grad", [True, False])
+def test_parts_of_the_stacks_add_up(A, ne, d, S, T, nparts, grad):
+    from qml_lightning_amd import _lib, ops
+    from qml_lightning_amd.ops import _ptr, _stream
+    L = _lib.lib()
+    types, x, D, bias, alpha = _model(A, ne, d, S, T, A)
+    ss, off = ops.sort_by_type(types, torch.arange(A, dtype=torch.int32, device=dev()), ne)
+    bmax = bias.abs().max().reshape(1)
+
+    def run(n):
+        e = torch.zeros(n, A, device=dev())
+        gx = torch.full((n, A, d), 3.0, device=dev()) if grad else None
+        args = (_ptr(x), _ptr(off), _ptr(ss), _ptr(D), _ptr(bias), _ptr(alpha), _ptr(bmax), A, ne, d, S, T, 0.3)
+        rc = L.qmll_sorf_energy_parts(*args, n, _ptr(e), A, _ptr(gx), _stream()) if n > 1 else \
+            L.qmll_sorf_energy_sorted(*args, _ptr(e), _ptr(gx), _stream())
+        assert rc == 0, _lib.last_error()
+        return e.double().sum(0), None if gx is None else gx.double().sum(0)
+
+    (e1, g1), (en, gn) = run(1), run(nparts)
+    # the same features in another grouping: sums of S d terms of at most |alpha| norm each, rounded to fp32
+    terms = float(alpha.abs().max()) * np.sqrt(2.0 / (S * d)) * np.sqrt(S * d) * 2.0 ** -24
+    assert float((en - e1).abs().max()) <= 16 * terms * np.sqrt(S * d)
+    if grad:
+        assert float((gn - g1).abs().max()) <= 16 * terms * np.sqrt(S * d) * np.sqrt(d) * 0.3
+        known = int(off[ne])
+        assert (gn[known:] == 0).all()
+
+
+# 32 columns of one, two and four atoms, 128 columns of four, 32 of eight, partial columns; with parts, and with more atoms than
+# the small kernels take
+@pytest.mark.parametrize("A,ne,R,d", [(1, 1, 168, 64), (30, 3, 312, 128), (200, 3, 312, 128), (700, 2, 168, 128), (1500, 3, 312, 128),
+                                      (3000, 5, 720, 64), (600, 4, 496, 256), (40, 2, 168, 100), (4200, 3, 312, 128)])
+@pytest.mark.parametrize("nparts", [1, 3])
+def test_small_projections(A, ne, R, d, nparts):
+    from qml_lightning_amd import _lib, ops
+    from qml_lightning_amd.ops import _ptr, _stream
+    L = _lib.lib()
+    g = torch.Generator(device="cpu").manual_seed(R + A)
+    types = torch.randint(0, ne + 1, (A,), generator=g).int().to(dev())
+    ss, off = ops.sort_by_type(types, torch.arange(A, dtype=torch.int32, device=dev()), ne)
+    known = int(off[ne])
+    rep, U = torch.randn(A, R, generator=g).to(dev()), torch.randn(ne, R, d, generator=g).to(dev())
+    gx = torch.randn(nparts, A, d, generator=g).to(dev())
+    n = 1 if A % 3 else 3
+    e = torch.randn(nparts, A, generator=g).to(dev())
+    total, e_total = gx.double().sum(0), e.double().sum(0).view(-1, n).sum(1)
+    x = torch.full((A, d), 9.0, device=dev())
+    assert L.qmll_project_typed(_ptr(rep), _ptr(ss), _ptr(off), _ptr(U), None, A, ne, R, d, _ptr(x), _stream()) == 0
+    g_rep = torch.full((A, R), 9.0, device=dev())
+    energies = torch.empty(A // n, device=dev())
+    rc = L.qmll_project_typed_backward_parts(_ptr(gx), nparts, _ptr(ss), _ptr(off), _ptr(U), None, _ptr(types), A, A, ne, R, d, _ptr(g_rep),
+                                             _ptr(e), A // n, n, _ptr(energies), _stream())
+    assert rc == 0, _lib.last_error()
+    slots = ss[:known].long()
+    for t in range(ne):
+        a, b = int(off[t]), int(off[t + 1])
+        rows, back = rep[slots[a:b]].double() @ U[t].double(), total[a:b] @ U[t].double().T
+        # fp32 sums of R (d) products
+        assert float((x[a:b] - rows).abs().max()) <= 4 * R ** 0.5 * 2.0 ** -24 * float(rows.abs().max()) if b > a else True
+        assert float((g_rep[slots[a:b]] - back).abs().max()) <= 4 * (d + nparts) ** 0.5 * 2.0 ** -24 * float(back.abs().max()) if b > a else True
+    unknown = (types >= ne).nonzero()[:, 0]
+    assert (g_rep[unknown] == 0).all()
+    assert float((energies - e_total).abs().max()) <= 4 * nparts * n * 2.0 ** -24 * float(e.abs().max())
