@@ -98,6 +98,7 @@ PROTOTYPES = {
     "qmll_gram_modular_f64": [P, P, c_int, c_int, P, P, P, c_size_t, P],
     "qmll_gram_mirror_f64": [P, c_int, P],
     "qmll_cholesky_workspace_bytes": [c_int],
+    "qmll_copy_upper_f64": [P, c_longlong, c_int, P, c_longlong, P],
     "qmll_cholesky_f64": [P, c_int, c_longlong, P, P, P],
     "qmll_cholesky_solve_f64": [P, c_int, c_longlong, P, P, P],
     "qmll_gram_tile_f64": [P, P, c_int, c_int, c_int, c_int, P, P, P],

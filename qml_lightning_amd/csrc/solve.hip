@@ -653,7 +653,7 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
                                                        unsigned spin_limit) {
     __shared__ double part[SQ][NB], vec[NB];
     const int k = nblk - 1 - (int)blockIdx.x, k0 = k * NB;
-    const int tid = threadIdx.x, c = tid & (NB - 1), q = tid / NB;
+    const int tid = threadIdx.x, lane = tid & 63, c = tid & (NB - 1), q = tid / NB;
     const int csub = tid & 15, rowgrp = tid >> 4;          // sixteen lanes of eight columns along a row; rows rowgrp + 32 a
     const double* invT = invs + (size_t)k * 2 * NB * NB + NB * NB;
     double iv[SR];
@@ -671,25 +671,20 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
 #pragma unroll
             for (int e = 0; e < 8; ++e) u[a][e] = col0 + e < F ? row[e] : 0.0;
         }
-        unsigned long long bits[8];
-        bool pending = false;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            bits[e] = peek(xs + col0 + e);
-            pending |= bits[e] == NOT_YET;
-        }
-        for (unsigned n = 0; __builtin_amdgcn_ballot_w64(pending) != 0ULL && n < spin_limit; ++n) {
+        // every wavefront polls the block's 128 values, two a lane, and hands each lane its eight (a lane that polled all it
+        // needs itself took eight loads a poll, and the launch 1.18 ms at 16384 features instead of BWD_NOW)
+        const double* theirs = xs + j * NB + 2 * lane;
+        unsigned long long b0 = peek(theirs), b1 = peek(theirs + 1);
+        for (unsigned n = 0; __builtin_amdgcn_ballot_w64(b0 == NOT_YET || b1 == NOT_YET) != 0ULL && n < spin_limit; ++n) {
             __builtin_amdgcn_s_sleep(4);
-            pending = false;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                bits[e] = peek(xs + col0 + e);
-                pending |= bits[e] == NOT_YET;
-            }
+            b0 = peek(theirs);
+            b1 = peek(theirs + 1);
         }
+        const double x0 = b0 == NOT_YET ? __builtin_nan("") : __longlong_as_double((long long)b0);
+        const double x1 = b1 == NOT_YET ? __builtin_nan("") : __longlong_as_double((long long)b1);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const double xv = bits[e] == NOT_YET ? __builtin_nan("") : __longlong_as_double((long long)bits[e]);
+            const double xv = __shfl(e & 1 ? x1 : x0, 4 * csub + (e >> 1), 64);
 #pragma unroll
             for (int a = 0; a < 4; ++a) acc[a] = fma(-u[a][e], xv, acc[a]);
         }
@@ -711,6 +706,24 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
 __global__ __launch_bounds__(256) void fill_words64_kernel(unsigned long long* p, int n, unsigned long long v) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+// the 128 x 128 tiles on or above the diagonal of A into U (the lower ones are never read); grid (column, row of tiles)
+__global__ __launch_bounds__(256) void copy_upper_kernel(const double* __restrict__ A, long long lda, double* __restrict__ U,
+                                                         long long ldu, int F) {
+    if (blockIdx.x < blockIdx.y) return;
+    const int c = blockIdx.x * NB + (threadIdx.x & 63) * 2, r0 = blockIdx.y * NB + (threadIdx.x >> 6);
+    const bool pairs = c + 1 < F && (lda | ldu) % 2 == 0 && ((uintptr_t)A | (uintptr_t)U) % 16 == 0;
+#pragma unroll 8
+    for (int r = r0; r < min(F, (int)(blockIdx.y + 1) * NB); r += 4) {
+        const double* from = A + (size_t)r * lda + c;
+        double* to = U + (size_t)r * ldu + c;
+        if (pairs) *reinterpret_cast<double2_t*>(to) = *reinterpret_cast<const double2_t*>(from);
+        else {
+            if (c < F) to[0] = from[0];
+            if (c + 1 < F) to[1] = from[1];
+        }
+    }
 }
 
 }  // namespace
@@ -790,6 +803,16 @@ int factor_block(double* A, int F, long long ld, int P0, int k0, double* invs, i
 }
 
 }  // namespace
+
+extern "C" int qmll_copy_upper_f64(const double* A, long long lda, int F, double* U, long long ldu, qmll_stream_t stream) {
+    QMLL_REQUIRE(F > 0 && lda >= F && ldu >= F, QMLL_ERR_INVALID, "qmll_copy_upper_f64: bad size F=%d lda=%lld ldu=%lld", F, lda, ldu);
+    QMLL_REQUIRE(A && U, QMLL_ERR_INVALID, "qmll_copy_upper_f64: null pointer");
+    const unsigned n = ((unsigned)F + NB - 1) / NB;
+    QMLL_REQUIRE(n <= 65535, QMLL_ERR_INVALID, "qmll_copy_upper_f64: F=%d too large", F);
+    hipLaunchKernelGGL(copy_upper_kernel, dim3(n, n), dim3(256), 0, (hipStream_t)stream, A, lda, U, ldu, F);
+    QMLL_CHECK_LAUNCH("qmll_copy_upper_f64");
+    return QMLL_OK;
+}
 
 extern "C" int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace, int* info, qmll_stream_t stream_) {
     hipStream_t stream = (hipStream_t)stream_;

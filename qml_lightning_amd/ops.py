@@ -812,10 +812,15 @@ def cholesky_solve_spd(A, b, overwrite_a=False):
     F = int(A.shape[0])
     if b.dtype != torch.float64 or b.numel() != F:
         raise RuntimeError("cholesky_solve_spd: b must hold F float64 values")
-    U = A if overwrite_a else A.clone()
+    U = A if overwrite_a else torch.empty_like(A)
     ld = int(U.stride(0))
     if ld % 2 != 0:
         raise RuntimeError("cholesky_solve_spd: the row stride must be even")
+    if not overwrite_a:
+        if int(A.stride(0)) >= F:
+            check(_lib.lib().qmll_copy_upper_f64(_ptr(A), int(A.stride(0)), F, _ptr(U), ld, _stream()), "qmll_copy_upper_f64")
+        else:
+            U.copy_(A)                          # rows that overlap
     L = _lib.lib()
     work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device=A.device)
     info = torch.zeros(1, dtype=torch.int32, device=A.device)
