@@ -672,7 +672,7 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
             for (int e = 0; e < 8; ++e) u[a][e] = col0 + e < F ? row[e] : 0.0;
         }
         // every wavefront polls the block's 128 values, two a lane, and hands each lane its eight (a lane that polled all it
-        // needs itself took eight loads a poll, and the launch 1.18 ms at 16384 features instead of BWD_NOW)
+        // needs itself took eight loads a poll, and the launch 1.18 ms at 16384 features instead of 0.72)
         const double* theirs = xs + j * NB + 2 * lane;
         unsigned long long b0 = peek(theirs), b1 = peek(theirs + 1);
         for (unsigned n = 0; __builtin_amdgcn_ballot_w64(b0 == NOT_YET || b1 == NOT_YET) != 0ULL && n < spin_limit; ++n) {
