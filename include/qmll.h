@@ -561,6 +561,11 @@ int qmll_copy_upper_f64(const double* A, long long lda, int F, double* U, long l
  * (hipMalloc; what torch allocates), not in host-mapped or managed memory. */
 int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace, int* info, qmll_stream_t stream);
 
+/* The same with qmll_cholesky_slabs_bytes(F) of device memory more (16-byte aligned, or NULL): large matrices whose F is a multiple of
+ * 128 then take the updates by their first rows as exact int8 products.  0 bytes: there are no such rows, NULL is as good. */
+size_t qmll_cholesky_slabs_bytes(int F);
+int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* workspace, void* slabs, int* info, qmll_stream_t stream);
+
 /* b <- (U^T U)^-1 b for one right-hand side b[F], U and workspace from qmll_cholesky_f64.  One launch per
  * direction, a workgroup per 128-row block; the blocks wait for one another's results with bounded waits,
  * and one that runs out (never seen) leaves NaN in b rather than a wrong number.  Calls that share a

@@ -99,6 +99,8 @@ PROTOTYPES = {
     "qmll_gram_mirror_f64": [P, c_int, P],
     "qmll_cholesky_workspace_bytes": [c_int],
     "qmll_copy_upper_f64": [P, c_longlong, c_int, P, c_longlong, P],
+    "qmll_cholesky_slabs_bytes": [c_int],
+    "qmll_cholesky_slabs_f64": [P, c_int, c_longlong, P, P, P, P],
     "qmll_cholesky_f64": [P, c_int, c_longlong, P, P, P],
     "qmll_cholesky_solve_f64": [P, c_int, c_longlong, P, P, P],
     "qmll_gram_tile_f64": [P, P, c_int, c_int, c_int, c_int, P, P, P],
@@ -110,7 +112,8 @@ PROTOTYPES = {
     "qmll_probe_mix": [c_int, c_int, c_int, P, P],
 }
 _RESTYPES = {"qmll_last_error": c_char_p, "qmll_sorf_signs_bytes": c_size_t, "qmll_rff_presplit_bytes": c_size_t, "qmll_rff_energy_workspace_bytes": c_size_t, "qmll_sorf_matrix_workspace_bytes": c_size_t, "qmll_reductor_presplit_bytes": c_size_t, "qmll_sort_by_type_workspace": c_size_t, "qmll_sort_atoms_workspace": c_size_t,
-             "qmll_cholesky_workspace_bytes": c_size_t, "qmll_gram_workspace_bytes": c_size_t, "qmll_gram_modular_workspace_bytes": c_size_t,
+             "qmll_cholesky_workspace_bytes": c_size_t, "qmll_cholesky_slabs_bytes": c_size_t,
+             "qmll_gram_workspace_bytes": c_size_t, "qmll_gram_modular_workspace_bytes": c_size_t,
              "qmll_probe_out_bytes": c_size_t, "qmll_probe_rate": c_double,
              "qmll_probe_mix": c_double}
 

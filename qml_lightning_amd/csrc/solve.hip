@@ -15,8 +15,8 @@
 // For whole tiles (F a multiple of 128) a panel and the trailing update of the panel before it are ONE
 // launch (panel_kernel below); any other F takes a launch per step with the tile kernel of gram.hip.
 // Only elements on or above the diagonal are read; below the diagonal only the lower halves of
-// the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.  Large matrices take the update of what is below a slab of
-// 4096 rows in one piece from the int8 matrix cores (slab_end below).
+// the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.  Large matrices take the updates by all rows
+// but the last few thousand from the int8 matrix cores (slab_end below).
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -28,10 +28,14 @@
 // of n columns with row stride ldz
 int qmll_internal_syrk_upper(const double* Z, int M, int n, long long ldz, double* C, long long ldc, double sign,
                              hipStream_t stream);
-// gram_modular.hip: C[F,F] (row stride ldc, tiles on or above the diagonal) += sign Z^T Z, and the workspace it takes
-int qmll_internal_modular_syrk(const double* Z, long long ldz, const double* y, int M, int F, double* C, long long ldc, double sign,
-                               double* ZTy, void* workspace, const char* who, hipStream_t stream);
-size_t qmll_internal_modular_bytes(int M, int F);
+// gram_modular.hip: a slab of `rows` rows of the factor and the n columns from its first diagonal entry on (A): scales, the
+// residues of rows that are final, the update of what is behind i0 by the slab's first k rows
+size_t qmll_internal_slab_bytes(int rows, int n);
+int qmll_internal_slab_begin(const double* A, long long ld, int rows, int n, void* workspace, const char* who, hipStream_t stream);
+int qmll_internal_slab_rows(const double* A, long long ld, int rows, int n, int k0, int m, int f0, void* workspace, const char* who,
+                            hipStream_t stream);
+int qmll_internal_slab_update(double* A, long long ld, int rows, int n, int k, int i0, int band, void* workspace, const char* who,
+                              hipStream_t stream);
 
 // gram.hip: C[ra,n] = or += sign * Za^T Zb, Za = M x ra (row stride lda), Zb = M x n (row stride ldb)
 int qmll_internal_gemm_tn(const double* Za, long long lda, int ra, const double* Zb, long long ldb, int n, int M,
@@ -360,7 +364,7 @@ constexpr int P_UN = P_CPT / 2;         // 16-byte units per thread
 constexpr unsigned FLAG_DONE = 1u, FLAG_FAILED = 0x80000000u;   // (a counter never gets near the second)
 constexpr int PBLK = OB / NB;                        // blocks per panel
 constexpr int FLAGS_PER_PANEL = PBLK + PBLK * PBLK;  // "block l factored": [l]; "strip (l, b) done": [PBLK + l PBLK + b]
-constexpr int SPLIT_HEADS_BELOW = 48 * 49 / 2;       // trailing tiles
+constexpr int SPLIT_HEADS_BELOW = 48;       // trailing tiles per edge
 constexpr unsigned SPIN_LIMIT = 1u << 21;   // polls of about a microsecond each before a wait gives up
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
@@ -482,7 +486,7 @@ __device__ __forceinline__ unsigned await(unsigned* flag, unsigned target, unsig
 // then nown_pad ids for the column owners, then the tiles of the trailing matrix below this panel, nt per edge
 // (0: none).  flags: FLAGS_PER_PANEL words, then one counter per column (head tiles done), all zero.
 __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, int F, int R0, int P0, int nblk,
-                                                      int nhead_pad, int nown, int nown_pad, int ntr, int nt, TileMap tm,
+                                                      int nhead_pad, int nown, int nown_pad, int nt, TileMap tm,
                                                       double* invs, int* info, unsigned* flags, unsigned spin_limit) {
     // the tile product and the factorisation never run at the same time: one piece of LDS for both, which
     // is what lets two workgroups share a CU (2 x 74 KB)
@@ -517,8 +521,7 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
     bid -= nhead_pad;
     if (bid >= nown_pad) {                                   // a tile of the trailing matrix
         int ti, tj;
-        if (ntr == nt) tile_of_block<true>((unsigned)(bid - nown_pad), nt, nt, tm, ti, tj);
-        else tile_of_block<false>((unsigned)(bid - nown_pad), ntr, nt, tm, ti, tj);
+        tile_of_block<true>((unsigned)(bid - nown_pad), nt, nt, tm, ti, tj);
         if (ti < 0 || ti > tj) return;
         const int Q = P0 + nblk * NB;
         const int i0 = Q + ti * NB, c0 = Q + tj * NB;
@@ -732,22 +735,25 @@ __global__ __launch_bounds__(256) void copy_upper_kernel(const double* __restric
 // exchange copy of x of the backward solve (whole blocks each), and the flags of the panel launches (per panel:
 // FLAGS_PER_PANEL + one counter per block column)
 namespace {
-// Slabs of 4096 rows while at least 8192 rows are left below: the panels of a slab update the slab's own rows only, and what
-// is below the slab takes one update 4096 deep from the int8 matrix cores (gram_modular.hip), which at that depth run at
-// more than twice the fp64 rate (4.2 ms for the 12288 columns below the first slab of 16384, 9.6 ms as part of the panels'
-// launches).  The last 8192 and more rows keep their fp64 updates, which hide behind the chain of the panels.
-// 16384 features, factorisation and solves: 34.1 ms without slabs, 30.7 / 28.9 / 28.5 / 29.6 with 2048 / 3072 / 4096 / 6144 rows;
-// 12288 features: 18.3 and 17.5 / 17.0 / 16.9 / 17.2.
-constexpr int SLAB = 4096, SLAB_REST = 8192;
+// Slabs: while more than 4096 rows are left, the rows of the factor above them act on the rest through exact int8 products
+// (gram_modular.hip), before each panel of 512 rows on the panel's own rows only and at a slab's end on everything below it, so that
+// the matrix is read and written once per slab and not once per panel.  In the last 4096 rows the panel launches of fp64 products
+// are as fast, which are short there and wait for their chain of factorisations.  Up to 12288 rows a slab (15 bytes an entry
+// for the residues, 3 GB at 16384 features); below 7168 features there is nothing to gain.  ms without slabs and with:
+// 24576 features 90.5 / 57.2, 16384 32.8 / 25.4, 10240 12.6 / 11.9, 8192 8.86 / 8.54, 7168 7.31 / 7.19, 6144 5.95 / 5.93, 5120
+// 4.66 / 4.70; slabs of 4096 rows 28.3 at 16384; a rest of 8192 rows 26.7 there and, at 10240, 12.9 against 12.0.
+constexpr int SLAB = 12288, SLAB_REST = 4096, SLAB_LEAST = 3072;
 // end of the slab of rows that starts at s0
-int slab_end(int s0, int F) { return F - s0 - SLAB >= SLAB_REST ? s0 + SLAB : F; }
+int slab_end(int s0, int F) {
+    const int below = (F - s0 - SLAB_REST) / OB * OB;          // rows that may go into slabs
+    return below >= SLAB_LEAST ? s0 + std::min(SLAB, below) : F;
+}
 
 struct Workspace {
     double* invs;
     double* z;
     double* xs;
     unsigned* panel_flags;
-    void* slab;          // workspace of the slabs' updates
     size_t nblk, npanel, bytes;
 };
 Workspace workspace_layout(void* base, int F) {
@@ -760,16 +766,6 @@ Workspace workspace_layout(void* base, int F) {
     w.panel_flags = reinterpret_cast<unsigned*>(w.xs + w.nblk * NB);
     w.bytes = (w.nblk * 2 * NB * NB + 2 * w.nblk * NB) * sizeof(double) +
               w.npanel * (FLAGS_PER_PANEL + w.nblk) * sizeof(unsigned) + 256;
-    if (F % NB == 0 && slab_end(0, F) < F) {
-        w.bytes = (w.bytes + 1023) / 1024 * 1024;
-        w.slab = reinterpret_cast<char*>(base) + w.bytes;
-        size_t most = 0;
-        for (int s0 = 0, s1 = slab_end(0, F); s1 < F; s0 = s1, s1 = slab_end(s0, F))
-            most = std::max(most, qmll_internal_modular_bytes(s1 - s0, F - s1));
-        w.bytes += most;
-    } else {
-        w.slab = nullptr;
-    }
     return w;
 }
 }  // namespace
@@ -777,6 +773,14 @@ Workspace workspace_layout(void* base, int F) {
 extern "C" size_t qmll_cholesky_workspace_bytes(int F) {
     if (F <= 0) return 0;
     return workspace_layout(nullptr, F).bytes;
+}
+
+extern "C" size_t qmll_cholesky_slabs_bytes(int F) {
+    if (F <= 0 || F % NB != 0) return 0;
+    size_t most = 0;
+    for (int s0 = 0, s1 = slab_end(0, F); s1 < F; s0 = s1, s1 = slab_end(s0, F))
+        most = std::max(most, qmll_internal_slab_bytes(s1 - s0, F - s0));
+    return most;
 }
 
 namespace {
@@ -814,13 +818,19 @@ extern "C" int qmll_copy_upper_f64(const double* A, long long lda, int F, double
     return QMLL_OK;
 }
 
-extern "C" int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace, int* info, qmll_stream_t stream_) {
+extern "C" int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace, int* info, qmll_stream_t stream) {
+    return qmll_cholesky_slabs_f64(A, F, ld, workspace, nullptr, info, stream);
+}
+
+extern "C" int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* workspace, void* slabs, int* info, qmll_stream_t stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     QMLL_REQUIRE(F > 0 && ld >= F, QMLL_ERR_INVALID, "qmll_cholesky_f64: bad size F=%d ld=%lld", F, ld);
     QMLL_REQUIRE(ld < (1LL << 23), QMLL_ERR_INVALID, "qmll_cholesky_f64: row stride %lld too large", ld);
     QMLL_REQUIRE(A && workspace && info, QMLL_ERR_INVALID, "qmll_cholesky_f64: null pointer");
     QMLL_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, QMLL_ERR_INVALID,
                  "qmll_cholesky_f64: the workspace must be 16-byte aligned");
+    QMLL_REQUIRE(reinterpret_cast<uintptr_t>(slabs) % 16 == 0, QMLL_ERR_INVALID,
+                 "qmll_cholesky_f64: the slabs' workspace must be 16-byte aligned");
     const Workspace ws = workspace_layout(workspace, F);
     double* invs = ws.invs;
     // whole tiles and 16-byte loads: one launch per panel, which also carries the trailing update of the panel
@@ -832,39 +842,48 @@ extern "C" int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace
         const int nflags = (F + OB - 1) / OB * per_panel;
         hipLaunchKernelGGL(zero_words_kernel, dim3((nflags + 255) / 256), dim3(256), 0, stream, flags, nflags);
         QMLL_CHECK_LAUNCH("qmll_cholesky_f64");
-        int S0 = 0, S1 = slab_end(0, F);                      // rows of this slab
+        const char* who = "qmll_cholesky_f64";
+        int S0 = 0, S1 = slabs ? slab_end(0, F) : F;          // rows of this slab; the last one has S1 = F
         for (int P0 = 0; P0 < F; P0 += OB) {
             const int pend = P0 + OB < F ? P0 + OB : F;       // this panel: rows [P0, pend)
-            if (P0 == S1) {                                   // the slab before is done: its update of everything below it
-                const int rc = qmll_internal_modular_syrk(A + (size_t)S0 * ld + S1, ld, nullptr, S1 - S0, F - S1,
-                                                          A + (size_t)S1 * ld + S1, ld, -1.0, nullptr, ws.slab, "qmll_cholesky_f64",
-                                                          stream);
+            double* slab = A + (size_t)S0 * ld + S0;
+            if (P0 > S0 && S1 < F) {                          // the panel before this one is final
+                int rc = qmll_internal_slab_rows(slab, ld, S1 - S0, F - S0, P0 - OB - S0, OB, P0 - S0, slabs, who, stream);
                 if (rc != QMLL_OK) return rc;
+                // what this panel, or with a slab's last panel everything below, takes from the slab's rows
+                rc = qmll_internal_slab_update(slab, ld, S1 - S0, F - S0, P0 - S0, P0 - S0, P0 < S1 ? OB / 256 : 0, slabs, who, stream);
+                if (rc != QMLL_OK) return rc;
+            }
+            if (P0 == S1) {
                 S0 = S1;
                 S1 = slab_end(S0, F);
+                slab = A + (size_t)S0 * ld + S0;
             }
-            const int R0 = P0 > S0 ? P0 - OB : P0;            // the panel before it in the slab
+            if (P0 == S0 && S1 < F) {
+                const int rc = qmll_internal_slab_begin(slab, ld, S1 - S0, F - S0, slabs, who, stream);
+                if (rc != QMLL_OK) return rc;
+            }
+            // the panel before it, whose update this launch carries: in the last slab only
+            const int R0 = S1 == F && P0 > S0 ? P0 - OB : P0;
             const int nblk = (pend - P0) / NB;
             const int ncol = (F - P0) / NB;                   // columns of tiles from the panel's first to the last
             const int nt = P0 > R0 ? (F - pend) / NB : 0;
-            const int ntr = P0 > R0 ? (S1 - pend) / NB : 0;   // rows of tiles below the panel that take its predecessor's update
-            const int ntrail = ntr * nt - ntr * (ntr - 1) / 2;
             const int nown = ncol;
             // The head tiles (this panel's rows of the update of the panel before) go to workgroups of their own
             // once the trailing matrix is small, where a launch lasts as long as its slowest owner: four head tiles
             // and ten strip / update products in a row, 540 us, against a chain of four factorisations of 390.
             // While the trailing tiles keep the chip busy for longer than that, the owners take their head tiles
             // themselves and no slot waits for another.
-            const bool split_heads = P0 > R0 && ntrail <= SPLIT_HEADS_BELOW;
+            const bool split_heads = P0 > R0 && nt <= SPLIT_HEADS_BELOW;
             const int nown_pad = (nown + NXCD - 1) / NXCD * NXCD;
             const int nhead = split_heads ? nblk * (nblk + 1) / 2 + (ncol - nblk) * nblk : 0;
             const int nhead_pad = (nhead + NXCD - 1) / NXCD * NXCD;
             long long per_xcd = 0;
-            TileMap tm = gram_tile_map(ntr > 0 ? ntr : 1, nt > 0 ? nt : 1, ntr == nt, per_xcd);
-            const long long grid = (long long)nhead_pad + nown_pad + (ntr > 0 ? per_xcd * NXCD : 0);
+            TileMap tm = gram_tile_map(nt > 0 ? nt : 1, nt > 0 ? nt : 1, true, per_xcd);
+            const long long grid = (long long)nhead_pad + nown_pad + (nt > 0 ? per_xcd * NXCD : 0);
             QMLL_REQUIRE(grid < 2147483647LL, QMLL_ERR_INVALID, "qmll_cholesky_f64: too many tiles");
             hipLaunchKernelGGL(panel_kernel, dim3((unsigned)grid), dim3(PT), 0, stream, A, ld, F, R0, P0, nblk, nhead_pad,
-                               nown, nown_pad, ntr, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
+                               nown, nown_pad, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
             QMLL_CHECK_LAUNCH("qmll_cholesky_f64");
         }
         return QMLL_OK;

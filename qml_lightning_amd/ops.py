@@ -825,7 +825,13 @@ def cholesky_solve_spd(A, b, overwrite_a=False):
     work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device=A.device)
     info = torch.zeros(1, dtype=torch.int32, device=A.device)
     x = b.detach().clone().contiguous()
-    check(L.qmll_cholesky_f64(_ptr(U), F, ld, _ptr(work), _ptr(info), _stream()), "qmll_cholesky_f64")
+    slabs, nbytes = None, int(L.qmll_cholesky_slabs_bytes(F))
+    if nbytes:
+        try:
+            slabs = torch.empty(nbytes, dtype=torch.uint8, device=A.device)
+        except torch.cuda.OutOfMemoryError:
+            pass                                # the factorisation does without
+    check(L.qmll_cholesky_slabs_f64(_ptr(U), F, ld, _ptr(work), _ptr(slabs), _ptr(info), _stream()), "qmll_cholesky_f64")
     check(L.qmll_cholesky_solve_f64(_ptr(U), F, ld, _ptr(work), _ptr(x), _stream()), "qmll_cholesky_solve_f64")
     return x, info
 

@@ -131,11 +131,14 @@ def test_modular_gram_in_a_graph_is_the_eager_result():
         assert torch.equal(C, ref), seed
 
 
-def test_factorisation_in_slabs():
-    """12288 features is the smallest matrix whose first 4096 rows are a slab of their own: the residual of the solve within the
-    backward error of a factorisation of that size, a pivot that is not positive and a NaN below the slab reported."""
-    from qml_lightning_amd import ops
-    F = 12288
+# 7168 features: the smallest matrix with a slab (3072 rows); 7296: its columns end within a tile of 256; 12288: 8192 rows;
+# 19456: two slabs, of 12288 and 3072 rows
+@pytest.mark.parametrize("F", [7168, 7296, 12288, 19456])
+def test_factorisation_in_slabs(F):
+    """The residual of the solve within the backward error of a factorisation of that size, the factor next to that of the general
+    path (no workspace for slabs), a pivot that is not positive and a NaN below the slab reported."""
+    from qml_lightning_amd import _lib, ops
+    L = _lib.lib()
     g = torch.Generator(device=dev()).manual_seed(9)
     Z = torch.randn(F + 300, F, dtype=torch.float64, device=dev(), generator=g) * 0.01
     Z *= torch.exp(torch.randn(F, dtype=torch.float64, device=dev(), generator=g))
@@ -144,11 +147,25 @@ def test_factorisation_in_slabs():
     del Z
     A.diagonal().add_(1e-3)
     b = torch.randn(F, 1, dtype=torch.float64, device=dev(), generator=g)
+    assert L.qmll_cholesky_slabs_bytes(F) > 0 and L.qmll_cholesky_slabs_bytes(F - 1) == 0 and L.qmll_cholesky_slabs_bytes(7040) == 0
     x, info = ops.cholesky_solve_spd(A, b)
     assert int(info.item()) == 0
     # |A x - b| <= c n eps |A| |x| (a backward stable solve; c = 1 is far from what a random matrix shows)
     assert float((A @ x - b).norm()) <= F * 2.0 ** -53 * float(A.norm()) * float(x.norm())
-    for row, col, value, expect in ((10000, 10000, -1.0, 10001), (6000, 10500, float("nan"), None)):
+    # either factor: |U^T U - A| <= (n + 1) eps |U^T||U| entry by entry, and that is at most sqrt(a_ii a_jj) (Higham, theorem 10.3)
+    work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device=dev())
+    slabs = torch.empty(int(L.qmll_cholesky_slabs_bytes(F)), dtype=torch.uint8, device=dev())
+    rows = torch.arange(0, F, 997, device=dev())
+    scale = A.diagonal()[rows, None].sqrt() * A.diagonal()[None, :].sqrt()
+    for s in (slabs, None):
+        U = A.clone()
+        info.zero_()
+        ops.check(L.qmll_cholesky_slabs_f64(ops._ptr(U), F, F, ops._ptr(work), ops._ptr(s), ops._ptr(info), ops._stream()), "chol")
+        assert int(info.item()) == 0
+        U.triu_()
+        assert float(((U[:, rows].T @ U - A[rows]).abs() / scale).max()) <= 2 * (F + 1) * 2.0 ** -53
+        del U
+    for row, col, value, expect in ((F - 2000, F - 2000, -1.0, F - 1999), (1000, F - 1500, float("nan"), None)):
         kept = A[row, col].item()
         A[row, col] = value
         A[col, row] = value
@@ -156,3 +173,25 @@ def test_factorisation_in_slabs():
         assert int(info.item()) == expect if expect else int(info.item()) > 0
         A[row, col] = kept
         A[col, row] = kept
+
+
+def test_solve_without_memory_for_slabs(monkeypatch):
+    """Where the workspace of the slabs does not fit, the solve does without it."""
+    from qml_lightning_amd import ops
+    F = 7168
+    g = torch.Generator(device=dev()).manual_seed(4)
+    Z = torch.randn(F + 300, F, dtype=torch.float64, device=dev(), generator=g)
+    A = torch.zeros(F, F, dtype=torch.float64, device=dev())
+    ops.gram(Z, None, A, None)
+    b = torch.randn(F, 1, dtype=torch.float64, device=dev(), generator=g)
+    real, refused = torch.empty, []
+
+    def empty(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.cuda.OutOfMemoryError("planted")
+        return real(*args, **kwargs)
+    monkeypatch.setattr(torch, "empty", empty)
+    x, info = ops.cholesky_solve_spd(A, b)
+    assert refused and int(info.item()) == 0
+    assert float((A @ x - b).norm()) <= F * 2.0 ** -53 * float(A.norm()) * float(x.norm())
