@@ -121,16 +121,17 @@ __device__ __forceinline__ bool static_all(F&& f) {
 //      a reciprocal square root and the pivot row handed round with v_readlane, no barrier and no LDS inside;
 //      the same row operations on the identity give V = U_KK^-1;
 //   2. block row K: U(K,J) = V^T S(K,J), W(K,J) = V^T W(K,J), four MFMAs each, to LDS and to memory;
-//   3. S(I,J) -= U(K,I)^T U(K,J) and W(I,J) -= U(K,I)^T W(K,J) for the rows I > K.
+//   3. S(I,J) -= U(K,I)^T U(K,J) and W(I,J) -= U(K,I)^T W(K,J) for the rows I > K: S(K+1,K+1) at once, the others
+//      beside step 1 of K + 1, which waits for that one only (a 128 x 128 block in a launch of its own 45.5 us with all of them before it, 40.4 so).
 // 24 barriers instead of the 128 of an elimination pivot by pivot, and the multiply-adds on the matrix pipe.
 // Output: upper triangle of the block <- U11; inv[m*128+i] = U11^-1[m,i] = W[i,m]; invT[i*128+m] the same.
 // info: 0, or 1 + the index of the first pivot that is not positive (later launches then exit).
 
 // inv[m, 16 K + i] = W[16 K + i, m] for the columns m of block row K, from the strip in LDS: thread = (m, half a
-// row of sixteen), 64 contiguous bytes each
+// row of sixteen), 64 contiguous bytes each.  Wavefronts 4..7: 0 is the one that is waited for.
 __device__ __forceinline__ void store_inverse_columns(int K, double* inv, const PotrfShared& ps) {
-    const int m = (int)threadIdx.x >> 1, half = (int)threadIdx.x & 1;
-    if (m < (K + 1) * SB) {
+    const int m = ((int)threadIdx.x - PT / 2) >> 1, half = (int)threadIdx.x & 1;
+    if (m >= 0 && m < (K + 1) * SB) {
 #pragma unroll
         for (int q = 0; q < SB / 2; ++q) inv[m * NB + K * SB + half * (SB / 2) + q] = ps.wstrip[half * (SB / 2) + q][m];
     }
@@ -183,15 +184,15 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
         }
         // (every lane stores: the four copies write the same values)
 #pragma unroll
+        for (int i = 0; i < SB; ++i) ps.vblk[l16][i] = w[i];           // V[c, i] = W[i, c]
+        __syncthreads();                                               // V is in LDS
+        if (ps.failed) return false;
+#pragma unroll
         for (int i = 0; i < SB; ++i) {
-            ps.vblk[l16][i] = w[i];                                    // V[c, i] = W[i, c]
             const int row = K * SB + i, col = K * SB + l16;
             if (lane < SB && i <= l16 && col < nb) blk[(size_t)row * ld + col] = d[i];
         }
-        __syncthreads();                                               // V is in LDS
-        if (ps.failed) return false;
         __syncthreads();                                               // block row K is in LDS
-        store_inverse_columns(K, inv, ps);
     }
     return true;
 }
@@ -225,7 +226,8 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
             }
         }
     });
-    return static_all<NSB>([&](auto K_) -> bool {
+    // the diagonal sub-block K goes to wavefront 0
+    auto hand_diagonal = [&](auto K_) {
         constexpr int K = decltype(K_)::value;
         static_for<NSLOT>([&](auto s_) {
             constexpr int s = decltype(s_)::value, t = s * MWAVES + WV - 1;
@@ -237,7 +239,35 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
                 }
             }
         });
+    };
+    // the update by block row K of the next diagonal sub-block (only) or of all others
+    auto update = [&](auto K_, auto diagonal_) {
+        constexpr int K = decltype(K_)::value;
+        static_for<NSLOT>([&](auto s_) {
+            constexpr int s = decltype(s_)::value, t = s * MWAVES + WV - 1;
+            if constexpr (t < 2 * NSUB) {
+                constexpr SubId b = sub_id(t);
+                constexpr bool next = b.kind == 0 && b.i == K + 1 && b.j == K + 1;
+                if constexpr (b.i > K && (b.kind == 0 || b.j <= K) && next == decltype(diagonal_)::value) {
+                    const double* right = b.kind == 0 ? us_lane : ws_lane;
+#pragma unroll
+                    for (int kk = 0; kk < 4; ++kk) {
+                        const double fa = -us_lane[4 * kk * SSTRIDE + b.i * SB];
+                        const double fb = right[4 * kk * SSTRIDE + b.j * SB];
+                        sub[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, fb, sub[s], 0, 0, 0);
+                    }
+                }
+            }
+        });
+    };
+    hand_diagonal(std::integral_constant<int, 0>{});
+    return static_all<NSB>([&](auto K_) -> bool {
+        constexpr int K = decltype(K_)::value;
         __syncthreads();                                               // S(K,K) is in LDS
+        if constexpr (K > 0) {                                         // beside wavefront 0: what it does not wait for
+            update(std::integral_constant<int, K - 1>{}, std::false_type{});
+            store_inverse_columns(K - 1, inv, ps);
+        }
         __syncthreads();                                               // wavefront 0 has factored it: V is in LDS
         if (ps.failed) return false;
         double va[4];
@@ -267,22 +297,12 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
             }
         });
         __syncthreads();                                               // block row K is in LDS
-        store_inverse_columns(K, inv, ps);
-        static_for<NSLOT>([&](auto s_) {
-            constexpr int s = decltype(s_)::value, t = s * MWAVES + WV - 1;
-            if constexpr (t < 2 * NSUB) {
-                constexpr SubId b = sub_id(t);
-                if constexpr (b.i > K && (b.kind == 0 || b.j <= K)) {
-                    const double* right = b.kind == 0 ? us_lane : ws_lane;
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) {
-                        const double fa = -us_lane[4 * kk * SSTRIDE + b.i * SB];
-                        const double fb = right[4 * kk * SSTRIDE + b.j * SB];
-                        sub[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, fb, sub[s], 0, 0, 0);
-                    }
-                }
-            }
-        });
+        if constexpr (K + 1 < NSB) {
+            update(K_, std::true_type{});
+            hand_diagonal(std::integral_constant<int, K + 1>{});
+        } else {
+            store_inverse_columns(K, inv, ps);
+        }
         return true;
     });
 }
