@@ -143,17 +143,14 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
     const int lane = (int)threadIdx.x & 63, l16 = lane & 15;
     for (int K = 0; K < NSB; ++K) {
         __syncthreads();                                               // S(K,K) is in LDS
-        // column l16 of the sub-block in d, row l16 of V in w (the four groups of sixteen lanes hold copies)
-        double d[SB], w[SB];
+        // lanes 0..15: column l16 of the sub-block; the others: row l16 of V, which takes the same row operations
+        double v[SB];
 #pragma unroll
-        for (int i = 0; i < SB; ++i) {
-            d[i] = ps.dblk[i][l16];
-            w[i] = i == l16 ? 1.0 : 0.0;
-        }
+        for (int i = 0; i < SB; ++i) v[i] = lane < SB ? ps.dblk[i][l16] : i == l16 ? 1.0 : 0.0;
         int bad = -1;                                                  // the first pivot that is not positive
 #pragma unroll
         for (int j = 0; j < SB; ++j) {
-            double piv = value_of_lane(d[j], j);                       // the same value in every lane
+            double piv = value_of_lane(v[j], j);                       // the same value in every lane
             if (!(piv > 0.0)) {
                 bad = bad < 0 ? j : bad;
                 piv = 1.0;
@@ -163,34 +160,30 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
             const double h = 0.5 * piv;
             y = fma(y, fma(-h * y, y, 0.5), y);
             y = fma(y, fma(-h * y, y, 0.5), y);
-            const double u = d[j] * y;                                 // U[j, l16]
-            const double wj = w[j] * y;                                // W[j, l16]
-            d[j] = u;
-            w[j] = wj;
+            const double u = v[j] * y;                                 // U[j, l16], W[j, l16]
+            v[j] = u;
 #pragma unroll
             for (int i = j + 1; i < SB; ++i) {
-                const double ui = value_of_lane(u, i);                 // U[j, i] = L[i, j]
-                d[i] = fma(-ui, u, d[i]);
-                w[i] = fma(-ui, wj, w[i]);
-                // pins the update to this step (no instruction is emitted): nothing needs w before the end, so
-                // left alone the compiler computes all of it there and carries every multiplier of every step
-                // in scalar registers it does not have
-                asm volatile("" : "+v"(w[i]));
+                v[i] = fma(-value_of_lane(u, i), u, v[i]);             // U[j, i] = L[i, j]
+                // pins the update to this step (no instruction is emitted): left alone the compiler carries multipliers in scalar
+                // registers that it does not have
+                asm volatile("" : "+v"(v[i]));
             }
         }
         if (bad >= 0 && lane == 0) {
             *info = k0 + K * SB + bad + 1;
             ps.failed = 1;
         }
-        // (every lane stores: the four copies write the same values)
+        if (lane >= SB) {                                              // (the three copies write the same values)
 #pragma unroll
-        for (int i = 0; i < SB; ++i) ps.vblk[l16][i] = w[i];           // V[c, i] = W[i, c]
+            for (int i = 0; i < SB; ++i) ps.vblk[l16][i] = v[i];       // V[c, i] = W[i, c]
+        }
         __syncthreads();                                               // V is in LDS
         if (ps.failed) return false;
 #pragma unroll
         for (int i = 0; i < SB; ++i) {
             const int row = K * SB + i, col = K * SB + l16;
-            if (lane < SB && i <= l16 && col < nb) blk[(size_t)row * ld + col] = d[i];
+            if (lane < SB && i <= l16 && col < nb) blk[(size_t)row * ld + col] = v[i];
         }
         __syncthreads();                                               // block row K is in LDS
     }
@@ -393,15 +386,23 @@ struct TileShared {
     double a[2][PKB][PSTRIDE], b[2][PKB][PSTRIDE];
 };
 
+constexpr int TRIANGULAR = 1, DIAGONAL = 2;
 // The 128 x 128 tile at C (row stride ldc) = or += sign * Za^T Zb, Za and Zb `depth` rows (a multiple of 16) of 128
 // columns; the tile product of gram.hip for whole tiles (same staging, same MFMA order).  C may be Zb
 // (depth 128, overwrite): everything is read before anything is written.  Ends with a barrier.
+// TRIANGULAR: Za[m][i] = 0 for m > i (the inverse of a diagonal block), whose 16 x 16 sub-blocks below the diagonal are left out; DIAGONAL:
+// only the sub-blocks of C on or above the diagonal are wanted.  Either leaves 36 of 64: the chain of a panel is these
+// and the factorisations (82 us a block with whole products, 65 with these; 16384 features 25.0 -> 22.7 ms, 2048 1.59 -> 1.33).
+template <int MODE = 0>
 __device__ __forceinline__ void tile_product(const double* Za, long long lda, const double* Zb, long long ldb,
                                              int depth, double* C, long long ldc, double sign, bool overwrite,
                                              TileShared& sm) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave / 4) * 64, wj = (wave % 4) * 32;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // (uniform: a matrix instruction takes no lane mask)
+    // (wavefronts w and w + 4 share a SIMD: in a diagonal tile they have 10, 10, 8 and 8 of 16 sub-blocks on or above the diagonal)
+    const int wi = (wave / 4) * 64, wj = (wave < 4 ? wave : 7 - wave) * 32;
     const int l16 = lane & 15, lk = lane >> 4;
+    auto wanted = [&](int p, int q) { return MODE != DIAGONAL || wi + p * 16 <= wj + q * 16; };
     double4_t acc[4][2];
 #pragma unroll
     for (int p = 0; p < 4; ++p)
@@ -433,18 +434,40 @@ __device__ __forceinline__ void tile_product(const double* Za, long long lda, co
     for (int step = 0; step < nsteps; ++step) {
         const int cur = step & 1;
         if (step + 1 < nsteps) load_panels((step + 1) * PKB);   // in flight during the MFMAs
+        if constexpr (MODE == 0) {
 #pragma unroll
-        for (int kk = 0; kk < PKB; kk += 4) {
-            double fa[4], fb[2];
+            for (int kk = 0; kk < PKB; kk += 4) {
+                double fa[4], fb[2];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) fa[p] = sm.a[cur][kk + lk][wi + p * 16 + l16];
+                for (int p = 0; p < 4; ++p) fa[p] = sm.a[cur][kk + lk][wi + p * 16 + l16];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) fb[q] = sm.b[cur][kk + lk][wj + q * 16 + l16];
+                for (int q = 0; q < 2; ++q) fb[q] = sm.b[cur][kk + lk][wj + q * 16 + l16];
 #pragma unroll
-            for (int p = 0; p < 4; ++p)
+                for (int p = 0; p < 4; ++p)
 #pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[p], fb[q], acc[p][q], 0, 0, 0);
+                    for (int q = 0; q < 2; ++q)
+                        acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[p], fb[q], acc[p][q], 0, 0, 0);
+            }
+        } else {
+            double fb[2][4];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fb[q][k] = sm.b[cur][4 * k + lk][wj + q * 16 + l16];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                if (MODE == TRIANGULAR && step * PKB > wi + p * 16) continue;     // rows of zeros
+                if (!wanted(p, 1)) continue;
+                double fa[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fa[k] = sm.a[cur][4 * k + lk][wi + p * 16 + l16];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    if (!wanted(p, q)) continue;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[k], fb[q][k], acc[p][q], 0, 0, 0);
+                }
+            }
         }
         if (step + 1 < nsteps) store_panels(cur ^ 1);
         __syncthreads();
@@ -452,7 +475,8 @@ __device__ __forceinline__ void tile_product(const double* Za, long long lda, co
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < 2; ++q) {
+            if (!wanted(p, q)) continue;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 double* c = C + (size_t)(wi + p * 16 + lk + 4 * r) * ldc + wj + q * 16 + l16;
@@ -462,6 +486,7 @@ __device__ __forceinline__ void tile_product(const double* Za, long long lda, co
                 if (overwrite) *c = v;
                 else unsafeAtomicAdd(c, v);
             }
+        }
     __syncthreads();
 }
 
@@ -579,7 +604,7 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
         for (int w = bid; w < ncol; w += stride) {
             const int j0 = P0 + w * NB;                      // first column of the owned tiles
             double* tile = A + (size_t)k0 * ld + j0;
-            tile_product(inv, NB, tile, ld, NB, tile, ld, 1.0, true, sm);
+            tile_product<TRIANGULAR>(inv, NB, tile, ld, NB, tile, ld, 1.0, true, sm);
             if (bid < nblk) publish(flags + PBLK + l * PBLK + bid, FLAG_DONE);
             for (int b = l + 1; b <= mine; ++b) {
                 const unsigned bit = 1u << (l * PBLK + b);
@@ -587,8 +612,9 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
                     if (await(flags + PBLK + l * PBLK + b, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
                     strips_seen |= bit;
                 }
-                tile_product(A + (size_t)k0 * ld + P0 + b * NB, ld, tile, ld, NB, A + (size_t)(P0 + b * NB) * ld + j0, ld,
-                             -1.0, false, sm);
+                double* into = A + (size_t)(P0 + b * NB) * ld + j0;
+                if (b == bid) tile_product<DIAGONAL>(tile, ld, tile, ld, NB, into, ld, -1.0, false, sm);
+                else tile_product(A + (size_t)k0 * ld + P0 + b * NB, ld, tile, ld, NB, into, ld, -1.0, false, sm);
             }
         }
     }
@@ -760,8 +786,8 @@ namespace {
 // the matrix is read and written once per slab and not once per panel.  In the last 4096 rows the panel launches of fp64 products
 // are as fast, which are short there and wait for their chain of factorisations.  Up to 12288 rows a slab (15 bytes an entry
 // for the residues, 3 GB at 16384 features); below 7168 features there is nothing to gain.  ms without slabs and with:
-// 24576 features 90.5 / 57.2, 16384 32.8 / 25.4, 10240 12.6 / 11.9, 8192 8.86 / 8.54, 7168 7.31 / 7.19, 6144 5.95 / 5.93, 5120
-// 4.66 / 4.70; slabs of 4096 rows 28.3 at 16384; a rest of 8192 rows 26.7 there and, at 10240, 12.9 against 12.0.
+// 24576 features 90.3 / 54.4, 16384 31.6 / 23.0, 12288 16.2 / 13.8, 10240 11.3 / 10.3, 8192 7.6 / 7.3, 7168 6.1 / 6.0; a rest of 6144
+// rows 23.4 at 16384 and 10.6 at 10240, of 3072 rows 23.1 and 10.3.
 constexpr int SLAB = 12288, SLAB_REST = 4096, SLAB_LEAST = 3072;
 // end of the slab of rows that starts at s0
 int slab_end(int s0, int F) {
@@ -890,8 +916,9 @@ extern "C" int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* wor
             const int nt = P0 > R0 ? (F - pend) / NB : 0;
             const int nown = ncol;
             // The head tiles (this panel's rows of the update of the panel before) go to workgroups of their own
-            // once the trailing matrix is small, where a launch lasts as long as its slowest owner: four head tiles
-            // and ten strip / update products in a row, 540 us, against a chain of four factorisations of 390.
+            // once the trailing matrix is small, where a launch lasts as long as its slowest owner, which has four head
+            // tiles and ten strip / update products in a row (16384 features 22.9 ms without, 21.8 so; 8192 8.15 and 7.09;
+            // 4096 3.89 and 2.88; a line at 24 tiles an edge instead of 48 5.30 against 4.86 at 6144).
             // While the trailing tiles keep the chip busy for longer than that, the owners take their head tiles
             // themselves and no slot waits for another.
             const bool split_heads = P0 > R0 && nt <= SPLIT_HEADS_BELOW;
