@@ -205,11 +205,28 @@ __device__ __forceinline__ void find_tile(const int* __restrict__ type_offsets, 
         tile -= nt;
     }
 }
-// first unit of share g; with fewer units than shares the last shares are empty, else none is
-__device__ __forceinline__ int share_begin(int g, int nshares, int ntiles, int rounds) {
-    const int units = ntiles * rounds, used = min(nshares, units);
-    return g >= used ? units : (int)((long long)units * g / used);
+// First unit of share g of `nshares`, of which `slots` workgroups are resident at a time; with fewer units than shares the last ones
+// are empty.  Where there are two rounds of workgroups, the first takes whole tiles and the equal shares of the second level out what
+// is left, so that only those are cut: all tiles cut into equal shares end at the same time, but a tile in parts is written and
+// read once more (d = 128, 128 stacks with the gradient, all shares equal / whole tiles first: 60000 atoms 474 / 444 us,
+// 86016 653 / 628, 131072 972 / 923, 200000 1467 / 1394).  Not where less than an eighth of a tile a share is left, as few tiles are
+// then cut into very many parts: 52300 atoms (a sixteenth) 419 / 435, 49400 (all that is left) 390 / 558; 56000 (a seventh) 444 / 414.
+constexpr int LEAST_LEFT = 8;
+__device__ __forceinline__ int share_begin(int g, int nshares, int slots, int ntiles, int rounds) {
+    const int units = ntiles * rounds;
+    int whole = 0, each = 0;                                            // shares of whole tiles, tiles in each
+    if (nshares >= 2 * slots) {
+        whole = (nshares / slots - 1) * slots;
+        each = (ntiles + nshares - 1) / nshares;
+        // (at least 1 / LEAST_LEFT of a tile a share is left)
+        if ((long long)whole * each * LEAST_LEFT > (long long)ntiles * LEAST_LEFT - (nshares - whole)) whole = each = 0;
+    }
+    if (g < whole) return g * each * rounds;
+    const int left = units - whole * each * rounds, used = min(nshares - whole, left);
+    return g - whole >= used ? units : units - left + (int)((long long)left * (g - whole) / used);
 }
+template <int D, bool WITH_GRAD>
+constexpr int RESIDENT = (D == 128 && WITH_GRAD ? 3 : 4) * SM_CUS;
 
 // (at least two wavefronts per SIMD: with up to 256 registers the compiler lets the matrix instructions write vector
 // registers directly; asked for fewer it goes through accumulator registers, a move per value)
@@ -240,7 +257,8 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         }
         return;
     }
-    const int ubeg = share_begin(blockIdx.x, nshares, ntiles, rounds), uend = share_begin(blockIdx.x + 1, nshares, ntiles, rounds);
+    const int ubeg = share_begin(blockIdx.x, nshares, RESIDENT<D, WITH_GRAD>, ntiles, rounds);
+    const int uend = share_begin(blockIdx.x + 1, nshares, RESIDENT<D, WITH_GRAD>, ntiles, rounds);
 
     for (int u = ubeg; u < uend;) {
         const int tile = u / rounds, r0 = u - tile * rounds, r1 = min(rounds, r0 + uend - u);
@@ -456,12 +474,13 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
         return;
     }
     const int ntiles = tile_count(type_offsets, ne);
-    const int ubeg = share_begin(g, nshares, ntiles, rounds), uend = share_begin(g + 1, nshares, ntiles, rounds);
+    constexpr int slots = RESIDENT<D, WITH_GRAD>;
+    const int ubeg = share_begin(g, nshares, slots, ntiles, rounds), uend = share_begin(g + 1, nshares, slots, ntiles, rounds);
     if (ubeg == uend) return;
     const int tile = (uend - 1) / rounds, tbeg = tile * rounds, tend = tbeg + rounds;
     if (tbeg < ubeg || tend <= uend) return;
     int last = g + 1;                                    // the share in which the tile ends
-    while (share_begin(last + 1, nshares, ntiles, rounds) < tend) ++last;
+    while (share_begin(last + 1, nshares, slots, ntiles, rounds) < tend) ++last;
     int type, row0, rows;
     find_tile(type_offsets, ne, tile, type, row0, rows);
     const float* next = parts + (size_t)(g + 1) * SLOT;
@@ -490,7 +509,7 @@ static long long matrix_units(int A, int ne, int T, int S, int d) {
 }
 // Shares of a launch.  Three (d = 128 with the gradient) or four workgroups are resident per CU; twice as many shares level out
 // what the cut into whole shares leaves uneven, but a share of few rounds pays more for its parts than it gains.
-// Measured at d = 128, 128 stacks with the gradient, 3 / 6 shares per CU: 24000 atoms 206 / 207 us, 86016 atoms 668 / 643, and with two
+// Measured at d = 128, 128 stacks with the gradient, 3 / 6 shares per CU: 24000 atoms 206 / 207 us, 86016 atoms 668 / 628, and with two
 // transforms, 32 stacks, 24000 atoms 102 / 110.
 static int matrix_shares(long long units, int with_grad) {
     const long long per_cu = units / (SM_CUS * (with_grad ? 24 : 16));
