@@ -28,7 +28,7 @@ NPCAS, NSTACKS, SIGMA = 128, 128, 2.0
 NMOL_PREDICT, NMOL_TRAIN = 4096, 1000
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
-FP16_PEAK_TFLOPS = 2500.0         # dense v_mfma_f32_32x32x16_f16
+FP16_PEAK_TFLOPS = 2500.0         # dense fp16 matrix instructions
 FP64_PEAK_TFLOPS = 78.6
 INT8_PEAK_TOPS = 5033.0
 
@@ -234,7 +234,7 @@ def other_configs(torch, dev):
     fl5 = 4.0 * x5.shape[0] * x5.shape[1] * m5.nfeatures()          # x.W and its transpose product
     r5["rff_energy_sorted_kernel"] = {
         "seconds": t_rff, "bound": "mfma",
-        "pipe": "fp16 matrix cores (v_mfma_f32_32x32x16_f16), fp32 operands split in two fp16 parts (W once per model, x and "
+        "pipe": "fp16 matrix cores (v_mfma_f32_16x16x32_f16), fp32 operands split in two fp16 parts (W once per model, x and "
                 "the sine factors in the kernel), fp32 accumulation",
         "TFLOPs": fl5 / t_rff / 1e12, "executed_TFLOPs": 3.0 * fl5 / t_rff / 1e12, "peak_TFLOPs": FP16_PEAK_TFLOPS,
         "frac": 3.0 * fl5 / t_rff / 1e12 / FP16_PEAK_TFLOPS}
