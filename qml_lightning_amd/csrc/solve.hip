@@ -49,7 +49,7 @@ constexpr int PT = 512;           // threads of a factorisation workgroup (and o
 constexpr int SB = 16;            // sub-block edge of the diagonal-block factorisation (one fp64 MFMA tile)
 constexpr int NSB = NB / SB;      // sub-blocks per edge
 constexpr int NSUB = NSB * (NSB + 1) / 2;     // sub-blocks on or above (or on or below) the diagonal
-constexpr int MWAVES = PT / 64 - 1;           // wavefronts that hold sub-blocks; wavefront 0 factors the diagonal ones
+constexpr int MWAVES = PT / 64 - 2;           // wavefronts that hold sub-blocks; wavefront 0 factors the diagonal ones
 constexpr int NSLOT = (2 * NSUB + MWAVES - 1) / MWAVES;
 constexpr int SSTRIDE = NB + 16;  // doubles per row of a 16-row strip in LDS (rows 32 banks apart, see gram.hip)
 constexpr int DSTRIDE = SB + 1;
@@ -72,8 +72,8 @@ __device__ __forceinline__ double value_of_lane(double v, int lane) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Sub-block t of the list the wavefronts 1..7 are dealt their register slots from (wavefront w holds
-// t = 7 s + w - 1 in slot s): first the 36 sub-blocks of S on or above the diagonal, row by row, then the
+// Sub-block t of the list the wavefronts 1, 2, 3, 5, 6, 7 are dealt their register slots from (the w-th of them holds
+// t = 6 s + w - 1 in slot s): first the 36 sub-blocks of S on or above the diagonal, row by row, then the
 // 36 of W on or below it.  kind 0: S, 1: W.
 struct SubId {
     int kind, i, j;
@@ -113,16 +113,18 @@ __device__ __forceinline__ bool static_all(F&& f) {
 // Blocked right-looking Cholesky on 16 x 16 sub-blocks, S = U^T U, with the same block operations applied to
 // the identity: W = L^-1 = U^-T.  The sub-blocks live in registers in the accumulator layout of
 // v_mfma_f64_16x16x4_f64 (register r of a lane: row lane/16 + 4r, column lane%16), which is also the layout
-// of both operands (row = the summed index), so a sub-block feeds the matrix pipe as it stands.  Wavefronts
-// 1..7 hold the 72 sub-blocks, up to eleven each; which ones is fixed at compile time (one instance of the code
+// of both operands (row = the summed index), so a sub-block feeds the matrix pipe as it stands.  Six wavefronts
+// hold the 72 sub-blocks, twelve each; which ones is fixed at compile time (one instance of the code
 // per wavefront), so a finished sub-block's registers are free again and no index is computed at run time.
+// Wavefront 4 has none: it shares its SIMD with wavefront 0, whose fp64 arithmetic waits for matrix instructions there (dealt to
+// seven wavefronts a block in a launch of its own takes 35.6 us, to six 33.5; 2048 features 1.335 and 1.305 ms).
 // Wavefront 0 holds none and does the serial part.  Step K of eight:
 //   1. the owner of S(K,K) puts it into LDS; wavefront 0 factors it, a lane per column: sixteen pivots, each
 //      a reciprocal square root and the pivot row handed round with v_readlane, no barrier and no LDS inside;
 //      the same row operations on the identity give V = U_KK^-1;
 //   2. block row K: U(K,J) = V^T S(K,J), W(K,J) = V^T W(K,J), four MFMAs each, to LDS and to memory;
 //   3. S(I,J) -= U(K,I)^T U(K,J) and W(I,J) -= U(K,I)^T W(K,J) for the rows I > K: S(K+1,K+1) at once, the others
-//      beside step 1 of K + 1, which waits for that one only (a 128 x 128 block in a launch of its own 45.5 us with all of them before it, 40.4 so).
+//      beside step 1 of K + 1, which waits for that one only (a 128 x 128 block in a launch of its own took 45.5 us with all of them before it, 40.4 so).
 // 24 barriers instead of the 128 of an elimination pivot by pivot, and the multiply-adds on the matrix pipe.
 // Output: upper triangle of the block <- U11; inv[m*128+i] = U11^-1[m,i] = W[i,m]; invT[i*128+m] the same.
 // info: 0, or 1 + the index of the first pivot that is not positive (later launches then exit).
@@ -190,7 +192,20 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
     return true;
 }
 
-// wavefront WV = 1..7: its share of the sub-blocks
+// wavefront 4, which shares its SIMD with wavefront 0: no matrix instructions, the columns of the inverse only
+__device__ __forceinline__ bool potrf_store_wave(double* inv, PotrfShared& ps) {
+    for (int K = 0; K < NSB; ++K) {
+        __syncthreads();                                               // S(K,K) is in LDS
+        if (K > 0) store_inverse_columns(K - 1, inv, ps);
+        __syncthreads();                                               // V is in LDS
+        if (ps.failed) return false;
+        __syncthreads();                                               // block row K is in LDS
+    }
+    store_inverse_columns(NSB - 1, inv, ps);
+    return true;
+}
+
+// the WV-th (1..6) of the wavefronts 1, 2, 3, 5, 6, 7: its share of the sub-blocks
 template <int WV>
 __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int nb, double* inv, double* invT,
                                                 PotrfShared& ps) {
@@ -322,10 +337,10 @@ __device__ __forceinline__ bool potrf_block(double* A, long long ld, int k0, int
         case 1: ok = potrf_mfma_wave<1>(blk, ld, nb, inv, invT, ps); break;
         case 2: ok = potrf_mfma_wave<2>(blk, ld, nb, inv, invT, ps); break;
         case 3: ok = potrf_mfma_wave<3>(blk, ld, nb, inv, invT, ps); break;
-        case 4: ok = potrf_mfma_wave<4>(blk, ld, nb, inv, invT, ps); break;
-        case 5: ok = potrf_mfma_wave<5>(blk, ld, nb, inv, invT, ps); break;
-        case 6: ok = potrf_mfma_wave<6>(blk, ld, nb, inv, invT, ps); break;
-        default: ok = potrf_mfma_wave<7>(blk, ld, nb, inv, invT, ps); break;
+        case 4: ok = potrf_store_wave(inv, ps); break;
+        case 5: ok = potrf_mfma_wave<4>(blk, ld, nb, inv, invT, ps); break;
+        case 6: ok = potrf_mfma_wave<5>(blk, ld, nb, inv, invT, ps); break;
+        default: ok = potrf_mfma_wave<6>(blk, ld, nb, inv, invT, ps); break;
     }
     if (!ok) return false;                                        // every wavefront saw the same flag
     __syncthreads();
