@@ -808,7 +808,8 @@ namespace {
 // (gram_modular.hip), before each panel of 512 rows on the panel's own rows only and at a slab's end on everything below it, so that
 // the matrix is read and written once per slab and not once per panel.  In the last 4096 rows the panel launches of fp64 products
 // are as fast, which are short there and wait for their chain of factorisations.  Up to 12288 rows a slab (15 bytes an entry
-// for the residues, 3 GB at 16384 features); below 7168 features there is nothing to gain.  ms without slabs and with:
+// for the residues, 3 GB at 16384 features); below 7168 features there is nothing to gain.  ms without slabs and with, taken when a
+// block of the chain took 65 us (62 now, on both sides):
 // 24576 features 90.3 / 54.4, 16384 31.6 / 23.0, 12288 16.2 / 13.8, 10240 11.3 / 10.3, 8192 7.6 / 7.3, 7168 6.1 / 6.0; a rest of 6144
 // rows 23.4 at 16384 and 10.6 at 10240, of 3072 rows 23.1 and 10.3.
 constexpr int SLAB = 12288, SLAB_REST = 4096, SLAB_LEAST = 3072;
