@@ -621,7 +621,7 @@ def main():
         btar = model._targets(bd, 500, True, True)
         bz = torch.zeros(F, F, dtype=torch.float64, device=dev)
         by = torch.zeros(F, 1, dtype=torch.float64, device=dev)
-        t_bgram = timed(lambda: ops.gram(brow, btar, bz, by, mirror=False), iters=2)
+        t_bgram = timed(lambda: ops.gram(brow, btar, bz, by, mirror=False, within_norms=True), iters=2)
         batch_phases = {"molecules": 500, "rows": int(brow.shape[0]), "format_data_ms": t_format / (NMOL_TRAIN / 500) * 1e3,
                         "representation_and_jacobian_ms": t_rep * 1e3, "projection_of_all_rows_ms": (t_proj - t_rep) * 1e3,
                         "feature_rows_ms": t_rows * 1e3, "gram_ms": t_bgram * 1e3}
@@ -638,7 +638,7 @@ def main():
         yv = torch.randn(M, 1, dtype=torch.float64, device=dev)
         ZTZ = torch.zeros(F, F, dtype=torch.float64, device=dev)
         ZTy = torch.zeros(F, 1, dtype=torch.float64, device=dev)
-        t_gram = timed(lambda: ops.gram(rows, yv, ZTZ, ZTy), iters=2)
+        t_gram = timed(lambda: ops.gram(rows, yv, ZTZ, ZTy, within_norms=True), iters=2)
         gram_flops = float(M) * F * (F + 1) + 2.0 * M * F
         # exact int8 products modulo 14 numbers stand for the fp64 sums: TFLOPs are the sums', the unit's own operations beside it
         int8_ops = 14.0 * M * F * (F + 256)
@@ -647,7 +647,7 @@ def main():
         # half the width
         rows_h = rows[:32000, :F // 2].contiguous()
         ZTZ_h = torch.zeros(F // 2, F // 2, dtype=torch.float64, device=dev)
-        t_gram_h = timed(lambda: ops.gram(rows_h, None, ZTZ_h, None), iters=3)
+        t_gram_h = timed(lambda: ops.gram(rows_h, None, ZTZ_h, None, within_norms=True), iters=3)
         fl_h = 32000.0 * (F // 2) * (F // 2 + 1)
         int8_h = 14.0 * 32000 * (F // 2) * (F // 2 + 256)
         kernels["gram_f64_half_width"] = {"seconds": t_gram_h, "bound": "int8", "rows": 32000, "features": F // 2,

@@ -524,8 +524,10 @@ int qmll_gram_upper_ws_f64(const double* Z, const double* y, int M, int F, doubl
 
 /* The same sums on the int8 matrix cores (same part of kernel.py:190-192): the columns of Z are scaled by powers
  * of two and rounded to integers of norm 2^54, their products are formed exactly modulo 14 coprime numbers and
- * put together again.  An entry is off by about 2^-54 |z_i| |z_j|, whatever the number of rows; columns with NaN or
- * infinite entries, or with squares that leave fp64's range, send the call to the fp64 kernel, on the device.
+ * put together again.  An entry is off by about 2^-54 |z_i| |z_j|, whatever the number of rows: less than the fp64 kernel's
+ * error where the rows are large or small in all columns alike, but orders of magnitude more, relative to
+ * sum_k |z_ki z_kj|, where columns have their large entries in different rows.  The caller decides whether the columns' norms
+ * are the measure, as they are for a matrix that goes into a Cholesky factorisation.  Columns with NaN or infinite entries, or with squares that leave fp64's range, send the call to the fp64 kernel, on the device.
  * Upper tiles as qmll_gram_upper_f64; Z^T y in a fixed order.  The workspace (16-byte aligned) must hold
  * qmll_gram_modular_workspace_bytes(M, F) bytes; 0 means that the fp64 kernel is the faster one at this size. */
 size_t qmll_gram_modular_workspace_bytes(int M, int F);

@@ -879,12 +879,17 @@ def _gram_workspace(device):
     return ws
 
 
-def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True):
+def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True, within_norms=False):
     """ZTZ += Z^T Z (or the row block f0:f1 of it), ZTy += Z^T y, fp64, in place.
     mirror=False (full matrix only) accumulates just the tiles on or above the diagonal: a
-    caller adding several batches finishes with one `gram_mirror(ZTZ)`.  From 768 rows the full matrix comes from
-    exact integer products on the int8 matrix cores (an entry is off by about 2^-54 of the product of its two
-    columns' norms); fewer rows, row blocks and columns with NaN or infinite entries take the fp64 matrix cores."""
+    caller adding several batches finishes with one `gram_mirror(ZTZ)`.
+
+    Sums of fp64 products, an entry off by at most M 2^-53 sum_k |z_ki z_kj|.  within_norms=True says that an error of
+    2^-53 |z_i| |z_j| (the norms of the two columns) will do: from 768 rows the full matrix then comes from
+    exact integer products on the int8 matrix cores, up to three times as fast at full width.  On rows that are large
+    or small in all columns alike that error is the smaller one; where columns have their large entries in different
+    rows it can exceed the first by orders of magnitude, relative to the entry.  Row blocks, fewer rows, columns with NaN or
+    infinite entries, and calls for which there is no memory (up to 9 GiB) take the fp64 sums all the same."""
     if Zrows.dtype != torch.float64 or not Zrows.is_contiguous():
         raise RuntimeError("gram needs a contiguous float64 row matrix")
     M, F = Zrows.shape
@@ -895,7 +900,7 @@ def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True):
             raise RuntimeError("targets have %d rows, features have %d" % (yv.shape[0], M))
     zty = ZTy if ZTy is not None else None
     if f0 is None:
-        nbytes = int(_lib.lib().qmll_gram_modular_workspace_bytes(M, F))
+        nbytes = int(_lib.lib().qmll_gram_modular_workspace_bytes(M, F)) if within_norms else 0
         if nbytes:
             try:
                 work = torch.empty(nbytes, dtype=torch.uint8, device=Zrows.device)

@@ -215,7 +215,8 @@ def test_config5_rff_32768_features_batch_equals_its_parts():
     within(ZTy[:, 0], rows.T @ y, 1e-10, "rff ZTy")      # a sum over rows: the split into two batches does not matter
 
 
-def test_gram_16384_features_checksums_and_solve_residual():
+@pytest.mark.parametrize("within_norms", [False, True])
+def test_gram_16384_features_checksums_and_solve_residual(within_norms):
     """Z^T Z at the training width (16384 features) in two row batches: symmetry, trace = |Z|_F^2,
     (Z^T Z) v = Z^T (Z v), Z^T y; then the regularised solve on it."""
     from qml_lightning_amd import ops
@@ -230,7 +231,7 @@ def test_gram_16384_features_checksums_and_solve_residual():
     for M in (12000, 9001):                                  # the second batch ends in a partial panel
         Z = torch.randn(M, F, dtype=torch.float64, device=dev(), generator=g)
         y = torch.randn(M, 1, dtype=torch.float64, device=dev(), generator=g)
-        ops.gram(Z, y, ZTZ, ZTy, mirror=False)
+        ops.gram(Z, y, ZTZ, ZTy, mirror=False, within_norms=within_norms)
         ref_v += Z.T @ (Z @ v)
         ref_y += Z.T @ y
         fro += float((Z * Z).sum())
@@ -247,7 +248,8 @@ def test_gram_16384_features_checksums_and_solve_residual():
     assert resid <= 1e-10, resid
 
 
-def test_gram_32768_features_41000_rows_checksums():
+@pytest.mark.parametrize("within_norms", [False, True])
+def test_gram_32768_features_41000_rows_checksums(within_norms):
     """Z^T Z at the width and row count of the 32768-feature training configuration (500 molecules
     of 27 atoms with forces: 41000 rows) in its two batches of 250 molecules (20500 rows each):
     symmetry, trace = |Z|_F^2, (Z^T Z) v = Z^T (Z v), Z^T y."""
@@ -263,7 +265,7 @@ def test_gram_32768_features_41000_rows_checksums():
     for _ in range(2):
         Z = torch.randn(M, F, dtype=torch.float64, device=dev(), generator=g)
         y = torch.randn(M, 1, dtype=torch.float64, device=dev(), generator=g)
-        ops.gram(Z, y, ZTZ, ZTy, mirror=False)
+        ops.gram(Z, y, ZTZ, ZTy, mirror=False, within_norms=within_norms)
         ref_v += Z.T @ (Z @ v)
         ref_y += Z.T @ y
         fro += float((Z * Z).sum())

@@ -106,27 +106,97 @@ def test_columns_that_cannot_be_scaled_take_the_fp64_kernel(value):
     assert torch.equal(C.isnan(), fp64_kernel(Z, 1.0).isnan())
 
 
+def uneven_rows(kind):
+    """Rows whose columns have their large entries in different rows."""
+    rng = np.random.default_rng(17)
+    M, F = 800, 256
+    Z = rng.normal(size=(M, F))
+    if kind.startswith("lognormal"):
+        return Z * np.exp(float(kind.split()[1]) * rng.normal(size=(M, F)))
+    if kind == "own row":                         # one large entry per column, each in another row
+        Z[np.arange(F), np.arange(F)] *= 1e6
+        return Z
+    Z[:M // 2, :F // 2] *= 1e-9                   # two halves of the columns, each large where the other is small
+    Z[M // 2:, F // 2:] *= 1e-9
+    return Z
+
+
+@pytest.mark.parametrize("kind", ["lognormal 3", "lognormal 5", "own row", "halves"])
+def test_gram_holds_the_bound_of_fp64_sums_entry_by_entry(kind):
+    """A caller who has not said that the columns' norms are the measure gets every entry within M 2^-53 of the sum of its
+    products' magnitudes (a sum of M products in any order: (M - 1) additions and one rounding of each product)."""
+    from qml_lightning_amd import ops
+    Z = uneven_rows(kind)
+    M, F = Z.shape
+    C = torch.zeros(F, F, dtype=torch.float64, device=dev())
+    ops.gram(torch.tensor(Z, device=dev()), None, C, None)
+    Zl = Z.astype(np.longdouble)
+    off = np.abs(C.cpu().numpy() - Zl.T @ Zl) / (np.abs(Zl).T @ np.abs(Zl))
+    assert off.max() <= M * 2.0 ** -53, (kind, float(off.max()))
+
+
+@pytest.mark.parametrize("features", ["sorf", "rff"])
+@pytest.mark.parametrize("with_energies,with_forces", [(True, True), (False, True), (True, False)])
+def test_training_rows_lose_nothing_entry_by_entry(features, with_energies, with_forces):
+    """What training relies on in saying so: on its rows the root mean square over the entries of the error relative to the sum of the
+    products' magnitudes is no larger than that of the fp64 kernel, and none exceeds the bound of fp64 sums."""
+    from qml_lightning_amd.models.hadamard_features import HadamardFeaturesModel
+    from qml_lightning_amd.models.random_features import RandomFourrierFeaturesModel
+    from qml_lightning_amd.representations.FCHL import FCHLCuda
+    rng = np.random.default_rng(31)
+    np.random.seed(31)
+    elements = np.array([1, 6, 8])
+    nmol = 60 if with_forces else 800
+    counts = rng.integers(3, 10, nmol)
+    grid = np.stack(np.meshgrid(*[np.arange(3)] * 3, indexing="ij"), -1).reshape(-1, 3) * 1.6
+    X = [grid[rng.permutation(27)[:k]] + rng.uniform(-0.3, 0.3, (k, 3)) for k in counts]
+    Q = [rng.choice(elements, k) for k in counts]
+    E = rng.normal(size=nmol) if with_energies else None
+    Fo = [rng.normal(size=(k, 3)) for k in counts] if with_forces else None
+    cls = HadamardFeaturesModel if features == "sorf" else RandomFourrierFeaturesModel
+    m = cls(rep=FCHLCuda(species=elements), elements=elements, sigma=2.0, llambda=1e-5, npcas=64, nstacks=8, nbatch_train=nmol)
+    q, _ = torch.linalg.qr(torch.randn(3, m.rep.get_repsize(), 64, dtype=torch.float64, generator=torch.Generator().manual_seed(1)))
+    m.reductors = q.float().contiguous().to(dev())
+    data = m.format_data(X, Q, E=E, F=Fo)
+    proj, _ = m._training_batch(data, with_energies, with_forces)
+    rows = m._rows_from_projected(proj, with_forces, zero_energy_rows=not with_energies).contiguous()
+    M, F = rows.shape
+    assert M >= 768 and F == 512
+    Z = rows.cpu().numpy().astype(np.longdouble)
+    ref, mag = Z.T @ Z, np.abs(Z).T @ np.abs(Z)
+    fp64 = fp64_kernel(rows).cpu().numpy()
+    got = m.build_Z_components(X, Q, E=E, F=Fo, print_info=False)[0].cpu().numpy()
+    u = upper(F)
+
+    def errors(C):
+        d = (np.abs(C - ref) / mag)[u].astype(np.float64)
+        return np.sqrt((d * d).mean()), d.max()
+    print(features, with_energies, with_forces, M, "rms, max: modular %.2e %.2e, fp64 %.2e %.2e" % (errors(got) + errors(fp64)))
+    assert errors(got)[0] <= errors(fp64)[0]
+    assert errors(got)[1] <= M * 2.0 ** -53
+
+
 def test_modular_gram_in_a_graph_is_the_eager_result():
     g = torch.Generator(device="cpu").manual_seed(2)
     Z = torch.randn(1100, 300, dtype=torch.float64, generator=g).to(dev())
     from qml_lightning_amd import ops
     C = torch.zeros(300, 300, dtype=torch.float64, device=dev())
-    ops.gram(Z, None, C, None)
+    ops.gram(Z, None, C, None, within_norms=True)
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
-        ops.gram(Z, None, C.zero_(), None)
+        ops.gram(Z, None, C.zero_(), None, within_norms=True)
     torch.cuda.current_stream().wait_stream(s)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         C.zero_()
-        ops.gram(Z, None, C, None)
+        ops.gram(Z, None, C, None, within_norms=True)
     for seed in range(3):
         Z.copy_(torch.randn(1100, 300, dtype=torch.float64, generator=g))
         graph.replay()
         torch.cuda.synchronize()
         ref = torch.zeros_like(C)
-        ops.gram(Z, None, ref, None)
+        ops.gram(Z, None, ref, None, within_norms=True)
         torch.cuda.synchronize()
         assert torch.equal(C, ref), seed
 
