@@ -403,6 +403,13 @@ __global__ __launch_bounds__(256, 1) void modular_gemm_kernel(const signed char*
         }
 }
 
+// More than 64 KB of dynamic LDS have to be allowed, and what is allowed belongs to the device that is current: asked for before the
+// launches of each call, which costs the host less than a launch, instead of remembered for the process
+template <int N>
+hipError_t allow_stages() {
+    return hipFuncSetAttribute((const void*)modular_gemm_kernel<N>, hipFuncAttributeMaxDynamicSharedMemorySize, NSTAGE * STAGE);
+}
+
 // ---- reconstruction --------------------------------------------------------------------------------
 // thread = 16 entries of one accumulator: V = sum_i t_i (P / p_i) - P rint(sum_i t_i / p_i), every limb sum an
 // integer below 2^53 and so exact in fp64; C += V 2^-(2 gamma - e_i - e_j)
@@ -483,9 +490,8 @@ static int modular_syrk(const double* Z, long long ldz, const double* y, int M, 
     double* yparts = y ? parts + (size_t)pl.max_parts * F : nullptr;
     signed char* planes = (signed char*)(ws + pl.planes);
     signed char* results = (signed char*)(ws + pl.results);
-    static const hipError_t attr = hipFuncSetAttribute((const void*)modular_gemm_kernel<GRAM_MODULI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       NSTAGE * STAGE);
-    QMLL_REQUIRE(attr == hipSuccess, QMLL_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(attr));
+    const hipError_t lds = allow_stages<GRAM_MODULI>();
+    QMLL_REQUIRE(lds == hipSuccess, QMLL_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(lds));
     for (int m0 = 0; m0 < M; m0 += pl.rows) {
         const int m = M - m0 < pl.rows ? M - m0 : pl.rows;
         const double* z = Z + (size_t)m0 * ldz;
@@ -592,9 +598,8 @@ int qmll_internal_slab_update(double* A, long long ld, int rows, int n, int k, i
                               hipStream_t stream) {
     const Slab s = slab_layout(rows, n);
     char* ws = (char*)workspace;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)modular_gemm_kernel<CHOL_MODULI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       NSTAGE * STAGE);
-    QMLL_REQUIRE(attr == hipSuccess, QMLL_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(attr));
+    const hipError_t lds = allow_stages<CHOL_MODULI>();
+    QMLL_REQUIRE(lds == hipSuccess, QMLL_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(lds));
     const int off = i0 / 256, nt = s.nt - off;
     if (nt <= 0 || k <= 0) return QMLL_OK;
     const int tiles = band ? modular_band_tiles(std::min(band, nt), nt) : nt * (nt + 1) / 2;

@@ -78,6 +78,43 @@ def test_bad_arguments_are_refused_on_the_host():
     assert L.qmll_gram_f64(null, null, 0, 16, null, null, null) == _lib.QMLL_OK
 
 
+LARGE_LDS = """
+import ctypes, sys
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)      # found before the runtime that the library is linked to
+lib = ctypes.CDLL(sys.argv[2])
+P, I, N, LL = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_longlong
+lib.qmll_gram_modular_workspace_bytes.restype = N
+lib.qmll_gram_modular_f64.argtypes = [P, P, I, I, P, P, P, N, P]
+lib.qmll_cholesky_slabs_f64.argtypes = [P, I, LL, P, P, P, P]
+seen = []
+for device in (0, 1, 0, 2):
+    hip.recorded_set_device(device)
+    assert lib.qmll_gram_modular_f64(4096, None, 1000, 300, 4096, None, 4096, lib.qmll_gram_modular_workspace_bytes(1000, 300), None) == 0
+    seen.append(hip.recorded_large())
+    assert lib.qmll_cholesky_slabs_f64(4096, 7168, 7168, 4096, 4096, 4096, None) == 0
+    seen.append(hip.recorded_large())
+    print("device", device, "launches", hip.recorded_large(), "refused", hip.recorded_refused())
+assert all(a < b for a, b in zip([0] + seen, seen)), seen       # each of the two has such launches
+sys.exit(hip.recorded_refused() != 0)
+"""
+
+
+def test_large_lds_is_asked_for_on_every_device(tmp_path):
+    """A kernel with more than 64 KB of dynamic LDS has to be allowed it on the device that is current, not once per process: the
+    launches of the integer products on three devices in turn, recorded by tests/cpp/recorded_hip.cpp in place of the HIP runtime."""
+    import shutil
+    import subprocess
+    import sys
+    from qml_lightning_amd import _lib
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    so = str(tmp_path / "recorded_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(ROOT, "tests", "cpp", "recorded_hip.cpp"), "-o", so],
+                   check=True)
+    out = subprocess.run([sys.executable, "-c", LARGE_LDS, so, _lib.LIB_PATH], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from qml_lightning_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)
