@@ -201,6 +201,35 @@ def test_modular_gram_in_a_graph_is_the_eager_result():
         assert torch.equal(C, ref), seed
 
 
+# below and above the row count from which the fp64 kernel takes a workspace of its own
+@pytest.mark.parametrize("M,F", [(800, 300), (2100, 520)])
+def test_gram_without_memory_for_its_workspace(monkeypatch, M, F):
+    """Where the workspace of the integer products does not fit, the fp64 sums are taken, added to what is there, mirrored or not."""
+    from qml_lightning_amd import ops
+    g = torch.Generator(device="cpu").manual_seed(M)
+    Z, y = torch.randn(M, F, dtype=torch.float64, generator=g).to(dev()), torch.randn(M, 1, dtype=torch.float64, generator=g).to(dev())
+
+    def both(mirror, **kwargs):
+        C, zy = torch.full((F, F), 2.0, dtype=torch.float64, device=dev()), torch.ones(F, 1, dtype=torch.float64, device=dev())
+        ops.gram(Z, y, C, zy, mirror=mirror, **kwargs)
+        return C, zy
+    expect = [both(mirror) for mirror in (True, False)]
+    real, refused = torch.empty, []
+
+    def empty(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.cuda.OutOfMemoryError("planted")
+        return real(*args, **kwargs)
+    monkeypatch.setattr(torch, "empty", empty)
+    for mirror, (C, zy) in zip((True, False), expect):
+        got, got_y = both(mirror, within_norms=True)
+        assert torch.equal(got, C), mirror
+        # Z^T y is added with atomics, 1 + M terms in any order: two such sums differ by twice the bound of either
+        assert ((got_y - zy).abs() <= 2 * (M + 1) * 2.0 ** -53 * (1 + Z.abs().T @ y.abs())).all()
+    assert len(refused) == 2
+
+
 # 7168 features: the smallest matrix with a slab (3072 rows); 7296: its columns end within a tile of 256; 12288: 8192 rows;
 # 19456: two slabs, of 12288 and 3072 rows
 @pytest.mark.parametrize("F", [7168, 7296, 12288, 19456])
