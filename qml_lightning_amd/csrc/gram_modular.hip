@@ -624,7 +624,11 @@ int qmll_internal_slab_update(double* A, long long ld, int rows, int n, int k, i
 extern "C" size_t qmll_gram_modular_workspace_bytes(int M, int F) {
     // Below MODULAR_MIN_ROWS rows the bytes out of the products and their reconstruction, 2.3 ms at 16384 features whatever
     // the rows, outweigh the sums: 0.87 (fp64 kernel) against 2.3 ms for 128 rows, 1.60 / 2.64 for 320, 3.64 / 3.20 for
-    // 800, 8.6 / 4.7 for 2000; at 1024 features 0.042 / 0.055, 0.086 / 0.082, 0.25 / 0.10 and 0.41 / 0.12 ms.
+    // 800, 8.6 / 4.7 for 2000; at 1024 features 0.042 / 0.055 for 128 and 0.086 / 0.082 for 320.  The line holds at any width: the fp64 kernel has too few tiles to fill the chip where there
+    // are few features, and each of them a long sum, which the integer products cut into row ranges.  us, fp64 kernel / integer
+    // products, 768 rows and 32000: 24 features 168 / 89 and 4872 / 201, 256 (one padded tile) 162 / 98 and 4465 / 222, 512
+    // 162 / 102 and 4481 / 285, 1024 227 / 97 and 4554 / 497, 2048 246 / 125 and 4650 / 1102, 4096 437 / 297 and 9290 / 3552;
+    // 2048 rows 361 / 124, 410 / 136, 417 / 127, 417 / 114, 423 / 158 and 859 / 427.
     if (M < MODULAR_MIN_ROWS || F <= 0) return 0;
     return modular_plan(M, F).bytes;
 }
