@@ -564,7 +564,9 @@ int qmll_copy_upper_f64(const double* A, long long lda, int F, double* U, long l
 int qmll_cholesky_f64(double* A, int F, long long ld, void* workspace, int* info, qmll_stream_t stream);
 
 /* The same with qmll_cholesky_slabs_bytes(F) of device memory more (16-byte aligned, or NULL): large matrices whose F is a multiple of
- * 128 then take the updates by their first rows as exact int8 products.  0 bytes: there are no such rows, NULL is as good. */
+ * 128 then take the updates by their first rows as exact int8 products.  U^T U - A is then smaller in the measure of sqrt(a_ii a_jj), but no longer
+ * bounded by (|U|^T |U|)_ij, which can be far below it: NULL for matrices and right-hand sides of which that is asked.
+ * 0 bytes: there are no such rows, NULL is as good. */
 size_t qmll_cholesky_slabs_bytes(int F);
 int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* workspace, void* slabs, int* info, qmll_stream_t stream);
 

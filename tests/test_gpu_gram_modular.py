@@ -234,8 +234,8 @@ def test_gram_without_memory_for_its_workspace(monkeypatch, M, F):
 # 19456: two slabs, of 12288 and 3072 rows
 @pytest.mark.parametrize("F", [7168, 7296, 12288, 19456])
 def test_factorisation_in_slabs(F):
-    """The residual of the solve within the backward error of a factorisation of that size, the factor next to that of the general
-    path (no workspace for slabs), a pivot that is not positive and a NaN below the slab reported."""
+    """The residual of the solve within the backward error of a factorisation of that size, the factor, and that of the general path (no
+    workspace for slabs), in the measure of the diagonal, a pivot that is not positive and a NaN below the slab reported."""
     from qml_lightning_amd import _lib, ops
     L = _lib.lib()
     g = torch.Generator(device=dev()).manual_seed(9)
@@ -251,7 +251,8 @@ def test_factorisation_in_slabs(F):
     assert int(info.item()) == 0
     # |A x - b| <= c n eps |A| |x| (a backward stable solve; c = 1 is far from what a random matrix shows)
     assert float((A @ x - b).norm()) <= F * 2.0 ** -53 * float(A.norm()) * float(x.norm())
-    # either factor: |U^T U - A| <= (n + 1) eps |U^T||U| entry by entry, and that is at most sqrt(a_ii a_jj) (Higham, theorem 10.3)
+    # fp64 sums: |U^T U - A| <= (n + 1) eps |U^T||U| entry by entry, and that is at most sqrt(a_ii a_jj) (Higham, theorem 10.3); the
+    # integer products err by 2^-57 sqrt(n) sqrt(a_ii a_jj) at most
     work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device=dev())
     slabs = torch.empty(int(L.qmll_cholesky_slabs_bytes(F)), dtype=torch.uint8, device=dev())
     rows = torch.arange(0, F, 997, device=dev())
@@ -272,6 +273,30 @@ def test_factorisation_in_slabs(F):
         assert int(info.item()) == expect if expect else int(info.item()) > 0
         A[row, col] = kept
         A[col, row] = kept
+
+
+def test_solve_of_graded_systems_in_fp64_sums():
+    """Columns that are coupled to one row each and otherwise only by 1e-8, and a right side over ten decades: with fp64 sums asked
+    for, the residual stays entry by entry within that theorem's bound for a solve, (3 n + 1) 2^-53 |U|^T |U| |x|."""
+    from qml_lightning_amd import ops
+    F, n = 7168, 3000
+    g = torch.Generator(device=dev()).manual_seed(1)
+    A = torch.randn(F, F, dtype=torch.float64, device=dev(), generator=g) * 1e-8
+    A = A + A.T
+    i = torch.arange(n, device=dev())
+    A[i, i + 4000] += 0.5
+    A[i + 4000, i] += 0.5
+    A.diagonal().copy_(torch.ones(F))
+    b = torch.randn(F, 1, dtype=torch.float64, device=dev(), generator=g)
+    b *= torch.exp(6.0 * torch.randn(F, 1, dtype=torch.float64, device=dev(), generator=g))
+    x, info = ops.cholesky_solve_spd(A, b, within_norms=False)
+    assert int(info.item()) == 0
+    U = torch.linalg.cholesky(A, upper=True).abs()
+    bound = ((3 * F + 1) * 2.0 ** -53 * (U.T @ (U @ x.abs())))[:, 0].cpu().numpy()
+    An, xn, bn = A.cpu().numpy(), x[:, 0].cpu().numpy().astype(np.longdouble), b[:, 0].cpu().numpy()
+    for lo in range(0, F, 512):
+        r = np.abs(bn[lo:lo + 512] - An[lo:lo + 512].astype(np.longdouble) @ xn)
+        assert (r <= bound[lo:lo + 512]).all(), (lo, float((r / bound[lo:lo + 512]).max()))
 
 
 def test_solve_without_memory_for_slabs(monkeypatch):
