@@ -4,9 +4,10 @@
 #include <stddef.h>
 #include "gram_tiles.h"     // QMLL_HD
 
-// moduli, and gamma: columns are scaled to a norm in (2^(gamma-1), 2^gamma].  Products of both triangles of many rows lose more to the
-// rounding of an fp64 sum than to operands rounded to 2^-54 of the norm; the rows of a Cholesky factor do not (entries far below
-// their column's norm, sums that nearly vanish), and need the four bits that one modulus more gives.
+// moduli, and gamma: columns are scaled to a norm in (2^(gamma-1), 2^gamma].  Products over rows that are large or small in all columns
+// alike, as training rows are, lose more to the rounding of an fp64 sum than to operands rounded to 2^-54 of the norm; the rows of a
+// Cholesky factor do not (entries far below their column's norm, sums that nearly vanish), and need the four bits that one modulus
+// more gives.
 constexpr int GRAM_MODULI = 14, CHOL_MODULI = 15;
 constexpr int modular_gamma(int moduli) { return moduli == 14 ? 54 : 58; }
 constexpr int NORM_ROWS = 512;     // rows per partial sum of the column norms
