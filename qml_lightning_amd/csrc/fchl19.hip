@@ -722,6 +722,212 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
 }
 
 // ---------------------------------------------------------------------------------
+// forward, one wavefront per central atom, number of elements known to the compiler
+//
+// The same sums as fchl19_forward_kernel for the usual grids (LEAN_RS3 - 3 .. LEAN_RS3 three-body and up to 32 two-body bins), up to
+// five elements, no given list and at most 64 candidates, which one instruction's lanes hold.  That kernel is bound by the number of
+// its instructions, vector, scalar and LDS ones alike (1121 + 615 + 126 per atom of 20 neighbours and three elements), and by the LDS:
+// its bin loop reads 12 bytes per lane for one exponential, and the four SIMDs share 128 bytes a clock.  Here
+//  * the counts of the elements are scalars, so that the pairs' segments need no scan and no LDS, and all loops over elements and
+//    pairs are unrolled;
+//  * a lane holds two radial bins (six triples at a time instead of three), so that one read serves two exponentials, and the sums
+//    of six pairs are exchanged at once: 20 shuffles and one store instead of 24 and six;
+//  * a neighbour's record says where each of its triples stands, and a table entry has 12 bytes instead of 16, so that the whole
+//    list of 29 atoms fits 6.5 KB (a list in pieces costs a search per triple).
+// 967 + 251 + 122 instructions; 86016 atoms of 21, three elements 186 -> 136 us, 131235 atoms of 3 to 29, five elements 337 -> 251,
+// 64000 of 8 82 -> 50, 80000 of 40 413 -> 354.  Vector issue now takes nine tenths of the launch.  Two, four or eight atoms per
+// workgroup (fewer dispatches) and other depths of unrolling made no difference.
+// ---------------------------------------------------------------------------------
+constexpr int LEAN_RS3 = 20, LEAN_SLOTS = 6, LEAN_LANES = 10;    // bins; triples at a time, lanes (two bins each) of each
+template <int NS>
+__global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, float* __restrict__ rep) {
+    constexpr int NP = NS * (NS + 1) / 2;
+    extern __shared__ float smem[];
+    const int lane = threadIdx.x;
+    const int m = a.molIDs[blockIdx.x];
+    const int i = a.atomIDs[blockIdx.x];
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    const int nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
+    float* recA = smem;                                  // [cap][4]: d_ij, 1 / r
+    float* recB = recA + 4 * a.cap;                      // [cap][4]: sk3 r / 2, fc r^-d3, places (below)
+    float* trip = recB + 4 * a.cap;                      // [tcap][3]: sk3 rho, K cos, K sin; before them the two-body factors [cap][3]
+
+    const float* Xm = a.X + (size_t)m * a.n * 3;
+    const int own = lane < a.n ? lane : 0;
+    const float xj = Xm[own * 3 + 0], yj = Xm[own * 3 + 1], zj = Xm[own * 3 + 2];
+    const int et = a.types[(size_t)m * a.n + own];
+    const int z = lane & 31, half = lane >> 5;           // two-body: radial bin, neighbour of two
+    const float rs2v = z < nRs2 ? a.Rs2[z] : 1.0f;
+    const int slot = idiv_small(lane, LEAN_LANES), ll = lane - LEAN_LANES * slot;      // three-body: triple of six, pair of bins
+    const float rs3a = 2 * ll < nRs3 ? a.Rs3[2 * ll] : 0.0f, rs3b = 2 * ll + 1 < nRs3 ? a.Rs3[2 * ll + 1] : 0.0f;
+    const int total = min(a.natoms[m], a.n);
+
+    const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
+    const float sk3 = fsqrt(a.p.eta3 * LOG2E);   // exp(-eta3 (rho - Rs)^2) = exp2(-(sk3 rho - sk3 Rs)^2)
+    const float inv_rc = frcp(a.p.rcut);
+
+    // ---- neighbours: candidate = lane ----
+    float dx = Xm[i * 3 + 0] - xj, dy = Xm[i * 3 + 1] - yj, dz = Xm[i * 3 + 2] - zj;
+    if (a.cell != nullptr) min_image(dx, dy, dz, a.cell + (size_t)m * 9, a.inv_cell + (size_t)m * 9);
+    const float r2 = dx * dx + dy * dy + dz * dz;
+    const bool near = lane < total && r2 < a.p.rcut * a.p.rcut && r2 > 0.0f;
+    int count[NS], first[NS], rounds[NP], base[NP];
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int rank = 0, nn = 0;
+#pragma unroll
+    for (int e = 0; e < NS; ++e) {
+        const unsigned long long mask = __ballot(near && et == e);
+        count[e] = __popcll(mask);
+        first[e] = nn;
+        nn += count[e];
+        if (et == e) rank = __popcll(mask & below);
+    }
+    // the triples of an element pair are consecutive in the table, pairs row by row, each part padded to whole rounds
+    int length = 0;
+#pragma unroll
+    for (int p = 0, pq = 0; p < NS; ++p)
+#pragma unroll
+        for (int q = p; q < NS; ++q, ++pq) {
+            const int n = p == q ? (count[p] * (count[p] - 1)) >> 1 : count[p] * count[q];
+            rounds[pq] = (unsigned)(n + LEAN_SLOTS - 1) / LEAN_SLOTS;
+            base[pq] = length;
+            length += LEAN_SLOTS * rounds[pq];
+        }
+    if (near && et >= 0 && et < NS) {
+        // Where a triple of neighbours j < k (in list order) stands: place[type of j] + j, from k's record.  Five places of 11 bits
+        // and, above them, 11 times k's own type.  (A place is not negative: with type p there, the parts before (p, q) hold
+        // at least one triple for each neighbour of an earlier type.)
+        unsigned lo = 0, hi = 0;
+        int pos = rank;
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+            if (et == q) {
+                unsigned t[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+                for (int p = 0; p <= q; ++p) {
+                    const int pq = p * NS - p * (p - 1) / 2 + q - p;
+                    t[p] = (unsigned)(base[pq] - first[p] + (p == q ? __mul24(rank, rank - 1) >> 1 : __mul24(rank, count[p]))) & 0x7ff;
+                }
+                lo = t[0] | t[1] << 11 | t[2] << 22;
+                hi = t[2] >> 10 | t[3] << 1 | t[4] << 12 | (unsigned)(11 * q) << 23;
+                pos = rank + first[q];
+            }
+        }
+        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        float fc, dfc;
+        cutoff(r, inv_rc, fc, dfc);
+        const float l2r = flog2(r);
+        const float s2 = flog(fmaf(a.p.eta2 * ir, ir, 1.0f));
+        reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, ir);
+        reinterpret_cast<float4*>(recB)[pos] = make_float4(sk3 * 0.5f * r, fc * fexp2(-a.p.three_body_decay * l2r),
+                                                           __uint_as_float(lo), __uint_as_float(hi));
+        float* f2 = trip + 3 * pos;                       // mu, log2(e) / (2 sigma^2), r^-d2 fc / (sigma sqrt(2 pi))
+        f2[0] = fmaf(l2r, 0.6931471805599453f, -0.5f * s2);
+        f2[1] = 0.5f * LOG2E * frcp(s2);
+        f2[2] = frsq(s2) * 0.3989422804014327f * fexp2(-a.p.two_body_decay * l2r) * fc;
+    }
+    __syncthreads();
+
+    float* out = rep + ((size_t)m * a.n + i) * (NS * nRs2 + 2 * NP * nRs3);
+    // ---- two-body blocks ----
+    {
+        const float lnRs = flog(rs2v), invRs = frcp(rs2v);
+#pragma unroll
+        for (int e = 0; e < NS; ++e) {
+            const float* f = trip + 3 * (first[e] + half);
+            float acc = 0.0f;
+            auto add = [&](const float* at, bool there) {
+                float3v v;
+                __builtin_memcpy(&v, at, sizeof v);
+                const float u = lnRs - v.x;
+                acc = fmaf(there ? v.z : 0.0f, fexp2(-u * u * v.y), acc);
+            };
+            const int twos = count[e] >> 1;
+#pragma unroll 2
+            for (int it = 0; it < twos; ++it, f += 6) add(f, true);
+            if (count[e] & 1) add(half ? f - 3 : f, half == 0);
+            acc *= invRs;
+            acc += lane_xor<32>(acc);
+            if (lane < nRs2) out[e * nRs2 + lane] = acc;
+        }
+    }
+    __syncthreads();
+
+    // ---- the table ----
+    {
+        const float zw3 = zeta2 * a.p.three_body_weight, hd3 = -0.5f * a.p.three_body_decay;
+        const float4* rA = reinterpret_cast<const float4*>(recA);
+        const float4* rB = reinterpret_cast<const float4*>(recB);
+        for (int t = lane; 4 * t < 3 * length; t += QMLL_WAVE)               // the padding
+            reinterpret_cast<float4*>(trip)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+        const int ntrip = (nn * (nn - 1)) >> 1;
+        for (int tt = lane; tt < ntrip; tt += QMLL_WAVE) {
+            int j, k;
+            unrank_pair_kmajor(tt, j, k);
+            const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
+            const unsigned long long places = (unsigned long long)__float_as_uint(Bk.w) << 32 | __float_as_uint(Bk.z);
+            const int at = (int)((unsigned)(places >> (__float_as_uint(Bj.w) >> 23)) & 0x7ff) + j;
+            const float4 v = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
+            const float3v w = {v.x, v.y, v.z};
+            __builtin_memcpy(trip + 3 * at, &w, sizeof w);
+        }
+    }
+    __syncthreads();
+
+    // ---- three-body blocks ----
+    const float rsa = sk3 * rs3a, rsb = sk3 * rs3b;
+    const float* src = trip + (slot < LEAN_SLOTS ? 3 * slot : 0);
+    float* out3 = out + NS * nRs2;
+#pragma unroll
+    for (int g = 0; g < NP; g += LEAN_SLOTS) {
+        float v[LEAN_SLOTS][4];
+#pragma unroll
+        for (int s = 0; s < LEAN_SLOTS; ++s) {
+            float c0 = 0.f, s0 = 0.f, c1 = 0.f, s1 = 0.f;
+            if (g + s < NP) {
+#pragma unroll 2
+                for (int it = 0; it < rounds[g + s < NP ? g + s : 0]; ++it, src += 3 * LEAN_SLOTS) {
+                    float3v t;
+                    __builtin_memcpy(&t, src, sizeof t);
+                    const float d0 = t.x - rsa, d1 = t.x - rsb;
+                    const float e0 = fexp2(-d0 * d0), e1 = fexp2(-d1 * d1);
+                    c0 = fmaf(e0, t.y, c0);
+                    s0 = fmaf(e0, t.z, s0);
+                    c1 = fmaf(e1, t.y, c1);
+                    s1 = fmaf(e1, t.z, s1);
+                }
+            }
+            v[s][0] = c0, v[s][1] = s0, v[s][2] = c1, v[s][3] = s1;
+        }
+        // the six slots' sums of six element pairs: slot s ends up with pair s.  First between slots s and s + 3, each of which keeps
+        // three of the pairs, then among the three slots that hold the same three
+        float w[3][4];
+        const bool upper = slot >= 3;
+        const int other = upper ? lane - 30 : lane + 30;
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) w[s][c] = (upper ? v[s + 3][c] : v[s][c]) + __shfl(upper ? v[s][c] : v[s + 3][c], other, 64);
+        const int h = upper ? slot - 3 : slot;
+        const int next = h == 2 ? lane - 20 : lane + 10, last = h == 0 ? lane + 20 : lane - 10;
+        float4 o;
+        float* po = &o.x;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float mine = h == 0 ? w[0][c] : h == 1 ? w[1][c] : w[2][c];
+            const float from_next = __shfl(h == 0 ? w[2][c] : h == 1 ? w[0][c] : w[1][c], next, 64);    // the slot after this one: what it holds of mine
+            const float from_last = __shfl(h == 0 ? w[1][c] : h == 1 ? w[2][c] : w[0][c], last, 64);
+            po[c] = mine + from_next + from_last;
+        }
+        if (slot < LEAN_SLOTS && g + slot < NP) {
+            float* to = out3 + 2 * ((g + slot) * nRs3 + 2 * ll);
+            if (2 * ll + 1 < nRs3) __builtin_memcpy(to, &o, 16);
+            else if (2 * ll < nRs3) __builtin_memcpy(to, &o, 8);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // forward, several wavefronts per central atom
 //
 // For neighbourhoods too large for one wavefront's table (beyond 46 atoms) and for batches of few atoms, where one
@@ -1635,6 +1841,13 @@ int wavefronts_backward(int A, long long triples, bool big) {
     return big ? 4 : 1;
 }
 
+// What the kernels for a known number of elements take: five, because a place in the triple list has 11 bits of a 64-bit record; one
+// candidate per lane; two-body bins on half a wavefront; and three-body bins that fill at least 17 of the 20 they are laid out
+// for, where the general kernels have three sub-slots as well (with 16 they have four).
+bool lean_grids(const qmll_fchl_params* prm, const int* nlist, int n) {
+    return nlist == nullptr && prm->nspecies <= 5 && n <= QMLL_WAVE && prm->nRs2 <= 32 && prm->nRs3 <= LEAN_RS3 && prm->nRs3 > LEAN_RS3 - 4;
+}
+
 }  // namespace
 
 extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float* cell, const float* inv_cell,
@@ -1675,6 +1888,22 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
         else if (nw == 4) hipLaunchKernelGGL(fchl19_forward_wide_kernel<4>, dim3(A), dim3(256), lds, st, a, rep);
         else if (nw == 2) hipLaunchKernelGGL(fchl19_forward_wide_kernel<2>, dim3(A), dim3(128), lds, st, a, rep);
         else hipLaunchKernelGGL(fchl19_forward_wide_kernel<1>, dim3(A), dim3(64), lds, st, a, rep);
+        QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
+        return QMLL_OK;
+    }
+    if (lean_grids(prm, nlist, n)) {
+        const size_t entries = std::max<size_t>(alltrip + np * (LEAN_SLOTS - 1), a.cap);
+        const size_t lds = sizeof(float) * ((size_t)8 * a.cap + (3 * entries + 3) / 4 * 4);
+        auto launch = [&](auto nsc) {
+            hipLaunchKernelGGL(fchl19_forward_lean_kernel<decltype(nsc)::value>, dim3(A), dim3(64), lds, st, a, rep);
+        };
+        switch (ns) {
+            case 1: launch(std::integral_constant<int, 1>{}); break;
+            case 2: launch(std::integral_constant<int, 2>{}); break;
+            case 3: launch(std::integral_constant<int, 3>{}); break;
+            case 4: launch(std::integral_constant<int, 4>{}); break;
+            default: launch(std::integral_constant<int, 5>{}); break;
+        }
         QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
         return QMLL_OK;
     }
