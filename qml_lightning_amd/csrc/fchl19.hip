@@ -1491,6 +1491,280 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
 }
 
 // ---------------------------------------------------------------------------------
+// VJP, one wavefront per central atom, number of elements known to the compiler
+//
+// The same sums as fchl19_vjp_kernel<1> where fchl19_forward_lean_kernel has those of the forward kernel, and for the same reasons:
+// that kernel takes 1640 vector, 434 scalar and 137 LDS instructions per atom of 20 neighbours, and its bin loop reads 12 bytes per lane and
+// bin, six clocks of the LDS that four SIMDs share.  Here the grid is on scalar registers, the two bins of a 16-byte read are unrolled
+// with their places as constants, a lane stages the gradient of one radial bin of three pairs at a time (its constant factor is then in
+// a register), and the number of a triple's pair comes from the neighbours' records in two instructions: 1426 + 288 + 98 instructions.
+// 86016 atoms of 21, three elements 193 -> 165 us, 131235 atoms of 3 to 29, five elements 342 -> 290, 64000 of 8 89 -> 63, 80000 of 40
+// 476 -> 446.  Vector issue takes five sixths of the launch.
+// ---------------------------------------------------------------------------------
+template <int NS>
+__global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const float* __restrict__ grad_rep, float* __restrict__ grad_X) {
+    constexpr int NP = NS * (NS + 1) / 2;
+    constexpr int STEP = 3 * LEAN_RS3;                   // entries of the gradient's three-body part per load of the wavefront
+    extern __shared__ float smem[];
+    const int lane = threadIdx.x;
+    const int m = a.molIDs[blockIdx.x];
+    const int i = a.atomIDs[blockIdx.x];
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    const int nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
+    float* recA = smem;                                  // [cap][4]: d_ij, r
+    float* recB = recA + 4 * a.cap;                      // [cap][4]: 1 / r, fc, dfc / dr, the type's pairs (below)
+    float* force = recB + 4 * a.cap;                     // [tcap][4] forces on the neighbours, in copies
+    float* gin3 = force + 4 * a.tcap;                    // [NP][LEAN_RS3][2] incoming gradient of the three-body bins
+    float* gin2 = gin3 + 2 * NP * LEAN_RS3;              // [NS][32] and of the two-body ones, each divided by its Rs2
+    float* slnRs2 = gin2 + 32 * NS;                      // [32]
+    int* sj = (int*)(slnRs2 + 32);                       // [cap] atom index of neighbour j
+
+    const float* Xm = a.X + (size_t)m * a.n * 3;
+    const int own = lane < a.n ? lane : 0;
+    const float xo = Xm[own * 3 + 0], yo = Xm[own * 3 + 1], zo = Xm[own * 3 + 2];
+    const int et = a.types[(size_t)m * a.n + own];
+    const int total = min(a.natoms[m], a.n);
+    const int z = lane & 31;
+    const float rs2v = z < nRs2 ? a.Rs2[z] : 1.0f;
+    // three pairs' bins at a time: a lane has the same bin each time
+    const int third = idiv_small(lane, LEAN_RS3), l3 = lane - LEAN_RS3 * third;
+    const bool bin_ok = lane < STEP && l3 < nRs3;
+    const float rs3v = bin_ok ? a.Rs3[l3] : 0.0f;
+    const float* gsrc = grad_rep + ((size_t)m * a.n + i) * (NS * nRs2 + 2 * NP * nRs3);
+    float g2[(NS + 1) / 2];
+#pragma unroll
+    for (int k = 0; k < (NS + 1) / 2; ++k) {
+        const int e = 2 * k + (lane >> 5);
+        g2[k] = e < NS && z < nRs2 ? gsrc[e * nRs2 + z] : 0.0f;
+    }
+    float2 g3[(NP + 2) / 3];
+#pragma unroll
+    for (int k = 0; k < (NP + 2) / 3; ++k) {
+        g3[k] = make_float2(0.f, 0.f);
+        if (bin_ok && 3 * k + third < NP) __builtin_memcpy(&g3[k], gsrc + NS * nRs2 + 2 * ((3 * k + third) * nRs3 + l3), 8);
+    }
+    for (int t = lane; t < a.tcap; t += QMLL_WAVE) reinterpret_cast<float4*>(force)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+
+    const float inv_rc = frcp(a.p.rcut);
+    const float sk3 = fsqrt(a.p.eta3 * LOG2E);
+    const float hfac = -2.0f * a.p.eta3 * frcp(sk3);
+    const float mid = 0.5f * sk3 * a.p.rcut;             // the radial factor about the middle of the grid: see fchl19_vjp_kernel
+    const bool fast = !__any(bin_ok && !(fabsf(fmaf(sk3, rs3v, -mid)) <= 10.0f));
+    const float shift = fast ? mid : 0.0f;
+    const float ul = bin_ok ? fmaf(sk3, rs3v, -shift) : 0.0f;
+
+    // ---- neighbours: candidate = lane ----
+    float dx = Xm[i * 3 + 0] - xo, dy = Xm[i * 3 + 1] - yo, dz = Xm[i * 3 + 2] - zo;
+    if (a.cell != nullptr) min_image(dx, dy, dz, a.cell + (size_t)m * 9, a.inv_cell + (size_t)m * 9);
+    const float r2 = dx * dx + dy * dy + dz * dz;
+    const bool near = lane < total && r2 < a.p.rcut * a.p.rcut && r2 > 0.0f && et >= 0 && et < NS;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int nn = 0, pos = 0;
+    unsigned pairs = 0;                                  // number of the pair with type p at bits 4p, four times the own type from bit 20
+#pragma unroll
+    for (int e = 0; e < NS; ++e) {
+        const unsigned long long mask = __ballot(near && et == e);
+        if (et == e) {
+            unsigned w = 4u * e << 20;
+#pragma unroll
+            for (int p = 0; p < NS; ++p) {
+                const int lo = p < e ? p : e, hi = p < e ? e : p;
+                w |= (unsigned)(lo * NS - lo * (lo - 1) / 2 + hi - lo) << (4 * p);
+            }
+            pairs = w;
+            pos = nn + __popcll(mask & below);
+        }
+        nn += __popcll(mask);
+    }
+    if (near) {
+        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        float fc, dfc;
+        cutoff(r, inv_rc, fc, dfc);
+        reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, r);
+        reinterpret_cast<float4*>(recB)[pos] = make_float4(ir, fc, dfc, __uint_as_float(pairs));
+        sj[pos] = lane;
+    }
+    // the incoming gradient, times the constant factor of its bin
+    {
+        const float f2 = a.gscale * frcp(rs2v), f3 = a.gscale * (fast ? fexp2(-ul * ul) : 1.0f);
+        if (lane < 32) slnRs2[lane] = flog(rs2v);
+#pragma unroll
+        for (int k = 0; k < (NS + 1) / 2; ++k)
+            if (64 * k + lane < 32 * NS) gin2[64 * k + lane] = g2[k] * f2;
+#pragma unroll
+        for (int k = 0; k < (NP + 2) / 3; ++k)
+            if (lane < STEP && 3 * k + third < NP)
+                reinterpret_cast<float2*>(gin3)[STEP * k + lane] = make_float2(g3[k].x * f3, g3[k].y * f3);
+    }
+    __syncthreads();
+    const float4* rA = reinterpret_cast<const float4*>(recA);
+    const float4* rB = reinterpret_cast<const float4*>(recB);
+    float gix = 0.0f, giy = 0.0f, giz = 0.0f;
+
+    // ---- two-body: lanes = (bin group, neighbour); see fchl19_vjp_kernel ----
+    {
+        const int G = nn > 0 ? idiv_small(64, nn) : 1;       // nn < 64
+        const int g = G > 1 ? idiv_small(lane, nn) : 0, j = lane - g * nn;
+        const bool active = g < G && j < nn;
+        float gr = 0.0f;
+        float4 Aj = make_float4(0.f, 0.f, 0.f, 1.f), Bj = make_float4(1.f, 0.f, 0.f, 0.f);
+        if (active) {
+            Aj = rA[j];
+            Bj = rB[j];
+            const TwoBody tb = two_body_setup(Aj.w, Bj.y, Bj.z, a.p);
+            const float inv_s2 = frcp(tb.s2);
+            const float nc = -0.5f * LOG2E * inv_s2;
+            const float hs = 0.5f * tb.s2p * inv_s2;
+            const float q0 = fmaf(tb.fc, -hs - tb.d2_over_r, tb.dfc);
+            const float q1 = tb.fc * inv_s2 * tb.mup;
+            const float q2 = tb.fc * hs * inv_s2;
+            const float* gz = gin2 + (__float_as_uint(Bj.w) >> 22) * 32 + g;
+            const float* lz = slnRs2 + g;
+            for (int zz = g; zz < nRs2; zz += G, gz += G, lz += G) {
+                const float u = *lz - tb.mu;
+                const float e = fexp2(u * u * nc);
+                gr = fmaf(*gz * e, fmaf(fmaf(q2, u, q1), u, q0), gr);
+            }
+            gr *= tb.pre;
+        }
+        float tot = gr;
+        for (int k = 1; k < G; ++k) tot += __shfl(gr, (lane + nn * k) & 63, 64);
+        if (active && g == 0) {
+            const float ux = Aj.x * Bj.x, uy = Aj.y * Bj.x, uz = Aj.z * Bj.x;   // dr/dR_i
+            gix = tot * ux;
+            giy = tot * uy;
+            giz = tot * uz;
+            reinterpret_cast<float4*>(force)[j] = make_float4(-tot * ux, -tot * uy, -tot * uz, 0.0f);
+        }
+    }
+    __syncthreads();
+
+    // ---- three-body: lane = triple; see fchl19_vjp_kernel for the numbering, the copies and the formulas ----
+    float us[LEAN_RS3];                                  // the grid, on scalar registers
+#pragma unroll
+    for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
+    const int ntrip = (nn * (nn - 1)) >> 1;
+    const float zw3 = 0.014383766711652736f * a.p.three_body_weight;     // 2 exp(-pi^2 / 2)
+    const float d3 = a.p.three_body_decay;
+    const float inn = frcp((float)nn);
+    auto add_force = [&](float* p, float x, float y, float z) {
+        float4 f = *reinterpret_cast<float4*>(p);
+        f.x += x;
+        f.y += y;
+        f.z += z;
+        *reinterpret_cast<float4*>(p) = f;
+    };
+    for (int t0 = 0; t0 < ntrip; t0 += QMLL_WAVE) {
+        const int tt = t0 + lane;
+        if (tt >= ntrip) break;
+        const int s0 = __builtin_amdgcn_readfirstlane((int)(((float)t0 + 0.5f) * inn));
+        const int s = (int)(((float)tt + 0.5f) * inn), j = tt - __mul24(s, nn);
+        int k = j + s + 1;
+        if (k >= nn) k -= nn;
+        float* copy = force + 4 * __mul24(s - s0, nn);
+        const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
+        const float ia = Bj.x, ib = Bk.x;
+        const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
+        const float c2 = cx * cx + cy * cy + cz * cz;
+        const float ic = __builtin_amdgcn_rsqf(c2), c = c2 * ic;
+        const float vi = Aj.x * Ak.x + Aj.y * Ak.y + Aj.z * Ak.z;
+        const float dac = Aj.x * cx + Aj.y * cy + Aj.z * cz;
+        const float dcb = cx * Ak.x + cy * Ak.y + cz * Ak.z;
+        const float w = ia * ib, iaic = ia * ic, ibic = ib * ic;
+        const float ci = vi * w, cj = -dac * iaic, ck = dcb * ibic;
+        // a^2 b^2 - (d_ij.d_ik)^2 = |d_ij x d_ik|^2 (Lagrange): the cross product keeps full
+        // relative accuracy near collinear triples, where the difference of squares cancels
+        const float px = Aj.y * Ak.z - Aj.z * Ak.y, py = Aj.z * Ak.x - Aj.x * Ak.z, pz = Aj.x * Ak.y - Aj.y * Ak.x;
+        const float cross2 = px * px + py * py + pz * pz;
+        const float cosT = fminf(1.0f, fmaxf(-1.0f, ci));
+        const float sinT = fminf(1.0f, fsqrt(cross2) * w);
+        const float guard_inv = Aj.w * Ak.w * __builtin_amdgcn_rsqf(fmaxf(1e-10f, cross2));
+        const float q1 = cj * ck, q2 = ci * ck, q3 = ci * cj;
+        const float X = ci * q1, X2 = X + X;
+        const float P = fmaf(3.0f, X, 1.0f);
+        const float Pa3 = fmaf(q1, ib, fmaf(q2, ic, fmaf(-q3 * Aj.w, ibic, -X2 * ia)));
+        const float Pb3 = fmaf(q1, ia, fmaf(q3, ic, fmaf(-q2 * Ak.w, iaic, -X2 * ib)));
+        const float Pc3 = fmaf(q2, ia, fmaf(q3, ib, fmaf(-q1 * c, w, -X2 * ic)));
+        const float Z = zw3 * fexp2(-d3 * flog2(Aj.w * Ak.w * c));
+        const float fa = Bj.y, dfa = Bj.z, fb = Bk.y, dfb = Bk.z;
+        const float F = fa * fb, d3P = d3 * P, FP = F * P;
+        const float ka = fmaf(F, fmaf(3.0f, Pa3, -d3P * ia), P * dfa * fb);   // K_a / dec
+        const float kb = fmaf(F, fmaf(3.0f, Pb3, -d3P * ib), P * fa * dfb);
+        const float kc = F * fmaf(3.0f, Pc3, -d3P * ic);
+        // the bins of this triple's pair of types
+        const unsigned pair = __builtin_amdgcn_ubfe(__float_as_uint(Bk.w), __float_as_uint(Bj.w) >> 20, 4);
+        const float4* g = reinterpret_cast<const float4*>(gin3 + __mul24((int)pair, 2 * LEAN_RS3));
+        const float y = fmaf(sk3 * 0.5f, Aj.w + Ak.w, -shift);
+        float Gc = 0.f, Gs = 0.f, Hc = 0.f, Hs = 0.f;
+        if (fast) {
+            const float y2 = y + y, ny2 = -y * y;
+            auto bin = [&](float gc, float gs, float u) {
+                const float e = fexp2(fmaf(y2, u, ny2));
+                const float ue = u * e;
+                Gc = fmaf(gc, e, Gc);
+                Gs = fmaf(gs, e, Gs);
+                Hc = fmaf(gc, ue, Hc);
+                Hs = fmaf(gs, ue, Hs);
+            };
+#pragma unroll
+            for (int l = 0; l < LEAN_RS3; l += 2) {
+                const float4 gv = g[l / 2];
+                bin(gv.x, gv.y, us[l]);
+                bin(gv.z, gv.w, us[l + 1]);
+            }
+            Hc = fmaf(y, Gc, -Hc);
+            Hs = fmaf(y, Gs, -Hs);
+        } else {
+            auto bin = [&](float gc, float gs, float u) {
+                const float dl = y - u;
+                const float e = fexp2(-(dl * dl));
+                const float de = dl * e;
+                Gc = fmaf(gc, e, Gc);
+                Gs = fmaf(gs, e, Gs);
+                Hc = fmaf(gc, de, Hc);
+                Hs = fmaf(gs, de, Hs);
+            };
+#pragma unroll
+            for (int l = 0; l < LEAN_RS3; l += 2) {
+                const float4 gv = g[l / 2];
+                bin(gv.x, gv.y, us[l]);
+                bin(gv.z, gv.w, us[l + 1]);
+            }
+        }
+        const float S0 = Gc * cosT + Gs * sinT;
+        const float S1 = 0.5f * hfac * (Hc * cosT + Hs * sinT);                   // d rho/da = d rho/db = 1/2
+        const float Sth = (Gc * sinT - Gs * cosT) * guard_inv;                     // multiplies d cos_i
+        const float ea = Z * ia * fmaf(ka, S0, FP * fmaf(Sth, fmaf(-ci, ia, ib), S1));   // (d L / d a) / a
+        const float eb = Z * ib * fmaf(kb, S0, FP * fmaf(Sth, fmaf(-ci, ib, ia), S1));
+        const float ec = Z * ic * fmaf(kc, S0, -FP * Sth * c * w);
+        gix = fmaf(ea, Aj.x, fmaf(eb, Ak.x, gix));
+        giy = fmaf(ea, Aj.y, fmaf(eb, Ak.y, giy));
+        giz = fmaf(ea, Aj.z, fmaf(eb, Ak.z, giz));
+        add_force(copy + 4 * j, fmaf(ec, cx, -ea * Aj.x), fmaf(ec, cy, -ea * Aj.y), fmaf(ec, cz, -ea * Aj.z));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next read sees every lane's write (LDS instructions run in order)
+        add_force(copy + 4 * k, fmaf(-ec, cx, -eb * Ak.x), fmaf(-ec, cy, -eb * Ak.y), fmaf(-ec, cz, -eb * Ak.z));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    __syncthreads();
+    gix = wave_sum(gix);
+    giy = wave_sum(giy);
+    giz = wave_sum(giz);
+    float* gm = grad_X + (size_t)m * a.n * 3;
+    const int ncopies = force_copies(nn);
+    for (int it = lane; it < 3 * (nn + 1); it += QMLL_WAVE) {
+        const int x = idiv_small(it, 3), c = it - 3 * x;
+        float sum = c == 0 ? gix : c == 1 ? giy : giz;   // on atom i itself
+        int to = i;
+        if (x < nn) {
+            to = sj[x];
+            sum = 0.0f;
+            for (int q = 0; q < ncopies; ++q) sum += force[4 * (q * nn + x) + c];
+        }
+        atomicAdd(&gm[to * 3 + c], sum);
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // explicit Jacobian (and the representation itself when rep != NULL)
 //
 // Output-centric and atomic-free: the wavefront of central atom i produces, one target
@@ -1963,6 +2237,21 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
             QMLL_REQUIRE(compact <= LDS_LIMIT, QMLL_ERR_INVALID,
                          "qmll_fchl19_vjp: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", compact, n, R, LDS_LIMIT);
             hipLaunchKernelGGL((fchl19_vjp_kernel<1, true>), dim3(A), dim3(64), compact, st, a, grad_rep, grad_X);
+            break;
+        }
+        if (nw == 1 && lean_grids(prm, nlist, n)) {
+            const int ns = prm->nspecies;
+            const size_t lean = sizeof(float) * ((size_t)9 * a.cap + 4 * (size_t)a.tcap + ns * (ns + 1) * LEAN_RS3 + 32 * (ns + 1));
+            auto launch = [&](auto nsc) {
+                hipLaunchKernelGGL(fchl19_vjp_lean_kernel<decltype(nsc)::value>, dim3(A), dim3(64), lean, st, a, grad_rep, grad_X);
+            };
+            switch (ns) {
+                case 1: launch(std::integral_constant<int, 1>{}); break;
+                case 2: launch(std::integral_constant<int, 2>{}); break;
+                case 3: launch(std::integral_constant<int, 3>{}); break;
+                case 4: launch(std::integral_constant<int, 4>{}); break;
+                default: launch(std::integral_constant<int, 5>{}); break;
+            }
             break;
         }
         if (nw == 4) hipLaunchKernelGGL(fchl19_vjp_kernel<4>, dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);

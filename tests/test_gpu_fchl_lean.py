@@ -5,7 +5,7 @@ import pytest
 
 from oracle import fchl19
 from tests import helpers
-from tests.test_gpu_kernels import REL_REP, close, gpu_prm, make_batch, oracle_prm, t32, ti32
+from tests.test_gpu_kernels import REL_EF, REL_REP, close, gpu_prm, make_batch, oracle_prm, t32, ti32
 
 pytestmark = pytest.mark.gpu
 
@@ -49,6 +49,15 @@ class Batch:
         close(got[:self.B], rep, REL_REP, "rep")
         close(got[-self.B:], rep, REL_REP, "rep of the last copy")
 
+    def backward(self):
+        from qml_lightning_amd import ops
+        g = np.random.default_rng(2).normal(size=(self.B, self.oracle[0].shape[1], self.prm.repsize)).astype(np.float32)
+        v = fchl19.vjp(g, *self.oracle)
+        for scale in (1.0, -1.0):
+            got = ops.fchl_vjp(t32(self.tile(g)), *self.args, scale=scale)
+            close(got[:self.B], scale * v, REL_EF, "vjp")
+            close(got[-self.B:], scale * v, REL_EF, "vjp of the last copy")
+
 
 def batches():
     rng = np.random.default_rng(3)
@@ -78,3 +87,9 @@ ALL = {name: (a, kw) for name, a, kw in batches()}
 def test_forward(name):
     a, kw = ALL[name]
     Batch(*a, **kw).forward()
+
+
+@pytest.mark.parametrize("name", list(ALL))
+def test_backward(name):
+    a, kw = ALL[name]
+    Batch(*a, **kw).backward()
