@@ -936,7 +936,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, flo
 // the table, each sums a run of its entries, and the NW partial blocks are added
 // in a fixed order at the end: deterministic like the kernel above.
 // ---------------------------------------------------------------------------------
-template <int NW>
+template <int NW, bool LEAN>
 __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a, float* __restrict__ rep) {
     extern __shared__ float smem[];
     constexpr int NT = 64 * NW;
@@ -1016,15 +1016,15 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
     pair_segments(goff, pbase, ns, np, lane, 1, trip, 0);   // the same on every wavefront
     __syncthreads();
 
-    const int W3 = nRs3 < 64 ? nRs3 : 64;
-    const int TS = idiv_small(64, W3);
+    const int W3 = LEAN ? LEAN_LANES : nRs3 < 64 ? nRs3 : 64;      // LEAN: two bins per lane, see fchl19_forward_lean_kernel
+    const int TS = LEAN ? LEAN_SLOTS : idiv_small(64, W3);
     const int tsub = idiv_small(lane, W3), ll = lane - tsub * W3;
     constexpr int MAXLB = 4;                             // radial bins handled: up to 4 x 64
     float rsl[MAXLB];
 #pragma unroll
-    for (int b = 0; b < MAXLB; ++b) {
-        const int l = b * 64 + ll;
-        rsl[b] = (b * 64 < nRs3) ? sk3 * sRs3[l < nRs3 ? l : 0] : 0.0f;
+    for (int b = 0; b < (LEAN ? 2 : MAXLB); ++b) {
+        const int l = LEAN ? 2 * ll + b : b * 64 + ll;
+        rsl[b] = (LEAN || b * 64 < nRs3) ? sk3 * sRs3[l < nRs3 ? l : 0] : 0.0f;
     }
     const float zw3 = zeta2 * a.p.three_body_weight, hd3 = -0.5f * a.p.three_body_decay;
     const float4* rA = reinterpret_cast<const float4*>(recA);
@@ -1056,6 +1056,31 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
             const int rounds = idiv_small(count, TS), rest = count - rounds * TS;
             const float4* src = tab + s0 + (tsub < TS ? tsub : 0);
             float* dst = part + ((size_t)pq * NW + wave) * per;
+            if constexpr (LEAN) {
+                float v[4] = {0.f, 0.f, 0.f, 0.f};
+                auto add = [&](const float4* at) {
+                    const float3v t = *reinterpret_cast<const float3v*>(at);
+                    const float d0 = t.x - rsl[0], d1 = t.x - rsl[1];
+                    const float e0 = fexp2(-d0 * d0), e1 = fexp2(-d1 * d1);
+                    v[0] = fmaf(e0, t.y, v[0]);
+                    v[1] = fmaf(e0, t.z, v[1]);
+                    v[2] = fmaf(e1, t.y, v[2]);
+                    v[3] = fmaf(e1, t.z, v[3]);
+                };
+#pragma unroll 2
+                for (int it = 0; it < rounds; ++it) add(src + it * LEAN_SLOTS);
+                if (rest > 0) add(tsub < rest ? src + rounds * LEAN_SLOTS : tab + a.tcap);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    v[c] += __shfl(v[c], lane + 30, 64);
+                    v[c] += __shfl(v[c], lane + 10, 64) + __shfl(v[c], lane + 20, 64);
+                }
+                if (tsub == 0) {                         // this wavefront's words alone
+                    if (2 * ll < nRs3) dst[4 * ll] += v[0], dst[4 * ll + 1] += v[1];
+                    if (2 * ll + 1 < nRs3) dst[4 * ll + 2] += v[2], dst[4 * ll + 3] += v[3];
+                }
+                continue;
+            }
 #pragma unroll
             for (int b = 0; b < MAXLB; ++b) {
                 if (b * 64 < nRs3) {
@@ -1187,7 +1212,8 @@ __host__ __device__ __forceinline__ int force_copies(int nn) {
 // COMPACT (one wavefront): the form for capacities at which the copies above do not fit.  [cap] records of three floats hold
 // as many copies as the atom's own neighbours leave room for, at least one; where an instruction's lanes would need more, its
 // s-rows take turns.
-template <int NW, bool COMPACT = false>
+// LEAN: grids of LEAN_RS3 - 3 .. LEAN_RS3 bins, on scalar registers, as in fchl19_vjp_lean_kernel
+template <int NW, bool COMPACT = false, bool LEAN = false>
 __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const float* __restrict__ grad_rep,
                                                               float* __restrict__ grad_X) {
     extern __shared__ float smem[];
@@ -1199,7 +1225,8 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
     const int ns = a.p.nspecies, nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
     const int R2 = ns * nRs2;                        // two-body part of a representation row
-    const int NE3 = (ns * (ns + 1) / 2) * nRs3;      // (element pair, radial bin) entries of its three-body part
+    const int row3 = LEAN ? LEAN_RS3 : nRs3;         // an element pair's entries as they are staged
+    const int NE3 = (ns * (ns + 1) / 2) * row3;      // (element pair, radial bin) entries of its three-body part
 
     // [cap][4] per neighbour, read with one instruction each: (d_ij, r) and
     // (1 / r, fc, dfc / dr, element type); first in LDS, 16-byte aligned
@@ -1224,7 +1251,13 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // Global loads that do not depend on the neighbourhood (grid tables, the incoming gradient
     // row) are issued first and consumed after the staging, so their latency overlaps the
     // staging's own loads.
-    const float* gsrc = grad_rep + ((size_t)m * a.n + i) * (R2 + 2 * NE3);
+    const float* gsrc = grad_rep + ((size_t)m * a.n + i) * (R2 + ns * (ns + 1) * nRs3);
+    // entry e of the three-body part in the incoming row; negative: a bin that is not there
+    auto source3 = [&](int e) {
+        if (!LEAN) return e;
+        const int pq = idiv_small(e, LEAN_RS3), l = e - pq * LEAN_RS3;
+        return l < nRs3 ? __mul24(pq, nRs3) + l : -1;
+    };
     constexpr int GREG2 = NW > 2 ? 1 : 2, GREG3 = NW > 2 ? 1 : 4 / NW;   // values / (cos, sin) pairs per thread held in registers
     float gr2[GREG2], gr3c[GREG3], gr3s[GREG3];
 #pragma unroll
@@ -1232,8 +1265,9 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
 #pragma unroll
     for (int k = 0; k < GREG3; ++k) {
         const int e = tid + NT * k;
-        gr3c[k] = e < NE3 ? gsrc[R2 + 2 * e] : 0.0f;
-        gr3s[k] = e < NE3 ? gsrc[R2 + 2 * e + 1] : 0.0f;
+        const int from = e < NE3 ? source3(e) : -1;
+        gr3c[k] = from >= 0 ? gsrc[R2 + 2 * from] : 0.0f;
+        gr3s[k] = from >= 0 ? gsrc[R2 + 2 * from + 1] : 0.0f;
     }
     const float rs2v = lane < nRs2 ? a.Rs2[lane] : 1.0f;
     const float rs3v = lane < nRs3 ? a.Rs3[lane] : 0.0f;
@@ -1308,13 +1342,17 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // bin's constant factor s = 2^(-u^2): with e' = exp2(2 y u - y^2) the sums over the bins of g e and
     // of g (x - g_l) e are sum (g s) e' and y sum (g s) e' - sum (g s) (u e')
     auto stage3 = [&](int e, float gc, float gs) {
-        const float s_ = sfac[e - nRs3 * idiv_small(e, nRs3)];
+        const int l = e - row3 * idiv_small(e, row3);
+        const float s_ = sfac[LEAN ? min(l, nRs3 - 1) : l];
         reinterpret_cast<float2*>(gin3)[e] = make_float2(gc * s_, gs * s_);
     };
 #pragma unroll
     for (int k = 0; k < GREG3; ++k)
         if (tid + NT * k < NE3) stage3(tid + NT * k, gr3c[k], gr3s[k]);
-    for (int e = tid + NT * GREG3; e < NE3; e += NT) stage3(e, gsrc[R2 + 2 * e], gsrc[R2 + 2 * e + 1]);
+    for (int e = tid + NT * GREG3; e < NE3; e += NT) {
+        const int from = source3(e);
+        stage3(e, from >= 0 ? gsrc[R2 + 2 * from] : 0.0f, from >= 0 ? gsrc[R2 + 2 * from + 1] : 0.0f);
+    }
     __syncthreads();
 
     float gix = 0.0f, giy = 0.0f, giz = 0.0f;
@@ -1371,6 +1409,12 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     const int ntrip = nn * (nn - 1) / 2;
     const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
     const float d3 = a.p.three_body_decay;
+    float us[LEAN ? LEAN_RS3 : 1];                     // the grid, on scalar registers
+    if constexpr (LEAN) {
+        const float ul = lane < nRs3 ? fmaf(sk3, rs3v, -shift) : 0.0f;
+#pragma unroll
+        for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
+    }
     // copies of the force records that this atom uses: one for every s-row of an instruction, or as many as there is room for
     auto copies = [&] { return COMPACT ? min(force_copies(nn), idiv_small(a.tcap, max(nn, 1))) : force_copies(nn); };
     for (int tt = tid; tt < ntrip; tt += NT) {
@@ -1414,38 +1458,46 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
         // the (element pair, radial bin) entries of this triple's pair
         const int tj = __float_as_int(Bj.w), tk = __float_as_int(Bk.w);
         const int tp = min(tj, tk), tq = max(tj, tk);
-        const float2* g = reinterpret_cast<const float2*>(gin3) + __mul24(nRs3, __mul24(ns, tp) - (__mul24(tp, tp + 1) >> 1) + tq);
+        const float2* g = reinterpret_cast<const float2*>(gin3) + __mul24(row3, __mul24(ns, tp) - (__mul24(tp, tp + 1) >> 1) + tq);
         // exp(-eta3 (rho - Rs)^2) = exp2(-(x - g_l)^2), x = sk3 rho, the grid stored pre-scaled;
         // d e / d rho = -2 eta3 (rho - Rs) e = hfac (x - g_l) e, the factor applied after the sums
         const float y = fmaf(sk3 * 0.5f, Aj.w + Ak.w, -shift);
         float Gc = 0.f, Gs = 0.f, Hc = 0.f, Hs = 0.f;
+        auto bins = [&](auto bin) {
+            if constexpr (LEAN) {
+#pragma unroll
+                for (int l = 0; l < LEAN_RS3; l += 2) {
+                    const float4 gv = reinterpret_cast<const float4*>(g)[l / 2];
+                    bin(gv.x, gv.y, us[l]);
+                    bin(gv.z, gv.w, us[l + 1]);
+                }
+            } else {
+#pragma unroll 4
+                for (int l = 0; l < nRs3; ++l) bin(g[l].x, g[l].y, sRs3[l]);
+            }
+        };
         if (fast) {
             const float y2 = y + y, ny2 = -y * y;
-#pragma unroll 4
-            for (int l = 0; l < nRs3; ++l) {
-                const float2 gv = g[l];
-                const float u = sRs3[l];
+            bins([&](float gc, float gs, float u) {
                 const float e = fexp2(fmaf(y2, u, ny2));
                 const float ue = u * e;
-                Gc = fmaf(gv.x, e, Gc);
-                Gs = fmaf(gv.y, e, Gs);
-                Hc = fmaf(gv.x, ue, Hc);
-                Hs = fmaf(gv.y, ue, Hs);
-            }
+                Gc = fmaf(gc, e, Gc);
+                Gs = fmaf(gs, e, Gs);
+                Hc = fmaf(gc, ue, Hc);
+                Hs = fmaf(gs, ue, Hs);
+            });
             Hc = fmaf(y, Gc, -Hc);
             Hs = fmaf(y, Gs, -Hs);
         } else {
-#pragma unroll 4
-            for (int l = 0; l < nRs3; ++l) {
-                const float2 gv = g[l];
-                const float dl = y - sRs3[l];
+            bins([&](float gc, float gs, float u) {
+                const float dl = y - u;
                 const float e = fexp2(-(dl * dl));
                 const float de = dl * e;
-                Gc = fmaf(gv.x, e, Gc);
-                Gs = fmaf(gv.y, e, Gs);
-                Hc = fmaf(gv.x, de, Hc);
-                Hs = fmaf(gv.y, de, Hs);
-            }
+                Gc = fmaf(gc, e, Gc);
+                Gs = fmaf(gs, e, Gs);
+                Hc = fmaf(gc, de, Hc);
+                Hs = fmaf(gs, de, Hs);
+            });
         }
         const float S0 = Gc * cosT + Gs * sinT;
         const float S1 = 0.5f * hfac * (Hc * cosT + Hs * sinT);                   // d rho/da = d rho/db = 1/2
@@ -2105,21 +2157,33 @@ constexpr size_t LDS_LIMIT = 64 * 1024;
 // and at five elements 12 x 40: forward 11.9 / 10.5 / 10.4, 21 x 48: 14.7 / 13.5 / 18.5 and 10.0 / 9.7 / 10.4.  2016 atoms of 21: 11.7 / 16.6 and
 // 11.3 / 16.6 with 1 / 4.
 // big: the neighbourhood does not fit the one-wavefront kernel, or leaves it few wavefronts per CU.
-int wavefronts_forward(int A, long long triples, bool big) {
+// The kernels for a known number of elements (`lean`) do with fewer instructions per phase, so that one wavefront is the better choice
+// up to some thirty atoms however few there are (us, 1 / 4 / 8 forward, 1 / 4 backward, three elements):
+//   12 x 1, 12 x 40           4.4 / 6.8 / 7.0, 5.0 / 8.0 / 8.4          5.0 / 7.0, 5.4 / 7.7
+//   21 x 1, 21 x 12, 21 x 48  5.9 / 7.7 / 7.5, 6.1 / 8.1 / 7.8, 6.8 / 10.0 / 14.3        7.0 / 7.4, 7.2 / 7.7, 7.6 / 10.2
+//   29 x 1, 29 x 20 (four elements)     8.6 / 9.7 / 9.0, 9.7 / 11.7 / 12.5              10.3 / 9.0, 10.8 / 11.1
+//   32 x 8 (465), 32 x 32     9.1 / 9.0 / 8.3, 10.3 / 11.6 / 16.3       11.3 / 9.2, 11.9 / 13.4
+//   40 x 6 (741), 40 x 25, 40 x 50      11.9 / 10.1 / 8.9, 13.3 / 13.2 / 18.4, 15.5 / 21.8 / 27.6    15.0 / 10.4, 15.9 / 15.4, 21.0 / 23.9
+//   46 x 6 (990), 46 x 22, 46 x 45      15.4 / 13.0 / 12.9, 16.1 / 16.5 / 23.4, 22.4 / 27.6 / 38.1   18.7 / 11.2, 19.4 / 17.2, 31.2 / 28.2
+int wavefronts_forward(int A, long long triples, bool big, bool lean) {
+    if (lean && !big) return triples <= 420 ? 1 : A <= 256 ? 8 : triples > 600 && A <= 768 ? 4 : 1;
     if (A <= 256) return 8;
     if (A <= (triples > 256 ? 2048 : triples > 100 ? 1024 : triples > 30 ? 512 : 256)) return 4;
     return big ? 4 : 1;
 }
-int wavefronts_backward(int A, long long triples, bool big) {
+int wavefronts_backward(int A, long long triples, bool big, bool lean) {
+    if (lean && !big) return A <= (triples > 900 ? 2048 : triples > 600 ? 1024 : triples > 256 ? 512 : 0) ? 4 : 1;
     if (A <= (triples > 256 ? 2048 : triples > 100 ? 768 : 0)) return 4;
     return big ? 4 : 1;
 }
+
+bool usual_bins(const qmll_fchl_params* prm) { return prm->nRs3 <= LEAN_RS3 && prm->nRs3 > LEAN_RS3 - 4; }
 
 // What the kernels for a known number of elements take: five, because a place in the triple list has 11 bits of a 64-bit record; one
 // candidate per lane; two-body bins on half a wavefront; and three-body bins that fill at least 17 of the 20 they are laid out
 // for, where the general kernels have three sub-slots as well (with 16 they have four).
 bool lean_grids(const qmll_fchl_params* prm, const int* nlist, int n) {
-    return nlist == nullptr && prm->nspecies <= 5 && n <= QMLL_WAVE && prm->nRs2 <= 32 && prm->nRs3 <= LEAN_RS3 && prm->nRs3 > LEAN_RS3 - 4;
+    return nlist == nullptr && prm->nspecies <= 5 && n <= QMLL_WAVE && prm->nRs2 <= 32 && usual_bins(prm);
 }
 
 }  // namespace
@@ -2143,7 +2207,7 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     const int ns = prm->nspecies, np = ns * (ns + 1) / 2;
     hipStream_t st = (hipStream_t)stream;
     const bool big = alltrip > TCH_MAX;
-    for (int nw = wavefronts_forward(A, alltrip, big); nw > 1 || big; nw /= 2) {
+    for (int nw = wavefronts_forward(A, alltrip, big, lean_grids(prm, nlist, n)); nw > 1 || big; nw /= 2) {
         // the table holds the triple list, or 12 KB of it at a time
         a.tcap = alltrip <= TCH_WIDE ? (int)alltrip : TCH_WIDE;
         size_t lds = sizeof(float) * (4 * (size_t)(a.tcap + 1) + 12 * (size_t)a.cap + ns + 1 + 2 * prm->nRs2 + prm->nRs3 + np + 1 +
@@ -2158,10 +2222,13 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
                          "qmll_fchl19_forward: %zu B of LDS needed (max_atoms=%d, repsize=%d) exceeds %zu", lds, n, R, LDS_LIMIT);
             continue;
         }
-        if (nw == 8) hipLaunchKernelGGL(fchl19_forward_wide_kernel<8>, dim3(A), dim3(512), lds, st, a, rep);
-        else if (nw == 4) hipLaunchKernelGGL(fchl19_forward_wide_kernel<4>, dim3(A), dim3(256), lds, st, a, rep);
-        else if (nw == 2) hipLaunchKernelGGL(fchl19_forward_wide_kernel<2>, dim3(A), dim3(128), lds, st, a, rep);
-        else hipLaunchKernelGGL(fchl19_forward_wide_kernel<1>, dim3(A), dim3(64), lds, st, a, rep);
+        const bool lean = usual_bins(prm);
+        if (nw == 8 && lean) hipLaunchKernelGGL((fchl19_forward_wide_kernel<8, true>), dim3(A), dim3(512), lds, st, a, rep);
+        else if (nw == 4 && lean) hipLaunchKernelGGL((fchl19_forward_wide_kernel<4, true>), dim3(A), dim3(256), lds, st, a, rep);
+        else if (nw == 8) hipLaunchKernelGGL((fchl19_forward_wide_kernel<8, false>), dim3(A), dim3(512), lds, st, a, rep);
+        else if (nw == 4) hipLaunchKernelGGL((fchl19_forward_wide_kernel<4, false>), dim3(A), dim3(256), lds, st, a, rep);
+        else if (nw == 2) hipLaunchKernelGGL((fchl19_forward_wide_kernel<2, false>), dim3(A), dim3(128), lds, st, a, rep);
+        else hipLaunchKernelGGL((fchl19_forward_wide_kernel<1, false>), dim3(A), dim3(64), lds, st, a, rep);
         QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
         return QMLL_OK;
     }
@@ -2225,9 +2292,11 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     a.tcap = 1;
     for (int k = 1; k <= a.cap; ++k) a.tcap = a.tcap < k * force_copies(k) ? k * force_copies(k) : a.tcap;
     const long long maxnn = nlist ? a.cap : a.cap - 1;
-    for (int nw = wavefronts_backward(A, maxnn * (maxnn - 1) / 2, a.cap > 54);; nw /= 2) {
+    for (int nw = wavefronts_backward(A, maxnn * (maxnn - 1) / 2, a.cap > 54, lean_grids(prm, nlist, n));; nw /= 2) {
         // two records [cap][4], atom indices, force copies, type offsets, grids, the bins' constant factors, the gradient row
-        const size_t shared = (size_t)9 * a.cap + prm->nspecies + 1 + prm->nRs2 + 2 * prm->nRs3 + R;
+        const bool lean4 = nw == 4 && usual_bins(prm);
+        const size_t shared = (size_t)9 * a.cap + prm->nspecies + 1 + prm->nRs2 + 2 * prm->nRs3 + R +
+                              (lean4 ? (size_t)prm->nspecies * (prm->nspecies + 1) * (LEAN_RS3 - prm->nRs3) : 0);
         const size_t lds = sizeof(float) * (shared + 4 * (size_t)nw * a.tcap + (nw > 1 ? (size_t)prm->nspecies * nw : 0));
         if (lds > LDS_LIMIT && nw > 1) continue;
         hipStream_t st = (hipStream_t)stream;
@@ -2254,7 +2323,8 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
             }
             break;
         }
-        if (nw == 4) hipLaunchKernelGGL(fchl19_vjp_kernel<4>, dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);
+        if (lean4) hipLaunchKernelGGL((fchl19_vjp_kernel<4, false, true>), dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);
+        else if (nw == 4) hipLaunchKernelGGL(fchl19_vjp_kernel<4>, dim3(A), dim3(256), lds, st, a, grad_rep, grad_X);
         else if (nw == 2) hipLaunchKernelGGL(fchl19_vjp_kernel<2>, dim3(A), dim3(128), lds, st, a, grad_rep, grad_X);
         else hipLaunchKernelGGL(fchl19_vjp_kernel<1>, dim3(A), dim3(64), lds, st, a, grad_rep, grad_X);
         break;

@@ -1,5 +1,5 @@
-"""FCHL19 with the number of elements known to the compiler (usual grids, one wavefront per atom), at the edges of what takes it:
-element counts, grid sizes, capacities, atoms without neighbours, elements that are absent or unknown, periodic boxes."""
+"""FCHL19 with the number of elements known to the compiler (usual grids, one wavefront per atom) and with several wavefronts for
+few atoms of the same grids, at the edges of what takes them: element counts, grid sizes, capacities, atoms without neighbours, elements that are absent or unknown, periodic boxes."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from tests.test_gpu_kernels import REL_EF, REL_REP, close, gpu_prm, make_batch, 
 
 pytestmark = pytest.mark.gpu
 
-ATOMS = 2400                    # beyond this one wavefront per atom whatever the molecules
+ATOMS = 2400                    # beyond this one wavefront per atom wherever its kernel holds the triples
 
 
 def cube(rng, n, edge):
@@ -19,9 +19,9 @@ def cube(rng, n, edge):
 
 
 class Batch:
-    """Molecules, repeated until one wavefront takes an atom, and what the oracle says of them."""
+    """Molecules, repeated to at least `atoms` atoms, and what the oracle says of them."""
 
-    def __init__(self, coords, charges, species, cell=None, **kw):
+    def __init__(self, coords, charges, species, atoms=ATOMS, cell=None, **kw):
         self.prm = prm = oracle_prm(species, **kw)
         X, Z, aid, mid, nat = make_batch(coords, charges)
         B = len(coords)
@@ -35,7 +35,7 @@ class Batch:
             js = [j for j in nl[m, i, :cnt[m, i]] if ty[m, j] >= 0]
             nl[m, i], cnt[m, i] = js + [-1] * (nl.shape[2] - len(js)), len(js)
         self.oracle = (X, ty, aid, mid, nl, cnt, prm, cells, icells)
-        self.B, k = B, ATOMS // len(aid) + 1
+        self.B, k = B, atoms // len(aid) + 1
         tile = lambda a: np.concatenate([a] * k)       # noqa: E731
         box = (None, None) if cell is None else (t32(tile(cells)), t32(tile(icells)))
         self.tile = tile
@@ -76,6 +76,8 @@ def batches():
     # 10.5: beyond what the backward kernel's form about the middle of the grid takes
     c, q = helpers.fixed_composition_batch(helpers.ASPIRIN, 1, 8)
     yield "narrow bins", (c, q, [1, 6, 8]), dict(eta3=12.0)
+    for nrs3 in (17, 19):                               # and more triples than the table of several wavefronts holds
+        yield "box of 70, %d bins" % nrs3, ([cube(rng, 70, 10.0)], [rng.choice([1, 6, 8], 70)], [1, 6, 8]), dict(cell=10.0, nRs3=nrs3)
     for n in (32, 46, 64):                              # 64: several wavefronts
         yield "box of %d" % n, ([cube(rng, n, 9.0)], [rng.choice([1, 6, 8], n)], [1, 6, 8]), dict(cell=9.0)
 
@@ -83,13 +85,15 @@ def batches():
 ALL = {name: (a, kw) for name, a, kw in batches()}
 
 
+@pytest.mark.parametrize("atoms", [1, 300, ATOMS])
 @pytest.mark.parametrize("name", list(ALL))
-def test_forward(name):
+def test_forward(name, atoms):
     a, kw = ALL[name]
-    Batch(*a, **kw).forward()
+    Batch(*a, atoms=atoms, **kw).forward()
 
 
+@pytest.mark.parametrize("atoms", [1, 300, ATOMS])
 @pytest.mark.parametrize("name", list(ALL))
-def test_backward(name):
+def test_backward(name, atoms):
     a, kw = ALL[name]
-    Batch(*a, **kw).backward()
+    Batch(*a, atoms=atoms, **kw).backward()
