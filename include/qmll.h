@@ -164,6 +164,10 @@ int qmll_segment_offsets(const int* mol_index, int A, int nmol, int* seg, qmll_s
 int qmll_cos_features_f32(const float* coeffs, const float* bias, const int* mol_index, const int* seg, int A, int F,
                           int nmol, float* Zf, qmll_stream_t stream);
 
+/* The same with Zf overwritten, the table made on the way: seg i32 [nmol+2], neither of them initialised by the caller. */
+int qmll_cos_features_of_molecules_f32(const float* coeffs, const float* bias, const int* mol_index, int A, int F, int nmol,
+                                       int* seg, float* Zf, qmll_stream_t stream);
+
 /* Replaces sorf_gpu.compute_hadamard_features / compute_molecular_featurization
  * (hadamard_cuda.cpp:89-93; kernel hadamard_kernel.cu:541-563): same as above but every
  * fp32 feature value is widened and accumulated into Zf f64 [nmol,F] (in place). */
@@ -269,6 +273,15 @@ int qmll_sorf_energy_typed(const float* x_all, const int* types, const int* atom
 size_t qmll_sort_by_type_workspace(int A, int ne);
 int qmll_sort_by_type(const int* types, const int* slots, int A, int ne, void* workspace, size_t workspace_bytes,
                       int* sorted_slots, int* type_offsets, qmll_stream_t stream);
+
+/* The slots of a padded batch that hold each of `species`, by charge alone (the masks Z == e of
+ * hadamard_features.py:101-107, all elements at once): Z f32 [nslots] truncated to integers,
+ * species f32 [ne] -> rows i32 [nslots]: the slots of species[0], then of species[1], ..., ascending within
+ * each (zeros behind the last); offsets i32 [ne+1].  Of equal entries in species the last one gets the slots.
+ * workspace: device memory of at least qmll_charge_rows_workspace(nslots, ne) bytes.  ne <= 32. */
+size_t qmll_charge_rows_workspace(int nslots, int ne);
+int qmll_charge_rows(const float* Z, const float* species, int nslots, int ne, void* workspace, size_t workspace_bytes,
+                     int* rows, int* offsets, qmll_stream_t stream);
 
 /* qmll_sort_by_type for the listed atoms of a padded batch: slot of atom a = molIDs[a] * n +
  * atomIDs[a] (the index the reference builds as torch.where(Z == e) over the [B, n] charges,

@@ -51,6 +51,7 @@ PROTOTYPES = {
     "qmll_sorf_forward": [P, P, c_int, c_int, c_int, c_int, c_float, P, P],
     "qmll_sorf_adjoint": [P, P, c_int, c_int, c_int, c_int, c_float, P, P],
     "qmll_segment_offsets": [P, c_int, c_int, P, P],
+    "qmll_cos_features_of_molecules_f32": [P, P, P, c_int, c_int, c_int, P, P, P],
     "qmll_cos_features_f32": [P, P, P, P, c_int, c_int, c_int, P, P],
     "qmll_cos_features_f64": [P, P, P, P, c_int, c_int, c_int, P, P],
     "qmll_cos_features_backward": [P, P, P, P, c_int, c_int, c_int, P, P],
@@ -61,6 +62,8 @@ PROTOTYPES = {
     "qmll_typed_segments": [P, P, c_int, c_int, c_int, P, P],
     "qmll_sorf_energy_fused": [P, P, P, P, P, c_int, c_int, c_int, c_int, c_float, P, P, P],
     "qmll_sorf_energy_typed": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, P, P, P],
+    "qmll_charge_rows_workspace": [c_int, c_int],
+    "qmll_charge_rows": [P, P, c_int, c_int, P, c_size_t, P, P, P],
     "qmll_sort_by_type_workspace": [c_int, c_int],
     "qmll_sort_by_type": [P, P, c_int, c_int, P, c_size_t, P, P, P],
     "qmll_sort_atoms_workspace": [c_int, c_int],

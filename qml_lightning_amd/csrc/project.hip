@@ -46,8 +46,38 @@ __global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ 
     }
 }
 
+// index of charge z in a species list, -1 when it is not there (the rule of element_types_kernel)
+__device__ __forceinline__ int species_index(float z, const float* __restrict__ species, int ns) {
+    const int q = (int)z;
+    int t = -1;
+    for (int j = 0; j < ns; ++j)
+        if (q == (int)species[j]) t = j;
+    return t;
+}
+
+// the same counts from charges, whose element indices are written on the way
+__global__ __launch_bounds__(ST) void charge_count_kernel(const float* __restrict__ Z, const float* __restrict__ species, int A, int ne,
+                                                           int* __restrict__ types, int* __restrict__ counts) {
+    __shared__ int wcnt[ST / 64][MAXNE];
+    const int a = blockIdx.x * ST + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t = a < A ? species_index(Z[a], species, ne) : -1;
+    if (a < A) types[a] = t;
+    for (int e = 0; e < ne; ++e) {
+        const unsigned long long m = __ballot(t == e);
+        if (lane == 0) wcnt[wave][e] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x < ne) {
+        int s = 0;
+#pragma unroll
+        for (int w = 0; w < ST / 64; ++w) s += wcnt[w][threadIdx.x];
+        counts[blockIdx.x * ne + threadIdx.x] = s;
+    }
+}
+
 // sorted[pos] = slot of the atom, pos = start of its type + atoms of that type before it
-// (in workgroups before this one, in wavefronts before this one, in lanes before this one)
+// (in workgroups before this one, in wavefronts before this one, in lanes before this one); slots null: atom a is slot a
 __global__ __launch_bounds__(ST) void type_place_kernel(const int* __restrict__ types, const int* __restrict__ slots,
                                                          int A, int ne, const int* __restrict__ counts, int nb,
                                                          int* __restrict__ sorted, int* __restrict__ offsets) {
@@ -75,7 +105,7 @@ __global__ __launch_bounds__(ST) void type_place_kernel(const int* __restrict__ 
         }
     }
     const int a = b * ST + threadIdx.x;
-    const int slot = a < A ? slots[a] : 0;
+    const int slot = a < A ? (slots ? slots[a] : a) : 0;
     const int t = a < A ? types[slot] : -1;
     int rank = 0;
     for (int e = 0; e < ne; ++e) {
@@ -152,15 +182,6 @@ __global__ __launch_bounds__(SORT_SMALL) void type_sort_small_kernel(const int* 
     if (t >= 0 && t < ne) sorted[start[t] + wcnt[wave][t] + rank] = slot;
     // entries past the last typed atom name a valid slot, so gathers through them stay in bounds
     for (int i = start[ne] + a; i < A; i += SORT_SMALL) sorted[i] = 0;
-}
-
-// index of charge z in a species list, -1 when it is not there (the rule of element_types_kernel)
-__device__ __forceinline__ int species_index(float z, const float* __restrict__ species, int ns) {
-    const int q = (int)z;
-    int t = -1;
-    for (int j = 0; j < ns; ++j)
-        if (q == (int)species[j]) t = j;
-    return t;
 }
 
 // Everything a small padded batch needs before its first compute kernel, in ONE workgroup: the element
@@ -1122,6 +1143,35 @@ extern "C" int qmll_sort_by_type(const int* types, const int* slots, int A, int 
                        sorted_slots, type_offsets);
     QMLL_CHECK_LAUNCH("qmll_sort_by_type");
     return QMLL_OK;
+}
+
+extern "C" int qmll_charge_rows(const float* Z, const float* species, int nslots, int ne, void* workspace, size_t workspace_bytes,
+                                int* rows, int* offsets, qmll_stream_t stream) {
+    QMLL_REQUIRE(nslots >= 0 && ne > 0 && ne <= MAXNE, QMLL_ERR_INVALID, "qmll_charge_rows: bad size nslots=%d ne=%d (at most %d elements)",
+                 nslots, ne, MAXNE);
+    QMLL_REQUIRE(offsets, QMLL_ERR_INVALID, "qmll_charge_rows: null pointer");
+    if (nslots == 0) {
+        hipLaunchKernelGGL(zero_ints_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, offsets, ne + 1);
+        QMLL_CHECK_LAUNCH("qmll_charge_rows");
+        return QMLL_OK;
+    }
+    QMLL_REQUIRE(Z && species && rows && workspace, QMLL_ERR_INVALID, "qmll_charge_rows: null pointer");
+    QMLL_REQUIRE(workspace_bytes >= qmll_charge_rows_workspace(nslots, ne), QMLL_ERR_INVALID,
+                 "qmll_charge_rows: workspace of %zu bytes, %zu needed", workspace_bytes, qmll_charge_rows_workspace(nslots, ne));
+    const int nb = (nslots + ST - 1) / ST;
+    int* counts = static_cast<int*>(workspace);
+    int* types = counts + (size_t)nb * ne;
+    hipLaunchKernelGGL(charge_count_kernel, dim3(nb), dim3(ST), 0, (hipStream_t)stream, Z, species, nslots, ne, types, counts);
+    QMLL_CHECK_LAUNCH("qmll_charge_rows");
+    hipLaunchKernelGGL(type_place_kernel, dim3(nb), dim3(ST), 0, (hipStream_t)stream, types, (const int*)nullptr, nslots, ne, counts, nb,
+                       rows, offsets);
+    QMLL_CHECK_LAUNCH("qmll_charge_rows");
+    return QMLL_OK;
+}
+
+extern "C" size_t qmll_charge_rows_workspace(int nslots, int ne) {
+    if (nslots <= 0 || ne <= 0) return 0;
+    return qmll_sort_by_type_workspace(nslots, ne) + sizeof(int) * (size_t)nslots;
 }
 
 extern "C" size_t qmll_sort_atoms_workspace(int A, int ne) {

@@ -1465,20 +1465,41 @@ __global__ void segment_offsets_kernel(const int* __restrict__ mol_index, int A,
     for (int m = prev + 1; m <= cur; ++m) seg[m] = t;
 }
 
+// The same table by one workgroup, which needs no cleared flag.  Bound by launches where it is used: of the operator sequence's 76
+// launches for four elements (512 molecules of 3 to 29 atoms, 955 us, the host's) this and rows written instead of added to
+// zeros take 8, the search by charge_rows another eleven: 841 us.  Beyond 16 atoms per thread the table by many workgroups.
+constexpr int SEG_THREADS = 1024, SEG_ATOMS = 16 * SEG_THREADS;
+__global__ __launch_bounds__(SEG_THREADS) void segment_table_kernel(const int* __restrict__ mol_index, int A, int nmol, int* __restrict__ seg) {
+    bool bad = false;
+    for (int t = threadIdx.x; t <= A; t += SEG_THREADS) {
+        const int prev = t == 0 ? -1 : mol_index[t - 1];
+        const int cur = t == A ? nmol : mol_index[t];
+        if (prev > cur || cur < 0 || cur > nmol || (t < A && cur == nmol)) bad = true;
+        else
+            for (int m = prev + 1; m <= cur; ++m) seg[m] = t;
+    }
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) seg[nmol + 1] = bad;
+}
+__global__ void clear_flag_kernel(int* __restrict__ p) { *p = 0; }
+
 // Segmented, atomic-free cos features for molecule-major atoms: workgroup = (molecule,
 // feature tile); the molecule's atoms are streamed with four rows in flight, summed in
 // registers in atom order and added into Zf once (each Zf element has one owner).  Does
 // nothing when the segment table is flagged invalid; the atomic kernel then does the work.
-template <typename OutT, int V>
+// OVERWRITE: a molecule's row is written, with zeros where it has no atoms (and everywhere when the table is invalid, for the
+// atomics that follow), instead of added to.
+template <typename OutT, int V, bool OVERWRITE = false>
 __global__ __launch_bounds__(CF_THREADS) void cos_features_seg_kernel(const float* __restrict__ coeffs,
                                                                        const float* __restrict__ bias,
                                                                        const int* __restrict__ seg, int F, int nmol,
                                                                        float normf, OutT* __restrict__ Zf) {
-    if (seg[nmol + 1] != 0) return;
+    const bool invalid = seg[nmol + 1] != 0;
+    if (invalid && !OVERWRITE) return;
     const int mol = blockIdx.x;
     const int f = (blockIdx.y * CF_THREADS + threadIdx.x) * V;
-    const int a0 = seg[mol], a1 = seg[mol + 1];
-    if (f >= F || a1 <= a0) return;
+    const int a0 = invalid ? 0 : seg[mol], a1 = invalid ? 0 : seg[mol + 1];
+    if (f >= F || (a1 <= a0 && !OVERWRITE)) return;
     float b[V];
     load_f<V>(b, bias + f);
     OutT run[V];
@@ -1501,7 +1522,7 @@ __global__ __launch_bounds__(CF_THREADS) void cos_features_seg_kernel(const floa
     }
     OutT* z = Zf + (size_t)mol * F + f;
 #pragma unroll
-    for (int q = 0; q < V; ++q) z[q] += run[q];
+    for (int q = 0; q < V; ++q) z[q] = OVERWRITE ? run[q] : z[q] + run[q];
 }
 
 template <int V>
@@ -1940,6 +1961,11 @@ static dim3 feat_grid(int A, int F, int V) {
     return dim3((A + CF_ATOMS - 1) / CF_ATOMS, (F + CF_THREADS * V - 1) / (CF_THREADS * V));
 }
 
+// four columns per thread; small batches take one so that the grid still fills the device
+static bool seg_wide(int F, int nmol) {
+    return F % 4 == 0 && (long long)nmol * ((F + CF_THREADS * 4 - 1) / (CF_THREADS * 4)) >= 2048;
+}
+
 // launches of the forward feature kernels: segmented when a segment table is given (with
 // the atomic kernel behind it for a table flagged invalid), atomic otherwise
 template <typename OutT>
@@ -1951,9 +1977,7 @@ static int launch_cos_features(const char* who, const float* coeffs, const float
     QMLL_REQUIRE(coeffs && bias && mol_index && Zf, QMLL_ERR_INVALID, "%s: null pointer", who);
     const float normf = sqrtf(2.0f / (float)F);
     if (seg != nullptr && nmol > 0) {
-        // small batches take one column per thread so that the grid still fills the device
-        const bool wide = F % 4 == 0 && (long long)nmol * ((F + CF_THREADS * 4 - 1) / (CF_THREADS * 4)) >= 2048;
-        if (wide)
+        if (seg_wide(F, nmol))
             hipLaunchKernelGGL((cos_features_seg_kernel<OutT, 4>), dim3(nmol, (F + CF_THREADS * 4 - 1) / (CF_THREADS * 4)),
                                dim3(CF_THREADS), 0, stream, coeffs, bias, seg, F, nmol, normf, Zf);
         else
@@ -1977,6 +2001,40 @@ extern "C" int qmll_segment_offsets(const int* mol_index, int A, int nmol, int* 
     hipLaunchKernelGGL(segment_offsets_kernel, dim3(A / 256 + 1), dim3(256), 0, (hipStream_t)stream, mol_index, A, nmol,
                        seg);
     QMLL_CHECK_LAUNCH("qmll_segment_offsets");
+    return QMLL_OK;
+}
+
+extern "C" int qmll_cos_features_of_molecules_f32(const float* coeffs, const float* bias, const int* mol_index, int A, int F, int nmol,
+                                                  int* seg, float* Zf, qmll_stream_t stream) {
+    const char* who = "qmll_cos_features_of_molecules_f32";
+    int rc = check_feat(who, A, F, nmol);
+    if (rc) return rc;
+    if (nmol == 0) return QMLL_OK;
+    QMLL_REQUIRE(bias && seg && Zf && (A == 0 || (coeffs && mol_index)), QMLL_ERR_INVALID, "%s: null pointer", who);
+    hipStream_t st = (hipStream_t)stream;
+    if (A <= SEG_ATOMS) {
+        hipLaunchKernelGGL(segment_table_kernel, dim3(1), dim3(SEG_THREADS), 0, st, mol_index, A, nmol, seg);
+    } else {
+        hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, st, seg + nmol + 1);
+        hipLaunchKernelGGL(segment_offsets_kernel, dim3(A / 256 + 1), dim3(256), 0, st, mol_index, A, nmol, seg);
+    }
+    QMLL_CHECK_LAUNCH(who);
+    const float normf = sqrtf(2.0f / (float)F);
+    if (seg_wide(F, nmol))
+        hipLaunchKernelGGL((cos_features_seg_kernel<float, 4, true>), dim3(nmol, (F + CF_THREADS * 4 - 1) / (CF_THREADS * 4)),
+                           dim3(CF_THREADS), 0, st, coeffs, bias, seg, F, nmol, normf, Zf);
+    else
+        hipLaunchKernelGGL((cos_features_seg_kernel<float, 1, true>), dim3(nmol, (F + CF_THREADS - 1) / CF_THREADS), dim3(CF_THREADS), 0,
+                           st, coeffs, bias, seg, F, nmol, normf, Zf);
+    QMLL_CHECK_LAUNCH(who);
+    if (A == 0) return QMLL_OK;
+    if (F % 4 == 0)
+        hipLaunchKernelGGL((cos_features_kernel<float, 4>), feat_grid(A, F, 4), dim3(CF_THREADS), 0, st, coeffs, bias, mol_index, seg, A, F,
+                           nmol, normf, Zf);
+    else
+        hipLaunchKernelGGL((cos_features_kernel<float, 1>), feat_grid(A, F, 1), dim3(CF_THREADS), 0, st, coeffs, bias, mol_index, seg, A, F,
+                           nmol, normf, Zf);
+    QMLL_CHECK_LAUNCH(who);
     return QMLL_OK;
 }
 

@@ -329,13 +329,12 @@ Tensor cos_features_impl(const Tensor& coeffs, const Tensor& b, const Tensor& nm
     const int A = (int)c.size(0), F = (int)c.size(1), nmol = nmol_t.item<int>();                     // SORF.cpp:118
     TORCH_CHECK(bb.numel() == F && idx.numel() == A, "get_cos_features: coefficients are [", c.sizes(), "], bias has ",
                 bb.numel(), " entries, batch_indexes ", idx.numel());
-    Tensor out = at::zeros({nmol, F}, c.options());
-    if (A == 0) return out;
-    // segment table of the (ascending) molecule index, validated on the device
-    Tensor seg = at::zeros({nmol + 2}, c.options().dtype(at::kInt));
-    check(qmll_segment_offsets(ip(idx), A, nmol, seg.data_ptr<int>(), stream()), "qmll_segment_offsets");
-    check(qmll_cos_features_f32(fp(c), fp(bb), ip(idx), ip(seg), A, F, nmol, out.data_ptr<float>(), stream()),
-          "qmll_cos_features_f32");
+    if (A == 0) return at::zeros({nmol, F}, c.options());
+    // (the molecule index is ascending as a rule; that is looked at on the device)
+    Tensor out = at::empty({nmol, F}, c.options()), seg = at::empty({nmol + 2}, c.options().dtype(at::kInt));
+    check(qmll_cos_features_of_molecules_f32(fp(c), fp(bb), ip(idx), A, F, nmol, seg.data_ptr<int>(),
+                                             nmol ? out.data_ptr<float>() : nullptr, stream()),
+          "qmll_cos_features_of_molecules_f32");
     return out;
 }
 
@@ -476,6 +475,21 @@ std::tuple<Tensor, Tensor> sort_by_type(const Tensor& types, const Tensor& slots
                             A ? sorted.data_ptr<int>() : nullptr, offsets.data_ptr<int>(), stream()),
           "qmll_sort_by_type");
     return {sorted, offsets};
+}
+
+// rows of the flattened charges that hold each of `species`, and where each one's begin: qmll_charge_rows
+std::tuple<Tensor, Tensor> charge_rows(const Tensor& charges, const Tensor& species) {
+    need_cuda(charges, "charges");
+    need_cuda(species, "species");
+    Tensor Z = f32(charges).reshape({-1}), sp = f32(species);
+    const int N = (int)Z.size(0), ne = (int)sp.size(0);
+    Tensor rows = at::empty({N}, Z.options().dtype(at::kInt)), offsets = at::empty({ne + 1}, rows.options());
+    const size_t nbytes = qmll_charge_rows_workspace(N, ne);
+    Tensor work = at::empty({(int64_t)std::max<size_t>(nbytes / 4, 1)}, rows.options());
+    check(qmll_charge_rows(fp(Z), fp(sp), N, ne, work.data_ptr<int>(), nbytes, N ? rows.data_ptr<int>() : nullptr,
+                           offsets.data_ptr<int>(), stream()),
+          "qmll_charge_rows");
+    return {rows, offsets};
 }
 
 // sort_by_type of the listed atoms of a padded batch (slot = molIDs * n + atomIDs), one launch for small batches
@@ -919,6 +933,7 @@ TORCH_LIBRARY(qml_lightning_sorf, m) {
     m.def("sorf_energy", &sorf_energy);
     m.def("sorf_energy_typed", &sorf_energy_typed);
     m.def("sort_by_type", &sort_by_type);
+    m.def("charge_rows", &charge_rows);
     m.def("project_typed", &project_typed);
     m.def("project_typed_backward", &project_typed_backward);
     m.def("sorf_energy_sorted", &sorf_energy_sorted);

@@ -8,7 +8,7 @@ and differentiable in X.  With `fused=False` it is the reference's own operator 
 [atoms, nfeatures] coefficients and already returns the gradient with respect to the
 projected representation; the numbers are the same.
 """
-from typing import Final, List, Optional
+from typing import Final, List, Optional, Tuple
 
 import numpy as np
 import torch
@@ -79,6 +79,8 @@ def _register_fused_op():
 
     # element-sorted route: sort the atoms by type, project each with its own element's
     # reductor on the matrix cores (compact [A,d]), run the fused kernel on those rows
+    lib.define("charge_rows(Tensor charges, Tensor species) -> (Tensor, Tensor)")
+    lib.impl("charge_rows", lambda charges, species: ops.charge_rows(charges, species), "CompositeExplicitAutograd")
     lib.define("sort_by_type(Tensor types, Tensor slots, int ne) -> (Tensor, Tensor)")
     lib.impl("sort_by_type", lambda types, slots, ne: ops.sort_by_type(types, slots, ne), "CompositeExplicitAutograd")
     lib.define("project_typed(Tensor rep, Tensor sorted_slots, Tensor type_offsets, Tensor reductors, Tensor types) "
@@ -296,9 +298,24 @@ def model_species_for_sort(species, rep):
     return species
 
 
-def element_rows(Z, species):
-    """Rows of the flattened charges that hold each of `species`, element after element and ascending
-    within one, and how many each has: (rows [K], counts)."""
+@torch.jit.ignore
+def _eager_element_rows(Z, species, elements) -> Tuple[bool, torch.Tensor, List[int]]:
+    """element_rows in two launches and one wait, where each slot is of at most one element."""
+    kinds = elements.tolist()
+    if len(kinds) > 32 or len(set(kinds)) < len(kinds):
+        return False, Z, kinds
+    rows, offsets = torch.ops.qml_lightning_sorf.charge_rows(Z.detach(), species)
+    starts = offsets.tolist()
+    return True, rows[:starts[-1]], [b - a for a, b in zip(starts, starts[1:])]
+
+
+def element_rows(Z, species, elements):
+    """Rows of the flattened charges that hold each of `species` (of `elements`, on the host), element
+    after element and ascending within one, and how many each has: (rows [K], counts)."""
+    if not torch.jit.is_scripting():
+        done, found, sizes = _eager_element_rows(Z, species, elements)
+        if done:
+            return found, sizes
     match = Z.int().view(1, -1) == species.int().view(-1, 1)
     totals = match.sum(dim=1)                          # launched ahead of the search, which waits
     rows = torch.nonzero(match)[:, 1].contiguous()
@@ -484,23 +501,26 @@ class HadamardFeaturesModel(BaseKernel, torch.nn.Module):
         # searched at once and before the representation is asked for, so that the host waits for
         # this search alone and launches the rest behind it; one gather and, in its backward, one
         # index_add serve all elements.  512 molecules of 3 to 29 atoms, four elements, with forces:
-        # 113 launches and 1.22 ms with a search per element, 76 and 0.95 ms so.
-        rows, counts = element_rows(Z, self.species)
+        # 113 launches and 1.22 ms with a search per element, 76 and 0.95 ms with one in plain torch (as
+        # in a saved file), 0.84 ms with the search of `charge_rows` and the features in three launches.
+        rows, counts = element_rows(Z, self.species, self.elements)
         torch_rep = self.rep.forward(X, Z, atomIDs, molIDs, atom_counts, cell, inv_cell)
         nmol, natoms_max = torch_rep.shape[0], torch_rep.shape[1]      # [1, n] for one unbatched molecule
         nmol_tensor = torch.tensor(nmol)
         molecule_of_row = torch.div(rows, natoms_max, rounding_mode='floor').type(torch.int).split(counts)
         sub_of_element = torch_rep.view(nmol * natoms_max, torch_rep.shape[2]).index_select(0, rows).split(counts)
         Ztest = torch.zeros(0, device=X.device, dtype=torch.float32)
+        index_of_element: List[int] = self.element2index[self.elements].tolist()
+        reductors, diagonals, biases = self.reductors.unbind(0), self.Dmat.unbind(0), self.bias.unbind(0)
         for i, count in enumerate(counts):
             if count == 0:
                 continue
-            element_idx = self.element2index[self.elements[i]]
-            sub = project_representation(sub_of_element[i], self.reductors[element_idx])
-            coeffs = torch.ops.qml_lightning_sorf.get_SORF_coefficients(sub, self.Dmat[element_idx],
-                                                                        coeff_normalisation, self.ntransforms)
+            e = index_of_element[i]
+            sub = project_representation(sub_of_element[i], reductors[e])
+            coeffs = torch.ops.qml_lightning_sorf.get_SORF_coefficients(sub, diagonals[e], coeff_normalisation,
+                                                                        self.ntransforms)
             coeffs = coeffs.view(coeffs.shape[0], coeffs.shape[1] * coeffs.shape[2])
-            features = torch.ops.qml_lightning_sorf.get_cos_features(coeffs, self.bias[element_idx], nmol_tensor,
+            features = torch.ops.qml_lightning_sorf.get_cos_features(coeffs, biases[e], nmol_tensor,
                                                                      molecule_of_row[i])
             Ztest = features if Ztest.numel() == 0 else Ztest + features
         if Ztest.numel() == 0:

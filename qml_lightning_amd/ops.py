@@ -424,6 +424,20 @@ def sorf_energy_typed(x_all, types, atom_slots, Dmat, bias, alpha, normalisation
 # ---------------------------------------------------------------------------------------
 # element-sorted projection + fused energy
 # ---------------------------------------------------------------------------------------
+def charge_rows(charges, species):
+    """Rows of the flattened charges that hold each of `species` (element after element, ascending within one) and
+    where each one's begin -> (rows [nslots], offsets [ne+1])."""
+    Z, species = _f32(charges).reshape(-1), _f32(species)
+    N, ne = int(Z.shape[0]), int(species.shape[0])
+    rows = torch.empty(N, dtype=torch.int32, device=Z.device)
+    offsets = torch.empty(ne + 1, dtype=torch.int32, device=Z.device)
+    nbytes = int(_lib.lib().qmll_charge_rows_workspace(N, ne))
+    work = torch.empty(max(nbytes // 4, 1), dtype=torch.int32, device=Z.device)
+    check(_lib.lib().qmll_charge_rows(_ptr(Z), _ptr(species), N, ne, _ptr(work), nbytes, _ptr(rows), _ptr(offsets), _stream()),
+          "qmll_charge_rows")
+    return rows, offsets
+
+
 def sort_by_type(types, slots, ne):
     """Stable sort of the real atoms' slots by element type -> (sorted_slots [A], type_offsets [ne+1])."""
     types, slots = _i32(types).reshape(-1), _i32(slots).reshape(-1)

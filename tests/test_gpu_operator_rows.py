@@ -1,0 +1,54 @@
+"""What the operator sequence does in few launches: the search for the atoms of all elements, and cosine features written
+per molecule, against plain torch."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev():
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("nslots", [1, 255, 256, 257, 5000])
+@pytest.mark.parametrize("elements", [[1], [1, 6, 8], [8, 1, 6, 7, 9], list(range(1, 33)), list(range(1, 35)), [1, 6, 1]])
+def test_rows_of_elements(nslots, elements):
+    """One element, other orders, as many as the native search takes and more, an element listed twice."""
+    from qml_lightning_amd.models.hadamard_features import element_rows
+    rng = np.random.default_rng(nslots)
+    Z = torch.tensor(rng.choice([0, 1, 6, 7, 16], nslots).reshape(1, -1), dtype=torch.float32, device=dev())
+    rows, counts = element_rows(Z, torch.tensor(elements, dtype=torch.float32, device=dev()), torch.tensor(elements))
+    want = [torch.nonzero(Z.view(-1) == e)[:, 0] for e in elements]
+    assert counts == [len(w) for w in want]
+    assert torch.equal(rows.long(), torch.cat(want))
+
+
+def test_no_slots():
+    from qml_lightning_amd.models.hadamard_features import element_rows
+    rows, counts = element_rows(torch.zeros(0, 4, device=dev()), torch.tensor([1.0, 6.0], device=dev()), torch.tensor([1, 6]))
+    assert counts == [0, 0] and rows.numel() == 0
+
+
+@pytest.mark.parametrize("A,F,nmol,order", [(1, 4, 1, "up"), (7, 260, 5, "up"), (40, 64, 900, "up"), (300, 33, 3, "up"), (300, 128, 40, "mixed"),
+                                            (300, 128, 40, "out"), (16383, 8, 700, "up"), (16384, 8, 700, "up"), (16385, 8, 700, "up"),
+                                            (16385, 8, 700, "mixed"), (600, 4096, 2050, "up")])
+def test_cos_features_of_molecules(A, F, nmol, order):
+    """Molecules without atoms, one and several columns per thread, the table by one workgroup and by many, and an index that is not
+    ascending or leaves the range (its atoms are left out)."""
+    gen = torch.Generator(device=dev()).manual_seed(A + F)
+    c = torch.randn(A, F, device=dev(), generator=gen) * 2
+    b = torch.rand(F, device=dev(), generator=gen) * 6
+    idx = torch.randint(0, nmol, (A,), device=dev(), generator=gen)
+    if order == "up":
+        idx = idx.sort()[0]
+    if order == "out":
+        idx[::7] = nmol
+    torch.full((nmol, F), float("nan"), device=dev())              # what the result's memory may hold
+    got = torch.ops.qml_lightning_sorf.get_cos_features(c, b, torch.tensor(nmol), idx.int())
+    ok = idx < nmol
+    want = torch.zeros(nmol, F, device=dev(), dtype=torch.float64)
+    want.index_add_(0, idx[ok], np.sqrt(2.0 / F) * torch.cos(c[ok].double() + b.double()))
+    most = torch.bincount(idx).max().item()
+    # 3.7e-7 of a cosine, a rounding per sum
+    assert (got.double() - want).abs().max().item() < np.sqrt(2.0 / F) * most * (4e-7 + most * 6e-8)
