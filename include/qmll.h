@@ -324,6 +324,16 @@ int qmll_prepare_batch(const float* Z, const int* natoms, const float* species, 
                        size_t workspace_bytes, int* types, int* sort_types, int* sorted_slots, int* type_offsets,
                        float* zero, size_t zero_count, qmll_stream_t stream);
 
+/* qmll_prepare_batch, then qmll_fchl19_forward without a neighbour list on the element indices it wrote (prm->nspecies of
+ * `species`): in ONE launch for few atoms, up to five elements and the usual grids.  types i32 [B,n], rep f32 [B,n,R]
+ * (rows of listed atoms) and the rest as there. */
+int qmll_prepare_fchl19_forward(const float* X, const float* Z, const float* species, const float* model_species, int ne,
+                                const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
+                                const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
+                                const qmll_fchl_params* prm, void* workspace, size_t workspace_bytes, int* types,
+                                int* sort_types, int* sorted_slots, int* type_offsets, float* zero, size_t zero_count,
+                                float* rep, qmll_stream_t stream);
+
 /* The projection matrices ("reductors", f32 [ne,R,d], qml_lightning/models/kernel.py:28) are constants
  * of a model.  Beyond the small-batch kernels the two projections below multiply on the fp16 matrix cores with
  * every fp32 operand as two fp16 parts behind power-of-two scales (fp32 accumulation): the

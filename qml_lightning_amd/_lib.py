@@ -76,6 +76,8 @@ PROTOTYPES = {
     "qmll_project_typed_backward": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P],
     "qmll_project_typed_backward_sums": [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, c_int, c_int, P, P],
     "qmll_prepare_batch": [P, P, P, c_int, P, c_int, P, P, c_int, c_int, c_int, P, c_size_t, P, P, P, P, P, c_size_t, P],
+    "qmll_prepare_fchl19_forward": [P, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, POINTER(FchlParams), P, c_size_t, P, P, P, P,
+                                    P, c_size_t, P, P],
     "qmll_project_typed_backward_parts": [P, c_int, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, c_int, c_int, P, P],
     "qmll_sorf_energy_parts_count": [c_int] * 6,
     "qmll_sorf_energy_parts": [P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_float, c_int, P, c_int, P, P],

@@ -739,13 +739,105 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
 // workgroup (fewer dispatches) and other depths of unrolling made no difference.
 // ---------------------------------------------------------------------------------
 constexpr int LEAN_RS3 = 20, LEAN_SLOTS = 6, LEAN_LANES = 10;    // bins; triples at a time, lanes (two bins each) of each
-template <int NS>
-__global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, float* __restrict__ rep) {
+// What qmll_prepare_batch does for a small batch, by workgroups of the forward launch beside those of the atoms
+struct BatchPrep {
+    const float* Z;              // null: done by a launch of its own
+    const float* species;
+    const float* model_species;  // null: the model goes by `species`
+    int ne;                      // elements of the model
+    int A;
+    int slots;
+    int* types;
+    int* sort_types;
+    int* sorted;
+    int* offsets;
+    float* zero;
+    int zero_count;
+    int groups;                  // workgroups: the sort, then 256 slots and floats each
+};
+constexpr int PREP_ATOMS = 256, PREP_ELEMENTS = 8;
+
+__device__ __forceinline__ int index_of_charge(float z, const float* __restrict__ species, int ns) {
+    const int q = (int)z;
+    int t = -1;
+    for (int j = 0; j < ns; ++j)
+        if (q == (int)species[j]) t = j;
+    return t;
+}
+
+// group 0: the listed atoms sorted by the model's element (stable), one wavefront, 64 atoms at a time; the others: element indices of
+// the slots (0 for padded ones) and the zeros
+__device__ __forceinline__ void prepare_group(const FchlArgs& a, const BatchPrep& b, int group, int lane, int* lds) {
+    const float* list = b.model_species ? b.model_species : b.species;
+    const int ns = a.p.nspecies, nlist = b.model_species ? b.ne : ns;
+    if (group > 0) {
+        const int step = 64 * (b.groups - 1);
+        for (int s = (group - 1) * 64 + lane; s < b.slots; s += step) {
+            const int m = s / a.n;
+            const bool real = s - m * a.n < a.natoms[m];
+            b.types[s] = real ? index_of_charge(b.Z[s], b.species, ns) : 0;
+            if (b.model_species) b.sort_types[s] = real ? index_of_charge(b.Z[s], b.model_species, b.ne) : 0;
+        }
+        for (int t = (group - 1) * 64 + lane; t < b.zero_count; t += step) b.zero[t] = 0.0f;
+        return;
+    }
+    int total[PREP_ELEMENTS];
+#pragma unroll
+    for (int e = 0; e < PREP_ELEMENTS; ++e) total[e] = 0;
+#pragma unroll
+    for (int base = 0; base < PREP_ATOMS; base += QMLL_WAVE) {         // all loads in flight
+        const int at = base + lane;
+        int slot = 0, t = -1;
+        if (at < b.A) {
+            const int m = a.molIDs[at], i = a.atomIDs[at];
+            slot = m * a.n + i;
+            t = i < a.natoms[m] ? index_of_charge(b.Z[slot], list, nlist) : 0;
+            lds[at] = slot << 4 | (t + 1);
+        }
+#pragma unroll
+        for (int e = 0; e < PREP_ELEMENTS; ++e) total[e] += __popcll(__ballot(t == e));
+    }
+    int start = 0;
+#pragma unroll
+    for (int e = 0; e < PREP_ELEMENTS; ++e) {
+        const int n = total[e];
+        total[e] = start;                                // from here: where the next of this element goes
+        if (lane == 0 && e <= b.ne) b.offsets[e] = start;
+        start += n;
+    }
+    if (lane == 0 && b.ne == PREP_ELEMENTS) b.offsets[b.ne] = start;
+    for (int base = 0; base < b.A; base += QMLL_WAVE) {
+        const int at = base + lane;
+        const int v = at < b.A ? lds[at] : 0;
+        const int t = (v & 15) - 1;
+#pragma unroll
+        for (int e = 0; e < PREP_ELEMENTS; ++e) {
+            const unsigned long long mask = __ballot(t == e);
+            if (t == e) b.sorted[total[e] + __popcll(mask & ((1ull << lane) - 1ull))] = v >> 4;
+            total[e] += __popcll(mask);
+        }
+    }
+    // entries past the last typed atom name a valid slot, so gathers through them stay in bounds
+    for (int k = start + lane; k < b.A; k += QMLL_WAVE) b.sorted[k] = 0;
+}
+
+// PREP: the first groups of the launch prepare the batch, the atoms' workgroups take the elements from the charges (no launch ahead of
+// this one has written the types).
+template <int NS, bool PREP>
+__global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, BatchPrep b, float* __restrict__ rep) {
     constexpr int NP = NS * (NS + 1) / 2;
     extern __shared__ float smem[];
     const int lane = threadIdx.x;
-    const int m = a.molIDs[blockIdx.x];
-    const int i = a.atomIDs[blockIdx.x];
+    int atom = blockIdx.x;
+    if constexpr (PREP) {
+        if (atom < b.groups) {
+            prepare_group(a, b, atom, lane, reinterpret_cast<int*>(smem));
+            return;
+        }
+        atom -= b.groups;
+    }
+    const int m = a.molIDs[atom];
+    const int i = a.atomIDs[atom];
     if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
     const int nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
     float* recA = smem;                                  // [cap][4]: d_ij, 1 / r
@@ -755,7 +847,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, flo
     const float* Xm = a.X + (size_t)m * a.n * 3;
     const int own = lane < a.n ? lane : 0;
     const float xj = Xm[own * 3 + 0], yj = Xm[own * 3 + 1], zj = Xm[own * 3 + 2];
-    const int et = a.types[(size_t)m * a.n + own];
+    const int et = PREP ? index_of_charge(b.Z[(size_t)m * a.n + own], b.species, NS) : a.types[(size_t)m * a.n + own];
     const int z = lane & 31, half = lane >> 5;           // two-body: radial bin, neighbour of two
     const float rs2v = z < nRs2 ? a.Rs2[z] : 1.0f;
     const int slot = idiv_small(lane, LEAN_LANES), ll = lane - LEAN_LANES * slot;      // three-body: triple of six, pair of bins
@@ -2188,10 +2280,9 @@ bool lean_grids(const qmll_fchl_params* prm, const int* nlist, int n) {
 
 }  // namespace
 
-extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float* cell, const float* inv_cell,
-                                   const int* atomIDs, const int* molIDs, const int* natoms, const int* nlist,
-                                   const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
-                                   const float* Rs3, const qmll_fchl_params* prm, float* rep, qmll_stream_t stream) {
+static int forward(const float* X, const int* types, const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
+                   const int* natoms, const int* nlist, const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
+                   const float* Rs3, const qmll_fchl_params* prm, const BatchPrep& prep, float* rep, qmll_stream_t stream) {
     FchlArgs a;
     int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, nn_stride, A, B, n, Rs2, Rs3,
                        prm, "qmll_fchl19_forward");
@@ -2234,9 +2325,12 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     }
     if (lean_grids(prm, nlist, n)) {
         const size_t entries = std::max<size_t>(alltrip + np * (LEAN_SLOTS - 1), a.cap);
-        const size_t lds = sizeof(float) * ((size_t)8 * a.cap + (3 * entries + 3) / 4 * 4);
+        size_t lds = sizeof(float) * ((size_t)8 * a.cap + (3 * entries + 3) / 4 * 4);
+        if (prep.Z) lds = std::max(lds, sizeof(int) * (size_t)A);        // the sort's
         auto launch = [&](auto nsc) {
-            hipLaunchKernelGGL(fchl19_forward_lean_kernel<decltype(nsc)::value>, dim3(A), dim3(64), lds, st, a, rep);
+            constexpr int NS = decltype(nsc)::value;
+            if (prep.Z) hipLaunchKernelGGL((fchl19_forward_lean_kernel<NS, true>), dim3(prep.groups + A), dim3(64), lds, st, a, prep, rep);
+            else hipLaunchKernelGGL((fchl19_forward_lean_kernel<NS, false>), dim3(A), dim3(64), lds, st, a, prep, rep);
         };
         switch (ns) {
             case 1: launch(std::integral_constant<int, 1>{}); break;
@@ -2264,6 +2358,41 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
     hipLaunchKernelGGL(fchl19_forward_kernel, dim3(A), dim3(64), lds, st, a, rep);
     QMLL_CHECK_LAUNCH("qmll_fchl19_forward");
     return QMLL_OK;
+}
+
+extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float* cell, const float* inv_cell,
+                                   const int* atomIDs, const int* molIDs, const int* natoms, const int* nlist,
+                                   const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
+                                   const float* Rs3, const qmll_fchl_params* prm, float* rep, qmll_stream_t stream) {
+    return forward(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, nn_stride, A, B, n, Rs2, Rs3, prm, BatchPrep{}, rep,
+                   stream);
+}
+
+extern "C" int qmll_prepare_fchl19_forward(const float* X, const float* Z, const float* species, const float* model_species, int ne,
+                                           const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
+                                           const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
+                                           const qmll_fchl_params* prm, void* workspace, size_t workspace_bytes, int* types,
+                                           int* sort_types, int* sorted_slots, int* type_offsets, float* zero, size_t zero_count,
+                                           float* rep, qmll_stream_t stream) {
+    QMLL_REQUIRE(prm != nullptr, QMLL_ERR_INVALID, "qmll_prepare_fchl19_forward: null params");
+    const long long slots = (long long)B * n, maxnn = n > 1 ? n - 1 : 1, triples = maxnn * (maxnn - 1) / 2;
+    // One launch less and the bookkeeping beside the representation instead of ahead of it, where one wavefront does the sort before
+    // the atoms are done: energies and forces of 21 atoms 29.0 -> 26.0 us, 12 x 21 32.6 -> 29.4, 16 x 29 46.2 -> 43.3, but 42 x 12 (504
+    // atoms) 29.0 -> 29.8 and 100 x 12 37.4 -> 45.3.
+    BatchPrep b{};
+    if (A > 0 && A <= PREP_ATOMS && slots > 0 && slots <= 32 * PREP_ATOMS && zero_count <= 128 * PREP_ATOMS && ne > 0 && ne <= PREP_ELEMENTS &&
+        (model_species ? sort_types != nullptr : ne == prm->nspecies) && lean_grids(prm, nullptr, n) &&
+        wavefronts_forward(A, triples, triples > TCH_MAX, true) == 1 && Z && species && types && sorted_slots && type_offsets &&
+        (zero || zero_count == 0)) {
+        const long long work = std::max<long long>(slots, (long long)zero_count);
+        b = BatchPrep{Z, species, model_species, ne, A, (int)slots, types, sort_types, sorted_slots, type_offsets, zero, (int)zero_count,
+                      1 + (int)((work + 255) / 256)};
+    } else {
+        int rc = qmll_prepare_batch(Z, natoms, species, prm->nspecies, model_species, ne, atomIDs, molIDs, B, n, A, workspace,
+                                    workspace_bytes, types, sort_types, sorted_slots, type_offsets, zero, zero_count, stream);
+        if (rc != QMLL_OK) return rc;
+    }
+    return forward(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm, b, rep, stream);
 }
 
 extern "C" int qmll_fchl19_vjp(const float* X, const int* types, const float* cell, const float* inv_cell,

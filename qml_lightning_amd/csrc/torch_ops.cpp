@@ -791,10 +791,6 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
     const int64_t ngrad = with_grad ? 3 * nslots : 0, nzero = ngrad + nparts * nslots;
     Tensor out = at::empty({nzero}, in.X.options());
     float* e_slots = nzero ? out.data_ptr<float>() + ngrad : nullptr;
-    check(qmll_prepare_batch(fp(Zb), ip(in.natoms), fp(sp), in.prm.nspecies, fp(msp), ne, ip(in.atomIDs), ip(in.molIDs), B, n,
-                             A, sort_work, sort_bytes, types, own_list ? sort_types : nullptr, ss, off,
-                             nzero ? out.data_ptr<float>() : nullptr, (size_t)nzero, stream()),
-          "qmll_prepare_batch");
     auto pad = [](int64_t v) { return (v + 63) / 64 * 64; };          // every part 256-byte aligned
     const int64_t rep_n = pad(nslots * R), x_n = pad((int64_t)A * d), gx_n = pad((int64_t)A * d * nparts);
     Tensor scratch = at::empty({rep_n + x_n + (with_grad ? gx_n + rep_n : 0) + 64}, in.X.options());
@@ -804,7 +800,11 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
     float* g_rep = with_grad ? gx + gx_n : nullptr;
     // the forward kernel writes every bin of a listed atom's row, and only the rows of listed
     // atoms are read below, so the padded rows need no clearing
-    check(qmll_fchl19_forward(FCHL_ABI_T(in, types), rep, stream()), "qmll_fchl19_forward");
+    check(qmll_prepare_fchl19_forward(fp(in.X), fp(Zb), fp(sp), fp(msp), ne, fp(in.cell), fp(in.inv_cell), ip(in.atomIDs), ip(in.molIDs),
+                                      ip(in.natoms), A, B, n, fp(in.Rs2), fp(in.Rs3), &in.prm, sort_work, sort_bytes, types,
+                                      own_list ? sort_types : nullptr, ss, off, nzero ? out.data_ptr<float>() : nullptr,
+                                      (size_t)nzero, rep, stream()),
+          "qmll_prepare_fchl19_forward");
     Tensor split = reductors_split(red, A);
     check(qmll_project_typed(rep, ss, off, fp(red), vp(split), A, ne, R, d, x, stream()), "qmll_project_typed");
     if (rff)

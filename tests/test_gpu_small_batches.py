@@ -86,3 +86,45 @@ def test_small_projections(A, ne, R, d, nparts):
     unknown = (types >= ne).nonzero()[:, 0]
     assert (g_rep[unknown] == 0).all()
     assert float((energies - e_total).abs().max()) <= 4 * nparts * n * 2.0 ** -24 * float(e.abs().max())
+
+
+@pytest.mark.parametrize("elements", [[1, 6, 8], [8, 1], [6, 1, 9, 8, 7, 16, 17, 2], [1, 6, 7, 8, 9, 16, 17, 2, 3]])
+@pytest.mark.parametrize("atoms,pad", [(1, 0), (21, 0), (63, 1), (65, 0), (256, 0), (257, 0), (30, 40)])
+def test_batch_prepared_beside_the_representation(elements, atoms, pad):
+    """The one launch of few atoms against the separate kernels: up to 256 atoms, a model with its own element list (in another
+    order, more elements than the launch sorts), padded slots, atoms listed in another order than they are stored."""
+    import ctypes
+    from qml_lightning_amd import _lib, ops
+    from qml_lightning_amd.representations.FCHL import FCHLCuda
+    rng = np.random.default_rng(atoms)
+    rep = FCHLCuda(species=np.array([1, 6, 8]))
+    n = 21
+    B = (atoms + n - 1) // n
+    counts = np.minimum(n, atoms - n * np.arange(B))
+    n += pad
+    dev = torch.device("cuda:0")
+    X = torch.tensor(rng.uniform(0, 6, (B, n, 3)), dtype=torch.float32, device=dev)
+    Z = torch.tensor(np.where(np.arange(n) < counts[:, None], rng.choice([1, 6, 8, 16], (B, n)), 0), dtype=torch.float32, device=dev)
+    order = rng.permutation(atoms)
+    aid = torch.tensor(np.concatenate([np.arange(k) for k in counts])[order], dtype=torch.int32, device=dev)
+    mid = torch.tensor(np.repeat(np.arange(B), counts)[order], dtype=torch.int32, device=dev)
+    nat = torch.tensor(counts, dtype=torch.int32, device=dev)
+    msp = None if elements == [1, 6, 8] else torch.tensor(elements, dtype=torch.float32, device=dev)
+    types, stypes, ss, off, zeroed = ops.prepare_batch(Z, nat, rep.species, aid, mid, msp, 5 * B * n)
+    prm = ops.make_params(3, rep.Rs2, rep.Rs3, rep.eta2, rep.eta3, rep.two_body_decay, rep.three_body_weight,
+                          rep.three_body_decay, rep.rcut)
+    want = ops.fchl_forward(X, types, None, None, aid, mid, nat, rep.Rs2, rep.Rs3, prm)
+    ne = len(elements)
+    got = [torch.full_like(t, -7) for t in (types, stypes, ss, off)]
+    zero = torch.full((5 * B * n,), 3.0, device=dev)
+    r = torch.zeros_like(want)
+    work = torch.empty(65536, dtype=torch.int32, device=dev)
+    p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())       # noqa: E731
+    _lib.check(_lib.lib().qmll_prepare_fchl19_forward(
+        p(X), p(Z), p(rep.species), p(msp), ne, None, None, p(aid), p(mid), p(nat), atoms, B, n, p(rep.Rs2), p(rep.Rs3),
+        ctypes.byref(prm), p(work), 4 * 65536, p(got[0]), p(got[1]) if msp is not None else None, p(got[2]), p(got[3]), p(zero),
+        zero.numel(), p(r), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "qmll_prepare_fchl19_forward")
+    assert torch.equal(got[0], types) and (msp is None or torch.equal(got[1], stypes))
+    assert torch.equal(got[2], ss) and torch.equal(got[3], off)
+    assert not zero.any()
+    assert torch.equal(r, want)
