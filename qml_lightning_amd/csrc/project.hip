@@ -25,6 +25,21 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 constexpr int MAXNE = 32;     // element types the sort supports
 constexpr int ST = 256;       // threads = atoms per workgroup of the sort
 
+// the largest of the wavefront's values, in every lane: row rotations and lane swaps, no LDS
+__device__ __forceinline__ float wave_max(float m) {
+    auto row = [&](auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    m = fmaxf(m, row(std::integral_constant<int, 0x128>{}));      // row_ror:8
+    m = fmaxf(m, row(std::integral_constant<int, 0x124>{}));
+    m = fmaxf(m, row(std::integral_constant<int, 0x122>{}));
+    m = fmaxf(m, row(std::integral_constant<int, 0x121>{}));
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    m = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // ---- sort by element type ---------------------------------------------------------------
 // counts[b*ne + e] = atoms of type e among atoms b*256 .. b*256+255
 __global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ types, const int* __restrict__ slots,
@@ -622,6 +637,11 @@ __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part
 // the power of two of their largest entry and are split in registers, the chunk of U arrives as its
 // image; a chunk's product is summed from zero and added to the running sums by the vector unit with
 // the inverse factor (which also keeps the low bits of a small chunk beside a large sum).
+// A round is a chain (rows, their largest value, their parts, the image, products), which three wavefronts per SIMD do not hide: with the
+// largest value by row rotations instead of LDS shuffles and the parts split two at a time 496 x 128 takes 24.9 us for 8000 atoms
+// and 26.7 for 32583 (27.6 and 29.4 before), 312 x 128 18.6 for 16384 (20.2), 720 x 128 163 for 131235 (165).  Large batches run at
+// some 3 TB/s either way: rows two chunks ahead, the next chunk's parts beside this one's products, 64 columns per workgroup (half as
+// fast again) and tiles that begin at different chunks made no difference to them.
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void typed_gemm_f16_kernel(
     const float* __restrict__ A, int lda, const int* __restrict__ a_rows, const _Float16* __restrict__ images,
     const int* __restrict__ exponents, float* __restrict__ C, int ldc, const int* __restrict__ offsets, int ne, int K, int N,
@@ -678,8 +698,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     auto round = [&](int c, const _Float16* cur, _Float16* other) {
         // the rows of this chunk: the wavefront's power of two, two fp16 parts each
         float ma = max4(max4(max4(max4(0.0f, ra[0][0]), ra[0][1]), ra[1][0]), ra[1][1]);
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) ma = fmaxf(ma, __shfl_xor(ma, o, 64));
+        ma = wave_max(ma);
         if (__builtin_expect(not_finite(ma), 0)) {       // an infinity among the rows: the largest finite entry
             ma = 0.0f;
 #pragma unroll
@@ -688,8 +707,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
                 for (int e = 0; e < 2; ++e)
                     ma = fmaxf(fmaxf(fmaxf(ma, finite_abs(ra[s2][e].x)), fmaxf(finite_abs(ra[s2][e].y), finite_abs(ra[s2][e].z))),
                                finite_abs(ra[s2][e].w));
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) ma = fmaxf(ma, __shfl_xor(ma, o, 64));
+            ma = wave_max(ma);
         }
         const int ka = scale_exponent(ma);
         const float sa = pow2i(ka);
@@ -699,11 +717,13 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
             const float w[8] = {ra[s2][0].x * sa, ra[s2][0].y * sa, ra[s2][0].z * sa, ra[s2][0].w * sa,
                                 ra[s2][1].x * sa, ra[s2][1].y * sa, ra[s2][1].z * sa, ra[s2][1].w * sa};
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                _Float16 a_, c_;
-                split_f16(w[q], a_, c_);
-                ahv[s2][q] = a_;
-                alv[s2][q] = c_;
+            for (int q = 0; q < 8; q += 2) {
+                half2_t hi, lo;
+                split_pair(w[q], w[q + 1], hi, lo);
+                ahv[s2][q] = hi[0];
+                ahv[s2][q + 1] = hi[1];
+                alv[s2][q] = lo[0];
+                alv[s2][q + 1] = lo[1];
             }
         }
         // this chunk's image has landed (every wavefront waits for its own loads, then for the others),
@@ -801,16 +821,14 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
 #pragma unroll
             for (int q = 0; q < 8; ++q) m = fmaxf(m, fabsf(av[j][q]));
         }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        m = wave_max(m);
         if (__builtin_expect(not_finite(m), 0)) {        // an infinity among the rows: the largest finite entry
             m = 0.0f;
 #pragma unroll
             for (int j = 0; j < KS; ++j)
 #pragma unroll
                 for (int q = 0; q < 8; ++q) m = fmaxf(m, finite_abs(av[j][q]));
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+            m = wave_max(m);
         }
         const int ka = scale_exponent(m);
         const float sa = pow2i(ka);
@@ -818,11 +836,13 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
 #pragma unroll
         for (int j = 0; j < KS; ++j)
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                _Float16 a, c;
-                split_f16(av[j][q] * sa, a, c);
-                ah[j][q] = a;
-                al[j][q] = c;
+            for (int q = 0; q < 8; q += 2) {
+                half2_t hi, lo;
+                split_pair(av[j][q] * sa, av[j][q + 1] * sa, hi, lo);
+                ah[j][q] = hi[0];
+                ah[j][q + 1] = hi[1];
+                al[j][q] = lo[0];
+                al[j][q + 1] = lo[1];
             }
     }
     int dst[16];                        // destination rows of the 16 accumulator registers
