@@ -120,8 +120,9 @@ struct RffElements {
 // The tile holds as many 16-row blocks as the molecule's rows need (one matrix instruction per block and four k).
 // Bound by the fp64 matrix cores: 200 molecules of 3 to 29 atoms, 128 components, 8192 features: 7.3 ms, where a tile
 // of 64 rows for every molecule padded to 29 atoms, a launch per element and a kernel of its own for the energy
-// features took 16.3 ms (of which the rows left out by the row table are a half).  The sine and cosine cost up to a
-// sixth: every lane group of a column works them out.
+// features took 16.3 ms (of which the rows left out by the row table are a half).  A column's argument is one value per
+// atom, which all four lane groups would work the sine and cosine out of (a tenth of the launch): two or four atoms are
+// multiplied first, as the registers allow, and a lane group works them out for one of them (9.0 -> 8.25 ms in a trace, same bits).
 // W is fp32 in a model (converted exactly in the registers) or fp64.
 template <int D, typename TW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void rff_rows_kernel(
@@ -148,6 +149,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
     const int l16 = lane & 15, lk = lane >> 4;
     const int f = blockIdx.x * 64 + wave * 16 + l16;
     const bool fok = f < F;
+    const unsigned wcol = lk * F + (fok ? f : F - 1);       // (a column beyond the last computes that one and writes nothing)
     const double norm = sqrt(2.0 / (double)F);
     double zacc = 0.0;
 
@@ -190,48 +192,62 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 
         int cur = -1;
         TW wreg[KS];
         double bf = 0.0;
-        for (int done = 0; done < natoms; ++done) {
-            const int el = e;
-            float* tile = tiles[done & 1];
+        // the atoms in groups of NG: the sine and cosine of a column are worked out once per group, a lane group per atom
+        constexpr int NG = (NB <= 2 ? 4 : 2) / (sizeof(TW) == 4 ? 1 : 2);      // (what fits 256 registers)
+        for (int done = 0; done < natoms; done += NG) {
+            double4_t pacc[NG][NB];
+            double arg = 0.0;
 #pragma unroll
-            for (int v = 0; v < V4; ++v) {
-                const int idx = v * 256 + threadIdx.x;
-                const int row = idx / (D / 4), c4 = idx % (D / 4);
-                if (V4 * 256 == NB * 16 * D / 4 || row < NB * 16)
-                    *reinterpret_cast<float4*>(&tile[row * LD + c4 * 4]) = stage[v];
-            }
-            __syncthreads();
-            if (el != cur) {   // B fragments of this wavefront's 16 columns, all of K, resident for the element's atoms
-                const TW* We = static_cast<const TW*>(E.W[el]);
+            for (int g = 0; g < NG; ++g) {
+                if (done + g >= natoms) break;
+                const int el = e;
+                float* tile = tiles[(done + g) & 1];
 #pragma unroll
-                for (int kk = 0; kk < KS; ++kk) wreg[kk] = fok ? We[(size_t)(kk * 4 + lk) * F + f] : (TW)0;
-                bf = fok ? (double)static_cast<const TW*>(E.b[el])[f] : 0.0;
-                cur = el;
-            }
-            ++a;
-            settle();
-            if (e < E.ne) fetch(e, a);   // in flight during the MFMAs
-
-            double4_t pacc[NB];
-#pragma unroll
-            for (int p = 0; p < NB; ++p) pacc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int kk = 0; kk < KS; ++kk) {
-#pragma unroll
-                for (int p = 0; p < NB; ++p) {
-                    const double av = (double)tile[(p * 16 + l16) * LD + kk * 4 + lk];
-                    pacc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, (double)wreg[kk], pacc[p], 0, 0, 0);
+                for (int v = 0; v < V4; ++v) {
+                    const int idx = v * 256 + threadIdx.x;
+                    const int row = idx / (D / 4), c4 = idx % (D / 4);
+                    if (V4 * 256 == NB * 16 * D / 4 || row < NB * 16)
+                        *reinterpret_cast<float4*>(&tile[row * LD + c4 * 4]) = stage[v];
                 }
-            }
-            // accumulator register r of a 16x16 block holds row lane/16 + 4r, column lane%16:
-            // the x row (the last of the tile) is register 3 of the last block in lanes 48..63
-            const double s0 = __shfl(pacc[NB - 1][3], 48 + l16, 64) + bf;
-            double sn, cs;
-            sincos(s0, &sn, &cs);
-            zacc += norm * cs;
-            const double fd = norm * sn;
+                __syncthreads();
+                if (el != cur) {   // B fragments of this wavefront's 16 columns, all of K, resident for the element's atoms
+                    const TW* We = static_cast<const TW*>(E.W[el]);
 #pragma unroll
-            for (int p = 0; p < NB; ++p) gacc[p] += fd * pacc[p];
+                    for (int kk = 0; kk < KS; ++kk) wreg[kk] = (We + (size_t)(kk * 4) * F)[wcol];
+                    bf = (double)static_cast<const TW*>(E.b[el])[fok ? f : F - 1];
+                    cur = el;
+                }
+                ++a;
+                settle();
+                if (e < E.ne) fetch(e, a);   // in flight during the MFMAs
+
+#pragma unroll
+                for (int p = 0; p < NB; ++p) pacc[g][p] = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int kk = 0; kk < KS; ++kk) {
+#pragma unroll
+                    for (int p = 0; p < NB; ++p) {
+                        const double av = (double)tile[(p * 16 + l16) * LD + kk * 4 + lk];
+                        pacc[g][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, (double)wreg[kk], pacc[g][p], 0, 0, 0);
+                    }
+                }
+                // accumulator register r of a 16x16 block holds row lane/16 + 4r, column lane%16:
+                // the x row (the last of the tile) is register 3 of the last block in lanes 48..63
+                const double s0 = __shfl(pacc[g][NB - 1][3], 48 + l16, 64) + bf;
+                if ((lk & (NG - 1)) == g) arg = s0;
+            }
+            double sn, cs;
+            sincos(arg, &sn, &cs);
+            sn *= norm;
+            cs *= norm;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                if (done + g >= natoms) break;
+                zacc += __shfl(cs, 16 * g + l16, 64);
+                const double fd = __shfl(sn, 16 * g + l16, 64);
+#pragma unroll
+                for (int p = 0; p < NB; ++p) gacc[p] += fd * pacc[g][p];
+            }
         }
         if (!fok) return;
         if (with_energy && lk == 0) {
