@@ -25,7 +25,7 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 constexpr int MAXNE = 32;     // element types the sort supports
 constexpr int ST = 256;       // threads = atoms per workgroup of the sort
 
-// the largest of the wavefront's values, in every lane: row rotations and lane swaps, no LDS
+// the largest of the wavefront's values, as a scalar: row rotations and lane swaps, no LDS
 __device__ __forceinline__ float wave_max(float m) {
     auto row = [&](auto ctrl) {
         return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), decltype(ctrl)::value, 0xf, 0xf, false));
@@ -37,7 +37,8 @@ __device__ __forceinline__ float wave_max(float m) {
     auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
     m = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    m = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
 }
 
 // ---- sort by element type ---------------------------------------------------------------
@@ -308,15 +309,16 @@ constexpr int PKS = PK + 4;        // LDS row stride of k-contiguous tiles: 16-b
 
 // which sorted rows a workgroup owns: tiles never straddle two types.  group: rows per sorted
 // entry (1 for one row per atom; the offsets count entries)
+template <int RT = PM>
 __device__ __forceinline__ bool tile_of_block(const int* __restrict__ offsets, int ne, int b, int& type, int& row0,
                                               int& rows, int group = 1) {
     for (int t = 0; t < ne; ++t) {
         const int o0 = offsets[t] * group, o1 = offsets[t + 1] * group;
-        const int nt = (o1 - o0 + PM - 1) / PM;
+        const int nt = (o1 - o0 + RT - 1) / RT;
         if (b < nt) {
             type = t;
-            row0 = o0 + b * PM;
-            rows = min(PM, o1 - row0);
+            row0 = o0 + b * RT;
+            rows = min(RT, o1 - row0);
             return true;
         }
         b -= nt;
@@ -514,7 +516,7 @@ __device__ __forceinline__ void image_to_lds(const unsigned char* __restrict__ s
 #pragma unroll
     for (int u0 = 0; u0 < BYTES / 1024; u0 += PT / 64) {
         const int u = u0 + wave_s;
-        if (u < BYTES / 1024)
+        if (u0 + PT / 64 <= BYTES / 1024 || u < BYTES / 1024)
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + u * 1024 + lane16),
                                              (__attribute__((address_space(3))) void*)((unsigned char*)dst + u * 1024), 16, 0,
                                              0);
@@ -617,6 +619,9 @@ __global__ __launch_bounds__(PT) void reductor_presplit_bwd_kernel(const float* 
     for (int t = tid; t < Img::BYTES / 16; t += PT) dst[t] = reinterpret_cast<const float4*>(img)[t];
 }
 
+// s_waitcnt vmcnt(4), (16) and (0), the other counters left alone
+constexpr int WAIT_VM4 = 0x0f74, WAIT_VM16 = 0x4f70, WAIT_VM0 = 0x0f70;
+
 // 2^-(ka + kb) applied to a chunk's product as it is added to the running sums: one factor when it is
 // a float, two multiplies at the ends of the exponent range (operands near the largest or smallest floats)
 __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part, int ka, int kb) {
@@ -637,11 +642,15 @@ __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part
 // the power of two of their largest entry and are split in registers, the chunk of U arrives as its
 // image; a chunk's product is summed from zero and added to the running sums by the vector unit with
 // the inverse factor (which also keeps the low bits of a small chunk beside a large sum).
+// RT: rows per tile.  128: four wavefronts below each other; 64: two by two, each with half the columns, whose registers leave room for
+// the rows of two chunks on the way.
 // A round is a chain (rows, their largest value, their parts, the image, products), which three wavefronts per SIMD do not hide: with the
 // largest value by row rotations instead of LDS shuffles and the parts split two at a time 496 x 128 takes 24.9 us for 8000 atoms
-// and 26.7 for 32583 (27.6 and 29.4 before), 312 x 128 18.6 for 16384 (20.2), 720 x 128 163 for 131235 (165).  Large batches run at
-// some 3 TB/s either way: rows two chunks ahead, the next chunk's parts beside this one's products, 64 columns per workgroup (half as
-// fast again) and tiles that begin at different chunks made no difference to them.
+// and 26.7 for 32583 (27.6 and 29.4 before), 312 x 128 18.6 for 16384 (20.2).  Large batches run at some 3 TB/s: matrix and vector
+// units, LDS and first-level cache are each busy for a quarter to two fifths of the time.  What they gained from scalar exponents and
+// from loads without branches: 720 x 128, 98000 atoms 115 -> 111 us, 131235 153 -> 147, 262144 280 -> 265.  Rows two chunks ahead in
+// tiles of 128 spill; tiles of 64 there, with which they fit, read the images twice as often (131235 atoms 197).
+template <int RT>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void typed_gemm_f16_kernel(
     const float* __restrict__ A, int lda, const int* __restrict__ a_rows, const _Float16* __restrict__ images,
     const int* __restrict__ exponents, float* __restrict__ C, int ldc, const int* __restrict__ offsets, int ne, int K, int N,
@@ -649,8 +658,10 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     // the two images as arrays of their own: the compiler then knows that the loads into one do not
     // touch what is read from the other
     __shared__ __attribute__((aligned(16))) _Float16 sB0[FWD_IMG_HALVES], sB1[FWD_IMG_HALVES];
+    constexpr int CW = PM / RT, NJ = 4 / CW;             // wavefronts side by side, 32-column blocks of each
+    constexpr int AHEAD = RT == 64 ? 2 : 1;              // chunks of rows on the way
     int type, row0, rows;
-    if (!tile_of_block(offsets, ne, blockIdx.x, type, row0, rows, group)) return;
+    if (!tile_of_block<RT>(offsets, ne, blockIdx.x, type, row0, rows, group)) return;
     const int col0 = blockIdx.y * 128, ncb = gridDim.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 31, h = lane >> 5;
@@ -662,40 +673,48 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     const int* exps = exponents + (size_t)type * nchunks * ncb + blockIdx.y;
     image_to_lds<FWD_IMG_BYTES>(img0, sB0, wave_s, lane16);
 
-    // this lane's row of A: row 32 wave + i, of each chunk the k = 16 s + 8 h + (0..7), s = 0, 1
-    const int r = 32 * wave + i;
-    const bool rok = r < rows;
+    // this lane's row of A: row 32 (wave / CW) + i, of each chunk the k = 16 s + 8 h + (0..7), s = 0, 1.  A lane without a row
+    // reads the tile's last one and one beyond K the row's last four entries, so that every lane loads the same number of times
+    // and the waits can count on it
+    const int wrow = 32 * (wave / CW), jt0 = NJ * (wave % CW);
+    const int r = min(wrow + i, rows - 1);
     size_t src = 0;
-    if (rok) {
-        if (group > 1) {
-            const int e = (row0 + r) / group;
-            src = (size_t)a_rows[e] * group + (size_t)(row0 + r - e * group);
-        } else {
-            src = (size_t)(a_rows ? a_rows[row0 + r] : row0 + r);
-        }
+    if (group > 1) {
+        const int e = (row0 + r) / group;
+        src = (size_t)a_rows[e] * group + (size_t)(row0 + r - e * group);
+    } else {
+        src = (size_t)(a_rows ? a_rows[row0 + r] : row0 + r);
     }
-    const float* arow = A + src * lda + 8 * h;
-    float4 ra[2][2];
-    auto fetch = [&](int k0) {
+    const float* arow = A + src * lda;
+    float4 ra[AHEAD][2][2];
+    auto fetch = [&](int k0, float4 (&to)[2][2]) {
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int k = k0 + 16 * s2 + 8 * h + 4 * e;
-                ra[s2][e] = (rok && k < K) ? *reinterpret_cast<const float4*>(arow + k0 + 16 * s2 + 4 * e) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
+            for (int e = 0; e < 2; ++e)
+                to[s2][e] = *reinterpret_cast<const float4*>(arow + min(k0 + 16 * s2 + 8 * h + 4 * e, K - 4));
     };
     auto max4 = [](float m, float4 v) { return fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w)); };
 
-    float16_t acc[4];
+    float16_t acc[NJ];
 #pragma unroll
-    for (int jt = 0; jt < 4; ++jt)
+    for (int jt = 0; jt < NJ; ++jt)
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[jt][q] = 0.0f;
 
-    fetch(0);
-    // one chunk: its image is in `cur`, the next one is loaded into `other`
-    auto round = [&](int c, const _Float16* cur, _Float16* other) {
+    fetch(0, ra[0]);
+    if constexpr (AHEAD == 2) fetch(PK, ra[1]);
+    // one chunk: its image is in `cur`, the next one is loaded into `other`; its rows are in `ra`, which the next chunk to be
+    // loaded takes
+    auto round = [&](int c, const _Float16* cur, _Float16* other, float4 (&ra)[2][2]) {
+        if constexpr (AHEAD == 2) __builtin_amdgcn_s_waitcnt(WAIT_VM4);        // all but the rows of the chunk behind this one
+        if (c * PK + PK > K) {           // the last chunk: zeros beyond K
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    if (c * PK + 16 * s2 + 8 * h + 4 * e >= K) ra[s2][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
         // the rows of this chunk: the wavefront's power of two, two fp16 parts each
         float ma = max4(max4(max4(max4(0.0f, ra[0][0]), ra[0][1]), ra[1][0]), ra[1][1]);
         ma = wave_max(ma);
@@ -726,19 +745,24 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
                 alv[s2][q + 1] = lo[1];
             }
         }
-        // this chunk's image has landed (every wavefront waits for its own loads, then for the others),
-        // and the other copy, read in the round before, is free
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (c + 1 < nchunks) {
-            image_to_lds<FWD_IMG_BYTES>(img0 + (size_t)(c + 1) * ncb * FWD_IMG_BYTES, other, wave_s, lane16);
-            fetch((c + 1) * PK);
+        // this chunk's image has landed (every wavefront waits for its own loads, then for the others; rows of the chunk
+        // behind it, four loads issued later, may be on their way), and the other copy, read in the round before, is free
+        if constexpr (AHEAD == 2) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
         }
+        if (c + 1 < nchunks) image_to_lds<FWD_IMG_BYTES>(img0 + (size_t)(c + 1) * ncb * FWD_IMG_BYTES, other, wave_s, lane16);
+        if (AHEAD == 2 || c + 1 < nchunks) fetch((c + AHEAD) * PK, ra);
+        if constexpr (AHEAD == 2) __builtin_amdgcn_sched_barrier(0);           // issued here, not behind the products
         const int kb = exps[(size_t)c * ncb];
         const _Float16* sBh = cur;
         const _Float16* sBl = cur + 128 * FWD_LDH;
 #pragma unroll
-        for (int j0 = 0; j0 < 4; j0 += 2) {
+        for (int j0 = 0; j0 < NJ; j0 += 2) {
             float16_t part[2];
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj)
@@ -748,8 +772,8 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
             for (int s2 = 0; s2 < PK / 16; ++s2) {
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
-                    const half8_t bhv = *reinterpret_cast<const half8_t*>(&sBh[(32 * (j0 + jj) + i) * FWD_LDH + 16 * s2 + 8 * h]);
-                    const half8_t blv = *reinterpret_cast<const half8_t*>(&sBl[(32 * (j0 + jj) + i) * FWD_LDH + 16 * s2 + 8 * h]);
+                    const half8_t bhv = *reinterpret_cast<const half8_t*>(&sBh[(32 * (jt0 + j0 + jj) + i) * FWD_LDH + 16 * s2 + 8 * h]);
+                    const half8_t blv = *reinterpret_cast<const half8_t*>(&sBl[(32 * (jt0 + j0 + jj) + i) * FWD_LDH + 16 * s2 + 8 * h]);
                     part[jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(alv[s2], bhv, part[jj], 0, 0, 0);
                     part[jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahv[s2], blv, part[jj], 0, 0, 0);
                     part[jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahv[s2], bhv, part[jj], 0, 0, 0);
@@ -759,17 +783,19 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
             for (int jj = 0; jj < 2; ++jj) add_scaled(acc[j0 + jj], part[jj], ka, kb);
         }
     };
-    for (int c = 0; c < nchunks; c += 2) {
-        round(c, sB0, sB1);
-        if (c + 1 < nchunks) round(c + 1, sB1, sB0);
+    int c = 0;
+    for (; c + 1 < nchunks; c += 2) {
+        round(c, sB0, sB1, ra[0]);
+        round(c + 1, sB1, sB0, ra[AHEAD - 1]);
     }
+    if (c < nchunks) round(c, sB0, sB1, ra[0]);
 
 #pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-        const int col = col0 + 32 * jt + i;
+    for (int jt = 0; jt < NJ; ++jt) {
+        const int col = col0 + 32 * (jt0 + jt) + i;
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            const int row = 32 * wave + 8 * (q / 4) + 4 * h + (q % 4);
+            const int row = wrow + 8 * (q / 4) + 4 * h + (q % 4);
             if (row < rows && col < N) C[(size_t)(row0 + row) * ldc + col] = acc[jt][q];
         }
     }
@@ -845,16 +871,23 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
                 al[j][q + 1] = lo[1];
             }
     }
-    int dst[16];                        // destination rows of the 16 accumulator registers
+    float* dst[16];                     // of the 16 accumulator registers, in the first block; a row the tile does not have: row 0's
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int row = 32 * wave + 8 * (q / 4) + 4 * h + (q % 4);
-        dst[q] = row < rows ? (c_rows ? c_rows[row0 + row] : row0 + row) : -1;
+        const int at = row0 + (row < rows ? row : 0);
+        dst[q] = C + (size_t)(c_rows ? c_rows[at] : at) * ldc + i;
     }
     // one block of 32 columns: its image is in `cur`, the next one is loaded into `other`
+    // (a full tile stores sixteen times per block, all behind the next image's loads, and need not wait for the stores: 496 columns,
+    // 65536 atoms 50.4 -> 48.1 us, 86016 54.8 -> 50.5)
+    const bool full = rows == PM;
     auto round = [&](int b, const unsigned char* cur, unsigned char* other) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        asm volatile("" ::: "memory");
+        if (full && b > 0) __builtin_amdgcn_s_waitcnt(WAIT_VM16);
+        else __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
         if (b + 1 < nblk) image_to_lds<Img::BYTES>(img0 + (size_t)(b + 1) * Img::BYTES, other, wave_s, lane16);
         float16_t acc;
 #pragma unroll
@@ -871,11 +904,14 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
         }
         const float sinv = reinterpret_cast<const float*>(cur + Img::SINV)[i];
         const int col = 32 * b + i;
-        if (col < N) {
+        if (full && 32 * b + 32 <= N) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) dst[q][32 * b] = acc[q] * inv_sa * sinv;
+        } else if (col < N) {
             // the two inverse factors one after the other: their product need not be a float
 #pragma unroll
             for (int q = 0; q < 16; ++q)
-                if (dst[q] >= 0) C[(size_t)dst[q] * ldc + col] = acc[q] * inv_sa * sinv;
+                if (32 * wave + 8 * (q / 4) + 4 * h + (q % 4) < rows) dst[q][32 * b] = acc[q] * inv_sa * sinv;
         }
     };
     for (int b = 0; b < nblk; b += 2) {
@@ -1465,8 +1501,16 @@ extern "C" int qmll_project_typed(const float* rep, const int* sorted_slots, con
         const SplitLayout L = split_layout(ne, R, d);
         QMLL_REQUIRE(aligned16(reductors_split), QMLL_ERR_INVALID, "qmll_project_typed: reductors_split must be 16-byte aligned");
         const unsigned char* base = (const unsigned char*)reductors_split;
-        hipLaunchKernelGGL(typed_gemm_f16_kernel, dim3(tiles, d / 128), dim3(PT), 0, (hipStream_t)stream, rep, R, sorted_slots,
-                           (const _Float16*)base, (const int*)(base + L.fwd_bytes + L.bwd_bytes), x, d, type_offsets, ne, R, d, 1);
+        // Tiles of 64 rows while they leave no CU with more than two: twice the workgroups, each with half the products and
+        // conversions per round of a chain that is all latency there; beyond, the images, which a tile reads whole, decide.  496 x
+        // 128, tiles of 128 / 64 rows: 8000 atoms 25.7 / 20.1 us, 16384 26.9 / 24.2, 32768 36.3 / 37.4, 65536 53 / 61, 131072 105 / 139
+        if ((long long)tiles * (d / 128) <= 192) {
+            hipLaunchKernelGGL(typed_gemm_f16_kernel<64>, dim3((A + 63) / 64 + ne, d / 128), dim3(PT), 0, (hipStream_t)stream, rep, R, sorted_slots,
+                               (const _Float16*)base, (const int*)(base + L.fwd_bytes + L.bwd_bytes), x, d, type_offsets, ne, R, d, 1);
+        } else {
+            hipLaunchKernelGGL(typed_gemm_f16_kernel<128>, dim3(tiles, d / 128), dim3(PT), 0, (hipStream_t)stream, rep, R, sorted_slots,
+                               (const _Float16*)base, (const int*)(base + L.fwd_bytes + L.bwd_bytes), x, d, type_offsets, ne, R, d, 1);
+        }
     } else if (wide)
         hipLaunchKernelGGL((typed_gemm_kernel<false, true, 128>), grid, dim3(PT), 0, (hipStream_t)stream, rep, R, sorted_slots,
                            reductors, (size_t)R * d, d, x, d, (const int*)nullptr, type_offsets, ne, R, d, 1);
