@@ -1921,11 +1921,17 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
 // of JT floats; the (triple, radial bin) items of every target pass then only read it.  Without
 // the table each item recomputes its triple, nRs3 times over and again in the neighbour passes.
 constexpr int JT = 20;   // rho, bin offset, 6 alpha, 2 beta, u_ij, u_ik, u_jk, pad
+constexpr int JW_MOST = 4;       // wavefronts per central atom
+// what a wavefront wrote to LDS is there for its own lanes: LDS takes a wavefront's instructions in order
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 template <bool TABLE>
-__global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* __restrict__ rep,
+__global__ __launch_bounds__(64 * JW_MOST) void fchl19_jacobian_kernel(FchlArgs a, float* __restrict__ rep,
                                                               float* __restrict__ jac) {
     extern __shared__ float smem[];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int m = a.molIDs[blockIdx.x];
     const int i = a.atomIDs[blockIdx.x];
     if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
@@ -1936,17 +1942,22 @@ __global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* 
     float* slnRs2 = s.next;          // [nRs2]
     float* sinvRs2 = slnRs2 + nRs2;  // [nRs2]
     float* sRs3 = sinvRs2 + nRs2;    // [nRs3]
-    float* row = sRs3 + nRs3;        // [3][R] rows being assembled (+ [R] value row)
-    float* val = row + 3 * R;        // [R]   representation row (self pass only)
+    float* val = sRs3 + nRs3;        // [R]   representation row (self pass only)
+    const int shared = nw > 1;
+    int* next = reinterpret_cast<int*>(val + R);             // the next target (of several wavefronts)
+    float* row = val + R + shared + wave * 3 * R;            // [3][R] rows that this wavefront assembles
     // TABLE: [ntrip][JT], 16-byte aligned behind the rows
-    float* ttab = val + R + ((4 - ((size_t)(val + R - smem) & 3)) & 3);
+    float* ttab = val + R + shared + 3 * R * nw;
+    ttab += (4 - ((size_t)(ttab - smem) & 3)) & 3;
 
-    for (int t = lane; t < nRs2; t += QMLL_WAVE) {
+    for (int t = threadIdx.x; t < nRs2; t += blockDim.x) {
         const float v = a.Rs2[t];
         slnRs2[t] = flog(v);
         sinvRs2[t] = frcp(v);
     }
-    for (int t = lane; t < nRs3; t += QMLL_WAVE) sRs3[t] = a.Rs3[t];
+    for (int t = threadIdx.x; t < nRs3; t += blockDim.x) sRs3[t] = a.Rs3[t];
+    if (shared && threadIdx.x == 0) *next = 0;
+    // (every wavefront stages the same neighbours in the same places)
     const int nn = stage_neighbours(a, s, m, i, lane);
     __syncthreads();
 
@@ -1958,7 +1969,7 @@ __global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* 
         // T_c = zeta2 K e cosT, T_s = zeta2 K e sinT with e = exp(-eta3 (rho - Rs_l)^2): their partials
         // with respect to the three distances are e * alpha + (de/drho) * beta, alpha and beta per triple
         const int ntrip = nn * (nn - 1) / 2;
-        for (int tt = lane; tt < ntrip; tt += QMLL_WAVE) {
+        for (int tt = threadIdx.x; tt < ntrip; tt += blockDim.x) {
             int j, k;
             unrank_pair(tt, nn, j, k);
             const Triple t = triple_geometry(s, j, k);
@@ -1982,12 +1993,19 @@ __global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* 
         __syncthreads();
     }
 
-    // target = -1: central atom; target = 0..nn-1: neighbour at that list position
-    for (int target = -1; target < nn; ++target) {
+    // target = -1: central atom; target = 0..nn-1: neighbour at that list position.  Each wavefront takes the next one that is left,
+    // and the rows of its own: nothing below waits for another wavefront
+    for (int target = -1;; ++target) {
+        if (shared) {
+            int taken = 0;
+            if (lane == 0) taken = atomicAdd(next, 1);
+            target = __builtin_amdgcn_readfirstlane(taken) - 1;
+        }
+        if (target >= nn) break;
         for (int t = lane; t < 3 * R; t += QMLL_WAVE) row[t] = 0.0f;
         if (target < 0)
             for (int t = lane; t < R; t += QMLL_WAVE) val[t] = 0.0f;
-        __syncthreads();
+        wave_sync();
 
         // two-body: items (neighbour j, bin z); a neighbour target only sees its own pair
         {
@@ -2180,7 +2198,7 @@ __global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* 
                 }
             }
         }
-        __syncthreads();
+        wave_sync();
         const int tj = target < 0 ? i : s.j[target];
         float* dst = jbase + (size_t)tj * 3 * R;
         for (int t = lane; t < 3 * R; t += QMLL_WAVE) dst[t] = row[t];
@@ -2188,7 +2206,7 @@ __global__ __launch_bounds__(64) void fchl19_jacobian_kernel(FchlArgs a, float* 
             float* out = rep + ((size_t)m * a.n + i) * R;
             for (int t = lane; t < R; t += QMLL_WAVE) out[t] = val[t];
         }
-        __syncthreads();
+        wave_sync();
     }
 }
 
@@ -2482,12 +2500,20 @@ extern "C" int qmll_fchl19_jacobian(const float* X, const int* types, const floa
     // most max_atoms - 1 otherwise
     const size_t maxnn = nlist ? (size_t)a.cap : (size_t)(a.cap > 1 ? a.cap - 1 : 1);
     const size_t table = sizeof(float) * (JT * (maxnn * (maxnn - 1) / 2) + 4);
-    if (lds + table <= LDS_LIMIT) {
-        lds += table;
-        hipLaunchKernelGGL(fchl19_jacobian_kernel<true>, dim3(A), dim3(64), lds, (hipStream_t)stream, a, rep, jac);
-    } else {
-        hipLaunchKernelGGL(fchl19_jacobian_kernel<false>, dim3(A), dim3(64), lds, (hipStream_t)stream, a, rep, jac);
+    const bool with_table = lds + table <= LDS_LIMIT;
+    if (with_table) lds += table;
+    // Wavefronts per central atom: as many as give a CU the most, since an atom's rows are a chain of LDS round trips that only other
+    // wavefronts fill, and the LDS of its table serves them all.  One wavefront / this, the self rows a third of the work: 3200 atoms of
+    // 3 to 29, four elements (three wavefronts) 761 / 393 us; 21000 of 21, three elements (four) 1810 / 1089
+    const size_t per_wave = sizeof(float) * 3 * (size_t)R, cu = 160 * 1024;
+    int nw = 1;
+    for (int w = 2; w <= JW_MOST; ++w) {
+        const size_t bytes = lds + sizeof(int) + (w - 1) * per_wave;
+        if (bytes <= LDS_LIMIT && (cu / bytes) * w > (cu / (lds + (nw - 1) * per_wave)) * nw) nw = w;
     }
+    if (nw > 1) lds += sizeof(int) + (nw - 1) * per_wave;
+    if (with_table) hipLaunchKernelGGL(fchl19_jacobian_kernel<true>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac);
+    else hipLaunchKernelGGL(fchl19_jacobian_kernel<false>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac);
     QMLL_CHECK_LAUNCH("qmll_fchl19_jacobian");
     return QMLL_OK;
 }
