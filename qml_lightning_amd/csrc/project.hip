@@ -42,13 +42,10 @@ __device__ __forceinline__ float wave_max(float m) {
 }
 
 // ---- sort by element type ---------------------------------------------------------------
-// counts[b*ne + e] = atoms of type e among atoms b*256 .. b*256+255
-__global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ types, const int* __restrict__ slots,
-                                                         int A, int ne, int* __restrict__ counts) {
+// counts[b*ne + e] of the 256 atoms whose types t the workgroup's threads hold (-1: none)
+__device__ __forceinline__ void count_types(int t, int ne, int* __restrict__ counts) {
     __shared__ int wcnt[ST / 64][MAXNE];
-    const int a = blockIdx.x * ST + threadIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int t = a < A ? types[slots[a]] : -1;
     for (int e = 0; e < ne; ++e) {
         const unsigned long long m = __ballot(t == e);
         if (lane == 0) wcnt[wave][e] = __popcll(m);
@@ -60,6 +57,13 @@ __global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ 
         for (int w = 0; w < ST / 64; ++w) s += wcnt[w][threadIdx.x];
         counts[blockIdx.x * ne + threadIdx.x] = s;
     }
+}
+
+// counts[b*ne + e] = atoms of type e among atoms b*256 .. b*256+255
+__global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ types, const int* __restrict__ slots,
+                                                         int A, int ne, int* __restrict__ counts) {
+    const int a = blockIdx.x * ST + threadIdx.x;
+    count_types(a < A ? types[slots[a]] : -1, ne, counts);
 }
 
 // index of charge z in a species list, -1 when it is not there (the rule of element_types_kernel)
@@ -74,22 +78,10 @@ __device__ __forceinline__ int species_index(float z, const float* __restrict__ 
 // the same counts from charges, whose element indices are written on the way
 __global__ __launch_bounds__(ST) void charge_count_kernel(const float* __restrict__ Z, const float* __restrict__ species, int A, int ne,
                                                            int* __restrict__ types, int* __restrict__ counts) {
-    __shared__ int wcnt[ST / 64][MAXNE];
     const int a = blockIdx.x * ST + threadIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = a < A ? species_index(Z[a], species, ne) : -1;
     if (a < A) types[a] = t;
-    for (int e = 0; e < ne; ++e) {
-        const unsigned long long m = __ballot(t == e);
-        if (lane == 0) wcnt[wave][e] = __popcll(m);
-    }
-    __syncthreads();
-    if (threadIdx.x < ne) {
-        int s = 0;
-#pragma unroll
-        for (int w = 0; w < ST / 64; ++w) s += wcnt[w][threadIdx.x];
-        counts[blockIdx.x * ne + threadIdx.x] = s;
-    }
+    count_types(t, ne, counts);
 }
 
 // sorted[pos] = slot of the atom, pos = start of its type + atoms of that type before it
@@ -274,13 +266,15 @@ __global__ __launch_bounds__(SORT_SMALL) void prepare_small_kernel(
 }
 
 // The same bookkeeping for a large batch, short of the sort itself: element indices of every slot, the
-// slot of every listed atom, the zero fill; one grid-stride launch instead of three or four
+// slot of every listed atom, the zero fill; one grid-stride launch instead of three or four.  With `counts` the first workgroups also
+// count the types of 256 listed atoms each, which they take from the charges themselves: the sort's first pass, which was a launch of
+// 4.7 us.
 __global__ __launch_bounds__(256) void prepare_large_kernel(const float* __restrict__ Z, const int* __restrict__ natoms,
                                                             const float* __restrict__ species, int ns,
                                                             const float* __restrict__ model_species, int ne,
                                                             const int* __restrict__ atomIDs, const int* __restrict__ molIDs,
                                                             size_t nslots, int n, int A, int* __restrict__ types,
-                                                            int* __restrict__ sort_types, int* __restrict__ slots,
+                                                            int* __restrict__ sort_types, int* __restrict__ slots, int* __restrict__ counts,
                                                             float* __restrict__ zero, size_t zero_count) {
     const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
     for (size_t idx = first; idx < nslots; idx += step) {
@@ -289,9 +283,16 @@ __global__ __launch_bounds__(256) void prepare_large_kernel(const float* __restr
         types[idx] = real ? species_index(Z[idx], species, ns) : 0;
         if (model_species) sort_types[idx] = real ? species_index(Z[idx], model_species, ne) : 0;
     }
-    if (slots)
-        for (size_t a = first; a < (size_t)A; a += step) slots[a] = molIDs[a] * n + atomIDs[a];
     for (size_t i = first; i < zero_count; i += step) zero[i] = 0.0f;
+    if (slots && (size_t)blockIdx.x * ST < (size_t)A) {       // (a workgroup per 256 atoms there is)
+        int t = -1;
+        if (first < (size_t)A) {
+            const int m = molIDs[first], i = atomIDs[first], slot = m * n + i;
+            slots[first] = slot;
+            t = i < natoms[m] ? species_index(Z[slot], model_species ? model_species : species, model_species ? ne : ns) : 0;
+        }
+        count_types(t, ne, counts);
+    }
 }
 
 __global__ __launch_bounds__(256) void zero_floats_kernel(float* __restrict__ p, size_t count) {
@@ -801,6 +802,76 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     }
 }
 
+// sums[m] = sum_i values[m*n + i]: thread = row (the per-molecule energy of a padded batch)
+__device__ __forceinline__ void row_sums(const float* __restrict__ values, int B, int n, float* __restrict__ sums, int chunk) {
+    const int m = chunk * 256 + threadIdx.x;
+    if (m >= B) return;
+    float acc = 0.0f;
+    for (int i = 0; i < n; ++i) acc += values[(size_t)m * n + i];
+    sums[m] = acc;
+}
+// the same over nparts arrays of B n values each: a wavefront per molecule, all of its values in flight at once
+__device__ __forceinline__ void row_sums_of_parts(const float* __restrict__ values, int nparts, int B, int n,
+                                                  float* __restrict__ sums, int chunk) {
+    const int m = chunk * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (m >= B) return;
+    float acc = 0.0f;
+    for (int t = lane; t < nparts * n; t += 64) {
+        const int k = t / n;
+        acc += values[(size_t)k * B * n + (size_t)m * n + (t - k * n)];
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) sums[m] = acc;
+}
+__host__ __device__ __forceinline__ int sum_chunks(int B, int nparts) { return nparts > 1 ? (B + 3) / 4 : (B + 255) / 256; }
+
+// values[i] += the other parts' (nparts arrays of count each, `stride` apart), in order
+__global__ __launch_bounds__(256) void add_parts_kernel(float* __restrict__ values, size_t count, int nparts, size_t stride) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) {
+        float v = values[i];
+        for (int k = 1; k < nparts; ++k) v += values[k * stride + i];
+        values[i] = v;
+    }
+}
+
+// rows of real atoms whose element the model does not know get a zero gradient
+// (lane = slot; the rare untyped slots of a wavefront are then zeroed row by row by all lanes)
+__device__ __forceinline__ void zero_untyped_rows(const int* __restrict__ types, int N, int ne, int R,
+                                                  float* __restrict__ out, int chunk) {
+    const int slot = chunk * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int t = slot < N ? types[slot] : 0;
+    unsigned long long todo = __ballot(slot < N && (t < 0 || t >= ne));
+    while (todo) {
+        const int l = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        const size_t row = (size_t)(slot - lane + l) * R;
+        for (int c = lane; c < R; c += 64) out[row + c] = 0.0f;
+    }
+}
+
+// What the backward projection does beside its product, in workgroups of 256 threads: zero rows of unknown elements (a workgroup per
+// 256 slots), then the per-molecule energy sums.  They stand behind the tiles of the product where there are some, and were a
+// launch of 4.9 us.
+struct Aside {
+    const int* types;
+    int N, zero_groups, sum_groups;
+    const float* e_slots;
+    int nparts, B, n;
+    float* energies;
+};
+__device__ __forceinline__ void run_aside(const Aside& a, int group, int ne, int R, float* __restrict__ out) {
+    if (group < a.zero_groups)
+        zero_untyped_rows(a.types, a.N, ne, R, out, group);
+    else if (a.nparts > 1)
+        row_sums_of_parts(a.e_slots, a.nparts, a.B, a.n, a.energies, group - a.zero_groups);
+    else
+        row_sums(a.e_slots, a.B, a.n, a.energies, group - a.zero_groups);
+}
+__global__ __launch_bounds__(256) void zero_untyped_rows_kernel(Aside aside, int ne, int R, float* __restrict__ out) {
+    run_aside(aside, (int)blockIdx.x, ne, R, out);
+}
+
 // Transpose product for a short contraction (K = projected dimension 64, 128 or 256):
 //     C[c_rows[row], :] = A[row, :] . U_type^T,   A [rows, K] (the gradient rows), U_type [N, K] row-major.
 // A wavefront keeps its 32 rows of A in registers for the whole kernel (two fp16 parts behind the
@@ -814,7 +885,12 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
                                                                      const unsigned char* __restrict__ images,
                                                                      float* __restrict__ C, int ldc,
                                                                      const int* __restrict__ c_rows,
-                                                                     const int* __restrict__ offsets, int ne, int N) {
+                                                                     const int* __restrict__ offsets, int ne, int N, int tiles,
+                                                                     Aside aside) {
+    if ((int)blockIdx.x >= tiles) {
+        run_aside(aside, (int)blockIdx.x - tiles, ne, N, C);
+        return;
+    }
     using Img = BwdImage<K>;
     constexpr int KS = K / 16;         // matrix instructions along k per product term
     constexpr int LDB = Img::LDB;
@@ -918,66 +994,6 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
         round(b, sI0, sI1);
         if (b + 1 < nblk) round(b + 1, sI1, sI0);
     }
-}
-
-// sums[m] = sum_i values[m*n + i]: thread = row (the per-molecule energy of a padded batch)
-__device__ __forceinline__ void row_sums(const float* __restrict__ values, int B, int n, float* __restrict__ sums, int chunk) {
-    const int m = chunk * 256 + threadIdx.x;
-    if (m >= B) return;
-    float acc = 0.0f;
-    for (int i = 0; i < n; ++i) acc += values[(size_t)m * n + i];
-    sums[m] = acc;
-}
-// the same over nparts arrays of B n values each: a wavefront per molecule, all of its values in flight at once
-__device__ __forceinline__ void row_sums_of_parts(const float* __restrict__ values, int nparts, int B, int n,
-                                                  float* __restrict__ sums, int chunk) {
-    const int m = chunk * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (m >= B) return;
-    float acc = 0.0f;
-    for (int t = lane; t < nparts * n; t += 64) {
-        const int k = t / n;
-        acc += values[(size_t)k * B * n + (size_t)m * n + (t - k * n)];
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) sums[m] = acc;
-}
-__host__ __device__ __forceinline__ int sum_chunks(int B, int nparts) { return nparts > 1 ? (B + 3) / 4 : (B + 255) / 256; }
-
-// values[i] += the other parts' (nparts arrays of count each, `stride` apart), in order
-__global__ __launch_bounds__(256) void add_parts_kernel(float* __restrict__ values, size_t count, int nparts, size_t stride) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) {
-        float v = values[i];
-        for (int k = 1; k < nparts; ++k) v += values[k * stride + i];
-        values[i] = v;
-    }
-}
-
-// rows of real atoms whose element the model does not know get a zero gradient
-// (lane = slot; the rare untyped slots of a wavefront are then zeroed row by row by all lanes)
-__device__ __forceinline__ void zero_untyped_rows(const int* __restrict__ types, int N, int ne, int R,
-                                                  float* __restrict__ out, int chunk) {
-    const int slot = chunk * 256 + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int t = slot < N ? types[slot] : 0;
-    unsigned long long todo = __ballot(slot < N && (t < 0 || t >= ne));
-    while (todo) {
-        const int l = __ffsll((long long)todo) - 1;
-        todo &= todo - 1;
-        const size_t row = (size_t)(slot - lane + l) * R;
-        for (int c = lane; c < R; c += 64) out[row + c] = 0.0f;
-    }
-}
-
-__global__ __launch_bounds__(256) void zero_untyped_rows_kernel(const int* __restrict__ types, int N, int ne, int R,
-                                                                float* __restrict__ out, int zero_groups,
-                                                                const float* __restrict__ e_slots, int nparts, int B, int n,
-                                                                float* __restrict__ energies) {
-    if ((int)blockIdx.x < zero_groups)
-        zero_untyped_rows(types, N, ne, R, out, blockIdx.x);
-    else if (nparts > 1)
-        row_sums_of_parts(e_slots, nparts, B, n, energies, (int)blockIdx.x - zero_groups);
-    else                                               // workgroups past the slots: the per-molecule energy sums
-        row_sums(e_slots, B, n, energies, (int)blockIdx.x - zero_groups);
 }
 
 // Small batches (a molecule to a few thousand atoms): the tiled kernels above run a few workgroups
@@ -1315,16 +1331,20 @@ extern "C" int qmll_prepare_batch(const float* Z, const int* natoms, const float
     int* atom_slots = one_workgroup_sort ? nullptr : reinterpret_cast<int*>(static_cast<char*>(workspace) + counts_bytes);
     size_t work = slots > zero_count ? slots : zero_count;
     if ((size_t)A > work) work = (size_t)A;
+    int* counts = one_workgroup_sort ? nullptr : static_cast<int*>(workspace);
     const size_t groups = (work + 255) / 256;
-    hipLaunchKernelGGL(prepare_large_kernel, dim3((unsigned)(groups < 8192 ? groups : 8192)), dim3(256), 0, (hipStream_t)stream,
+    const size_t nb = ((size_t)A + ST - 1) / ST, most = nb > 8192 ? nb : 8192;
+    hipLaunchKernelGGL(prepare_large_kernel, dim3((unsigned)(groups < most ? groups : most)), dim3(256), 0, (hipStream_t)stream,
                        Z, natoms, species, nspecies, model_species, ne, atomIDs, molIDs, slots, n, A, types, sort_types,
-                       atom_slots, zero, zero_count);
+                       atom_slots, counts, zero, zero_count);
     QMLL_CHECK_LAUNCH("qmll_prepare_batch");
     if (one_workgroup_sort)
         return qmll_sort_atoms_by_type(model_species ? sort_types : types, atomIDs, molIDs, n, A, ne, nullptr, 0, sorted_slots,
                                        type_offsets, stream);
-    return qmll_sort_by_type(model_species ? sort_types : types, atom_slots, A, ne, workspace, counts_bytes, sorted_slots,
-                             type_offsets, stream);
+    hipLaunchKernelGGL(type_place_kernel, dim3((unsigned)nb), dim3(ST), 0, (hipStream_t)stream, model_species ? sort_types : types,
+                       atom_slots, A, ne, counts, (int)nb, sorted_slots, type_offsets);
+    QMLL_CHECK_LAUNCH("qmll_prepare_batch");
+    return QMLL_OK;
 }
 
 // ---- the same sort for callers that cannot allocate -------------------------------------
@@ -1591,13 +1611,15 @@ extern "C" int qmll_project_typed_backward_parts(float* gx, int nparts, const in
                            (hipStream_t)stream, gx, count, nparts, count);
         QMLL_CHECK_LAUNCH("qmll_project_typed_backward");
     }
-    if (!small && ((types && N > 0) || sums)) {
-        // the rows of unknown elements and the energy sums: one launch for the two
-        const int zero_groups = (types && N > 0) ? (N + 255) / 256 : 0;
-        const int sum_groups = sums ? sum_chunks(B, nparts) : 0;
-        QMLL_REQUIRE(g_rep || zero_groups == 0, QMLL_ERR_INVALID, "qmll_project_typed_backward: null pointer");
-        hipLaunchKernelGGL(zero_untyped_rows_kernel, dim3(zero_groups + sum_groups), dim3(256), 0, (hipStream_t)stream, types,
-                           N, ne, R, g_rep, zero_groups, e_slots, nparts, B, n, energies);
+    const Aside aside = {types, N, (types && N > 0) ? (N + 255) / 256 : 0, sums ? sum_chunks(B, nparts) : 0, e_slots, nparts, B, n, energies};
+    QMLL_REQUIRE(small || g_rep || aside.zero_groups == 0, QMLL_ERR_INVALID, "qmll_project_typed_backward: null pointer");
+    const int beside = aside.zero_groups + aside.sum_groups;
+    // short contraction: the gradient rows stay in registers, every row is read once.  At d = 256 a tile walks its columns
+    // at two wavefronts per SIMD, too slowly for a batch that has less than a tile for every fourth CU: fp32 kernel / this one at 496
+    // columns, 4200 atoms 29 / 34 us, 8000 atoms 41 / 35, 41796 atoms 146 / 62
+    const bool rows_in_registers = !small && vec && A > 0 && (d == 64 || d == 128 || (d == 256 && A >= 8000)) && reductors_split;
+    if (!small && !rows_in_registers && beside > 0) {
+        hipLaunchKernelGGL(zero_untyped_rows_kernel, dim3(beside), dim3(256), 0, (hipStream_t)stream, aside, ne, R, g_rep);
         QMLL_CHECK_LAUNCH("qmll_project_typed_backward");
     }
     if (A == 0) return QMLL_OK;
@@ -1620,24 +1642,22 @@ extern "C" int qmll_project_typed_backward_parts(float* gx, int nparts, const in
     }
         if (A < 64) LAUNCH_BT_SMALL(1) else if (A < 512) LAUNCH_BT_SMALL(4) else LAUNCH_BT_SMALL(8)
 #undef LAUNCH_BT_SMALL
-    } else if (vec && (d == 64 || d == 128 || (d == 256 && A >= 8000)) && reductors_split) {
-        // short contraction: the gradient rows stay in registers, every row is read once.  At d = 256 a tile walks its columns
-        // at two wavefronts per SIMD, too slowly for a batch that has less than a tile for every fourth CU: fp32 kernel / this one at 496
-        // columns, 4200 atoms 29 / 34 us, 8000 atoms 41 / 35, 41796 atoms 146 / 62
+    } else if (rows_in_registers) {
         const SplitLayout L = split_layout(ne, R, d);
         QMLL_REQUIRE(aligned16(reductors_split), QMLL_ERR_INVALID,
                      "qmll_project_typed_backward: reductors_split must be 16-byte aligned");
         const unsigned char* images = (const unsigned char*)reductors_split + L.fwd_bytes;
-        const dim3 g1((A + PM - 1) / PM + ne);
+        const int tiles = (A + PM - 1) / PM + ne;
+        const dim3 g1(tiles + beside);
         if (d == 128)
             hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<128>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,
-                               R, sorted_slots, type_offsets, ne, R);
+                               R, sorted_slots, type_offsets, ne, R, tiles, aside);
         else if (d == 256)
             hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<256>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,
-                               R, sorted_slots, type_offsets, ne, R);
+                               R, sorted_slots, type_offsets, ne, R, tiles, aside);
         else
             hipLaunchKernelGGL((typed_gemm_bt_rows_f16_kernel<64>), g1, dim3(PT), 0, (hipStream_t)stream, gx, images, g_rep,
-                               R, sorted_slots, type_offsets, ne, R);
+                               R, sorted_slots, type_offsets, ne, R, tiles, aside);
     } else if (vec)
         hipLaunchKernelGGL((typed_gemm_kernel<true, true, PN>), grid, dim3(PT), 0, (hipStream_t)stream, gx, d,
                            (const int*)nullptr, reductors, (size_t)R * d, d, g_rep, R, sorted_slots, type_offsets, ne, d, R);
