@@ -556,6 +556,10 @@ int qmll_gram_upper_ws_f64(const double* Z, const double* y, int M, int F, doubl
 size_t qmll_gram_modular_workspace_bytes(int M, int F);
 int qmll_gram_modular_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
                           size_t workspace_bytes, qmll_stream_t stream);
+/* The same with ZTZ written, not added to (its upper tiles; M > 0): the first batch of a sum needs no cleared matrix, 2 GB at
+ * 16384 features.  ZTy is added to as ever. */
+int qmll_gram_modular_write_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
+                                size_t workspace_bytes, qmll_stream_t stream);
 
 /* ZTZ[j,i] = ZTZ[i,j] for the tiles strictly above the diagonal: completes a matrix built with
  * qmll_gram_upper_f64 (both triangles bit-identical). */

@@ -101,6 +101,7 @@ PROTOTYPES = {
     "qmll_gram_upper_ws_f64": [P, P, c_int, c_int, P, P, P, c_size_t, P],
     "qmll_gram_modular_workspace_bytes": [c_int, c_int],
     "qmll_gram_modular_f64": [P, P, c_int, c_int, P, P, P, c_size_t, P],
+    "qmll_gram_modular_write_f64": [P, P, c_int, c_int, P, P, P, c_size_t, P],
     "qmll_gram_mirror_f64": [P, c_int, P],
     "qmll_cholesky_workspace_bytes": [c_int],
     "qmll_copy_upper_f64": [P, c_longlong, c_int, P, c_longlong, P],

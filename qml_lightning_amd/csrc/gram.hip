@@ -195,8 +195,9 @@ __global__ __launch_bounds__(GT, 2) void gram_kernel(const double* __restrict__ 
                     const double v = sign * acc[p][q][r];
                     if (split) {
                         C[(size_t)blockIdx.x * (TILE * TILE) + (size_t)(gi - i0) * TILE + (gj - j0)] = v;
-                    } else if (SYM) {
-                        C[(size_t)gi * ldc + gj] += v;             // the mirror image is a separate pass
+                    } else if (SYM) {                              // the mirror image is a separate pass
+                        double* c = C + (size_t)gi * ldc + gj;
+                        *c = overwrite ? v : *c + v;
                     } else if (overwrite) {
                         C[(size_t)(gi - f0) * ldc + gj] = v;
                     } else {
@@ -446,9 +447,9 @@ extern "C" int qmll_matmul_and_reduce(const float* A, const float* B, int Ar, in
 }
 
 // used by gram_modular.hip: C += sign Z^T Z on the tiles on or above the diagonal, on the device only if *only_if is not 0
-int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, const int* only_if,
-                          const char* who, hipStream_t stream) {
-    return gram_launch(Z, nullptr, M, F, 0, F, true, false, C, nullptr, stream, who, ldz, ldc, sign, nullptr, 0, 0, nullptr, 0, only_if);
+int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, int overwrite,
+                          const int* only_if, const char* who, hipStream_t stream) {
+    return gram_launch(Z, nullptr, M, F, 0, F, true, false, C, nullptr, stream, who, ldz, ldc, sign, nullptr, 0, overwrite, nullptr, 0, only_if);
 }
 
 // used by solve.hip: tiles on or above the diagonal of C[n,n] += sign * Z^T Z with strided operands

@@ -413,7 +413,7 @@ hipError_t allow_stages() {
 
 // ---- reconstruction --------------------------------------------------------------------------------
 // thread = half the entries of one lane's accumulator: V = sum_i t_i (P / p_i) - P rint(sum_i t_i / p_i), every limb sum an
-// integer below 2^53 and so exact in fp64; C += V 2^-(2 gamma - e_i - e_j)
+// integer below 2^53 and so exact in fp64; C += (overwrite: =) V 2^-(2 gamma - e_i - e_j)
 // Eight entries, so that the residues of all moduli and what is added to are on their way together; with
 // sixteen the registers held one modulus at a time and every one was waited for.  All of a factorisation of 16384 columns 1657 -> 1209 us,
 // two products of as many 1926 -> 1818 (4.4 TB/s)
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(const signed char* __r
                                                           int t0, int ntile,
                                                           int F, const int* __restrict__ expo, const double* __restrict__ sums,
                                                           const int* __restrict__ flag,
-                                                          double sign, double* __restrict__ C, long long ldc) {
+                                                          double sign, int overwrite, double* __restrict__ C, long long ldc) {
     if (*flag) return;
     const int tile = blockIdx.x / REC_PER_TILE, sub = blockIdx.x % REC_PER_TILE;
     int ti, tj;
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(const signed char* __r
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int i = i0 + (e & 3), j = j0 + (e >> 2) * 16;
-        old[e] = i < F && j < F ? C[(size_t)i * ldc + j] : 0.0;
+        old[e] = !overwrite && i < F && j < F ? C[(size_t)i * ldc + j] : 0.0;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -493,12 +493,13 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(const signed char* __r
 }  // namespace
 
 // gram.hip: the fp64 kernel over tiles on or above the diagonal, on the device only if *only_if is not 0
-int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, const int* only_if,
-                          const char* who, hipStream_t stream);
+int qmll_internal_gram_if(const double* Z, long long ldz, int M, int F, double* C, long long ldc, double sign, int overwrite,
+                          const int* only_if, const char* who, hipStream_t stream);
 
-// C[F,F] (row stride ldc, tiles on or above the diagonal) += sign Z^T Z, Z = M rows of F columns with row stride ldz; ZTy += Z^T y
+// C[F,F] (row stride ldc, tiles on or above the diagonal) += (overwrite: =) sign Z^T Z, Z = M rows of F columns with row stride ldz;
+// ZTy += Z^T y
 static int modular_syrk(const double* Z, long long ldz, const double* y, int M, int F, double* C, long long ldc, double sign,
-                               double* ZTy, void* workspace, const char* who, hipStream_t stream) {
+                               int overwrite, double* ZTy, void* workspace, const char* who, hipStream_t stream) {
     const ModularPlan pl = modular_plan(M, F);
     char* ws = (char*)workspace;
     int* flag = (int*)ws;
@@ -531,10 +532,10 @@ static int modular_syrk(const double* Z, long long ldz, const double* y, int M, 
                                pl.Fp, nk, pl.pieces, 0, 0, pl.nt, t0, nr, flag, results);
             QMLL_CHECK_LAUNCH(who);
             hipLaunchKernelGGL(reconstruct_kernel<GRAM_MODULI>, dim3((unsigned)nr * REC_PER_TILE), dim3(256), 0, stream, results, pl.pieces, 0, 0, pl.nt, t0, nr,
-                               F, expo, (const double*)nullptr, flag, sign, C, ldc);
+                               F, expo, (const double*)nullptr, flag, sign, overwrite && m0 == 0, C, ldc);
             QMLL_CHECK_LAUNCH(who);
         }
-        const int rc = qmll_internal_gram_if(z, ldz, m, F, C, ldc, sign, flag, who, stream);
+        const int rc = qmll_internal_gram_if(z, ldz, m, F, C, ldc, sign, overwrite && m0 == 0, flag, who, stream);
         if (rc != QMLL_OK) return rc;
     }
     return QMLL_OK;
@@ -633,7 +634,7 @@ int qmll_internal_slab_update(double* A, long long ld, int rows, int n, int k, i
         QMLL_CHECK_LAUNCH(who);
         hipLaunchKernelGGL(reconstruct_kernel<CHOL_MODULI>, dim3((unsigned)nr * REC_PER_TILE), dim3(256), 0, stream, (const signed char*)results, pieces, off,
                            std::min(band, nt), s.nt, t0, nr, n, (const int*)(ws + s.expo), (const double*)(ws + s.sums),
-                           (const int*)ws, -1.0, A, ld);
+                           (const int*)ws, -1.0, 0, A, ld);
         QMLL_CHECK_LAUNCH(who);
     }
     return QMLL_OK;
@@ -651,15 +652,25 @@ extern "C" size_t qmll_gram_modular_workspace_bytes(int M, int F) {
     return modular_plan(M, F).bytes;
 }
 
-extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
-                                     size_t workspace_bytes, qmll_stream_t stream) {
-    const char* who = "qmll_gram_modular_f64";
+static int gram_modular(const char* who, const double* Z, const double* y, int M, int F, int overwrite, double* ZTZ, double* ZTy,
+                        void* workspace, size_t workspace_bytes, qmll_stream_t stream) {
     QMLL_REQUIRE(M >= 0 && F > 0, QMLL_ERR_INVALID, "%s: bad size M=%d F=%d", who, M, F);
+    QMLL_REQUIRE(M > 0 || !overwrite, QMLL_ERR_INVALID, "%s: no rows to write from", who);
     if (M == 0) return QMLL_OK;
     QMLL_REQUIRE(Z && ZTZ && workspace, QMLL_ERR_INVALID, "%s: null pointer", who);
     QMLL_REQUIRE((y == nullptr) == (ZTy == nullptr), QMLL_ERR_INVALID, "%s: y and ZTy must both be given or both be NULL", who);
     const size_t need = modular_plan(M, F).bytes;
     QMLL_REQUIRE(workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, QMLL_ERR_INVALID,
                  "%s: needs %zu bytes of workspace, 16-byte aligned", who, need);
-    return modular_syrk(Z, F, y, M, F, ZTZ, F, 1.0, ZTy, workspace, who, (hipStream_t)stream);
+    return modular_syrk(Z, F, y, M, F, ZTZ, F, 1.0, overwrite, ZTy, workspace, who, (hipStream_t)stream);
+}
+
+extern "C" int qmll_gram_modular_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
+                                     size_t workspace_bytes, qmll_stream_t stream) {
+    return gram_modular("qmll_gram_modular_f64", Z, y, M, F, 0, ZTZ, ZTy, workspace, workspace_bytes, stream);
+}
+
+extern "C" int qmll_gram_modular_write_f64(const double* Z, const double* y, int M, int F, double* ZTZ, double* ZTy, void* workspace,
+                                           size_t workspace_bytes, qmll_stream_t stream) {
+    return gram_modular("qmll_gram_modular_write_f64", Z, y, M, F, 1, ZTZ, ZTy, workspace, workspace_bytes, stream);
 }

@@ -259,7 +259,10 @@ class BaseKernel():
         dev = self.device
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
-        ZTZ = torch.zeros(nf, nf, device=torch.device('cpu') if cpu_solve else dev, dtype=torch.float64)
+        # the plain sum over batches is written by its first one; the other forms add to zeros
+        plain = ntiles == 1 and not cpu_solve and not use_specialized_matmul
+        ZTZ = (torch.empty if plain and len(X) > 0 else torch.zeros)(nf, nf, device=torch.device('cpu') if cpu_solve else dev,
+                                                                     dtype=torch.float64)
         ZtrainY = torch.zeros(nf, 1, device=dev, dtype=torch.float64)
         start.record()
         mirror_pending = False
@@ -298,7 +301,8 @@ class BaseKernel():
                     # relative to the columns' norms is below that of fp64 sums here entry by entry (rms 5e-17 to 9e-17 of
                     # sum_k |z_ki z_kj| against 1.4e-15 to 3.7e-15, 1300 to 9600 rows of both models), and it is the
                     # measure of the Cholesky factorisation's own, F times larger, error
-                    ops.gram(rows, targets, ZTZ, ZtrainY, mirror=False, within_norms=True)    # upper tiles; mirrored once below
+                    # upper tiles; mirrored once below
+                    ops.gram(rows, targets, ZTZ, ZtrainY, mirror=False, within_norms=True, fresh=not mirror_pending)
                     mirror_pending = True
                 del rows
             if ntiles > 1:

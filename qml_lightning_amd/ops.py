@@ -898,10 +898,10 @@ def _gram_workspace(device):
     return ws
 
 
-def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True, within_norms=False):
+def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True, within_norms=False, fresh=False):
     """ZTZ += Z^T Z (or the row block f0:f1 of it), ZTy += Z^T y, fp64, in place.
     mirror=False (full matrix only) accumulates just the tiles on or above the diagonal: a
-    caller adding several batches finishes with one `gram_mirror(ZTZ)`.
+    caller adding several batches finishes with one `gram_mirror(ZTZ)`.  fresh=True: ZTZ holds nothing yet and is written.
 
     Sums of fp64 products, an entry off by at most M 2^-53 sum_k |z_ki z_kj|.  within_norms=True says that an error of
     2^-53 |z_i| |z_j| (the norms of the two columns) will do: from 768 rows the full matrix then comes from
@@ -926,11 +926,14 @@ def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True, within_norms=False):
             except torch.cuda.OutOfMemoryError:
                 work = None                     # the fp64 kernel needs no such workspace
             if work is not None:
-                check(_lib.lib().qmll_gram_modular_f64(_ptr(Zrows), _ptr(yv), M, F, _ptr(ZTZ), _ptr(zty), _ptr(work), nbytes,
-                                                       _stream()), "qmll_gram_modular_f64")
+                product = _lib.lib().qmll_gram_modular_write_f64 if fresh else _lib.lib().qmll_gram_modular_f64
+                check(product(_ptr(Zrows), _ptr(yv), M, F, _ptr(ZTZ), _ptr(zty), _ptr(work), nbytes, _stream()),
+                      "qmll_gram_modular_f64")
                 if mirror:
                     check(_lib.lib().qmll_gram_mirror_f64(_ptr(ZTZ), F, _stream()), "qmll_gram_mirror_f64")
                 return ZTZ, ZTy
+        if fresh:
+            ZTZ.zero_()
         # with a workspace the last, sparsely filled round of tiles is split over the idle CUs
         ws = _gram_workspace(Zrows.device) if M >= 2048 else None
         check(_lib.lib().qmll_gram_upper_ws_f64(_ptr(Zrows), _ptr(yv), M, F, _ptr(ZTZ), _ptr(zty), _ptr(ws),
@@ -939,6 +942,8 @@ def gram(Zrows, y, ZTZ, ZTy, f0=None, f1=None, mirror=True, within_norms=False):
         if mirror:
             check(_lib.lib().qmll_gram_mirror_f64(_ptr(ZTZ), F, _stream()), "qmll_gram_mirror_f64")
     else:
+        if fresh:
+            ZTZ.zero_()
         check(_lib.lib().qmll_gram_tile_f64(_ptr(Zrows), _ptr(yv), M, F, int(f0), int(f1), _ptr(ZTZ), _ptr(zty),
                                             _stream()), "qmll_gram_tile_f64")
     return ZTZ, ZTy

@@ -319,3 +319,31 @@ def test_solve_without_memory_for_slabs(monkeypatch):
     x, info = ops.cholesky_solve_spd(A, b)
     assert refused and int(info.item()) == 0
     assert float((A @ x - b).norm()) <= F * 2.0 ** -53 * float(A.norm()) * float(x.norm())
+
+
+# one launch of rows and two; edges of tiles; a column with an infinity, which takes the fp64 kernel
+@pytest.mark.parametrize("M,F", [(768, 24), (2000, 300), (70000, 130)])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_written_is_added_to_zeros(M, F, infinite):
+    """ZTZ written over whatever it holds is what adding to zeros gives, bit for bit; and so through `ops.gram`, below the
+    rows that the integer products take as well."""
+    from qml_lightning_amd import _lib, ops
+    from qml_lightning_amd.ops import _ptr, _stream
+    g = torch.Generator(device=dev()).manual_seed(F)
+    Z = torch.randn(M, F, dtype=torch.float64, device=dev(), generator=g)
+    if infinite:
+        Z[M // 2, F // 2] = float("inf")
+    want, _ = modular(Z)
+    C = torch.full((F, F), float("nan"), dtype=torch.float64, device=dev())
+    n = int(_lib.lib().qmll_gram_modular_workspace_bytes(M, F))
+    ws = torch.empty(n, dtype=torch.uint8, device=dev())
+    assert _lib.lib().qmll_gram_modular_write_f64(_ptr(Z), None, M, F, _ptr(C), None, _ptr(ws), n, _stream()) == 0, _lib.last_error()
+    up = upper(F)
+    np.testing.assert_array_equal(C.cpu().numpy()[up], want.cpu().numpy()[up])
+    for rows in (M, 200):
+        y = torch.randn(rows, dtype=torch.float64, device=dev(), generator=g)
+        got = [ops.gram(Z[:rows], y, torch.full((F, F), start, dtype=torch.float64, device=dev()),
+                        torch.zeros(F, 1, dtype=torch.float64, device=dev()), within_norms=True, fresh=fresh)
+               for start, fresh in ((0.0, False), (float("nan"), True))]
+        for a, b in zip(*got):
+            np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
