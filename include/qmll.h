@@ -129,6 +129,13 @@ int qmll_fchl19_jacobian(const float* X, const int* types, const float* cell, co
                          const int* nlist, const int* nneigh, int nn_stride,
                          int A, int B, int n, const float* Rs2, const float* Rs3,
                          const qmll_fchl_params* prm, float* rep, float* jac, qmll_stream_t stream);
+/* The same, and the other rows of every listed atom written with zeros: a caller that reads the rows of listed atoms alone need
+ * not fill the array. */
+int qmll_fchl19_jacobian_all_rows(const float* X, const int* types, const float* cell, const float* inv_cell,
+                         const int* atomIDs, const int* molIDs, const int* natoms,
+                         const int* nlist, const int* nneigh, int nn_stride,
+                         int A, int B, int n, const float* Rs2, const float* Rs3,
+                         const qmll_fchl_params* prm, float* rep, float* jac, qmll_stream_t stream);
 
 /* ---- SORF ------------------------------------------------------------------------ */
 

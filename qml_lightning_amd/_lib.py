@@ -48,6 +48,7 @@ PROTOTYPES = {
     "qmll_fchl19_vjp": _FCHL_COMMON + [P, P, P],
     "qmll_fchl19_vjp_scaled": _FCHL_COMMON + [P, c_float, P, P],
     "qmll_fchl19_jacobian": _FCHL_COMMON + [P, P, P],
+    "qmll_fchl19_jacobian_all_rows": _FCHL_COMMON + [P, P, P],
     "qmll_sorf_forward": [P, P, c_int, c_int, c_int, c_int, c_float, P, P],
     "qmll_sorf_adjoint": [P, P, c_int, c_int, c_int, c_int, c_float, P, P],
     "qmll_segment_offsets": [P, c_int, c_int, P, P],

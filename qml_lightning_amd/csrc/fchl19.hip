@@ -1929,7 +1929,7 @@ __device__ __forceinline__ void wave_sync() {
 }
 template <bool TABLE>
 __global__ __launch_bounds__(64 * JW_MOST) void fchl19_jacobian_kernel(FchlArgs a, float* __restrict__ rep,
-                                                              float* __restrict__ jac) {
+                                                              float* __restrict__ jac, int all_rows) {
     extern __shared__ float smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int m = a.molIDs[blockIdx.x];
@@ -2001,7 +2001,16 @@ __global__ __launch_bounds__(64 * JW_MOST) void fchl19_jacobian_kernel(FchlArgs 
             if (lane == 0) taken = atomicAdd(next, 1);
             target = __builtin_amdgcn_readfirstlane(taken) - 1;
         }
-        if (target >= nn) break;
+        if (target >= nn) {
+            // (all rows: then those of the atoms that are no target, three rows of zeros each)
+            const int j = target - nn;
+            if (!all_rows || j >= a.n) break;
+            bool seen = j == i;
+            for (int k = lane; k < nn; k += QMLL_WAVE) seen |= s.j[k] == j;
+            if (!__any(seen))
+                for (int t = lane; t < 3 * R; t += QMLL_WAVE) jbase[(size_t)j * 3 * R + t] = 0.0f;
+            continue;
+        }
         for (int t = lane; t < 3 * R; t += QMLL_WAVE) row[t] = 0.0f;
         if (target < 0)
             for (int t = lane; t < R; t += QMLL_WAVE) val[t] = 0.0f;
@@ -2480,11 +2489,9 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     return QMLL_OK;
 }
 
-extern "C" int qmll_fchl19_jacobian(const float* X, const int* types, const float* cell, const float* inv_cell,
-                                    const int* atomIDs, const int* molIDs, const int* natoms, const int* nlist,
-                                    const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
-                                    const float* Rs3, const qmll_fchl_params* prm, float* rep, float* jac,
-                                    qmll_stream_t stream) {
+static int jacobian(const float* X, const int* types, const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
+                    const int* natoms, const int* nlist, const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
+                    const float* Rs3, const qmll_fchl_params* prm, float* rep, float* jac, int all_rows, qmll_stream_t stream) {
     FchlArgs a;
     int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, nn_stride, A, B, n, Rs2, Rs3,
                        prm, "qmll_fchl19_jacobian");
@@ -2512,8 +2519,24 @@ extern "C" int qmll_fchl19_jacobian(const float* X, const int* types, const floa
         if (bytes <= LDS_LIMIT && (cu / bytes) * w > (cu / (lds + (nw - 1) * per_wave)) * nw) nw = w;
     }
     if (nw > 1) lds += sizeof(int) + (nw - 1) * per_wave;
-    if (with_table) hipLaunchKernelGGL(fchl19_jacobian_kernel<true>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac);
-    else hipLaunchKernelGGL(fchl19_jacobian_kernel<false>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac);
+    if (with_table) hipLaunchKernelGGL(fchl19_jacobian_kernel<true>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac, all_rows);
+    else hipLaunchKernelGGL(fchl19_jacobian_kernel<false>, dim3(A), dim3(64 * nw), lds, (hipStream_t)stream, a, rep, jac, all_rows);
     QMLL_CHECK_LAUNCH("qmll_fchl19_jacobian");
     return QMLL_OK;
+}
+
+extern "C" int qmll_fchl19_jacobian(const float* X, const int* types, const float* cell, const float* inv_cell,
+                                    const int* atomIDs, const int* molIDs, const int* natoms, const int* nlist,
+                                    const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
+                                    const float* Rs3, const qmll_fchl_params* prm, float* rep, float* jac,
+                                    qmll_stream_t stream) {
+    return jacobian(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, nn_stride, A, B, n, Rs2, Rs3, prm, rep, jac, 0, stream);
+}
+
+extern "C" int qmll_fchl19_jacobian_all_rows(const float* X, const int* types, const float* cell, const float* inv_cell,
+                                             const int* atomIDs, const int* molIDs, const int* natoms, const int* nlist,
+                                             const int* nneigh, int nn_stride, int A, int B, int n, const float* Rs2,
+                                             const float* Rs3, const qmll_fchl_params* prm, float* rep, float* jac,
+                                             qmll_stream_t stream) {
+    return jacobian(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, nn_stride, A, B, n, Rs2, Rs3, prm, rep, jac, 1, stream);
 }

@@ -14,6 +14,7 @@ import torch
 
 from .. import _lib, ops
 from ..cuda.utils_gpu import matmul_and_reduce
+from ..representations.FCHL import FCHLCuda
 
 
 def _default_device():
@@ -114,8 +115,10 @@ class BaseKernel():
         cells, inv_cells = data['cells'], data['inv_cells']
         B, n = charges.shape
         if with_forces:
+            # (of a formatted batch only the rows of listed atoms are read below)
+            unfilled = {'zero_fill': False} if isinstance(self.rep, FCHLCuda) and data.get('element_counts') is not None else {}
             representation, rep_derivative = self.rep.get_representation_and_derivative(
-                coordinates, charges, atomIDs, molIDs, natom_counts, cells, inv_cells)
+                coordinates, charges, atomIDs, molIDs, natom_counts, cells, inv_cells, **unfilled)
         else:
             representation = self.rep.get_representation(coordinates, charges, atomIDs, molIDs, natom_counts, cells,
                                                          inv_cells)

@@ -195,16 +195,19 @@ def fchl_vjp(grad_rep, X, types, cell, inv_cell, atomIDs, molIDs, natoms, Rs2, R
 
 
 def fchl_jacobian(X, types, cell, inv_cell, atomIDs, molIDs, natoms, Rs2, Rs3, prm, nlist=None, nneigh=None,
-                  with_rep=True):
-    """(rep f32 [B,n,R] or None, jac f32 [B,n,n,3,R]) (fchl_cuda.cpp:186-187)."""
+                  with_rep=True, zero_fill=True):
+    """(rep f32 [B,n,R] or None, jac f32 [B,n,n,3,R]) (fchl_cuda.cpp:186-187).  zero_fill=False: the rows of atoms that are not
+    listed hold anything; 1 GB need not be cleared for 200 molecules of up to 29 atoms."""
     X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, Rs2, Rs3 = _fchl_prepare(
         X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, Rs2, Rs3)
     B, n, _ = X.shape
     R = repsize(prm)
-    rep = torch.zeros((B, n, R), dtype=torch.float32, device=X.device) if with_rep else None
-    jac = torch.zeros((B, n, n, 3, R), dtype=torch.float32, device=X.device)
+    make = torch.zeros if zero_fill else torch.empty
+    rep = make((B, n, R), dtype=torch.float32, device=X.device) if with_rep else None
+    jac = make((B, n, n, 3, R), dtype=torch.float32, device=X.device)
+    write = _lib.lib().qmll_fchl19_jacobian if zero_fill else _lib.lib().qmll_fchl19_jacobian_all_rows
     args = _fchl_args(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nlist, nneigh, Rs2, Rs3, prm)
-    check(_lib.lib().qmll_fchl19_jacobian(*args, _ptr(rep), _ptr(jac), _stream()), "qmll_fchl19_jacobian")
+    check(write(*args, _ptr(rep), _ptr(jac), _stream()), "qmll_fchl19_jacobian")
     return rep, jac
 
 

@@ -73,14 +73,14 @@ class FCHLCuda(torch.nn.Module):
 
     @torch.jit.unused
     def get_representation_and_derivative(self, X, Z, atomIDs, molIDs, atom_counts, cell=None, inv_cell=None,
-                                          nneighbours=None, neighbourlist=None):
-        """(rep [B,n,R], grad [B,n,n,3,R]) (FCHL.py:82-97)."""
+                                          nneighbours=None, neighbourlist=None, zero_fill=True):
+        """(rep [B,n,R], grad [B,n,n,3,R]) (FCHL.py:82-97).  zero_fill=False: rows of atoms that are not listed hold anything."""
         element_types = self.get_element_types(X, Z, atom_counts)
         from .. import ops
         prm = ops.make_params(self.nspecies, self.Rs2, self.Rs3, self.eta2, self.eta3, self.two_body_decay,
                               self.three_body_weight, self.three_body_decay, self.rcut)
         rep, jac = ops.fchl_jacobian(X, element_types, cell, inv_cell, atomIDs, molIDs, atom_counts, self.Rs2,
-                                     self.Rs3, prm, neighbourlist, nneighbours)
+                                     self.Rs3, prm, neighbourlist, nneighbours, zero_fill=zero_fill)
         return rep, jac
 
     @torch.jit.unused
