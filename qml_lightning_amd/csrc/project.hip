@@ -662,7 +662,9 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     constexpr int CW = PM / RT, NJ = 4 / CW;             // wavefronts side by side, 32-column blocks of each
     constexpr int AHEAD = RT == 64 ? 2 : 1;              // chunks of rows on the way
     int type, row0, rows;
-    if (!tile_of_block<RT>(offsets, ne, blockIdx.x, type, row0, rows, group)) return;
+    // (from the last tile to the first: what the representation's launch wrote last is in the cache that all XCDs share; 131235 rows of 720
+    // in 141 -> 137 us behind it)
+    if (!tile_of_block<RT>(offsets, ne, gridDim.x - 1 - blockIdx.x, type, row0, rows, group)) return;
     const int col0 = blockIdx.y * 128, ncb = gridDim.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 31, h = lane >> 5;
