@@ -620,8 +620,9 @@ __global__ __launch_bounds__(PT) void reductor_presplit_bwd_kernel(const float* 
     for (int t = tid; t < Img::BYTES / 16; t += PT) dst[t] = reinterpret_cast<const float4*>(img)[t];
 }
 
-// s_waitcnt vmcnt(4), (16) and (0), the other counters left alone
-constexpr int WAIT_VM4 = 0x0f74, WAIT_VM16 = 0x4f70, WAIT_VM0 = 0x0f70;
+// s_waitcnt: vmcnt(4) alone, and ahead of a barrier, behind which what this wavefront has read in LDS may be overwritten, lgkmcnt(0)
+// alone or with vmcnt(16) or (0)
+constexpr int WAIT_VM4 = 0x0f74, WAIT_LDS = 0xc07f, WAIT_LDS_VM16 = 0x4070, WAIT_LDS_VM0 = 0x0070;
 
 // 2^-(ka + kb) applied to a chunk's product as it is added to the running sums: one factor when it is
 // a float, two multiplies at the ends of the exponent range (operands near the largest or smallest floats)
@@ -752,6 +753,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
         // behind it, four loads issued later, may be on their way), and the other copy, read in the round before, is free
         if constexpr (AHEAD == 2) {
             asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(WAIT_LDS);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         } else {
@@ -962,8 +964,8 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
     const bool full = rows == PM;
     auto round = [&](int b, const unsigned char* cur, unsigned char* other) {
         asm volatile("" ::: "memory");
-        if (full && b > 0) __builtin_amdgcn_s_waitcnt(WAIT_VM16);
-        else __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+        if (full && b > 0) __builtin_amdgcn_s_waitcnt(WAIT_LDS_VM16);
+        else __builtin_amdgcn_s_waitcnt(WAIT_LDS_VM0);
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (b + 1 < nblk) image_to_lds<Img::BYTES>(img0 + (size_t)(b + 1) * Img::BYTES, other, wave_s, lane16);
