@@ -52,3 +52,42 @@ def test_cos_features_of_molecules(A, F, nmol, order):
     most = torch.bincount(idx).max().item()
     # 3.7e-7 of a cosine, a rounding per sum
     assert (got.double() - want).abs().max().item() < np.sqrt(2.0 / F) * most * (4e-7 + most * 6e-8)
+
+
+def test_traced_model_on_other_batches():
+    """torch.jit.trace records the search, not what it found in the example's batch."""
+    from qml_lightning_amd.models.hadamard_features import HadamardFeaturesModel
+    from qml_lightning_amd.representations.FCHL import FCHLCuda
+    from tests import helpers
+    elements = np.array([1, 6, 8])
+    np.random.seed(0)
+    m = HadamardFeaturesModel(rep=FCHLCuda(species=elements), elements=elements, ntransforms=1, sigma=2.0, npcas=32, nstacks=4, fused=False)
+    gen = torch.Generator(device=dev()).manual_seed(1)
+    m.reductors = torch.randn(m.reductors.shape, device=dev(), generator=gen) * 0.1
+    m.alpha = torch.randn(m.nfeatures(), device=dev(), dtype=torch.float64, generator=gen)
+    keys = ("charges", "atomIDs", "molIDs", "natom_counts", "cells", "inv_cells")
+
+    def batch(seed):
+        rng = np.random.default_rng(seed)
+        X = np.stack([helpers.random_geometry(rng, 9, 5.0, 0.9) for _ in range(6)])
+        Q = rng.choice(elements, (6, 9))
+        Q[:, :3] = elements                                # (an element that the example lacks stays out of the trace)
+        data = m.format_data(X, Q)
+        return data["coordinates"].requires_grad_(True), [data[k] for k in keys]
+
+    class Energies(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.model = m
+
+        def forward(self, X, *rest):
+            return self.model.forward(X, *rest)
+
+    X, rest = batch(0)
+    traced = torch.jit.trace(Energies(), (X, *rest), check_trace=False)
+    for seed in (0, 1, 2):
+        X, rest = batch(seed)
+        got, want = traced(X, *rest), m.forward(X, *rest)
+        assert torch.equal(got, want)
+        g, w = (torch.autograd.grad(e.sum(), X)[0] for e in (got, want))
+        assert (g - w).abs().max().item() <= 1e-5 * w.abs().max().item()       # forces are summed by atomics
