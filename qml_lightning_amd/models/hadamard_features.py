@@ -308,7 +308,10 @@ def _eager_element_rows(Z, species, elements) -> Tuple[bool, torch.Tensor, List[
         return True, torch.cat(found), [f.shape[0] for f in found]
     if len(kinds) > 32 or len(set(kinds)) < len(kinds):
         return False, Z, kinds
-    rows, offsets = torch.ops.qml_lightning_sorf.charge_rows(Z.detach(), species)
+    Z = Z.detach()
+    if Z.dtype == torch.float64:
+        Z = Z.trunc()                                  # charges are truncated as they are given, not as fp32 has them
+    rows, offsets = torch.ops.qml_lightning_sorf.charge_rows(Z, species)
     starts = offsets.tolist()
     return True, rows[:starts[-1]], [b - a for a, b in zip(starts, starts[1:])]
 

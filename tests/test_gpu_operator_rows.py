@@ -24,6 +24,14 @@ def test_rows_of_elements(nslots, elements):
     assert torch.equal(rows.long(), torch.cat(want))
 
 
+def test_charges_are_truncated_in_their_own_type():
+    """A float64 charge just below a whole one, which rounds up to it in float32, is the lower element's."""
+    from qml_lightning_amd.models.hadamard_features import element_rows
+    Z = torch.tensor([[6.0, 6.0 - 1e-9, 7.0 - 1e-9, 1.5, 0.0]], dtype=torch.float64, device=dev())
+    rows, counts = element_rows(Z, torch.tensor([1.0, 5.0, 6.0], device=dev()), torch.tensor([1, 5, 6]))
+    assert counts == [1, 1, 2] and rows.tolist() == [3, 1, 0, 2]
+
+
 def test_no_slots():
     from qml_lightning_amd.models.hadamard_features import element_rows
     rows, counts = element_rows(torch.zeros(0, 4, device=dev()), torch.tensor([1.0, 6.0], device=dev()), torch.tensor([1, 6]))
