@@ -319,6 +319,7 @@ def _eager_element_rows(Z, species, elements) -> Tuple[bool, torch.Tensor, List[
 def element_rows(Z, species, elements):
     """Rows of the flattened charges that hold each of `species` (of `elements`, on the host), element
     after element and ascending within one, and how many each has: (rows [K], counts)."""
+    species = species.to(Z.device)                     # (a model whose tensors were moved one by one)
     if not torch.jit.is_scripting():
         done, found, sizes = _eager_element_rows(Z, species, elements)
         if done:

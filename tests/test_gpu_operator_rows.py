@@ -32,6 +32,14 @@ def test_charges_are_truncated_in_their_own_type():
     assert counts == [1, 1, 2] and rows.tolist() == [3, 1, 0, 2]
 
 
+def test_species_elsewhere():
+    """The list of elements need not be where the charges are."""
+    from qml_lightning_amd.models.hadamard_features import element_rows
+    Z = torch.tensor([[6.0, 1.0, 8.0, 1.0]], device=dev())
+    rows, counts = element_rows(Z, torch.tensor([1.0, 6.0]), torch.tensor([1, 6]))
+    assert counts == [2, 1] and rows.tolist() == [1, 3, 0]
+
+
 def test_no_slots():
     from qml_lightning_amd.models.hadamard_features import element_rows
     rows, counts = element_rows(torch.zeros(0, 4, device=dev()), torch.tensor([1.0, 6.0], device=dev()), torch.tensor([1, 6]))
