@@ -115,10 +115,13 @@ class BaseKernel():
         cells, inv_cells = data['cells'], data['inv_cells']
         B, n = charges.shape
         if with_forces:
-            # (of a formatted batch only the rows of listed atoms are read below)
-            unfilled = {'zero_fill': False} if isinstance(self.rep, FCHLCuda) and data.get('element_counts') is not None else {}
-            representation, rep_derivative = self.rep.get_representation_and_derivative(
-                coordinates, charges, atomIDs, molIDs, natom_counts, cells, inv_cells, **unfilled)
+            # (of a formatted batch only the rows of listed atoms are read below; a representation's own derivative need not
+            # have the option)
+            derivative = self.rep.get_representation_and_derivative
+            ours = getattr(derivative, '__func__', None) is FCHLCuda.get_representation_and_derivative
+            unfilled = {'zero_fill': False} if ours and data.get('element_counts') is not None else {}
+            representation, rep_derivative = derivative(coordinates, charges, atomIDs, molIDs, natom_counts, cells, inv_cells,
+                                                        **unfilled)
         else:
             representation = self.rep.get_representation(coordinates, charges, atomIDs, molIDs, natom_counts, cells,
                                                          inv_cells)

@@ -301,3 +301,34 @@ def test_rff_fused_true_refuses_a_width_without_a_fused_kernel():
     auto = RandomFourrierFeaturesModel(rep=rep, elements=np.array([1, 6]), nstacks=2, npcas=256)
     assert auto.fused is False
     assert RandomFourrierFeaturesModel(rep=rep, elements=np.array([1, 6]), nstacks=2, npcas=64).fused is True
+
+
+@pytest.mark.parametrize("where", ["class", "object"])
+def test_training_takes_a_representation_with_a_derivative_of_its_own(where):
+    """A subclass (or an object) whose get_representation_and_derivative has the reference's arguments alone is called with those."""
+    from qml_lightning_amd.models.kernel import BaseKernel
+    from qml_lightning_amd.representations.FCHL import FCHLCuda
+    calls = []
+
+    def own(X, Z, atomIDs, molIDs, atom_counts, cell=None, inv_cell=None):
+        calls.append(X.shape)
+        return torch.zeros(*Z.shape, 5), torch.zeros(*Z.shape, Z.shape[1], 3, 5)
+
+    class Own(FCHLCuda):
+        def __init__(self):
+            torch.nn.Module.__init__(self)
+
+        def get_representation_and_derivative(self, *args, **kw):
+            return own(*args, **kw)
+
+    if where == "class":
+        rep = Own()
+    else:
+        rep = FCHLCuda.__new__(FCHLCuda)
+        torch.nn.Module.__init__(rep)
+        rep.get_representation_and_derivative = own
+    model = BaseKernel.__new__(BaseKernel)
+    model.rep, model.reductors, model.elements, model.element2index = rep, torch.zeros(1, 5, 4), torch.tensor([6]), torch.zeros(7, dtype=torch.long)
+    data = {k: None for k in ("atomIDs", "molIDs", "natom_counts", "cells", "inv_cells")}
+    data.update(coordinates=torch.zeros(2, 3, 3), charges=torch.ones(2, 3), element_counts={1: 6})     # no atom of the model's element
+    assert model._batch_projected(data, True)["items"] == [] and calls == [(2, 3, 3)]
