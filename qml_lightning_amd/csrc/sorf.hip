@@ -1462,7 +1462,7 @@ __global__ void segment_offsets_kernel(const int* __restrict__ mol_index, int A,
         seg[nmol + 1] = 1;
         return;
     }
-    for (int m = prev + 1; m <= cur; ++m) seg[m] = t;
+    for (int m = max(prev, -1) + 1; m <= cur; ++m) seg[m] = t;      // (a negative index before this one: the flag is raised there)
 }
 
 // The same table by one workgroup, which needs no cleared flag.  Bound by launches where it is used: of the operator sequence's 76
@@ -1476,7 +1476,7 @@ __global__ __launch_bounds__(SEG_THREADS) void segment_table_kernel(const int* _
         const int cur = t == A ? nmol : mol_index[t];
         if (prev > cur || cur < 0 || cur > nmol || (t < A && cur == nmol)) bad = true;
         else
-            for (int m = prev + 1; m <= cur; ++m) seg[m] = t;
+            for (int m = max(prev, -1) + 1; m <= cur; ++m) seg[m] = t;
     }
     bad = __syncthreads_or(bad);
     if (threadIdx.x == 0) seg[nmol + 1] = bad;

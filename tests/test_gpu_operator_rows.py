@@ -47,8 +47,8 @@ def test_no_slots():
 
 
 @pytest.mark.parametrize("A,F,nmol,order", [(1, 4, 1, "up"), (7, 260, 5, "up"), (40, 64, 900, "up"), (300, 33, 3, "up"), (300, 128, 40, "mixed"),
-                                            (300, 128, 40, "out"), (16383, 8, 700, "up"), (16384, 8, 700, "up"), (16385, 8, 700, "up"),
-                                            (16385, 8, 700, "mixed"), (600, 4096, 2050, "up")])
+                                            (300, 128, 40, "out"), (300, 128, 40, "below"), (16383, 8, 700, "up"), (16384, 8, 700, "up"),
+                                            (16385, 8, 700, "up"), (16385, 8, 700, "mixed"), (16385, 8, 700, "below"), (600, 4096, 2050, "up")])
 def test_cos_features_of_molecules(A, F, nmol, order):
     """Molecules without atoms, one and several columns per thread, the table by one workgroup and by many, and an index that is not
     ascending or leaves the range (its atoms are left out)."""
@@ -60,12 +60,15 @@ def test_cos_features_of_molecules(A, F, nmol, order):
         idx = idx.sort()[0]
     if order == "out":
         idx[::7] = nmol
+    if order == "below":
+        idx = idx.sort()[0]
+        idx[::7] = -5                                      # and behind each a valid one, whose entries begin at 0
     torch.full((nmol, F), float("nan"), device=dev())              # what the result's memory may hold
     got = torch.ops.qml_lightning_sorf.get_cos_features(c, b, torch.tensor(nmol), idx.int())
-    ok = idx < nmol
+    ok = (idx >= 0) & (idx < nmol)
     want = torch.zeros(nmol, F, device=dev(), dtype=torch.float64)
     want.index_add_(0, idx[ok], np.sqrt(2.0 / F) * torch.cos(c[ok].double() + b.double()))
-    most = torch.bincount(idx).max().item()
+    most = torch.bincount(idx[ok]).max().item()
     # 3.7e-7 of a cosine, a rounding per sum
     assert (got.double() - want).abs().max().item() < np.sqrt(2.0 / F) * most * (4e-7 + most * 6e-8)
 
