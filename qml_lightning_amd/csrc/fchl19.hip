@@ -67,6 +67,11 @@ constexpr float PI_F = 3.14159265358979323846f;
 // three floats read from a 16-byte-aligned LDS entry with a single 12-byte instruction (a 16-byte
 // read of the same entry occupies the LDS pipe a third longer)
 typedef float float3v __attribute__((ext_vector_type(3)));
+// an entry of tables that have twelve bytes each, where float3v (sixteen, with a gap) would reach into the next one
+struct Float3 {
+    float x, y, z;
+};
+static_assert(sizeof(Float3) == 12, "a table entry");
 
 // LDS neighbour arrays of one central atom, sorted by element type (stable in j within a
 // type); goff[e]..goff[e+1] is the slice of type e.
@@ -929,7 +934,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             const float* f = trip + 3 * (first[e] + half);
             float acc = 0.0f;
             auto add = [&](const float* at, bool there) {
-                float3v v;
+                Float3 v;
                 __builtin_memcpy(&v, at, sizeof v);
                 const float u = lnRs - v.x;
                 acc = fmaf(there ? v.z : 0.0f, fexp2(-u * u * v.y), acc);
@@ -960,7 +965,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             const unsigned long long places = (unsigned long long)__float_as_uint(Bk.w) << 32 | __float_as_uint(Bk.z);
             const int at = (int)((unsigned)(places >> (__float_as_uint(Bj.w) >> 23)) & 0x7ff) + j;
             const float4 v = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
-            const float3v w = {v.x, v.y, v.z};
+            const Float3 w = {v.x, v.y, v.z};
             __builtin_memcpy(trip + 3 * at, &w, sizeof w);
         }
     }
@@ -979,7 +984,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             if (g + s < NP) {
 #pragma unroll 2
                 for (int it = 0; it < rounds[g + s < NP ? g + s : 0]; ++it, src += 3 * LEAN_SLOTS) {
-                    float3v t;
+                    Float3 t;
                     __builtin_memcpy(&t, src, sizeof t);
                     const float d0 = t.x - rsa, d1 = t.x - rsb;
                     const float e0 = fexp2(-d0 * d0), e1 = fexp2(-d1 * d1);
