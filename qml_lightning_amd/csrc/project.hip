@@ -624,6 +624,13 @@ __global__ __launch_bounds__(PT) void reductor_presplit_bwd_kernel(const float* 
 // alone or with vmcnt(16) or (0)
 constexpr int WAIT_VM4 = 0x0f74, WAIT_LDS = 0xc07f, WAIT_LDS_VM16 = 0x4070, WAIT_LDS_VM0 = 0x0070;
 
+// Between an image's loads and what a counted wait lets stay on its way behind them: a wait for all but the last N operations has the
+// image in only if N of them were issued after it
+__device__ __forceinline__ void image_ahead() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0x48f);               // (arithmetic and LDS may cross)
+}
+
 // 2^-(ka + kb) applied to a chunk's product as it is added to the running sums: one factor when it is
 // a float, two multiplies at the ends of the exponent range (operands near the largest or smallest floats)
 __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part, int ka, int kb) {
@@ -676,6 +683,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
                                 ((size_t)type * nchunks * ncb + blockIdx.y) * FWD_IMG_BYTES;
     const int* exps = exponents + (size_t)type * nchunks * ncb + blockIdx.y;
     image_to_lds<FWD_IMG_BYTES>(img0, sB0, wave_s, lane16);
+    if constexpr (AHEAD == 2) image_ahead();
 
     // this lane's row of A: row 32 (wave / CW) + i, of each chunk the k = 16 s + 8 h + (0..7), s = 0, 1.  A lane without a row
     // reads the tile's last one and one beyond K the row's last four entries, so that every lane loads the same number of times
@@ -761,6 +769,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
             __syncthreads();
         }
         if (c + 1 < nchunks) image_to_lds<FWD_IMG_BYTES>(img0 + (size_t)(c + 1) * ncb * FWD_IMG_BYTES, other, wave_s, lane16);
+        if constexpr (AHEAD == 2) image_ahead();
         if (AHEAD == 2 || c + 1 < nchunks) fetch((c + AHEAD) * PK, ra);
         if constexpr (AHEAD == 2) __builtin_amdgcn_sched_barrier(0);           // issued here, not behind the products
         const int kb = exps[(size_t)c * ncb];
@@ -969,6 +978,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (b + 1 < nblk) image_to_lds<Img::BYTES>(img0 + (size_t)(b + 1) * Img::BYTES, other, wave_s, lane16);
+        image_ahead();
         float16_t acc;
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
