@@ -657,10 +657,8 @@ __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part
 // largest value by row rotations instead of LDS shuffles and the parts split two at a time 496 x 128 takes 24.9 us for 8000 atoms
 // and 26.7 for 32583 (27.6 and 29.4 before), 312 x 128 18.6 for 16384 (20.2).  Large batches run at some 3 TB/s: matrix and vector
 // units, LDS and first-level cache are each busy for a quarter to two fifths of the time.  What they gained from scalar exponents and
-// from loads without branches: 720 x 128, 98000 atoms 124 -> 111 us, 131235 162 -> 148.  Tiles of 128 rows fill all 168 registers: five
-// that did not fit, and a copy of the loop's last round, cost the batches of one to two tiles per CU a tenth (496 x 128, 33000 atoms 41.6
-// us with them, 37.4 without; 55000 46.0, 41.8; 720 x 128, 37000 58.6, 51.2).  Rows two chunks ahead in tiles of 128 spill; tiles of 64
-// there, with which they fit, read the images twice as often (131072 atoms of 496 132 us, 103).
+// from loads without branches: 720 x 128, 98000 atoms 115 -> 111 us, 131235 153 -> 147, 262144 280 -> 265.  Rows two chunks ahead in
+// tiles of 128 spill; tiles of 64 there, with which they fit, read the images twice as often (131235 atoms 197).
 template <int RT>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void typed_gemm_f16_kernel(
     const float* __restrict__ A, int lda, const int* __restrict__ a_rows, const _Float16* __restrict__ images,
@@ -690,7 +688,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     // this lane's row of A: row 32 (wave / CW) + i, of each chunk the k = 16 s + 8 h + (0..7), s = 0, 1.  A lane without a row
     // reads the tile's last one and one beyond K the row's last four entries, so that every lane loads the same number of times
     // and the waits can count on it
-    const int wrow = 32 * (wave_s / CW), jt0 = NJ * (wave_s % CW);
+    const int wrow = 32 * (wave / CW), jt0 = NJ * (wave % CW);
     const int r = min(wrow + i, rows - 1);
     size_t src = 0;
     if (group > 1) {
@@ -701,20 +699,12 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     }
     const float* arow = A + src * lda;
     float4 ra[AHEAD][2][2];
-    // 8 h, made anew for each chunk (hence the second operand): it is the register too many that would otherwise be kept in memory
-    // and waited for, with all loads on the way, in every round
-    auto upper_half = [&](int k0) {
-        int v;
-        asm("v_cndmask_b32 %0, 0, 8, %1" : "=v"(v) : "s"(0xffffffff00000000ull), "s"(k0));
-        return v;
-    };
     auto fetch = [&](int k0, float4 (&to)[2][2]) {
-        const int h8 = upper_half(k0);
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
             for (int e = 0; e < 2; ++e)
-                to[s2][e] = *reinterpret_cast<const float4*>(arow + min(k0 + 16 * s2 + h8 + 4 * e, K - 4));
+                to[s2][e] = *reinterpret_cast<const float4*>(arow + min(k0 + 16 * s2 + 8 * h + 4 * e, K - 4));
     };
     auto max4 = [](float m, float4 v) { return fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w)); };
 
@@ -731,12 +721,11 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
     auto round = [&](int c, const _Float16* cur, _Float16* other, float4 (&ra)[2][2]) {
         if constexpr (AHEAD == 2) __builtin_amdgcn_s_waitcnt(WAIT_VM4);        // all but the rows of the chunk behind this one
         if (c * PK + PK > K) {           // the last chunk: zeros beyond K
-            const int h8 = upper_half(c);
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
                 for (int e = 0; e < 2; ++e)
-                    if (c * PK + 16 * s2 + h8 + 4 * e >= K) ra[s2][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (c * PK + 16 * s2 + 8 * h + 4 * e >= K) ra[s2][e] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         // the rows of this chunk: the wavefront's power of two, two fp16 parts each
         float ma = max4(max4(max4(max4(0.0f, ra[0][0]), ra[0][1]), ra[1][0]), ra[1][1]);
@@ -808,28 +797,19 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void ty
             for (int jj = 0; jj < 2; ++jj) add_scaled(acc[j0 + jj], part[jj], ka, kb);
         }
     };
-    if constexpr (AHEAD == 2) {          // (two rounds that the compiler need not join: it would copy rows that are on their way)
-        int c = 0;
-        for (; c + 1 < nchunks; c += 2) {
-            round(c, sB0, sB1, ra[0]);
-            round(c + 1, sB1, sB0, ra[1]);
-        }
-        if (c < nchunks) round(c, sB0, sB1, ra[0]);
-    } else {
-        for (int c = 0; c < nchunks; c += 2) {
-            round(c, sB0, sB1, ra[0]);
-            if (c + 1 < nchunks) round(c + 1, sB1, sB0, ra[0]);
-        }
+    int c = 0;
+    for (; c + 1 < nchunks; c += 2) {
+        round(c, sB0, sB1, ra[0]);
+        round(c + 1, sB1, sB0, ra[AHEAD - 1]);
     }
+    if (c < nchunks) round(c, sB0, sB1, ra[0]);
 
-    const int at = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));     // the lane again: see upper_half
-    const int io = at & 31, ho = at >> 5;
 #pragma unroll
     for (int jt = 0; jt < NJ; ++jt) {
-        const int col = col0 + 32 * (jt0 + jt) + io;
+        const int col = col0 + 32 * (jt0 + jt) + i;
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            const int row = wrow + 8 * (q / 4) + 4 * ho + (q % 4);
+            const int row = wrow + 8 * (q / 4) + 4 * h + (q % 4);
             if (row < rows && col < N) C[(size_t)(row0 + row) * ldc + col] = acc[jt][q];
         }
     }
@@ -1555,11 +1535,10 @@ extern "C" int qmll_project_typed(const float* rep, const int* sorted_slots, con
         const SplitLayout L = split_layout(ne, R, d);
         QMLL_REQUIRE(aligned16(reductors_split), QMLL_ERR_INVALID, "qmll_project_typed: reductors_split must be 16-byte aligned");
         const unsigned char* base = (const unsigned char*)reductors_split;
-        // Tiles of 64 rows while they leave no CU with more than one: twice the workgroups, each with half the products and
+        // Tiles of 64 rows while they leave no CU with more than two: twice the workgroups, each with half the products and
         // conversions per round of a chain that is all latency there; beyond, the images, which a tile reads whole, decide.  496 x
-        // 128, tiles of 128 / 64 rows: 8000 atoms 28.6 / 24.0 us, 16000 30.2 / 26.4, 17000 30.7 / 31.2, 24000 32.7 / 34.5, 32768 37 / 45, 65536
-        // 59 / 70, 131072 103 / 132; 496 x 256: 5000 29 / 23.9, 9000 29.9 / 30.3
-        if ((long long)((A + 63) / 64) * (d / 128) <= 256) {
+        // 128, tiles of 128 / 64 rows: 8000 atoms 25.7 / 20.1 us, 16384 26.9 / 24.2, 32768 36.3 / 37.4, 65536 53 / 61, 131072 105 / 139
+        if ((long long)tiles * (d / 128) <= 192) {
             hipLaunchKernelGGL(typed_gemm_f16_kernel<64>, dim3((A + 63) / 64 + ne, d / 128), dim3(PT), 0, (hipStream_t)stream, rep, R, sorted_slots,
                                (const _Float16*)base, (const int*)(base + L.fwd_bytes + L.bwd_bytes), x, d, type_offsets, ne, R, d, 1);
         } else {
