@@ -620,9 +620,8 @@ __global__ __launch_bounds__(PT) void reductor_presplit_bwd_kernel(const float* 
     for (int t = tid; t < Img::BYTES / 16; t += PT) dst[t] = reinterpret_cast<const float4*>(img)[t];
 }
 
-// s_waitcnt: vmcnt(4) alone, and ahead of a barrier, behind which what this wavefront has read in LDS may be overwritten, lgkmcnt(0)
-// alone or with vmcnt(16) or (0)
-constexpr int WAIT_VM4 = 0x0f74, WAIT_LDS = 0xc07f, WAIT_LDS_VM16 = 0x4070, WAIT_LDS_VM0 = 0x0070;
+// s_waitcnt: vmcnt(4) alone, and ahead of a barrier, behind which what this wavefront has read in LDS may be overwritten, lgkmcnt(0) alone
+constexpr int WAIT_VM4 = 0x0f74, WAIT_LDS = 0xc07f;
 
 // Between an image's loads and what a counted wait lets stay on its way behind them: a wait for all but the last N operations has the
 // image in only if N of them were issued after it
@@ -891,7 +890,8 @@ __global__ __launch_bounds__(256) void zero_untyped_rows_kernel(Aside aside, int
 // wavefront's power of two), so every row of A is read exactly once; the workgroup walks the N columns
 // in blocks of 32, each block's image arriving in LDS while the previous block is multiplied, and every
 // 32 x 32 block of C leaves straight from the accumulators through the two inverse factors.
-// (K = 256: the parts of the rows take 128 registers, hence two wavefronts per SIMD.  Against fp64 the relative error is 1.9e-7,
+// (K = 256: the parts of the rows take 128 registers, hence two wavefronts per SIMD; twelve that do not fit are read back ahead of the
+// first block.  Against fp64 the relative error is 1.9e-7,
 // of the fp32 matrix instructions 2.9e-7, from 4200 to 66000 atoms and three to five elements.)
 template <int K>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2 : K == 128 ? 3 : 4))) void typed_gemm_bt_rows_f16_kernel(const float* __restrict__ A,
@@ -960,25 +960,22 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
                 al[j][q + 1] = lo[1];
             }
     }
-    float* dst[16];                     // of the 16 accumulator registers, in the first block; a row the tile does not have: row 0's
+    int dst[16];                        // rows of the 16 accumulator registers; a row the tile does not have: row 0
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int row = 32 * wave + 8 * (q / 4) + 4 * h + (q % 4);
         const int at = row0 + (row < rows ? row : 0);
-        dst[q] = C + (size_t)(c_rows ? c_rows[at] : at) * ldc + i;
+        dst[q] = c_rows ? c_rows[at] : at;
     }
     // one block of 32 columns: its image is in `cur`, the next one is loaded into `other`
-    // (a full tile stores sixteen times per block, all behind the next image's loads, and need not wait for the stores: 496 columns,
-    // 65536 atoms 50.4 -> 48.1 us, 86016 54.8 -> 50.5)
+    // The wait takes in the stores of the block before.  Waiting for all but those sixteen made the compiler add waits of its own, for the
+    // image that had just been asked for, and copy the first round; pointers in place of row numbers take registers that K = 256 has not
+    // (counted waits and pointers / this: 496 columns x 128, 41796 atoms 44.0 / 41.1 us, 9000 27.1 / 24.9; 720 x 256, 41796 94 / 86, 9000 52.5 / 46)
     const bool full = rows == PM;
     auto round = [&](int b, const unsigned char* cur, unsigned char* other) {
-        asm volatile("" ::: "memory");
-        if (full && b > 0) __builtin_amdgcn_s_waitcnt(WAIT_LDS_VM16);
-        else __builtin_amdgcn_s_waitcnt(WAIT_LDS_VM0);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
         if (b + 1 < nblk) image_to_lds<Img::BYTES>(img0 + (size_t)(b + 1) * Img::BYTES, other, wave_s, lane16);
-        image_ahead();
         float16_t acc;
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
@@ -996,12 +993,12 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(K == 256 ? 2
         const int col = 32 * b + i;
         if (full && 32 * b + 32 <= N) {
 #pragma unroll
-            for (int q = 0; q < 16; ++q) dst[q][32 * b] = acc[q] * inv_sa * sinv;
+            for (int q = 0; q < 16; ++q) C[(size_t)dst[q] * ldc + col] = acc[q] * inv_sa * sinv;
         } else if (col < N) {
             // the two inverse factors one after the other: their product need not be a float
 #pragma unroll
             for (int q = 0; q < 16; ++q)
-                if (32 * wave + 8 * (q / 4) + 4 * h + (q % 4) < rows) dst[q][32 * b] = acc[q] * inv_sa * sinv;
+                if (32 * wave + 8 * (q / 4) + 4 * h + (q % 4) < rows) C[(size_t)dst[q] * ldc + col] = acc[q] * inv_sa * sinv;
         }
     };
     for (int b = 0; b < nblk; b += 2) {

@@ -1,5 +1,5 @@
-"""The projections' kernels wait for an image in LDS with a count of what was issued behind its loads.  The source pins that order; here
-it is read off the code that the compiler made, on the CPU."""
+"""The projections' kernels as the compiler makes them, on the CPU.  They wait for an image in LDS with a count of what was issued behind
+its loads: the source pins that order, which is read off the assembly here."""
 import os
 import re
 import shutil
@@ -8,11 +8,6 @@ import subprocess
 import pytest
 
 from qml_lightning_amd import build
-
-# (kernel, what the wait lets stay on its way, how many of them)
-KERNELS = [("typed_gemm_f16_kernelILi64E", "r", 4), ("typed_gemm_bt_rows_f16_kernelILi64E", "w", 16),
-           ("typed_gemm_bt_rows_f16_kernelILi128E", "w", 16), ("typed_gemm_bt_rows_f16_kernelILi256E", "w", 16)]
-
 
 def operations(text):
     """One letter per instruction: L load into LDS, r load, w store, B barrier, W wait for all but the last operations (a count), 0 wait
@@ -33,24 +28,23 @@ def operations(text):
     return out
 
 
-def images_are_waited_for(ops, kind, count):
-    """Every wait that counts stands behind an image's loads and `count` operations of `kind` after them, and every barrier is followed by
-    the next image's loads before anything else."""
+def images_are_waited_for(ops, count):
+    """Every wait that counts stands behind an image's loads and `count` loads after them, and every barrier is followed by the next
+    image's loads before anything else."""
     waits = [m.start() for m in re.finditer("W", ops)]
     for at in waits:
         behind = ops[ops.rindex("L", 0, at) + 1:at] if "L" in ops[:at] else ""
-        if behind.count(kind) < count:
+        if behind.count("r") < count:
             return False
     return bool(waits) and all(ops[m.end():m.end() + 1] == "L" for m in re.finditer("B", ops))
 
 
 def test_what_is_looked_for():
     good = "LLLrrrrrrrr" + "WBLLrrrr" * 3 + "WBLLwww"
-    assert images_are_waited_for(good, "r", 4)
-    assert not images_are_waited_for(good.replace("BLLrrrr", "BrLLrrr", 1), "r", 4)       # a load ahead of the image's
-    assert not images_are_waited_for("LLLrrrrWBLLrrrWBLL", "r", 4)                        # one too few behind them
-    assert not images_are_waited_for("LL0BLL" + "w" * 15 + "LWBLL", "w", 16)               # an image's load behind the stores
-    assert images_are_waited_for("LL0BLL" + "w" * 16 + "WBLL", "w", 16)
+    assert images_are_waited_for(good, 4)
+    assert not images_are_waited_for(good.replace("BLLrrrr", "BrLLrrr", 1), 4)       # a load ahead of the image's
+    assert not images_are_waited_for("LLLrrrrWBLLrrrWBLL", 4)                        # one too few behind them
+    assert not images_are_waited_for("LLLrrrrWBLLrrrLrWBLL", 4)                      # an image's load among them
 
 
 @pytest.fixture(scope="module")
@@ -63,7 +57,19 @@ def assembly(tmp_path_factory):
     return open(out).read()
 
 
-@pytest.mark.parametrize("kernel,kind,count", KERNELS)
-def test_images_are_issued_ahead(assembly, kernel, kind, count):
-    text = re.search(r"^_ZN\S*%s\S*:(.*?)^\s*\.section" % kernel, assembly, re.S | re.M).group(1)
-    assert images_are_waited_for(operations(text), kind, count)
+def code(assembly, kernel):
+    return operations(re.search(r"^_ZN\S*%s\S*:(.*?)^\s*\.section" % kernel, assembly, re.S | re.M).group(1))
+
+
+def test_images_are_issued_ahead(assembly):
+    assert images_are_waited_for(code(assembly, "typed_gemm_f16_kernelILi64E"), 4)
+
+
+@pytest.mark.parametrize("columns", [64, 128, 256])
+def test_an_image_on_its_way_is_not_waited_for(assembly, columns):
+    """In the transposed kernel the next image's loads overlap the products: no wait for all of them between the image's loads and the
+    stores of the block."""
+    ops = code(assembly, "typed_gemm_bt_rows_f16_kernelILi%dE" % columns)
+    assert "W" not in ops
+    for m in re.finditer("BL+", ops):
+        assert ops[m.end()] == "w"
