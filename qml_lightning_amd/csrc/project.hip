@@ -656,8 +656,12 @@ __device__ __forceinline__ void add_scaled(float16_t& acc, const float16_t& part
 // largest value by row rotations instead of LDS shuffles and the parts split two at a time 496 x 128 takes 24.9 us for 8000 atoms
 // and 26.7 for 32583 (27.6 and 29.4 before), 312 x 128 18.6 for 16384 (20.2).  Large batches run at some 3 TB/s: matrix and vector
 // units, LDS and first-level cache are each busy for a quarter to two fifths of the time.  What they gained from scalar exponents and
-// from loads without branches: 720 x 128, 98000 atoms 115 -> 111 us, 131235 153 -> 147, 262144 280 -> 265.  Rows two chunks ahead in
-// tiles of 128 spill; tiles of 64 there, with which they fit, read the images twice as often (131235 atoms 197).
+// from loads without branches: 720 x 128, 98000 atoms 124 -> 114 us, 131235 162 -> 153.  Rows two chunks ahead in
+// tiles of 128 spill; tiles of 64 there, with which they fit, read the images twice as often (131072 atoms of 496 132 us, 109).
+// The kernel of 128 rows keeps five registers in memory, read back ahead of an odd last round and of the stores, and the loop's odd last round is a
+// third copy of its code: together a tenth of the launch for one to two tiles per CU (496 x 128, 33000 atoms 41.6 us, 37.4 without, 37.5
+// before scalar exponents; 65536 55.5, 58.2, 58.5).  The form without them was taken back all the same: behind and ahead of it every other kernel of a
+// prediction with 256 components ran 2 to 3 % slower, as at a lower clock (41796 atoms, 32768 features 1152 -> 1194 us).
 template <int RT>
 __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(3))) void typed_gemm_f16_kernel(
     const float* __restrict__ A, int lda, const int* __restrict__ a_rows, const _Float16* __restrict__ images,
