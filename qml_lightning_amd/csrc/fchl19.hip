@@ -762,14 +762,6 @@ struct BatchPrep {
 };
 constexpr int PREP_ATOMS = 256, PREP_ELEMENTS = 8;
 
-__device__ __forceinline__ int index_of_charge(float z, const float* __restrict__ species, int ns) {
-    const int q = (int)z;
-    int t = -1;
-    for (int j = 0; j < ns; ++j)
-        if (q == (int)species[j]) t = j;
-    return t;
-}
-
 // group 0: the listed atoms sorted by the model's element (stable), one wavefront, 64 atoms at a time; the others: element indices of
 // the slots (0 for padded ones) and the zeros
 __device__ __forceinline__ void prepare_group(const FchlArgs& a, const BatchPrep& b, int group, int lane, int* lds) {
@@ -780,8 +772,8 @@ __device__ __forceinline__ void prepare_group(const FchlArgs& a, const BatchPrep
         for (int s = (group - 1) * 64 + lane; s < b.slots; s += step) {
             const int m = s / a.n;
             const bool real = s - m * a.n < a.natoms[m];
-            b.types[s] = real ? index_of_charge(b.Z[s], b.species, ns) : 0;
-            if (b.model_species) b.sort_types[s] = real ? index_of_charge(b.Z[s], b.model_species, b.ne) : 0;
+            b.types[s] = real ? species_index(b.Z[s], b.species, ns) : 0;
+            if (b.model_species) b.sort_types[s] = real ? species_index(b.Z[s], b.model_species, b.ne) : 0;
         }
         for (int t = (group - 1) * 64 + lane; t < b.zero_count; t += step) b.zero[t] = 0.0f;
         return;
@@ -796,7 +788,7 @@ __device__ __forceinline__ void prepare_group(const FchlArgs& a, const BatchPrep
         if (at < b.A) {
             const int m = a.molIDs[at], i = a.atomIDs[at];
             slot = m * a.n + i;
-            t = i < a.natoms[m] ? index_of_charge(b.Z[slot], list, nlist) : 0;
+            t = i < a.natoms[m] ? species_index(b.Z[slot], list, nlist) : 0;
             lds[at] = slot << 4 | (t + 1);
         }
 #pragma unroll
@@ -852,7 +844,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
     const float* Xm = a.X + (size_t)m * a.n * 3;
     const int own = lane < a.n ? lane : 0;
     const float xj = Xm[own * 3 + 0], yj = Xm[own * 3 + 1], zj = Xm[own * 3 + 2];
-    const int et = PREP ? index_of_charge(b.Z[(size_t)m * a.n + own], b.species, NS) : a.types[(size_t)m * a.n + own];
+    const int et = PREP ? species_index(b.Z[(size_t)m * a.n + own], b.species, NS) : a.types[(size_t)m * a.n + own];
     const int z = lane & 31, half = lane >> 5;           // two-body: radial bin, neighbour of two
     const float rs2v = z < nRs2 ? a.Rs2[z] : 1.0f;
     const int slot = idiv_small(lane, LEAN_LANES), ll = lane - LEAN_LANES * slot;      // three-body: triple of six, pair of bins

@@ -94,14 +94,7 @@ __global__ __launch_bounds__(256) void element_types_kernel(const float* __restr
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)B * n) return;
     const int m = idx / n, i = idx - (size_t)m * n;
-    int t = 0;
-    if (i < natoms[m]) {
-        const int q = (int)Z[idx];
-        t = -1;
-        for (int j = 0; j < ns; ++j)
-            if (q == (int)species[j]) t = j;
-    }
-    types[idx] = t;
+    types[idx] = i < natoms[m] ? species_index(Z[idx], species, ns) : 0;
 }
 
 static int check_nb(const float* X, const int* natoms, const float* cell, const float* inv_cell, int B, int n,

@@ -66,15 +66,6 @@ __global__ __launch_bounds__(ST) void type_count_kernel(const int* __restrict__ 
     count_types(a < A ? types[slots[a]] : -1, ne, counts);
 }
 
-// index of charge z in a species list, -1 when it is not there (the rule of element_types_kernel)
-__device__ __forceinline__ int species_index(float z, const float* __restrict__ species, int ns) {
-    const int q = (int)z;
-    int t = -1;
-    for (int j = 0; j < ns; ++j)
-        if (q == (int)species[j]) t = j;
-    return t;
-}
-
 // the same counts from charges, whose element indices are written on the way
 __global__ __launch_bounds__(ST) void charge_count_kernel(const float* __restrict__ Z, const float* __restrict__ species, int A, int ne,
                                                            int* __restrict__ types, int* __restrict__ counts) {

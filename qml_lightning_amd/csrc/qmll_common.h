@@ -34,6 +34,15 @@ int qmll_sorf_rows_if(const float* x, const int* type_offsets, const int* sorted
                       const float* alpha, int A, int ne, int d, int S, int T, float normalisation, const int* only_if, float* e_slots,
                       float* gx, hipStream_t stream);
 
+// index of charge z, truncated, in a species list: -1 when it is not there, of equal entries the last
+__device__ __forceinline__ int species_index(float z, const float* __restrict__ species, int ns) {
+    const int q = (int)z;
+    int t = -1;
+    for (int j = 0; j < ns; ++j)
+        if (q == (int)species[j]) t = j;
+    return t;
+}
+
 static inline bool qmll_is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 static inline int qmll_log2(int v) {
     int l = 0;
