@@ -93,27 +93,44 @@ def test_small_projections(A, ne, R, d, nparts):
 def test_batch_prepared_beside_the_representation(elements, atoms, pad):
     """The one launch of few atoms against the separate kernels: up to 256 atoms, a model with its own element list (in another
     order, more elements than the launch sorts), padded slots, atoms listed in another order than they are stored."""
+    _prepared_beside_the_representation([1, 6, 8], elements, atoms, pad, None)
+
+
+@pytest.mark.parametrize("species", [[1], [6, 1], [1, 6, 8], [1, 6, 7, 8], [1, 6, 7, 8, 9], [1, 6, 7, 8, 9, 16]])
+@pytest.mark.parametrize("elements", [None, [8, 1]])
+@pytest.mark.parametrize("edge", [None, 6.5])
+def test_batch_prepared_beside_the_representation_of_any_species(species, elements, edge):
+    """A kernel for each number of the representation's elements (six take the separate kernels), free and in boxes."""
+    for atoms in (1, 64, 250):
+        _prepared_beside_the_representation(species, elements or species, atoms, 3, edge)
+
+
+def _prepared_beside_the_representation(species, elements, atoms, pad, edge):
     import ctypes
     from qml_lightning_amd import _lib, ops
     from qml_lightning_amd.representations.FCHL import FCHLCuda
     rng = np.random.default_rng(atoms)
-    rep = FCHLCuda(species=np.array([1, 6, 8]))
+    rep = FCHLCuda(species=np.array(species))
     n = 21
     B = (atoms + n - 1) // n
     counts = np.minimum(n, atoms - n * np.arange(B))
     n += pad
     dev = torch.device("cuda:0")
     X = torch.tensor(rng.uniform(0, 6, (B, n, 3)), dtype=torch.float32, device=dev)
-    Z = torch.tensor(np.where(np.arange(n) < counts[:, None], rng.choice([1, 6, 8, 16], (B, n)), 0), dtype=torch.float32, device=dev)
+    Z = torch.tensor(np.where(np.arange(n) < counts[:, None], rng.choice(sorted({1, 6, 8, 16} | set(species)), (B, n)), 0), dtype=torch.float32, device=dev)
     order = rng.permutation(atoms)
     aid = torch.tensor(np.concatenate([np.arange(k) for k in counts])[order], dtype=torch.int32, device=dev)
     mid = torch.tensor(np.repeat(np.arange(B), counts)[order], dtype=torch.int32, device=dev)
     nat = torch.tensor(counts, dtype=torch.int32, device=dev)
-    msp = None if elements == [1, 6, 8] else torch.tensor(elements, dtype=torch.float32, device=dev)
+    cell = icell = None
+    if edge is not None:
+        cell = torch.eye(3, device=dev).mul(edge).expand(B, 3, 3).contiguous()
+        icell = torch.eye(3, device=dev).div(edge).expand(B, 3, 3).contiguous()
+    msp = None if elements == species else torch.tensor(elements, dtype=torch.float32, device=dev)
     types, stypes, ss, off, zeroed = ops.prepare_batch(Z, nat, rep.species, aid, mid, msp, 5 * B * n)
-    prm = ops.make_params(3, rep.Rs2, rep.Rs3, rep.eta2, rep.eta3, rep.two_body_decay, rep.three_body_weight,
+    prm = ops.make_params(len(species), rep.Rs2, rep.Rs3, rep.eta2, rep.eta3, rep.two_body_decay, rep.three_body_weight,
                           rep.three_body_decay, rep.rcut)
-    want = ops.fchl_forward(X, types, None, None, aid, mid, nat, rep.Rs2, rep.Rs3, prm)
+    want = ops.fchl_forward(X, types, cell, icell, aid, mid, nat, rep.Rs2, rep.Rs3, prm)
     ne = len(elements)
     got = [torch.full_like(t, -7) for t in (types, stypes, ss, off)]
     zero = torch.full((5 * B * n,), 3.0, device=dev)
@@ -121,7 +138,7 @@ def test_batch_prepared_beside_the_representation(elements, atoms, pad):
     work = torch.empty(65536, dtype=torch.int32, device=dev)
     p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())       # noqa: E731
     _lib.check(_lib.lib().qmll_prepare_fchl19_forward(
-        p(X), p(Z), p(rep.species), p(msp), ne, None, None, p(aid), p(mid), p(nat), atoms, B, n, p(rep.Rs2), p(rep.Rs3),
+        p(X), p(Z), p(rep.species), p(msp), ne, p(cell), p(icell), p(aid), p(mid), p(nat), atoms, B, n, p(rep.Rs2), p(rep.Rs3),
         ctypes.byref(prm), p(work), 4 * 65536, p(got[0]), p(got[1]) if msp is not None else None, p(got[2]), p(got[3]), p(zero),
         zero.numel(), p(r), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "qmll_prepare_fchl19_forward")
     assert torch.equal(got[0], types) and (msp is None or torch.equal(got[1], stypes))
