@@ -1622,7 +1622,7 @@ extern "C" int qmll_project_typed_backward_parts(float* gx, int nparts, const in
     const int beside = aside.zero_groups + aside.sum_groups;
     // short contraction: the gradient rows stay in registers, every row is read once.  At d = 256 a tile walks its columns
     // at two wavefronts per SIMD, too slowly for a batch that has less than a tile for every fourth CU: fp32 kernel / this one at 496
-    // columns, 4200 atoms 29 / 34 us, 8000 atoms 41 / 35, 41796 atoms 146 / 62
+    // columns, 4200 atoms 35 / 34 us, 6000 35 / 35, 8000 46 / 36, 41796 141 / 62 with the data in no cache (29 / 34 at 4200 with it in one)
     const bool rows_in_registers = !small && vec && A > 0 && (d == 64 || d == 128 || (d == 256 && A >= 8000)) && reductors_split;
     if (!small && !rows_in_registers && beside > 0) {
         hipLaunchKernelGGL(zero_untyped_rows_kernel, dim3(beside), dim3(256), 0, (hipStream_t)stream, aside, ne, R, g_rep);
