@@ -19,11 +19,14 @@
 // / gradients, rows kernel -> this one, relative: d = 128, 128 stacks 3.7e-7 / 3.1e-7 -> 2.3e-7 / 2.2e-7, two transforms, 32 stacks
 // 3.1e-7 / 3.1e-7 -> 2.4e-7 / 2.4e-7; with arguments twice as large and falling components 4.7e-7 / 4.6e-7 -> 4.2e-7 / 4.3e-7 at most.
 // Power-of-two scales keep everything in fp16's range: x per atom
-// (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per call.
+// (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per call.  With one transform x has a fixed scale, whose
+// inverse is in the H_16 blocks, so that the accumulators hold revolutions and can start from the bias behind the inverse of the
+// register part's stages: the fma that scaled and added it, 32 per stack, is gone (131072 atoms, 64 stacks, energies only 248 -> 226 us;
+// with the gradient 86016 atoms, 128 stacks 630 -> 624).
 //
 // Instruction issue bounds it, as it does the kernel without matrix instructions (sorf_energy_rows_kernel, which at
 // d = 128 spends 162 vector instructions per 4 atoms and stack, 64 of them cross-lane ones at half rate): here 16 atoms
-// and a stack take 320 plain, 64 conversion and 64 transcendental vector instructions and 16 matrix instructions, and
+// and a stack take 275 plain, 64 conversion and 64 transcendental vector instructions and 16 matrix instructions, and
 // the matrix instructions take issue time of their own (giving one butterfly stage of either side to them leaves the
 // time as it was, giving them two makes it 16 % longer).  Two tiles of atoms per wavefront, one stack per barrier,
 // eight wavefronts per workgroup and four wavefronts per SIMD (with spills) were measured too: 0 to 4 % slower.
@@ -49,6 +52,9 @@ constexpr int SM_WAVES = 4;                  // wavefronts per workgroup
 constexpr int SM_ATOMS = 16 * SM_WAVES;
 constexpr float INV2PI = 0.15915494309189535f;
 constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are taken off the sine argument first
+// One transform: x (in revolutions) goes times 2^SM_EXP into its two fp16 parts: an entry is then off by 2^-33 at most beside its 23
+// bits, far below the rounding of an argument, and atoms of sum |x| up to 128 revolutions fit
+constexpr int SM_EXP = 8;
 
 // stacks per buffer: one barrier for so many (and at least 3 workgroups in LDS)
 constexpr int stacks_per_round(int d, int T) { return d * T <= 128 ? 2 : 1; }
@@ -65,7 +71,8 @@ __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h
 struct Forms {
     half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal
     float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
-    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2 (from fp64: the smaller the argument, the less its rounding)
+    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2 (from fp64: the smaller the argument, the less its rounding); with one
+                          // transform what its accumulators start from, of which the stages over the block index make that
     float* alpha;         // [S][d] 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
     int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
 };
@@ -81,11 +88,11 @@ __device__ __forceinline__ float workgroup_max(float m, float* wmax) {
     return m;
 }
 
-// workgroup 0: alpha; then one per (element, stack).  bias and alpha may be null: the images and bounds alone
+// workgroup 0: alpha; then one per (element, stack).  bias and alpha may be null: the images and bounds alone.  The blocks are +-factor.
 constexpr int PREP_THREADS = 512;
 template <int D, int T>
 __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float* __restrict__ Dmat, const float* __restrict__ bias,
-                                                                    const float* __restrict__ alpha, int S, Forms f) {
+                                                                    const float* __restrict__ alpha, int S, float factor, Forms f) {
     constexpr int NB = D / 16;
     __shared__ float wmax[PREP_THREADS / 64];
     __shared__ float h[D];
@@ -114,8 +121,8 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
             half8_t v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float sd = row[16 * b + 4 * q + r];
-                const _Float16 hv = (_Float16)(h16_negative(i, 4 * q + r) ? -sd : sd);
+                const float sd = row[16 * b + 4 * q + r], v1 = sd * factor;
+                const _Float16 hv = (_Float16)(h16_negative(i, 4 * q + r) ? -v1 : v1);
                 v[r] = hv;
                 v[r + 4] = hv;
                 unfit |= !(fabsf(sd) == 1.0f);
@@ -142,9 +149,18 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     const bool any_unfit = __syncthreads_or(unfit);
     if (bias != nullptr) {
         const size_t at = ((size_t)e * S + s) * D;
-        for (int t = tid; t < D; t += PREP_THREADS) {
+        auto revolutions = [&](int t) {
             const double r = (double)bias[at + t] * 0.15915494309189533577;
-            f.bias[at + t] = (float)(r - rint(r));
+            return r - rint(r);
+        };
+        for (int t = tid; t < D; t += PREP_THREADS) {
+            double v = revolutions(t);
+            if constexpr (T == 1) {      // the stages over the block index are their own inverse but for the factor NB
+                v = 0.0;
+                for (int b = 0; b < NB; ++b) v += h16_negative(t >> 4, b) ? -revolutions(16 * b + (t & 15)) : revolutions(16 * b + (t & 15));
+                v /= NB;
+            }
+            f.bias[at + t] = (float)v;
         }
     }
     if (tid == 0) f.largest[(size_t)e * S + s] = any_unfit ? HUGE_VALF : largest;
@@ -182,7 +198,7 @@ struct StackBuffer {      // what a stack needs, in LDS
     static constexpr int NB = D / 16;
     half8_t signs[T * NB * 64];
     float diag[T * D];
-    float bias[D];        // in revolutions
+    float bias[D];        // in revolutions (see Forms)
     float alpha[D];       // scaled
 };
 
@@ -309,10 +325,10 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const bool live = first < rows;                      // of the whole wavefront
         const bool aok = first + col < rows;
 
-        // x in revolutions, split behind the atom's power of two
+        // x in revolutions, split behind a power of two
         half8_t xop[NB];
-        float inv;
-        bool track;
+        float inv, to_scale;
+        bool wide;
         {
             const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
             f4_t xv[NB];
@@ -328,13 +344,15 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             }
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
-            // every argument is at most sum |x|, times the largest entry of H D_1 H for a second transform, + |bias|: where that
-            // stays below UMAX no stack looks at its arguments
+            // Every argument is at most sum |x|, times the largest entry of H D_1 H for a second transform, + |bias|: where that
+            // stays below UMAX no stack looks at its arguments.  One transform: below the second limit all atoms share one power of
+            // two, whose inverse is in the H_16 blocks.
             const float bound = fmaf(sum, largest, 0.5f);
-            track = __any(!(bound <= UMAX));
-            const int kx = not_finite(sum) ? 0 : scale_exponent(sum);
+            wide = __any(!(bound <= UMAX && (T == 2 || sum < (float)(1 << (15 - SM_EXP)))));
+            const int kx = T == 1 && !wide ? SM_EXP : not_finite(sum) ? 0 : scale_exponent(sum);
             const float sx = pow2i(kx);
-            inv = pow2i(-kx);
+            inv = pow2i((T == 1 ? SM_EXP : 0) - kx);
+            to_scale = pow2i(kx - SM_EXP);
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
 #pragma unroll
@@ -357,35 +375,47 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[b] = zero;
 
-        auto stack = [&](const Buffer& B) {
+        auto stack = [&](const Buffer& B, auto narrow) __attribute__((always_inline)) {
+            const bool look = !decltype(narrow)::value && wide;
             const half8_t* signs = B.signs + lane;
             f4_t v[NB];
+            auto bias = [&](int b) { return *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q); };
+            if constexpr (T == 1) {
+                // The accumulators start not from zero, so that the register part's stages add the bias on the way (an instruction
+                // per value less, and one rounding less).
+                f4_t c[NB];
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const half8_t a = signs[b * 64];
-                v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xop[b], zero, 0, 0, 0);
-            }
-            block_stages<NB>(v);
-            if constexpr (T == 2) {
+                for (int b = 0; b < NB; ++b) c[b] = bias(b);
+                if (__builtin_expect(look, 0)) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) c[b] *= to_scale;
+                }
+#pragma unroll
+                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[b * 64], xop[b], c[b], 0, 0, 0);
+                block_stages<NB>(v);
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[b * 64], xop[b], zero, 0, 0, 0);
+                block_stages<NB>(v);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[(NB + b) * 64], split4(v[b]), zero, 0, 0, 0);
+                block_stages<NB>(v);
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const half8_t a = signs[(NB + b) * 64];
-                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, split4(v[b]), zero, 0, 0, 0);
+                    const f4_t bv = bias(b);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[b][r] = fmaf(v[b][r], inv, bv[r]);
                 }
-                block_stages<NB>(v);
             }
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const f4_t bv = *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[b][r] = fmaf(v[b][r], inv, bv[r]);
-            }
-            if (__builtin_expect(track, 0)) {
+            if (__builtin_expect(look, 0)) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (fabsf(v[b][r]) > UMAX) v[b][r] -= rintf(v[b][r]);      // exact
+                    for (int r = 0; r < 4; ++r) {
+                        const float u = T == 1 ? v[b][r] * inv : v[b][r];
+                        v[b][r] = fabsf(u) > UMAX ? u - rintf(u) : u;      // exact
+                    }
             }
             float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
 #pragma unroll
@@ -422,7 +452,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 }
             }
         };
-        auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB]) {
+        auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB], auto narrow) __attribute__((always_inline)) {
             // these stacks' data has landed (every wavefront waits for its own loads, then for the others), and the
             // other buffer, read in the round before, is free
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -431,12 +461,18 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             if (!live) return;
 #pragma unroll
             for (int k = 0; k < SPB; ++k)
-                if (s + k < s1) stack(cur[k]);
+                if (s + k < s1) stack(cur[k], narrow);
         };
-        for (int s = s0; s < s1; s += 2 * SPB) {
-            round(s, buf0, buf1);
-            if (s + SPB < s1) round(s + SPB, buf1, buf0);
-        }
+        auto all_rounds = [&](auto narrow) __attribute__((always_inline)) {
+            for (int s = s0; s < s1; s += 2 * SPB) {
+                round(s, buf0, buf1, narrow);
+                if (s + SPB < s1) round(s + SPB, buf1, buf0, narrow);
+            }
+        };
+        // Energies only: the short stack without the two branches (131072 atoms, 64 stacks 238 -> 225 us); with the gradient they cost
+        // nothing.
+        if (WITH_GRAD || __builtin_expect(__syncthreads_or(wide), 0)) all_rounds(std::false_type{});
+        else all_rounds(std::true_type{});
 
         const float inv_alpha = alpha_scaled[(size_t)S * D];
         energy += __shfl_xor(energy, 16, 64);
@@ -555,13 +591,13 @@ extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int wit
     return (double)A * S * T * d / 128.0 >= (with_grad ? 2e6 : 1.5e6);
 }
 
-static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, const Forms& f,
-                           hipStream_t st) {
+static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, float factor,
+                           const Forms& f, hipStream_t st) {
     const dim3 grid(ne * S + 1), block(PREP_THREADS);
-    if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, f);
-    else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, f);
-    else if (T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, f);
-    else hipLaunchKernelGGL((sorf_prepare_kernel<128, 2>), grid, block, 0, st, D, bias, alpha, S, f);
+    if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else if (T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else hipLaunchKernelGGL((sorf_prepare_kernel<128, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
 }
 
 extern "C" size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d) {
@@ -576,7 +612,7 @@ extern "C" int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void
     Forms f = {};
     f.images = (half8_t*)out;
     f.largest = (float*)((char*)out + (size_t)ne * T * S * (d / 16) * 1024);
-    launch_prepare(D, nullptr, nullptr, ne, T, S, d, f, (hipStream_t)stream);
+    launch_prepare(D, nullptr, nullptr, ne, T, S, d, 1.0f, f, (hipStream_t)stream);
     QMLL_CHECK_LAUNCH("qmll_sorf_signs");
     return QMLL_OK;
 }
@@ -606,7 +642,7 @@ extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, 
     const int nshares = matrix_shares(matrix_units(A, ne, T, S, d), gx != nullptr);
     const dim3 grid(nshares + (gx ? (A >= 65536 ? 64 : (A >> 10) + 1) : 0));
     hipStream_t st = (hipStream_t)stream;
-    launch_prepare(D, bias, alpha, ne, T, S, d, f, st);
+    launch_prepare(D, bias, alpha, ne, T, S, d, T == 1 ? 1.0f / (1 << SM_EXP) : 1.0f, f, st);
     auto launch = [&](auto dc, auto tc, auto gc) {
         constexpr int DD = decltype(dc)::value, TT = decltype(tc)::value;
         constexpr bool GG = decltype(gc)::value;

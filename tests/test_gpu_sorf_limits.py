@@ -1,0 +1,48 @@
+"""One transform on the matrix cores, with rows on either side of the sums up to which all atoms share one power of two (128
+revolutions) and a stack leaves its arguments as they are (1500 radians)."""
+import numpy as np
+import pytest
+
+from oracle import sorf
+from qml_lightning_amd import _lib, ops
+from tests.test_gpu_kernels import t32, ti32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mixed", [False, True])       # all rows on one side, or one row in a wavefront beyond
+def test_rows_around_the_limits(monkeypatch, d, mixed):
+    monkeypatch.setattr(_lib.lib(), "qmll_sorf_matrix_pays", lambda *a: 1)
+    rng = np.random.default_rng(d + mixed)
+    ne, S, norm, A = 2, 5, 2.0, 40
+    F = S * d
+    D = np.where(rng.uniform(-1, 1, (ne, 1, S, d)) > 0, 1.0, -1.0).astype(np.float32)
+    b = rng.uniform(0, 2 * np.pi, (ne, F)).astype(np.float32)
+    alpha = rng.normal(size=F).astype(np.float32)
+    off = np.array([0, 20, A], dtype=np.int32)
+    shapes = rng.normal(size=(A, d))
+    shapes[::3] *= np.eye(d)[rng.integers(d, size=len(shapes[::3]))] + 1e-3        # one large component: the argument is the sum
+    for limit in (128.0, 1500.0 / (2 * np.pi)):
+        for near in (0.98, 0.999, 1.001, 1.02):
+            of = np.full(A, near)
+            if mixed:
+                of = np.where(np.arange(A) % 16 == 5, near, 0.01)
+            # (sum |x| in revolutions, behind the kernel's factor norm / sqrt(d))
+            x = (shapes / np.abs(shapes).sum(1, keepdims=True) * (of * limit)[:, None] * 2 * np.pi * np.sqrt(d) / norm).astype(np.float32)
+            e_ref, g_ref, err = np.zeros(A), np.zeros((A, d)), np.zeros((A, 1))
+            for a in range(A):
+                t = int(a >= off[1])
+                c = sorf.sorf_coefficients(x[a][None, :].astype(np.float64), D[t], norm).reshape(1, F)
+                e_ref[a] = (np.sqrt(2.0 / F) * np.cos(c + b[t]) * alpha).sum()
+                gc = -np.sqrt(2.0 / F) * np.sin(c + b[t]) * alpha
+                g_ref[a] = sorf.sorf_adjoint(gc.reshape(1, S, d), D[t], norm)[0]
+                # an argument is off by at most 2^-22 of the bound on it and the sine unit by 2^-20; features add up at worst
+                bound = np.abs(x[a]).sum() * norm / np.sqrt(d) + 2 * np.pi
+                err[a] = np.sqrt(2.0 / F) * np.abs(alpha).sum() * (bound * 2.0 ** -22 + 2.0 ** -20)
+            for grad in (True, False):
+                e, gx = ops.sorf_energy_sorted(t32(x), ti32(off), ti32(np.arange(A)), t32(D), t32(b), t32(alpha), norm, 1, A,
+                                               with_grad=grad)
+                assert (np.abs(e.cpu().numpy() - e_ref) <= err[:, 0]).all(), (limit, near)
+                if grad:
+                    assert (np.abs(gx.cpu().numpy() - g_ref) <= err * norm / np.sqrt(d)).all(), (limit, near)
