@@ -14,10 +14,12 @@
 // diagonal must hold +-1) and moved into LDS by direct loads, a round ahead.  The gradient is split per stack (a
 // conversion, a mixed-precision subtraction and a conversion per value); both parts are rounded to nearest, 23 bits
 // together, one less than fp32: the largest error of an operand is 2^-23 of its binade, the root mean square 0.7 x 2^-24.
-// What that adds is taken off elsewhere, in the forms: bias is reduced to half a revolution in fp64 (the argument's rounding
-// is the largest error of either kernel) and the constant factors are rounded once.  Against fp64, root mean square of energies
+// What that adds is taken off elsewhere, in the forms: bias is reduced to a quarter of a revolution in fp64 (the argument's
+// rounding is the largest error of either kernel) and the constant factors are rounded once.  Against fp64, root mean square of energies
 // / gradients, rows kernel -> this one, relative: d = 128, 128 stacks 3.7e-7 / 3.1e-7 -> 2.3e-7 / 2.2e-7, two transforms, 32 stacks
 // 3.1e-7 / 3.1e-7 -> 2.4e-7 / 2.4e-7; with arguments twice as large and falling components 4.7e-7 / 4.6e-7 -> 4.2e-7 / 4.3e-7 at most.
+// (The accumulators that start from the bias round it with every partial sum: reduced to a half revolution only, energies and gradients
+// of 512 rows were 2.7e-7 / 2.5e-7 where the fma had given 2.5e-7 / 2.3e-7, three draws; to a quarter 2.4e-7 / 2.3e-7.)
 // Power-of-two scales keep everything in fp16's range: x per atom
 // (sum |x| to [2^13, 2^14), which bounds every partial transform), alpha per call.  With one transform x has a fixed scale, whose
 // inverse is in the H_16 blocks, so that the accumulators hold revolutions and can start from the bias behind the inverse of the
@@ -71,9 +73,11 @@ __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h
 struct Forms {
     half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal
     float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
-    float* bias;          // [ne][S][d] in revolutions, -1/2 to 1/2 (from fp64: the smaller the argument, the less its rounding); with one
-                          // transform what its accumulators start from, of which the stages over the block index make that
-    float* alpha;         // [S][d] 2^k with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them), then 2^-k
+    // Bias in revolutions, reduced to a quarter either way in fp64: the smaller the argument, the less its rounding.  What is taken off is
+    // whole halves, and the sign that an odd number of them gives cosine and sine is alpha's.
+    float* bias;          // [ne][S][d]; with one transform what its accumulators start from, of which the stages over the block index make that
+    float* alpha;         // [ne][S][d] +-2^k alpha with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them),
+                          // then 2^-k
     int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
 };
 
@@ -88,7 +92,7 @@ __device__ __forceinline__ float workgroup_max(float m, float* wmax) {
     return m;
 }
 
-// workgroup 0: alpha; then one per (element, stack).  bias and alpha may be null: the images and bounds alone.  The blocks are +-factor.
+// a workgroup per (element, stack).  bias and alpha may both be null: the images and bounds alone.  The blocks are +-factor.
 constexpr int PREP_THREADS = 512;
 template <int D, int T>
 __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float* __restrict__ Dmat, const float* __restrict__ bias,
@@ -97,20 +101,7 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     __shared__ float wmax[PREP_THREADS / 64];
     __shared__ float h[D];
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0) {
-        if (alpha == nullptr) return;
-        float m = 0.0f;
-#pragma unroll 8
-        for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
-        m = workgroup_max(m, wmax);
-        const int k = max(scale_exponent(m) - log2nb<NB>(), -126);
-        const float sc = pow2i(k);
-#pragma unroll 8
-        for (int t = tid; t < S * D; t += PREP_THREADS) f.alpha[t] = alpha[t] * sc;
-        if (tid == 0) f.alpha[(size_t)S * D] = pow2i(-k);
-        return;
-    }
-    const int e = (blockIdx.x - 1) / S, s = blockIdx.x - 1 - e * S;
+    const int e = blockIdx.x / S, s = blockIdx.x - e * S;
     bool unfit = false;
 #pragma unroll
     for (int m = 0; m < T; ++m) {
@@ -148,20 +139,32 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     }
     const bool any_unfit = __syncthreads_or(unfit);
     if (bias != nullptr) {
-        const size_t at = ((size_t)e * S + s) * D;
-        auto revolutions = [&](int t) {
-            const double r = (double)bias[at + t] * 0.15915494309189533577;
-            return r - rint(r);
-        };
-        for (int t = tid; t < D; t += PREP_THREADS) {
-            double v = revolutions(t);
+        __shared__ double rev[D];
+        const size_t at = ((size_t)e * S + s) * D + tid;
+        const float mine = tid < D ? alpha[s * D + tid] : 0.0f;
+        bool odd = false;
+        if (tid < D) {
+            const double b = (double)bias[at], n = rint(b * 0.31830988618379067154);
+            odd = n != 2.0 * rint(0.5 * n);
+            rev[tid] = fma(b, 0.15915494309189533577, -0.5 * n);
+        }
+        float m = 0.0f;                  // the call's scale of alpha: every workgroup finds the same value
+#pragma unroll 8
+        for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
+        m = workgroup_max(m, wmax);      // (its barriers are also those between the writes of rev and the reads)
+        const int k = max(scale_exponent(m) - log2nb<NB>(), -126);
+        if (tid < D) {
+            double v = rev[tid];
             if constexpr (T == 1) {      // the stages over the block index are their own inverse but for the factor NB
                 v = 0.0;
-                for (int b = 0; b < NB; ++b) v += h16_negative(t >> 4, b) ? -revolutions(16 * b + (t & 15)) : revolutions(16 * b + (t & 15));
-                v /= NB;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) v += h16_negative(tid >> 4, b) ? -rev[16 * b + (tid & 15)] : rev[16 * b + (tid & 15)];
+                v *= 1.0 / NB;
             }
-            f.bias[at + t] = (float)v;
+            f.bias[at] = (float)v;
+            f.alpha[at] = mine * (odd ? -pow2i(k) : pow2i(k));
         }
+        if (blockIdx.x == 0 && tid == 0) f.alpha[(size_t)gridDim.x * D] = pow2i(-k);
     }
     if (tid == 0) f.largest[(size_t)e * S + s] = any_unfit ? HUGE_VALF : largest;
 }
@@ -293,6 +296,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const float* Dt = Dmat + (size_t)type * T * S * D;
         const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
         const float* bt = bias_rev + (size_t)type * S * D;
+        const float* at = alpha_scaled + (size_t)type * S * D;
 
         // stack s into a buffer: direct global-to-LDS loads of 16 bytes per lane, in 1 KiB blocks shared out over the wavefronts
         auto load16 = [&](const void* src, void* dst) {
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             for (int u = 0; u < T * NB; u += SM_WAVES) load16(src + (u + wave) * 1024 + lane16, dst + (u + wave) * 1024);
             if (lane < D / 4) {      // a row of D floats
                 if (wave == 0) load16(bt + (size_t)s * D + lane * 4, to.bias);
-                if (wave == 1) load16(alpha_scaled + (size_t)s * D + lane * 4, to.alpha);
+                if (wave == 1) load16(at + (size_t)s * D + lane * 4, to.alpha);
                 if constexpr (WITH_GRAD) {
                     if (wave == 2) load16(Dt + (size_t)s * D + lane * 4, to.diag);
                     if (T == 2 && wave == 3) load16(Dt + ((size_t)S + s) * D + lane * 4, to.diag + (T - 1) * D);
@@ -474,7 +478,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         if (WITH_GRAD || __builtin_expect(__syncthreads_or(wide), 0)) all_rounds(std::false_type{});
         else all_rounds(std::true_type{});
 
-        const float inv_alpha = alpha_scaled[(size_t)S * D];
+        const float inv_alpha = alpha_scaled[(size_t)ne * S * D];
         energy += __shfl_xor(energy, 16, 64);
         energy += __shfl_xor(energy, 32, 64);
         if (!aok) continue;
@@ -564,7 +568,7 @@ static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, i
     f.largest = (float*)take((size_t)ne * S * sizeof(float));
     f.unfit = (int*)take(sizeof(int));
     f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
-    f.alpha = (float*)take(((size_t)S * d + 1) * sizeof(float));
+    f.alpha = (float*)take(((size_t)ne * S * d + 1) * sizeof(float));
     parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float));
     return at;
 }
@@ -593,7 +597,7 @@ extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int wit
 
 static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, float factor,
                            const Forms& f, hipStream_t st) {
-    const dim3 grid(ne * S + 1), block(PREP_THREADS);
+    const dim3 grid(ne * S), block(PREP_THREADS);
     if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else if (T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
