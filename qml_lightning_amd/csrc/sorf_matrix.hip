@@ -169,6 +169,18 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     if (tid == 0) f.largest[(size_t)e * S + s] = any_unfit ? HUGE_VALF : largest;
 }
 
+// Which wavefront of a SIMD issues first.  A plain vector instruction takes the issue two clocks, a conversion four, a sine or cosine
+// eight, and a matrix instruction seven beside either of the latter and all of its sixteen beside plain ones: so the wavefronts whose
+// phase has the slow instructions go ahead, and the others fill in with their additions.  Left to themselves they run into the same
+// phase together.  86016 atoms, 128 components, 128 stacks with the gradient: all equal 624 us; the sines and cosines ahead 581; these and the
+// splits with their matrix instructions 548; the stages between the two above the first ones 539; the adjoint's end above them too,
+// and the matrix instructions above the sines 526.  Energies only, 131072 atoms, 64 stacks 226 -> 213; two transforms, 32 stacks, 33000
+// atoms 143 -> 122 (127 without the forward's second splits).  The first matrix instructions, whose operands come from LDS, gained nothing.
+template <int P>
+__device__ __forceinline__ void precedence() {
+    __builtin_amdgcn_s_setprio(P);
+}
+
 // butterflies over the block index
 template <int NB>
 __device__ __forceinline__ void block_stages(f4_t (&v)[NB]) {
@@ -401,9 +413,11 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
                 for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[b * 64], xop[b], zero, 0, 0, 0);
                 block_stages<NB>(v);
+                precedence<2>();
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
                     v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[(NB + b) * 64], split4(v[b]), zero, 0, 0, 0);
+                precedence<0>();
                 block_stages<NB>(v);
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
@@ -421,6 +435,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                         v[b][r] = fabsf(u) > UMAX ? u - rintf(u) : u;      // exact
                     }
             }
+            precedence<2>();
             float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
@@ -433,27 +448,35 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 }
             }
             energy += part;
-            if constexpr (WITH_GRAD) {
+            if constexpr (!WITH_GRAD) {
+                precedence<0>();
+            } else {
+                precedence<1>();
                 block_stages<NB>(v);
+                precedence<3>();
                 if constexpr (T == 2) {
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
                         const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + D + 16 * b + 4 * q);
                         v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hback, split4(v[b]), zero, 0, 0, 0) * dv;
                     }
+                    precedence<1>();
                     block_stages<NB>(v);
+                    precedence<3>();
                 }
                 // summed from zero and added by the vector unit: the matrix instruction aligns its products to the
                 // accumulator it is given, and against a sum over many stacks their low bits would be cut off
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
                     v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hop, split4(v[b]), zero, 0, 0, 0);
+                precedence<1>();
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
                     const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + 16 * b + 4 * q);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(v[b][r], dv[r], acc[b][r]);
                 }
+                precedence<0>();
             }
         };
         auto round = [&](int s, const Buffer (&cur)[SPB], Buffer (&other)[SPB], auto narrow) __attribute__((always_inline)) {
