@@ -433,7 +433,7 @@ int qmll_sorf_energy_parts(const float* x, const int* type_offsets, const int* s
                            const float* alpha, const float* bias_absmax, int A, int ne, int d, int S, int T, float normalisation,
                            int nparts, float* e_parts, int nslots, float* gx_parts, qmll_stream_t stream);
 
-/* qmll_sorf_energy_sorted on the half-precision matrix cores (large batches; d = 64 or 128, T = 1 or 2; diagonals of +-1:
+/* qmll_sorf_energy_sorted on the half-precision matrix cores (large batches; d = 64, 128 or 256, T = 1 or 2; diagonals of +-1:
  * where the device finds others the call runs as qmll_sorf_energy_sorted does).  x, D, work and gx 16-byte aligned.
  * work: device memory of qmll_sorf_matrix_workspace_bytes (0: no kernel takes the shape), for this call alone; the signs in
  * the form that is multiplied with, bias in revolutions and alpha behind a power of two are made there by every call.  fp32
@@ -444,7 +444,7 @@ int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad);   
 int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, const int* sorted_slots, const float* D, const float* bias,
                             const float* alpha, int A, int ne, int d, int S, int T, float normalisation, void* work,
                             size_t work_bytes, float* e_slots, float* gx, qmll_stream_t stream);
-/* The first part of those forms alone, for whoever wants to look at them: the H_16 blocks behind the signs of D, then a
+/* The first part of those forms alone (d = 64 or 128), for whoever wants to look at them: the H_16 blocks behind the signs of D, then a
  * float per (element, stack): the largest entry of H D_1 H (T = 1: 1), infinite where a diagonal is not +-1. */
 size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d);
 int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void* out, size_t out_bytes, qmll_stream_t stream);

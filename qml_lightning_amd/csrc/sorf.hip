@@ -1833,7 +1833,8 @@ int qmll_sorf_rows_if(const float* x, const int* type_offsets, const int* sorted
         else by_transforms(log2d, std::false_type{});
     };
     if (d == 64) by_grad(std::integral_constant<int, 6>{});
-    else by_grad(std::integral_constant<int, 7>{});
+    else if (d == 128) by_grad(std::integral_constant<int, 7>{});
+    else by_grad(std::integral_constant<int, 8>{});
     QMLL_CHECK_LAUNCH("qmll_sorf_energy_matrix");
     return QMLL_OK;
 }

@@ -1,5 +1,5 @@
 // Fused SORF energy and gradient on element-sorted rows (the contract of qmll_sorf_energy_sorted) with the in-row part of
-// the Walsh-Hadamard transforms on the half-precision matrix cores, for d = 64 or 128 and one or two transforms per stack.
+// the Walsh-Hadamard transforms on the half-precision matrix cores, for d = 64, 128 or 256 and one or two transforms per stack.
 //
 // H_d = H_{d/16} (x) H_16.  A wavefront carries 16 atoms through a stack.  v_mfma_f32_16x16x32_f16 multiplies the
 // +-1 block H_16 (exact in fp16) with a 16 x 16 block of the vectors (index within the block x atom), each fp32 entry
@@ -39,8 +39,14 @@
 // part each, which sorf_parts_kernel adds in order.
 // Measured with the gradient / energies only, rows kernel -> this call, at d = 128, 128 stacks: 86016 atoms 764 -> 653 us / 456 -> 305;
 // 24000 atoms 222 -> 214 / 133 -> 108; two transforms, 32 stacks, 33000 atoms 148 -> 143 / 78 -> 75, 86016 atoms 369 -> 314 / 194 -> 148;
-// d = 64, 128 stacks, 86016 atoms 360 -> 309 / 230 -> 147.  Of that 5 us go to the forms and 3 to 4 to the launch behind.  (At d = 256 the
-// registers leave two wavefronts per SIMD and it is no faster: 880 -> 890 us, so the rows kernel stays.)
+// d = 64, 128 stacks, 86016 atoms 360 -> 309 / 230 -> 147.  Of that 5 us go to the forms and 3 to 4 to the launch behind.  (These
+// are from before the precedence below and the accumulators that start from the bias.)
+//
+// d = 256: with all of 16 vectors the registers leave two wavefronts per SIMD, which take 890 us for 41796 atoms, 128 stacks where the rows
+// kernel takes 822.  So the sixteen columns are eight atoms times the two halves of their vectors: the registers, and three wavefronts per SIMD, are
+// those of d = 128, and the eighth index bit is one more stage between lanes eight apart, an addition that reads its partner through the DPP
+// network.  The halves have diagonals of their own and share the H_16 block, which is plain and stays in registers: the signs are flipped in the
+// split operand, an exclusive or per register.  622 us; energies only 447 -> 295; two transforms, 32 stacks 596 -> 322 / 207 -> 169.
 #include <algorithm>
 #include <type_traits>
 
@@ -49,9 +55,12 @@
 namespace {
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef int int4_t __attribute__((ext_vector_type(4)));
 
 constexpr int SM_WAVES = 4;                  // wavefronts per workgroup
-constexpr int SM_ATOMS = 16 * SM_WAVES;
+// d = 256: the sixteen columns of a wavefront's operands are eight atoms times the two halves of their vectors
+__host__ __device__ constexpr int column_halves(int d) { return d == 256 ? 2 : 1; }
+__host__ __device__ constexpr int tile_atoms(int d) { return 16 * SM_WAVES / column_halves(d); }
 constexpr float INV2PI = 0.15915494309189535f;
 constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are taken off the sine argument first
 // One transform: x (in revolutions) goes times 2^SM_EXP into its two fp16 parts: an entry is then off by 2^-33 at most beside its 23
@@ -59,11 +68,21 @@ constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are ta
 constexpr int SM_EXP = 8;
 
 // stacks per buffer: one barrier for so many (and at least 3 workgroups in LDS)
-constexpr int stacks_per_round(int d, int T) { return d * T <= 128 ? 2 : 1; }
+constexpr int stacks_per_round(int d, int T) { return d * T <= 128 || d == 256 ? 2 : 1; }
 constexpr int SM_CUS = 256;
 
-template <int NB>
-constexpr int log2nb() { return NB == 4 ? 2 : 3; }
+// index bits of a vector that are not in its 16-point blocks
+template <int D>
+constexpr int block_bits() { return D == 64 ? 2 : D == 128 ? 3 : 4; }
+
+// where entry k of a vector stands in the rows that a stack reads from LDS: at d = 256 the two halves of a block side by side, as the
+// lanes of a wavefront read them at the same time
+template <int D>
+__device__ __forceinline__ int row_place(int k) {
+    return D == 256 ? (k & 0x70) << 1 | (k >> 7) << 4 | (k & 15) : k;
+}
+// bytes per (element, stack) of the forms that the first operands come from
+__host__ __device__ constexpr int image_bytes(int d, int T) { return d == 256 ? T * 1536 : T * d * 64; }
 
 // one 16-point block operand: half t of lane (i, q) is sign * H_16[i][4q + t % 4]
 __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h) & 1; }
@@ -71,11 +90,13 @@ __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h
 // What a launch needs of the model beside its tensors.  Made by every call (sorf_prepare_kernel, 4 us of 150 and more): nothing
 // is kept that a write to the tensors could leave behind, and no other stream or captured graph has to wait for it.
 struct Forms {
-    half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal
+    half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal.  d = 256: [ne][S], of the
+                          // diagonals [T][256] in the order of row_place, then the sign bits of the halves [T][4][half, lane / 16][16 bytes]
     float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
     // Bias in revolutions, reduced to a quarter either way in fp64: the smaller the argument, the less its rounding.  What is taken off is
     // whole halves, and the sign that an odd number of them gives cosine and sine is alpha's.
-    float* bias;          // [ne][S][d]; with one transform what its accumulators start from, of which the stages over the block index make that
+    float* bias;          // [ne][S][d]; with one transform what its accumulators start from, of which the stages over the block index make that;
+                          // this and alpha in the order of row_place
     float* alpha;         // [ne][S][d] +-2^k alpha with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them),
                           // then 2^-k
     int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
@@ -98,6 +119,7 @@ template <int D, int T>
 __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float* __restrict__ Dmat, const float* __restrict__ bias,
                                                                     const float* __restrict__ alpha, int S, float factor, Forms f) {
     constexpr int NB = D / 16;
+    constexpr bool HALVES = D == 256;
     __shared__ float wmax[PREP_THREADS / 64];
     __shared__ float h[D];
     const int tid = threadIdx.x;
@@ -106,6 +128,20 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
 #pragma unroll
     for (int m = 0; m < T; ++m) {
         const float* row = Dmat + (((size_t)e * T + m) * S + s) * D;
+        if constexpr (HALVES) {
+            char* image = (char*)f.images + ((size_t)e * S + s) * image_bytes(D, T);
+            if (tid < D) {
+                // the second half of a transform's result has its sign pending, which the next diagonal takes
+                const float sd = row[tid], v = m > 0 && tid >= D / 2 ? -sd : sd;
+                unfit |= !(fabsf(sd) == 1.0f);
+                reinterpret_cast<float*>(image)[m * D + row_place<D>(tid)] = v;
+                // blocks 2 j and 2 j + 1 of a half next to each other, four sign bits of 16 each
+                const int b = (tid >> 4) & 7, q = (tid >> 2) & 3;
+                reinterpret_cast<unsigned short*>(image + T * D * 4 + m * 512)[((b >> 1) * 8 + (tid >> 7) * 4 + q) * 8 + (b & 1) * 4 + (tid & 3)] =
+                    v < 0.0f ? 0x8000 : 0;
+            }
+            continue;
+        }
         half8_t* dst = f.images + (((size_t)e * S + s) * T + m) * NB * 64;
         for (int t = tid; t < NB * 64; t += PREP_THREADS) {
             const int b = t >> 6, lane = t & 63, i = lane & 15, q = lane >> 4;
@@ -140,7 +176,7 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
     const bool any_unfit = __syncthreads_or(unfit);
     if (bias != nullptr) {
         __shared__ double rev[D];
-        const size_t at = ((size_t)e * S + s) * D + tid;
+        const size_t at = ((size_t)e * S + s) * D + tid, to = ((size_t)e * S + s) * D + row_place<D>(tid & (D - 1));
         const float mine = tid < D ? alpha[s * D + tid] : 0.0f;
         bool odd = false;
         if (tid < D) {
@@ -152,7 +188,7 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
 #pragma unroll 8
         for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
         m = workgroup_max(m, wmax);      // (its barriers are also those between the writes of rev and the reads)
-        const int k = max(scale_exponent(m) - log2nb<NB>(), -126);
+        const int k = max(scale_exponent(m) - block_bits<D>(), -126);
         if (tid < D) {
             double v = rev[tid];
             if constexpr (T == 1) {      // the stages over the block index are their own inverse but for the factor NB
@@ -160,9 +196,11 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
 #pragma unroll
                 for (int b = 0; b < NB; ++b) v += h16_negative(tid >> 4, b) ? -rev[16 * b + (tid & 15)] : rev[16 * b + (tid & 15)];
                 v *= 1.0 / NB;
+            } else if (HALVES && tid >= D / 2) {
+                v = -v;                  // (the sign that is pending)
             }
-            f.bias[at] = (float)v;
-            f.alpha[at] = mine * (odd ? -pow2i(k) : pow2i(k));
+            f.bias[to] = (float)v;
+            f.alpha[to] = mine * (odd ? -pow2i(k) : pow2i(k));
         }
         if (blockIdx.x == 0 && tid == 0) f.alpha[(size_t)gridDim.x * D] = pow2i(-k);
     }
@@ -200,6 +238,32 @@ __device__ __forceinline__ void block_stages(f4_t (&v)[NB]) {
     }
 }
 
+// The butterflies between the two halves of a vector, which lie eight lanes apart: v + c * partner, one instruction.  With c = 1 in the
+// first half and -1 in the second the second comes out with the other sign, which stays pending; with -c it is the transposed stage.
+// (two registers sets behind one pair of wait states, which the writes before may need)
+#define QMLL_HALF_STAGE8(x, y, c)                                                                                                   \
+    asm("s_nop 1\n\t"                                                                                                               \
+        "v_fmac_f32_dpp %0, %0, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %1, %1, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %2, %2, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %3, %3, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %4, %4, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %5, %5, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %6, %6, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %7, %7, %8 row_ror:8 row_mask:0xf bank_mask:0xf"                                                            \
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3])                            \
+        : "v"(c))
+template <int NB>
+__device__ __forceinline__ void half_stage(f4_t (&v)[NB], float c) {
+#pragma unroll
+    for (int b = 0; b < NB; b += 2) {
+        float x[4] = {v[b][0], v[b][1], v[b][2], v[b][3]}, y[4] = {v[b + 1][0], v[b + 1][1], v[b + 1][2], v[b + 1][3]};
+        QMLL_HALF_STAGE8(x, y, c);
+        v[b] = (f4_t){x[0], x[1], x[2], x[3]};
+        v[b + 1] = (f4_t){y[0], y[1], y[2], y[3]};
+    }
+}
+
 // four values as the lane's eight k entries of an operand: high parts, then low parts, both rounded to nearest
 __device__ __forceinline__ half8_t split4(f4_t v) {
     half2_t h0, h1, l0, l1;
@@ -216,21 +280,30 @@ struct StackBuffer {      // what a stack needs, in LDS
     float bias[D];        // in revolutions (see Forms)
     float alpha[D];       // scaled
 };
+template <int T>
+struct StackBuffer<256, T> {      // all of it in the order of row_place
+    float diag[T * 256];
+    int4_t signs[T * 32];
+    float bias[256];
+    float alpha[256];
+};
 
-// Tiles of 64 atoms of one element; a share of the launch is a range of (tile, round of SPB stacks) units, tile after tile.
+// Tiles of 64 (d = 256: 32) atoms of one element; a share of the launch is a range of (tile, round of SPB stacks) units, tile after tile.
+template <int ATOMS>
 __device__ __forceinline__ int tile_count(const int* __restrict__ type_offsets, int ne) {
     int n = 0;
-    for (int t = 0; t < ne; ++t) n += (type_offsets[t + 1] - type_offsets[t] + SM_ATOMS - 1) / SM_ATOMS;
+    for (int t = 0; t < ne; ++t) n += (type_offsets[t + 1] - type_offsets[t] + ATOMS - 1) / ATOMS;
     return n;
 }
+template <int ATOMS>
 __device__ __forceinline__ void find_tile(const int* __restrict__ type_offsets, int ne, int tile, int& type, int& row0, int& rows) {
     type = row0 = rows = 0;
     for (int t = 0; t < ne; ++t) {
-        const int o0 = type_offsets[t], o1 = type_offsets[t + 1], nt = (o1 - o0 + SM_ATOMS - 1) / SM_ATOMS;
+        const int o0 = type_offsets[t], o1 = type_offsets[t + 1], nt = (o1 - o0 + ATOMS - 1) / ATOMS;
         if (tile < nt) {
             type = t;
-            row0 = o0 + tile * SM_ATOMS;
-            rows = min(SM_ATOMS, o1 - row0);
+            row0 = o0 + tile * ATOMS;
+            rows = min(ATOMS, o1 - row0);
             return;
         }
         tile -= nt;
@@ -257,7 +330,7 @@ __device__ __forceinline__ int share_begin(int g, int nshares, int slots, int nt
     return g - whole >= used ? units : units - left + (int)((long long)left * (g - whole) / used);
 }
 template <int D, bool WITH_GRAD>
-constexpr int RESIDENT = (D == 128 && WITH_GRAD ? 3 : 4) * SM_CUS;
+constexpr int RESIDENT = (D >= 128 && WITH_GRAD ? 3 : 4) * SM_CUS;
 
 // (at least two wavefronts per SIMD: with up to 256 registers the compiler lets the matrix instructions write vector
 // registers directly; asked for fewer it goes through accumulator registers, a move per value)
@@ -267,7 +340,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
     const float* __restrict__ Dmat, const half8_t* __restrict__ images, const float* __restrict__ bias_rev,
     const float* __restrict__ alpha_scaled, const float* __restrict__ bounds, int ne, int A, int S, int nshares, float xs, float gscale,
     float normf, float* __restrict__ parts, float* __restrict__ e_slots, float* __restrict__ gx) {
-    constexpr int NB = D / 16;
+    constexpr int HALVES = column_halves(D), NB = D / (16 * HALVES), WAVE_ATOMS = 16 / HALVES, ATOMS = tile_atoms(D);
     using Buffer = StackBuffer<D, T>;
     // two buffers as two arrays: the compiler then knows that loads into one do not touch what is read from the other
     constexpr int SPB = stacks_per_round(D, T);
@@ -276,9 +349,11 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4;
+    const int atom = col & (WAVE_ATOMS - 1), half = HALVES == 2 ? col >> 3 : 0;
+    const int at4 = 16 * half + 4 * q;                                  // this lane's entries of a block, in the order of row_place
     const int rounds = (S + SPB - 1) / SPB;
 
-    const int ntiles = tile_count(type_offsets, ne);
+    const int ntiles = tile_count<ATOMS>(type_offsets, ne);
     if ((int)blockIdx.x >= nshares) {
         // a workgroup beyond the shares: its part of the gradient rows of atoms of unknown elements, which are zero
         if constexpr (WITH_GRAD) {
@@ -294,7 +369,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
     for (int u = ubeg; u < uend;) {
         const int tile = u / rounds, r0 = u - tile * rounds, r1 = min(rounds, r0 + uend - u);
         int type, row0, rows;
-        find_tile(type_offsets, ne, tile, type, row0, rows);
+        find_tile<ATOMS>(type_offsets, ne, tile, type, row0, rows);
         const bool first_piece = r0 == 0;                               // else a part: only a share's first tile can be one
         if (u != ubeg) __syncthreads();                                 // the buffers of the tile before are free
         u += r1 - r0;
@@ -306,7 +381,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         if (largest == HUGE_VALF) continue;                             // not +-1: the rows kernel behind this one writes all
 
         const float* Dt = Dmat + (size_t)type * T * S * D;
-        const unsigned char* it = reinterpret_cast<const unsigned char*>(images + (size_t)type * S * T * NB * 64);
+        const unsigned char* it = reinterpret_cast<const unsigned char*>(images) + (size_t)type * S * image_bytes(D, T);
         const float* bt = bias_rev + (size_t)type * S * D;
         const float* at = alpha_scaled + (size_t)type * S * D;
 
@@ -317,7 +392,15 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         };
         const unsigned lane16 = (unsigned)lane * 16u;
         auto fetch = [&](int s, Buffer& to) {
-            const unsigned char* src = it + (size_t)s * (T * NB * 1024);
+            const unsigned char* src = it + (size_t)s * image_bytes(D, T);
+            if constexpr (HALVES == 2) {      // a row of 256 floats is one such load
+                if (wave == 0) load16(bt + (size_t)s * D + lane * 4, to.bias);
+                if (wave == 1) load16(at + (size_t)s * D + lane * 4, to.alpha);
+                if (WITH_GRAD && wave == 2) load16(src + lane16, to.diag);
+                if (WITH_GRAD && T == 2 && wave == 0) load16(src + 1024 + lane16, to.diag + (T - 1) * D);
+                if (wave == 3 && lane < 32 * T) load16(src + T * 1024 + lane16, to.signs);
+                return;
+            }
             unsigned char* dst = reinterpret_cast<unsigned char*>(to.signs);
 #pragma unroll
             for (int u = 0; u < T * NB; u += SM_WAVES) load16(src + (u + wave) * 1024 + lane16, dst + (u + wave) * 1024);
@@ -337,16 +420,16 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         };
         fetch_all(s0, buf0);
 
-        const int first = 16 * wave;                         // of this wavefront's atoms
+        const int first = WAVE_ATOMS * wave;                 // of this wavefront's atoms
         const bool live = first < rows;                      // of the whole wavefront
-        const bool aok = first + col < rows;
+        const bool aok = first + atom < rows;
 
         // x in revolutions, split behind a power of two
         half8_t xop[NB];
         float inv, to_scale;
         bool wide;
         {
-            const float* xr = x + (size_t)(row0 + (aok ? first + col : 0)) * D + 4 * q;
+            const float* xr = x + (size_t)(row0 + (aok ? first + atom : 0)) * D + D / 2 * half + 4 * q;
             f4_t xv[NB];
             float sum = 0.0f;
 #pragma unroll
@@ -360,6 +443,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             }
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
+            if constexpr (HALVES == 2) sum += __shfl_xor(sum, 8, 64);
             // Every argument is at most sum |x|, times the largest entry of H D_1 H for a second transform, + |bias|: where that
             // stays below UMAX no stack looks at its arguments.  One transform: below the second limit all atoms share one power of
             // two, whose inverse is in the H_16 blocks.
@@ -377,14 +461,18 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             }
         }
         // the plain H_16 block, and the one behind the second transform's adjoint, scaled back into fp16's range
-        constexpr int BACK = 4 + log2nb<NB>() - 1;
-        half8_t hop, hback;
+        constexpr int BACK = 4 + block_bits<D>() - 1;
+        half8_t hop, hback, hfirst;
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const bool neg = h16_negative(col, 4 * q + (t & 3));
             hop[t] = neg ? (_Float16)-1.0f : (_Float16)1.0f;
             hback[t] = neg ? (_Float16)(-1.0f / (1 << BACK)) : (_Float16)(1.0f / (1 << BACK));
+            hfirst[t] = neg ? (_Float16)(-1.0f / (1 << SM_EXP)) : (_Float16)(1.0f / (1 << SM_EXP));
         }
+        const float cross = half ? -1.0f : 1.0f;
+        float uncross = -cross;
+        asm("" : "+v"(uncross));                             // kept in a register
         const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
         f4_t acc[NB];
         float energy = 0.0f;
@@ -393,9 +481,38 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
 
         auto stack = [&](const Buffer& B, auto narrow) __attribute__((always_inline)) {
             const bool look = !decltype(narrow)::value && wide;
-            const half8_t* signs = B.signs + lane;
             f4_t v[NB];
-            auto bias = [&](int b) { return *reinterpret_cast<const f4_t*>(B.bias + 16 * b + 4 * q); };
+            // four entries of block b from a row
+            auto entries = [&](const float* row, int b) { return *reinterpret_cast<const f4_t*>(row + 16 * HALVES * b + at4); };
+            auto bias = [&](int b) { return entries(B.bias, b); };
+            // transform m's 16-point blocks of `from` (split) behind its diagonal
+            auto blocks = [&](int m, auto from, auto start) __attribute__((always_inline)) {
+                if constexpr (HALVES == 2) {
+#pragma unroll
+                    for (int j = 0; j < NB / 2; ++j) {
+                        const int4_t sg = B.signs[m * 32 + j * 8 + half * 4 + q];
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const int b = 2 * j + k;
+                            const int4_t flip = {sg[2 * k], sg[2 * k + 1], sg[2 * k], sg[2 * k + 1]};
+                            const half8_t op = __builtin_bit_cast(half8_t, __builtin_bit_cast(int4_t, from(b)) ^ flip);
+                            v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(T == 1 ? hfirst : hop, op, start(b), 0, 0, 0);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(B.signs[(m * NB + b) * 64 + lane], from(b), start(b), 0, 0, 0);
+                }
+            };
+            auto stages = [&] {
+                block_stages<NB>(v);
+                if constexpr (HALVES == 2) half_stage<NB>(v, cross);
+            };
+            auto transposed_stages = [&] {
+                block_stages<NB>(v);
+                if constexpr (HALVES == 2) half_stage<NB>(v, uncross);
+            };
             if constexpr (T == 1) {
                 // The accumulators start not from zero, so that the register part's stages add the bias on the way (an instruction
                 // per value less, and one rounding less).
@@ -406,19 +523,15 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
                     for (int b = 0; b < NB; ++b) c[b] *= to_scale;
                 }
-#pragma unroll
-                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[b * 64], xop[b], c[b], 0, 0, 0);
-                block_stages<NB>(v);
+                blocks(0, [&](int b) { return xop[b]; }, [&](int b) { return c[b]; });
+                stages();
             } else {
-#pragma unroll
-                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[b * 64], xop[b], zero, 0, 0, 0);
-                block_stages<NB>(v);
+                blocks(0, [&](int b) { return xop[b]; }, [&](int) { return zero; });
+                stages();
                 precedence<2>();
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(signs[(NB + b) * 64], split4(v[b]), zero, 0, 0, 0);
+                blocks(1, [&](int b) { return split4(v[b]); }, [&](int) { return zero; });
                 precedence<0>();
-                block_stages<NB>(v);
+                stages();
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
                     const f4_t bv = bias(b);
@@ -439,7 +552,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             float part = 0.0f;                               // of this stack: the running sum takes one rounding per stack
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const f4_t av = *reinterpret_cast<const f4_t*>(B.alpha + 16 * b + 4 * q);
+                const f4_t av = entries(B.alpha, b);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float u = v[b][r];
@@ -452,16 +565,16 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 precedence<0>();
             } else {
                 precedence<1>();
-                block_stages<NB>(v);
+                transposed_stages();
                 precedence<3>();
                 if constexpr (T == 2) {
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
-                        const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + D + 16 * b + 4 * q);
+                        const f4_t dv = entries(B.diag + D, b);
                         v[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hback, split4(v[b]), zero, 0, 0, 0) * dv;
                     }
                     precedence<1>();
-                    block_stages<NB>(v);
+                    transposed_stages();
                     precedence<3>();
                 }
                 // summed from zero and added by the vector unit: the matrix instruction aligns its products to the
@@ -472,7 +585,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 precedence<1>();
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
-                    const f4_t dv = *reinterpret_cast<const f4_t*>(B.diag + 16 * b + 4 * q);
+                    const f4_t dv = entries(B.diag, b);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(v[b][r], dv[r], acc[b][r]);
                 }
@@ -504,17 +617,18 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const float inv_alpha = alpha_scaled[(size_t)ne * S * D];
         energy += __shfl_xor(energy, 16, 64);
         energy += __shfl_xor(energy, 32, 64);
+        if constexpr (HALVES == 2) energy += __shfl_xor(energy, 8, 64);
         if (!aok) continue;
-        const int in_tile = first + col;
-        if (q == 0) {
+        const int in_tile = first + atom;
+        if (q == 0 && half == 0) {
             const float e = energy * inv_alpha * normf;
             if (first_piece) e_slots[out_index[row0 + in_tile]] = e;
-            else parts[(size_t)blockIdx.x * SM_ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
+            else parts[(size_t)blockIdx.x * ATOMS * (WITH_GRAD ? D + 1 : 1) + in_tile] = e;
         }
         if constexpr (WITH_GRAD) {
             const float gs = gscale * inv_alpha * (T == 2 ? (float)(1 << BACK) : 1.0f);
-            float* to = first_piece ? gx + (size_t)row0 * D : parts + (size_t)blockIdx.x * SM_ATOMS * (D + 1) + SM_ATOMS;
-            float* gr = to + (size_t)in_tile * D + 4 * q;
+            float* to = first_piece ? gx + (size_t)row0 * D : parts + (size_t)blockIdx.x * ATOMS * (D + 1) + ATOMS;
+            float* gr = to + (size_t)in_tile * D + D / 2 * half + 4 * q;
 #pragma unroll
             for (int b = 0; b < NB; ++b) *reinterpret_cast<f4_t*>(gr + 16 * b) = acc[b] * gs;
         }
@@ -527,7 +641,8 @@ template <int D, bool WITH_GRAD>
 __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__ type_offsets, const int* __restrict__ out_index, int ne,
                                                          int S, int rounds, const float* __restrict__ parts, Forms f,
                                                          float* __restrict__ e_slots, float* __restrict__ gx) {
-    constexpr size_t SLOT = SM_ATOMS * (WITH_GRAD ? D + 1 : 1);
+    constexpr int ATOMS = tile_atoms(D);
+    constexpr size_t SLOT = ATOMS * (WITH_GRAD ? D + 1 : 1);
     const int g = blockIdx.x, nshares = (int)gridDim.x - 1;
     if (g == nshares) {
         bool unfit = false;
@@ -536,7 +651,7 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
         if (threadIdx.x == 0) *f.unfit = unfit;
         return;
     }
-    const int ntiles = tile_count(type_offsets, ne);
+    const int ntiles = tile_count<ATOMS>(type_offsets, ne);
     constexpr int slots = RESIDENT<D, WITH_GRAD>;
     const int ubeg = share_begin(g, nshares, slots, ntiles, rounds), uend = share_begin(g + 1, nshares, slots, ntiles, rounds);
     if (ubeg == uend) return;
@@ -545,7 +660,7 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
     int last = g + 1;                                    // the share in which the tile ends
     while (share_begin(last + 1, nshares, slots, ntiles, rounds) < tend) ++last;
     int type, row0, rows;
-    find_tile(type_offsets, ne, tile, type, row0, rows);
+    find_tile<ATOMS>(type_offsets, ne, tile, type, row0, rows);
     const float* next = parts + (size_t)(g + 1) * SLOT;
     const int nparts = last - g;
     for (int t = threadIdx.x; t < rows; t += 256) {
@@ -558,7 +673,7 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
         for (int t = threadIdx.x; t < rows * (D / 4); t += 256) {
             f4_t* to = reinterpret_cast<f4_t*>(gx + (size_t)row0 * D) + t;
             f4_t v = *to;
-            for (int b = 0; b < nparts; ++b) v += *reinterpret_cast<const f4_t*>(next + b * SLOT + SM_ATOMS + 4 * t);
+            for (int b = 0; b < nparts; ++b) v += *reinterpret_cast<const f4_t*>(next + b * SLOT + ATOMS + 4 * t);
             *to = v;
         }
     }
@@ -568,7 +683,7 @@ __global__ __launch_bounds__(256) void sorf_parts_kernel(const int* __restrict__
 
 static int matrix_rounds(int T, int S, int d) { return (S + stacks_per_round(d, T) - 1) / stacks_per_round(d, T); }
 static long long matrix_units(int A, int ne, int T, int S, int d) {
-    return ((long long)(A + SM_ATOMS - 1) / SM_ATOMS + ne) * matrix_rounds(T, S, d);
+    return ((long long)(A + tile_atoms(d) - 1) / tile_atoms(d) + ne) * matrix_rounds(T, S, d);
 }
 // Shares of a launch.  Three (d = 128 with the gradient) or four workgroups are resident per CU; twice as many shares level out
 // what the cut into whole shares leaves uneven, but a share of few rounds pays more for its parts than it gains.
@@ -587,17 +702,17 @@ static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, i
         at += (bytes + 15) / 16 * 16;
         return p;
     };
-    f.images = (half8_t*)take((size_t)ne * T * S * (d / 16) * 1024);
+    f.images = (half8_t*)take((size_t)ne * S * image_bytes(d, T));
     f.largest = (float*)take((size_t)ne * S * sizeof(float));
     f.unfit = (int*)take(sizeof(int));
     f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
     f.alpha = (float*)take(((size_t)ne * S * d + 1) * sizeof(float));
-    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * SM_ATOMS * (with_grad ? d + 1 : 1) * sizeof(float));
+    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * tile_atoms(d) * (with_grad ? d + 1 : 1) * sizeof(float));
     return at;
 }
 
 static int matrix_shape(int ne, int T, int S, int d) {
-    return ne > 0 && S > 0 && (T == 1 || T == 2) && (d == 64 || d == 128) && (long long)ne * S < (1ll << 31) - 1 &&
+    return ne > 0 && S > 0 && (T == 1 || T == 2) && (d == 64 || d == 128 || d == 256) && (long long)ne * S < (1ll << 31) - 1 &&
            (long long)S * d < (1ll << 31);
 }
 
@@ -608,14 +723,16 @@ extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, 
 }
 
 // What this kernel gains per atom and stack has to carry three launches more and the parts of the cut tiles, 25 us with the
-// gradient and 15 us without.  Measured, rows kernel / this call, with the gradient: d = 128, 128 stacks, 12000 atoms 124 / 130 us (1.5e6
-// in the units below), 20000 atoms 191 / 186 (2.6e6); two transforms, 32 stacks, 24000 atoms 108 / 110 (1.5e6), 33000 atoms 148 / 143 (2.1e6);
-// d = 64, 128 stacks, 24000 atoms 107 / 112, 33000 atoms 144 / 138; 8 stacks, 86016 atoms 70 / 78 (0.7e6).  Energies only: d = 128, 128
-// stacks, 12000 atoms 69 / 70, 20000 atoms 112 / 94; two transforms, 32 stacks, 24000 atoms 58 / 60, 33000 atoms 78 / 75; d = 64, 128 stacks,
-// 12000 atoms 36 / 41 (0.8e6), 20000 atoms 57 / 52 (1.3e6).
+// gradient and 15 us without.  Measured, rows kernel / this call, in units of 1e6 below.  With the gradient, one transform: d = 128, 128 stacks
+// 10000 atoms (1.3) 100 / 106 us, 12000 (1.5) 117 / 116, 17000 161 / 142, 32 stacks 40000 atoms (1.3) 101 / 102; d = 64 18000 (1.2) 84 / 84;
+// d = 256 5000 (1.3) 112 / 120, 7000 (1.8) 151 / 144.  Two transforms, 32 stacks: d = 128 14000 atoms (0.9) 68 / 81, 18000 (1.2) 86 / 88,
+// 24000 (1.5) 111 / 101; d = 64 30000 (1.0) 68 / 71, 40000 (1.3) 87 / 79; d = 256, where the rows kernel has few wavefronts per SIMD, 4000
+// (0.5) 70 / 78, 6000 (0.8) 101 / 86.  Energies only: d = 128 10000 (1.3) 61 / 64, 12000 (1.5) 71 / 68; d = 64 18000 (1.2) 54 / 53; d = 256
+// 5000 (1.3) 63 / 67, 7000 (1.8) 85 / 82; two transforms, d = 128 24000 (1.5) 61 / 63, d = 256 14000 (1.8) 76 / 77.
 extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
     if (!matrix_shape(ne, T, S, d) || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
-    return (double)A * S * T * d / 128.0 >= (with_grad ? 2e6 : 1.5e6);
+    const double line = d == 256 ? (T == 1 ? 1.5e6 : with_grad ? 0.75e6 : 1.8e6) : with_grad ? 2e6 : 1.5e6;
+    return (double)A * S * T * d / 128.0 >= line;
 }
 
 static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, float factor,
@@ -623,22 +740,26 @@ static void launch_prepare(const float* D, const float* bias, const float* alpha
     const dim3 grid(ne * S), block(PREP_THREADS);
     if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
-    else if (T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else if (d == 128 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else if (d == 256 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<256, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
+    else if (d == 256) hipLaunchKernelGGL((sorf_prepare_kernel<256, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else hipLaunchKernelGGL((sorf_prepare_kernel<128, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
 }
 
+static int signs_shape(int ne, int T, int S, int d) { return matrix_shape(ne, T, S, d) && d <= 128; }
+
 extern "C" size_t qmll_sorf_signs_bytes(int ne, int T, int S, int d) {
-    return matrix_shape(ne, T, S, d) ? (size_t)ne * T * S * (d / 16) * 1024 + (size_t)ne * S * sizeof(float) : 0;
+    return signs_shape(ne, T, S, d) ? (size_t)ne * S * image_bytes(d, T) + (size_t)ne * S * sizeof(float) : 0;
 }
 
 extern "C" int qmll_sorf_signs(const float* D, int ne, int T, int S, int d, void* out, size_t out_bytes, qmll_stream_t stream) {
-    QMLL_REQUIRE(matrix_shape(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: no kernel takes ne=%d T=%d S=%d d=%d", ne, T, S, d);
+    QMLL_REQUIRE(signs_shape(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: no kernel takes ne=%d T=%d S=%d d=%d", ne, T, S, d);
     QMLL_REQUIRE(D && out && ((uintptr_t)out & 15) == 0, QMLL_ERR_INVALID, "qmll_sorf_signs: null or misaligned pointer");
     QMLL_REQUIRE(out_bytes >= qmll_sorf_signs_bytes(ne, T, S, d), QMLL_ERR_INVALID, "qmll_sorf_signs: output of %zu bytes, %zu are needed",
                  out_bytes, qmll_sorf_signs_bytes(ne, T, S, d));
     Forms f = {};
     f.images = (half8_t*)out;
-    f.largest = (float*)((char*)out + (size_t)ne * T * S * (d / 16) * 1024);
+    f.largest = (float*)((char*)out + (size_t)ne * S * image_bytes(d, T));
     launch_prepare(D, nullptr, nullptr, ne, T, S, d, 1.0f, f, (hipStream_t)stream);
     QMLL_CHECK_LAUNCH("qmll_sorf_signs");
     return QMLL_OK;
@@ -684,7 +805,8 @@ extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, 
     };
     auto by_d = [&](auto tc) {
         if (d == 64) by_grad(std::integral_constant<int, 64>{}, tc);
-        else by_grad(std::integral_constant<int, 128>{}, tc);
+        else if (d == 128) by_grad(std::integral_constant<int, 128>{}, tc);
+        else by_grad(std::integral_constant<int, 256>{}, tc);
     };
     if (T == 1) by_d(std::integral_constant<int, 1>{});
     else by_d(std::integral_constant<int, 2>{});
