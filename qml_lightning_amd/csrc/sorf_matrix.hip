@@ -685,13 +685,15 @@ static int matrix_rounds(int T, int S, int d) { return (S + stacks_per_round(d, 
 static long long matrix_units(int A, int ne, int T, int S, int d) {
     return ((long long)(A + tile_atoms(d) - 1) / tile_atoms(d) + ne) * matrix_rounds(T, S, d);
 }
-// Shares of a launch.  Three (d = 128 with the gradient) or four workgroups are resident per CU; twice as many shares level out
-// what the cut into whole shares leaves uneven, but a share of few rounds pays more for its parts than it gains.
-// Measured at d = 128, 128 stacks with the gradient, 3 / 6 shares per CU: 24000 atoms 206 / 207 us, 86016 atoms 668 / 628, and with two
-// transforms, 32 stacks, 24000 atoms 102 / 110.
-static int matrix_shares(long long units, int with_grad) {
-    const long long per_cu = units / (SM_CUS * (with_grad ? 24 : 16));
-    return (int)std::min(units, (long long)SM_CUS * std::max(3ll, std::min(6ll, per_cu)));
+// Shares of a launch: as many as workgroups are resident, which then all end at the same time, or twice as many where a share of those
+// still has many units and the whole tiles of the first round (share_begin) save parts.  Any other number leaves a round of
+// workgroups part empty: four shares per CU where three are resident take 292 us for 33000 atoms at d = 128, 128 stacks with the gradient,
+// three 228; 60000 atoms with two transforms, 32 stacks 234 and 201.  One round / two: with the gradient 45000 atoms (30 units a
+// share) 297 / 313 us, 65000 (42) 409 / 409, 200000 1166 / 1158; energies only 55300 atoms (27) 191 / 195, 100000 (49) 314 / 304, and at
+// d = 256 34000 (33) 265 / 263, 60000 443 / 419.
+static long long matrix_shares(long long units, int d, int with_grad) {
+    const long long resident = SM_CUS * (d >= 128 && with_grad ? 3 : 4);
+    return std::min(units, units >= 2 * resident * (with_grad ? 48 : 32) ? 2 * resident : resident);
 }
 
 // the workspace of a call: the forms, every part of them 16-byte aligned, then the parts of the cut tiles; its size for base = null
@@ -707,7 +709,7 @@ static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, i
     f.unfit = (int*)take(sizeof(int));
     f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
     f.alpha = (float*)take(((size_t)ne * S * d + 1) * sizeof(float));
-    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), with_grad) * tile_atoms(d) * (with_grad ? d + 1 : 1) * sizeof(float));
+    parts = (float*)take((size_t)matrix_shares(matrix_units(A, ne, T, S, d), d, with_grad) * tile_atoms(d) * (with_grad ? d + 1 : 1) * sizeof(float));
     return at;
 }
 
@@ -731,7 +733,7 @@ extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, 
 // 5000 (1.3) 63 / 67, 7000 (1.8) 85 / 82; two transforms, d = 128 24000 (1.5) 61 / 63, d = 256 14000 (1.8) 76 / 77.
 extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
     if (!matrix_shape(ne, T, S, d) || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
-    const double line = d == 256 ? (T == 1 ? 1.5e6 : with_grad ? 0.75e6 : 1.8e6) : with_grad ? 2e6 : 1.5e6;
+    const double line = with_grad ? (T == 1 ? 1.5e6 : d == 256 ? 0.75e6 : 1.2e6) : (T == 1 ? 1.5e6 : 1.8e6);
     return (double)A * S * T * d / 128.0 >= line;
 }
 
@@ -787,7 +789,7 @@ extern "C" int qmll_sorf_energy_matrix(const float* x, const int* type_offsets, 
     // x into revolutions, and the factors of the gradient and of the energy, each rounded once
     const double scale = (double)normalisation / (T == 1 ? sqrt((double)d) : (double)d), norm = sqrt(2.0 / ((double)S * d));
     const float xs = (float)(scale * 0.15915494309189533577), gscale = (float)(-scale * norm), normf = (float)norm;
-    const int nshares = matrix_shares(matrix_units(A, ne, T, S, d), gx != nullptr);
+    const int nshares = (int)matrix_shares(matrix_units(A, ne, T, S, d), d, gx != nullptr);
     const dim3 grid(nshares + (gx ? (A >= 65536 ? 64 : (A >> 10) + 1) : 0));
     hipStream_t st = (hipStream_t)stream;
     launch_prepare(D, bias, alpha, ne, T, S, d, T == 1 ? 1.0f / (1 << SM_EXP) : 1.0f, f, st);
