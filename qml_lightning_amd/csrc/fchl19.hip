@@ -335,6 +335,81 @@ __device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(
 __device__ __forceinline__ float flog2(float x) { return __builtin_amdgcn_logf(x); }
 constexpr float LOG2E = 1.4426950408889634f;
 
+// sqrt(x) from x and its reciprocal root, to half an ulp: sk3 times the last bits of a distance moves the weights of the radial bins
+__device__ __forceinline__ float root(float x, float inv) {
+    const float r = x * inv;
+    return fmaf(0.5f * inv, fmaf(-r, r, x), r);
+}
+
+// ---- evenly spaced radial bins --------------------------------------------------------------
+// exp2(-(y - u_l)^2) for bins u_l = u_a + k h is w Q^k exp2(-(k h)^2) with w = exp2(-(y - u_a)^2) and Q = exp2(2 h (y - u_a)): the sums over a
+// group of five bins are w times a polynomial in Q, whose coefficients take the constant factors, and their derivatives by y follow
+// from the polynomial's.  That is one exponential of the transcendental unit per group, and one multiply-add per bin for each sum (Q of all
+// groups is one more exponential times a constant each).  Groups of five keep Q^4 in range and its relative error at four
+// roundings; where a bin's weight counts, y is near the bin and the arguments of both exponentials are small.  Of 20 bins' 140
+// instructions, 20 of them exponentials, 118 and 5 are left.  86016 atoms of 21, three elements, backward 186 -> 172 us; 16 boxes of 96 atoms
+// 56.9 -> 50.8, and the forward kernel of several wavefronts per atom, where a lane's second bin is its first times a
+// factor of the triple, 48.8 -> 45.8.  The forward kernel of one wavefront per atom keeps both exponentials: the factor
+// made its table entries 16 bytes, and 131235 atoms of 3 to 29, five elements went from 275 to 293 us.
+constexpr int RS3_GROUP = 5;
+
+// The spacing of the bins u (lane: bin l, if ok) about the middle of the range, to a rounding of the grid's, or 0: uneven, or
+// so wide that Q could leave 2^16 (y is within mid of the middle) or exp2(2 h u) 2^8.
+__device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid) {
+    const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(u)));
+    const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(u), nRs3 - 1));
+    const float h = (last - first) * frcp((float)(nRs3 - 1));
+    const float edge = fmaxf(fabsf(first), fabsf(last)), widest = mid + edge;
+    const bool fits = fabsf(fmaf((float)-l, h, u - first)) <= 2.4e-7f * widest && widest * fabsf(h) <= 8.0f && edge * fabsf(h) <= 4.0f;
+    return __any(ok && !fits) ? 0.0f : h;
+}
+
+// The same for bins 2 l and 2 l + 1 on a lane, l < (nRs3 + 1) / 2 on the first lanes
+__device__ __forceinline__ float even_spacing_pairs(float ua, float ub, int l, int nRs3, float mid) {
+    const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ua)));
+    const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nRs3 & 1 ? ua : ub), (nRs3 - 1) >> 1));
+    const float h = (last - first) * frcp((float)(nRs3 - 1));
+    const float edge = fmaxf(fabsf(first), fabsf(last)), widest = mid + edge, slack = 2.4e-7f * widest;
+    const float at = fmaf((float)(2 * l), h, first);
+    const bool fits = fabsf(ua - at) <= slack && (2 * l + 1 >= nRs3 || fabsf(ub - at - h) <= slack) && widest * fabsf(h) <= 8.0f && edge * fabsf(h) <= 4.0f;
+    return __any(2 * l < nRs3 && !fits) ? 0.0f : h;
+}
+
+// the constant factor of bin l, s = u_l - u_a behind the first of its group: exp2(-s^2), the bin's own place instead of k h where y is on it
+__device__ __forceinline__ float group_factor(float u, int l, int lane, float h) {
+    const int k = l % RS3_GROUP;
+    const float s = u - __shfl(u, lane - k, 64);
+    return fexp2(s * (s - 2.0f * h * (float)k));
+}
+
+// exp2(2 h y), the factor of Q that all groups share, and what the product's rounding left out: Q goes to the fourth power.
+// STOP: distances from a given list may be anything.  It stops at 2^18, which no y within mid of the middle reaches (with the default
+// grid the weights are below 2^-80 there), and Q^4 stays in range.
+template <bool STOP>
+__device__ __forceinline__ float group_ratio(float h, float y) {
+    const float x = 2.0f * h * y, e = fexp2(STOP ? fminf(x, 18.0f) : x);
+    return fmaf(e * 0.6931472f, fmaf(2.0f * h, y, -x), e);
+}
+
+// G += sum_k g_k w Q^k, H += sum_k g_k (d - k h) w Q^k
+__device__ __forceinline__ void group_sums(const float2* g, float d, float w, float Q, float h, float& Gc, float& Gs, float& Hc, float& Hs) {
+    const float2 g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3], g4 = g[4];
+    const float hQ = h * Q;
+    auto one = [&](float c0, float c1, float c2, float c3, float c4, float& G, float& H) {
+        float P = fmaf(c4, Q, c3), D = c4;               // polynomial and derivative
+        D = fmaf(D, Q, P);
+        P = fmaf(P, Q, c2);
+        D = fmaf(D, Q, P);
+        P = fmaf(P, Q, c1);
+        D = fmaf(D, Q, P);
+        P = fmaf(P, Q, c0);
+        G = fmaf(w, P, G);
+        H = fmaf(w, fmaf(d, P, -hQ * D), H);
+    };
+    one(g0.x, g1.x, g2.x, g3.x, g4.x, Gc, Hc);
+    one(g0.y, g1.y, g2.y, g3.y, g4.y, Gs, Hs);
+}
+
 // row index of pair t in the list of pairs (j<k) over nn items, rows enumerated j = 0..nn-2
 __device__ __forceinline__ void unrank_pair(int t, int nn, int& j, int& k) {
     const float b = (float)(2 * nn - 1);
@@ -400,13 +475,13 @@ __device__ __forceinline__ Triple triple_geometry(const Stage& s, int j, int k) 
     return t;
 }
 
-// what the forward kernels keep of a neighbour, written by the lane that found it: d_ij and 1 / r; sk3 r / 2, fc r^-d3,
+// what the forward kernels keep of a neighbour, written by the lane that found it: d_ij and 1 / r; sk3 r / 2 - half_mid, fc r^-d3,
 // element type, index within the type | neighbours of the type << 16; mu_j, log2(e) / (2 sigma_j^2),
 // r^-d2 fc / (sigma sqrt(2 pi))
-__device__ __forceinline__ void forward_records(const qmll_fchl_params& p, float sk3, float inv_rc, float* recA, float* recB,
+__device__ __forceinline__ void forward_records(const qmll_fchl_params& p, float sk3, float half_mid, float inv_rc, float* recA, float* recB,
                                                 float* s2b, int pos, int rank, int count, int e, float dx, float dy, float dz,
                                                 float r2) {
-    const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+    const float ir = __builtin_amdgcn_rsqf(r2), r = root(r2, ir);
     float fc, dfc;
     cutoff(r, inv_rc, fc, dfc);
     const float l2r = flog2(r);
@@ -416,7 +491,7 @@ __device__ __forceinline__ void forward_records(const qmll_fchl_params& p, float
         0.5f * LOG2E * frcp(s2),
         frsq(s2) * 0.3989422804014327f * fexp2(-p.two_body_decay * l2r) * fc, 0.0f);
     reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, ir);
-    reinterpret_cast<float4*>(recB)[pos] = make_float4(sk3 * 0.5f * r, fc * fexp2(-p.three_body_decay * l2r),
+    reinterpret_cast<float4*>(recB)[pos] = make_float4(fmaf(sk3 * 0.5f, r, -half_mid), fc * fexp2(-p.three_body_decay * l2r),
                                                        __int_as_float(e), __int_as_float(rank | (count << 16)));
 }
 
@@ -551,7 +626,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_num_sgpr(96))) void fchl1
     // every neighbour's factors of the two-body bins and of the triples, by the lane that found it
     const int nn = visit_neighbours(
         a, goff, m, i, lane, [&](int pos, int rank, int count, int e, int, float dx, float dy, float dz, float r2) {
-            forward_records(a.p, sk3, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
+            forward_records(a.p, sk3, 0.0f, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
         });
     if (lane < nRs2) {
         slnRs2[lane] = flog(rs2v);
@@ -902,7 +977,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
                 pos = rank + first[q];
             }
         }
-        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        const float ir = __builtin_amdgcn_rsqf(r2), r = root(r2, ir);
         float fc, dfc;
         cutoff(r, inv_rc, fc, dfc);
         const float l2r = flog2(r);
@@ -1055,11 +1130,12 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
     const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
     const float sk3 = fsqrt(a.p.eta3 * LOG2E);
     const float inv_rc = frcp(a.p.rcut);
+    const float mid = LEAN ? 0.5f * sk3 * a.p.rcut : 0.0f;       // LEAN: distances and bins about the middle of the range
     const float rs2v = tid < nRs2 ? a.Rs2[tid] : 1.0f;
     const float rs3v = tid < nRs3 ? a.Rs3[tid] : 0.0f;
     const int nn = visit_neighbours_wide<NW>(
         a, goff, wcount, m, i, tid, [&](int pos, int rank, int count, int e, int, float dx, float dy, float dz, float r2) {
-            forward_records(a.p, sk3, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
+            forward_records(a.p, sk3, 0.5f * mid, inv_rc, recA, recB, s2b, pos, rank, count, e, dx, dy, dz, r2);
         });
     for (int t = tid; t < np * NW * per; t += NT) part[t] = 0.0f;
     for (int t = tid; t < nRs2; t += NT) {
@@ -1113,8 +1189,11 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
 #pragma unroll
     for (int b = 0; b < (LEAN ? 2 : MAXLB); ++b) {
         const int l = LEAN ? 2 * ll + b : b * 64 + ll;
-        rsl[b] = (LEAN || b * 64 < nRs3) ? sk3 * sRs3[l < nRs3 ? l : 0] : 0.0f;
+        rsl[b] = (LEAN || b * 64 < nRs3) ? fmaf(sk3, sRs3[l < nRs3 ? l : 0], -mid) : 0.0f;
     }
+    // LEAN, an even grid: the second of a lane's two weights is the first times exp2(2 h y), once per triple, and this constant
+    const float h = LEAN ? even_spacing_pairs(rsl[0], rsl[1], ll, nRs3, mid) : 0.0f;
+    const float step = rsl[1] - rsl[0], factor = LEAN && h != 0.0f ? fexp2(step * (step - 2.0f * h) - 2.0f * h * rsl[0]) : 1.0f;
     const float zw3 = zeta2 * a.p.three_body_weight, hd3 = -0.5f * a.p.three_body_decay;
     const float4* rA = reinterpret_cast<const float4*>(recA);
     const float4* rB = reinterpret_cast<const float4*>(recB);
@@ -1131,7 +1210,9 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
             else unrank_triple(goff, pbase, ns, np, tt, j, k);
             const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
             const int to = whole ? triple_place(pbase, ns, Bj, Bk) : tt - t0;
-            reinterpret_cast<float4*>(trip)[to] = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
+            float4 entry = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
+            if constexpr (LEAN) entry.w = group_ratio<true>(h, entry.x);
+            reinterpret_cast<float4*>(trip)[to] = entry;
         }
         __syncthreads();
         // this wavefront's share of the chunk: a run of consecutive entries, which meets few element pairs
@@ -1147,18 +1228,24 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
             float* dst = part + ((size_t)pq * NW + wave) * per;
             if constexpr (LEAN) {
                 float v[4] = {0.f, 0.f, 0.f, 0.f};
-                auto add = [&](const float4* at) {
-                    const float3v t = *reinterpret_cast<const float3v*>(at);
+                auto add = [&](const float4* at, auto even) {
+                    const float4 t = *at;
                     const float d0 = t.x - rsl[0], d1 = t.x - rsl[1];
-                    const float e0 = fexp2(-d0 * d0), e1 = fexp2(-d1 * d1);
+                    const float e0 = fexp2(-d0 * d0), e1 = decltype(even)::value ? e0 * t.w : fexp2(-d1 * d1);
                     v[0] = fmaf(e0, t.y, v[0]);
                     v[1] = fmaf(e0, t.z, v[1]);
                     v[2] = fmaf(e1, t.y, v[2]);
                     v[3] = fmaf(e1, t.z, v[3]);
                 };
+                auto run = [&](auto even) {
 #pragma unroll 2
-                for (int it = 0; it < rounds; ++it) add(src + it * LEAN_SLOTS);
-                if (rest > 0) add(tsub < rest ? src + rounds * LEAN_SLOTS : tab + a.tcap);
+                    for (int it = 0; it < rounds; ++it) add(src + it * LEAN_SLOTS, even);
+                    if (rest > 0) add(tsub < rest ? src + rounds * LEAN_SLOTS : tab + a.tcap, even);
+                };
+                if (h != 0.0f) run(std::true_type{});
+                else run(std::false_type{});
+                v[2] *= factor;
+                v[3] *= factor;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     v[c] += __shfl(v[c], lane + 30, 64);
@@ -1378,7 +1465,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     for (int t = lane; t < a.tcap; t += QMLL_WAVE) set_force(mine + FR * t, 0.f, 0.f, 0.f);
     const float inv_rc = frcp(a.p.rcut);
     auto emit = [&](int pos, int, int, int e, int j, float dx, float dy, float dz, float r2) {
-        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        const float ir = __builtin_amdgcn_rsqf(r2), r = root(r2, ir);
         float fc, dfc;
         cutoff(r, inv_rc, fc, dfc);
         reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, r);
@@ -1396,9 +1483,13 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // factor does not depend on the triple and goes into the staged gradient once per atom; the first
     // is one fma and the exponential per (triple, bin).  It is at most 2^(u_l^2), so the form is taken
     // only while u_l^2 <= 100 for every bin (eta3 rcut^2 up to about 270); beyond, the plain form runs.
+    // LEAN: see group_sums; where the grid is not even, the plain form.
     const float mid = 0.5f * sk3 * a.p.rcut;
-    bool fast;
-    {
+    const float ul = LEAN && lane < nRs3 ? fmaf(sk3, rs3v, -mid) : 0.0f;
+    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid) : 0.0f;
+    const bool even = LEAN && spacing != 0.0f;
+    bool fast = false;
+    if constexpr (!LEAN) {
         float um = fabsf(fmaf(sk3, rs3v, -mid));
         if (lane >= nRs3) um = 0.0f;
         for (int t = lane + QMLL_WAVE; t < nRs3; t += QMLL_WAVE) um = fmaxf(um, fabsf(fmaf(sk3, a.Rs3[t], -mid)));
@@ -1410,7 +1501,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
         um = fmaxf(um, lane_xor<32>(um));
         fast = __builtin_amdgcn_readfirstlane(__float_as_int(um)) <= __float_as_int(10.0f);
     }
-    const float shift = fast ? mid : 0.0f;
+    const float shift = LEAN || fast ? mid : 0.0f;
     // the gradient of the two-body bins, each divided by its grid point (the bin's 1 / Rs2 factor)
 #pragma unroll
     for (int k = 0; k < GREG2; ++k) {
@@ -1421,7 +1512,11 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
         gin2[t] = gsrc[t] * (a.gscale * frcp(a.Rs2[t - nRs2 * idiv_small(t, nRs2)]));
     if (lane < nRs2 && wave == 0) slnRs2[lane] = flog(rs2v);
     for (int t = tid + QMLL_WAVE; t < nRs2; t += NT) slnRs2[t] = flog(a.Rs2[t]);
-    for (int t = tid; t < nRs3; t += NT) {
+    if constexpr (LEAN) {
+        const float f = a.gscale * (even ? group_factor(ul, lane, lane, spacing) : 1.0f);
+        if (tid < nRs3) sfac[tid] = f;
+    }
+    for (int t = LEAN ? nRs3 : tid; t < nRs3; t += NT) {
         const float u = fmaf(sk3, t == lane ? rs3v : a.Rs3[t], -shift);
         sRs3[t] = u;
         sfac[t] = a.gscale * (fast ? fexp2(-u * u) : 1.0f);
@@ -1498,11 +1593,13 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     const int ntrip = nn * (nn - 1) / 2;
     const float zeta2 = 0.014383766711652736f;   // 2 exp(-pi^2 / 2)
     const float d3 = a.p.three_body_decay;
-    float us[LEAN ? LEAN_RS3 : 1];                     // the grid, on scalar registers
+    float us[LEAN ? LEAN_RS3 : 1], ratio[LEAN_RS3 / RS3_GROUP];        // the grid, on scalar registers
     if constexpr (LEAN) {
-        const float ul = lane < nRs3 ? fmaf(sk3, rs3v, -shift) : 0.0f;
+        const float v = fexp2(-2.0f * spacing * ul);
 #pragma unroll
         for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
+#pragma unroll
+        for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) ratio[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), RS3_GROUP * q));
     }
     // copies of the force records that this atom uses: one for every s-row of an instruction, or as many as there is room for
     auto copies = [&] { return COMPACT ? min(force_copies(nn), idiv_small(a.tcap, max(nn, 1))) : force_copies(nn); };
@@ -1565,7 +1662,14 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
                 for (int l = 0; l < nRs3; ++l) bin(g[l].x, g[l].y, sRs3[l]);
             }
         };
-        if (fast) {
+        if (even) {
+            const float B = group_ratio<true>(spacing, y);
+#pragma unroll
+            for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) {
+                const float d = y - us[LEAN ? RS3_GROUP * q : 0];
+                group_sums(g + RS3_GROUP * q, d, fexp2(-(d * d)), B * ratio[q], spacing, Gc, Gs, Hc, Hs);
+            }
+        } else if (fast) {
             const float y2 = y + y, ny2 = -y * y;
             bins([&](float gc, float gs, float u) {
                 const float e = fexp2(fmaf(y2, u, ny2));
@@ -1638,9 +1742,9 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
 // that kernel takes 1640 vector, 434 scalar and 137 LDS instructions per atom of 20 neighbours, and its bin loop reads 12 bytes per lane and
 // bin, six clocks of the LDS that four SIMDs share.  Here the grid is on scalar registers, the two bins of a 16-byte read are unrolled
 // with their places as constants, a lane stages the gradient of one radial bin of three pairs at a time (its constant factor is then in
-// a register), and the number of a triple's pair comes from the neighbours' records in two instructions: 1426 + 288 + 98 instructions.
-// 86016 atoms of 21, three elements 193 -> 165 us, 131235 atoms of 3 to 29, five elements 342 -> 290, 64000 of 8 89 -> 63, 80000 of 40
-// 476 -> 446.  Vector issue takes five sixths of the launch.
+// a register), and the number of a triple's pair comes from the neighbours' records in two instructions: 1426 + 288 + 98 instructions
+// (before the bins were taken in groups).  86016 atoms of 21, three elements 193 -> 165 us, 131235 atoms of 3 to 29, five elements
+// 342 -> 290, 64000 of 8 89 -> 63, 80000 of 40 476 -> 446.  Vector issue takes five sixths of the launch.
 // ---------------------------------------------------------------------------------
 template <int NS>
 __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const float* __restrict__ grad_rep, float* __restrict__ grad_X) {
@@ -1689,10 +1793,10 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
     const float inv_rc = frcp(a.p.rcut);
     const float sk3 = fsqrt(a.p.eta3 * LOG2E);
     const float hfac = -2.0f * a.p.eta3 * frcp(sk3);
-    const float mid = 0.5f * sk3 * a.p.rcut;             // the radial factor about the middle of the grid: see fchl19_vjp_kernel
-    const bool fast = !__any(bin_ok && !(fabsf(fmaf(sk3, rs3v, -mid)) <= 10.0f));
-    const float shift = fast ? mid : 0.0f;
-    const float ul = bin_ok ? fmaf(sk3, rs3v, -shift) : 0.0f;
+    const float mid = 0.5f * sk3 * a.p.rcut;             // distances and bins about the middle of the range: half the rounding
+    const float ul = bin_ok ? fmaf(sk3, rs3v, -mid) : 0.0f;
+    const float spacing = even_spacing(ul, l3, bin_ok, nRs3, mid);
+    const bool even = spacing != 0.0f;
 
     // ---- neighbours: candidate = lane ----
     float dx = Xm[i * 3 + 0] - xo, dy = Xm[i * 3 + 1] - yo, dz = Xm[i * 3 + 2] - zo;
@@ -1718,7 +1822,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         nn += __popcll(mask);
     }
     if (near) {
-        const float ir = __builtin_amdgcn_rsqf(r2), r = r2 * ir;
+        const float ir = __builtin_amdgcn_rsqf(r2), r = root(r2, ir);
         float fc, dfc;
         cutoff(r, inv_rc, fc, dfc);
         reinterpret_cast<float4*>(recA)[pos] = make_float4(dx, dy, dz, r);
@@ -1727,7 +1831,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
     }
     // the incoming gradient, times the constant factor of its bin
     {
-        const float f2 = a.gscale * frcp(rs2v), f3 = a.gscale * (fast ? fexp2(-ul * ul) : 1.0f);
+        const float f2 = a.gscale * frcp(rs2v), f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
         if (lane < 32) slnRs2[lane] = flog(rs2v);
 #pragma unroll
         for (int k = 0; k < (NS + 1) / 2; ++k)
@@ -1781,9 +1885,14 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
     __syncthreads();
 
     // ---- three-body: lane = triple; see fchl19_vjp_kernel for the numbering, the copies and the formulas ----
-    float us[LEAN_RS3];                                  // the grid, on scalar registers
+    float us[LEAN_RS3], ratio[LEAN_RS3 / RS3_GROUP];     // the grid, on scalar registers
 #pragma unroll
     for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
+    {
+        const float v = fexp2(-2.0f * spacing * ul);
+#pragma unroll
+        for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) ratio[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), RS3_GROUP * q));
+    }
     const int ntrip = (nn * (nn - 1)) >> 1;
     const float zw3 = 0.014383766711652736f * a.p.three_body_weight;     // 2 exp(-pi^2 / 2)
     const float d3 = a.p.three_body_decay;
@@ -1835,26 +1944,16 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         // the bins of this triple's pair of types
         const unsigned pair = __builtin_amdgcn_ubfe(__float_as_uint(Bk.w), __float_as_uint(Bj.w) >> 20, 4);
         const float4* g = reinterpret_cast<const float4*>(gin3 + __mul24((int)pair, 2 * LEAN_RS3));
-        const float y = fmaf(sk3 * 0.5f, Aj.w + Ak.w, -shift);
+        const float y = fmaf(sk3 * 0.5f, Aj.w + Ak.w, -mid);
         float Gc = 0.f, Gs = 0.f, Hc = 0.f, Hs = 0.f;
-        if (fast) {
-            const float y2 = y + y, ny2 = -y * y;
-            auto bin = [&](float gc, float gs, float u) {
-                const float e = fexp2(fmaf(y2, u, ny2));
-                const float ue = u * e;
-                Gc = fmaf(gc, e, Gc);
-                Gs = fmaf(gs, e, Gs);
-                Hc = fmaf(gc, ue, Hc);
-                Hs = fmaf(gs, ue, Hs);
-            };
+        if (even) {
+            const float B = group_ratio<false>(spacing, y);
+            const float2* g2 = reinterpret_cast<const float2*>(g);
 #pragma unroll
-            for (int l = 0; l < LEAN_RS3; l += 2) {
-                const float4 gv = g[l / 2];
-                bin(gv.x, gv.y, us[l]);
-                bin(gv.z, gv.w, us[l + 1]);
+            for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) {
+                const float d = y - us[RS3_GROUP * q];
+                group_sums(g2 + RS3_GROUP * q, d, fexp2(-(d * d)), B * ratio[q], spacing, Gc, Gs, Hc, Hs);
             }
-            Hc = fmaf(y, Gc, -Hc);
-            Hs = fmaf(y, Gs, -Hs);
         } else {
             auto bin = [&](float gc, float gs, float u) {
                 const float dl = y - u;
