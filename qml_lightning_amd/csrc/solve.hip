@@ -129,6 +129,20 @@ __device__ __forceinline__ bool static_all(F&& f) {
 // Output: upper triangle of the block <- U11; inv[m*128+i] = U11^-1[m,i] = W[i,m]; invT[i*128+m] the same.
 // info: 0, or 1 + the index of the first pivot that is not positive (later launches then exit).
 
+// Stores and loads past the caches of this XCD, whose L2 the others do not see: no fence, which would write a whole L2 back or
+// drop it, is needed beside them.
+__device__ __forceinline__ void store_past_caches(double* p, double v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_past_caches(unsigned* p, unsigned v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_past_caches(const double* p) {
+    return __longlong_as_double((long long)__hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT));
+}
+
 // inv[m, 16 K + i] = W[16 K + i, m] for the columns m of block row K, from the strip in LDS: thread = (m, half a
 // row of sixteen), 64 contiguous bytes each.  Wavefronts 4..7: 0 is the one that is waited for.
 __device__ __forceinline__ void store_inverse_columns(int K, double* inv, const PotrfShared& ps) {
@@ -200,13 +214,34 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
     return true;
 }
 
-// wavefront 4, which shares its SIMD with wavefront 0: no matrix instructions, the columns of the inverse only
-__device__ __forceinline__ bool potrf_store_wave(double* inv, PotrfShared& ps) {
+// wavefront 4, which shares its SIMD with wavefront 0: no matrix instructions.  It writes the columns of the inverse, and block row K of U
+// right of the diagonal and the diagonal sub-block of the inverse past the caches, for the workgroups that follow this factorisation step
+// by step (follow_block): *steps is the number of block rows that are there.  All of a step's stores are this wavefront's, so that waiting
+// for them is all the order they need.
+__device__ __forceinline__ bool potrf_store_wave(double* blk, long long ld, int nb, double* inv, double* invT, unsigned* steps,
+                                                 PotrfShared& ps) {
+    const int lane = (int)threadIdx.x & 63;
+    auto done = [&](unsigned count) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (steps && lane == 0) store_past_caches(steps, count);
+    };
     for (int K = 0; K < NSB; ++K) {
         __syncthreads();                                               // S(K,K) is in LDS
-        if (K > 0) store_inverse_columns(K - 1, inv, ps);
+        if (K > 0) {
+            const int row0 = (K - 1) * SB;
+#pragma unroll 4
+            for (int r = 0; r < SB; ++r)
+                for (int col = K * SB + lane; col < nb; col += QMLL_WAVE)
+                    if (row0 + r < nb) store_past_caches(&blk[(size_t)(row0 + r) * ld + col], ps.ustrip[r][col]);
+            done((unsigned)K);
+            store_inverse_columns(K - 1, inv, ps);
+        }
         __syncthreads();                                               // V is in LDS
         if (ps.failed) return false;
+#pragma unroll
+        for (int e = lane; e < SB * SB; e += QMLL_WAVE)                // W(K,K) = V^T
+            store_past_caches(&invT[(K * SB + e / SB) * NB + K * SB + e % SB], ps.vblk[e % SB][e / SB]);
+        if (K == NSB - 1) done(NSB);
         __syncthreads();                                               // block row K is in LDS
     }
     store_inverse_columns(NSB - 1, inv, ps);
@@ -220,7 +255,6 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
     const int lane = (int)threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
     const int ldi = (int)ld;
     // per-lane parts of every address; what is added per sub-block is a constant
-    double* const blk_lane = blk + (size_t)lk * ld + l16;
     double* const invT_lane = invT + lk * NB + l16;
     double* const us_lane = &ps.ustrip[lk][l16];
     double* const ws_lane = &ps.wstrip[lk][l16];
@@ -301,12 +335,10 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         if constexpr (b.kind == 0) {
-                            us_lane[4 * r * SSTRIDE + b.j * SB] = res[r];
-                            if (b.j * SB + l16 < nb && K * SB + lk + 4 * r < nb)
-                                blk_lane[(size_t)(K * SB + 4 * r) * ld + b.j * SB] = res[r];
+                            us_lane[4 * r * SSTRIDE + b.j * SB] = res[r];                   // (wavefront 4 writes it to memory)
                         } else {
                             ws_lane[4 * r * SSTRIDE + b.j * SB] = res[r];
-                            invT_lane[(K * SB + 4 * r) * NB + b.j * SB] = res[r];
+                            if constexpr (b.j < K) invT_lane[(K * SB + 4 * r) * NB + b.j * SB] = res[r];
                         }
                     }
                 }
@@ -325,7 +357,7 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
 
 // Called by all PT threads of the workgroup.  False when a pivot is not positive (info is then set).
 __device__ __forceinline__ bool potrf_block(double* A, long long ld, int k0, int nb, double* inv, double* invT,
-                                            int* info, PotrfShared& ps) {
+                                            int* info, unsigned* steps, PotrfShared& ps) {
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double* blk = A + (size_t)k0 * ld + k0;
@@ -345,7 +377,7 @@ __device__ __forceinline__ bool potrf_block(double* A, long long ld, int k0, int
         case 1: ok = potrf_mfma_wave<1>(blk, ld, nb, inv, invT, ps); break;
         case 2: ok = potrf_mfma_wave<2>(blk, ld, nb, inv, invT, ps); break;
         case 3: ok = potrf_mfma_wave<3>(blk, ld, nb, inv, invT, ps); break;
-        case 4: ok = potrf_store_wave(inv, ps); break;
+        case 4: ok = potrf_store_wave(blk, ld, nb, inv, invT, steps, ps); break;
         case 5: ok = potrf_mfma_wave<4>(blk, ld, nb, inv, invT, ps); break;
         case 6: ok = potrf_mfma_wave<5>(blk, ld, nb, inv, invT, ps); break;
         default: ok = potrf_mfma_wave<6>(blk, ld, nb, inv, invT, ps); break;
@@ -359,7 +391,7 @@ __global__ __launch_bounds__(PT, 4) void potrf_block_kernel(double* A, long long
                                                          double* invT, int* info) {
     __shared__ PotrfShared ps;
     if (*info != 0) return;
-    potrf_block(A, ld, k0, nb, inv, invT, info, ps);
+    potrf_block(A, ld, k0, nb, inv, invT, info, nullptr, ps);
 }
 
 // ---- one launch per panel -------------------------------------------------------------------
@@ -369,18 +401,26 @@ __global__ __launch_bounds__(PT, 4) void potrf_block_kernel(double* A, long long
 // tiles a panel is one launch instead, and that launch also carries the trailing update of the panel
 // before it.
 //
-// Column owners.  Workgroup w < (F - P0) / 128 owns the column of tiles w of the panel's rows (columns
-// P0 + 128 w ...).  It first gives its tiles the update of the previous panel (rows R0 .. P0 of the
-// factor, already final: the part of that panel's trailing update that falls into this panel's rows),
-// then walks down its column:
+// The chain.  Workgroup b < 4 owns block column b of the panel.  It first gives its tiles the update of the previous panel (rows
+// R0 .. P0 of the factor, already final: the part of that panel's trailing update that falls into this panel's rows), then, for each
+// block l < b, follows the factorisation of block l on its CU step by step (follow_block): the strip (l, b) and the update of
+// its own diagonal tile are done a step after the factorisation is.  Then it factors its diagonal tile and publishes the inverse.
+//     for l < b:  wait for "tile (l, b) has its updates";  follow block l;  publish "strip (l, b)"
+//     factor block b, handing out its block rows as they are done;  publish "block b factored"
+// The updates of the panel's tiles beside its diagonal, tile (b, w) -= strip(l, b)^T strip(l, w), stand between one factorisation and the next
+// but one, so that four workgroups each take a quarter of such a tile.  These owners and quarters wait for each other: they are the first
+// workgroups behind the head tiles (sixteen, of a CU each), so that all of them are resident before any other of the launch.
+// us per solve before this chain (strip and updates behind the whole block's inverse, a workgroup to a column of tiles) and with it: 512
+// features 260 / 186, 2048 1281 / 951, 4096 2800 / 2048, 8192 6900 / 5560, 16384 22030 / 19950, 24576 51460 / 48520.  A block of the chain takes 44 us,
+// 68 before, 30 of them its factorisation.  With 151 to 166 registers a workgroup has a CU to itself; held to the 128 of two the
+// followers spilled (51 us a block), and nothing else gained from the second.
+//
+// Column owners.  One or two workgroups own a column of tiles (or half of it) of the panel's rows right of the panel:
+//     first the update of the previous panel, as above;  then for l = 0 .. 3:
 //     wait for "block l factored";  tile(l, w) = U11_l^-T tile(l, w)                      row strip
-//     for the block rows b > l of its column: wait for "strip (l, b) done";
-//                                              tile(b, w) -= tile(l, b)^T tile(l, w)      update, 128 deep
-// and the owner of column l, which reaches its diagonal tile with every update applied, factors it and
-// publishes the inverse.  A workgroup only ever waits for owners of columns left of its own, which have
-// lower workgroup ids; ids are dispatched in order, so whoever is waited for is running or done,
-// whatever the number of workgroups resident at a time.  Every wait is bounded all the same: a wait that
-// runs out sets info to -1 and the workgroup leaves.
+//     for the block rows b > l:  wait for "strip (l, b) done";  tile(b, w) -= strip(l, b)^T tile(l, w)
+// They wait for lower workgroup ids only.  Every wait is bounded; one that runs out sets info to -1 and the workgroup leaves.  (Waiting polls with
+// relaxed loads: with an acquire at each poll the waiting owners kept emptying the L2 of those at work, a panel of 120 columns 326 us, 280 so.)
 //
 // Head tiles.  Once the trailing matrix is small a launch lasts as long as its slowest owner, and four of an
 // owner's fourteen tile products are that first update.  The host then puts workgroups for those tiles in
@@ -399,7 +439,10 @@ constexpr int P_CPT = NB / P_TPR;       // doubles per thread and row
 constexpr int P_UN = P_CPT / 2;         // 16-byte units per thread
 constexpr unsigned FLAG_DONE = 1u, FLAG_FAILED = 0x80000000u;   // (a counter never gets near the second)
 constexpr int PBLK = OB / NB;                        // blocks per panel
-constexpr int FLAGS_PER_PANEL = PBLK + PBLK * PBLK;  // "block l factored": [l]; "strip (l, b) done": [PBLK + l PBLK + b]
+// "block l factored": [l]; "strip (l, b) done": [PBLK + l PBLK + b]; block rows of block l that are there: [STEPS + l]; quarters of updates
+// that tile (b, w) of the panel's own columns has had: [QUARTERS + b PBLK + w]
+constexpr int STEPS = PBLK + PBLK * PBLK, QUARTERS = STEPS + PBLK, FLAGS_PER_PANEL = QUARTERS + PBLK * PBLK;
+constexpr int CUS = 256;
 constexpr int SPLIT_HEADS_BELOW = 48;       // trailing tiles per edge
 constexpr unsigned SPIN_LIMIT = 1u << 21;   // polls of about a microsecond each before a wait gives up
 
@@ -409,64 +452,61 @@ struct TileShared {
     double a[2][PKB][PSTRIDE], b[2][PKB][PSTRIDE];
 };
 
-constexpr int TRIANGULAR = 1, DIAGONAL = 2;
-// The 128 x 128 tile at C (row stride ldc) = or += sign * Za^T Zb, Za and Zb `depth` rows (a multiple of 16) of 128
-// columns; the tile product of gram.hip for whole tiles (same staging, same MFMA order).  C may be Zb
+constexpr int TRIANGULAR = 1;
+// The 128 x COLS tile at C (row stride ldc) = or += sign * Za^T Zb, Za `depth` rows (a multiple of 32) of 128
+// columns, Zb of COLS; the tile product of gram.hip for whole tiles (same staging, same MFMA order).  C may be Zb
 // (depth 128, overwrite): everything is read before anything is written.  Ends with a barrier.
-// TRIANGULAR: Za[m][i] = 0 for m > i (the inverse of a diagonal block), whose 16 x 16 sub-blocks below the diagonal are left out; DIAGONAL:
-// only the sub-blocks of C on or above the diagonal are wanted.  Either leaves 36 of 64: the chain of a panel is these
-// and the factorisations (82 us a block with whole products, 65 with these; 16384 features 25.0 -> 22.7 ms, 2048 1.59 -> 1.33).
-template <int MODE = 0>
+// TRIANGULAR: Za[m][i] = 0 for m > i (the inverse of a diagonal block), whose 16 x 16 sub-blocks below the diagonal are left out:
+// 36 of 64 remain.
+template <int COLS, int MODE = 0>
 __device__ __forceinline__ void tile_product(const double* Za, long long lda, const double* Zb, long long ldb,
                                              int depth, double* C, long long ldc, double sign, bool overwrite,
                                              TileShared& sm) {
+    static_assert(COLS == NB || COLS == NB / 2, "whole tiles or their halves");
+    constexpr int P = COLS == NB ? 4 : 2;                          // sub-blocks of a wavefront one below the other (two beside each other)
+    constexpr int B_CPT = COLS / P_TPR, B_UN = B_CPT / 2;
+    constexpr int AHEAD = COLS == NB ? 1 : 2;                      // steps on the way
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // (uniform: a matrix instruction takes no lane mask)
-    // (wavefronts w and w + 4 share a SIMD: in a diagonal tile they have 10, 10, 8 and 8 of 16 sub-blocks on or above the diagonal)
-    const int wi = (wave / 4) * 64, wj = (wave < 4 ? wave : 7 - wave) * 32;
+    const int wj = (COLS == NB ? wave & 3 : wave & 1) * 32;
+    // first row of sub-block p: in half a tile a wavefront has rows from both ends, which makes their work on a triangle equal
+    auto wi = [&](int p) { return COLS == NB ? (wave / 4) * 64 + p * 16 : (p == 0 ? wave / 2 : NSB - 1 - wave / 2) * 16; };
     const int l16 = lane & 15, lk = lane >> 4;
-    auto wanted = [&](int p, int q) { return MODE != DIAGONAL || wi + p * 16 <= wj + q * 16; };
-    double4_t acc[4][2];
+    double4_t acc[P][2];
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int q = 0; q < 2; ++q) acc[p][q] = (double4_t){0.0, 0.0, 0.0, 0.0};
-    const int lr = tid / P_TPR, lc = (tid % P_TPR) * P_CPT;
-    double2_t ra[P_UN], rb[P_UN];
-    auto load_panels = [&](int m0) {
+    const int lr = tid / P_TPR, lc = (tid % P_TPR) * P_CPT, lcb = (tid % P_TPR) * B_CPT;
+    double2_t ra[AHEAD][P_UN], rb[AHEAD][B_UN];
+    auto load_panels = [&](int m0, double2_t (&ta)[P_UN], double2_t (&tb)[B_UN]) {
         const double2_t* pa = reinterpret_cast<const double2_t*>(Za + (size_t)(m0 + lr) * lda + lc);
-        const double2_t* pb = reinterpret_cast<const double2_t*>(Zb + (size_t)(m0 + lr) * ldb + lc);
+        const double2_t* pb = reinterpret_cast<const double2_t*>(Zb + (size_t)(m0 + lr) * ldb + lcb);
 #pragma unroll
-        for (int q = 0; q < P_UN; ++q) ra[q] = pa[q];
+        for (int q = 0; q < P_UN; ++q) ta[q] = pa[q];
 #pragma unroll
-        for (int q = 0; q < P_UN; ++q) rb[q] = pb[q];
-    };
-    auto store_panels = [&](int buf) {
-        double2_t* da = reinterpret_cast<double2_t*>(&sm.a[buf][lr][lc]);
-        double2_t* db = reinterpret_cast<double2_t*>(&sm.b[buf][lr][lc]);
-#pragma unroll
-        for (int q = 0; q < P_UN; ++q) da[q] = ra[q];
-#pragma unroll
-        for (int q = 0; q < P_UN; ++q) db[q] = rb[q];
+        for (int q = 0; q < B_UN; ++q) tb[q] = pb[q];
     };
     const int nsteps = depth / PKB;
-    load_panels(0);
-    store_panels(0);
-    __syncthreads();
-#pragma unroll 1
-    for (int step = 0; step < nsteps; ++step) {
-        const int cur = step & 1;
-        if (step + 1 < nsteps) load_panels((step + 1) * PKB);   // in flight during the MFMAs
+    auto one_step = [&](int step, int cur, double2_t (&ta)[P_UN], double2_t (&tb)[B_UN]) {
+        double2_t* da = reinterpret_cast<double2_t*>(&sm.a[cur][lr][lc]);
+        double2_t* db = reinterpret_cast<double2_t*>(&sm.b[cur][lr][lcb]);
+#pragma unroll
+        for (int q = 0; q < P_UN; ++q) da[q] = ta[q];
+#pragma unroll
+        for (int q = 0; q < B_UN; ++q) db[q] = tb[q];
+        __syncthreads();
+        if (step + AHEAD < nsteps) load_panels((step + AHEAD) * PKB, ta, tb);   // in flight during the MFMAs
         if constexpr (MODE == 0) {
 #pragma unroll
             for (int kk = 0; kk < PKB; kk += 4) {
-                double fa[4], fb[2];
+                double fa[P], fb[2];
 #pragma unroll
-                for (int p = 0; p < 4; ++p) fa[p] = sm.a[cur][kk + lk][wi + p * 16 + l16];
+                for (int p = 0; p < P; ++p) fa[p] = sm.a[cur][kk + lk][wi(p) + l16];
 #pragma unroll
                 for (int q = 0; q < 2; ++q) fb[q] = sm.b[cur][kk + lk][wj + q * 16 + l16];
 #pragma unroll
-                for (int p = 0; p < 4; ++p)
+                for (int p = 0; p < P; ++p)
 #pragma unroll
                     for (int q = 0; q < 2; ++q)
                         acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[p], fb[q], acc[p][q], 0, 0, 0);
@@ -478,49 +518,51 @@ __device__ __forceinline__ void tile_product(const double* Za, long long lda, co
 #pragma unroll
                 for (int k = 0; k < 4; ++k) fb[q][k] = sm.b[cur][4 * k + lk][wj + q * 16 + l16];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                if (MODE == TRIANGULAR && step * PKB > wi + p * 16) continue;     // rows of zeros
-                if (!wanted(p, 1)) continue;
+            for (int p = 0; p < P; ++p) {
+                if (step * PKB > wi(p)) continue;                                // rows of zeros
                 double fa[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) fa[k] = sm.a[cur][4 * k + lk][wi + p * 16 + l16];
+                for (int k = 0; k < 4; ++k) fa[k] = sm.a[cur][4 * k + lk][wi(p) + l16];
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    if (!wanted(p, q)) continue;
+                for (int q = 0; q < 2; ++q)
 #pragma unroll
                     for (int k = 0; k < 4; ++k) acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[k], fb[q][k], acc[p][q], 0, 0, 0);
-                }
             }
         }
-        if (step + 1 < nsteps) store_panels(cur ^ 1);
-        __syncthreads();
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) load_panels(u * PKB, ra[u], rb[u]);
+#pragma unroll 1
+    for (int step = 0; step < nsteps; step += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) one_step(step + u, AHEAD == 1 ? step & 1 : u, ra[u], rb[u]);
     }
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int p = 0; p < P; ++p)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            if (!wanted(p, q)) continue;
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                double* c = C + (size_t)(wi + p * 16 + lk + 4 * r) * ldc + wj + q * 16 + l16;
+                double* c = C + (size_t)(wi(p) + lk + 4 * r) * ldc + wj + q * 16 + l16;
                 const double v = sign * acc[p][q][r];
-                // (the sum is left to the memory side: no wait for the old value; every element of C takes
-                // exactly one addition per launch, so the result does not depend on any order)
+                // (the sum is left to the memory side: no wait for the old value; every element of C takes its
+                // additions in one order, so the result does not depend on any)
                 if (overwrite) *c = v;
                 else unsafeAtomicAdd(c, v);
             }
-        }
     __syncthreads();
 }
 
 // every store of the workgroup so far becomes visible to the device, then the flag is set / counted up
+// (one wavefront writes the L2 back, when the stores of all of them have reached it: not 0, which the factorisation that may come next waits
+// for)
 __device__ __forceinline__ void publish(unsigned* flag, unsigned value) {
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == PT / 2) __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void publish_one_more(unsigned* counter) {
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -530,10 +572,11 @@ __device__ __forceinline__ void publish_one_more(unsigned* counter) {
 __device__ __forceinline__ unsigned await(unsigned* flag, unsigned target, unsigned spin_limit, int* info,
                                           unsigned& seen) {
     if (threadIdx.x == 0) {
-        unsigned v = __hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         for (unsigned n = 0; v < target && n < spin_limit; ++n) {
             __builtin_amdgcn_s_sleep(32);
-            v = __hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+            v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((n & 63) == 63 && __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;     // someone has failed
         }
         if (v < target) {
             atomicCAS(info, 0, -1);
@@ -548,19 +591,178 @@ __device__ __forceinline__ unsigned await(unsigned* flag, unsigned target, unsig
     return v;
 }
 
+// A quarter of the tile at C -= Za^T Zb, Za and Zb 128 rows of 128 columns: all loads on the way at once, since the chain of a panel waits for
+// it.  Ends with a barrier.
+__device__ __forceinline__ void quarter_product(const double* Za, const double* Zb, long long ld, double* C, int quarter, TileShared& sm) {
+    constexpr int Q = NB / 2, STAGES = NB / PKB;
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i0 = Q * (quarter >> 1), j0 = Q * (quarter & 1), wi = (wave >> 1) * SB, wj = (wave & 1) * 2 * SB;
+    const int lr = tid / 32, lc = (tid % 32) * 2;
+    double2_t ra[STAGES], rb[STAGES];
+#pragma unroll
+    for (int k = 0; k < STAGES; ++k) {
+        ra[k] = *reinterpret_cast<const double2_t*>(Za + (size_t)(PKB * k + lr) * ld + i0 + lc);
+        rb[k] = *reinterpret_cast<const double2_t*>(Zb + (size_t)(PKB * k + lr) * ld + j0 + lc);
+    }
+    double4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+    for (int k = 0; k < STAGES; ++k) {
+        *reinterpret_cast<double2_t*>(&sm.a[k & 1][lr][lc]) = ra[k];
+        *reinterpret_cast<double2_t*>(&sm.b[k & 1][lr][lc]) = rb[k];
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < PKB; kk += 4) {
+            const double fa = sm.a[k & 1][kk + lk][wi + l16];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa, sm.b[k & 1][kk + lk][wj + q * SB + l16], acc[q], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            unsafeAtomicAdd(C + (size_t)(i0 + wi + lk + 4 * r) * ld + j0 + wj + q * SB + l16, -acc[q][r]);
+    __syncthreads();
+}
+
+struct FollowShared {
+    double us[SB][SSTRIDE];       // block row K of U, right of the diagonal
+    double ts[SB][SSTRIDE];       // block row K of the strip
+    double v[SB][DSTRIDE];        // the inverse of the diagonal sub-block
+};
+
+// The strip T <- U11^-T T of the tile at (k0, j0) and the update of the diagonal tile at (j0, j0), D -= T^T T (on and above its
+// diagonal), step by step beside the factorisation of the block at (k0, k0) on another CU: with block row K of U and the inverse V
+// of its diagonal sub-block, T(K) <- V^T (T(K) - S(K)), S(I) += U(K,I)^T T(K) for I > K, D += T(K)^T T(K).  A wavefront has 16 columns of
+// T and S in the accumulator layout, which is that of both operands, and every eighth sub-block of D.  (S by itself: subtracted from T as
+// it comes, every product would round T; solutions of 256 to 2048 features were off by a tenth more.)
+// Waiting for the whole block instead, then the strip, then the update, put two products of 8 us each and two trips through memory behind
+// each factorisation of the chain.
+// Ends with everything of this workgroup's in memory.  False: the factorisation failed, or the wait ran out (info is then -1).
+__device__ __forceinline__ bool follow_block(double* A, long long ld, int k0, int j0, const double* invT, unsigned* steps,
+                                             unsigned spin_limit, int* info, unsigned& seen, FollowShared& fs) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));      // (or the addresses of all steps are worked out ahead of the caller's loop, and spilled)
+    const int lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int DSLOT = (NSUB + PT / 64 - 1) / (PT / 64);
+    const double* U = A + (size_t)k0 * ld + k0;
+    double* at = A + (size_t)(k0 + lk) * ld + j0 + SB * wave + l16;     // walks down the tile, four rows at a time (and is kept from being
+    auto down = [&](double*& q) {                                       // worked out ahead of the loops, in registers that are not there)
+        q += 4 * ld;
+        asm volatile("" : "+v"(q));
+    };
+    double4_t S[NSB], D[DSLOT];
+    int di[DSLOT], dj[DSLOT];
+#pragma unroll
+    for (int I = 0; I < NSB; ++I) S[I] = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < DSLOT; ++s) {
+        D[s] = (double4_t){0.0, 0.0, 0.0, 0.0};
+        int t = 8 * s + wave, i = 0;
+        while (i < NSB && t >= NSB - i) t -= NSB - i++;
+        di[s] = i;                                                     // NSB: there is none
+        dj[s] = i + t;
+    }
+    const int ur = tid / 32, uc = tid % 32;
+    double nv = 0.0, nu[NB / 32] = {0.0, 0.0, 0.0, 0.0};               // this thread's part of a step on its way from memory
+    auto fetch = [&](auto K_) {
+        constexpr int K = decltype(K_)::value;
+        if (tid < SB * SB) nv = load_past_caches(&invT[(K * SB + tid / SB) * NB + K * SB + tid % SB]);
+#pragma unroll
+        for (int q = (K + 1) * SB / 32; q < NB / 32; ++q)
+            if (uc + 32 * q >= (K + 1) * SB) nu[q] = load_past_caches(&U[(size_t)(K * SB + ur) * ld + uc + 32 * q]);
+    };
+    unsigned there = 0u;                                               // block rows that were there when last looked
+    return static_all<NSB>([&](auto K_) -> bool {
+        constexpr int K = decltype(K_)::value;
+        double4_t rest;                                                // T(K)
+        {
+            double* q = at;
+#pragma unroll
+            for (int r = 0; r < 4; ++r, down(q)) rest[r] = *q;
+        }
+        if (there < K + 1u) {
+            if (tid == 0) {
+                unsigned v = __hip_atomic_load(steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (unsigned n = 0; v < K + 1u && n < spin_limit; ++n) {
+                    __builtin_amdgcn_s_sleep(4);
+                    v = __hip_atomic_load(steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (v < K + 1u) {
+                    atomicCAS(info, 0, -1);
+                    v = FLAG_FAILED;
+                }
+                seen = v;
+            }
+            __syncthreads();
+            there = __builtin_amdgcn_readfirstlane(seen);
+            if (there & FLAG_FAILED) return false;
+            fetch(K_);
+        }
+        if (tid < SB * SB) fs.v[tid % SB][tid / SB] = nv;
+#pragma unroll
+        for (int q = (K + 1) * SB / 32; q < NB / 32; ++q) fs.us[ur][uc + 32 * q] = nu[q];      // (columns left of the diagonal are not read)
+        __syncthreads();
+        if constexpr (K + 1 < NSB) {
+            if (there > K + 1u) fetch(std::integral_constant<int, K + 1>{});       // beside this step's products
+        }
+        rest -= S[K];
+        double4_t res = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) res = __builtin_amdgcn_mfma_f64_16x16x4f64(fs.v[4 * kk + lk][l16], rest[kk], res, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r, down(at)) {
+            fs.ts[lk + 4 * r][SB * wave + l16] = res[r];
+            *at = res[r];
+        }
+#pragma unroll
+        for (int I = K + 1; I < NSB; ++I) {
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                S[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(fs.us[4 * kk + lk][SB * I + l16], res[kk], S[I], 0, 0, 0);
+            if (I % 2 == 0) __builtin_amdgcn_sched_barrier(0);         // (or all operands are read first)
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < DSLOT; ++s)
+            if (di[s] < NSB) {
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+                    D[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(fs.ts[4 * kk + lk][SB * di[s] + l16], fs.ts[4 * kk + lk][SB * dj[s] + l16],
+                                                                D[s], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        if constexpr (K == NSB - 1) {
+#pragma unroll
+            for (int s = 0; s < DSLOT; ++s)
+                if (di[s] < NSB) {
+                    double* c = A + (size_t)(j0 + SB * di[s] + lk) * ld + j0 + SB * dj[s] + l16;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r, down(c)) unsafeAtomicAdd(c, -D[s][r]);
+                }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+        return true;
+    });
+}
+
 // Panel rows [P0, P0 + 128 nblk); [R0, P0) are the rows of the panel before it, whose update the trailing
 // matrix has not had yet (R0 = P0: nothing outstanding).  Workgroup ids: [0, nhead_pad) the tiles of this
 // panel's rows that take that update ("head": column w has min(w, nblk - 1) + 1 of them, columns in order),
 // then nown_pad ids for the column owners, then the tiles of the trailing matrix below this panel, nt per edge
 // (0: none).  flags: FLAGS_PER_PANEL words, then one counter per column (head tiles done), all zero.
-__global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, int F, int R0, int P0, int nblk,
-                                                      int nhead_pad, int nown, int nown_pad, int nt, TileMap tm,
+__global__ __launch_bounds__(PT, 2) void panel_kernel(double* A, long long ld, int F, int R0, int P0, int nblk,
+                                                      int nhead_pad, int sharers, int nown_pad, int nt, TileMap tm,
                                                       double* invs, int* info, unsigned* flags, unsigned spin_limit) {
-    // the tile product and the factorisation never run at the same time: one piece of LDS for both, which
-    // is what lets two workgroups share a CU (2 x 74 KB)
+    // the tile product, the factorisation and the following of one never run at the same time: one piece of LDS for all (74 KB)
     __shared__ __attribute__((aligned(16))) union {
         TileShared tile;
         PotrfShared potrf;
+        FollowShared follow;
     } lds;
     TileShared& sm = lds.tile;
     PotrfShared& ps = lds.potrf;
@@ -581,7 +783,7 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
         }
         const int k0 = P0 + b * NB, j0 = P0 + w * NB;
         if (j0 >= F) return;
-        tile_product(A + (size_t)R0 * ld + k0, ld, A + (size_t)R0 * ld + j0, ld, P0 - R0, A + (size_t)k0 * ld + j0, ld,
+        tile_product<NB>(A + (size_t)R0 * ld + k0, ld, A + (size_t)R0 * ld + j0, ld, P0 - R0, A + (size_t)k0 * ld + j0, ld,
                      -1.0, false, sm);
         publish_one_more(heads_done + w);
         return;
@@ -593,52 +795,86 @@ __global__ __launch_bounds__(PT, 4) void panel_kernel(double* A, long long ld, i
         if (ti < 0 || ti > tj) return;
         const int Q = P0 + nblk * NB;
         const int i0 = Q + ti * NB, c0 = Q + tj * NB;
-        tile_product(A + (size_t)R0 * ld + i0, ld, A + (size_t)R0 * ld + c0, ld, P0 - R0, A + (size_t)i0 * ld + c0, ld,
+        tile_product<NB>(A + (size_t)R0 * ld + i0, ld, A + (size_t)R0 * ld + c0, ld, P0 - R0, A + (size_t)i0 * ld + c0, ld,
                      -1.0, false, sm);
         return;
     }
-    // a column owner: owner o < nblk has column o of the panel, the one with its diagonal tile in it; the others
-    // have every (nown - nblk)-th column right of the panel
-    if (bid >= nown) return;
+    // Quarters of the panel's tiles right of its diagonal ones, whose updates stand between a factorisation of the chain and the next but one:
+    // four workgroups for tile (b, w), 1 <= b < w < nblk.  They come ahead of the other owners, so that they are running while owners wait for them.
+    const int nquarter = 2 * (nblk - 1) * (nblk - 2);
+    if (bid >= nblk && bid < nblk + nquarter) {
+        __builtin_amdgcn_s_setprio(3);                       // (a CU may have other workgroups)
+        int b = 1, w = 2, t = (bid - nblk) >> 2;
+        while (t >= w - 1) t -= w++ - 1;
+        b += t;
+            double* into = A + (size_t)(P0 + b * NB) * ld + P0 + w * NB;
+        for (int l = 0; l < b; ++l) {
+            const double* strips = A + (size_t)(P0 + l * NB) * ld + P0;
+            if (await(flags + PBLK + l * PBLK + b, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
+            if (await(flags + PBLK + l * PBLK + w, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
+            quarter_product(strips + b * NB, strips + w * NB, ld, into, (bid - nblk) & 3, sm);
+            publish_one_more(flags + QUARTERS + b * PBLK + w);
+        }
+        return;
+    }
+    // a column owner: owner o < nblk has column o of the panel, the one with its diagonal tile in it; one or two each (`sharers`) have a
+    // column of tiles right of the panel
     const int ncol = (F - P0) / NB;
-    const int stride = bid < nblk ? ncol : nown - nblk;
+    const int right = bid - nblk - nquarter;                 // of the panel
+    const int w = bid < nblk ? bid : nblk + right / sharers;
+    if (w >= ncol) return;
+    const int j0 = P0 + w * NB + (bid < nblk ? 0 : right % sharers * (NB / 2));
+    const int jend = P0 + w * NB + (bid < nblk || right % sharers == sharers - 1 ? NB : NB / 2);
     const int mine = bid < nblk ? bid : nblk - 1;            // last block row with a tile on or above the diagonal
     if (P0 > R0 && nhead_pad > 0) {
-        for (int w = bid; w < ncol; w += stride)
-            if (await(heads_done + w, (unsigned)(mine + 1), spin_limit, info, seen) == FLAG_FAILED) return;
+        if (await(heads_done + w, (unsigned)(mine + 1), spin_limit, info, seen) == FLAG_FAILED) return;
     } else if (P0 > R0) {                                    // no workgroups for the head tiles: the owner's own work
-        for (int w = bid; w < ncol; w += stride)
-            for (int b = 0; b <= mine; ++b)
-                tile_product(A + (size_t)R0 * ld + P0 + b * NB, ld, A + (size_t)R0 * ld + P0 + w * NB, ld, P0 - R0,
-                             A + (size_t)(P0 + b * NB) * ld + P0 + w * NB, ld, -1.0, false, sm);
+        for (int b = 0; b <= mine; ++b) {
+            const double* above = A + (size_t)R0 * ld;
+            double* into = A + (size_t)(P0 + b * NB) * ld + j0;
+            if (jend - j0 == NB) tile_product<NB>(above + P0 + b * NB, ld, above + j0, ld, P0 - R0, into, ld, -1.0, false, sm);
+            else tile_product<NB / 2>(above + P0 + b * NB, ld, above + j0, ld, P0 - R0, into, ld, -1.0, false, sm);
+        }
     }
-    unsigned strips_seen = 0u;                               // "strip (l, b) done" flags this workgroup has seen set
+    if (bid < nblk) {                                        // the panel's own columns, which the chain is waiting for
+        __builtin_amdgcn_s_setprio(3);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+#pragma unroll 1
+        for (int l = 0; l < bid; ++l) {
+            const int k0 = P0 + l * NB;
+            if (l > 0) {                                      // the tile has had its updates by the strips above
+                if (await(flags + QUARTERS + l * PBLK + bid, 4u * l, spin_limit, info, seen) == FLAG_FAILED) return;
+            }
+            unsigned* strip_done = flags + PBLK + l * PBLK + bid;
+            if (!follow_block(A, ld, k0, j0, invs + ((size_t)(k0 / NB) * 2 + 1) * NB * NB, flags + STEPS + l, spin_limit, info, seen,
+                              lds.follow)) {
+                if (threadIdx.x == 0) store_past_caches(strip_done, FLAG_FAILED);
+                return;
+            }
+            publish(strip_done, FLAG_DONE);
+        }
+        double* inv = invs + (size_t)(j0 / NB) * 2 * NB * NB;     // the own diagonal tile: every update is in
+        const bool ok = potrf_block(A, ld, j0, NB, inv, inv + NB * NB, info, flags + STEPS + bid, ps);
+        // on failure every workgroup right of this column leaves at one of these flags, before it could wait for
+        // anything that is now never set
+        if (!ok && threadIdx.x == 0) store_past_caches(flags + STEPS + bid, FLAG_FAILED);
+        publish(flags + bid, ok ? FLAG_DONE : FLAG_FAILED);
+        return;
+    }
     for (int l = 0; l < nblk; ++l) {
         const int k0 = P0 + l * NB;
-        double* inv = invs + (size_t)(k0 / NB) * 2 * NB * NB;
-        if (l == bid) {                                      // the own diagonal tile: every update is in
-            const bool ok = potrf_block(A, ld, k0, NB, inv, inv + NB * NB, info, ps);
-            // on failure every workgroup right of this column leaves at this flag, before it could wait for
-            // anything that is now never set
-            publish(flags + l, ok ? FLAG_DONE : FLAG_FAILED);
-            return;
-        }
+        const double* inv = invs + (size_t)(k0 / NB) * 2 * NB * NB;
         if (await(flags + l, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
-        for (int w = bid; w < ncol; w += stride) {
-            const int j0 = P0 + w * NB;                      // first column of the owned tiles
-            double* tile = A + (size_t)k0 * ld + j0;
-            tile_product<TRIANGULAR>(inv, NB, tile, ld, NB, tile, ld, 1.0, true, sm);
-            if (bid < nblk) publish(flags + PBLK + l * PBLK + bid, FLAG_DONE);
-            for (int b = l + 1; b <= mine; ++b) {
-                const unsigned bit = 1u << (l * PBLK + b);
-                if (b != bid && !(strips_seen & bit)) {
-                    if (await(flags + PBLK + l * PBLK + b, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
-                    strips_seen |= bit;
-                }
-                double* into = A + (size_t)(P0 + b * NB) * ld + j0;
-                if (b == bid) tile_product<DIAGONAL>(tile, ld, tile, ld, NB, into, ld, -1.0, false, sm);
-                else tile_product(A + (size_t)k0 * ld + P0 + b * NB, ld, tile, ld, NB, into, ld, -1.0, false, sm);
-            }
+        for (int j = j0; j < jend; j += NB / 2) {
+            double* tile = A + (size_t)k0 * ld + j;
+            tile_product<NB / 2, TRIANGULAR>(inv, NB, tile, ld, NB, tile, ld, 1.0, true, sm);
+        }
+        for (int b = l + 1; b < nblk; ++b) {
+            if (await(flags + PBLK + l * PBLK + b, FLAG_DONE, spin_limit, info, seen) != FLAG_DONE) return;
+            const double* strip = A + (size_t)k0 * ld + P0 + b * NB;
+            if (jend - j0 == NB) tile_product<NB>(strip, ld, A + (size_t)k0 * ld + j0, ld, NB, A + (size_t)(P0 + b * NB) * ld + j0, ld, -1.0, false, sm);
+            else tile_product<NB / 2>(strip, ld, A + (size_t)k0 * ld + j0, ld, NB, A + (size_t)(P0 + b * NB) * ld + j0, ld, -1.0, false, sm);
         }
     }
 }
@@ -809,7 +1045,7 @@ namespace {
 // the matrix is read and written once per slab and not once per panel.  In the last 4096 rows the panel launches of fp64 products
 // are as fast, which are short there and wait for their chain of factorisations.  Up to 12288 rows a slab (15 bytes an entry
 // for the residues, 3 GB at 16384 features); below 7168 features there is nothing to gain.  ms without slabs and with, taken when a
-// block of the chain took 65 us (62 now, on both sides):
+// block of the chain took 65 us (44 now, on both sides):
 // 24576 features 90.3 / 54.4, 16384 31.6 / 23.0, 12288 16.2 / 13.8, 10240 11.3 / 10.3, 8192 7.6 / 7.3, 7168 6.1 / 6.0; a rest of 6144
 // rows 23.4 at 16384 and 10.6 at 10240, of 3072 rows 23.1 and 10.3.
 constexpr int SLAB = 12288, SLAB_REST = 4096, SLAB_LEAST = 3072;
@@ -938,7 +1174,6 @@ extern "C" int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* wor
             const int nblk = (pend - P0) / NB;
             const int ncol = (F - P0) / NB;                   // columns of tiles from the panel's first to the last
             const int nt = P0 > R0 ? (F - pend) / NB : 0;
-            const int nown = ncol;
             // The head tiles (this panel's rows of the update of the panel before) go to workgroups of their own
             // once the trailing matrix is small, where a launch lasts as long as its slowest owner, which has four head
             // tiles and ten strip / update products in a row (16384 features 22.9 ms without, 21.8 so; 8192 8.15 and 7.09;
@@ -946,7 +1181,11 @@ extern "C" int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* wor
             // While the trailing tiles keep the chip busy for longer than that, the owners take their head tiles
             // themselves and no slot waits for another.
             const bool split_heads = P0 > R0 && nt <= SPLIT_HEADS_BELOW;
-            const int nown_pad = (nown + NXCD - 1) / NXCD * NXCD;
+            // Two workgroups to a column of tiles right of the panel while all of them have a CU, since the launch lasts as long as a column's
+            // four strips and six updates (640 features 372 -> 315 us, 4096 2.54 -> 2.19 ms); with more they would come one after the other.
+            const int nchain = nblk + 2 * (nblk - 1) * (nblk - 2);            // the panel's own columns and their quarter tiles
+            const int sharers = nchain + 2 * (ncol - nblk) <= CUS ? 2 : 1;
+            const int nown_pad = (nchain + sharers * (ncol - nblk) + NXCD - 1) / NXCD * NXCD;
             const int nhead = split_heads ? nblk * (nblk + 1) / 2 + (ncol - nblk) * nblk : 0;
             const int nhead_pad = (nhead + NXCD - 1) / NXCD * NXCD;
             long long per_xcd = 0;
@@ -954,7 +1193,7 @@ extern "C" int qmll_cholesky_slabs_f64(double* A, int F, long long ld, void* wor
             const long long grid = (long long)nhead_pad + nown_pad + (nt > 0 ? per_xcd * NXCD : 0);
             QMLL_REQUIRE(grid < 2147483647LL, QMLL_ERR_INVALID, "qmll_cholesky_f64: too many tiles");
             hipLaunchKernelGGL(panel_kernel, dim3((unsigned)grid), dim3(PT), 0, stream, A, ld, F, R0, P0, nblk, nhead_pad,
-                               nown, nown_pad, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
+                               sharers, nown_pad, nt, tm, invs, info, flags + (size_t)(P0 / OB) * per_panel, SPIN_LIMIT);
             QMLL_CHECK_LAUNCH("qmll_cholesky_f64");
         }
         return QMLL_OK;
