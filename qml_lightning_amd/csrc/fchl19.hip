@@ -893,24 +893,17 @@ __device__ __forceinline__ void prepare_group(const FchlArgs& a, const BatchPrep
     for (int k = start + lane; k < b.A; k += QMLL_WAVE) b.sorted[k] = 0;
 }
 
-// PREP: the first groups of the launch prepare the batch, the atoms' workgroups take the elements from the charges (no launch ahead of
-// this one has written the types).
-template <int NS, bool PREP>
-__global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, BatchPrep b, float* __restrict__ rep) {
+// what a wavefront wrote to LDS is there for its own lanes: LDS takes a wavefront's instructions in order
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One wavefront writes atom i's row to `out`; FROM_CHARGES: the elements are taken from the charges.  sync: what makes the wavefront's LDS writes
+// visible to itself.
+template <int NS, bool FROM_CHARGES, class Sync>
+__device__ __forceinline__ void lean_forward(const FchlArgs& a, const BatchPrep& b, int m, int i, int lane, float* smem, float* out, Sync sync) {
     constexpr int NP = NS * (NS + 1) / 2;
-    extern __shared__ float smem[];
-    const int lane = threadIdx.x;
-    int atom = blockIdx.x;
-    if constexpr (PREP) {
-        if (atom < b.groups) {
-            prepare_group(a, b, atom, lane, reinterpret_cast<int*>(smem));
-            return;
-        }
-        atom -= b.groups;
-    }
-    const int m = a.molIDs[atom];
-    const int i = a.atomIDs[atom];
-    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
     const int nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
     float* recA = smem;                                  // [cap][4]: d_ij, 1 / r
     float* recB = recA + 4 * a.cap;                      // [cap][4]: sk3 r / 2, fc r^-d3, places (below)
@@ -919,7 +912,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
     const float* Xm = a.X + (size_t)m * a.n * 3;
     const int own = lane < a.n ? lane : 0;
     const float xj = Xm[own * 3 + 0], yj = Xm[own * 3 + 1], zj = Xm[own * 3 + 2];
-    const int et = PREP ? species_index(b.Z[(size_t)m * a.n + own], b.species, NS) : a.types[(size_t)m * a.n + own];
+    const int et = FROM_CHARGES ? species_index(b.Z[(size_t)m * a.n + own], b.species, NS) : a.types[(size_t)m * a.n + own];
     const int z = lane & 31, half = lane >> 5;           // two-body: radial bin, neighbour of two
     const float rs2v = z < nRs2 ? a.Rs2[z] : 1.0f;
     const int slot = idiv_small(lane, LEAN_LANES), ll = lane - LEAN_LANES * slot;      // three-body: triple of six, pair of bins
@@ -990,9 +983,8 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
         f2[1] = 0.5f * LOG2E * frcp(s2);
         f2[2] = frsq(s2) * 0.3989422804014327f * fexp2(-a.p.two_body_decay * l2r) * fc;
     }
-    __syncthreads();
+    sync();
 
-    float* out = rep + ((size_t)m * a.n + i) * (NS * nRs2 + 2 * NP * nRs3);
     // ---- two-body blocks ----
     {
         const float lnRs = flog(rs2v), invRs = frcp(rs2v);
@@ -1015,7 +1007,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             if (lane < nRs2) out[e * nRs2 + lane] = acc;
         }
     }
-    __syncthreads();
+    sync();
 
     // ---- the table ----
     {
@@ -1036,7 +1028,7 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             __builtin_memcpy(trip + 3 * at, &w, sizeof w);
         }
     }
-    __syncthreads();
+    sync();
 
     // ---- three-body blocks ----
     const float rsa = sk3 * rs3a, rsb = sk3 * rs3b;
@@ -1088,6 +1080,109 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
             if (2 * ll + 1 < nRs3) __builtin_memcpy(to, &o, 16);
             else if (2 * ll < nRs3) __builtin_memcpy(to, &o, 8);
         }
+    }
+}
+
+// PREP: the first groups of the launch prepare the batch, the atoms' workgroups take the elements from the charges (no launch ahead of
+// this one has written the types).
+template <int NS, bool PREP>
+__global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, BatchPrep b, float* __restrict__ rep) {
+    extern __shared__ float smem[];
+    const int lane = threadIdx.x;
+    int atom = blockIdx.x;
+    if constexpr (PREP) {
+        if (atom < b.groups) {
+            prepare_group(a, b, atom, lane, reinterpret_cast<int*>(smem));
+            return;
+        }
+        atom -= b.groups;
+    }
+    const int m = a.molIDs[atom];
+    const int i = a.atomIDs[atom];
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    const int R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
+    lean_forward<NS, PREP>(a, b, m, i, lane, smem, rep + ((size_t)m * a.n + i) * R, [] { __syncthreads(); });
+}
+
+// The representation of few atoms and its projection in one launch, beside the preparation of the batch: a workgroup per atom, whose first
+// wavefront forms the row in LDS while the reductor's rows are on their way into the registers of all eight and the others count
+// the atom's place in the sorted list.  x[place, :] = row . U.  21 atoms of three elements, 128 components: 6.5 + 4.3 us in two launches, 9.6 so,
+// and 4 us of the host's time for the launch.
+constexpr int FP_WAVES = 8;
+// rows of a reductor that the registers of eight wavefronts hold beside the rest, in both directions: five elements of the default grids at
+// 64 components, four at 128
+constexpr int held_rows(int d) { return d == 64 ? 768 : 512; }
+template <int NS, int D>
+__global__ __launch_bounds__(64 * FP_WAVES) void fchl19_forward_projected_kernel(FchlArgs a, BatchPrep b, const float* __restrict__ reductors,
+                                                                                 float* __restrict__ x) {
+    extern __shared__ float smem[];
+    constexpr int CL = D / 4, KS = 64 * FP_WAVES / CL, MINE = held_rows(D) / KS; // lanes along the columns, slices of the rows, rows of each
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x < b.groups) {
+        if (wave == 0) prepare_group(a, b, blockIdx.x, lane, reinterpret_cast<int*>(smem));
+        return;
+    }
+    const int atom = blockIdx.x - b.groups, R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
+    const float* list = b.model_species ? b.model_species : b.species;
+    const int nlist = b.model_species ? b.ne : a.p.nspecies;
+    // element of a listed atom by the model's list, as prepare_group has it; -1: not in the sorted list
+    auto element = [&](int at) {
+        const int m = a.molIDs[at], i = a.atomIDs[at];
+        if (m < 0 || m >= a.B || i < 0 || i >= a.n) return -1;
+        return i < a.natoms[m] ? species_index(b.Z[(size_t)m * a.n + i], list, nlist) : 0;
+    };
+    const int m = a.molIDs[atom], i = a.atomIDs[atom];
+    const int e = __builtin_amdgcn_readfirstlane(element(atom));
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n || e < 0 || e >= b.ne) return;
+    float* row = smem;                                   // [R4] the representation
+    float* part = row + ((R + 3) & ~3);                  // [FP_WAVES][D]
+    int* before = reinterpret_cast<int*>(part + FP_WAVES * D);           // [PREP_ATOMS / 64]
+    float* own = reinterpret_cast<float*>(before + PREP_ATOMS / 64);
+    const int c4 = tid % CL, ks = tid / CL;
+    const float4* U = reinterpret_cast<const float4*>(reductors + (size_t)e * R * D) + c4;
+    float4 u[MINE];
+#pragma unroll
+    for (int k = 0; k < MINE; ++k) {
+        u[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (KS * k < R) u[k] = U[(size_t)min(ks + KS * k, R - 1) * CL];
+    }
+    if (wave == 0) {
+        lean_forward<NS, true>(a, b, m, i, lane, own, row, [] { wave_sync(); });
+    } else if (wave <= PREP_ATOMS / 64) {                // the atoms ahead of this one in the sorted list
+        const int at = tid - 64;
+        const int t = at < b.A ? element(at) : -1;
+        const int count = __popcll(__ballot(t >= 0 && (t < e || (t == e && at < atom))));
+        if (lane == 0) before[wave - 1] = count;
+    }
+    __syncthreads();
+    float4 sums[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+#pragma unroll
+    for (int k = 0; k < MINE; ++k) {
+        if (KS * k >= R) break;
+        const float r = ks + KS * k < R ? row[ks + KS * k] : 0.0f;
+        float4& t = sums[k & 1];
+        t.x = fmaf(r, u[k].x, t.x);
+        t.y = fmaf(r, u[k].y, t.y);
+        t.z = fmaf(r, u[k].z, t.z);
+        t.w = fmaf(r, u[k].w, t.w);
+    }
+    float4 acc = make_float4(sums[0].x + sums[1].x, sums[0].y + sums[1].y, sums[0].z + sums[1].z, sums[0].w + sums[1].w);
+    float* v = &acc.x;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if constexpr (CL == 16) v[c] += lane_xor<16>(v[c]);
+        v[c] += lane_xor<32>(v[c]);
+    }
+    if (lane < CL) reinterpret_cast<float4*>(part)[wave * CL + lane] = acc;
+    __syncthreads();
+    if (tid < D) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < FP_WAVES; ++w) sum += part[w * D + tid];
+        int place = 0;
+#pragma unroll
+        for (int w = 0; w < PREP_ATOMS / 64; ++w) place += before[w];
+        x[(size_t)place * D + tid] = sum;
     }
 }
 
@@ -1746,23 +1841,24 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
 // (before the bins were taken in groups).  86016 atoms of 21, three elements 193 -> 165 us, 131235 atoms of 3 to 29, five elements
 // 342 -> 290, 64000 of 8 89 -> 63, 80000 of 40 476 -> 446.  Vector issue takes five sixths of the launch.
 // ---------------------------------------------------------------------------------
-template <int NS>
-__global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const float* __restrict__ grad_rep, float* __restrict__ grad_X) {
+// NW > 1: the wavefronts of the workgroup share the triples (and have copies of the forces each); gradient() is then called, by all of them,
+// when the neighbours are staged, and returns the atom's row of the incoming gradient.
+template <int NS, int NW, class Gradient>
+__device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float* smem, Gradient&& gradient, float* __restrict__ grad_X) {
     constexpr int NP = NS * (NS + 1) / 2;
     constexpr int STEP = 3 * LEAN_RS3;                   // entries of the gradient's three-body part per load of the wavefront
-    extern __shared__ float smem[];
-    const int lane = threadIdx.x;
-    const int m = a.molIDs[blockIdx.x];
-    const int i = a.atomIDs[blockIdx.x];
-    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    constexpr bool ONE = NW == 1;
+    const int lane = ONE ? threadIdx.x : threadIdx.x & 63, wave = ONE ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nRs2 = a.p.nRs2, nRs3 = a.p.nRs3;
     float* recA = smem;                                  // [cap][4]: d_ij, r
     float* recB = recA + 4 * a.cap;                      // [cap][4]: 1 / r, fc, dfc / dr, the type's pairs (below)
-    float* force = recB + 4 * a.cap;                     // [tcap][4] forces on the neighbours, in copies
-    float* gin3 = force + 4 * a.tcap;                    // [NP][LEAN_RS3][2] incoming gradient of the three-body bins
+    float* force = recB + 4 * a.cap;                     // [NW][tcap][4] forces on the neighbours, in copies
+    float* gin3 = force + 4 * NW * a.tcap;               // [NP][LEAN_RS3][2] incoming gradient of the three-body bins
     float* gin2 = gin3 + 2 * NP * LEAN_RS3;              // [NS][32] and of the two-body ones, each divided by its Rs2
     float* slnRs2 = gin2 + 32 * NS;                      // [32]
     int* sj = (int*)(slnRs2 + 32);                       // [cap] atom index of neighbour j
+    float* own_force = reinterpret_cast<float*>(sj + a.cap);       // NW > 1: [NW][3], what the wavefronts have for atom i itself
+    float* mine = force + 4 * wave * a.tcap;
 
     const float* Xm = a.X + (size_t)m * a.n * 3;
     const int own = lane < a.n ? lane : 0;
@@ -1775,20 +1871,21 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
     const int third = idiv_small(lane, LEAN_RS3), l3 = lane - LEAN_RS3 * third;
     const bool bin_ok = lane < STEP && l3 < nRs3;
     const float rs3v = bin_ok ? a.Rs3[l3] : 0.0f;
-    const float* gsrc = grad_rep + ((size_t)m * a.n + i) * (NS * nRs2 + 2 * NP * nRs3);
+    const float* gsrc = nullptr;
+    if constexpr (ONE) gsrc = gradient();
     float g2[(NS + 1) / 2];
 #pragma unroll
     for (int k = 0; k < (NS + 1) / 2; ++k) {
         const int e = 2 * k + (lane >> 5);
-        g2[k] = e < NS && z < nRs2 ? gsrc[e * nRs2 + z] : 0.0f;
+        g2[k] = ONE && e < NS && z < nRs2 ? gsrc[e * nRs2 + z] : 0.0f;
     }
     float2 g3[(NP + 2) / 3];
 #pragma unroll
     for (int k = 0; k < (NP + 2) / 3; ++k) {
         g3[k] = make_float2(0.f, 0.f);
-        if (bin_ok && 3 * k + third < NP) __builtin_memcpy(&g3[k], gsrc + NS * nRs2 + 2 * ((3 * k + third) * nRs3 + l3), 8);
+        if (ONE && bin_ok && 3 * k + third < NP) __builtin_memcpy(&g3[k], gsrc + NS * nRs2 + 2 * ((3 * k + third) * nRs3 + l3), 8);
     }
-    for (int t = lane; t < a.tcap; t += QMLL_WAVE) reinterpret_cast<float4*>(force)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int t = lane; t < a.tcap; t += QMLL_WAVE) reinterpret_cast<float4*>(mine)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
 
     const float inv_rc = frcp(a.p.rcut);
     const float sk3 = fsqrt(a.p.eta3 * LOG2E);
@@ -1821,7 +1918,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         }
         nn += __popcll(mask);
     }
-    if (near) {
+    if (near && wave == 0) {
         const float ir = __builtin_amdgcn_rsqf(r2), r = root(r2, ir);
         float fc, dfc;
         cutoff(r, inv_rc, fc, dfc);
@@ -1830,7 +1927,17 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         sj[pos] = lane;
     }
     // the incoming gradient, times the constant factor of its bin
-    {
+    if constexpr (!ONE) {
+        gsrc = gradient();
+        const float f2 = a.gscale * frcp(rs2v), f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
+        if (wave == 0 && lane < 32) slnRs2[lane] = flog(rs2v);
+        for (int e = 2 * wave + (lane >> 5); e < NS; e += 2 * NW) gin2[32 * e + z] = z < nRs2 ? gsrc[e * nRs2 + z] * f2 : 0.0f;
+        for (int pq = 3 * wave + third; pq < NP; pq += 3 * NW) {
+            float2 g = make_float2(0.f, 0.f);
+            if (bin_ok) g = make_float2(gsrc[NS * nRs2 + 2 * (pq * nRs3 + l3)] * f3, gsrc[NS * nRs2 + 2 * (pq * nRs3 + l3) + 1] * f3);
+            if (lane < STEP) reinterpret_cast<float2*>(gin3)[LEAN_RS3 * pq + l3] = g;
+        }
+    } else {
         const float f2 = a.gscale * frcp(rs2v), f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
         if (lane < 32) slnRs2[lane] = flog(rs2v);
 #pragma unroll
@@ -1847,7 +1954,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
     float gix = 0.0f, giy = 0.0f, giz = 0.0f;
 
     // ---- two-body: lanes = (bin group, neighbour); see fchl19_vjp_kernel ----
-    {
+    if (wave == 0) {
         const int G = nn > 0 ? idiv_small(64, nn) : 1;       // nn < 64
         const int g = G > 1 ? idiv_small(lane, nn) : 0, j = lane - g * nn;
         const bool active = g < G && j < nn;
@@ -1879,10 +1986,10 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
             gix = tot * ux;
             giy = tot * uy;
             giz = tot * uz;
-            reinterpret_cast<float4*>(force)[j] = make_float4(-tot * ux, -tot * uy, -tot * uz, 0.0f);
+            reinterpret_cast<float4*>(mine)[j] = make_float4(-tot * ux, -tot * uy, -tot * uz, 0.0f);
         }
     }
-    __syncthreads();
+    if constexpr (ONE) __syncthreads();                  // (the others have copies of their own)
 
     // ---- three-body: lane = triple; see fchl19_vjp_kernel for the numbering, the copies and the formulas ----
     float us[LEAN_RS3], ratio[LEAN_RS3 / RS3_GROUP];     // the grid, on scalar registers
@@ -1904,14 +2011,14 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         f.z += z;
         *reinterpret_cast<float4*>(p) = f;
     };
-    for (int t0 = 0; t0 < ntrip; t0 += QMLL_WAVE) {
+    for (int t0 = QMLL_WAVE * wave; t0 < ntrip; t0 += QMLL_WAVE * NW) {
         const int tt = t0 + lane;
         if (tt >= ntrip) break;
         const int s0 = __builtin_amdgcn_readfirstlane((int)(((float)t0 + 0.5f) * inn));
         const int s = (int)(((float)tt + 0.5f) * inn), j = tt - __mul24(s, nn);
         int k = j + s + 1;
         if (k >= nn) k -= nn;
-        float* copy = force + 4 * __mul24(s - s0, nn);
+        float* copy = mine + 4 * __mul24(s - s0, nn);
         const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
         const float ia = Bj.x, ib = Bk.x;
         const float cx = Ak.x - Aj.x, cy = Ak.y - Aj.y, cz = Ak.z - Aj.z;
@@ -1985,23 +2092,121 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
         add_force(copy + 4 * k, fmaf(-ec, cx, -eb * Ak.x), fmaf(-ec, cy, -eb * Ak.y), fmaf(-ec, cz, -eb * Ak.z));
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __syncthreads();
+    if constexpr (ONE) __syncthreads();
     gix = wave_sum(gix);
     giy = wave_sum(giy);
     giz = wave_sum(giz);
+    if constexpr (!ONE) {
+        if (lane == 0) own_force[3 * wave] = gix, own_force[3 * wave + 1] = giy, own_force[3 * wave + 2] = giz;
+        __syncthreads();
+    }
     float* gm = grad_X + (size_t)m * a.n * 3;
     const int ncopies = force_copies(nn);
-    for (int it = lane; it < 3 * (nn + 1); it += QMLL_WAVE) {
+    const int busy = ONE ? 1 : min(NW, max(1, (ntrip + QMLL_WAVE - 1) / QMLL_WAVE));      // wavefronts that have had triples, or the two-body part
+    for (int it = ONE ? lane : threadIdx.x; it < 3 * (nn + 1); it += QMLL_WAVE * NW) {
         const int x = idiv_small(it, 3), c = it - 3 * x;
         float sum = c == 0 ? gix : c == 1 ? giy : giz;   // on atom i itself
         int to = i;
         if (x < nn) {
             to = sj[x];
             sum = 0.0f;
-            for (int q = 0; q < ncopies; ++q) sum += force[4 * (q * nn + x) + c];
+            for (int w = 0; w < busy; ++w)
+                for (int q = 0; q < ncopies; ++q) sum += force[4 * (w * a.tcap + q * nn + x) + c];
+        } else if (!ONE) {
+            sum = 0.0f;
+            for (int w = 0; w < busy; ++w) sum += own_force[3 * w + c];
         }
         atomicAdd(&gm[to * 3 + c], sum);
     }
+}
+
+template <int NS>
+__global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const float* __restrict__ grad_rep, float* __restrict__ grad_X) {
+    extern __shared__ float smem[];
+    const int m = a.molIDs[blockIdx.x];
+    const int i = a.atomIDs[blockIdx.x];
+    if (m < 0 || m >= a.B || i < 0 || i >= a.n) return;   // malformed index: write nothing
+    const int R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
+    lean_vjp<NS, 1>(a, m, i, smem, [&] { return grad_rep + ((size_t)m * a.n + i) * R; }, grad_X);
+}
+
+// The backward projection and the VJP of few atoms in one launch: a workgroup per atom (in sorted order) forms its row of the
+// representation's gradient in LDS, g_rep = sum of the parts of gx . U^T, four lanes to an entry, and takes it from there.  Both
+// were chains of latencies in launches of their own; here the reductor's rows are on their way while the neighbours are staged, and the
+// triples are shared by eight wavefronts.  Workgroups behind the atoms sum the energies of eight molecules each.  21 atoms, 128
+// components: 4.1 + 7.2 us, 8.3 so.  With the forward pair (above) energies and forces of 1 x 21 atoms take 21.3 us (28.5), 12 x 21 25.4 (30.7),
+// 8 x 29 26.0 (32.1), 20 x 12 at 64 components 21.0 (26.2).  Beyond 256 atoms the workgroups, a CU each, come in rounds: 16 x 21 41.7 (37.7); with rows
+// read in several pieces (five elements or 256 components) the pieces wait for memory: 2 x 29, five elements, 128 components 34.4 (32.9).
+struct ProjectedGradient {
+    const float* gx;              // [nparts][A][d]
+    int nparts;
+    const int* sorted_slots;
+    const int* type_offsets;
+    const float* reductors;       // [ne][R][d]
+    int ne, A;
+    const float* e_slots;         // [nparts][B n]
+    float* energies;              // or null
+};
+constexpr int PV_WAVES = 8, PV_ATOMS = 256;      // (a workgroup has a CU to itself)
+template <int NS, int D>
+__global__ __launch_bounds__(64 * PV_WAVES) void fchl19_projected_vjp_kernel(FchlArgs a, ProjectedGradient pg, float* __restrict__ grad_X) {
+    extern __shared__ float smem[];
+    constexpr int NT = 64 * PV_WAVES, ROWS = NT / 4, KQ = D / 16, AHEAD = held_rows(D) / ROWS;
+    const int tid = threadIdx.x, R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
+    const int pos = blockIdx.x;
+    if (pos >= pg.A) {                                   // energies: a wavefront per molecule
+        const int mol = (pos - pg.A) * PV_WAVES + (tid >> 6), lane = tid & 63;
+        if (mol >= a.B) return;
+        float acc = 0.0f;
+        for (int t = lane; t < pg.nparts * a.n; t += 64) {
+            const int part = t / a.n;
+            acc += pg.e_slots[((size_t)part * a.B + mol) * a.n + (t - part * a.n)];
+        }
+        acc = wave_sum(acc);
+        if (lane == 0) pg.energies[mol] = acc;
+        return;
+    }
+    if (pos >= pg.type_offsets[pg.ne]) return;           // atoms of elements that the model does not know come last and have no gradient
+    int e = 0;
+    while (e + 1 < pg.ne && pos >= pg.type_offsets[e + 1]) ++e;
+    const float* U = pg.reductors + (size_t)e * R * D;
+    const int q = tid & 3, r0 = tid >> 2;
+    float4 u[AHEAD][KQ];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+        for (int c = 0; c < KQ; ++c) {
+            u[j][c] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (ROWS * j < R) u[j][c] = reinterpret_cast<const float4*>(U + (size_t)min(r0 + ROWS * j, R - 1) * D)[q + 4 * c];
+        }
+    float v = 0.0f;
+    if (tid < D) {
+        const float* g = pg.gx + (size_t)pos * D + tid;
+#pragma unroll 12
+        for (int k = 0; k < pg.nparts; ++k) v += g[(size_t)k * pg.A * D];
+    }
+    const int slot = pg.sorted_slots[pos], m = slot / a.n, i = slot - m * a.n;
+    float* sg = smem;                                    // [D] gx
+    float* row = sg + D;                                 // [R4] g_rep
+    lean_vjp<NS, PV_WAVES>(a, m, i, row + ((R + 3) & ~3), [&]() -> const float* {
+        if (tid < D) sg[tid] = v;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            if (ROWS * j >= R) break;
+            float sum = 0.0f;
+#pragma unroll
+            for (int c = 0; c < KQ; ++c) {
+                const float4 g = reinterpret_cast<const float4*>(sg)[q + 4 * c];
+                sum = fmaf(u[j][c].x, g.x, fmaf(u[j][c].y, g.y, fmaf(u[j][c].z, g.z, fmaf(u[j][c].w, g.w, sum))));
+            }
+            sum += lane_xor<1>(sum);
+            sum += lane_xor<2>(sum);
+            if (q == 0 && r0 + ROWS * j < R) row[r0 + ROWS * j] = sum;
+        }
+        __syncthreads();
+        return row;
+    }, grad_X);
 }
 
 // ---------------------------------------------------------------------------------
@@ -2018,11 +2223,6 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
 // the table each item recomputes its triple, nRs3 times over and again in the neighbour passes.
 constexpr int JT = 20;   // rho, bin offset, 6 alpha, 2 beta, u_ij, u_ik, u_jk, pad
 constexpr int JW_MOST = 4;       // wavefronts per central atom
-// what a wavefront wrote to LDS is there for its own lanes: LDS takes a wavefront's instructions in order
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 template <bool TABLE>
 __global__ __launch_bounds__(64 * JW_MOST) void fchl19_jacobian_kernel(FchlArgs a, float* __restrict__ rep,
                                                               float* __restrict__ jac, int all_rows) {
@@ -2491,6 +2691,21 @@ extern "C" int qmll_fchl19_forward(const float* X, const int* types, const float
                    stream);
 }
 
+// Where the batch can be prepared beside the representation.  One launch less and the bookkeeping beside the representation instead of ahead
+// of it, where one wavefront does the sort before the atoms are done: energies and forces of 21 atoms 29.0 -> 26.0 us, 12 x 21 32.6 -> 29.4,
+// 16 x 29 46.2 -> 43.3, but 42 x 12 (504 atoms) 29.0 -> 29.8 and 100 x 12 37.4 -> 45.3.
+static bool prepared_beside(int A, long long slots, size_t zero_count, int ne, int n, const qmll_fchl_params* prm) {
+    const long long maxnn = n > 1 ? n - 1 : 1, triples = maxnn * (maxnn - 1) / 2;
+    return A > 0 && A <= PREP_ATOMS && slots > 0 && slots <= 32 * PREP_ATOMS && zero_count <= 128 * PREP_ATOMS && ne > 0 && ne <= PREP_ELEMENTS &&
+           lean_grids(prm, nullptr, n) && wavefronts_forward(A, triples, triples > TCH_MAX, true) == 1;
+}
+static BatchPrep prep_of(const float* Z, const float* species, const float* model_species, int ne, int A, long long slots, int* types,
+                         int* sort_types, int* sorted_slots, int* type_offsets, float* zero, size_t zero_count) {
+    const long long work = std::max<long long>(slots, (long long)zero_count);
+    return BatchPrep{Z, species, model_species, ne, A, (int)slots, types, sort_types, sorted_slots, type_offsets, zero, (int)zero_count,
+                     1 + (int)((work + 255) / 256)};
+}
+
 extern "C" int qmll_prepare_fchl19_forward(const float* X, const float* Z, const float* species, const float* model_species, int ne,
                                            const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
                                            const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
@@ -2498,24 +2713,71 @@ extern "C" int qmll_prepare_fchl19_forward(const float* X, const float* Z, const
                                            int* sort_types, int* sorted_slots, int* type_offsets, float* zero, size_t zero_count,
                                            float* rep, qmll_stream_t stream) {
     QMLL_REQUIRE(prm != nullptr, QMLL_ERR_INVALID, "qmll_prepare_fchl19_forward: null params");
-    const long long slots = (long long)B * n, maxnn = n > 1 ? n - 1 : 1, triples = maxnn * (maxnn - 1) / 2;
-    // One launch less and the bookkeeping beside the representation instead of ahead of it, where one wavefront does the sort before
-    // the atoms are done: energies and forces of 21 atoms 29.0 -> 26.0 us, 12 x 21 32.6 -> 29.4, 16 x 29 46.2 -> 43.3, but 42 x 12 (504
-    // atoms) 29.0 -> 29.8 and 100 x 12 37.4 -> 45.3.
+    const long long slots = (long long)B * n;
     BatchPrep b{};
-    if (A > 0 && A <= PREP_ATOMS && slots > 0 && slots <= 32 * PREP_ATOMS && zero_count <= 128 * PREP_ATOMS && ne > 0 && ne <= PREP_ELEMENTS &&
-        (model_species ? sort_types != nullptr : ne == prm->nspecies) && lean_grids(prm, nullptr, n) &&
-        wavefronts_forward(A, triples, triples > TCH_MAX, true) == 1 && Z && species && types && sorted_slots && type_offsets &&
-        (zero || zero_count == 0)) {
-        const long long work = std::max<long long>(slots, (long long)zero_count);
-        b = BatchPrep{Z, species, model_species, ne, A, (int)slots, types, sort_types, sorted_slots, type_offsets, zero, (int)zero_count,
-                      1 + (int)((work + 255) / 256)};
+    if (prepared_beside(A, slots, zero_count, ne, n, prm) && (model_species ? sort_types != nullptr : ne == prm->nspecies) && Z && species &&
+        types && sorted_slots && type_offsets && (zero || zero_count == 0)) {
+        b = prep_of(Z, species, model_species, ne, A, slots, types, sort_types, sorted_slots, type_offsets, zero, zero_count);
     } else {
         int rc = qmll_prepare_batch(Z, natoms, species, prm->nspecies, model_species, ne, atomIDs, molIDs, B, n, A, workspace,
                                     workspace_bytes, types, sort_types, sorted_slots, type_offsets, zero, zero_count, stream);
         if (rc != QMLL_OK) return rc;
     }
     return forward(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm, b, rep, stream);
+}
+
+static bool projected_takes(int A, long long slots, size_t zero_count, int ne, int n, const qmll_fchl_params* prm, int d) {
+    return prepared_beside(A, slots, zero_count, ne, n, prm) && (d == 64 || d == 128) &&
+           prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3 <= held_rows(d);
+}
+
+extern "C" int qmll_prepare_fchl19_project_pays(int A, int B, int n, size_t zero_count, int ne, const qmll_fchl_params* prm, int d) {
+    return prm && projected_takes(A, (long long)B * n, zero_count, ne, n, prm, d) ? 1 : 0;
+}
+
+extern "C" int qmll_prepare_fchl19_project(const float* X, const float* Z, const float* species, const float* model_species, int ne,
+                                           const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
+                                           const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
+                                           const qmll_fchl_params* prm, int* types, int* sort_types, int* sorted_slots, int* type_offsets,
+                                           float* zero, size_t zero_count, const float* reductors, int d, float* x, qmll_stream_t stream) {
+    FchlArgs a;
+    int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm,
+                       "qmll_prepare_fchl19_project");
+    if (rc) return rc;
+    const long long slots = (long long)B * n;
+    QMLL_REQUIRE(projected_takes(A, slots, zero_count, ne, n, prm, d), QMLL_ERR_INVALID,
+                 "qmll_prepare_fchl19_project: A=%d n=%d ne=%d d=%d: not a call it takes", A, n, ne, d);
+    QMLL_REQUIRE(Z && species && sorted_slots && type_offsets && reductors && x && (zero || zero_count == 0), QMLL_ERR_INVALID,
+                 "qmll_prepare_fchl19_project: null pointer");
+    QMLL_REQUIRE(model_species ? sort_types != nullptr : ne == prm->nspecies, QMLL_ERR_INVALID,
+                 "qmll_prepare_fchl19_project: %d elements of %d species without a list of their own", ne, prm->nspecies);
+    QMLL_REQUIRE(reinterpret_cast<uintptr_t>(reductors) % 16 == 0, QMLL_ERR_INVALID,
+                 "qmll_prepare_fchl19_project: reductors must be 16-byte aligned");
+    const BatchPrep b = prep_of(Z, species, model_species, ne, A, slots, types, sort_types, sorted_slots, type_offsets, zero, zero_count);
+    const int ns = prm->nspecies, np = ns * (ns + 1) / 2, R = ns * prm->nRs2 + 2 * np * prm->nRs3;
+    const long long maxnn = n > 1 ? n - 1 : 1, triples = std::max(maxnn * (maxnn - 1) / 2, 1ll);
+    const size_t entries = std::max<size_t>(triples + np * (LEAN_SLOTS - 1), a.cap);
+    const size_t lds = std::max(sizeof(float) * (((R + 3) & ~3) + (size_t)FP_WAVES * d + PREP_ATOMS / 64 + (size_t)8 * a.cap + (3 * entries + 3) / 4 * 4),
+                                sizeof(int) * (size_t)A);                                     // (the sort's)
+    QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID, "qmll_prepare_fchl19_project: %zu B of LDS needed exceeds %zu", lds, LDS_LIMIT);
+    hipStream_t st = (hipStream_t)stream;
+    auto launch = [&](auto nsc, auto dc) {
+        hipLaunchKernelGGL((fchl19_forward_projected_kernel<decltype(nsc)::value, decltype(dc)::value>), dim3(b.groups + A),
+                           dim3(64 * FP_WAVES), lds, st, a, b, reductors, x);
+    };
+    auto by_species = [&](auto dc) {
+        switch (ns) {
+            case 1: launch(std::integral_constant<int, 1>{}, dc); break;
+            case 2: launch(std::integral_constant<int, 2>{}, dc); break;
+            case 3: launch(std::integral_constant<int, 3>{}, dc); break;
+            case 4: launch(std::integral_constant<int, 4>{}, dc); break;
+            default: launch(std::integral_constant<int, 5>{}, dc); break;
+        }
+    };
+    if (d == 64) by_species(std::integral_constant<int, 64>{});
+    else by_species(std::integral_constant<int, 128>{});
+    QMLL_CHECK_LAUNCH("qmll_prepare_fchl19_project");
+    return QMLL_OK;
 }
 
 extern "C" int qmll_fchl19_vjp(const float* X, const int* types, const float* cell, const float* inv_cell,
@@ -2582,6 +2844,60 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
         break;
     }
     QMLL_CHECK_LAUNCH("qmll_fchl19_vjp");
+    return QMLL_OK;
+}
+
+static bool projected_vjp_takes(int A, int n, const qmll_fchl_params* prm, int d) {
+    const long long maxnn = n > 1 ? n - 1 : 1;
+    return A > 0 && A <= PV_ATOMS && (d == 64 || d == 128) && lean_grids(prm, nullptr, n) && n <= 54 &&
+           prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3 <= held_rows(d);
+}
+
+extern "C" int qmll_fchl19_projected_vjp_pays(int A, int n, const qmll_fchl_params* prm, int d) {
+    return prm && projected_vjp_takes(A, n, prm, d) ? 1 : 0;
+}
+
+extern "C" int qmll_fchl19_projected_vjp(const float* X, const int* types, const float* cell, const float* inv_cell, const int* atomIDs,
+                                         const int* molIDs, const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
+                                         const qmll_fchl_params* prm, const float* gx, int nparts, const int* sorted_slots,
+                                         const int* type_offsets, const float* reductors, int ne, int d, float scale, float* grad_X,
+                                         const float* e_slots, float* energies, qmll_stream_t stream) {
+    FchlArgs a;
+    int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm,
+                       "qmll_fchl19_projected_vjp");
+    if (rc) return rc;
+    QMLL_REQUIRE(projected_vjp_takes(A, n, prm, d), QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: A=%d n=%d d=%d: not a call it takes", A, n, d);
+    QMLL_REQUIRE(gx && sorted_slots && type_offsets && reductors && grad_X && ne > 0 && nparts > 0, QMLL_ERR_INVALID,
+                 "qmll_fchl19_projected_vjp: null pointer, or no elements or parts");
+    QMLL_REQUIRE(reinterpret_cast<uintptr_t>(reductors) % 16 == 0, QMLL_ERR_INVALID,
+                 "qmll_fchl19_projected_vjp: reductors must be 16-byte aligned");
+    QMLL_REQUIRE(!energies || e_slots, QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: energies without e_slots");
+    a.gscale = scale;
+    a.tcap = 1;
+    for (int k = 1; k <= a.cap; ++k) a.tcap = std::max(a.tcap, k * force_copies(k));
+    const int ns = prm->nspecies, R = ns * prm->nRs2 + ns * (ns + 1) * prm->nRs3;
+    const size_t lds = sizeof(float) * (d + ((R + 3) & ~3) + (size_t)9 * a.cap + 4 * PV_WAVES * (size_t)a.tcap + ns * (ns + 1) * LEAN_RS3 +
+                                        32 * (ns + 1) + 3 * PV_WAVES);
+    QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: %zu B of LDS needed exceeds %zu", lds, LDS_LIMIT);
+    const ProjectedGradient pg = {gx, nparts, sorted_slots, type_offsets, reductors, ne, A, e_slots, energies};
+    const dim3 grid(A + (energies ? (B + PV_WAVES - 1) / PV_WAVES : 0));
+    hipStream_t st = (hipStream_t)stream;
+    auto launch = [&](auto nsc, auto dc) {
+        hipLaunchKernelGGL((fchl19_projected_vjp_kernel<decltype(nsc)::value, decltype(dc)::value>), grid, dim3(64 * PV_WAVES), lds, st, a, pg,
+                           grad_X);
+    };
+    auto by_species = [&](auto dc) {
+        switch (ns) {
+            case 1: launch(std::integral_constant<int, 1>{}, dc); break;
+            case 2: launch(std::integral_constant<int, 2>{}, dc); break;
+            case 3: launch(std::integral_constant<int, 3>{}, dc); break;
+            case 4: launch(std::integral_constant<int, 4>{}, dc); break;
+            default: launch(std::integral_constant<int, 5>{}, dc); break;
+        }
+    };
+    if (d == 64) by_species(std::integral_constant<int, 64>{});
+    else by_species(std::integral_constant<int, 128>{});
+    QMLL_CHECK_LAUNCH("qmll_fchl19_projected_vjp");
     return QMLL_OK;
 }
 
