@@ -409,20 +409,21 @@ int qmll_project_typed_backward_parts(float* gx, int nparts, const int* sorted_s
                                       float* energies, qmll_stream_t stream);
 
 /* qmll_prepare_fchl19_forward and qmll_project_typed of few atoms in one launch, the representation never written: x f32 [A,d] in sorted
- * order (rows past type_offsets[ne] are not written).  Only for calls for which qmll_prepare_fchl19_project_pays returns 1.  reductors
+ * order (rows past type_offsets[ne] are not written); beyond 256 atoms the preparation is a launch of its own, with qmll_prepare_batch's
+ * workspace.  Only for calls for which qmll_fchl19_projected_pays returns 1.  reductors
  * f32 [ne,R,d], 16-byte aligned. */
-int qmll_prepare_fchl19_project_pays(int A, int B, int n, size_t zero_count, int ne, const qmll_fchl_params* prm, int d);
+int qmll_fchl19_projected_pays(int A, int n, const qmll_fchl_params* prm, int d);
 int qmll_prepare_fchl19_project(const float* X, const float* Z, const float* species, const float* model_species, int ne,
                                 const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
                                 const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
-                                const qmll_fchl_params* prm, int* types, int* sort_types, int* sorted_slots, int* type_offsets,
-                                float* zero, size_t zero_count, const float* reductors, int d, float* x, qmll_stream_t stream);
+                                const qmll_fchl_params* prm, void* workspace, size_t workspace_bytes, int* types, int* sort_types,
+                                int* sorted_slots, int* type_offsets, float* zero, size_t zero_count, const float* reductors, int d,
+                                float* x, qmll_stream_t stream);
 
 /* qmll_project_typed_backward_parts and qmll_fchl19_vjp_scaled of few atoms in one launch, the representation's gradient never written:
  * grad_X += scale * J^T (sum of the nparts parts of gx . reductors[type]^T); atoms past type_offsets[ne] contribute nothing.  gx f32
  * [nparts,A,d] and e_slots f32 [nparts,B*n] as qmll_sorf_energy_parts writes them; energies f32 [B] or NULL.  Only for calls for which
- * qmll_fchl19_projected_vjp_pays returns 1.  reductors 16-byte aligned. */
-int qmll_fchl19_projected_vjp_pays(int A, int n, const qmll_fchl_params* prm, int d);
+ * qmll_fchl19_projected_pays returns 1.  reductors 16-byte aligned. */
 int qmll_fchl19_projected_vjp(const float* X, const int* types, const float* cell, const float* inv_cell, const int* atomIDs,
                               const int* molIDs, const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
                               const qmll_fchl_params* prm, const float* gx, int nparts, const int* sorted_slots,

@@ -47,10 +47,9 @@ PROTOTYPES = {
     "qmll_fchl19_forward": _FCHL_COMMON + [P, P],
     "qmll_fchl19_vjp": _FCHL_COMMON + [P, P, P],
     "qmll_fchl19_vjp_scaled": _FCHL_COMMON + [P, c_float, P, P],
-    "qmll_prepare_fchl19_project_pays": [c_int, c_int, c_int, c_size_t, c_int, POINTER(FchlParams), c_int],
-    "qmll_prepare_fchl19_project": [P, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, POINTER(FchlParams), P, P, P, P, P, c_size_t,
-                                    P, c_int, P, P],
-    "qmll_fchl19_projected_vjp_pays": [c_int, c_int, POINTER(FchlParams), c_int],
+    "qmll_fchl19_projected_pays": [c_int, c_int, POINTER(FchlParams), c_int],
+    "qmll_prepare_fchl19_project": [P, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, POINTER(FchlParams), P, c_size_t, P, P, P, P,
+                                    P, c_size_t, P, c_int, P, P],
     "qmll_fchl19_projected_vjp": [P] * 7 + [c_int, c_int, c_int, P, P, POINTER(FchlParams), P, c_int, P, P, P, c_int, c_int, c_float, P, P, P, P],
     "qmll_fchl19_jacobian": _FCHL_COMMON + [P, P, P],
     "qmll_fchl19_jacobian_all_rows": _FCHL_COMMON + [P, P, P],

@@ -1108,21 +1108,24 @@ __global__ __launch_bounds__(64) void fchl19_forward_lean_kernel(FchlArgs a, Bat
 // wavefront forms the row in LDS while the reductor's rows are on their way into the registers of all eight and the others count
 // the atom's place in the sorted list.  x[place, :] = row . U.  21 atoms of three elements, 128 components: 6.5 + 4.3 us in two launches, 9.6 so,
 // and 4 us of the host's time for the launch.
-constexpr int FP_WAVES = 8;
+// PREP = false: the batch has been prepared, and the workgroups follow the sorted list.
+constexpr int MOST_WAVES = 8;
 // rows of a reductor that the registers of eight wavefronts hold beside the rest, in both directions: five elements of the default grids at
-// 64 components, four at 128
-constexpr int held_rows(int d) { return d == 64 ? 768 : 512; }
-template <int NS, int D>
-__global__ __launch_bounds__(64 * FP_WAVES) void fchl19_forward_projected_kernel(FchlArgs a, BatchPrep b, const float* __restrict__ reductors,
-                                                                                 float* __restrict__ x) {
+// 64 components, four at 128; of four and two wavefronts
+constexpr int held_rows(int d, int waves) { return waves == MOST_WAVES ? (d == 64 ? 768 : 512) : 96 * waves * 64 / d; }
+constexpr int fewest_rows(int ns) { return ns + ns * (ns + 1) * (LEAN_RS3 - 3); }                // that a representation of the lean grids has
+template <int NS, int D, int W, bool PREP>
+__global__ __launch_bounds__(64 * W) void fchl19_forward_projected_kernel(FchlArgs a, BatchPrep b, const float* __restrict__ reductors,
+                                                                          float* __restrict__ x) {
+    static_assert(!PREP || W > PREP_ATOMS / 64, "a wavefront for every 64 atoms of the list, and one for the representation");
     extern __shared__ float smem[];
-    constexpr int CL = D / 4, KS = 64 * FP_WAVES / CL, MINE = held_rows(D) / KS; // lanes along the columns, slices of the rows, rows of each
+    constexpr int CL = D / 4, KS = 64 * W / CL, MINE = held_rows(D, W) / KS;     // lanes along the columns, slices of the rows, rows of each
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if ((int)blockIdx.x < b.groups) {
+    if (PREP && (int)blockIdx.x < b.groups) {
         if (wave == 0) prepare_group(a, b, blockIdx.x, lane, reinterpret_cast<int*>(smem));
         return;
     }
-    const int atom = blockIdx.x - b.groups, R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
+    const int atom = PREP ? blockIdx.x - b.groups : blockIdx.x, R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
     const float* list = b.model_species ? b.model_species : b.species;
     const int nlist = b.model_species ? b.ne : a.p.nspecies;
     // element of a listed atom by the model's list, as prepare_group has it; -1: not in the sorted list
@@ -1131,12 +1134,22 @@ __global__ __launch_bounds__(64 * FP_WAVES) void fchl19_forward_projected_kernel
         if (m < 0 || m >= a.B || i < 0 || i >= a.n) return -1;
         return i < a.natoms[m] ? species_index(b.Z[(size_t)m * a.n + i], list, nlist) : 0;
     };
-    const int m = a.molIDs[atom], i = a.atomIDs[atom];
-    const int e = __builtin_amdgcn_readfirstlane(element(atom));
+    int m, i, e = 0;
+    if constexpr (PREP) {
+        m = a.molIDs[atom];
+        i = a.atomIDs[atom];
+        e = __builtin_amdgcn_readfirstlane(element(atom));
+    } else {
+        if (atom >= b.offsets[b.ne]) return;
+        while (e + 1 < b.ne && atom >= b.offsets[e + 1]) ++e;
+        const int slot = b.sorted[atom];
+        m = slot / a.n;
+        i = slot - m * a.n;
+    }
     if (m < 0 || m >= a.B || i < 0 || i >= a.n || e < 0 || e >= b.ne) return;
     float* row = smem;                                   // [R4] the representation
-    float* part = row + ((R + 3) & ~3);                  // [FP_WAVES][D]
-    int* before = reinterpret_cast<int*>(part + FP_WAVES * D);           // [PREP_ATOMS / 64]
+    float* part = row + ((R + 3) & ~3);                  // [W][D]
+    int* before = reinterpret_cast<int*>(part + W * D);  // [PREP_ATOMS / 64]
     float* own = reinterpret_cast<float*>(before + PREP_ATOMS / 64);
     const int c4 = tid % CL, ks = tid / CL;
     const float4* U = reinterpret_cast<const float4*>(reductors + (size_t)e * R * D) + c4;
@@ -1147,8 +1160,8 @@ __global__ __launch_bounds__(64 * FP_WAVES) void fchl19_forward_projected_kernel
         if (KS * k < R) u[k] = U[(size_t)min(ks + KS * k, R - 1) * CL];
     }
     if (wave == 0) {
-        lean_forward<NS, true>(a, b, m, i, lane, own, row, [] { wave_sync(); });
-    } else if (wave <= PREP_ATOMS / 64) {                // the atoms ahead of this one in the sorted list
+        lean_forward<NS, PREP>(a, b, m, i, lane, own, row, [] { wave_sync(); });
+    } else if (PREP && wave <= PREP_ATOMS / 64) {                // the atoms ahead of this one in the sorted list
         const int at = tid - 64;
         const int t = at < b.A ? element(at) : -1;
         const int count = __popcll(__ballot(t >= 0 && (t < e || (t == e && at < atom))));
@@ -1178,10 +1191,12 @@ __global__ __launch_bounds__(64 * FP_WAVES) void fchl19_forward_projected_kernel
     if (tid < D) {
         float sum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < FP_WAVES; ++w) sum += part[w * D + tid];
-        int place = 0;
+        for (int w = 0; w < W; ++w) sum += part[w * D + tid];
+        int place = PREP ? 0 : atom;
+        if constexpr (PREP) {
 #pragma unroll
-        for (int w = 0; w < PREP_ATOMS / 64; ++w) place += before[w];
+            for (int w = 0; w < PREP_ATOMS / 64; ++w) place += before[w];
+        }
         x[(size_t)place * D + tid] = sum;
     }
 }
@@ -2133,7 +2148,7 @@ __global__ __launch_bounds__(64) void fchl19_vjp_lean_kernel(FchlArgs a, const f
 // The backward projection and the VJP of few atoms in one launch: a workgroup per atom (in sorted order) forms its row of the
 // representation's gradient in LDS, g_rep = sum of the parts of gx . U^T, four lanes to an entry, and takes it from there.  Both
 // were chains of latencies in launches of their own; here the reductor's rows are on their way while the neighbours are staged, and the
-// triples are shared by eight wavefronts.  Workgroups behind the atoms sum the energies of eight molecules each.  21 atoms, 128
+// triples are shared by eight wavefronts.  Workgroups behind the atoms sum the energies, a wavefront per molecule.  21 atoms, 128
 // components: 4.1 + 7.2 us, 8.3 so.  With the forward pair (above) energies and forces of 1 x 21 atoms take 21.3 us (28.5), 12 x 21 25.4 (30.7),
 // 8 x 29 26.0 (32.1), 20 x 12 at 64 components 21.0 (26.2).  Beyond 256 atoms the workgroups, a CU each, come in rounds: 16 x 21 41.7 (37.7); with rows
 // read in several pieces (five elements or 256 components) the pieces wait for memory: 2 x 29, five elements, 128 components 34.4 (32.9).
@@ -2147,15 +2162,14 @@ struct ProjectedGradient {
     const float* e_slots;         // [nparts][B n]
     float* energies;              // or null
 };
-constexpr int PV_WAVES = 8, PV_ATOMS = 256;      // (a workgroup has a CU to itself)
-template <int NS, int D>
-__global__ __launch_bounds__(64 * PV_WAVES) void fchl19_projected_vjp_kernel(FchlArgs a, ProjectedGradient pg, float* __restrict__ grad_X) {
+template <int NS, int D, int W>
+__global__ __launch_bounds__(64 * W) void fchl19_projected_vjp_kernel(FchlArgs a, ProjectedGradient pg, float* __restrict__ grad_X) {
     extern __shared__ float smem[];
-    constexpr int NT = 64 * PV_WAVES, ROWS = NT / 4, KQ = D / 16, AHEAD = held_rows(D) / ROWS;
+    constexpr int ROWS = 16 * W, KQ = D / 16, AHEAD = held_rows(D, W) / ROWS;
     const int tid = threadIdx.x, R = NS * a.p.nRs2 + NS * (NS + 1) * a.p.nRs3;
     const int pos = blockIdx.x;
     if (pos >= pg.A) {                                   // energies: a wavefront per molecule
-        const int mol = (pos - pg.A) * PV_WAVES + (tid >> 6), lane = tid & 63;
+        const int mol = (pos - pg.A) * W + (tid >> 6), lane = tid & 63;
         if (mol >= a.B) return;
         float acc = 0.0f;
         for (int t = lane; t < pg.nparts * a.n; t += 64) {
@@ -2188,7 +2202,7 @@ __global__ __launch_bounds__(64 * PV_WAVES) void fchl19_projected_vjp_kernel(Fch
     const int slot = pg.sorted_slots[pos], m = slot / a.n, i = slot - m * a.n;
     float* sg = smem;                                    // [D] gx
     float* row = sg + D;                                 // [R4] g_rep
-    lean_vjp<NS, PV_WAVES>(a, m, i, row + ((R + 3) & ~3), [&]() -> const float* {
+    lean_vjp<NS, W>(a, m, i, row + ((R + 3) & ~3), [&]() -> const float* {
         if (tid < D) sg[tid] = v;
         __syncthreads();
 #pragma unroll
@@ -2726,56 +2740,91 @@ extern "C" int qmll_prepare_fchl19_forward(const float* X, const float* Z, const
     return forward(X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm, b, rep, stream);
 }
 
-static bool projected_takes(int A, long long slots, size_t zero_count, int ne, int n, const qmll_fchl_params* prm, int d) {
-    return prepared_beside(A, slots, zero_count, ne, n, prm) && (d == 64 || d == 128) &&
-           prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3 <= held_rows(d);
+// Wavefronts per atom of the launches that take the projections in, 0: not taken.  Up to 256 atoms eight, a CU to each workgroup.  With
+// more, two or four if they hold the reductor, and as many atoms as are resident at a time (twelve wavefronts per CU).  Energies and forces,
+// 64 components, launches apart / so, us: two elements (two wavefronts) 300 atoms of 12 29.7 / 26.1, 1200 29.7 / 27.5, 1992 31.0 / 36.4; three
+// elements (four) 492 29.4 / 26.7, 792 29.6 / 34.4; 100 x 12 through autograd 119.8 / 88.5.  Only where the representation is the work of one
+// wavefront: 3 x 40 atoms, 128 components, backward alone 31.9 / 32.9.
+static int projected_waves(int A, int n, const qmll_fchl_params* prm, int d) {
+    const int R = prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3;
+    const long long maxnn = n > 1 ? n - 1 : 1, triples = maxnn * (maxnn - 1) / 2;
+    if (A <= 0 || (d != 64 && d != 128) || !lean_grids(prm, nullptr, n) || wavefronts_forward(A, triples, triples > TCH_MAX, true) != 1) return 0;
+    if (A <= PREP_ATOMS) return R <= held_rows(d, 8) ? 8 : 0;
+    if (R <= held_rows(d, 2)) return A <= 6 * 256 ? 2 : 0;
+    return R <= held_rows(d, 4) && A <= 3 * 256 ? 4 : 0;
 }
-
-extern "C" int qmll_prepare_fchl19_project_pays(int A, int B, int n, size_t zero_count, int ne, const qmll_fchl_params* prm, int d) {
-    return prm && projected_takes(A, (long long)B * n, zero_count, ne, n, prm, d) ? 1 : 0;
+// f(number of species, components, wavefronts) as constants, for what there can be
+template <class F>
+static void with_projected_shape(int ns, int d, int waves, F f) {
+    auto by_waves = [&](auto nsc, auto dc) {
+        constexpr int NS = decltype(nsc)::value, D = decltype(dc)::value;
+        if constexpr (fewest_rows(NS) <= held_rows(D, 2)) {
+            if (waves == 2) f(nsc, dc, std::integral_constant<int, 2>{});
+        }
+        if constexpr (fewest_rows(NS) <= held_rows(D, 4)) {
+            if (waves == 4) f(nsc, dc, std::integral_constant<int, 4>{});
+        }
+        if (waves == 8) f(nsc, dc, std::integral_constant<int, 8>{});
+    };
+    auto by_species = [&](auto dc) {
+        switch (ns) {
+            case 1: by_waves(std::integral_constant<int, 1>{}, dc); break;
+            case 2: by_waves(std::integral_constant<int, 2>{}, dc); break;
+            case 3: by_waves(std::integral_constant<int, 3>{}, dc); break;
+            case 4: by_waves(std::integral_constant<int, 4>{}, dc); break;
+            default: by_waves(std::integral_constant<int, 5>{}, dc); break;
+        }
+    };
+    if (d == 64) by_species(std::integral_constant<int, 64>{});
+    else by_species(std::integral_constant<int, 128>{});
+}
+extern "C" int qmll_fchl19_projected_pays(int A, int n, const qmll_fchl_params* prm, int d) {
+    return prm && projected_waves(A, n, prm, d) > 0 ? 1 : 0;
 }
 
 extern "C" int qmll_prepare_fchl19_project(const float* X, const float* Z, const float* species, const float* model_species, int ne,
                                            const float* cell, const float* inv_cell, const int* atomIDs, const int* molIDs,
                                            const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
-                                           const qmll_fchl_params* prm, int* types, int* sort_types, int* sorted_slots, int* type_offsets,
-                                           float* zero, size_t zero_count, const float* reductors, int d, float* x, qmll_stream_t stream) {
+                                           const qmll_fchl_params* prm, void* workspace, size_t workspace_bytes, int* types,
+                                           int* sort_types, int* sorted_slots, int* type_offsets, float* zero, size_t zero_count,
+                                           const float* reductors, int d, float* x, qmll_stream_t stream) {
     FchlArgs a;
     int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm,
                        "qmll_prepare_fchl19_project");
     if (rc) return rc;
     const long long slots = (long long)B * n;
-    QMLL_REQUIRE(projected_takes(A, slots, zero_count, ne, n, prm, d), QMLL_ERR_INVALID,
-                 "qmll_prepare_fchl19_project: A=%d n=%d ne=%d d=%d: not a call it takes", A, n, ne, d);
-    QMLL_REQUIRE(Z && species && sorted_slots && type_offsets && reductors && x && (zero || zero_count == 0), QMLL_ERR_INVALID,
-                 "qmll_prepare_fchl19_project: null pointer");
+    const int waves = projected_waves(A, n, prm, d);
+    QMLL_REQUIRE(waves > 0, QMLL_ERR_INVALID, "qmll_prepare_fchl19_project: A=%d n=%d d=%d: not a call it takes", A, n, d);
+    QMLL_REQUIRE(Z && species && sorted_slots && type_offsets && reductors && x && ne > 0 && (zero || zero_count == 0), QMLL_ERR_INVALID,
+                 "qmll_prepare_fchl19_project: null pointer or no elements");
     QMLL_REQUIRE(model_species ? sort_types != nullptr : ne == prm->nspecies, QMLL_ERR_INVALID,
                  "qmll_prepare_fchl19_project: %d elements of %d species without a list of their own", ne, prm->nspecies);
     QMLL_REQUIRE(reinterpret_cast<uintptr_t>(reductors) % 16 == 0, QMLL_ERR_INVALID,
                  "qmll_prepare_fchl19_project: reductors must be 16-byte aligned");
-    const BatchPrep b = prep_of(Z, species, model_species, ne, A, slots, types, sort_types, sorted_slots, type_offsets, zero, zero_count);
     const int ns = prm->nspecies, np = ns * (ns + 1) / 2, R = ns * prm->nRs2 + 2 * np * prm->nRs3;
+    const bool beside = waves == 8 && prepared_beside(A, slots, zero_count, ne, n, prm);
+    BatchPrep b = prep_of(Z, species, model_species, ne, A, slots, types, sort_types, sorted_slots, type_offsets, zero, zero_count);
+    if (!beside) {
+        rc = qmll_prepare_batch(Z, natoms, species, ns, model_species, ne, atomIDs, molIDs, B, n, A, workspace, workspace_bytes, types,
+                                sort_types, sorted_slots, type_offsets, zero, zero_count, stream);
+        if (rc != QMLL_OK) return rc;
+    }
     const long long maxnn = n > 1 ? n - 1 : 1, triples = std::max(maxnn * (maxnn - 1) / 2, 1ll);
     const size_t entries = std::max<size_t>(triples + np * (LEAN_SLOTS - 1), a.cap);
-    const size_t lds = std::max(sizeof(float) * (((R + 3) & ~3) + (size_t)FP_WAVES * d + PREP_ATOMS / 64 + (size_t)8 * a.cap + (3 * entries + 3) / 4 * 4),
-                                sizeof(int) * (size_t)A);                                     // (the sort's)
+    const size_t lds = std::max(sizeof(float) * (((R + 3) & ~3) + (size_t)waves * d + PREP_ATOMS / 64 + (size_t)8 * a.cap + (3 * entries + 3) / 4 * 4),
+                                beside ? sizeof(int) * (size_t)A : 0);                        // (the sort's)
     QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID, "qmll_prepare_fchl19_project: %zu B of LDS needed exceeds %zu", lds, LDS_LIMIT);
     hipStream_t st = (hipStream_t)stream;
-    auto launch = [&](auto nsc, auto dc) {
-        hipLaunchKernelGGL((fchl19_forward_projected_kernel<decltype(nsc)::value, decltype(dc)::value>), dim3(b.groups + A),
-                           dim3(64 * FP_WAVES), lds, st, a, b, reductors, x);
-    };
-    auto by_species = [&](auto dc) {
-        switch (ns) {
-            case 1: launch(std::integral_constant<int, 1>{}, dc); break;
-            case 2: launch(std::integral_constant<int, 2>{}, dc); break;
-            case 3: launch(std::integral_constant<int, 3>{}, dc); break;
-            case 4: launch(std::integral_constant<int, 4>{}, dc); break;
-            default: launch(std::integral_constant<int, 5>{}, dc); break;
+    with_projected_shape(ns, d, waves, [&](auto nsc, auto dc, auto wc) {
+        constexpr int NS = decltype(nsc)::value, D = decltype(dc)::value, W = decltype(wc)::value;
+        if constexpr (W == 8) {
+            if (beside) {
+                hipLaunchKernelGGL((fchl19_forward_projected_kernel<NS, D, W, true>), dim3(b.groups + A), dim3(64 * W), lds, st, a, b, reductors, x);
+                return;
+            }
         }
-    };
-    if (d == 64) by_species(std::integral_constant<int, 64>{});
-    else by_species(std::integral_constant<int, 128>{});
+        hipLaunchKernelGGL((fchl19_forward_projected_kernel<NS, D, W, false>), dim3(A), dim3(64 * W), lds, st, a, b, reductors, x);
+    });
     QMLL_CHECK_LAUNCH("qmll_prepare_fchl19_project");
     return QMLL_OK;
 }
@@ -2847,16 +2896,6 @@ extern "C" int qmll_fchl19_vjp_scaled(const float* X, const int* types, const fl
     return QMLL_OK;
 }
 
-static bool projected_vjp_takes(int A, int n, const qmll_fchl_params* prm, int d) {
-    const long long maxnn = n > 1 ? n - 1 : 1;
-    return A > 0 && A <= PV_ATOMS && (d == 64 || d == 128) && lean_grids(prm, nullptr, n) && n <= 54 &&
-           prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3 <= held_rows(d);
-}
-
-extern "C" int qmll_fchl19_projected_vjp_pays(int A, int n, const qmll_fchl_params* prm, int d) {
-    return prm && projected_vjp_takes(A, n, prm, d) ? 1 : 0;
-}
-
 extern "C" int qmll_fchl19_projected_vjp(const float* X, const int* types, const float* cell, const float* inv_cell, const int* atomIDs,
                                          const int* molIDs, const int* natoms, int A, int B, int n, const float* Rs2, const float* Rs3,
                                          const qmll_fchl_params* prm, const float* gx, int nparts, const int* sorted_slots,
@@ -2866,7 +2905,8 @@ extern "C" int qmll_fchl19_projected_vjp(const float* X, const int* types, const
     int rc = fill_args(a, X, types, cell, inv_cell, atomIDs, molIDs, natoms, nullptr, nullptr, 0, A, B, n, Rs2, Rs3, prm,
                        "qmll_fchl19_projected_vjp");
     if (rc) return rc;
-    QMLL_REQUIRE(projected_vjp_takes(A, n, prm, d), QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: A=%d n=%d d=%d: not a call it takes", A, n, d);
+    const int waves = projected_waves(A, n, prm, d);
+    QMLL_REQUIRE(waves > 0, QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: A=%d n=%d d=%d: not a call it takes", A, n, d);
     QMLL_REQUIRE(gx && sorted_slots && type_offsets && reductors && grad_X && ne > 0 && nparts > 0, QMLL_ERR_INVALID,
                  "qmll_fchl19_projected_vjp: null pointer, or no elements or parts");
     QMLL_REQUIRE(reinterpret_cast<uintptr_t>(reductors) % 16 == 0, QMLL_ERR_INVALID,
@@ -2876,27 +2916,15 @@ extern "C" int qmll_fchl19_projected_vjp(const float* X, const int* types, const
     a.tcap = 1;
     for (int k = 1; k <= a.cap; ++k) a.tcap = std::max(a.tcap, k * force_copies(k));
     const int ns = prm->nspecies, R = ns * prm->nRs2 + ns * (ns + 1) * prm->nRs3;
-    const size_t lds = sizeof(float) * (d + ((R + 3) & ~3) + (size_t)9 * a.cap + 4 * PV_WAVES * (size_t)a.tcap + ns * (ns + 1) * LEAN_RS3 +
-                                        32 * (ns + 1) + 3 * PV_WAVES);
+    const size_t lds = sizeof(float) * (d + ((R + 3) & ~3) + (size_t)9 * a.cap + 4 * waves * (size_t)a.tcap + ns * (ns + 1) * LEAN_RS3 +
+                                        32 * (ns + 1) + 3 * waves);
     QMLL_REQUIRE(lds <= LDS_LIMIT, QMLL_ERR_INVALID, "qmll_fchl19_projected_vjp: %zu B of LDS needed exceeds %zu", lds, LDS_LIMIT);
     const ProjectedGradient pg = {gx, nparts, sorted_slots, type_offsets, reductors, ne, A, e_slots, energies};
-    const dim3 grid(A + (energies ? (B + PV_WAVES - 1) / PV_WAVES : 0));
-    hipStream_t st = (hipStream_t)stream;
-    auto launch = [&](auto nsc, auto dc) {
-        hipLaunchKernelGGL((fchl19_projected_vjp_kernel<decltype(nsc)::value, decltype(dc)::value>), grid, dim3(64 * PV_WAVES), lds, st, a, pg,
-                           grad_X);
-    };
-    auto by_species = [&](auto dc) {
-        switch (ns) {
-            case 1: launch(std::integral_constant<int, 1>{}, dc); break;
-            case 2: launch(std::integral_constant<int, 2>{}, dc); break;
-            case 3: launch(std::integral_constant<int, 3>{}, dc); break;
-            case 4: launch(std::integral_constant<int, 4>{}, dc); break;
-            default: launch(std::integral_constant<int, 5>{}, dc); break;
-        }
-    };
-    if (d == 64) by_species(std::integral_constant<int, 64>{});
-    else by_species(std::integral_constant<int, 128>{});
+    const dim3 grid(A + (energies ? (B + waves - 1) / waves : 0));
+    with_projected_shape(ns, d, waves, [&](auto nsc, auto dc, auto wc) {
+        constexpr int NS = decltype(nsc)::value, D = decltype(dc)::value, W = decltype(wc)::value;
+        hipLaunchKernelGGL((fchl19_projected_vjp_kernel<NS, D, W>), grid, dim3(64 * W), lds, (hipStream_t)stream, a, pg, grad_X);
+    });
     QMLL_CHECK_LAUNCH("qmll_fchl19_projected_vjp");
     return QMLL_OK;
 }

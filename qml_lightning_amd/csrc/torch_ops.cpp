@@ -794,18 +794,19 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
     auto pad = [](int64_t v) { return (v + 63) / 64 * 64; };          // every part 256-byte aligned
     const int64_t rep_n = pad(nslots * R), x_n = pad((int64_t)A * d), gx_n = pad((int64_t)A * d * nparts);
     // few atoms: the representation and its projection, and the two backward, are a launch each
-    const bool aligned = reinterpret_cast<uintptr_t>(fp(red)) % 16 == 0;
-    const bool rep_in_launch = aligned && qmll_prepare_fchl19_project_pays(A, B, n, (size_t)nzero, ne, &in.prm, d);
-    const bool both = with_grad && aligned && qmll_fchl19_projected_vjp_pays(A, n, &in.prm, d);
-    Tensor scratch = at::empty({(rep_in_launch ? 0 : rep_n) + x_n + (with_grad ? gx_n + (both ? 0 : rep_n) : 0) + 64}, in.X.options());
+    const bool projected = reinterpret_cast<uintptr_t>(fp(red)) % 16 == 0 && qmll_fchl19_projected_pays(A, n, &in.prm, d);
+    const int64_t kept_rep_n = projected ? 0 : rep_n;
+    Tensor scratch = at::empty({kept_rep_n + x_n + (with_grad ? gx_n + kept_rep_n : 0) + 64}, in.X.options());
     float* rep = scratch.data_ptr<float>();
-    float* x = rep + (rep_in_launch ? 0 : rep_n);
+    float* x = rep + kept_rep_n;
     float* gx = with_grad ? x + x_n : nullptr;
     float* g_rep = with_grad ? gx + gx_n : nullptr;
-    if (rep_in_launch) {
+    Tensor split;
+    if (projected) {
         check(qmll_prepare_fchl19_project(fp(in.X), fp(Zb), fp(sp), fp(msp), ne, fp(in.cell), fp(in.inv_cell), ip(in.atomIDs), ip(in.molIDs),
-                                          ip(in.natoms), A, B, n, fp(in.Rs2), fp(in.Rs3), &in.prm, types, own_list ? sort_types : nullptr, ss,
-                                          off, nzero ? out.data_ptr<float>() : nullptr, (size_t)nzero, fp(red), d, x, stream()),
+                                          ip(in.natoms), A, B, n, fp(in.Rs2), fp(in.Rs3), &in.prm, sort_work, sort_bytes, types,
+                                          own_list ? sort_types : nullptr, ss, off, nzero ? out.data_ptr<float>() : nullptr,
+                                          (size_t)nzero, fp(red), d, x, stream()),
               "qmll_prepare_fchl19_project");
     } else {
         // the forward kernel writes every bin of a listed atom's row, and only the rows of listed
@@ -815,10 +816,9 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
                                           own_list ? sort_types : nullptr, ss, off, nzero ? out.data_ptr<float>() : nullptr,
                                           (size_t)nzero, rep, stream()),
               "qmll_prepare_fchl19_forward");
-    }
-    Tensor split = rep_in_launch && (both || !with_grad) ? Tensor() : reductors_split(red, A);
-    if (!rep_in_launch)
+        split = reductors_split(red, A);
         check(qmll_project_typed(rep, ss, off, fp(red), vp(split), A, ne, R, d, x, stream()), "qmll_project_typed");
+    }
     if (rff)
         rff_energy_sorted_raw(x, off, ss, A, d, ne, Dmat, bias, alpha, e_slots, gx);
     else
@@ -831,7 +831,7 @@ Tensor fchl_sorf_energy_impl(FCHL_TENSORS, MODEL_TENSORS, bool with_grad, Tensor
         return energies;
     }
     Tensor gX = out.narrow(0, 0, 3 * nslots).view({B, n, 3});
-    if (both) {
+    if (projected) {
         check(qmll_fchl19_projected_vjp(fp(in.X), types, fp(in.cell), fp(in.inv_cell), ip(in.atomIDs), ip(in.molIDs), ip(in.natoms), A, B, n,
                                         fp(in.Rs2), fp(in.Rs3), &in.prm, gx, nparts, ss, off, fp(red), ne, d, gscale,
                                         gX.data_ptr<float>(), e_slots, B ? energies.data_ptr<float>() : nullptr, stream()),

@@ -1,5 +1,5 @@
-"""Few atoms: the representation with its projection and the two backward are one launch each (up to 256 atoms, 64 or 128 components,
-768 or 512 entries of the representation).  Energies and forces against the same model by the separate operators, which never take those
+"""Few atoms: the representation with its projection and the two backward are one launch each (64 or 128 components; up to 256 atoms
+with 768 or 512 entries of the representation, 768 with half as many, 1536 with a quarter).  Energies and forces against the same model by the separate operators, which never take those
 launches, at the edges of what does and where it no longer is taken.  Both are fp32 sums in another order: 2-norm errors against
 fp64 are 5e-7 on either route, a fiftieth of the tolerance."""
 import numpy as np
@@ -62,6 +62,14 @@ def test_lists_of_elements(species, elements, npcas):
     rng = np.random.default_rng(len(species))
     coords, charges = helpers.fixed_composition_batch(rng.choice(species, 14), 4, 2, box=6.0)
     check(species, elements, npcas, coords, charges)
+
+
+@pytest.mark.parametrize("species,npcas,natoms,molecules", [([1, 6], 64, 12, 128), ([1, 6], 64, 12, 129), ([1, 6], 64, 29, 9), ([6], 128, 7, 200),
+                                                            ([1, 6, 8], 64, 12, 64), ([1, 6, 8], 64, 12, 65), ([1, 6], 128, 24, 32), ([1, 6, 8], 128, 20, 13)])
+def test_more_atoms(species, npcas, natoms, molecules):
+    rng = np.random.default_rng(natoms)
+    coords, charges = helpers.fixed_composition_batch(rng.choice(species, natoms), molecules, natoms, box=max(4.0, 1.9 * natoms ** (1 / 3)))
+    check(species, species, npcas, coords, charges)
 
 
 def test_ragged_molecules_boxes_and_grids():
