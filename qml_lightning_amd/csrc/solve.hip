@@ -216,32 +216,37 @@ __device__ __forceinline__ bool potrf_factor_wave(double* blk, long long ld, int
 
 // wavefront 4, which shares its SIMD with wavefront 0: no matrix instructions.  It writes the columns of the inverse, and block row K of U
 // right of the diagonal and the diagonal sub-block of the inverse past the caches, for the workgroups that follow this factorisation step
-// by step (follow_block): *steps is the number of block rows that are there.  All of a step's stores are this wavefront's, so that waiting
+// by step (follow_block): *steps is the number of block rows that are there.  (Nobody does where steps is null: the wavefronts that work
+// them out then store both; 704 features in launches of their own 659 us with the detour, 630 so.)  All of a step's stores are this wavefront's, so that waiting
 // for them is all the order they need.
 __device__ __forceinline__ bool potrf_store_wave(double* blk, long long ld, int nb, double* inv, double* invT, unsigned* steps,
                                                  PotrfShared& ps) {
     const int lane = (int)threadIdx.x & 63;
     auto done = [&](unsigned count) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (steps && lane == 0) store_past_caches(steps, count);
+        if (lane == 0) store_past_caches(steps, count);
     };
     for (int K = 0; K < NSB; ++K) {
         __syncthreads();                                               // S(K,K) is in LDS
         if (K > 0) {
-            const int row0 = (K - 1) * SB;
+            if (steps) {
+                const int row0 = (K - 1) * SB;
 #pragma unroll 4
-            for (int r = 0; r < SB; ++r)
-                for (int col = K * SB + lane; col < nb; col += QMLL_WAVE)
-                    if (row0 + r < nb) store_past_caches(&blk[(size_t)(row0 + r) * ld + col], ps.ustrip[r][col]);
-            done((unsigned)K);
+                for (int r = 0; r < SB; ++r)
+                    for (int col = K * SB + lane; col < nb; col += QMLL_WAVE)
+                        if (row0 + r < nb) store_past_caches(&blk[(size_t)(row0 + r) * ld + col], ps.ustrip[r][col]);
+                done((unsigned)K);
+            }
             store_inverse_columns(K - 1, inv, ps);
         }
         __syncthreads();                                               // V is in LDS
         if (ps.failed) return false;
+        if (steps) {
 #pragma unroll
-        for (int e = lane; e < SB * SB; e += QMLL_WAVE)                // W(K,K) = V^T
-            store_past_caches(&invT[(K * SB + e / SB) * NB + K * SB + e % SB], ps.vblk[e % SB][e / SB]);
-        if (K == NSB - 1) done(NSB);
+            for (int e = lane; e < SB * SB; e += QMLL_WAVE)            // W(K,K) = V^T
+                store_past_caches(&invT[(K * SB + e / SB) * NB + K * SB + e % SB], ps.vblk[e % SB][e / SB]);
+            if (K == NSB - 1) done(NSB);
+        }
         __syncthreads();                                               // block row K is in LDS
     }
     store_inverse_columns(NSB - 1, inv, ps);
@@ -251,10 +256,11 @@ __device__ __forceinline__ bool potrf_store_wave(double* blk, long long ld, int 
 // the WV-th (1..6) of the wavefronts 1, 2, 3, 5, 6, 7: its share of the sub-blocks
 template <int WV>
 __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int nb, double* inv, double* invT,
-                                                PotrfShared& ps) {
+                                                bool handed_out, PotrfShared& ps) {
     const int lane = (int)threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
     const int ldi = (int)ld;
     // per-lane parts of every address; what is added per sub-block is a constant
+    double* const blk_lane = blk + (size_t)lk * ld + l16;
     double* const invT_lane = invT + lk * NB + l16;
     double* const us_lane = &ps.ustrip[lk][l16];
     double* const ws_lane = &ps.wstrip[lk][l16];
@@ -335,10 +341,12 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         if constexpr (b.kind == 0) {
-                            us_lane[4 * r * SSTRIDE + b.j * SB] = res[r];                   // (wavefront 4 writes it to memory)
+                            us_lane[4 * r * SSTRIDE + b.j * SB] = res[r];
+                            if (!handed_out && b.j * SB + l16 < nb && K * SB + lk + 4 * r < nb)
+                                blk_lane[(size_t)(K * SB + 4 * r) * ld + b.j * SB] = res[r];
                         } else {
                             ws_lane[4 * r * SSTRIDE + b.j * SB] = res[r];
-                            if constexpr (b.j < K) invT_lane[(K * SB + 4 * r) * NB + b.j * SB] = res[r];
+                            if (b.j < K || !handed_out) invT_lane[(K * SB + 4 * r) * NB + b.j * SB] = res[r];
                         }
                     }
                 }
@@ -356,6 +364,8 @@ __device__ __forceinline__ bool potrf_mfma_wave(double* blk, long long ld, int n
 }
 
 // Called by all PT threads of the workgroup.  False when a pivot is not positive (info is then set).
+// HANDED_OUT: step by step, with the number of steps in *steps.
+template <bool HANDED_OUT>
 __device__ __forceinline__ bool potrf_block(double* A, long long ld, int k0, int nb, double* inv, double* invT,
                                             int* info, unsigned* steps, PotrfShared& ps) {
     const int tid = threadIdx.x;
@@ -374,13 +384,13 @@ __device__ __forceinline__ bool potrf_block(double* A, long long ld, int k0, int
     bool ok;
     switch (wave) {
         case 0: ok = potrf_factor_wave(blk, ld, k0, nb, inv, info, ps); break;
-        case 1: ok = potrf_mfma_wave<1>(blk, ld, nb, inv, invT, ps); break;
-        case 2: ok = potrf_mfma_wave<2>(blk, ld, nb, inv, invT, ps); break;
-        case 3: ok = potrf_mfma_wave<3>(blk, ld, nb, inv, invT, ps); break;
-        case 4: ok = potrf_store_wave(blk, ld, nb, inv, invT, steps, ps); break;
-        case 5: ok = potrf_mfma_wave<4>(blk, ld, nb, inv, invT, ps); break;
-        case 6: ok = potrf_mfma_wave<5>(blk, ld, nb, inv, invT, ps); break;
-        default: ok = potrf_mfma_wave<6>(blk, ld, nb, inv, invT, ps); break;
+        case 1: ok = potrf_mfma_wave<1>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
+        case 2: ok = potrf_mfma_wave<2>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
+        case 3: ok = potrf_mfma_wave<3>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
+        case 4: ok = potrf_store_wave(blk, ld, nb, inv, invT, HANDED_OUT ? steps : nullptr, ps); break;
+        case 5: ok = potrf_mfma_wave<4>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
+        case 6: ok = potrf_mfma_wave<5>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
+        default: ok = potrf_mfma_wave<6>(blk, ld, nb, inv, invT, HANDED_OUT, ps); break;
     }
     if (!ok) return false;                                        // every wavefront saw the same flag
     __syncthreads();
@@ -391,7 +401,7 @@ __global__ __launch_bounds__(PT, 4) void potrf_block_kernel(double* A, long long
                                                          double* invT, int* info) {
     __shared__ PotrfShared ps;
     if (*info != 0) return;
-    potrf_block(A, ld, k0, nb, inv, invT, info, nullptr, ps);
+    potrf_block<false>(A, ld, k0, nb, inv, invT, info, nullptr, ps);
 }
 
 // ---- one launch per panel -------------------------------------------------------------------
@@ -855,7 +865,7 @@ __global__ __launch_bounds__(PT, 2) void panel_kernel(double* A, long long ld, i
             publish(strip_done, FLAG_DONE);
         }
         double* inv = invs + (size_t)(j0 / NB) * 2 * NB * NB;     // the own diagonal tile: every update is in
-        const bool ok = potrf_block(A, ld, j0, NB, inv, inv + NB * NB, info, flags + STEPS + bid, ps);
+        const bool ok = potrf_block<true>(A, ld, j0, NB, inv, inv + NB * NB, info, flags + STEPS + bid, ps);
         // on failure every workgroup right of this column leaves at one of these flags, before it could wait for
         // anything that is now never set
         if (!ok && threadIdx.x == 0) store_past_caches(flags + STEPS + bid, FLAG_FAILED);
