@@ -603,6 +603,9 @@ size_t qmll_cholesky_workspace_bytes(int F);
 /* U = A on the 128 x 128 tiles on or above the diagonal (F x F, row strides lda and ldu): all that qmll_cholesky_f64 reads of a
  * matrix that the caller wants to keep.  The rest of U is not written. */
 int qmll_copy_upper_f64(const double* A, long long lda, int F, double* U, long long ldu, qmll_stream_t stream);
+/* The same into U [Fp,Fp], Fp >= F, whose diagonal goes on with ones and whose other entries past F are zero: the factor is that of A with
+ * ones behind it. */
+int qmll_copy_upper_padded_f64(const double* A, long long lda, int F, double* U, long long ldu, int Fp, qmll_stream_t stream);
 
 /* In-place fp64 Cholesky factorisation A = U^T U of the F x F matrix A (row-major, row stride ld
  * doubles, ld even).  Reads only elements on or above the diagonal; on exit they hold U.  Below

@@ -110,6 +110,7 @@ PROTOTYPES = {
     "qmll_gram_mirror_f64": [P, c_int, P],
     "qmll_cholesky_workspace_bytes": [c_int],
     "qmll_copy_upper_f64": [P, c_longlong, c_int, P, c_longlong, P],
+    "qmll_copy_upper_padded_f64": [P, c_longlong, c_int, P, c_longlong, c_int, P],
     "qmll_cholesky_slabs_bytes": [c_int],
     "qmll_cholesky_slabs_f64": [P, c_int, c_longlong, P, P, P, P],
     "qmll_cholesky_f64": [P, c_int, c_longlong, P, P, P],

@@ -1028,18 +1028,19 @@ __global__ __launch_bounds__(256) void fill_words64_kernel(unsigned long long* p
 
 // the 128 x 128 tiles on or above the diagonal of A into U (the lower ones are never read); grid (column, row of tiles)
 __global__ __launch_bounds__(256) void copy_upper_kernel(const double* __restrict__ A, long long lda, double* __restrict__ U,
-                                                         long long ldu, int F) {
+                                                         long long ldu, int F, int Fp) {
     if (blockIdx.x < blockIdx.y) return;
     const int c = blockIdx.x * NB + (threadIdx.x & 63) * 2, r0 = blockIdx.y * NB + (threadIdx.x >> 6);
     const bool pairs = c + 1 < F && (lda | ldu) % 2 == 0 && ((uintptr_t)A | (uintptr_t)U) % 16 == 0;
 #pragma unroll 8
-    for (int r = r0; r < min(F, (int)(blockIdx.y + 1) * NB); r += 4) {
+    for (int r = r0; r < min(Fp, (int)(blockIdx.y + 1) * NB); r += 4) {
         const double* from = A + (size_t)r * lda + c;
         double* to = U + (size_t)r * ldu + c;
-        if (pairs) *reinterpret_cast<double2_t*>(to) = *reinterpret_cast<const double2_t*>(from);
+        if (pairs && r < F) *reinterpret_cast<double2_t*>(to) = *reinterpret_cast<const double2_t*>(from);
         else {
-            if (c < F) to[0] = from[0];
-            if (c + 1 < F) to[1] = from[1];
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                if (c + k < Fp) to[k] = r < F && c + k < F ? from[k] : r == c + k ? 1.0 : 0.0;
         }
     }
 }
@@ -1125,11 +1126,16 @@ int factor_block(double* A, int F, long long ld, int P0, int k0, double* invs, i
 }  // namespace
 
 extern "C" int qmll_copy_upper_f64(const double* A, long long lda, int F, double* U, long long ldu, qmll_stream_t stream) {
-    QMLL_REQUIRE(F > 0 && lda >= F && ldu >= F, QMLL_ERR_INVALID, "qmll_copy_upper_f64: bad size F=%d lda=%lld ldu=%lld", F, lda, ldu);
+    return qmll_copy_upper_padded_f64(A, lda, F, U, ldu, F, stream);
+}
+
+extern "C" int qmll_copy_upper_padded_f64(const double* A, long long lda, int F, double* U, long long ldu, int Fp, qmll_stream_t stream) {
+    QMLL_REQUIRE(F > 0 && Fp >= F && lda >= F && ldu >= Fp, QMLL_ERR_INVALID, "qmll_copy_upper_f64: bad size F=%d of %d lda=%lld ldu=%lld", F, Fp,
+                 lda, ldu);
     QMLL_REQUIRE(A && U, QMLL_ERR_INVALID, "qmll_copy_upper_f64: null pointer");
-    const unsigned n = ((unsigned)F + NB - 1) / NB;
+    const unsigned n = ((unsigned)Fp + NB - 1) / NB;
     QMLL_REQUIRE(n <= 65535, QMLL_ERR_INVALID, "qmll_copy_upper_f64: F=%d too large", F);
-    hipLaunchKernelGGL(copy_upper_kernel, dim3(n, n), dim3(256), 0, (hipStream_t)stream, A, lda, U, ldu, F);
+    hipLaunchKernelGGL(copy_upper_kernel, dim3(n, n), dim3(256), 0, (hipStream_t)stream, A, lda, U, ldu, F, Fp);
     QMLL_CHECK_LAUNCH("qmll_copy_upper_f64");
     return QMLL_OK;
 }

@@ -1,5 +1,6 @@
 """The Cholesky factorisation's panels, whose columns follow the factorisation of a diagonal block step by step: one to four blocks in the
-last panel, with and without columns beside it; the first pivot that is not positive in each block; the same bits each time."""
+last panel, with and without columns beside it; the first pivot that is not positive in each block; the same bits each time.  Sizes that
+are no whole blocks are solved in a copy with ones behind the matrix."""
 import pytest
 import torch
 
@@ -15,13 +16,14 @@ def problem(F, seed):
     return A, A @ torch.randn(F, 1, device="cuda", dtype=torch.float64, generator=gen)
 
 
-@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 7, 8, 13])
-def test_blocks_of_a_panel(blocks):
+@pytest.mark.parametrize("F", [128 * blocks for blocks in (1, 2, 3, 4, 5, 6, 7, 8, 13)] + [2, 126, 130, 320, 510, 514, 1090])
+def test_blocks_of_a_panel(F):
     from qml_lightning_amd import ops
-    F = 128 * blocks
-    A, b = problem(F, blocks)
+    A, b = problem(F, F)
+    kept = A.clone(), b.clone()
     x, info = ops.cholesky_solve_spd(A, b)
-    assert int(info) == 0
+    assert int(info) == 0 and x.shape == b.shape
+    assert torch.equal(A, kept[0]) and torch.equal(b, kept[1])
     # backward error of a Cholesky solve: at most 3 (F + 1) eps |A| |x| for each component, and far below it as a rule
     bound = 3.0 * (F + 1) * 2.0 ** -53 * (A.abs() @ x.abs())
     assert ((A @ x - b).abs() <= 0.25 * bound).all()
@@ -29,11 +31,29 @@ def test_blocks_of_a_panel(blocks):
     assert torch.equal(again, x)
 
 
-@pytest.mark.parametrize("blocks,pivot", [(1, 77), (4, 5), (4, 130), (4, 300), (4, 511), (5, 200), (9, 640), (9, 900)])
+@pytest.mark.parametrize("blocks,pivot", [(1, 77), (4, 5), (4, 130), (4, 300), (4, 511), (5, 200), (9, 640), (9, 900), (2.5, 319), (4.5, 40)])
 def test_first_pivot_that_is_not_positive(blocks, pivot):
     from qml_lightning_amd import ops
-    F = 128 * blocks
+    F = int(128 * blocks)
     A, b = problem(F, 3)
     A[pivot, pivot] = -1.0
     _, info = ops.cholesky_solve_spd(A, b)
     assert int(info) == pivot + 1
+
+
+@pytest.mark.parametrize("F,offset", [(384, 1), (512, 1), (300, 1), (1090, 0)])
+def test_in_place_in_a_wider_buffer(F, offset):
+    """Rows 8 bytes past an aligned address: whole blocks are factored by a launch per step, the other sizes in their padded copy,
+    whose factor ends up in the matrix."""
+    from qml_lightning_amd import ops
+    A, b = problem(F, F)
+    wide = torch.full((F, F + 8), 7.0, device="cuda", dtype=torch.float64)
+    view = wide[:, offset:offset + F]
+    view.copy_(A)
+    x, info = ops.cholesky_solve_spd(view, b, overwrite_a=True)
+    assert int(info) == 0 and x.shape == b.shape
+    assert ((A @ x - b).abs() <= 0.75 * (F + 1) * 2.0 ** -53 * (A.abs() @ x.abs())).all()
+    U = torch.triu(view)
+    bound = 2 * (F + 1) * 2.0 ** -53 * (U.abs().T @ U.abs())        # (F + 1) eps for the factorisation, as much for the product here
+    assert ((U.T @ U - A).abs() <= bound).all()
+    assert (wide[:, :offset] == 7.0).all() and (wide[:, offset + F:] == 7.0).all()
