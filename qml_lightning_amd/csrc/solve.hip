@@ -13,7 +13,8 @@
 // above the diagonal.  The depth of 512 is what makes the trailing update MFMA-bound: at a
 // depth of 128 the read-modify-write of the trailing matrix dominates.
 // For whole tiles (F a multiple of 128) a panel and the trailing update of the panel before it are ONE
-// launch (panel_kernel below); any other F takes a launch per step with the tile kernel of gram.hip.
+// launch (panel_kernel below); any other F takes a launch per step with the tile kernel of gram.hip. A caller
+// that copies the matrix anyway pads it to whole tiles (qmll_copy_upper_padded_f64): 704 features 633 -> 356 us.
 // Only elements on or above the diagonal are read; below the diagonal only the lower halves of
 // the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.  Large matrices take the updates by all rows
 // but the last few thousand from the int8 matrix cores (slab_end below).

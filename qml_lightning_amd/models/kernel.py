@@ -365,7 +365,8 @@ class BaseKernel():
         flops; LU remains the fallback when rounding has left the matrix numerically indefinite.
 
         overwrite_a: A (symmetric, both triangles stored) may be used up.  The factorisation then
-        works in A itself instead of in a copy of it (2 GB at 16 384 features); it touches the
+        works in A itself instead of in a copy of it (2 GB at 16 384 features; sizes past 128 that are
+        no multiple of it are factored in a padded copy all the same, if there is memory for it); it touches the
         upper triangle and the 128 x 128 tiles on the diagonal only, so those tiles are kept aside
         (16 MB) and, should a pivot fail, A is put together again from them and its lower
         triangle before LU takes it."""
