@@ -14,7 +14,7 @@
 // depth of 128 the read-modify-write of the trailing matrix dominates.
 // For whole tiles (F a multiple of 128) a panel and the trailing update of the panel before it are ONE
 // launch (panel_kernel below); any other F takes a launch per step with the tile kernel of gram.hip. A caller
-// that copies the matrix anyway pads it to whole tiles (qmll_copy_upper_padded_f64): 704 features 633 -> 356 us.
+// that copies the matrix anyway pads it to whole tiles (qmll_copy_upper_padded_f64): 704 features 633 -> 348 us.
 // Only elements on or above the diagonal are read; below the diagonal only the lower halves of
 // the 128x128 diagonal tiles are overwritten.  Flops: F^3/3.  Large matrices take the updates by all rows
 // but the last few thousand from the int8 matrix cores (slab_end below).
@@ -910,6 +910,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* p, int n) {
 constexpr int ST = 512;            // threads of a solve workgroup
 constexpr int SQ = ST / NB;        // row quarters: thread (c = tid % 128, q = tid / 128) has rows 32 q .. 32 q + 31
 constexpr int SR = NB / SQ;
+typedef double columns_t __attribute__((ext_vector_type(2), aligned(8)));     // of any row: the matrix may be a view
 constexpr unsigned long long NOT_YET = 0x7FF8C0DEC0DE0001ULL;
 
 __device__ __forceinline__ unsigned long long peek(const double* p) {
@@ -973,7 +974,7 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
     __shared__ double part[SQ][NB], vec[NB];
     const int k = nblk - 1 - (int)blockIdx.x, k0 = k * NB;
     const int tid = threadIdx.x, lane = tid & 63, c = tid & (NB - 1), q = tid / NB;
-    const int csub = tid & 15, rowgrp = tid >> 4;          // sixteen lanes of eight columns along a row; rows rowgrp + 32 a
+    const int csub = tid & 15, rowgrp = tid >> 4;          // sixteen lanes of four pairs of columns along a row; rows rowgrp + 32 a
     const double* invT = invs + (size_t)k * 2 * NB * NB + NB * NB;
     double iv[SR];
 #pragma unroll
@@ -982,16 +983,27 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
 #pragma unroll
     for (int a = 0; a < 4; ++a) acc[a] = csub == 0 ? z[k0 + rowgrp + 32 * a] : 0.0;
     for (int j = nblk - 1; j > k; --j) {
-        const int col0 = j * NB + 8 * csub;
-        double u[4][8];
+        // columns 32 e + 2 csub and the next: a load takes 256 bytes of a row, where eight neighbouring columns a lane took 32 loads of a
+        // word in each of many lines: the launch 16.4 -> 10.5 us at 512 features, 63 -> 38 at 2048, 725 -> 419 at 16384.  One row a load, with
+        // all its columns in a wavefront, needs sums over 64 lanes at the end: 26, 100 and 796 us
+        const int col0 = j * NB + 2 * csub;
+        columns_t u[4][4];
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
             const double* row = U + (size_t)(k0 + rowgrp + 32 * a) * ld + col0;     // k < nblk - 1: a whole block of rows
+            if (j * NB + NB <= F) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) u[a][e] = col0 + e < F ? row[e] : 0.0;
+                for (int e = 0; e < 4; ++e) u[a][e] = *reinterpret_cast<const columns_t*>(row + 32 * e);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    u[a][e][0] = col0 + 32 * e < F ? row[32 * e] : 0.0;
+                    u[a][e][1] = col0 + 32 * e + 1 < F ? row[32 * e + 1] : 0.0;
+                }
+            }
         }
         // every wavefront polls the block's 128 values, two a lane, and hands each lane its eight (a lane that polled all it
-        // needs itself took eight loads a poll, and the launch 1.18 ms at 16384 features instead of 0.72)
+        // needs itself took eight loads a poll, and the launch 1.18 ms at 16384 features where this took 0.72)
         const double* theirs = xs + j * NB + 2 * lane;
         unsigned long long b0 = peek(theirs), b1 = peek(theirs + 1);
         for (unsigned n = 0; __builtin_amdgcn_ballot_w64(b0 == NOT_YET || b1 == NOT_YET) != 0ULL && n < spin_limit; ++n) {
@@ -1003,9 +1015,9 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
         const double x1 = b1 == NOT_YET ? __builtin_nan("") : __longlong_as_double((long long)b1);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const double xv = __shfl(e & 1 ? x1 : x0, 4 * csub + (e >> 1), 64);
+            const double xv = __shfl(e & 1 ? x1 : x0, csub + 16 * (e >> 1), 64);
 #pragma unroll
-            for (int a = 0; a < 4; ++a) acc[a] = fma(-u[a][e], xv, acc[a]);
+            for (int a = 0; a < 4; ++a) acc[a] = fma(-u[a][e >> 1][e & 1], xv, acc[a]);
         }
     }
 #pragma unroll

@@ -838,7 +838,7 @@ def cholesky_solve_spd(A, b, overwrite_a=False, within_norms=True):
         raise RuntimeError("cholesky_solve_spd: the row stride must be even")
     # Sizes that are no multiple of 128 are factored in a copy of whole blocks of 128, with ones on the diagonal behind A: one launch
     # per panel of four blocks instead of one per step of each, and the integer products from 7168 features on (704 features 633 ->
-    # 356 us, 1472 1400 -> 708, 16 002 45.6 -> 19.5 ms; 130 128 -> 104).  A single block has its one launch either way, and would pay
+    # 348 us, 1472 1400 -> 687, 16 002 45.6 -> 19.2 ms; 130 128 -> 102).  A single block has its one launch either way, and would pay
     # for the copy (64 features 48 -> 61 us).
     n = F
     U = A

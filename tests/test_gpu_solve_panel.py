@@ -57,3 +57,21 @@ def test_in_place_in_a_wider_buffer(F, offset):
     bound = 2 * (F + 1) * 2.0 ** -53 * (U.abs().T @ U.abs())        # (F + 1) eps for the factorisation, as much for the product here
     assert ((U.T @ U - A).abs() <= bound).all()
     assert (wide[:, :offset] == 7.0).all() and (wide[:, offset + F:] == 7.0).all()
+
+
+@pytest.mark.parametrize("F", [130, 255, 514, 642])
+def test_ragged_sizes_in_the_c_interface(F):
+    """The last block of the launches per step and of the two triangular solves ends inside a tile, in rows of any alignment."""
+    from qml_lightning_amd import _lib, ops
+    A, b = problem(F, F)
+    ld = F + 2 + F % 2                                  # even, as the interface asks for
+    U = torch.zeros(F, ld, device="cuda", dtype=torch.float64)
+    U[:, :F] = A
+    L = _lib.lib()
+    work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device="cuda")
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    x = b.clone()
+    _lib.check(L.qmll_cholesky_f64(ops._ptr(U), F, ld, ops._ptr(work), ops._ptr(info), ops._stream()), "qmll_cholesky_f64")
+    _lib.check(L.qmll_cholesky_solve_f64(ops._ptr(U), F, ld, ops._ptr(work), ops._ptr(x), ops._stream()), "qmll_cholesky_solve_f64")
+    assert int(info) == 0
+    assert ((A @ x - b).abs() <= 0.75 * (F + 1) * 2.0 ** -53 * (A.abs() @ x.abs())).all()
