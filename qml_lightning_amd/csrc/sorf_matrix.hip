@@ -64,8 +64,12 @@ __host__ __device__ constexpr int tile_atoms(int d) { return 16 * SM_WAVES / col
 constexpr float INV2PI = 0.15915494309189535f;
 constexpr float UMAX = 1500.0f * INV2PI;     // beyond, whole revolutions are taken off the sine argument first
 // One transform: x (in revolutions) goes times 2^SM_EXP into its two fp16 parts: an entry is then off by 2^-33 at most beside its 23
-// bits, far below the rounding of an argument, and atoms of sum |x| up to 128 revolutions fit
+// bits, and atoms of sum |x| up to 128 revolutions fit.  Beside an ordinary bias that is far below the rounding of an argument; where
+// some stack's bias is small (below a sixteenth of a revolution in the mean; phases drawn evenly have an eighth), an atom whose entries
+// are below SM_LEAST in the mean has a power of two of its own, as those beyond 128 have (no bias and sum |x| = 2e-3 revolutions at
+// d = 128: gradients 3.2e-6 off with the common one, 3.1e-7 so).
 constexpr int SM_EXP = 8;
+constexpr float SM_LEAST = 1.0f / 512, SMALL_BIAS = 1.0f / 16;
 
 // stacks per buffer: one barrier for so many (and at least 3 workgroups in LDS)
 constexpr int stacks_per_round(int d, int T) { return d * T <= 128 || d == 256 ? 2 : 1; }
@@ -92,7 +96,8 @@ __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h
 struct Forms {
     half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal.  d = 256: [ne][S], of the
                           // diagonals [T][256] in the order of row_place, then the sign bits of the halves [T][4][half, lane / 16][16 bytes]
-    float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1), infinite where a diagonal is not +-1
+    float* largest;       // [ne][S]: the largest entry of H D_1 H (one transform: 1, or 2 where the stack's bias is small), infinite where a
+                          // diagonal is not +-1
     // Bias in revolutions, reduced to a quarter either way in fp64: the smaller the argument, the less its rounding.  What is taken off is
     // whole halves, and the sign that an odd number of them gives cosine and sine is alpha's.
     float* bias;          // [ne][S][d]; with one transform what its accumulators start from, of which the stages over the block index make that;
@@ -188,6 +193,13 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
 #pragma unroll 8
         for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
         m = workgroup_max(m, wmax);      // (its barriers are also those between the writes of rev and the reads)
+        if constexpr (T == 1) {
+            float sum = 0.0f;
+            if (tid < 64)
+                for (int t = tid; t < D; t += 64) sum += fabsf((float)rev[t]);
+            sum = wave_sum(sum);         // (of the first wavefront)
+            if (sum < D * SMALL_BIAS) largest = 2.0f;
+        }
         const int k = max(scale_exponent(m) - block_bits<D>(), -126);
         if (tid < D) {
             double v = rev[tid];
@@ -446,9 +458,9 @@ __global__ __launch_bounds__(64 * SM_WAVES) __attribute__((amdgpu_waves_per_eu(2
             if constexpr (HALVES == 2) sum += __shfl_xor(sum, 8, 64);
             // Every argument is at most sum |x|, times the largest entry of H D_1 H for a second transform, + |bias|: where that
             // stays below UMAX no stack looks at its arguments.  One transform: below the second limit all atoms share one power of
-            // two, whose inverse is in the H_16 blocks.
-            const float bound = fmaf(sum, largest, 0.5f);
-            wide = __any(!(bound <= UMAX && (T == 2 || sum < (float)(1 << (15 - SM_EXP)))));
+            // two, whose inverse is in the H_16 blocks.  (Rows that are not there are zeros.)
+            const float bound = fmaf(sum, largest, 0.5f), least = largest > 1.0f ? D * SM_LEAST : 0.0f;
+            wide = __any(!(bound <= UMAX && (T == 2 || (sum < (float)(1 << (15 - SM_EXP)) && (sum >= least || sum == 0.0f)))));
             const int kx = T == 1 && !wide ? SM_EXP : not_finite(sum) ? 0 : scale_exponent(sum);
             const float sx = pow2i(kx);
             inv = pow2i((T == 1 ? SM_EXP : 0) - kx);
