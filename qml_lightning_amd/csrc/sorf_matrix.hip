@@ -91,7 +91,7 @@ __host__ __device__ constexpr int image_bytes(int d, int T) { return d == 256 ? 
 // one 16-point block operand: half t of lane (i, q) is sign * H_16[i][4q + t % 4]
 __device__ __forceinline__ bool h16_negative(int i, int h) { return __popc(i & h) & 1; }
 
-// What a launch needs of the model beside its tensors.  Made by every call (sorf_prepare_kernel, 4 us of 150 and more): nothing
+// What a launch needs of the model beside its tensors.  Made by every call (sorf_prepare_kernel, 4 us of 150 and more up to 128 stacks): nothing
 // is kept that a write to the tensors could leave behind, and no other stream or captured graph has to wait for it.
 struct Forms {
     half8_t* images;      // [ne][S][T][NB][64 lanes]: the H_16 blocks behind the signs of their diagonal.  d = 256: [ne][S], of the
@@ -104,6 +104,7 @@ struct Forms {
                           // this and alpha in the order of row_place
     float* alpha;         // [ne][S][d] +-2^k alpha with the largest entry at [2^13, 2^14) / NB (a transform's register part sums NB of them),
                           // then 2^-k
+    float* pieces;        // [alpha_pieces]: the largest entry of each piece of alpha
     int* unfit;           // 1: some diagonal is not +-1, and sorf_energy_rows_kernel takes the call
 };
 
@@ -118,8 +119,24 @@ __device__ __forceinline__ float workgroup_max(float m, float* wmax) {
     return m;
 }
 
-// a workgroup per (element, stack).  bias and alpha may both be null: the images and bounds alone.  The blocks are +-factor.
+// The call's scale of alpha comes from its largest entry, which every workgroup of sorf_prepare_kernel has to know.  Up to ALPHA_ALONE
+// entries each looks through all of alpha itself; that is S workgroups' reads of S D entries, and beyond a launch ahead finds the largest
+// of every ALPHA_PIECE of them and the workgroups look through those.  Whole calls of four elements at d = 128, alone / so: 512 stacks, 3000
+// atoms 163 / 154 us, energies only 98 / 88; 2048 stacks, 1500 atoms 526 / 292 and 397 / 161; 256 stacks (32768 entries) 127 / 128.
 constexpr int PREP_THREADS = 512;
+constexpr int ALPHA_ALONE = 32768, ALPHA_PIECE = 8192;
+__host__ __device__ constexpr int alpha_pieces(int S, int D) { return (int)(((long long)S * D + ALPHA_PIECE - 1) / ALPHA_PIECE); }
+__global__ __launch_bounds__(PREP_THREADS) void sorf_alpha_pieces_kernel(const float* __restrict__ alpha, int n, float* __restrict__ largest) {
+    __shared__ float wmax[PREP_THREADS / 64];
+    const int begin = blockIdx.x * ALPHA_PIECE, end = n - begin < ALPHA_PIECE ? n : begin + ALPHA_PIECE;
+    float m = 0.0f;
+#pragma unroll 8
+    for (int t = begin + threadIdx.x; t < end; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
+    m = workgroup_max(m, wmax);
+    if (threadIdx.x == 0) largest[blockIdx.x] = m;
+}
+
+// a workgroup per (element, stack).  bias and alpha may both be null: the images and bounds alone.  The blocks are +-factor.
 template <int D, int T>
 __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float* __restrict__ Dmat, const float* __restrict__ bias,
                                                                     const float* __restrict__ alpha, int S, float factor, Forms f) {
@@ -190,8 +207,10 @@ __global__ __launch_bounds__(PREP_THREADS) void sorf_prepare_kernel(const float*
             rev[tid] = fma(b, 0.15915494309189533577, -0.5 * n);
         }
         float m = 0.0f;                  // the call's scale of alpha: every workgroup finds the same value
+        const float* from = S * D > ALPHA_ALONE ? f.pieces : alpha;
+        const int entries = S * D > ALPHA_ALONE ? alpha_pieces(S, D) : S * D;
 #pragma unroll 8
-        for (int t = tid; t < S * D; t += PREP_THREADS) m = fmaxf(m, finite_abs(alpha[t]));
+        for (int t = tid; t < entries; t += PREP_THREADS) m = fmaxf(m, finite_abs(from[t]));
         m = workgroup_max(m, wmax);      // (its barriers are also those between the writes of rev and the reads)
         if constexpr (T == 1) {
             float sum = 0.0f;
@@ -718,6 +737,7 @@ static size_t matrix_workspace(char* base, int A, int ne, int T, int S, int d, i
     };
     f.images = (half8_t*)take((size_t)ne * S * image_bytes(d, T));
     f.largest = (float*)take((size_t)ne * S * sizeof(float));
+    f.pieces = (float*)take(alpha_pieces(S, d) * sizeof(float));
     f.unfit = (int*)take(sizeof(int));
     f.bias = (float*)take((size_t)ne * S * d * sizeof(float));
     f.alpha = (float*)take(((size_t)ne * S * d + 1) * sizeof(float));
@@ -743,15 +763,21 @@ extern "C" size_t qmll_sorf_matrix_workspace_bytes(int A, int ne, int T, int S, 
 // 24000 (1.5) 111 / 101; d = 64 30000 (1.0) 68 / 71, 40000 (1.3) 87 / 79; d = 256, where the rows kernel has few wavefronts per SIMD, 4000
 // (0.5) 70 / 78, 6000 (0.8) 101 / 86.  Energies only: d = 128 10000 (1.3) 61 / 64, 12000 (1.5) 71 / 68; d = 64 18000 (1.2) 54 / 53; d = 256
 // 5000 (1.3) 63 / 67, 7000 (1.8) 85 / 82; two transforms, d = 128 24000 (1.5) 61 / 63, d = 256 14000 (1.8) 76 / 77.
+// The same product of more stacks and fewer atoms makes more forms, and more parts of each tile: with the gradient, d = 128, 256 stacks 6000
+// atoms (1.5) 118 / 128, 384 4000 (1.5) 122 / 138, 512 3000 (1.5) 125 / 154 and 3515 (1.8) 160 / 160, 2048 878 (1.8) 175 / 283 and 1318 (2.7)
+// 339 / 292; d = 64, 2048 1757 (1.8) 183 / 199; two transforms, d = 128, 128 4687 (1.2) 100 / 112 and 7031 (1.8) 134 / 129, 512 1171 (1.2)
+// 188 / 205.  At d = 256 the rows kernel has as few workgroups then: 512 stacks 1171 atoms (1.2) 190 / 167.
 extern "C" int qmll_sorf_matrix_pays(int A, int ne, int T, int S, int d, int with_grad) {
     if (!matrix_shape(ne, T, S, d) || matrix_units(A, ne, T, S, d) >= (1ll << 31)) return 0;
-    const double line = with_grad ? (T == 1 ? 1.5e6 : d == 256 ? 0.75e6 : 1.2e6) : (T == 1 ? 1.5e6 : 1.8e6);
+    double line = with_grad ? (T == 1 ? 1.5e6 : d == 256 ? 0.75e6 : 1.2e6) : (T == 1 ? 1.5e6 : 1.8e6);
+    if (with_grad && d <= 128) line = std::min(2e6, line * pow(std::max(1.0, S / (T == 1 ? 128.0 : 32.0)), 1.0 / 6.0));
     return (double)A * S * T * d / 128.0 >= line;
 }
 
 static void launch_prepare(const float* D, const float* bias, const float* alpha, int ne, int T, int S, int d, float factor,
                            const Forms& f, hipStream_t st) {
     const dim3 grid(ne * S), block(PREP_THREADS);
+    if (alpha && S * d > ALPHA_ALONE) hipLaunchKernelGGL(sorf_alpha_pieces_kernel, dim3(alpha_pieces(S, d)), block, 0, st, alpha, S * d, f.pieces);
     if (d == 64 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<64, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else if (d == 64) hipLaunchKernelGGL((sorf_prepare_kernel<64, 2>), grid, block, 0, st, D, bias, alpha, S, factor, f);
     else if (d == 128 && T == 1) hipLaunchKernelGGL((sorf_prepare_kernel<128, 1>), grid, block, 0, st, D, bias, alpha, S, factor, f);

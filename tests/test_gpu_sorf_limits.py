@@ -81,3 +81,36 @@ def test_small_arguments_without_bias(monkeypatch, d, steep, size, alone):
         _, gx = ops.sorf_energy_sorted(x, ti32([0, n]), ti32(np.arange(n)), D, b, alpha, norm, 1, n)
         errors[name] = float(((gx.double() - gr)[small].norm() / gr[small].norm()))
     assert errors["matrix"] <= 1.5 * errors["rows"], errors
+
+
+@pytest.mark.parametrize("d,S", [(128, 256), (128, 257), (64, 513), (256, 200)])      # 32768 entries, and more
+@pytest.mark.parametrize("T", [1, 2])
+def test_scale_of_many_coefficients(monkeypatch, d, S, T):
+    """The largest alpha may be in any piece of it, and infinite ones do not count: the entries around it are tiny, and the answer is
+    that of the rows kernel to a few 2^-24 of the sums."""
+    monkeypatch.setattr(_lib.lib(), "qmll_sorf_matrix_pays", lambda *a: 1)
+    n, ne, F = 40, 2, S * d
+    g = torch.Generator(device="cuda").manual_seed(S)
+    D = torch.randint(0, 2, (ne, T, S, d), device="cuda", generator=g).float() * 2 - 1
+    b = 6.28 * torch.rand(ne, F, device="cuda", generator=g)
+    x = torch.randn(n, d, device="cuda", generator=g)
+    off, slots = ti32([0, 17, n]), ti32(np.arange(n))
+    for at in (0, 8191, 8192, F // 2, F - 1):
+        alpha = 1e-6 * torch.randn(F, device="cuda", generator=g)
+        alpha[at] = 3e4
+        got = {}
+        for name in ("rows", "matrix"):
+            monkeypatch.setattr(_lib.lib(), "qmll_sorf_matrix_pays", lambda *a: int(name == "matrix"))
+            got[name] = ops.sorf_energy_sorted(x, off, slots, D, b, alpha, 1.5, T, n)
+        for r, m in zip(got["rows"], got["matrix"]):
+            assert torch.isfinite(m).all()
+            assert (m - r).norm() <= 1e-5 * r.norm()
+
+
+def test_few_atoms_of_many_stacks_stay_on_the_rows_kernel():
+    """With the gradient and up to 128 components the line between the two kernels rises with the stacks, as the forms and the parts of a
+    tile do."""
+    pays = _lib.lib().qmll_sorf_matrix_pays
+    for T, S, low, high in ((1, 128, 11600, 11900), (1, 512, 3600, 3800), (1, 2048, 970, 980), (2, 32, 18700, 18800), (2, 512, 1800, 1960)):
+        assert not pays(low, 4, T, S, 128, 1) and pays(high, 4, T, S, 128, 1), (T, S)
+    assert pays(1000, 4, 2, 200, 256, 1) and pays(12100, 4, 1, 128, 128, 0) and pays(3000, 4, 1, 512, 128, 0)
