@@ -354,13 +354,18 @@ __device__ __forceinline__ float root(float x, float inv) {
 constexpr int RS3_GROUP = 5;
 
 // The spacing of the bins u (lane: bin l, if ok) about the middle of the range, to a rounding of the grid's, or 0: uneven, or
-// so wide that Q could leave 2^16 (y is within mid of the middle) or exp2(2 h u) 2^8.
-__device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid) {
+// so wide that Q could leave 2^(2 line) (y is within mid of the middle) or exp2(2 h u) 2^line.  Q^4 times a coefficient has to be finite, since the
+// weight before it may have underflown: with a line of 13 it is for coefficients of 10^6 and more (20 bins with eta3 = 2.7 up to 8.1 A, 17
+// up to 7.5).  Where distances may be anything, see group_ratio, it is 8 (6.4 and 5.9 A).  What is beyond takes its bins one by one, about the
+// middle of the range.  42000 atoms of 21, three elements, backward, in groups / one by one: 6 A 78 / 84 us, 8 A 89 / 97 (plain weights 99), 17 bins at
+// 6 A 78 / 84; 16 x 96 atoms 27.3 / 27.5 (28.1), at 8 A - / 52.6 (54.2), at 10 A - / 63.1 (65.0).
+constexpr float LINE_WITHIN = 13.0f, LINE_ANY = 8.0f;
+__device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid, float line) {
     const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(u)));
     const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(u), nRs3 - 1));
     const float h = (last - first) * frcp((float)(nRs3 - 1));
     const float edge = fmaxf(fabsf(first), fabsf(last)), widest = mid + edge;
-    const bool fits = fabsf(fmaf((float)-l, h, u - first)) <= 2.4e-7f * widest && widest * fabsf(h) <= 8.0f && edge * fabsf(h) <= 4.0f;
+    const bool fits = fabsf(fmaf((float)-l, h, u - first)) <= 2.4e-7f * widest && widest * fabsf(h) <= line && edge * fabsf(h) <= 0.5f * line;
     return __any(ok && !fits) ? 0.0f : h;
 }
 
@@ -371,7 +376,8 @@ __device__ __forceinline__ float even_spacing_pairs(float ua, float ub, int l, i
     const float h = (last - first) * frcp((float)(nRs3 - 1));
     const float edge = fmaxf(fabsf(first), fabsf(last)), widest = mid + edge, slack = 2.4e-7f * widest;
     const float at = fmaf((float)(2 * l), h, first);
-    const bool fits = fabsf(ua - at) <= slack && (2 * l + 1 >= nRs3 || fabsf(ub - at - h) <= slack) && widest * fabsf(h) <= 8.0f && edge * fabsf(h) <= 4.0f;
+    const bool fits = fabsf(ua - at) <= slack && (2 * l + 1 >= nRs3 || fabsf(ub - at - h) <= slack) && widest * fabsf(h) <= LINE_ANY &&
+                      edge * fabsf(h) <= 0.5f * LINE_ANY;
     return __any(2 * l < nRs3 && !fits) ? 0.0f : h;
 }
 
@@ -383,8 +389,8 @@ __device__ __forceinline__ float group_factor(float u, int l, int lane, float h)
 }
 
 // exp2(2 h y), the factor of Q that all groups share, and what the product's rounding left out: Q goes to the fourth power.
-// STOP: distances from a given list may be anything.  It stops at 2^18, which no y within mid of the middle reaches (with the default
-// grid the weights are below 2^-80 there), and Q^4 stays in range.
+// STOP: distances from a given list may be anything.  It stops at 2^18, which no y within mid of the middle reaches behind LINE_ANY (the weights
+// are below 2^-60 there), and Q^4 stays in range.
 template <bool STOP>
 __device__ __forceinline__ float group_ratio(float h, float y) {
     const float x = 2.0f * h * y, e = fexp2(STOP ? fminf(x, 18.0f) : x);
@@ -1593,12 +1599,12 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // factor does not depend on the triple and goes into the staged gradient once per atom; the first
     // is one fma and the exponential per (triple, bin).  It is at most 2^(u_l^2), so the form is taken
     // only while u_l^2 <= 100 for every bin (eta3 rcut^2 up to about 270); beyond, the plain form runs.
-    // LEAN: see group_sums; where the grid is not even, the plain form.
+    // LEAN: see group_sums; where the grid is not even, these two forms.
     const float mid = 0.5f * sk3 * a.p.rcut;
     const float ul = LEAN && lane < nRs3 ? fmaf(sk3, rs3v, -mid) : 0.0f;
-    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid) : 0.0f;
+    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid, LINE_ANY) : 0.0f;
     const bool even = LEAN && spacing != 0.0f;
-    bool fast = false;
+    bool fast = LEAN && !__any(!(fabsf(ul) <= 10.0f));
     if constexpr (!LEAN) {
         float um = fabsf(fmaf(sk3, rs3v, -mid));
         if (lane >= nRs3) um = 0.0f;
@@ -1623,7 +1629,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     if (lane < nRs2 && wave == 0) slnRs2[lane] = flog(rs2v);
     for (int t = tid + QMLL_WAVE; t < nRs2; t += NT) slnRs2[t] = flog(a.Rs2[t]);
     if constexpr (LEAN) {
-        const float f = a.gscale * (even ? group_factor(ul, lane, lane, spacing) : 1.0f);
+        const float f = a.gscale * (even ? group_factor(ul, lane, lane, spacing) : fast ? fexp2(-ul * ul) : 1.0f);
         if (tid < nRs3) sfac[tid] = f;
     }
     for (int t = LEAN ? nRs3 : tid; t < nRs3; t += NT) {
@@ -1705,7 +1711,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     const float d3 = a.p.three_body_decay;
     float us[LEAN ? LEAN_RS3 : 1], ratio[LEAN_RS3 / RS3_GROUP];        // the grid, on scalar registers
     if constexpr (LEAN) {
-        const float v = fexp2(-2.0f * spacing * ul);
+        const float v = group_ratio<false>(-spacing, ul);
 #pragma unroll
         for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
 #pragma unroll
@@ -1907,8 +1913,8 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
     const float hfac = -2.0f * a.p.eta3 * frcp(sk3);
     const float mid = 0.5f * sk3 * a.p.rcut;             // distances and bins about the middle of the range: half the rounding
     const float ul = bin_ok ? fmaf(sk3, rs3v, -mid) : 0.0f;
-    const float spacing = even_spacing(ul, l3, bin_ok, nRs3, mid);
-    const bool even = spacing != 0.0f;
+    const float spacing = even_spacing(ul, l3, bin_ok, nRs3, mid, LINE_WITHIN);
+    const bool even = spacing != 0.0f, fast = !__any(!(fabsf(ul) <= 10.0f));        // see fchl19_vjp_kernel for the forms
 
     // ---- neighbours: candidate = lane ----
     float dx = Xm[i * 3 + 0] - xo, dy = Xm[i * 3 + 1] - yo, dz = Xm[i * 3 + 2] - zo;
@@ -1942,9 +1948,10 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
         sj[pos] = lane;
     }
     // the incoming gradient, times the constant factor of its bin
+    const float f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : fast ? fexp2(-ul * ul) : 1.0f);
     if constexpr (!ONE) {
         gsrc = gradient();
-        const float f2 = a.gscale * frcp(rs2v), f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
+        const float f2 = a.gscale * frcp(rs2v);
         if (wave == 0 && lane < 32) slnRs2[lane] = flog(rs2v);
         for (int e = 2 * wave + (lane >> 5); e < NS; e += 2 * NW) gin2[32 * e + z] = z < nRs2 ? gsrc[e * nRs2 + z] * f2 : 0.0f;
         for (int pq = 3 * wave + third; pq < NP; pq += 3 * NW) {
@@ -1953,7 +1960,7 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
             if (lane < STEP) reinterpret_cast<float2*>(gin3)[LEAN_RS3 * pq + l3] = g;
         }
     } else {
-        const float f2 = a.gscale * frcp(rs2v), f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
+        const float f2 = a.gscale * frcp(rs2v);
         if (lane < 32) slnRs2[lane] = flog(rs2v);
 #pragma unroll
         for (int k = 0; k < (NS + 1) / 2; ++k)
@@ -2011,7 +2018,7 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
 #pragma unroll
     for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
     {
-        const float v = fexp2(-2.0f * spacing * ul);
+        const float v = group_ratio<false>(-spacing, ul);
 #pragma unroll
         for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) ratio[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), RS3_GROUP * q));
     }
@@ -2077,20 +2084,36 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
                 group_sums(g2 + RS3_GROUP * q, d, fexp2(-(d * d)), B * ratio[q], spacing, Gc, Gs, Hc, Hs);
             }
         } else {
-            auto bin = [&](float gc, float gs, float u) {
-                const float dl = y - u;
-                const float e = fexp2(-(dl * dl));
-                const float de = dl * e;
-                Gc = fmaf(gc, e, Gc);
-                Gs = fmaf(gs, e, Gs);
-                Hc = fmaf(gc, de, Hc);
-                Hs = fmaf(gs, de, Hs);
-            };
+            auto bins = [&](auto bin) {
 #pragma unroll
-            for (int l = 0; l < LEAN_RS3; l += 2) {
-                const float4 gv = g[l / 2];
-                bin(gv.x, gv.y, us[l]);
-                bin(gv.z, gv.w, us[l + 1]);
+                for (int l = 0; l < LEAN_RS3; l += 2) {
+                    const float4 gv = g[l / 2];
+                    bin(gv.x, gv.y, us[l]);
+                    bin(gv.z, gv.w, us[l + 1]);
+                }
+            };
+            if (fast) {
+                const float y2 = y + y, ny2 = -y * y;
+                bins([&](float gc, float gs, float u) {
+                    const float e = fexp2(fmaf(y2, u, ny2));
+                    const float ue = u * e;
+                    Gc = fmaf(gc, e, Gc);
+                    Gs = fmaf(gs, e, Gs);
+                    Hc = fmaf(gc, ue, Hc);
+                    Hs = fmaf(gs, ue, Hs);
+                });
+                Hc = fmaf(y, Gc, -Hc);
+                Hs = fmaf(y, Gs, -Hs);
+            } else {
+                bins([&](float gc, float gs, float u) {
+                    const float dl = y - u;
+                    const float e = fexp2(-(dl * dl));
+                    const float de = dl * e;
+                    Gc = fmaf(gc, e, Gc);
+                    Gs = fmaf(gs, e, Gs);
+                    Hc = fmaf(gc, de, Hc);
+                    Hs = fmaf(gs, de, Hs);
+                });
             }
         }
         const float S0 = Gc * cosT + Gs * sinT;

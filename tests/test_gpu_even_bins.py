@@ -66,3 +66,28 @@ def test_weights_beyond_the_range_of_the_ratio(kw, natoms):
 @pytest.mark.parametrize("spread", [1.3, 4.0])
 def test_distances_beyond_the_cutoff(spread):
     check(30, 1, 20, "even", 3, spread=spread)
+
+
+@pytest.mark.parametrize("natoms", [12, 50, 66])
+@pytest.mark.parametrize("nrs3,kw", [(20, dict(rcut=6.4)), (20, dict(rcut=6.5)), (17, dict(rcut=6.0)), (20, dict(rcut=8.0)), (20, dict(rcut=8.1)),
+                                     (20, dict(rcut=8.2)), (17, dict(rcut=8.0)), (20, dict(rcut=10.0))])
+def test_either_side_of_the_lines(nrs3, kw, natoms):
+    """Cutoffs around those up to which even bins are taken in groups (6.4 A where distances may be anything, 8.1 A for molecules of up to 64 atoms),
+    and beyond: the bins one by one, about the middle of the range."""
+    check(natoms, 1, nrs3, "even", 7, **kw)
+
+
+@pytest.mark.parametrize("size", [1e-12, 1e6])
+def test_gradients_of_any_size(size):
+    """The sums over a group reach 2^104 of its coefficients where the weight before them has underflown."""
+    from qml_lightning_amd import ops
+    rng = np.random.default_rng(2)
+    coords, charges = helpers.fixed_composition_batch(rng.choice([1, 6, 8], 30), 1, 2, box=14.0)
+    prm = oracle_prm([1, 6, 8], rcut=8.1)
+    X, Z, aid, mid, nat = make_batch(coords, charges)
+    types = fchl19.element_types(Z, nat, prm.species)
+    args = [t32(X), ti32(types), None, None, ti32(aid), ti32(mid), ti32(nat), t32(prm.Rs2), t32(prm.Rs3), gpu_prm(prm)]
+    g = torch.randn(X.shape[0], X.shape[1], prm.nspecies * prm.nRs2 + prm.nspecies * (prm.nspecies + 1) * prm.nRs3, device="cuda")
+    ref = ops.fchl_vjp(g, *args)
+    got = ops.fchl_vjp(g * size, *args) / size
+    assert torch.isfinite(got).all() and (got - ref).norm() <= 1e-5 * ref.norm()
