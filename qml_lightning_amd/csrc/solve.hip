@@ -902,6 +902,8 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* p, int n) {
 // through memory per step of the chain.  Every workgroup waits only for workgroups with lower ids (the backward
 // launch numbers the blocks from the end), so whoever is waited for is running or done; the waits are bounded
 // all the same, and one that runs out hands on a NaN, which ends up in the solution instead of a wrong number.
+// Every sum is four, put together at its end: as fast (a step is its trip through memory), and its rounding errors add up over a quarter as many
+// terms.
 constexpr int ST = 512;            // threads of a solve workgroup
 constexpr int SQ = ST / NB;        // row quarters: thread (c = tid % 128, q = tid / 128) has rows 32 q .. 32 q + 31
 constexpr int SR = NB / SQ;
@@ -920,10 +922,10 @@ __device__ __forceinline__ void hand_on(double* p, double v) {
 // out[c] = sum_m M[m,c] vec[m] with the thread's 32 rows of M in registers; the four partial sums through LDS
 __device__ __forceinline__ double block_product(const double (&iv)[SR], const double* vec, double (*part)[NB], int c,
                                                 int q) {
-    double s = 0.0;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int m = 0; m < SR; ++m) s = fma(iv[m], vec[SR * q + m], s);
-    part[q][c] = s;
+    for (int m = 0; m < SR; ++m) s[m & 3] = fma(iv[m], vec[SR * q + m], s[m & 3]);
+    part[q][c] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
     return (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
 }
@@ -938,7 +940,7 @@ __global__ __launch_bounds__(ST) void fwd_solve_kernel(const double* U, long lon
 #pragma unroll
     for (int m = 0; m < SR; ++m) iv[m] = inv[(SR * q + m) * NB + c];
     const bool colok = k0 + c < F;
-    double acc = (q == 0 && colok) ? b[k0 + c] : 0.0;
+    double acc[4] = {(q == 0 && colok) ? b[k0 + c] : 0.0, 0.0, 0.0, 0.0};
     for (int i = 0; i < k; ++i) {
         const double* tile = U + (size_t)(i * NB + SR * q) * ld + k0 + c;
         double u[SR];
@@ -953,9 +955,9 @@ __global__ __launch_bounds__(ST) void fwd_solve_kernel(const double* U, long lon
         }
         const double zr = bits == NOT_YET ? __builtin_nan("") : __longlong_as_double((long long)bits);
 #pragma unroll
-        for (int r = 0; r < SR; ++r) acc = fma(-u[r], value_of_lane(zr, r), acc);
+        for (int r = 0; r < SR; ++r) acc[r & 3] = fma(-u[r], value_of_lane(zr, r), acc[r & 3]);
     }
-    part[q][c] = acc;
+    part[q][c] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     __syncthreads();
     if (tid < NB) vec[tid] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
     __syncthreads();
@@ -974,9 +976,12 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
     double iv[SR];
 #pragma unroll
     for (int m = 0; m < SR; ++m) iv[m] = invT[(SR * q + m) * NB + c];
-    double acc[4];
+    double acc[4][4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) acc[a] = csub == 0 ? z[k0 + rowgrp + 32 * a] : 0.0;
+    for (int a = 0; a < 4; ++a) {
+        acc[a][0] = csub == 0 ? z[k0 + rowgrp + 32 * a] : 0.0;
+        acc[a][1] = acc[a][2] = acc[a][3] = 0.0;
+    }
     for (int j = nblk - 1; j > k; --j) {
         // columns 32 e + 2 csub and the next: a load takes 256 bytes of a row, where eight neighbouring columns a lane took 32 loads of a
         // word in each of many lines: the launch 16.4 -> 10.5 us at 512 features, 63 -> 38 at 2048, 725 -> 419 at 16384.  One row a load, with
@@ -1012,14 +1017,15 @@ __global__ __launch_bounds__(ST) void bwd_solve_kernel(const double* U, long lon
         for (int e = 0; e < 8; ++e) {
             const double xv = __shfl(e & 1 ? x1 : x0, csub + 16 * (e >> 1), 64);
 #pragma unroll
-            for (int a = 0; a < 4; ++a) acc[a] = fma(-u[a][e >> 1][e & 1], xv, acc[a]);
+            for (int a = 0; a < 4; ++a) acc[a][e & 3] = fma(-u[a][e >> 1][e & 1], xv, acc[a][e & 3]);
         }
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
+        double sum = (acc[a][0] + acc[a][1]) + (acc[a][2] + acc[a][3]);
 #pragma unroll
-        for (int m = 8; m >= 1; m >>= 1) acc[a] += __shfl_xor(acc[a], m, 16);
-        if (csub == 0) vec[rowgrp + 32 * a] = acc[a];
+        for (int m = 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 16);
+        if (csub == 0) vec[rowgrp + 32 * a] = sum;
     }
     __syncthreads();
     const double xk = block_product(iv, vec, part, c, q);

@@ -75,3 +75,32 @@ def test_ragged_sizes_in_the_c_interface(F):
     _lib.check(L.qmll_cholesky_solve_f64(ops._ptr(U), F, ld, ops._ptr(work), ops._ptr(x), ops._stream()), "qmll_cholesky_solve_f64")
     assert int(info) == 0
     assert ((A @ x - b).abs() <= 0.75 * (F + 1) * 2.0 ** -53 * (A.abs() @ x.abs())).all()
+
+
+@pytest.mark.parametrize("F", [1024, 4096])
+def test_sums_of_the_triangular_solves(F):
+    """U with a unit diagonal and all entries of one sign, so that the products of a row add up: a running sum over F terms is off by some
+    sqrt(F) roundings, four of a quarter of the terms by fewer.  The residual in long double."""
+    import numpy as np
+    from qml_lightning_amd import _lib, ops
+    L = _lib.lib()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(F)
+    U = torch.triu(torch.rand(F, F, device="cuda", dtype=torch.float64, generator=gen) / F, 1)
+    U.diagonal().add_(1.0)
+    A = U.T @ U
+    x = torch.rand(F, device="cuda", dtype=torch.float64, generator=gen)
+    work = torch.empty(int(L.qmll_cholesky_workspace_bytes(F)) // 8 + 1, dtype=torch.float64, device="cuda")
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(L.qmll_cholesky_f64(ops._ptr(A), F, F, ops._ptr(work), ops._ptr(info), ops._stream()), "qmll_cholesky_f64")
+    assert int(info) == 0
+    V = torch.triu(A)                                   # the factor as it was stored
+    Vh = V.cpu().numpy().astype(np.longdouble)
+    b = Vh.T @ (Vh @ x.cpu().numpy().astype(np.longdouble))
+    bd = b.astype(np.float64)
+    sol = torch.as_tensor(bd, device="cuda").clone()
+    _lib.check(L.qmll_cholesky_solve_f64(ops._ptr(A), F, F, ops._ptr(work), ops._ptr(sol), ops._stream()), "qmll_cholesky_solve_f64")
+    got = sol.cpu().numpy().astype(np.longdouble)
+    residual = Vh.T @ (Vh @ got) - bd.astype(np.longdouble)
+    # of either size 0.10 sqrt(F) eps, where one running sum per row or column gave 0.17
+    assert np.linalg.norm(residual) <= 0.13 * F ** 0.5 * 2.0 ** -53 * np.linalg.norm(b)
