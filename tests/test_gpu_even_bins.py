@@ -1,5 +1,5 @@
-"""The radial bins of the three-body part: kernels for 17 to 20 of them take evenly spaced ones in groups of five (a polynomial in the
-ratio of two weights) and any others one by one; both against the oracle on the same grid, and distances far beyond the cutoff from a
+"""The radial bins of the three-body part: kernels for 17 to 20 of them take evenly spaced ones of ordinary cutoffs in groups of five (a
+polynomial in the ratio of two weights) and any others one by one; both against the oracle on the same grid, and distances far beyond the cutoff from a
 given list.  Tolerance: largest error over largest value, REL_REP; forces are sums of both signs over the bins, ten times that
 (2-norm errors are 2e-7 to 6e-7 on either route)."""
 import numpy as np
@@ -54,6 +54,8 @@ def test_grids(grid, natoms, molecules):
 @pytest.mark.parametrize("nrs3", [17, 18, 19])
 @pytest.mark.parametrize("natoms,molecules", [(14, 2), (50, 1)])
 def test_bins_that_are_not_there(nrs3, natoms, molecules):
+    """(17 of them, 0.35 A apart, are taken in groups where distances end at the cutoff, in molecules of up to 64 atoms on one wavefront, and one by
+    one elsewhere.)"""
     check(natoms, molecules, nrs3, "even", nrs3)
 
 

@@ -59,6 +59,24 @@ def test_in_place_in_a_wider_buffer(F, offset):
     assert (wide[:, :offset] == 7.0).all() and (wide[:, offset + F:] == 7.0).all()
 
 
+@pytest.mark.parametrize("F,beside", [(128, 2), (512, 2), (512, 8), (640, 2), (1152, 2), (1664, 6)])
+def test_panels_in_a_wider_buffer(F, beside):
+    """Whole blocks whose rows are longer than the matrix, aligned as the panels' launches need: tiles side by side then share lines of
+    memory at their edges, and what is beside the matrix stays."""
+    from qml_lightning_amd import ops
+    A, b = problem(F, F)
+    plain, _ = ops.cholesky_solve_spd(A, b)
+    wide = torch.full((F, F + beside), 7.0, device="cuda", dtype=torch.float64)
+    view = wide[:, :F]
+    view.copy_(A)
+    assert view.data_ptr() % 16 == 0
+    x, info = ops.cholesky_solve_spd(view, b, overwrite_a=True)
+    assert int(info) == 0 and torch.equal(x, plain)          # the same sums in the same order
+    U = torch.triu(view)
+    assert ((U.T @ U - A).abs() <= 2 * (F + 1) * 2.0 ** -53 * (U.abs().T @ U.abs())).all()
+    assert (wide[:, F:] == 7.0).all()
+
+
 @pytest.mark.parametrize("F", [130, 255, 514, 642])
 def test_ragged_sizes_in_the_c_interface(F):
     """The last block of the launches per step and of the two triangular solves ends inside a tile, in rows of any alignment."""

@@ -7,6 +7,7 @@ from oracle import sorf
 from qml_lightning_amd import _lib, ops
 from tests import test_gpu_kernels as kernels
 from tests.test_gpu_kernels import t32, ti32
+from tests.test_gpu_sorf_shares import shares
 from tests.test_gpu_sorf_limits import test_rows_around_the_limits as rows_around_the_limits
 
 pytestmark = pytest.mark.gpu
@@ -60,11 +61,13 @@ def test_as_exact_as_the_rows_kernel(monkeypatch, T, S, steep):
     kernels.test_sorf_matrix_kernel_is_as_exact_as_the_rows_kernel(monkeypatch, 256, T, S, steep)
 
 
-# with the gradient 768 workgroups are resident and 1536 the shares: less than an eighth of a tile a share left, an eighth, and two rounds
+# with the gradient 768 workgroups are resident; with 1536 shares: less than an eighth of a tile a share left, an eighth, next to nothing
+# behind two tiles each, and whole tiles first again.  With 64 stacks the first three have too few rounds for that, and 768 shares
+@pytest.mark.parametrize("S", [64, 256])
 @pytest.mark.parametrize("tiles", [863, 864, 1537, 2400])
-def test_whole_tiles_first(tiles):
+def test_whole_tiles_first(tiles, S):
     import torch
-    L, S, d, ne = _lib.lib(), 64, 256, 2
+    L, d, ne = _lib.lib(), 256, 2
     g = torch.Generator(device="cuda").manual_seed(tiles)
     first = tiles // 3
     counts = (32 * first - 5, 32 * (tiles - first) - 31)
@@ -75,7 +78,7 @@ def test_whole_tiles_first(tiles):
     alpha = torch.randn(S * d, device="cuda", generator=g)
     off = torch.tensor([0, counts[0], A], dtype=torch.int32, device="cuda")
     slots = torch.randperm(A, device="cuda", generator=g).int()
-    assert L.qmll_sorf_matrix_pays(A, ne, 1, S, d, 1)
+    assert L.qmll_sorf_matrix_pays(A, ne, 1, S, d, 1) and shares(A, ne, S, d, 1) == (768 if S == 64 and tiles < 2000 else 1536)
     e, gx = ops.sorf_energy_sorted(x, off, slots, D, bias, alpha, 0.7, 1, A)
     p = 2
     ep, gp = torch.zeros(p, A, device="cuda"), torch.empty(p, A, d, device="cuda")
