@@ -2766,8 +2766,10 @@ extern "C" int qmll_prepare_fchl19_forward(const float* X, const float* Z, const
 // Wavefronts per atom of the launches that take the projections in, 0: not taken.  Up to 256 atoms eight, a CU to each workgroup.  With
 // more, two or four if they hold the reductor, and as many atoms as are resident at a time (twelve wavefronts per CU).  Energies and forces,
 // 64 components, launches apart / so, us: two elements (two wavefronts) 300 atoms of 12 29.7 / 26.1, 1200 29.7 / 27.5, 1992 31.0 / 36.4; three
-// elements (four) 492 29.4 / 26.7, 792 29.6 / 34.4; 100 x 12 through autograd 119.8 / 88.5.  Only where the representation is the work of one
-// wavefront: 3 x 40 atoms, 128 components, backward alone 31.9 / 32.9.
+// elements (four) 492 29.4 / 26.7, 792 29.6 / 34.4; 100 x 12 through autograd 117 / 110.  Larger molecules too, also where the backward launch by
+// itself would have four wavefronts an atom: two elements 33 atoms 495 32.4 / 28.8, 1485 39.0 / 34.6; 38 atoms 798 37.5 / 32.2, 1482 44.8 / 37.6; 46
+// atoms 782 43.5 / 39.0, 1472 50.3 / 43.0; one element, 128 components, 46 atoms 1196 48.5 / 43.0; three elements, 36 atoms 756 40.4 / 32.9.  Only
+// where the representation is the work of one wavefront: 3 x 40 atoms, 128 components, backward alone 31.9 / 32.9.
 static int projected_waves(int A, int n, const qmll_fchl_params* prm, int d) {
     const int R = prm->nspecies * prm->nRs2 + prm->nspecies * (prm->nspecies + 1) * prm->nRs3;
     const long long maxnn = n > 1 ? n - 1 : 1, triples = maxnn * (maxnn - 1) / 2;

@@ -826,7 +826,8 @@ def cholesky_solve_spd(A, b, overwrite_a=False, within_norms=True):
     meaningless.  A is destroyed when overwrite_a is True.
 
     U^T U differs from A by c F 2^-53 sqrt(a_ii a_jj), the measure in which a Cholesky factorisation is judged, and from 7168
-    features on by less of it than with fp64 sums alone (exact integer products, where there is memory for them).
+    features on, whether or not they are whole blocks of 128, by less of it than with fp64 sums alone (exact integer products, where there is
+    memory for them).
     within_norms=False asks for fp64 sums throughout, whose error also stays below c F 2^-53 (|U|^T |U|)_ij: that matters where
     entries of A far below sqrt(a_ii a_jj) decide entries of x that are far below its largest ones."""
     if A.dtype != torch.float64 or A.dim() != 2 or A.shape[0] != A.shape[1] or A.stride(1) != 1:
