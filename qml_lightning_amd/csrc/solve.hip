@@ -430,8 +430,9 @@ __global__ __launch_bounds__(PT, 4) void potrf_block_kernel(double* A, long long
 //     first the update of the previous panel, as above;  then for l = 0 .. 3:
 //     wait for "block l factored";  tile(l, w) = U11_l^-T tile(l, w)                      row strip
 //     for the block rows b > l:  wait for "strip (l, b) done";  tile(b, w) -= strip(l, b)^T tile(l, w)
-// They wait for lower workgroup ids only.  Every wait is bounded; one that runs out sets info to -1 and the workgroup leaves, and as every wait looks at
-// info the others leave behind it.  (Setting all flags that the workgroup still owes as well took the factorisation 0.3 % longer.  Waiting polls with
+// They wait for lower workgroup ids only.  Every wait is bounded; one that runs out sets info to -1 and the workgroup leaves, and as every
+// wait looks at info now and then the others leave behind it.  (The look is kept off the way that the chain takes, and setting the flags that the
+// workgroup still owes is not worth it: either took 16384 features 0.3 to 0.6 % longer.  Waiting polls with
 // relaxed loads: with an acquire at each poll the waiting owners kept emptying the L2 of those at work, a panel of 120 columns 326 us, 280 so.)
 //
 // Head tiles.  Once the trailing matrix is small a launch lasts as long as its slowest owner, and four of an
@@ -702,9 +703,10 @@ __device__ __forceinline__ bool follow_block(double* A, long long ld, int k0, in
                 for (unsigned n = 0; v < K + 1u && n < spin_limit; ++n) {
                     __builtin_amdgcn_s_sleep(4);
                     v = __hip_atomic_load(steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if ((n & 63) == 63 && __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;      // as in await
+                    if (__builtin_expect((n & 4095) == 4095, 0) && __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+                        n = spin_limit - 1;
                 }
-                if (v < K + 1u) {
+                if (__builtin_expect(v < K + 1u, 0)) {
                     atomicCAS(info, 0, -1);
                     v = FLAG_FAILED;
                 }
@@ -869,7 +871,7 @@ __global__ __launch_bounds__(PT, 2) void panel_kernel(double* A, long long ld, i
         }
         double* inv = invs + (size_t)(j0 / NB) * 2 * NB * NB;     // the own diagonal tile: every update is in
         const bool ok = potrf_block<true>(A, ld, j0, NB, inv, inv + NB * NB, info, flags + STEPS + bid, ps);
-        // on failure every workgroup right of this column leaves at one of these flags (or when it finds info set)
+        // where a pivot is not positive every workgroup right of this column leaves at one of these flags; where a wait has run out, at info
         if (!ok && threadIdx.x == 0) store_past_caches(flags + STEPS + bid, FLAG_FAILED);
         publish(flags + bid, ok ? FLAG_DONE : FLAG_FAILED);
         return;
