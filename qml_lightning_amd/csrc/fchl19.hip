@@ -356,9 +356,11 @@ constexpr int RS3_GROUP = 5;
 // The spacing of the bins u (lane: bin l, if ok) about the middle of the range, to a rounding of the grid's, or 0: uneven, or
 // so wide that Q could leave 2^(2 line) (y is within mid of the middle) or exp2(2 h u) 2^line.  Q^4 times a coefficient has to be finite, since the
 // weight before it may have underflown: with a line of 13 it is for coefficients of 10^6 and more (20 bins with eta3 = 2.7 up to 8.1 A, 17
-// up to 7.5).  Where distances may be anything, see group_ratio, it is 8 (6.4 and 5.9 A).  What is beyond takes its bins one by one, about the
-// middle of the range.  42000 atoms of 21, three elements, backward, in groups / one by one: 6 A 78 / 84 us, 8 A 89 / 97 (plain weights 99), 17 bins at
-// 6 A 78 / 84; 16 x 96 atoms 27.3 / 27.5 (28.1), at 8 A - / 52.6 (54.2), at 10 A - / 63.1 (65.0).
+// up to 7.5).  Where distances come from a given list and may be anything, see group_ratio, it is 8 (6.4 and 5.9 A).  What is beyond takes its bins one by one, about the
+// middle of the range (fchl19_vjp_kernel has both forms).  42000 atoms of 21, three elements, backward, in groups / one by one: 6 A 78 / 84 us, 8 A
+// 89 / 97, 17 bins at 6 A 78 / 84; at 10 A - / 98.4 (weights from the distance to each bin 99.7); 16 x 96 atoms at 8 A 47.6 / 52.6, at 10 A - / 63.1
+// (65.0).  Errors against 64 bits, 28 and 70 atoms: 6 A 3.6e-7 and 3.5e-7, 8 A 4.3e-7 and 4.6e-7, 10 A 5.1e-7 and 5.6e-7 (4.2e-7 and 4.7e-7; the middle's
+// form before distances were refined 5.6e-7 and 5.5e-7).
 constexpr float LINE_WITHIN = 13.0f, LINE_ANY = 8.0f;
 __device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid, float line) {
     const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(u)));
@@ -389,8 +391,8 @@ __device__ __forceinline__ float group_factor(float u, int l, int lane, float h)
 }
 
 // exp2(2 h y), the factor of Q that all groups share, and what the product's rounding left out: Q goes to the fourth power.
-// STOP: distances from a given list may be anything.  It stops at 2^18, which no y within mid of the middle reaches behind LINE_ANY (the weights
-// are below 2^-60 there), and Q^4 stays in range.
+// STOP: distances from a given list may be anything.  It stops at 2^18, where the weights are below 2^-49 behind either line (no y of the default
+// grid within mid of the middle gets there), and behind LINE_ANY Q^4 stays in range.
 template <bool STOP>
 __device__ __forceinline__ float group_ratio(float h, float y) {
     const float x = 2.0f * h * y, e = fexp2(STOP ? fminf(x, 18.0f) : x);
@@ -1602,7 +1604,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // LEAN: see group_sums; where the grid is not even, these two forms.
     const float mid = 0.5f * sk3 * a.p.rcut;
     const float ul = LEAN && lane < nRs3 ? fmaf(sk3, rs3v, -mid) : 0.0f;
-    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid, LINE_ANY) : 0.0f;
+    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid, a.nlist ? LINE_ANY : LINE_WITHIN) : 0.0f;
     const bool even = LEAN && spacing != 0.0f;
     bool fast = LEAN && !__any(!(fabsf(ul) <= 10.0f));
     if constexpr (!LEAN) {

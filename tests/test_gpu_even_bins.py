@@ -54,8 +54,7 @@ def test_grids(grid, natoms, molecules):
 @pytest.mark.parametrize("nrs3", [17, 18, 19])
 @pytest.mark.parametrize("natoms,molecules", [(14, 2), (50, 1)])
 def test_bins_that_are_not_there(nrs3, natoms, molecules):
-    """(17 of them, 0.35 A apart, are taken in groups where distances end at the cutoff, in molecules of up to 64 atoms on one wavefront, and one by
-    one elsewhere.)"""
+    """(17 of them, 0.35 A apart, are taken in groups where distances end at the cutoff, and one by one with a given list.)"""
     check(natoms, molecules, nrs3, "even", nrs3)
 
 
@@ -66,16 +65,24 @@ def test_weights_beyond_the_range_of_the_ratio(kw, natoms):
 
 
 @pytest.mark.parametrize("spread", [1.3, 4.0])
-def test_distances_beyond_the_cutoff(spread):
-    check(30, 1, 20, "even", 3, spread=spread)
+@pytest.mark.parametrize("rcut", [6.0, 6.4, 8.0])
+def test_distances_beyond_the_cutoff(spread, rcut):
+    check(30, 1, 20, "even", 3, spread=spread, rcut=rcut)
+
+
+@pytest.mark.parametrize("natoms", [12, 66])
+@pytest.mark.parametrize("share", [0.4, 0.7])
+def test_bins_in_the_middle_of_the_range(natoms, share):
+    """Distances far beyond all bins, where the ratio of two weights stops short."""
+    GRIDS["middle"] = lambda n, rc: np.linspace(0.5 * (1 - share) * rc, 0.5 * (1 + share) * rc, n)
+    check(natoms, 1, 20, "middle", 4, rcut=9.0)
 
 
 @pytest.mark.parametrize("natoms", [12, 50, 66])
 @pytest.mark.parametrize("nrs3,kw", [(20, dict(rcut=6.4)), (20, dict(rcut=6.5)), (17, dict(rcut=6.0)), (20, dict(rcut=8.0)), (20, dict(rcut=8.1)),
                                      (20, dict(rcut=8.2)), (17, dict(rcut=8.0)), (20, dict(rcut=10.0))])
 def test_either_side_of_the_lines(nrs3, kw, natoms):
-    """Cutoffs around those up to which even bins are taken in groups (6.4 A where distances may be anything, 8.1 A for molecules of up to 64 atoms),
-    and beyond: the bins one by one, about the middle of the range."""
+    """Cutoffs around those up to which even bins are taken in groups (6.4 A where distances may be anything, else 8.1 A), and beyond: the bins one by one, about the middle of the range."""
     check(natoms, 1, nrs3, "even", 7, **kw)
 
 
