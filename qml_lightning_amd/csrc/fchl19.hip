@@ -353,21 +353,22 @@ __device__ __forceinline__ float root(float x, float inv) {
 // made its table entries 16 bytes, and 131235 atoms of 3 to 29, five elements went from 275 to 293 us.
 constexpr int RS3_GROUP = 5;
 
-// The spacing of the bins u (lane: bin l, if ok) about the middle of the range, to a rounding of the grid's, or 0: uneven, or
-// so wide that Q could leave 2^(2 line) (y is within mid of the middle) or exp2(2 h u) 2^line.  Q^4 times a coefficient has to be finite, since the
-// weight before it may have underflown: with a line of 13 it is for coefficients of 10^6 and more (20 bins with eta3 = 2.7 up to 8.1 A, 17
-// up to 7.5).  Where distances come from a given list and may be anything, see group_ratio, it is 8 (6.4 and 5.9 A).  What is beyond takes its bins one by one, about the
-// middle of the range (fchl19_vjp_kernel has both forms).  42000 atoms of 21, three elements, backward, in groups / one by one: 6 A 78 / 84 us, 8 A
-// 89 / 97, 17 bins at 6 A 78 / 84; at 10 A - / 98.4 (weights from the distance to each bin 99.7); 16 x 96 atoms at 8 A 47.6 / 52.6, at 10 A - / 63.1
-// (65.0).  Errors against 64 bits, 28 and 70 atoms: 6 A 3.6e-7 and 3.5e-7, 8 A 4.3e-7 and 4.6e-7, 10 A 5.1e-7 and 5.6e-7 (4.2e-7 and 4.7e-7; the middle's
-// form before distances were refined 5.6e-7 and 5.5e-7).
-constexpr float LINE_WITHIN = 13.0f, LINE_ANY = 8.0f;
-__device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid, float line) {
+// The spacing of the bins u (lane: bin l, if ok) about the middle of the range, to a rounding of the grid's, or 0: uneven, or too wide.
+// Q^4 times a coefficient has to be finite, since the weight before it may have underflown.  Where Q could leave 2^(2 line) (y is within mid of the
+// middle) or exp2(2 h u) 2^line, `stops` is set, and Q is to stop at 2^24: with bins up to 1.2 apart the weights are below 2^-27 there.  A line
+// of 13 leaves room for coefficients of 10^6 and more (20 bins with eta3 = 2.7 up to 8.1 A, 17 up to 7.5); where distances come from a given list and may be
+// anything, see group_ratio, it is 8 (6.4 and 5.9 A).  Bins 1.2 apart are those of 12.1 and 10.3 A.
+// 42000 atoms of 21, three elements, backward, in groups / one by one: 6 A 78 / 86 us, 8 A 89 / 99, 10 A 90 / 99, 12 A 91 / 100, 17 bins at 6 A 78 / 85; 16 x
+// 96 atoms at 8 A 47.1 / 53.2, at 10 A 56.4 / 65.0, at 12 A 62.3 / 70.9.  Errors against 64 bits, 28 and 70 atoms: 6 A 3.5e-7, 8 A 4.1e-7 and 4.5e-7 / 4.3e-7
+// and 4.6e-7, 10 A 4.4e-7 and 4.9e-7 / 4.3e-7 and 4.7e-7, 12 A 5.1e-7 and 5.4e-7 / 5.0e-7 and 5.4e-7.
+constexpr float LINE_WITHIN = 13.0f, LINE_ANY = 8.0f, WIDEST_SPACING = 1.2f, RATIO_STOP = 16777216.0f;
+__device__ __forceinline__ float even_spacing(float u, int l, bool ok, int nRs3, float mid, float line, bool& stops) {
     const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(u)));
     const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(u), nRs3 - 1));
     const float h = (last - first) * frcp((float)(nRs3 - 1));
     const float edge = fmaxf(fabsf(first), fabsf(last)), widest = mid + edge;
-    const bool fits = fabsf(fmaf((float)-l, h, u - first)) <= 2.4e-7f * widest && widest * fabsf(h) <= line && edge * fabsf(h) <= 0.5f * line;
+    const bool fits = fabsf(fmaf((float)-l, h, u - first)) <= 2.4e-7f * widest && fabsf(h) <= WIDEST_SPACING && widest * fabsf(h) <= 40.0f;
+    stops = __any(!(widest * fabsf(h) <= line && edge * fabsf(h) <= 0.5f * line));
     return __any(ok && !fits) ? 0.0f : h;
 }
 
@@ -391,11 +392,11 @@ __device__ __forceinline__ float group_factor(float u, int l, int lane, float h)
 }
 
 // exp2(2 h y), the factor of Q that all groups share, and what the product's rounding left out: Q goes to the fourth power.
-// STOP: distances from a given list may be anything.  It stops at 2^18, where the weights are below 2^-49 behind either line (no y of the default
-// grid within mid of the middle gets there), and behind LINE_ANY Q^4 stays in range.
-template <bool STOP>
+// Distances from a given list may be anything: it stops at 2^STOP (0: not).  2^18 is where the weights are below 2^-49 behind either line (no y of the
+// default grid within mid of the middle gets there), and behind LINE_ANY Q^4 stays in range; where Q stops by itself, 2^100.
+template <int STOP>
 __device__ __forceinline__ float group_ratio(float h, float y) {
-    const float x = 2.0f * h * y, e = fexp2(STOP ? fminf(x, 18.0f) : x);
+    const float x = 2.0f * h * y, e = fexp2(STOP ? fminf(x, (float)STOP) : x);
     return fmaf(e * 0.6931472f, fmaf(2.0f * h, y, -x), e);
 }
 
@@ -1329,7 +1330,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_forward_wide_kernel(FchlArgs a
             const float4 Aj = rA[j], Ak = rA[k], Bj = rB[j], Bk = rB[k];
             const int to = whole ? triple_place(pbase, ns, Bj, Bk) : tt - t0;
             float4 entry = table_entry(zw3, hd3, Aj, Bj, Ak, Bk);
-            if constexpr (LEAN) entry.w = group_ratio<true>(h, entry.x);
+            if constexpr (LEAN) entry.w = group_ratio<18>(h, entry.x);
             reinterpret_cast<float4*>(trip)[to] = entry;
         }
         __syncthreads();
@@ -1601,12 +1602,13 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     // factor does not depend on the triple and goes into the staged gradient once per atom; the first
     // is one fma and the exponential per (triple, bin).  It is at most 2^(u_l^2), so the form is taken
     // only while u_l^2 <= 100 for every bin (eta3 rcut^2 up to about 270); beyond, the plain form runs.
-    // LEAN: see group_sums; where the grid is not even, these two forms.
+    // LEAN: see group_sums; where the grid is not even, the plain form.
     const float mid = 0.5f * sk3 * a.p.rcut;
     const float ul = LEAN && lane < nRs3 ? fmaf(sk3, rs3v, -mid) : 0.0f;
-    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid, a.nlist ? LINE_ANY : LINE_WITHIN) : 0.0f;
+    bool stops = false;
+    const float spacing = LEAN ? even_spacing(ul, lane, lane < nRs3, nRs3, mid, a.nlist ? LINE_ANY : LINE_WITHIN, stops) : 0.0f;
     const bool even = LEAN && spacing != 0.0f;
-    bool fast = LEAN && !__any(!(fabsf(ul) <= 10.0f));
+    bool fast = false;
     if constexpr (!LEAN) {
         float um = fabsf(fmaf(sk3, rs3v, -mid));
         if (lane >= nRs3) um = 0.0f;
@@ -1631,7 +1633,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     if (lane < nRs2 && wave == 0) slnRs2[lane] = flog(rs2v);
     for (int t = tid + QMLL_WAVE; t < nRs2; t += NT) slnRs2[t] = flog(a.Rs2[t]);
     if constexpr (LEAN) {
-        const float f = a.gscale * (even ? group_factor(ul, lane, lane, spacing) : fast ? fexp2(-ul * ul) : 1.0f);
+        const float f = a.gscale * (even ? group_factor(ul, lane, lane, spacing) : 1.0f);
         if (tid < nRs3) sfac[tid] = f;
     }
     for (int t = LEAN ? nRs3 : tid; t < nRs3; t += NT) {
@@ -1713,7 +1715,7 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
     const float d3 = a.p.three_body_decay;
     float us[LEAN ? LEAN_RS3 : 1], ratio[LEAN_RS3 / RS3_GROUP];        // the grid, on scalar registers
     if constexpr (LEAN) {
-        const float v = group_ratio<false>(-spacing, ul);
+        const float v = group_ratio<0>(-spacing, ul);
 #pragma unroll
         for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
 #pragma unroll
@@ -1780,13 +1782,17 @@ __global__ __launch_bounds__(64 * NW) void fchl19_vjp_kernel(FchlArgs a, const f
                 for (int l = 0; l < nRs3; ++l) bin(g[l].x, g[l].y, sRs3[l]);
             }
         };
-        if (even) {
-            const float B = group_ratio<true>(spacing, y);
+        auto groups = [&](float B, auto stop) {
 #pragma unroll
             for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) {
-                const float d = y - us[LEAN ? RS3_GROUP * q : 0];
-                group_sums(g + RS3_GROUP * q, d, fexp2(-(d * d)), B * ratio[q], spacing, Gc, Gs, Hc, Hs);
+                const float d = y - us[LEAN ? RS3_GROUP * q : 0], Q = B * ratio[q];
+                group_sums(g + RS3_GROUP * q, d, fexp2(-(d * d)), decltype(stop)::value ? fminf(Q, RATIO_STOP) : Q, spacing, Gc, Gs, Hc, Hs);
             }
+        };
+        if (__builtin_expect(even && !stops, 1)) {
+            groups(group_ratio<18>(spacing, y), std::false_type{});
+        } else if (even) {
+            groups(group_ratio<100>(spacing, y), std::true_type{});
         } else if (fast) {
             const float y2 = y + y, ny2 = -y * y;
             bins([&](float gc, float gs, float u) {
@@ -1915,8 +1921,9 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
     const float hfac = -2.0f * a.p.eta3 * frcp(sk3);
     const float mid = 0.5f * sk3 * a.p.rcut;             // distances and bins about the middle of the range: half the rounding
     const float ul = bin_ok ? fmaf(sk3, rs3v, -mid) : 0.0f;
-    const float spacing = even_spacing(ul, l3, bin_ok, nRs3, mid, LINE_WITHIN);
-    const bool even = spacing != 0.0f, fast = !__any(!(fabsf(ul) <= 10.0f));        // see fchl19_vjp_kernel for the forms
+    bool stops;
+    const float spacing = even_spacing(ul, l3, bin_ok, nRs3, mid, LINE_WITHIN, stops);
+    const bool even = spacing != 0.0f;
 
     // ---- neighbours: candidate = lane ----
     float dx = Xm[i * 3 + 0] - xo, dy = Xm[i * 3 + 1] - yo, dz = Xm[i * 3 + 2] - zo;
@@ -1950,7 +1957,7 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
         sj[pos] = lane;
     }
     // the incoming gradient, times the constant factor of its bin
-    const float f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : fast ? fexp2(-ul * ul) : 1.0f);
+    const float f3 = !bin_ok ? 0.0f : a.gscale * (even ? group_factor(ul, l3, lane, spacing) : 1.0f);
     if constexpr (!ONE) {
         gsrc = gradient();
         const float f2 = a.gscale * frcp(rs2v);
@@ -2020,7 +2027,7 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
 #pragma unroll
     for (int l = 0; l < LEAN_RS3; ++l) us[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ul), l));
     {
-        const float v = group_ratio<false>(-spacing, ul);
+        const float v = group_ratio<0>(-spacing, ul);
 #pragma unroll
         for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) ratio[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), RS3_GROUP * q));
     }
@@ -2077,45 +2084,34 @@ __device__ __forceinline__ void lean_vjp(const FchlArgs& a, int m, int i, float*
         const float4* g = reinterpret_cast<const float4*>(gin3 + __mul24((int)pair, 2 * LEAN_RS3));
         const float y = fmaf(sk3 * 0.5f, Aj.w + Ak.w, -mid);
         float Gc = 0.f, Gs = 0.f, Hc = 0.f, Hs = 0.f;
-        if (even) {
-            const float B = group_ratio<false>(spacing, y);
+        auto groups = [&](auto stop) {
+            const float B = group_ratio<0>(spacing, y);
             const float2* g2 = reinterpret_cast<const float2*>(g);
 #pragma unroll
             for (int q = 0; q < LEAN_RS3 / RS3_GROUP; ++q) {
-                const float d = y - us[RS3_GROUP * q];
-                group_sums(g2 + RS3_GROUP * q, d, fexp2(-(d * d)), B * ratio[q], spacing, Gc, Gs, Hc, Hs);
+                const float d = y - us[RS3_GROUP * q], Q = B * ratio[q];
+                group_sums(g2 + RS3_GROUP * q, d, fexp2(-(d * d)), decltype(stop)::value ? fminf(Q, RATIO_STOP) : Q, spacing, Gc, Gs, Hc, Hs);
             }
+        };
+        if (__builtin_expect(even && !stops, 1)) {
+            groups(std::false_type{});
+        } else if (even) {
+            groups(std::true_type{});
         } else {
-            auto bins = [&](auto bin) {
-#pragma unroll
-                for (int l = 0; l < LEAN_RS3; l += 2) {
-                    const float4 gv = g[l / 2];
-                    bin(gv.x, gv.y, us[l]);
-                    bin(gv.z, gv.w, us[l + 1]);
-                }
+            auto bin = [&](float gc, float gs, float u) {
+                const float dl = y - u;
+                const float e = fexp2(-(dl * dl));
+                const float de = dl * e;
+                Gc = fmaf(gc, e, Gc);
+                Gs = fmaf(gs, e, Gs);
+                Hc = fmaf(gc, de, Hc);
+                Hs = fmaf(gs, de, Hs);
             };
-            if (fast) {
-                const float y2 = y + y, ny2 = -y * y;
-                bins([&](float gc, float gs, float u) {
-                    const float e = fexp2(fmaf(y2, u, ny2));
-                    const float ue = u * e;
-                    Gc = fmaf(gc, e, Gc);
-                    Gs = fmaf(gs, e, Gs);
-                    Hc = fmaf(gc, ue, Hc);
-                    Hs = fmaf(gs, ue, Hs);
-                });
-                Hc = fmaf(y, Gc, -Hc);
-                Hs = fmaf(y, Gs, -Hs);
-            } else {
-                bins([&](float gc, float gs, float u) {
-                    const float dl = y - u;
-                    const float e = fexp2(-(dl * dl));
-                    const float de = dl * e;
-                    Gc = fmaf(gc, e, Gc);
-                    Gs = fmaf(gs, e, Gs);
-                    Hc = fmaf(gc, de, Hc);
-                    Hs = fmaf(gs, de, Hs);
-                });
+#pragma unroll
+            for (int l = 0; l < LEAN_RS3; l += 2) {
+                const float4 gv = g[l / 2];
+                bin(gv.x, gv.y, us[l]);
+                bin(gv.z, gv.w, us[l + 1]);
             }
         }
         const float S0 = Gc * cosT + Gs * sinT;

@@ -65,7 +65,7 @@ def test_weights_beyond_the_range_of_the_ratio(kw, natoms):
 
 
 @pytest.mark.parametrize("spread", [1.3, 4.0])
-@pytest.mark.parametrize("rcut", [6.0, 6.4, 8.0])
+@pytest.mark.parametrize("rcut", [6.0, 6.4, 8.0, 10.0])
 def test_distances_beyond_the_cutoff(spread, rcut):
     check(30, 1, 20, "even", 3, spread=spread, rcut=rcut)
 
@@ -80,9 +80,11 @@ def test_bins_in_the_middle_of_the_range(natoms, share):
 
 @pytest.mark.parametrize("natoms", [12, 50, 66])
 @pytest.mark.parametrize("nrs3,kw", [(20, dict(rcut=6.4)), (20, dict(rcut=6.5)), (17, dict(rcut=6.0)), (20, dict(rcut=8.0)), (20, dict(rcut=8.1)),
-                                     (20, dict(rcut=8.2)), (17, dict(rcut=8.0)), (20, dict(rcut=10.0))])
+                                     (20, dict(rcut=8.2)), (17, dict(rcut=8.0)), (20, dict(rcut=10.0)),
+                                     (20, dict(rcut=12.0)), (20, dict(rcut=12.3)), (17, dict(rcut=10.2)), (17, dict(rcut=10.5))])
 def test_either_side_of_the_lines(nrs3, kw, natoms):
-    """Cutoffs around those up to which even bins are taken in groups (6.4 A where distances may be anything, else 8.1 A), and beyond: the bins one by one, about the middle of the range."""
+    """Cutoffs around those up to which the ratio of two weights has room (6.4 A where distances may be anything, else 8.1 A), beyond, where it
+    stops short, and past 12.1 A (17 bins: 10.3), where bins are taken one by one."""
     check(natoms, 1, nrs3, "even", 7, **kw)
 
 
