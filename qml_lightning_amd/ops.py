@@ -842,19 +842,11 @@ def cholesky_solve_spd(A, b, overwrite_a=False, within_norms=True):
     # 348 us, 1472 1400 -> 687, 16 002 45.6 -> 19.2 ms; 130 128 -> 102).  A single block has its one launch either way, and would pay
     # for the copy (64 features 48 -> 61 us).
     n = F
-    U = A
-    if int(A.stride(0)) < F:
-        U = A if overwrite_a else A.clone(memory_format=torch.contiguous_format)          # rows that overlap
-    elif not overwrite_a or (F > 128 and F % 128 and int(A.stride(0)) < 1 << 23):
-        n = F if F <= 128 else (F + 127) // 128 * 128
-        try:
-            U = torch.empty(n, n, dtype=torch.float64, device=A.device)
-            check(_lib.lib().qmll_copy_upper_padded_f64(_ptr(A), int(A.stride(0)), F, _ptr(U), n, n, _stream()), "qmll_copy_upper_f64")
-        except torch.cuda.OutOfMemoryError:
-            if not overwrite_a:
-                raise
-            n = F                               # in A itself
-    ld = int(U.stride(0))
+    overlapping = int(A.stride(0)) < F
+    if F > 128 and not overlapping and (not overwrite_a or int(A.stride(0)) < 1 << 23):
+        n = (F + 127) // 128 * 128
+    copied = not overlapping and (not overwrite_a or n != F)
+    # what cannot be done without comes ahead of the copy, which an overwritten A can be
     L = _lib.lib()
     work = torch.empty(int(L.qmll_cholesky_workspace_bytes(n)) // 8 + 1, dtype=torch.float64, device=A.device)
     info = torch.zeros(1, dtype=torch.int32, device=A.device)
@@ -864,6 +856,16 @@ def cholesky_solve_spd(A, b, overwrite_a=False, within_norms=True):
         x = torch.zeros(n, dtype=torch.float64, device=A.device)
         _ptr(b)
         x[:F] = b.detach().reshape(F)
+    U = A if overwrite_a or copied else A.clone(memory_format=torch.contiguous_format)
+    if copied:
+        try:
+            U = torch.empty(n, n, dtype=torch.float64, device=A.device)
+            check(L.qmll_copy_upper_padded_f64(_ptr(A), int(A.stride(0)), F, _ptr(U), n, n, _stream()), "qmll_copy_upper_f64")
+        except torch.cuda.OutOfMemoryError:
+            if not overwrite_a:
+                raise
+            n = F                               # in A itself
+    ld = int(U.stride(0))
     slabs, nbytes = None, int(L.qmll_cholesky_slabs_bytes(n)) if within_norms else 0
     if nbytes:
         try:
@@ -874,7 +876,7 @@ def cholesky_solve_spd(A, b, overwrite_a=False, within_norms=True):
     if overwrite_a and n != F:
         check(L.qmll_copy_upper_f64(_ptr(U), n, F, _ptr(A), int(A.stride(0)), _stream()), "qmll_copy_upper_f64")
     check(L.qmll_cholesky_solve_f64(_ptr(U), n, ld, _ptr(work), _ptr(x), _stream()), "qmll_cholesky_solve_f64")
-    return x if n == F else x[:F].view(b.shape), info
+    return x[:F].view(b.shape) if x.dim() == 1 else x, info
 
 
 def format_batch(packed, parts, B, n, total, with_forces):

@@ -122,3 +122,26 @@ def test_sums_of_the_triangular_solves(F):
     residual = Vh.T @ (Vh @ got) - bd.astype(np.longdouble)
     # of either size 0.10 sqrt(F) eps, where one running sum per row or column gave 0.17
     assert np.linalg.norm(residual) <= 0.13 * F ** 0.5 * 2.0 ** -53 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("F", [704, 706])
+def test_no_memory_for_the_padded_copy(monkeypatch, F):
+    """A matrix that may be used up is factored in place where there is room for the workspace but not for a copy beside it, whichever of
+    the two is asked for first."""
+    from qml_lightning_amd import ops
+    A, b = problem(F, F)
+    kept = A.clone()
+    n = (F + 127) // 128 * 128
+    real, left = torch.empty, [8 * n * n + 1024]            # the copy alone fits, and so does the workspace
+
+    def empty(*args, **kwargs):
+        out = real(*args, **kwargs)
+        left[0] -= out.numel() * out.element_size()
+        if left[0] < 0:
+            left[0] += out.numel() * out.element_size()
+            raise torch.cuda.OutOfMemoryError("planted")
+        return out
+    monkeypatch.setattr(torch, "empty", empty)
+    x, info = ops.cholesky_solve_spd(A, b, overwrite_a=True)
+    assert int(info) == 0 and x.shape == b.shape
+    assert ((kept @ x - b).abs() <= 0.75 * (F + 1) * 2.0 ** -53 * (kept.abs() @ x.abs())).all()
